@@ -67,8 +67,9 @@ int dgi_causal_conv(void* out, int out_f32, const void* x, int x_f32, int x_stri
                     const int* seq_slots, int n_seq, int act, int residual, hipStream_t s);
 int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const void* dt_raw, int dt_f32, int dt_stride,
                  const float* dt_bias, const float* a_log, const float* d_skip, float* state, const int* positions,
-                 const int* seq_row0, const int* seq_slots, int n_seq, int heads, int dv, int N, int G, float* ws,
-                 float* wsd, int L, int nchunks, hipStream_t s);
+                 const int* seq_row0, const int* seq_slots, int n_seq, int heads, int dv, int N, int G, int chunked, int segs,
+                 int seg_rows, float* ws, float* wsd, hipStream_t s);
+int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg_rows);
 int dgi_gated_group_norm(void* out, int out_f32, const float* y, const void* z, int z_f32, int z_stride, const float* w,
                          int T, int C, int groups, float eps, hipStream_t s);
 int dgi_moe_route(int* idx, float* wts, const float* logits, int l_stride, const float* corr, int T, int R, int top,
@@ -78,12 +79,12 @@ int dgi_glu_rows(void* out, const void* gu, int gu_stride, int rows, int I, int 
 int dgi_stream_add_norm(float* x, int T, int W, const void* y, int y_stride, int y_f32, const float* post_w,
                         const float* next_w, float eps, void* out, int out_f32, const void* y2, int y2_stride, int y2_f32,
                         float mult, hipStream_t s);
+int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                     int v_stride, int in_f32, const float* aux1, int aux1_stride, const float* aux2, int aux2_stride,
                     const float* par1, const float* par2, float* state, float* norm, float* mx, const int* positions,
                     const int* seq_row0, const int* seq_slots, int n_seq, int H, int G, int dk, int dv, float cap,
                     int rows, float* norm_new, float* mx_new, hipStream_t st);
-int dgi_linear_scan_columns(int dk, int dv, int H, int n_seq, int rows);
 int dgi_token_shift(void* out, int out_f32, const void* h, int h_f32, int h_stride, const float* mu, int nmix, float* tail,
                     const int* positions, const int* row_seq, const int* seq_row0, const int* seq_slots, int n_seq, int T,
                     int W, hipStream_t st);
@@ -480,7 +481,7 @@ void causal_conv(at::Tensor out, const at::Tensor& x, const at::Tensor& w, const
 void ssm_scan(at::Tensor y, const at::Tensor& xbc, const at::Tensor& dt_raw, const at::Tensor& dt_bias,
               const at::Tensor& a_log, const at::Tensor& d_skip, at::Tensor state, const at::Tensor& positions,
               const at::Tensor& seq_row0, const at::Tensor& seq_slots, int64_t heads, int64_t dv, int64_t N, int64_t G,
-              c10::optional<at::Tensor> ws, c10::optional<at::Tensor> wsd, int64_t L, int64_t nchunks) {
+              bool chunked) {
   check_f32(y, "y"); check_f32(xbc, "xbc"); check_f32(state, "state");
   const int df = act_kind(dt_raw, "dt_raw");
   check_rows(dt_raw, "dt_raw");
@@ -490,19 +491,18 @@ void ssm_scan(at::Tensor y, const at::Tensor& xbc, const at::Tensor& dt_raw, con
   TORCH_CHECK(state.dim() == 4 && state.size(1) == heads && state.size(2) == dv && state.size(3) == N, "state must be [slots, heads, dv, N]");
   check_f32(dt_bias, "dt_bias", heads); check_f32(a_log, "a_log", heads); check_f32(d_skip, "d_skip", heads);
   const int n_seq = (int)seq_slots.numel();
-  float *wsp = nullptr, *wdp = nullptr;
-  if (ws.has_value()) {
-    TORCH_CHECK(wsd.has_value() && L >= 1 && nchunks >= 1, "ssm_scan: the chunked form needs both workspaces");
-    check_f32(*ws, "ws", (int64_t)n_seq * nchunks * heads * dv * N);
-    check_f32(*wsd, "wsd", (int64_t)n_seq * nchunks * heads);
-    TORCH_CHECK(nchunks * L >= T, "ssm_scan: nchunks * L must cover the longest portion");
-    wsp = ws->data_ptr<float>(); wdp = wsd->data_ptr<float>();
+  int segs = 1, seg_rows = 0;
+  at::Tensor ws, wsd;
+  if (chunked && n_seq > 0) segs = dgi_ssm_segments(n_seq, (int)heads, (int)dv, T, &seg_rows);
+  if (segs > 1) {
+    ws = at::empty({n_seq, segs, heads, dv, N}, state.options());
+    wsd = at::empty({n_seq, segs, heads}, state.options());
   }
   check_rc(dgi_ssm_scan(y.data_ptr<float>(), xbc.data_ptr<float>(), (int)xbc.stride(0), dt_raw.data_ptr(), df,
                         (int)dt_raw.stride(0), dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), d_skip.data_ptr<float>(),
                         state.data_ptr<float>(), i32p(positions, "positions", T), i32p(seq_row0, "seq_row0", n_seq + 1),
-                        i32p(seq_slots, "seq_slots"), n_seq, (int)heads, (int)dv, (int)N, (int)G, wsp, wdp, (int)L,
-                        (int)nchunks, cur_stream()), "ssm_scan");
+                        i32p(seq_slots, "seq_slots"), n_seq, (int)heads, (int)dv, (int)N, (int)G, chunked, segs, seg_rows,
+                        segs > 1 ? ws.data_ptr<float>() : nullptr, segs > 1 ? wsd.data_ptr<float>() : nullptr, cur_stream()), "ssm_scan");
 }
 
 void gated_group_norm(at::Tensor out, const at::Tensor& y, const at::Tensor& z, const at::Tensor& w, int64_t groups,
@@ -884,10 +884,11 @@ void linear_scan(at::Tensor y, int64_t mode, const at::Tensor& q, const at::Tens
     nrm = norm->data_ptr<float>(); mxp = mx->data_ptr<float>();
   }
   const int n_seq = (int)seq_slots.numel();
-  // a matrix memory whose heads span several column blocks stages its new normaliser / maximum (committed by a second launch)
+  // a matrix memory whose heads span several workgroups stages its new normaliser / maximum (committed by a second launch)
   at::Tensor norm_new, mx_new;
   float *nn = nullptr, *mn = nullptr;
-  if (mode == 2 && n_seq > 0 && dgi_linear_scan_columns((int)dk, (int)dv, (int)H, n_seq, T) < dv) {
+  if (mode == 2 && n_seq > 0 && dgi_linear_scan_staged((int)dk, (int)dv, (int)H, n_seq, T, q.data_ptr(), (int)q.stride(0), k.data_ptr(),
+                                                      (int)k.stride(0), f)) {
     norm_new = at::empty({n_seq, H, dk}, state.options());
     mx_new = at::empty({n_seq, H}, state.options());
     nn = norm_new.data_ptr<float>(); mn = mx_new.data_ptr<float>();
@@ -1171,8 +1172,7 @@ TORCH_LIBRARY_FRAGMENT(dgi, m) {
   m.def("causal_conv(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, Tensor(b!)? tail, Tensor positions, Tensor row_seq, "
         "Tensor seq_row0, Tensor seq_slots, int act, bool residual) -> ()");
   m.def("ssm_scan(Tensor(a!) y, Tensor xbc, Tensor dt_raw, Tensor dt_bias, Tensor a_log, Tensor d_skip, Tensor(b!) state, "
-        "Tensor positions, Tensor seq_row0, Tensor seq_slots, int heads, int dv, int N, int G, Tensor(c!)? ws=None, "
-        "Tensor(d!)? wsd=None, int L=0, int nchunks=0) -> ()");
+        "Tensor positions, Tensor seq_row0, Tensor seq_slots, int heads, int dv, int N, int G, bool chunked=False) -> ()");
   m.def("gated_group_norm(Tensor(a!) out, Tensor y, Tensor z, Tensor w, int groups, float eps) -> ()");
   m.def("moe_route(Tensor(a!) idx, Tensor(b!) wts, Tensor logits, Tensor? correction, int sigmoid=0, bool renorm=False, float wscale=1.0) -> ()");
   m.def("glu_rows(Tensor(a!) out, Tensor gu, int kind, float limit, float alpha, Tensor? row_scale) -> ()");

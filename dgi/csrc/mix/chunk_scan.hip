@@ -1,22 +1,39 @@
-// dgi/csrc/mix/chunk_scan.hip — linear_scan's decayed recurrences (gla, light: see linear_scan.hip) for prompt portions, sixteen
-// tokens at a time in fp32 matrix products (v_mfma_f32_16x16x4_f32):
+// dgi/csrc/mix/chunk_scan.hip — prompt portions of the recurrences that carry a matrix S [dk, dv] per head (linear_scan.hip has
+// their definitions, ssm_scan.hip that of ssm), sixteen tokens at a time in fp32 matrix products (v_mfma_f32_16x16x4_f32).
 //
-//     S_t = diag(a_t) S_(t-1) + k_t v_t^T,   o_t = S_t^T q_t                       S [dk, dv] fp32
+// For tokens t, s of a chunk that starts from the state S, with D[t, s] the product of the decays of the tokens after s up to t
+// and A_t that of all tokens up to t:
 //
-// With b_t the product of the decays of the chunk's tokens up to t (per key channel) and b the product of all sixteen,
+//     o_t = A_t S^T q_t + sum_(s <= t) P[t, s] u_s,   P[t, s] = D[t, s] (q_t . k_s) c_s          S <- A_15 S + sum_s D[15, s] c_s k_s u_s^T
 //
-//     o_t = (q_t b_t)^T S + sum_(s <= t) [(q_t b_t) . (k_s / b_s)] v_s,        S <- diag(b) S + sum_s (k_s b / b_s) v_s^T
+// light: u = v, c = 1;  ssm: q = C, k = B, u = x, c = dt;  mlstm: c = the input gate, o divided by the normaliser;
+// wkv: the decays are per key channel, so they sit inside the products: q_t and k_s are scaled by the decays between them and
+// the middle of the chunk (so chunk halves, not chunks, have to stay in the fp32 range), the state products use prefix and suffix
+// products and no division;  it reads before it writes: s < t, and the bonus on the diagonal;
+// delta: u solves (I + T) u = beta (v - A S^T k), T[t, s] = beta_t D[t, s] (k_t . k_s) below the diagonal: block forward
+// substitution with blocks of four tokens, each block one matrix product with M_b = [inverse of its diagonal block - I;
+// - T below it times that inverse].  (gla: chunk_scan_decay.hip.)
 //
-// A workgroup owns (sequence, head, 16 value columns).  Four waves compute: wave w holds the state rows of the 16-channel
-// tiles w, w + 4, .. in registers, in the layout the products leave them (the key index inside a product is permuted so that the
-// state registers are its operand as they are).  The waves' partial score tiles and outputs meet in LDS.  Four more
-// waves prepare: wave w loads the same channels of the next chunk, forms the running products and writes the scaled
-// operands to the other LDS buffer, and stores the previous chunk's outputs.  Their loads run NP chunks ahead in a register
-// ring (the chunk loop is unrolled NP times).  Two barriers per chunk.
+// A workgroup owns (sequence, head, NC blocks of 16 value columns) and is a pipeline of waves that hand chunks on through LDS, one
+// barrier per chunk:
+//   preparing waves  load q / k (and the channel decays) two chunks ahead in registers and write them (scaled) to LDS;
+//   gates wave       gates of 64 tokens at a time (in four steps, so that none is long), D and A of each chunk;
+//   scores waves     two that take turns: q . k, P and (delta) M;
+//   state waves      one per column block: the state rows of all key channels of its 16 columns stay in registers, in the layout the
+//                    products leave them (the key index inside a product is permuted so that the registers are its operand as
+//                    they are; delta permutes the tokens the same way, so u is an operand as it is), so no wave waits for
+//                    another's partial sums; the state before the chunk goes to LDS;  a normaliser wave beside them (mlstm);
+//   output waves     one per column block: read-out of that state, P u, the store.
+// So a chunk's products (per column block 2 dk / 4 + 4 of 32 cycles each, delta 3 dk / 4 + 8, beside dk / 4 or dk / 2 for the scores)
+// spread over the compute unit's four matrix cores; what bounds a chunk is the longest role's chain: the state wave's (delta: read-out
+// by k, substitution, update) or a preparing wave's arithmetic (wkv): a wave issues an instruction every four to five cycles at best, so
+// addresses are lane offsets kept in registers, and rows past the end a branch of their own.  Measured, a step of 2 prompts of 4096 rows in
+// all, 64 heads, states 64 x 64 (ssm 128 x 64), against the same token by token on the vector ALUs (linear_scan.hip, ssm_scan.hip):
+// delta 173 us (726), ssm 196 (637), wkv 250 (some 630), light 167 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 92 (322).
 //
-// Products of decays can leave the fp32 range.  A wave whose channels decay by more than 1e28 within a chunk gets the raw
-// values instead and runs that chunk token by token on the same registers (its contribution to the outputs is a
-// sum over its own channels, so waves may differ).  A portion at position 0 reads no state.
+// Half-chunk products of channel decays below 1e-28 leave the range of the scaled operands; the wave that prepares such channels
+// then sums their scores token by token instead.  An infinity or NaN among a chunk's u takes a path that keeps it from the tokens
+// before it (a matrix product multiplies it by their zeros).  A portion at position 0 reads no state.
 #include <type_traits>
 #include "../common.h"
 
@@ -24,298 +41,1033 @@ using namespace dgi;
 
 namespace {
 
-template <typename T> __device__ __forceinline__ float ldf(const T* p);
-template <> __device__ __forceinline__ float ldf<float>(const float* p) { return *p; }
-template <> __device__ __forceinline__ float ldf<uint16_t>(const uint16_t* p) { return bf16_to_f32(*p); }
-
+constexpr int WKV = 0, DELTA = 1, MLSTM = 2, LIGHT = 4, SSM = 5;      // 3: gla, chunk_scan_decay.hip
 constexpr int C = 16;              // tokens per chunk
 constexpr int TR = 20;             // padded row of sixteen tokens
 constexpr float SAFE = 1e-28f;
 
 struct ChunkArgs {
-  float* y;
-  const void *q, *k, *v;
+  float* y;                        // [T, H * dv]
+  const void *q, *k, *v;           // rows with their own strides (elements); wkv: q the receptance; ssm: C, B, x
   int q_stride, k_stride, v_stride;
-  const float* decay;              // per channel: [T, H * dk]; per head: [H]
-  int decay_stride;
-  float* state;
+  const void *aux1, *aux2;         // per token: w_raw [T, H*dk] | b_raw | i_raw | - | dt_raw;  - | a_raw | f_raw | - | -
+  int aux1_stride, aux2_stride, aux_bf16;
+  const float *par1, *par2, *par3; // w0 | a_log | - | decay [H] | a_log;  u | dt_bias | - | - | dt_bias;  ssm: d_skip
+  float *state, *norm, *mx;        // state [slots, H, dk, dv] (ssm: [slots, H, dv, dk])
+  float *norm_new, *mx_new;        // mlstm with several workgroups per head: staged, as in linear_scan
   const int *positions, *seq_row0, *seq_slots;
-  int H, dk, dv;
+  int H, G, dk, dv;
+  int n_seq;
+  int pass, seg_rows;              // ssm in segments: 0 whole portions, 1 and 2 the two passes
+  float *ws, *wsd;                 // [n_seq, segments, H, dv, dk] states, [n_seq, segments, H] decays
+  int skip_rows;                   // sequences of at most this many rows are not this launch's
+  float cap;
 };
 
+template <typename T> __device__ __forceinline__ float ldf(const T* p);
+template <> __device__ __forceinline__ float ldf<float>(const float* p) { return *p; }
+template <> __device__ __forceinline__ float ldf<uint16_t>(const uint16_t* p) { return bf16_to_f32(*p); }
 __device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float silu(float x) { return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f)); }
+__device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
+__device__ __forceinline__ float logsigmoid_f(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < __builtin_inff(); }
 
-// LIGHT: one decay per head and SiLU on q, k, v; else a decay per token and channel and q scaled by dk^-1/2.
-// TD: 16-channel tiles per wave (dk <= 64 TD)
-template <bool LIGHT, typename TI, int TD>
-__global__ __launch_bounds__(512) void chunk_scan_kernel(const ChunkArgs a) {
-  constexpr int DP = 64 * TD, QR = DP + 4;
-  constexpr int BUF = 2 * C * QR + DP * TR + C * TR + DP + 4;
+// four consecutive elements as they lie in memory
+template <typename T> struct Raw4;
+template <> struct Raw4<float> { float4 v; };
+template <> struct Raw4<uint16_t> { uint2 v; };
+__device__ __forceinline__ void widen(const Raw4<float>& r, float* f) { f[0] = r.v.x; f[1] = r.v.y; f[2] = r.v.z; f[3] = r.v.w; }
+__device__ __forceinline__ void widen(const Raw4<uint16_t>& r, float* f) {
+  f[0] = __uint_as_float(r.v.x << 16); f[1] = __uint_as_float(r.v.x & 0xffff0000u);
+  f[2] = __uint_as_float(r.v.y << 16); f[3] = __uint_as_float(r.v.y & 0xffff0000u);
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+
+// e^x to about an ulp: 2^(x log2 e) with the product in two parts.  x within [-200, 6], where e^-e^x covers every fp32 value below 1.
+__device__ __forceinline__ float exp_2part(float x) {
+  const float h = x * 1.44269502f, l = fmaf(x, 1.44269502f, -h) + x * 1.92596299e-8f;
+  const float e = __builtin_amdgcn_exp2f(h);
+  return fmaf(e, l * 0.693147181f, e);
+}
+__device__ __forceinline__ float exp_neg_exp(float x) {
+  const float r = exp_2part(-exp_2part(fminf(fmaxf(x, -200.f), 5.f)));
+  return x == x ? r : x;
+}
+
+// Sums of sixteen values over the 64 lanes: lane l gets the total of v[l & 15].  Each step halves the values a lane keeps.
+__device__ __forceinline__ float sum16(const float* v, int lane) {
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+  float w[8], x[4], z[2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w[i] = (b0 ? v[2 * i + 1] : v[2 * i]) + dpp_move<0xB1>(b0 ? v[2 * i] : v[2 * i + 1]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = (b1 ? w[2 * i + 1] : w[2 * i]) + dpp_move<0x4E>(b1 ? w[2 * i] : w[2 * i + 1]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) z[i] = (b2 ? x[2 * i + 1] : x[2 * i]) + __shfl_xor(b2 ? x[2 * i] : x[2 * i + 1], 4, 64);
+  float r = (b3 ? z[1] : z[0]) + dpp_move<0x128>(b3 ? z[0] : z[1]);
+  r += __shfl_xor(r, 16, 64);
+  return r + __shfl_xor(r, 32, 64);
+}
+
+// LDS (floats) and roles of a workgroup.  NT: 16-channel tiles (dk <= 16 NT).  A chunk's steps, in order: q / k written, scores (two
+// steps; one for NT 16, whose buffers must be fewer), state, output: an array read d steps after it is written has d + 1 buffers.
+template <int MODE, int NT>
+struct Lay {
+  static constexpr bool CH = MODE == WKV;                      // decays per key channel
+  static constexpr bool TURNS = CH || MODE == LIGHT;           // two sets of preparing waves take turns, two steps a chunk
+  static constexpr int NC = NT <= 8 ? 2 : 1, W2 = NT <= 8 ? 2 : 1;
+  static constexpr int NS = NT / 4;                            // preparing waves of 64 channels
+  // Waves: state, output, then gates and normaliser (or preparing waves), scores, (more) preparing waves: waves four apart share a SIMD,
+  // and the scores' products are best beside the output waves', the fewest.
+  static constexpr int SETS = CH && NT == 4 ? 2 : 1;           // channel decays: one set of preparing waves for the scores, one for the state
+  static constexpr int PREPS = (TURNS ? 2 : 1) * NS * SETS;    // preparing waves, EARLY of them before the scores waves
+  static constexpr int EARLY = NC == 1 ? 0 : (CH ? 2 : (MODE == MLSTM ? 0 : 1));
+  static constexpr int OUT = NC, GATES = 2 * NC, NORM = GATES + 1, SCORES = NC == 1 ? 4 : 6, PREP = SCORES + W2;
+  static constexpr int WAVES = PREP + PREPS - EARLY;
+  static constexpr int LEAD = 2 + W2 + (TURNS ? 1 : 0);        // steps before the first output
+  static constexpr int DP = 16 * NT, QR = DP + 4, ROWS = C * QR;
+  static constexpr int QB = 3 + W2, KB = 2 + W2;               // buffers of q and k
+  static constexpr int Q = 0;                                  // [QB][16][QR] q (channel decays: times the prefix products)
+  static constexpr int K = Q + QB * ROWS;                      // [KB][16][QR] k; channel decays: [2][16][QR] scaled for the scores
+  static constexpr int QT = K + (CH ? 2 : KB) * ROWS;          // CH: [2][16][QR] q scaled for the scores
+  static constexpr int KT = QT + (CH ? 2 * ROWS : 0);          // CH: [KB][DP][TR] k times the suffix products, by channel
+  static constexpr int DEC = KT + (CH ? KB * DP * TR : 0);     // CH: [KB][DP] decay of the whole chunk
+  static constexpr int ST = DEC + (CH ? KB * DP : 0);          // [2][NC][NT][64][4] state before the chunk, as the state wave holds it
+  static constexpr int U = ST + 2 * NC * DP * 16;              // DELTA: [2][NC][64][4] u
+  static constexpr int P = U + (MODE == DELTA ? 2 * NC * 256 : 0);     // [4][16][TR]
+  static constexpr int M = P + 4 * C * TR;                     // DELTA: [2][16][TR]
+  static constexpr int T = M + (MODE == DELTA ? 2 * C * TR : 0);       // DELTA: [2][16][TR]
+  static constexpr int SC = T + (MODE == DELTA ? 2 * C * TR : 0);      // [4][96] per-token factors, see below
+  static constexpr int GT = SC + (CH ? 0 : 4 * 96);            // [2][3][64] gates of 64 tokens
+  static constexpr int DM = GT + (CH ? 0 : 384);               // [4][64][4] D as the scores wave holds P^T, [4][16] A
+  static constexpr int NRM = DM + (CH ? 0 : 4 * 272);              // DELTA: [4][NS][32] squared norms;  MLSTM: [DP] normaliser
+  static constexpr int RAW = NRM + (MODE == DELTA ? 4 * NS * 32 : (MODE == MLSTM ? DP : 0));      // CH: [2][NS][RAWN]
+  static constexpr int RAWN = 276;
+  static constexpr int END = RAW + (CH ? 2 * NS * RAWN : 0);
+};
+// per-token factors [16] each: 0 of the state read-out, 16 of the state update, 32 delta: beta, mlstm: row sums of P, then 1 / normaliser,
+// 48 delta: -beta A / |k|, mlstm: exp(-maximum), 64 mlstm: A, 80 (one number) decay of the chunk
+
+// two waves per SIMD at least: within 256 registers the products take ordinary registers, without moves to accumulation ones
+template <int MODE, typename TI, int NT>
+__global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_kernel(const ChunkArgs a) {
+  using L = Lay<MODE, NT>;
+  constexpr int QR = L::QR, DP = L::DP, NS = L::NS, LEAD = L::LEAD;
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  float* redA = sm + 2 * BUF;      // [4][16][17]
-  float* redO = redA + 4 * 16 * 17 + 4;      // [4][16][16]
-  const int seq = blockIdx.x, head = blockIdx.y, col0 = blockIdx.z * 16;
-  const int row0 = a.seq_row0[seq], n = a.seq_row0[seq + 1] - row0;
-  if (n <= 0) return;
-  const int p0 = a.positions[row0], slot = a.seq_slots[seq];
+  // consecutive workgroups (which go to different XCDs) own consecutive heads; a head's workgroups come n_seq * H later
+  const int head = blockIdx.x % a.H, seq = blockIdx.x / a.H % a.n_seq, zb = blockIdx.x / a.H / a.n_seq, seg = MODE == SSM ? blockIdx.y : 0;
+  int row0 = a.seq_row0[seq], n = a.seq_row0[seq + 1] - row0;
+  if (n <= a.skip_rows) return;
+  const int slot = a.seq_slots[seq];
+  // ssm in segments (see below): 1 the state of a segment from nothing, to the workspace; 2 outputs from the state found there
+  bool stored = a.positions[row0] > 0, last = true;
+  if (MODE == SSM && a.pass) {
+    row0 += seg * a.seg_rows;
+    n -= seg * a.seg_rows;
+    last = n <= a.seg_rows;
+    if (n <= 0 || (last && a.pass == 1)) return;
+    n = min(n, a.seg_rows);
+    stored = a.pass == 2;
+  }
   const int H = a.H, dk = a.dk, dv = a.dv;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int kvh = head / (H / a.G);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int n16 = lane & 15, g = lane >> 4;
-  const bool computes = wave < 4;
-  const int w = wave & 3;
-  const int chunks = (n + C - 1) / C;
-  const float qscale = LIGHT ? 1.f : 1.f / sqrtf((float)dk);
-  const float hdecay = LIGHT ? a.decay[head] : 0.f;
+  const int chunks = ((n + C - 1) / C + 1) & ~1;      // an even number: a chunk past the end changes nothing
+  const float qscale = 1.f / sqrtf((float)dk);
+  const TI* qb = (const TI*)a.q + (size_t)row0 * a.q_stride + (size_t)kvh * dk;
+  const TI* kb = (const TI*)a.k + (size_t)row0 * a.k_stride + (size_t)kvh * dk;
 
-  auto Qs = [&](int b) { return sm + b * BUF; };                             // [16][QR]   q b_t
-  auto Ks = [&](int b) { return sm + b * BUF + C * QR; };                    // [16][QR]   k / b_t
-  auto KT = [&](int b) { return sm + b * BUF + 2 * C * QR; };                // [DP][TR]   k b / b_t by channel (raw chunk: decays)
-  auto VT = [&](int b) { return sm + b * BUF + 2 * C * QR + DP * TR; };      // [16][TR]   v by column
-  auto Bc = [&](int b) { return sm + b * BUF + 2 * C * QR + DP * TR + C * TR; };      // [DP]
-  auto Raw = [&](int b) { return sm + b * BUF + 2 * C * QR + DP * TR + C * TR + DP; };      // [4] wave runs the chunk raw
-
-  // ---- preparing waves: lane = (channel n16 of the tile, tokens 4 g ..)
-  constexpr int NP = TD == 1 ? 4 : (TD == 2 ? 2 : 1);
-  // kept as loaded: a conversion at the load would wait for it on the spot
-  TI rq[NP][TD][4], rk[NP][TD][4], rv[NP];
-  float rd[NP][TD][4];
-  const TI* qb = (const TI*)a.q + (size_t)row0 * a.q_stride + head * dk;
-  const TI* kb = (const TI*)a.k + (size_t)row0 * a.k_stride + head * dk;
-  const TI* vb = (const TI*)a.v + (size_t)row0 * a.v_stride + (size_t)head * dv + col0;
-  const float* db = LIGHT ? nullptr : a.decay + (size_t)row0 * a.decay_stride + head * dk;
-  // loads run unconditionally (rows and channels clamped into the portion); prepare() drops what is outside
-  auto load = [&](int ci, int st) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = min(ci * C + 4 * g + i, n - 1);
-#pragma unroll
-      for (int td = 0; td < TD; ++td) {
-        const int ch = min(16 * (td * 4 + w) + n16, dk - 1);
-        rq[st][td][i] = qb[(size_t)t * a.q_stride + ch];
-        rk[st][td][i] = kb[(size_t)t * a.k_stride + ch];
-        if constexpr (!LIGHT) rd[st][td][i] = db[(size_t)t * a.decay_stride + ch];
-      }
-    }
-    rv[st] = vb[(size_t)min(ci * C + 4 * w + g, n - 1) * a.v_stride + min(n16, dv - 1 - col0)];
+  // Every role passes chunks + LEAD barriers.  Loads run unconditionally (rows and channels clamped into the portion) in loops of two
+  // chunks: a load behind a branch, or one whose registers are renamed at the end of a loop, would be waited for on the spot.
+  auto barriers = [&](int m) {
+    for (int i = 0; i < m; ++i) __syncthreads();
   };
-  auto silu = [](float x) {
-    return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-  };
-  auto prepare = [&](int ci, int st) {
-    const int b = ci & 1, left = n - ci * C;         // tokens from this chunk on
-    float q[TD][4], k[TD][4], d[TD][4], bt[TD][4], tot[TD];
-    bool raw = false;
+  const int prep = wave >= L::PREP ? wave - L::PREP + L::EARLY : (wave < L::SCORES && wave >= L::SCORES - L::EARLY ? wave - (L::SCORES - L::EARLY) : -1);
+  if (prep >= 0) {
+    // ============================================================================================== preparing waves
+    const int w = prep % NS, turn = prep / NS % 2, set = prep / (2 * NS);       // set: 0 the scores' operands, 1 the state's (or 0: both)
+    if constexpr (L::CH) {
+      // lane = channel.  Chunk c takes two steps of its wave: decays, then products and LDS.
+      const int ch = 64 * w + lane, cc = min(ch, dk - 1);
+      const bool in = ch < dk;
+      const unsigned oq = cc * sizeof(TI), od = cc * 4;
+      const char* db = (const char*)((const float*)a.aux1 + (size_t)row0 * a.aux1_stride + (size_t)head * dk);
+      TI rq[C], rk[C];
+      float rd[C], d[C];
+      const float w0 = a.par1[(size_t)head * dk + cc], bonus = a.par2[(size_t)head * dk + cc];
+      const float qs = in ? 1.f : 0.f;               // channels past dk: q = 0
+      // the lane's offsets from a chunk's first row are kept, the row's address advances in scalar registers
+      unsigned vq[C], vk[C], vd[C];
 #pragma unroll
-    for (int td = 0; td < TD; ++td) {
-      const bool in = 16 * (td * 4 + w) + n16 < dk;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const bool ok = in && 4 * g + i < left;
-        q[td][i] = ok ? ldf<TI>(&rq[st][td][i]) : 0.f;
-        k[td][i] = ok ? ldf<TI>(&rk[st][td][i]) : 0.f;
-        if constexpr (LIGHT) d[td][i] = ok ? hdecay : 1.f;
-        else d[td][i] = ok ? rd[st][td][i] : 1.f;
+      for (int t = 0; t < C; ++t) {
+        vq[t] = (unsigned)t * a.q_stride * (unsigned)sizeof(TI) + oq;
+        vk[t] = (unsigned)t * a.k_stride * (unsigned)sizeof(TI) + oq;
+        vd[t] = (unsigned)t * a.aux1_stride * 4u + od;
       }
-    }
-    const float v = (4 * w + g < left && col0 + n16 < dv) ? ldf<TI>(&rv[st]) : 0.f;
+      auto load_d = [&](int c) {
+        const int first = min(c * C, n - 1);
+        const char* p = db + (size_t)first * a.aux1_stride * 4;
+        asm volatile("" : "+s"(p));
+        if (first + C <= n) {
 #pragma unroll
-    for (int td = 0; td < TD; ++td) {
-      bt[td][0] = d[td][0];
-#pragma unroll
-      for (int i = 1; i < 4; ++i) bt[td][i] = bt[td][i - 1] * d[td][i];
-      const float p = bt[td][3];
-      const float p0_ = __shfl(p, n16, 64), p1_ = __shfl(p, n16 + 16, 64), p2_ = __shfl(p, n16 + 32, 64), p3_ = __shfl(p, n16 + 48, 64);
-      const float e = (g > 0 ? p0_ : 1.f) * (g > 1 ? p1_ : 1.f) * (g > 2 ? p2_ : 1.f);
-      tot[td] = p0_ * p1_ * p2_ * p3_;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) bt[td][i] *= e;
-      raw |= !(tot[td] > SAFE);
-    }
-    raw = __any(raw);
-#pragma unroll
-    for (int td = 0; td < TD; ++td) {
-      const int ch = 16 * (td * 4 + w) + n16;
-      float kt[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float qi = LIGHT ? silu(q[td][i]) : q[td][i] * qscale, ki = LIGHT ? silu(k[td][i]) : k[td][i];
-        if (raw) {
-          kt[i] = d[td][i];
+          for (int t = 0; t < C; ++t) rd[t] = *reinterpret_cast<const float*>(p + vd[t]);
         } else {
-          qi *= bt[td][i];
-          ki *= __builtin_amdgcn_rcpf(bt[td][i]);
-          kt[i] = ki * tot[td];
-        }
-        Qs(b)[(4 * g + i) * QR + ch] = qi;
-        Ks(b)[(4 * g + i) * QR + ch] = ki;
-      }
-      *reinterpret_cast<float4*>(KT(b) + ch * TR + 4 * g) = make_float4(kt[0], kt[1], kt[2], kt[3]);
-      if (g == 0) Bc(b)[ch] = tot[td];
-    }
-    VT(b)[n16 * TR + 4 * w + g] = LIGHT ? silu(v) : v;
-    if (lane == 0) Raw(b)[w] = raw ? 1.f : 0.f;
-  };
-  auto store = [&](int ci) {       // outputs of chunk ci: one per lane of the preparing waves
-    const int t = 4 * w + g, col = col0 + n16;
-    const float* r = redO + t * 16 + n16;
-    const float o = (r[0] + r[256]) + (r[512] + r[768]);
-    if (ci * C + t < n && col < dv) a.y[(size_t)(row0 + ci * C + t) * H * dv + (size_t)head * dv + col] = o;
-  };
-
-  // The two roles run loops of their own (a wave never changes its role) with the same barriers: two per chunk, one before.
-  if (!computes) {
-    const int last = chunks - 1;
 #pragma unroll
-    for (int st = 0; st < NP; ++st) load(min(st, last), st);
-    prepare(0, 0);
-    load(min(NP, last), 0);
-    __syncthreads();
-    // st: the chunk's place in the register ring (its index modulo NP)
-    auto step = [&](int ci, auto stage) {
-      constexpr int nx = (decltype(stage)::value + 1) % NP;
-      if (ci > 0) store(ci - 1);
-      if (ci < last) {
-        prepare(ci + 1, nx);
-        load(min(ci + 1 + NP, last), nx);
+          for (int t = 0; t < C; ++t) rd[t] = *reinterpret_cast<const float*>(p + ((unsigned)min(t, n - 1 - first) * a.aux1_stride * 4u + od));
+        }
+      };
+      auto load_qk = [&](int c) {
+        const int first = min(c * C, n - 1);
+        const char *q = (const char*)(qb + (size_t)first * a.q_stride), *k = (const char*)(kb + (size_t)first * a.k_stride);
+        asm volatile("" : "+s"(q), "+s"(k));
+        if (first + C <= n) {
+#pragma unroll
+          for (int t = 0; t < C; ++t) {
+            rq[t] = *reinterpret_cast<const TI*>(q + vq[t]);
+            rk[t] = *reinterpret_cast<const TI*>(k + vk[t]);
+          }
+        } else {
+#pragma unroll
+          for (int t = 0; t < C; ++t) {
+            const unsigned r = (unsigned)min(t, n - 1 - first) * (unsigned)sizeof(TI);
+            rq[t] = *reinterpret_cast<const TI*>(q + (r * a.q_stride + oq));
+            rk[t] = *reinterpret_cast<const TI*>(k + (r * a.k_stride + oq));
+          }
+        }
+      };
+      auto decays = [&]() {
+#pragma unroll
+        for (int t = 0; t < C; ++t) d[t] = exp_neg_exp(rd[t] + w0);
+      };
+      auto prepare = [&](int c) {
+        const int left = n - c * C;
+        float* Q = sm + L::Q + (c % L::QB) * L::ROWS + ch;
+        float* QT = sm + L::QT + (c & 1) * L::ROWS + ch;
+        float* K = sm + L::K + (c & 1) * L::ROWS + ch;
+        float* KT = sm + L::KT + ((c % L::KB) * DP + ch) * TR;
+        float q[C], k[C];
+#pragma unroll
+        for (int t = 0; t < C; ++t) {
+          q[t] = ldf<TI>(&rq[t]) * qs;
+          k[t] = ldf<TI>(&rk[t]);
+        }
+        if (left < C) {                                      // rows past the portion: nothing read, nothing written, no decay
+#pragma unroll
+          for (int t = 0; t < C; ++t)
+            if (t >= left) { q[t] = 0.f; k[t] = 0.f; d[t] = 1.f; }
+        }
+        float s[C];
+        if (L::SETS == 1 || set == 1) {
+          // suffix products: the state's update
+          float run = 1.f;
+#pragma unroll
+          for (int t = C - 1; t >= 0; --t) {
+            s[t] = k[t] * run;
+            run *= d[t];
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(KT + 4 * i) = make_float4(s[4 * i], s[4 * i + 1], s[4 * i + 2], s[4 * i + 3]);
+          sm[L::DEC + (c % L::KB) * DP + ch] = run;
+          // prefix products: the state's read-out, before the token's own decay
+          float f = 1.f;
+#pragma unroll
+          for (int t = 0; t < C; ++t) {
+            const float before = f;
+            f *= d[t];
+            Q[t * QR] = q[t] * before;
+          }
+        }
+        if (L::SETS == 2 && set == 1) return;
+        // the scores' scales, from the middle of the chunk out
+        float lo = 1.f, hi = 1.f;
+#pragma unroll
+        for (int t = 7; t >= 0; --t) {                       // lo: decays of the tokens after t up to the middle
+          const float own = lo * d[t];
+          QT[t * QR] = q[t] * __builtin_amdgcn_rcpf(own);
+          K[t * QR] = k[t] * lo;
+          lo = own;
+        }
+#pragma unroll
+        for (int t = 8; t < C; ++t) {                        // hi: decays from the middle on up to t
+          const float before = hi;
+          hi *= d[t];
+          QT[t * QR] = q[t] * before;
+          K[t * QR] = k[t] * __builtin_amdgcn_rcpf(hi);
+        }
+        float* R = sm + L::RAW + ((c & 1) * NS + w) * L::RAWN;
+        const bool raw = __any(!(lo > SAFE && hi > SAFE));
+        if (lane == 0) R[0] = raw ? 1.f : 0.f;
+#pragma unroll
+        for (int t = 0; t < C; ++t) s[t] = q[t] * bonus * k[t];
+        const float bo = sum16(s, lane);
+        if (lane < C) R[4 + lane] = bo;
+        if (__builtin_expect(raw, 0)) {                      // scores of these 64 channels token by token
+#pragma unroll 1
+          for (int i = 0; i < C; ++i) {
+            float ki = 0.f, run1 = 1.f;
+#pragma unroll
+            for (int t = 0; t < C; ++t) ki = t == i ? k[t] : ki;
+#pragma unroll
+            for (int t = 0; t < C; ++t) {
+              const float before = run1;
+              run1 = t > i ? run1 * d[t] : run1;
+              s[t] = t >= i ? q[t] * ki * before : 0.f;
+            }
+            const float o = sum16(s, lane);
+            if (lane < C) R[20 + i * C + lane] = o;
+          }
+        }
+      };
+      load_d(turn);
+      load_qk(turn);
+      barriers(turn);
+      for (int c = turn; c < chunks; c += 2) {
+        decays();
+        load_d(c + 2);
+        __syncthreads();
+        prepare(c);
+        load_qk(c + 2);
+        __syncthreads();
       }
-      __syncthreads();
-      __syncthreads();
-    };
-    for (int ci = 0; ci < chunks; ci += NP) {
-      step(ci, std::integral_constant<int, 0>{});
-      if constexpr (NP > 1) {
-        if (ci + 1 < chunks) step(ci + 1, std::integral_constant<int, 1>{});
-      }
-      if constexpr (NP > 2) {
-        if (ci + 2 < chunks) step(ci + 2, std::integral_constant<int, 2>{});
-        if (ci + 3 < chunks) step(ci + 3, std::integral_constant<int, 3>{});
+      barriers(LEAD - turn);
+    } else {
+      // lane = (token, quarter): sixteen channels of a token in four pieces
+      const int t = lane >> 2, j = lane & 3;
+      Raw4<TI> rq[2][4], rk[2][4];
+      // the lane's offsets from a chunk's first row are kept, the row's address advances in scalar registers
+      unsigned vx[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vx[i] = (unsigned)min(64 * w + 16 * i + 4 * j, dk - 4) * (unsigned)sizeof(TI);
+      const unsigned vq = (unsigned)t * a.q_stride * (unsigned)sizeof(TI), vk = (unsigned)t * a.k_stride * (unsigned)sizeof(TI);
+      auto load = [&](int c, int st) {
+        const int first = min(c * C, n - 1);
+        const char *pq = (const char*)(qb + (size_t)first * a.q_stride), *pk = (const char*)(kb + (size_t)first * a.k_stride);
+        asm volatile("" : "+s"(pq), "+s"(pk));
+        unsigned oq = vq, ok = vk;
+        if (first + C > n) {
+          const unsigned r = (unsigned)min(t, n - 1 - first) * (unsigned)sizeof(TI);
+          oq = r * a.q_stride;
+          ok = r * a.k_stride;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          rq[st][i] = *reinterpret_cast<const Raw4<TI>*>(pq + (oq + vx[i]));
+          rk[st][i] = *reinterpret_cast<const Raw4<TI>*>(pk + (ok + vx[i]));
+        }
+      };
+      float q[4][4], k[4][4];
+      auto take = [&](int c, int st) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          widen(rq[st][i], q[i]);
+          widen(rk[st][i], k[i]);
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            if (MODE == LIGHT) q[i][x] = silu(q[i][x]);
+          }
+        }
+        if (n - c * C < C || dk < DP) {                      // rows past the portion, channels past dk: zeros
+          const bool ok = c * C + t < n;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const bool in = ok && 64 * w + 16 * i + 4 * j + x < dk;
+              q[i][x] = in ? q[i][x] : 0.f;
+              k[i][x] = in ? k[i][x] : 0.f;
+            }
+        }
+      };
+      auto put = [&](int c) {
+        if constexpr (MODE == LIGHT) {                       // zeros stay zeros
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) k[i][x] = silu(k[i][x]);
+        }
+        float* Q = sm + L::Q + (c % L::QB) * L::ROWS + t * QR + 64 * w + 4 * j;
+        float* K = sm + L::K + (c % L::KB) * L::ROWS + t * QR + 64 * w + 4 * j;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          *reinterpret_cast<float4*>(Q + 16 * i) = make_float4(q[i][0], q[i][1], q[i][2], q[i][3]);
+          *reinterpret_cast<float4*>(K + 16 * i) = make_float4(k[i][0], k[i][1], k[i][2], k[i][3]);
+        }
+        if constexpr (MODE == DELTA) {
+          float sq = 0.f, sk = 0.f;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              sq += q[i][x] * q[i][x];
+              sk += k[i][x] * k[i][x];
+            }
+          sq += dpp_move<0xB1>(sq); sk += dpp_move<0xB1>(sk);
+          sq += dpp_move<0x4E>(sq); sk += dpp_move<0x4E>(sk);
+          float* N = sm + L::NRM + ((c & 3) * NS + w) * 32;
+          if (j == 0) { N[t] = sk; N[16 + t] = sq; }
+        }
+      };
+      if constexpr (L::TURNS) {
+        load(turn, 0);
+        barriers(turn);
+        for (int c = turn; c < chunks; c += 2) {
+          take(c, 0);
+          load(c + 2, 0);
+          __syncthreads();
+          put(c);
+          __syncthreads();
+        }
+        barriers(LEAD - turn);
+      } else {
+        load(0, 0);
+        load(1, 1);
+        for (int c = 0; c < chunks; c += 2) {
+          take(c, 0);
+          load(c + 2, 0);
+          put(c);
+          __syncthreads();
+          take(c + 1, 1);
+          load(c + 3, 1);
+          put(c + 1);
+          __syncthreads();
+        }
+        barriers(LEAD);
       }
     }
-    store(last);
     return;
   }
 
-  // ---- computing waves: state rows 4 g + r of the wave's tiles, column n16
-  f32x4 S[TD];
-  const int col = col0 + n16;
-  const size_t sbase = ((size_t)slot * H + head) * dk;
+  if (wave >= L::SCORES && wave < L::PREP) {
+    // ============================================================================================== scores waves
+    const int turn = wave - L::SCORES;
+    f32x4 pa, ka;                                    // keys s = 4 g + r by queries (delta: also keys) t = n16
+    float bon;
+    auto products = [&](int c) {
+      const float* Q = sm + (L::CH ? L::QT + (c & 1) * L::ROWS : L::Q + (c % L::QB) * L::ROWS);
+      const float* K = sm + L::K + (L::CH ? c & 1 : c % L::KB) * L::ROWS;
+      f32x4 pb = {0.f, 0.f, 0.f, 0.f}, kk = {0.f, 0.f, 0.f, 0.f};
+      pa = pb;
+      ka = pb;
+      bon = 0.f;
 #pragma unroll
-  for (int td = 0; td < TD; ++td)
+      for (int w = 0; w < NS; ++w) {
+        const float* R = sm + L::RAW + ((c & 1) * NS + w) * L::RAWN;
+        if constexpr (L::CH) bon += R[4 + n16];
+        if (L::CH && R[0] != 0.f) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pa[r] += R[20 + (4 * g + r) * C + n16];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int o = n16 * QR + 64 * w + 16 * i + 4 * g;
+            const float4 qf = ld4(Q + o), kf = ld4(K + o);
+            pa = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf.x, pa, 0, 0, 0);
+            pb = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf.y, pb, 0, 0, 0);
+            pa = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf.z, pa, 0, 0, 0);
+            pb = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf.w, pb, 0, 0, 0);
+            if constexpr (MODE == DELTA) {
+              ka = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, kf.x, ka, 0, 0, 0);
+              kk = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, kf.y, kk, 0, 0, 0);
+              ka = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, kf.z, ka, 0, 0, 0);
+              kk = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, kf.w, kk, 0, 0, 0);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pa[r] += pb[r];
+        ka[r] += kk[r];
+      }
+    };
+    auto finish = [&](int c) {
+      float* P = sm + L::P + (c & 3) * C * TR;
+      float p[4];
+      if constexpr (L::CH) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int s = 4 * g + r;
+          p[r] = s < n16 ? pa[r] : (s == n16 ? bon : 0.f);
+        }
+        *reinterpret_cast<float4*>(P + n16 * TR + 4 * g) = make_float4(p[0], p[1], p[2], p[3]);
+      } else {
+        const float* G = sm + L::GT + ((c >> 2) & 1) * 192 + 16 * (c & 3);
+        const float* DM = sm + L::DM + (c & 3) * 272;
+        const float4 wr = ld4(G + 64 + 4 * g), d4 = ld4(DM + 4 * lane);       // write factors of the tokens s
+        const float D[4] = {d4.x, d4.y, d4.z, d4.w}, A = DM[256 + n16];
+        float cf[4] = {wr.x, wr.y, wr.z, wr.w}, qs = 1.f, rk = 1.f;
+        if constexpr (MODE == MLSTM) qs = qscale;
+        if constexpr (MODE == DELTA) {
+          float sk = 0.f, sq = 0.f;
+          float* N = sm + L::NRM + (c & 3) * NS * 32;
+#pragma unroll
+          for (int w = 0; w < NS; ++w) {
+            sk += N[32 * w + n16];
+            sq += N[32 * w + 16 + n16];
+          }
+          rk = 1.f / sqrtf(sk + 1e-6f);              // 1 / |k_t|
+          qs = qscale / sqrtf(sq + 1e-6f);
+          __builtin_amdgcn_wave_barrier();
+          if (g == 0) N[n16] = rk;                   // for the tokens s
+          __builtin_amdgcn_wave_barrier();
+          const float4 x = ld4(N + 4 * g);
+          cf[0] = x.x; cf[1] = x.y; cf[2] = x.z; cf[3] = x.w;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) p[r] = 4 * g + r <= n16 ? pa[r] * qs * cf[r] * D[r] : 0.f;
+        float* S = sm + L::SC + (c & 3) * 96;
+        if (g == 0) S[n16] = A * qs;
+        if (n16 == 15) {                             // delta: the order of u's registers, see below
+          if constexpr (MODE == DELTA) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[16 + 4 * r + g] = D[r] * cf[r];
+          } else {
+            *reinterpret_cast<float4*>(S + 16 + 4 * g) = make_float4(D[0] * cf[0], D[1] * cf[1], D[2] * cf[2], D[3] * cf[3]);
+          }
+          if (g == 0) S[80] = A;
+        }
+        if constexpr (MODE == DELTA) {
+          const float beta = G[128 + n16];
+          const int place = 4 * (n16 & 3) + (n16 >> 2);
+          if (g == 0) { S[32 + place] = beta; S[48 + place] = -beta * A * rk; }
+          // u is held with register b, lane group g' <-> token 4 b + g': columns of P in that order
+#pragma unroll
+          for (int r = 0; r < 4; ++r) P[n16 * TR + 4 * r + g] = p[r];
+          float* T = sm + L::T + (c & 1) * C * TR;
+          float tt[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) tt[r] = 4 * g + r < n16 ? beta * rk * cf[r] * D[r] * ka[r] : 0.f;
+          *reinterpret_cast<float4*>(T + n16 * TR + 4 * g) = make_float4(tt[0], tt[1], tt[2], tt[3]);
+          __builtin_amdgcn_wave_barrier();
+          // M: lane = (row n16, block g): m (I + T_gg) = row of the identity (own block) or - T (blocks below)
+          const float4 row = ld4(T + n16 * TR + 4 * g);
+          const float4 t1 = ld4(T + (4 * g + 1) * TR + 4 * g), t2 = ld4(T + (4 * g + 2) * TR + 4 * g), t3 = ld4(T + (4 * g + 3) * TR + 4 * g);
+          const bool own = (n16 >> 2) == g, below = (n16 >> 2) > g;
+          const int e = n16 & 3;
+          const float e0 = own && e == 0 ? 1.f : 0.f, e1 = own && e == 1 ? 1.f : 0.f, e2 = own && e == 2 ? 1.f : 0.f, e3 = own && e == 3 ? 1.f : 0.f;
+          const float m3 = below ? -row.w : e3;
+          const float m2 = (below ? -row.z : e2) - m3 * t3.z;
+          const float m1 = (below ? -row.y : e1) - m2 * t2.y - m3 * t3.y;
+          const float m0 = (below ? -row.x : e0) - m1 * t1.x - m2 * t2.x - m3 * t3.x;
+          float* M = sm + L::M + (c & 1) * C * TR + (4 * e + (n16 >> 2)) * TR + g;      // row: the register place of token n16
+          M[0] = m0 - e0; M[4] = m1 - e1; M[8] = m2 - e2; M[12] = m3 - e3;
+        } else {
+          *reinterpret_cast<float4*>(P + n16 * TR + 4 * g) = make_float4(p[0], p[1], p[2], p[3]);
+        }
+        if constexpr (MODE == MLSTM) {
+          float rs = (p[0] + p[1]) + (p[2] + p[3]);
+          rs += __shfl_xor(rs, 16, 64);
+          rs += __shfl_xor(rs, 32, 64);
+          if (g == 0) { S[32 + n16] = rs; S[48 + n16] = G[128 + n16]; S[64 + n16] = A * qs; }
+        }
+      }
+    };
+    barriers(LEAD - 1 - L::W2 + turn);
+    for (int c = turn; c < chunks; c += L::W2) {
+      products(c);
+      if constexpr (L::W2 == 2) __syncthreads();
+      finish(c);
+      __syncthreads();
+    }
+    barriers(1 + L::W2 - turn);
+    return;
+  }
+
+  if constexpr (!L::CH) {
+    if (wave == L::GATES) {
+      // ============================================================================================ gates, 64 tokens (one per lane) in four steps
+      float ga = 0.f, gb = 0.f;                      // raw gates of the next 64 tokens
+      float p1 = 0.f, p2 = 0.f;
+      if constexpr (MODE == DELTA || MODE == SSM) { p1 = -expf(a.par1[head]); p2 = a.par2[head]; }
+      if constexpr (MODE == LIGHT) p1 = a.par1[head];
+      float m_run = 0.f, m_old = 0.f, m_new = 0.f, x = 0.f, z = 0.f;       // mlstm: running maximum, input gate, forget gate
+      if constexpr (MODE == MLSTM) {
+        if (stored) m_run = a.mx[(size_t)slot * H + head];
+      }
+      auto load_gates = [&](int b) {
+        const size_t t = row0 + min(b * 64 + lane, n - 1);
+        if constexpr (MODE == DELTA || MODE == MLSTM) {
+          ga = ((const float*)a.aux1)[t * a.aux1_stride + head];
+          gb = ((const float*)a.aux2)[t * a.aux2_stride + head];
+        } else if constexpr (MODE == SSM) {
+          const size_t at = t * a.aux1_stride + head;
+          ga = a.aux_bf16 ? bf16_to_f32(((const uint16_t*)a.aux1)[at]) : ((const float*)a.aux1)[at];
+        }
+      };
+      // phase 0: each token's own; mlstm 1 - 3: the running maximum over a third of the tokens (a serial chain of adds and maxima);
+      // 3: to LDS
+      auto gates = [&](int b, int phase) {
+        if (phase == 0) {
+          if constexpr (MODE == LIGHT) {
+            x = p1;
+          } else if constexpr (MODE == SSM) {
+            x = softplus_f(ga + p2);
+            z = expf(p1 * x);
+          } else if constexpr (MODE == DELTA) {
+            z = expf(p1 * softplus_f(gb + p2));
+            x = 1.f / (1.f + expf(-ga));
+          } else {
+            // tokens past the portion leave the maximum as it is
+            const bool ok = b * 64 + lane < n;
+            x = ok ? a.cap * tanhf(ga / a.cap) : -__builtin_inff();
+            z = ok ? logsigmoid_f(a.cap * tanhf(gb / a.cap)) : 0.f;
+          }
+          load_gates(b + 1);
+        }
+        if constexpr (MODE == MLSTM) {
+          // every lane carries the maximum; each token's goes to LDS (the factors' place of the tokens' gates)
+          float* G = sm + L::GT + (b & 1) * 192;
+          auto run = [&](auto from, auto to) {
+            if (from.value == 0) G[128] = m_run;
+#pragma unroll
+            for (int t = from.value; t < to.value; ++t) {
+              const float f = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, z), t));
+              const float i = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), t));
+              m_run = fmaxf(f + m_run, i);
+              G[t] = m_run;
+            }
+          };
+          if (phase == 1) run(std::integral_constant<int, 0>{}, std::integral_constant<int, 22>{});
+          if (phase == 2) run(std::integral_constant<int, 22>{}, std::integral_constant<int, 43>{});
+          if (phase == 3) {
+            run(std::integral_constant<int, 43>{}, std::integral_constant<int, 64>{});
+            __builtin_amdgcn_wave_barrier();
+            m_new = G[lane];
+            m_old = lane ? G[lane - 1] : G[128];
+            __builtin_amdgcn_wave_barrier();
+          }
+        }
+        if (phase == 3) {
+          // decay | write factor | mlstm: exp(-maximum), delta: write strength; tokens past the portion: no decay, nothing written
+          const bool ok = b * 64 + lane < n;
+          float* G = sm + L::GT + (b & 1) * 192 + lane;
+          G[0] = !ok ? 1.f : (MODE == LIGHT ? x : (MODE == MLSTM ? expf(z + m_old - m_new) : z));
+          G[64] = !ok ? 0.f : (MODE == LIGHT ? 1.f : (MODE == MLSTM ? expf(x - m_new) : x));
+          G[128] = !ok ? 0.f : (MODE == MLSTM ? expf(-m_new) : x);
+        }
+      };
+      // D[t = n16, s = 4 g + r] and A_t of a chunk: one running product down from t
+      auto products = [&](int c) {
+        const float* G = sm + L::GT + ((c >> 2) & 1) * 192 + 16 * (c & 3);
+        float D[4] = {0.f, 0.f, 0.f, 0.f}, A = 1.f;
+#pragma unroll
+        for (int i = 3; i >= 0; --i) {
+          const float4 d4 = ld4(G + 4 * i);
+          const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+          for (int r = 3; r >= 0; --r) {
+            const int u = 4 * i + r;
+            D[r] = i == g ? (u <= n16 ? A : 0.f) : D[r];
+            A *= u <= n16 ? dd[r] : 1.f;
+          }
+        }
+        float* DM = sm + L::DM + (c & 3) * 272;
+        *reinterpret_cast<float4*>(DM + 4 * lane) = make_float4(D[0], D[1], D[2], D[3]);
+        if (g == 0) DM[256 + n16] = A;
+      };
+      load_gates(0);
+      for (int k = 0; k < 4; ++k) gates(0, k);
+      for (int i = 0; i < chunks + LEAD; ++i) {
+        const int c = i - (LEAD - 1 - L::W2);        // as the scores waves count: while they use a batch, the next one is made
+        const int b = (c >> 2) + 1;
+        if (c >= 0 && b * 64 < n) gates(b, c & 3);
+        // read a step later, by the second half of the scores (NT 16: in the next step, with the first)
+        const int ready = L::W2 == 2 ? c : c + 1;
+        if (ready >= 0 && ready < chunks) products(ready);
+        __syncthreads();
+      }
+      if constexpr (MODE == MLSTM) {
+        if (zb == 0 && lane == 0) (a.mx_new ? a.mx_new[(size_t)seq * H + head] : a.mx[(size_t)slot * H + head]) = m_run;
+      }
+      return;
+    }
+  }
+
+  if constexpr (MODE == MLSTM) {
+    if (wave == L::NORM) {
+      // ============================================================================================ normaliser (lane = channel)
+      float nrm[NS];
+      const size_t nb = ((size_t)slot * H + head) * dk;
+#pragma unroll
+      for (int w = 0; w < NS; ++w) nrm[w] = (stored && 64 * w + lane < dk) ? a.norm[nb + 64 * w + lane] : 0.f;
+      barriers(LEAD - 1);
+      for (int c = 0; c < chunks; ++c) {
+        const float* Q = sm + L::Q + (c % L::QB) * L::ROWS;
+        const float* K = sm + L::K + (c % L::KB) * L::ROWS;
+        float* S = sm + L::SC + (c & 3) * 96;
+        float* N = sm + L::NRM;
+#pragma unroll
+        for (int w = 0; w < NS; ++w) N[64 * w + lane] = nrm[w];
+        __builtin_amdgcn_wave_barrier();
+        // normaliser . q_t: the scores' row sums and the chunk's starting normaliser; lane = (token n16, quarter of the channels)
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          const float4 nv = ld4(N + 16 * i + 4 * g), qv = ld4(Q + n16 * QR + 16 * i + 4 * g);
+          dot += nv.x * qv.x + nv.y * qv.y + nv.z * qv.z + nv.w * qv.w;
+        }
+        dot += __shfl_xor(dot, 16, 64);
+        dot += __shfl_xor(dot, 32, 64);
+        const float nq = S[32 + n16] + dot * S[64 + n16];
+        const float inv = 1.f / (fmaxf(fabsf(nq), S[48 + n16]) + 1e-6f);
+        float add[NS] = {};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float4 f4 = ld4(S + 16 + 4 * i);
+          const float f[4] = {f4.x, f4.y, f4.z, f4.w};
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int w = 0; w < NS; ++w) add[w] += f[r] * K[(4 * i + r) * QR + 64 * w + lane];
+        }
+        const float at = S[80];
+#pragma unroll
+        for (int w = 0; w < NS; ++w) nrm[w] = at * nrm[w] + add[w];
+        __builtin_amdgcn_wave_barrier();
+        if (g == 0) S[32 + n16] = inv;
+        __syncthreads();
+      }
+      __syncthreads();
+      if (zb == 0) {
+        float* np = a.norm_new ? a.norm_new + ((size_t)seq * H + head) * dk : a.norm + nb;
+#pragma unroll
+        for (int w = 0; w < NS; ++w)
+          if (64 * w + lane < dk) np[64 * w + lane] = nrm[w];
+      }
+      return;
+    }
+  }
+
+  const bool outputs = wave >= L::OUT;
+  const int cw = outputs ? wave - L::OUT : wave;     // column block of the workgroup
+  const int col = (zb * L::NC + cw) * 16 + n16, colc = min(col, dv - 1);
+  const bool cok = col < dv;
+  const TI* vb = (const TI*)a.v + (size_t)row0 * a.v_stride + (size_t)head * dv;
+  // u's register r: token 4 g + r; delta: 4 r + g
+  auto tok = [&](int r) { return MODE == DELTA ? 4 * r + g : 4 * g + r; };
+  TI rv[2][4];
+  unsigned vv[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) vv[r] = (unsigned)(tok(r) * a.v_stride + colc) * (unsigned)sizeof(TI);
+  auto load_v = [&](int c, int st) {
+    const int first = min(c * C, n - 1);
+    const char* p = (const char*)(vb + (size_t)first * a.v_stride);
+    asm volatile("" : "+s"(p));
+    if (first + C <= n) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rv[st][r] = *reinterpret_cast<const TI*>(p + vv[r]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        rv[st][r] = *reinterpret_cast<const TI*>(p + (unsigned)(min(tok(r), n - 1 - first) * a.v_stride + colc) * (unsigned)sizeof(TI));
+    }
+  };
+  auto take_v = [&](int c, int st, float* u) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = ldf<TI>(&rv[st][r]);
+    if ((c + 1) * C > n) {                           // rows past the portion
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[r] = c * C + tok(r) < n ? u[r] : 0.f;
+    }
+    if constexpr (MODE == LIGHT) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) u[r] = silu(u[r]);
+    }
+    load_v(c + 2, st);
+  };
+  load_v(0, 0);
+  load_v(1, 1);
+
+  if (!outputs) {
+    // ============================================================================================== state waves
+    // state rows (channels) 16 i + 4 g + r, column n16
+    f32x4 S[NT];
+    const size_t sbase = ((size_t)slot * H + head) * dk * dv, wbase = (((size_t)seq * gridDim.y + seg) * H + head) * dk * dv;
+    const float* from = MODE == SSM && a.pass ? a.ws + wbase : a.state + sbase;
+    float* to = MODE == SSM && a.pass == 1 ? a.ws + wbase : a.state + sbase;
+    float all = 1.f;                                 // ssm, pass 1: decay of the segment
+    auto sat = [&](int ch) { return MODE == SSM ? (size_t)colc * dk + ch : (size_t)ch * dv + colc; };
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int ch = 16 * i + 4 * g + r;
+        S[i][r] = (stored && ch < dk && cok) ? from[sat(ch)] : 0.f;
+      }
+    barriers(LEAD - 1);
+    auto step = [&](int c, int st) {
+      const float* K = sm + L::K + (c % L::KB) * L::ROWS;
+      const float* KT = sm + L::KT + ((c % L::KB) * DP + n16) * TR + 4 * g;
+      const float* DE = sm + L::DEC + (c % L::KB) * DP + 4 * g;
+      const float* F = sm + L::SC + (c & 3) * 96;
+      float u[4], x[4];
+      take_v(c, st, u);
+      float* ST = sm + L::ST + ((c & 1) * L::NC + cw) * DP * 16 + 4 * lane;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4*>(ST + 256 * i) = S[i];
+      const float at = L::CH ? 1.f : F[80];
+      if constexpr (MODE == SSM) all *= at;
+      if constexpr (MODE == DELTA) {
+        // x = beta v - beta A S^T k / |k|, rows in the order of u's registers
+        f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = {0.f, 0.f, 0.f, 0.f};
+        const float* Kr = K + (4 * (n16 & 3) + (n16 >> 2)) * QR + 4 * g;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          const float4 kf = ld4(Kr + 16 * i);
+          x0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, S[i][0], x0, 0, 0, 0);
+          x1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, S[i][1], x1, 0, 0, 0);
+          x0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, S[i][2], x0, 0, 0, 0);
+          x1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, S[i][3], x1, 0, 0, 0);
+        }
+        f32x4 X;
+        bool bad = false;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          X[r] = F[32 + 4 * g + r] * u[r] + F[48 + 4 * g + r] * (x0[r] + x1[r]);
+          bad |= !finite(X[r]);
+        }
+        if (__builtin_expect(!__any(bad), 1)) {
+          const float4 mf = ld4(sm + L::M + (c & 1) * C * TR + n16 * TR + 4 * g);
+          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.x, X[0], X, 0, 0, 0);
+          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.y, X[1], X, 0, 0, 0);
+          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.z, X[2], X, 0, 0, 0);
+          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.w, X[3], X, 0, 0, 0);
+        } else {
+          const float* T = sm + L::T + (c & 1) * C * TR;
+#pragma unroll
+          for (int s = 0; s < C; ++s) {
+            const float us = __shfl(X[s >> 2], (s & 3) * 16 + n16, 64);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (4 * r + g > s) X[r] -= T[(4 * r + g) * TR + s] * us;
+          }
+        }
+        *reinterpret_cast<f32x4*>(sm + L::U + ((c & 1) * L::NC + cw) * 256 + 4 * lane) = X;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[r] = X[r];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = L::CH ? u[r] : u[r] * F[16 + 4 * g + r];
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        float kt[4];
+        f32x4 s = S[i];
+        if constexpr (L::CH) {
+          const float4 k4 = ld4(KT + 16 * i * TR), de = ld4(DE + 16 * i);
+          kt[0] = k4.x; kt[1] = k4.y; kt[2] = k4.z; kt[3] = k4.w;
+          s[0] *= de.x; s[1] *= de.y; s[2] *= de.z; s[3] *= de.w;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            kt[r] = K[tok(r) * QR + 16 * i + n16];
+            s[r] *= at;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[r], x[r], s, 0, 0, 0);
+        S[i] = s;
+      }
+      __syncthreads();
+    };
+    for (int c = 0; c < chunks; c += 2) {
+      step(c, 0);
+      step(c + 1, 1);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int ch = 16 * i + 4 * g + r;
+        if (ch < dk && cok && (a.pass != 2 || last)) to[sat(ch)] = S[i][r];
+      }
+    if (MODE == SSM && a.pass == 1 && zb == 0 && wave == 0 && lane == 0) a.wsd[((size_t)seq * gridDim.y + seg) * H + head] = all;
+    return;
+  }
+
+  // ================================================================================================ output waves
+  if (MODE == SSM && a.pass == 1) {
+    barriers(chunks + LEAD);
+    return;
+  }
+  const float skip = MODE == SSM ? a.par3[head] : 0.f;
+  float* yb = a.y + (size_t)row0 * H * dv + (size_t)head * dv;
+  unsigned vy[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) vy[r] = (unsigned)((4 * g + r) * (H * dv) + colc) * 4u;
+  barriers(LEAD);
+  auto step = [&](int c, int st) {
+    const int left = n - c * C;
+    const float* Q = sm + L::Q + (c % L::QB) * L::ROWS + n16 * QR + 4 * g;
+    const float* F = sm + L::SC + (c & 3) * 96 + 4 * g;
+    const float* ST = sm + L::ST + ((c & 1) * L::NC + cw) * DP * 16 + 4 * lane;
+    const float* P = sm + L::P + (c & 3) * C * TR;
+    float u[4];
+    if constexpr (MODE == DELTA) {
+      const float4 u4 = ld4(sm + L::U + ((c & 1) * L::NC + cw) * 256 + 4 * lane);
+      u[0] = u4.x; u[1] = u4.y; u[2] = u4.z; u[3] = u4.w;
+    } else {
+      take_v(c, st, u);
+    }
+    const float4 pf = ld4(P + n16 * TR + 4 * g);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    if (__builtin_expect(!__any(!finite(u[0]) || !finite(u[1]) || !finite(u[2]) || !finite(u[3])), 1)) {
+      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.x, u[0], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.y, u[1], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.z, u[2], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.w, u[3], o, 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int s = 0; s < C; ++s) {
+        const float us = MODE == DELTA ? __shfl(u[s >> 2], (s & 3) * 16 + n16, 64) : __shfl(u[s & 3], (s >> 2) * 16 + n16, 64);
+        const int at = MODE == DELTA ? 4 * (s & 3) + (s >> 2) : s;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * g + r >= s) o[r] += P[(4 * g + r) * TR + at] * us;
+      }
+    }
+    f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const float4 qf = ld4(Q + 16 * i), s = ld4(ST + 256 * i);
+      o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.x, s.x, o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.y, s.y, o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.z, s.z, o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.w, s.w, o1, 0, 0, 0);
+    }
+    float out[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int ch = 16 * (td * 4 + w) + 4 * g + r;
-      S[td][r] = (p0 > 0 && ch < dk && col < dv) ? a.state[(sbase + ch) * dv + col] : 0.f;
+      out[r] = o[r] + (o0[r] + o1[r]) * (L::CH ? 1.f : F[r]);
+      if constexpr (MODE == MLSTM) out[r] *= F[32 + r];
+      if constexpr (MODE == SSM) out[r] += skip * u[r];
     }
-  __syncthreads();
-  for (int ci = 0; ci < chunks; ++ci) {
-    const int b = ci & 1;
-    f32x4 accO = {0.f, 0.f, 0.f, 0.f};
-    f32x4 accA = {0.f, 0.f, 0.f, 0.f};
-    if (Raw(b)[w] == 0.f) {
-      const float4 vf = ld4(VT(b) + n16 * TR + 4 * g);
+    char* yc = (char*)(yb + (size_t)c * C * H * dv);
+    asm volatile("" : "+s"(yc));
+    if (left >= C) {
+      if (cok) {
 #pragma unroll
-      for (int td = 0; td < TD; ++td) {
-        const int ch0 = 16 * (td * 4 + w);
-        const float4 qf = ld4(Qs(b) + n16 * QR + ch0 + 4 * g), kf = ld4(Ks(b) + n16 * QR + ch0 + 4 * g);
-        const float4 kt = ld4(KT(b) + (ch0 + n16) * TR + 4 * g), bc = ld4(Bc(b) + ch0 + 4 * g);
-        f32x4 u = S[td];
-        accA = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.x, kf.x, accA, 0, 0, 0);
-        accO = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.x, u[0], accO, 0, 0, 0);
-        accA = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.y, kf.y, accA, 0, 0, 0);
-        accO = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.y, u[1], accO, 0, 0, 0);
-        accA = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.z, kf.z, accA, 0, 0, 0);
-        accO = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.z, u[2], accO, 0, 0, 0);
-        accA = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.w, kf.w, accA, 0, 0, 0);
-        accO = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.w, u[3], accO, 0, 0, 0);
-        u[0] *= bc.x; u[1] *= bc.y; u[2] *= bc.z; u[3] *= bc.w;
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(kt.x, vf.x, u, 0, 0, 0);
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(kt.y, vf.y, u, 0, 0, 0);
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(kt.z, vf.z, u, 0, 0, 0);
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(kt.w, vf.w, u, 0, 0, 0);
-        S[td] = u;
+        for (int r = 0; r < 4; ++r) *reinterpret_cast<float*>(yc + vy[r]) = out[r];
       }
     } else {
 #pragma unroll
-      for (int t = 0; t < C; ++t) {
-        const float vj = VT(b)[n16 * TR + t];
-        float o = 0.f;
-#pragma unroll
-        for (int td = 0; td < TD; ++td) {
-          const int c4 = 16 * (td * 4 + w) + 4 * g;
-          const float4 qf = ld4(Qs(b) + t * QR + c4), kf = ld4(Ks(b) + t * QR + c4);
-          const float* al = KT(b) + c4 * TR + t;
-          S[td][0] = al[0] * S[td][0] + kf.x * vj;
-          S[td][1] = al[TR] * S[td][1] + kf.y * vj;
-          S[td][2] = al[2 * TR] * S[td][2] + kf.z * vj;
-          S[td][3] = al[3 * TR] * S[td][3] + kf.w * vj;
-          o += S[td][0] * qf.x + S[td][1] * qf.y + S[td][2] * qf.z + S[td][3] * qf.w;
-        }
-        o += __shfl_xor(o, 16, 64);
-        o += __shfl_xor(o, 32, 64);
-        if (g == (t >> 2)) accO[t & 3] = o;
-      }
+      for (int r = 0; r < 4; ++r)
+        if (cok && 4 * g + r < left) *reinterpret_cast<float*>(yc + vy[r]) = out[r];
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) redA[(w * 16 + 4 * g + r) * 17 + n16] = accA[r];
     __syncthreads();
-    // scores of key token 4 w + g for query token n16, all channels; keys up to the query
-    const int s = 4 * w + g;
-    const float* r = redA + n16 * 17 + s;
-    const float p = s <= n16 ? (r[0] + r[16 * 17]) + (r[2 * 16 * 17] + r[3 * 16 * 17]) : 0.f;
-    accO = __builtin_amdgcn_mfma_f32_16x16x4f32(p, VT(b)[n16 * TR + s], accO, 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) redO[w * 256 + (4 * g + i) * 16 + n16] = accO[i];
-    __syncthreads();
+  };
+  for (int c = 0; c < chunks; c += 2) {
+    step(c, 0);
+    step(c + 1, 1);
   }
-#pragma unroll
-  for (int td = 0; td < TD; ++td)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int ch = 16 * (td * 4 + w) + 4 * g + r;
-      if (ch < dk && col < dv) a.state[(sbase + ch) * dv + col] = S[td][r];
-    }
 }
 
-template <bool LIGHT, typename TI, int TD>
+// Between the passes of ssm in segments: per state element, walk a portion's segments in order; the workspace then holds every
+// segment's incoming state.
+__global__ __launch_bounds__(256) void ssm_segments_kernel(float* __restrict__ ws, const float* __restrict__ wsd, const float* __restrict__ state,
+                                                           const int* __restrict__ positions, const int* __restrict__ seq_row0,
+                                                           const int* __restrict__ seq_slots, int H, int per_head, int segs, int seg_rows,
+                                                           int skip_rows) {
+  const int seq = blockIdx.x, head = blockIdx.y, e = blockIdx.z * 256 + threadIdx.x;
+  const int row0 = seq_row0[seq], n = seq_row0[seq + 1] - row0;
+  if (e >= per_head || n <= skip_rows) return;
+  float S = positions[row0] > 0 ? state[((size_t)seq_slots[seq] * H + head) * per_head + e] : 0.f;
+  const int used = (n + seg_rows - 1) / seg_rows;
+  for (int i = 0; i < used; ++i) {
+    float* p = ws + (((size_t)seq * segs + i) * H + head) * per_head + e;
+    const float own = i + 1 < used ? *p : 0.f;
+    *p = S;
+    if (i + 1 < used) S = wsd[((size_t)seq * segs + i) * H + head] * S + own;
+  }
+}
+
+template <int MODE, typename TI, int NT>
 int launch_one(const ChunkArgs& a, dim3 grid, hipStream_t st) {
-  constexpr int DP = 64 * TD;
-  constexpr size_t lds = (size_t)(2 * (2 * C * (DP + 4) + DP * TR + C * TR + DP + 4) + 4 * 16 * 17 + 4 + 4 * 256) * 4;
+  using L = Lay<MODE, NT>;
+  constexpr size_t lds = (size_t)L::END * 4;
   static_assert(lds <= 160 * 1024, "LDS");
-  auto kernel = chunk_scan_kernel<LIGHT, TI, TD>;
+  auto kernel = chunk_scan_kernel<MODE, TI, NT>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
   }
-  kernel<<<grid, 512, lds, st>>>(a);
+  kernel<<<grid, 64 * L::WAVES, lds, st>>>(a);
   return 0;
 }
 
-template <bool LIGHT, typename TI>
+template <int MODE, typename TI>
 int launch_dims(const ChunkArgs& a, dim3 grid, hipStream_t st) {
-  if (a.dk <= 64) return launch_one<LIGHT, TI, 1>(a, grid, st);
-  if (a.dk <= 128) return launch_one<LIGHT, TI, 2>(a, grid, st);
-  return launch_one<LIGHT, TI, 4>(a, grid, st);
+  if (a.dk <= 64) return launch_one<MODE, TI, 4>(a, grid, st);
+  if (a.dk <= 128) return launch_one<MODE, TI, 8>(a, grid, st);
+  if constexpr (MODE != SSM) return -3;
+  else return launch_one<MODE, TI, 16>(a, grid, st);
+}
+
+template <int MODE>
+int launch_mode(const ChunkArgs& a, int in_f32, dim3 grid, hipStream_t st) {
+  return in_f32 ? launch_dims<MODE, float>(a, grid, st) : launch_dims<MODE, uint16_t>(a, grid, st);
 }
 
 }  // namespace
 
-// light: decay [H] and SiLU on q / k / v; else decay [T, H * dk] rows with their stride.  dk at most 256.
-extern "C" int dgi_chunk_scan(float* y, int light, const void* q, int q_stride, const void* k, int k_stride, const void* v,
-                              int v_stride, int in_f32, const float* decay, int decay_stride, float* state,
-                              const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int H, int dk, int dv,
-                              hipStream_t st) {
+// Whether prompt portions of these shapes run here: key sizes of at most 128 (ssm: 256), and, but for wkv,
+// rows of q and k that can be read four elements at a time.
+extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32) {
+  if (mode == 3 || dk <= 0 || dk > (mode == SSM ? 256 : 128)) return 0;
+  if (mode == WKV) return 1;
+  const int piece = in_f32 ? 15 : 7;               // bytes of four elements, less one
+  return dk % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && (((uintptr_t)q | (uintptr_t)k) & piece) == 0;
+}
+
+// mode as above (light: par1 the decays; ssm: q = C, k = B, v = x, aux1 = dt_raw (aux_bf16), par1 a_log, par2 dt_bias, par3 d_skip).
+// Needs dgi_chunk_scan_ok.  skip_rows: sequences of at most that many rows are left to another launch.  segs > 1 (ssm): portions are
+// cut into segments of seg_rows rows (a multiple of 16, segs of them at least as long as the longest portion) that run side by side: each one's
+// state from nothing, a short serial pass over those states, then the outputs from each segment's incoming state.  About
+// twice the work, for steps whose heads leave most of the chip idle.
+extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
+                              int v_stride, int in_f32, const void* aux1, int aux1_stride, const void* aux2, int aux2_stride,
+                              int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
+                              float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
+                              const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
+                              int segs, int seg_rows, float* ws, float* wsd, hipStream_t st) {
   if (n_seq == 0) return 0;
-  if (dk <= 0 || dk > 256 || dv <= 0 || H <= 0 || H > 65535 || (dv + 15) / 16 > 65535 || !decay) return -3;
+  const int cols = dk <= 128 ? 32 : 16;            // value columns of a workgroup
+  const long long nz = (dv + cols - 1) / cols;
+  if (!dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32) || dv <= 0 || H <= 0 || G <= 0 || H % G) return -3;
+  if (mode == MLSTM && nz > 1 && (!norm_new || !mx_new)) return -7;
   ChunkArgs a;
   a.y = y; a.q = q; a.k = k; a.v = v;
   a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride;
-  a.decay = decay; a.decay_stride = decay_stride; a.state = state;
+  a.aux1 = aux1; a.aux2 = aux2; a.aux1_stride = aux1_stride; a.aux2_stride = aux2_stride; a.aux_bf16 = aux_bf16;
+  a.par1 = par1; a.par2 = par2; a.par3 = par3; a.cap = cap;
+  a.state = state; a.norm = norm; a.mx = mx; a.norm_new = norm_new; a.mx_new = mx_new;
   a.positions = positions; a.seq_row0 = seq_row0; a.seq_slots = seq_slots;
-  a.H = H; a.dk = dk; a.dv = dv;
-  const dim3 grid(n_seq, H, (dv + 15) / 16);
-  int rc;
-  if (light) rc = in_f32 ? launch_dims<true, float>(a, grid, st) : launch_dims<true, uint16_t>(a, grid, st);
-  else rc = in_f32 ? launch_dims<false, float>(a, grid, st) : launch_dims<false, uint16_t>(a, grid, st);
+  a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.skip_rows = skip_rows;
+  if (n_seq * nz * H > 0x3fffffff || segs > 65535 || (segs > 1 && (mode != SSM || !ws || !wsd || seg_rows <= 0))) return -3;
+  a.n_seq = n_seq; a.seg_rows = seg_rows; a.ws = ws; a.wsd = wsd;
+  a.pass = segs > 1 ? 1 : 0;
+  const dim3 grid((unsigned)(n_seq * nz * H), segs > 1 ? segs : 1);
+  if (a.pass) {
+    int rc = launch_dims<SSM, float>(a, grid, st);
+    if (rc) return rc;
+    ssm_segments_kernel<<<dim3(n_seq, H, (dk * dv + 255) / 256), 256, 0, st>>>(ws, wsd, state, positions, seq_row0, seq_slots, H, dk * dv, segs,
+                                                                               seg_rows, skip_rows);
+    a.pass = 2;
+  }
+  int rc = -2;
+  switch (mode) {
+    case WKV: rc = launch_mode<WKV>(a, in_f32, grid, st); break;
+    case DELTA: rc = launch_mode<DELTA>(a, in_f32, grid, st); break;
+    case MLSTM: rc = launch_mode<MLSTM>(a, in_f32, grid, st); break;
+    case LIGHT: rc = launch_mode<LIGHT>(a, in_f32, grid, st); break;
+    case SSM: rc = in_f32 ? launch_dims<SSM, float>(a, grid, st) : -2; break;
+  }
   if (rc) return rc;
   DGI_CHECK_LAUNCH();
   return 0;

@@ -28,7 +28,8 @@
 // running maximum is a serial pass of one thread (adds and maxima; its exponentials are parallel again).
 // The token loop reads LDS only.  Everything is fp32; q / k / v arrive as bf16 or fp32.
 // A portion that starts at position 0 reads no state; the state is written back at the end of the portion.
-// Prompt portions of gla and light run in chunks of sixteen tokens on the matrix cores instead (chunk_scan.hip).
+// Prompt portions run in chunks of sixteen tokens on the matrix cores instead (chunk_scan.hip): what is left here are steps of
+// single rows and short portions, key sizes above 128 (gla, light: 256), and rows of delta and mlstm that cannot be read in fours.
 #include "../common.h"
 
 using namespace dgi;
@@ -60,6 +61,7 @@ struct ScanArgs {
   int H, G, dk, dv;
   int KS, CW, nwc, CB;           // key slices per wave, columns per wave, computing waves, columns per workgroup
   float cap;
+  int most;                      // sequences of more rows are another launch's (0: all sequences)
 };
 
 // Sums inside the vector ALU (data-parallel-primitive moves) instead of __shfl_xor, which goes through the LDS permute
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(256) void linear_scan_kernel(const ScanArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int seq = blockIdx.x, head = blockIdx.y, cblk = blockIdx.z;
   const int row0 = a.seq_row0[seq], n = a.seq_row0[seq + 1] - row0;
-  if (n <= 0) return;
+  if (n <= 0 || (a.most > 0 && n > a.most)) return;
   const int p0 = a.positions[row0], slot = a.seq_slots[seq];
   const int dk = a.dk, dv = a.dv, H = a.H;
   const int kvh = head / (H / a.G);
@@ -851,6 +853,15 @@ static int scan_columns(int KS, int dv) {
   return nwc * CW;
 }
 
+static int compute_units() {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
+    return n > 0 ? n : 256;
+  }();
+  return cus;
+}
+
 // Key channels per thread.  A decode-shaped step streams the states: 16 channels per thread, all columns of a head in
 // one workgroup.  A prompt portion is a dependent chain per (sequence, head, column) whose length per token grows with
 // the channels a thread holds, so while the grid stays within two workgroups per compute unit a head is spread over
@@ -859,11 +870,7 @@ static int scan_columns(int KS, int dv) {
 static int scan_channels(int dk, int dv, int H, int n_seq, int rows) {
   if (dk > 256) return 32;
   if (rows <= 4 * n_seq) return 16;
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
-    return n > 0 ? n : 256;
-  }();
+  const int cus = compute_units();
   for (int R = 4; R <= 8; R *= 2) {
     int KS = 1;
     while (KS * R < dk) KS <<= 1;
@@ -875,12 +882,53 @@ static int scan_channels(int dk, int dv, int H, int n_seq, int rows) {
   return 16;
 }
 
-extern "C" int dgi_chunk_scan(float* y, int light, const void* q, int q_stride, const void* k, int k_stride, const void* v,
-                              int v_stride, int in_f32, const float* decay, int decay_stride, float* state,
-                              const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int H, int dk, int dv,
-                              hipStream_t st);
+extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
+                              int v_stride, int in_f32, const void* aux1, int aux1_stride, const void* aux2, int aux2_stride,
+                              int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
+                              float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
+                              const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
+                              int segs, int seg_rows, float* ws, float* wsd, hipStream_t st);
+extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
+extern "C" int dgi_chunk_scan_decay(float* y, int light, const void* q, int q_stride, const void* k, int k_stride, const void* v,
+                                   int v_stride, int in_f32, const float* decay, int decay_stride, float* state,
+                                   const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int H, int dk, int dv,
+                                   int skip_rows, hipStream_t st);
+
+constexpr int SHORT = 16;            // rows up to which a sequence stays with this file's kernel beside a chunked launch (one chunk)
+constexpr int APART_FROM = 8;        // sequences of a step above which those are looked for
+
+// The kernel of a step's prompt portions: 0 this file's (no portions, or shapes the others do not take), 1 chunk_scan.hip, 2 chunk_scan_decay.hip.
+// chunk_scan.hip takes a third to a quarter of this file's time per row, but the time of some 80 rows more per portion (its pipeline fills) and
+// a second launch beside decode rows (measured, 32 heads: 4 of 5 steps with portions of 46 rows and less are slower there).  Known here are
+// the step's rows and sequences: on average more than 64 rows a sequence, or 256 rows more than sequences.
+// gla and light have chunk_scan_decay.hip too, with little to fill: better than this file's kernel from some four rows a sequence on, or 128 rows
+// beside decode rows.  light leaves it for chunk_scan.hip where its workgroups (16 columns) outnumber the compute units (2 prompts
+// of 4096 rows in all, 64 heads of 64: 214 against 167 us; 2 prompts of 462 rows, 32 heads: 21 against 24).
+static int chunk_form(int mode, int dk, int dv, int G, int H, const void* q, int q_stride, const void* k, int k_stride, int in_f32, int n_seq,
+                      int rows) {
+  const bool portions = rows > 64 * n_seq || rows - n_seq >= 256;
+  const bool ok = portions && dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32);
+  if ((mode == GLA || mode == LIGHT) && dk <= 256 && G == H) {
+    if (ok && rows > 64 * n_seq && (long)n_seq * H * ((dv + 15) / 16) > compute_units()) return 1;
+    return rows > 4 * n_seq || rows - n_seq >= 128 ? 2 : 0;
+  }
+  return ok;
+}
+
+// whether the matrix memory of a step has several workgroups per head in one of its launches: its normaliser and maximum are staged
+extern "C" int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
+                                      int in_f32) {
+  const bool chunked = chunk_form(MLSTM, dk, dv, H, H, q, q_stride, k, k_stride, in_f32, n_seq, rows) != 0;
+  if (chunked && dv > 32) return 1;
+  if (chunked && n_seq <= APART_FROM) return 0;
+  const int R = scan_channels(dk, dv, H, n_seq, chunked ? n_seq : rows);
+  int KS = 1;
+  while (KS * R < dk) KS <<= 1;
+  return KS <= 16 && scan_columns(KS, dv) < dv;
+}
 
 // mode 0 wkv, 1 delta, 2 mlstm, 3 gla, 4 light; q / k / v bf16 or fp32 (in_f32) with row strides in elements; rows: rows of the step.
+// norm_new / mx_new: mlstm's staged normaliser / maximum (needed where a head spans several workgroups).
 extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                                int v_stride, int in_f32, const float* aux1, int aux1_stride, const float* aux2,
                                int aux2_stride, const float* par1, const float* par2, float* state, float* norm, float* mx,
@@ -893,57 +941,60 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   if (mode == WKV && (!par1 || !par2)) return -4;
   if (mode == DELTA && (!par1 || !par2 || !aux2)) return -4;
   if ((mode == LIGHT && !par1) || (mode != LIGHT && !aux1)) return -4;
-  const bool short_rows = rows <= 4 * n_seq;       // rows of the step: at most four per sequence on average
-  // prompt portions of the decayed recurrences: sixteen tokens at a time on the matrix cores (chunk_scan.hip)
-  if ((mode == GLA || mode == LIGHT) && dk <= 256 && G == H && (!short_rows || rows - n_seq >= 32))
-    return dgi_chunk_scan(y, mode == LIGHT, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? par1 : aux1,
-                          mode == LIGHT ? 0 : aux1_stride, state, positions, seq_row0, seq_slots, n_seq, H, dk, dv, st);
-  const int R = scan_channels(dk, dv, H, n_seq, rows);
-  int KS = 1;
-  while (KS * R < dk) KS <<= 1;
-  if (KS > 16) return -5;
-  ScanArgs a;
-  a.y = y; a.q = q; a.k = k; a.v = v;
-  a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride;
-  a.aux1 = aux1; a.aux2 = aux2; a.aux1_stride = aux1_stride; a.aux2_stride = aux2_stride;
-  a.par1 = par1; a.par2 = par2; a.state = state; a.norm = norm; a.mx = mx;
-  a.positions = positions; a.seq_row0 = seq_row0; a.seq_slots = seq_slots;
-  a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.cap = cap;
-  a.KS = KS; a.CW = 64 / KS;
-  a.CB = scan_columns(KS, dv);
-  a.nwc = a.CB / a.CW;
-  const int nz = (dv + a.CB - 1) / a.CB;
-  if (H > 65535 || nz > 65535) return -5;
-  const bool staged = mode == MLSTM && nz > 1;
-  if (staged && (!norm_new || !mx_new)) return -7;
-  a.norm_new = staged ? norm_new : nullptr;
-  a.mx_new = staged ? mx_new : nullptr;
-  const dim3 grid(n_seq, H, nz);
-  int rc;
+  bool short_rows = rows <= 4 * n_seq;             // rows of the step: at most four per sequence on average
+  const bool staged = mode == MLSTM && norm_new && mx_new;
+  // Prompt portions: sixteen tokens at a time on the matrix cores (chunk_scan.hip).  Among many sequences there are decode
+  // rows beside the portions: those of at most SHORT rows stay with this kernel, in a launch of their own.
+  const int form = chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows);
+  const int apart = n_seq > APART_FROM && (form == 1 || (form == 2 && rows <= 4 * n_seq)) ? SHORT : 0;
+  if (form) {
+    const int rc = form == 1 ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
+                                              aux2, aux2_stride, 0, par1, par2, nullptr, cap, state, norm, mx, norm_new, mx_new, positions,
+                                              seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, 0, nullptr, nullptr, st)
+                             : dgi_chunk_scan_decay(y, mode == LIGHT, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? par1 : aux1,
+                                                   mode == LIGHT ? 0 : aux1_stride, state, positions, seq_row0, seq_slots, n_seq, H, dk, dv,
+                                                   apart, st);
+    if (rc) return rc;
+    short_rows = true;
+  }
+  if (!form || apart) {
+    const int R = short_rows ? scan_channels(dk, dv, H, n_seq, n_seq) : scan_channels(dk, dv, H, n_seq, rows);
+    int KS = 1;
+    while (KS * R < dk) KS <<= 1;
+    if (KS > 16) return -5;
+    ScanArgs a;
+    a.y = y; a.q = q; a.k = k; a.v = v;
+    a.q_stride = q_stride; a.k_stride = k_stride; a.v_stride = v_stride;
+    a.aux1 = aux1; a.aux2 = aux2; a.aux1_stride = aux1_stride; a.aux2_stride = aux2_stride;
+    a.par1 = par1; a.par2 = par2; a.state = state; a.norm = norm; a.mx = mx;
+    a.positions = positions; a.seq_row0 = seq_row0; a.seq_slots = seq_slots;
+    a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.cap = cap; a.most = apart;
+    a.KS = KS; a.CW = 64 / KS;
+    a.CB = scan_columns(KS, dv);
+    a.nwc = a.CB / a.CW;
+    const int nz = (dv + a.CB - 1) / a.CB;
+    if (H > 65535 || nz > 65535) return -5;
+    if (mode == MLSTM && nz > 1 && !staged) return -7;
+    a.norm_new = staged ? norm_new : nullptr;
+    a.mx_new = staged ? mx_new : nullptr;
+    const dim3 grid(n_seq, H, nz);
+    int rc;
 #define DGI_SCAN(M_)                                                                                      \
-  rc = in_f32 ? launch_scan<M_, float>(a, R, short_rows, grid, st) : launch_scan<M_, uint16_t>(a, R, short_rows, grid, st)
-  if (mode == WKV) DGI_SCAN(WKV);
-  else if (mode == DELTA) DGI_SCAN(DELTA);
-  else if (mode == MLSTM) DGI_SCAN(MLSTM);
-  else if (mode == GLA) DGI_SCAN(GLA);
-  else DGI_SCAN(LIGHT);
+    rc = in_f32 ? launch_scan<M_, float>(a, R, short_rows, grid, st) : launch_scan<M_, uint16_t>(a, R, short_rows, grid, st)
+    if (mode == WKV) DGI_SCAN(WKV);
+    else if (mode == DELTA) DGI_SCAN(DELTA);
+    else if (mode == MLSTM) DGI_SCAN(MLSTM);
+    else if (mode == GLA) DGI_SCAN(GLA);
+    else DGI_SCAN(LIGHT);
 #undef DGI_SCAN
-  if (rc) return rc;
-  DGI_CHECK_LAUNCH();
+    if (rc) return rc;
+    DGI_CHECK_LAUNCH();
+  }
   if (staged) {
     mlstm_commit_kernel<<<n_seq, 256, 0, st>>>(norm, mx, norm_new, mx_new, seq_row0, seq_slots, H, dk);
     DGI_CHECK_LAUNCH();
   }
   return 0;
-}
-
-// value columns one workgroup covers in this step (the matrix memory stages its normaliser when dv exceeds it)
-extern "C" int dgi_linear_scan_columns(int dk, int dv, int H, int n_seq, int rows) {
-  const int R = scan_channels(dk, dv, H, n_seq, rows);
-  int KS = 1;
-  while (KS * R < dk) KS <<= 1;
-  if (KS > 16) return 0;
-  return scan_columns(KS, dv);
 }
 
 extern "C" int dgi_token_shift(void* out, int out_f32, const void* h, int h_f32, int h_stride, const float* mu, int nmix,

@@ -8,8 +8,7 @@
 //     y_t = S^T C_t + d_skip[h] * x_t
 //
 // S starts as state[slot][h] (stored transposed, [dv][N]; zero when the portion starts at position 0) and goes back there after
-// the last row; decode rows (one token) and prompt portions run the same code, so the result does
-// not depend on how a prompt was cut.  x | B | C come as one fp32 row (the convolution's output).
+// the last row.  This kernel takes decode rows and short portions, long ones go through chunk_scan.hip.  x | B | C come as one fp32 row (the convolution's output).
 //
 // Work split: a workgroup owns (sequence, head, 16 value columns); thread (column v, n-lane l) keeps
 // S[n][v] for n = 4 l + 64 q + j in registers, so the y reduction over n is four DPP rotate-adds inside a
@@ -58,8 +57,7 @@ __global__ __launch_bounds__(COLS * NL) void ssm_scan_kernel(
     float* __restrict__ y, const float* __restrict__ xbc, int xbc_stride, const TD* __restrict__ dt_raw, int dt_stride,
     const float* __restrict__ dt_bias, const float* __restrict__ a_log, const float* __restrict__ d_skip,
     float* __restrict__ state, const int* __restrict__ positions, const int* __restrict__ seq_row0,
-    const int* __restrict__ seq_slots, int heads, int dv, int N, int G, int mode, int L, int nchunks,
-    float* __restrict__ ws, float* __restrict__ wsd) {
+    const int* __restrict__ seq_slots, int heads, int dv, int N, int G, int most) {
   constexpr int NP = 64 * NQ;
   constexpr int PB = (TT * NP) / (COLS * NL);          // B (and C) values a thread stages per tile
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -68,26 +66,19 @@ __global__ __launch_bounds__(COLS * NL) void ssm_scan_kernel(
   float* sX = sC + TT * NP;
   float* sDt = sX + TT * COLS;
   float* sDa = sDt + TT;
-  // mode 0: a workgroup runs a sequence's whole portion from its state slot and back.  Modes 1 and 3
-  // run one chunk of L rows (blockIdx.x = sequence * nchunks + chunk): 1 from a zero state into the
-  // workspace (no outputs; also the chunk's summed log decay), 3 from the workspace state into y.
-  const int seq = mode ? blockIdx.x / nchunks : blockIdx.x, h = blockIdx.y;
-  const int chunk = mode ? blockIdx.x - seq * nchunks : 0;
+  const int seq = blockIdx.x, h = blockIdx.y;
   const int tid = threadIdx.x;
   const int l = tid & (NL - 1), col = tid >> 4;
   const int v = blockIdx.z * COLS + col;
-  const int s0 = seq_row0[seq], s1 = seq_row0[seq + 1];
-  const int r0 = s0 + chunk * L, r1 = mode ? min(s1, r0 + L) : s1;
-  if (r1 <= r0) return;
+  const int r0 = seq_row0[seq], r1 = seq_row0[seq + 1];
+  if (r1 <= r0 || (most > 0 && r1 - r0 > most)) return;          // longer portions: chunk_scan.hip, in a launch of its own
   const bool vok = v < dv;
   const int g = h / (heads / G);
   const int inner = heads * dv;
   const float* bp = xbc + inner + (size_t)g * N;
   const float* cp = bp + (size_t)G * N;
-  float* sp = mode ? ws + (((size_t)blockIdx.x * heads + h) * dv + v) * N
-                   : state + (((size_t)seq_slots[seq] * heads + h) * dv + v) * N;     // [..][head][v][n]
-  const bool fresh = mode == 1 || (mode == 0 && positions[s0] == 0);
-  float ldec = 0.f;                                    // mode 1: sum of log decays (threads < TT)
+  float* sp = state + (((size_t)seq_slots[seq] * heads + h) * dv + v) * N;     // [..][head][v][n]
+  const bool fresh = positions[r0] == 0;
   float S[NQ][4];
 #pragma unroll
   for (int q = 0; q < NQ; ++q)
@@ -129,7 +120,6 @@ __global__ __launch_bounds__(COLS * NL) void ssm_scan_kernel(
       const float dt = fmaxf(z, 0.f) + log1pf(expf(-fabsf(z)));
       sDt[tid] = dt;
       sDa[tid] = expf(na * dt);
-      if (t0 + tid < r1) ldec += na * dt;
     }
     __syncthreads();
     if (t0 + TT < r1) prefetch(t0 + TT);                 // in flight while this tile is consumed
@@ -148,18 +138,11 @@ __global__ __launch_bounds__(COLS * NL) void ssm_scan_kernel(
         S[q][3] = a * S[q][3] + b4.w * dx;
         acc += S[q][0] * c4.x + S[q][1] * c4.y + S[q][2] * c4.z + S[q][3] * c4.w;
       }
-      if (mode != 1) {                                   // mode 1: chunk states only, no outputs
-        acc = row16_sum(acc);
-        if (l == 0 && vok) y[(size_t)(t0 + k) * inner + (size_t)h * dv + v] = acc + dsk * xv;
-      }
+      acc = row16_sum(acc);
+      if (l == 0 && vok) y[(size_t)(t0 + k) * inner + (size_t)h * dv + v] = acc + dsk * xv;
     }
   }
-  if (mode == 1 && blockIdx.z == 0 && tid < TT) {      // TT lanes of wave 0
-#pragma unroll
-    for (int o = TT / 2; o > 0; o >>= 1) ldec += __shfl_xor(ldec, o, 64);
-    if (tid == 0) wsd[(size_t)blockIdx.x * heads + h] = ldec;
-  }
-  if (vok && mode != 3) {
+  if (vok) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
 #pragma unroll
@@ -168,29 +151,6 @@ __global__ __launch_bounds__(COLS * NL) void ssm_scan_kernel(
         if (n < N) sp[n] = S[q][j];
       }
   }
-}
-
-// Between the two chunk passes: per (sequence, head, state element) walk the chunks in order,
-// S_in[c] <- S;  S <- exp(logdecay[c]) * S + S_local[c], starting from the state slot (zero at
-// position 0); the workspace then holds every chunk's incoming state and the slot the final one.
-__global__ __launch_bounds__(256) void ssm_chunk_states_kernel(
-    float* __restrict__ ws, const float* __restrict__ wsd, float* __restrict__ state, const int* __restrict__ positions,
-    const int* __restrict__ seq_row0, const int* __restrict__ seq_slots, int heads, int per_head, int L, int nchunks) {
-  const int seq = blockIdx.x, h = blockIdx.y;
-  const int e = blockIdx.z * 256 + threadIdx.x;
-  if (e >= per_head) return;
-  const int s0 = seq_row0[seq], n = seq_row0[seq + 1] - s0;
-  if (n <= 0) return;
-  float* sp = state + ((size_t)seq_slots[seq] * heads + h) * per_head + e;
-  float S = positions[s0] == 0 ? 0.f : *sp;
-  const int nc = (n + L - 1) / L;
-  for (int c = 0; c < nc; ++c) {
-    float* wp = ws + (((size_t)seq * nchunks + c) * heads + h) * per_head + e;
-    const float loc = *wp;
-    *wp = S;
-    S = expf(wsd[((size_t)seq * nchunks + c) * heads + h]) * S + loc;
-  }
-  *sp = S;
 }
 
 template <typename TZ, typename TO>
@@ -283,46 +243,65 @@ __global__ __launch_bounds__(256) void gated_group_norm_reg_kernel(
 
 }  // namespace
 
-// ws / wsd: workspace for the chunked form ([n_seq * nchunks][heads][dv][N] states and [n_seq * nchunks][heads]
-// log decays) or null: one pass, sequence by sequence.  The chunked form splits every portion into chunks
-// of L rows that run in parallel (local states from zero, a short serial pass over the chunk states, then
-// the outputs from each chunk's incoming state): twice the recurrence work, nchunks times the workgroups.
-// It reassociates the fp32 sums, so fp32 models keep the one-pass form.
+extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
+                              int v_stride, int in_f32, const void* aux1, int aux1_stride, const void* aux2, int aux2_stride,
+                              int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
+                              float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
+                              const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
+                              int segs, int seg_rows, float* ws, float* wsd, hipStream_t st);
+
+extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
+
+// chunked: portions go sixteen tokens at a time through the matrix cores (chunk_scan.hip, where the shapes allow it).  Its workgroups have a
+// compute unit to themselves and a pipeline to fill, so among more than APART_FROM sequences those of at most SHORT rows stay with this
+// file's kernel (12 portions of 39 rows, 32 heads: 31 us against 51 there).
+constexpr int SHORT = 48, APART_FROM = 8;
+
+// Segments (of *seg_rows rows) that a chunked step's portions are cut into (1: whole portions).  rows - n_seq + 1 bounds the longest portion.
+// Two passes over a segment take 2 (seg_rows / 16 + 5) chunks' time and the state pass some 10 us, one over a whole portion
+// rows / 16 + 5: worth it from about 512 rows on while the workgroups (32 columns of a head) leave half of the chip idle (1444 rows, 16 heads of
+// 48 columns, state 128: see chunk_scan.hip).
+extern "C" int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg_rows) {
+  const long groups = (long)n_seq * heads * ((dv + 31) / 32);
+  const int longest = rows - n_seq + 1;
+  *seg_rows = 0;
+  if (groups <= 0 || groups > 128 || longest < 512) return 1;
+  const long fit = 384 / groups, most = longest / 128;
+  const int segs = (int)(fit < most ? fit : most);
+  if (segs < 3) return 1;
+  *seg_rows = (longest / segs + 15) / 16 * 16;
+  return (longest + *seg_rows - 1) / *seg_rows;
+}
+
 extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const void* dt_raw, int dt_f32, int dt_stride,
                             const float* dt_bias, const float* a_log, const float* d_skip, float* state,
                             const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int heads,
-                            int dv, int N, int G, float* ws, float* wsd, int L, int nchunks, hipStream_t s) {
+                            int dv, int N, int G, int chunked, int segs, int seg_rows, float* ws, float* wsd, hipStream_t s) {
   if (n_seq == 0) return 0;
   if (G <= 0 || heads % G) return -2;
   if (N > 256 || N <= 0 || dv <= 0) return -3;
-  if (ws && (L < 1 || nchunks < 1 || !wsd)) return -5;
   if (heads > 65535 || (dv + COLS - 1) / COLS > 65535) return -4;
+  int most = 0;
+  const float* B = xbc + (size_t)heads * dv;
+  if (chunked && dgi_chunk_scan_ok(5, N, B + (size_t)G * N, xbc_stride, B, xbc_stride, 1)) {
+    most = n_seq > APART_FROM ? SHORT : 0;
+    const int rc = dgi_chunk_scan(y, 5, B + (size_t)G * N, xbc_stride, B, xbc_stride, xbc, xbc_stride, 1, dt_raw, dt_stride, nullptr, 0,
+                                  !dt_f32, a_log, dt_bias, d_skip, 0.f, state, nullptr, nullptr, nullptr, nullptr, positions, seq_row0,
+                                  seq_slots, n_seq, heads, G, N, dv, most, segs, seg_rows, ws, wsd, s);
+    if (rc || !most) return rc;
+  }
   const int nq = (N + 63) / 64;
-  auto launch = [&](int mode) {
-    const dim3 grid(mode ? n_seq * nchunks : n_seq, heads, (dv + COLS - 1) / COLS);
-#define DGI_SCAN(TD, NQ)                                                                                                \
+  const dim3 grid(n_seq, heads, (dv + COLS - 1) / COLS);
+#define DGI_SCAN(TD, NQ)                                                                                              \
   ssm_scan_kernel<TD, NQ><<<grid, COLS * NL, (size_t)(2 * TT * 64 * NQ + TT * COLS + 2 * TT) * 4, s>>>(             \
       y, xbc, xbc_stride, (const TD*)dt_raw, dt_stride, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, \
-      heads, dv, N, G, mode, L, nchunks, ws, wsd)
-    if (dt_f32) {
-      if (nq <= 1) DGI_SCAN(float, 1); else if (nq <= 2) DGI_SCAN(float, 2); else DGI_SCAN(float, 4);
-    } else {
-      if (nq <= 1) DGI_SCAN(uint16_t, 1); else if (nq <= 2) DGI_SCAN(uint16_t, 2); else DGI_SCAN(uint16_t, 4);
-    }
-#undef DGI_SCAN
-  };
-  if (!ws) {
-    launch(0);
-    DGI_CHECK_LAUNCH();
-    return 0;
+      heads, dv, N, G, most)
+  if (dt_f32) {
+    if (nq <= 1) DGI_SCAN(float, 1); else if (nq <= 2) DGI_SCAN(float, 2); else DGI_SCAN(float, 4);
+  } else {
+    if (nq <= 1) DGI_SCAN(uint16_t, 1); else if (nq <= 2) DGI_SCAN(uint16_t, 2); else DGI_SCAN(uint16_t, 4);
   }
-  launch(1);
-  DGI_CHECK_LAUNCH();
-  const int per_head = dv * N;
-  ssm_chunk_states_kernel<<<dim3(n_seq, heads, (per_head + 255) / 256), 256, 0, s>>>(ws, wsd, state, positions, seq_row0,
-                                                                                      seq_slots, heads, per_head, L, nchunks);
-  DGI_CHECK_LAUNCH();
-  launch(3);
+#undef DGI_SCAN
   DGI_CHECK_LAUNCH();
   return 0;
 }

@@ -177,9 +177,7 @@ def ssm_scan_ref(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0
     return y.reshape(T, inner)
 
 
-SCAN_CHUNK = int(os.environ.get("DGI_SCAN_CHUNK", "128"))       # rows per chunk of the chunked scan (0: off)
-SCAN_WS_BYTES = 512 << 20                                      # largest chunk-state workspace
-SCAN_CHUNK_BELOW = int(os.environ.get("DGI_SCAN_CHUNK_BELOW", "512"))   # one-pass workgroups below which steps are chunked
+SCAN_CHUNK = int(os.environ.get("DGI_SCAN_CHUNK", "16"))       # 0: portions row by row unless a call asks for chunks
 
 
 def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads: int, dv: int,
@@ -190,28 +188,16 @@ def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, se
     S [N, dv] in fp32 read from / written to ``state`` [slots, heads, dv, N] (value-major; zero at position 0).
     Returns y [T, heads*dv] fp32.
 
-    On the GPU a step with long portions of few sequences runs in chunks of ``SCAN_CHUNK`` rows in
-    parallel (local chunk states, a serial pass over them, outputs from each chunk's incoming state)
-    when the model is bf16 (``chunked`` None) — the same recurrence with its fp32 sums reassociated;
-    fp32 models, short steps and steps with enough sequences to fill the chip run each sequence in one pass."""
+    On the GPU a step with prompt portions takes them sixteen rows at a time on the matrix cores — the same recurrence
+    with its fp32 sums reassociated; steps of single rows, and every step with ``chunked`` False, go row by row."""
     if _native(xbc):
         T, n_seq = xbc.shape[0], seq_slots.shape[0]
         y = torch.empty(T, heads * dv, dtype=torch.float32, device=xbc.device)
-        longest = T - n_seq + 1                       # no portion is longer (every sequence has a row)
-        L = SCAN_CHUNK
         if chunked is None:
-            # worth twice the recurrence work only while one-pass workgroups (sequence x head x 16 columns)
-            # cannot fill the chip: measured slower than one pass from 512 workgroups on
-            chunked = dt_raw.dtype != torch.float32 and n_seq * heads * -(-dv // 16) < SCAN_CHUNK_BELOW
-        if chunked and L > 0 and longest >= 4 * L:
-            nch = -(-longest // L)
-            if n_seq * nch * heads * dv * N * 4 <= SCAN_WS_BYTES:
-                ws = torch.empty(n_seq * nch * heads * dv * N, dtype=torch.float32, device=xbc.device)
-                wsd = torch.empty(n_seq * nch * heads, dtype=torch.float32, device=xbc.device)
-                _call("ssm_scan", y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots,
-                      heads, dv, N, G, ws, wsd, L, nch)
-                return y
-        _call("ssm_scan", y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G)
+            # a third of the time per row, but some 80 rows' time more per portion and a second launch beside decode rows (12
+            # portions of 39 rows, 32 heads: 51 us against 32 row by row); known here are the step's rows and sequences only
+            chunked = SCAN_CHUNK > 0 and (T > 64 * n_seq or T - n_seq >= 512)
+        _call("ssm_scan", y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G, bool(chunked))
         return y
     return ssm_scan_ref(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G)
 
