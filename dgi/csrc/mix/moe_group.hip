@@ -13,10 +13,11 @@
 //                                 of an output sit in the same lane, so the activation is the product's epilogue;
 //                  down:          B = down [E, N, K], A = the rows gate-up left, row(place) = place.
 //
-// Two kernels.  Few rows per expert (decode steps): bounded by the expert weights' bytes.  A workgroup owns 64 weight
+// Three kernels.  Few rows per expert (decode steps): bounded by the expert weights' bytes.  A workgroup owns 64 weight
 // rows and up to 64 places; its four waves take a quarter of K each, weights and rows go from memory straight into
 // operand registers (16x16x32 products), and the four partial sums meet in LDS.  Many rows: tiles of 128 places by 128
-// weight rows, K in steps of 64 through two LDS stages (32x32x16 products).
+// weight rows, K in steps of 64 through two LDS stages (32x32x16 products).  Very many: 256 by 256, loaded to LDS
+// directly and multiplied by two groups of waves in turn.
 //
 // The tile a workgroup owns is found from seg alone, so the grid is sized for the worst split of the places over the
 // experts and a workgroup past the last tile leaves.  Weights are the A operand: a lane's result is four consecutive
@@ -335,18 +336,267 @@ __global__ __launch_bounds__(256, 2) void moe_group_tiles_kernel(GroupArgs g, in
   }
 }
 
+// ---- very many rows per expert: up to 256 places x 256 weight rows (GLU: 128 outputs, gate and up), K in steps of 64
+// through two LDS stages of 64 KB, eight waves of 128 places x 64 weight rows.  The matrix cores bound it, so they have to
+// be fed: loads go to LDS directly, and the two waves of a SIMD run one section apart (one reads its operands and issues
+// loads while the other multiplies; every section ends at a barrier), so a SIMD's matrix core is never without work.
+//
+// An expert's n places are shared out evenly over ceil(n / 256) tiles, and a tile of r places multiplies
+// H = ceil(r / 64) blocks of 16 per wave and section, not 4: an expert of 520 places costs 3 x 3/4 tiles, not 3.
+// Tiles are counted expert by expert, an expert's places fastest, and every XCD takes a contiguous run: the 32 tiles it
+// works on at a time are a few tiles of places by about ten of weights of one or two experts, which meet in its L2
+// (places of all experts first: each tile would read weights of its own).
+//
+// 16 experts, K 4096, ff 3584, 512 places each: gate-up 796 us -> 406 (1184 TF/s), down 407 -> 187 (1288); 1024 places
+// each 1342 and 1327 TF/s, 256 each 1028 (one tile of places: the weights come at 4.8 TB/s).  What is left is the last
+// round of tiles: 520 places each are 5.25 rounds of 256 workgroups and take 513 us.
+constexpr int WIDE = 256;
+constexpr int W_TILE = WIDE * 64 * 2;                  // one operand of one stage, bytes
+constexpr int W_STAGE = 2 * W_TILE;
+
+struct WideTile {
+  int e, lo, hi, nt;                                   // expert, places [lo, hi), weight tile
+};
+
+// Tile blockIdx.x of the places' tiles times `ntn` weight tiles; false past the last.  Uniform over the workgroup.
+__device__ __forceinline__ bool find_wide(const int* __restrict__ seg, int E, int ntn, WideTile& t) {
+  const int lane = threadIdx.x & 63;
+  int total = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int ee = e0 + lane;
+    total += ee < E ? (seg[ee + 1] - seg[ee] + WIDE - 1) / WIDE : 0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+  total *= ntn;
+  const int chunk = (total + 7) >> 3, at = blockIdx.x >> 3, id = (blockIdx.x & 7) * chunk + at;
+  if (at >= chunk || id >= total) return false;
+  int base = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int ee = e0 + lane;
+    const int s0 = ee < E ? seg[ee] : 0, s1 = ee < E ? seg[ee + 1] : 0;
+    const int n = (s1 - s0 + WIDE - 1) / WIDE;
+    int inc = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += v;
+    }
+    const unsigned long long m = __ballot((base + inc) * ntn > id);
+    if (m) {
+      const int l = __ffsll(m) - 1;
+      const int tiles = __shfl(n, l, 64), first = base + __shfl(inc, l, 64) - tiles;
+      const int a = __shfl(s0, l, 64), b = __shfl(s1, l, 64);
+      const int per = (b - a + tiles - 1) / tiles, j = (id - first * ntn) % tiles;
+      t.e = e0 + l;
+      t.nt = (id - first * ntn) / tiles;
+      t.lo = a + j * per;
+      t.hi = min(b, a + (j + 1) * per);
+      return t.lo < t.hi;
+    }
+    base += __shfl(inc, 63, 64);
+  }
+  return false;
+}
+
+__device__ __forceinline__ void load_lds16(const char* src, char* lds) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+// Two neighbouring blocks of 16 outputs (four of each per lane) as one 16-byte store: lane group g ends up with eight
+// consecutive outputs, first block 0-7 (g 0), second 0-7 (g 1), first 8-15 (g 2), second 8-15 (g 3).
+__device__ __forceinline__ void st_pair(uint16_t* row, int n0, int N, int g, const float (&a)[4], const float (&b)[4]) {
+  const auto s0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[0], a[1]), pack_bf16x2(b[0], b[1]), false, false);
+  const auto s1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(a[2], a[3]), pack_bf16x2(b[2], b[3]), false, false);
+  const int n = n0 + 16 * (g & 1) + 4 * (g & 2);
+  if (n < N) *reinterpret_cast<uint4*>(row + n) = make_uint4(s0[0], s1[0], s0[1], s1[1]);   // N is a multiple of 8
+}
+
+// K a multiple of 128, N of 8, out at a 16-byte boundary; rows of A and the weights of an expert under 2 GiB each.
+template <bool GLU>
+__global__ __launch_bounds__(512) void moe_group_wide_kernel(GroupArgs g, int ntn) {
+  __shared__ __attribute__((aligned(16))) char lds[2 * W_STAGE];               // [stage][places | weights], rows of 128 bytes
+  WideTile t;
+  if (!find_wide(g.seg, g.E, ntn, t)) return;
+  t.e = __builtin_amdgcn_readfirstlane(t.e);           // in scalar registers: bases and branches are
+  t.nt = __builtin_amdgcn_readfirstlane(t.nt);
+  t.lo = __builtin_amdgcn_readfirstlane(t.lo);
+  t.hi = __builtin_amdgcn_readfirstlane(t.hi);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wm = w >> 2, wn = w & 3;
+  const int H = (t.hi - t.lo + 63) >> 6;
+  constexpr int NO = GLU ? 128 : 256;
+  const int n0 = t.nt * NO;
+  // Staging: slab i = 64 LDS rows.  Slabs 2 m, 2 m + 1 hold the first and second 16 H places of wave row m (rows past
+  // 16 H repeat a place); slab i of the weights holds wave column i's rows (GLU: 32 gate rows, then the matching up rows).
+  // Chunk c of LDS row r is chunk c ^ (r >> 1 & 7) of its 64 elements: reads of 16 rows spread over all banks.
+  const char* A = reinterpret_cast<const char*>(g.a);
+  const char* B = reinterpret_cast<const char*>(g.b + (size_t)t.e * (GLU ? 2 : 1) * g.N * g.K);
+  unsigned ao[4], bo[4];
+  {
+    const int q = tid >> 3, c = ((tid & 7) ^ ((tid >> 4) & 7)) * 16;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int place = min(t.lo + i * 16 * H + min(q, 16 * H - 1), t.hi - 1);
+      ao[i] = (unsigned)(g.order ? g.order[place] / g.top : place) * (unsigned)g.a_stride * 2u + c;
+      const int n = GLU ? n0 + 32 * i + (q & 31) : n0 + 64 * i + q;
+      bo[i] = (unsigned)(min(n, g.N - 1) + (GLU && q >= 32 ? g.N : 0)) * (unsigned)g.K * 2u + c;
+    }
+  }
+  char* const la = lds + w * 1024;
+  // the step's base stays in scalar registers, a lane keeps 32-bit offsets (64-bit addresses per lane spill)
+  auto at = [](const char* p, int kt) {
+    p += (size_t)kt * 128;
+    asm volatile("" : "+s"(p));
+    return p;
+  };
+  auto ga = [&](int kt, int i, int st) { load_lds16(at(A, kt) + ao[i], la + st * W_STAGE + i * 8192); };
+  auto gb = [&](int kt, int i, int st) { load_lds16(at(B, kt) + bo[i], la + st * W_STAGE + W_TILE + i * 8192); };
+
+  const int lr = lane & 15, lg = lane >> 4, key = (lane >> 1) & 7;
+  const int p0 = (lg ^ key) * 16, p1 = ((4 + lg) ^ key) * 16;
+  const int abase = (wm * 128 + lr) * 128, bbase = W_TILE + (wn * 64 + lr) * 128;
+  f32x4 acc[2][4][4];                                  // [half][block of places][block of weights]
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[h][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  auto barrier = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the K loop with HB blocks of 16 places per half.  A step is two sections per wave:
+  //
+  //   section  reads                        products             loads issued                 landed before its barrier
+  //   0        first half, weights          first x weights      weights, slab 2 of step + 1  slabs 1, 3 of this step
+  //   1        second half                  second x weights     slabs 3, 1 of + 1, 0 of + 2  all of + 1 but slabs 3, 1
+  //
+  // A slab is loaded again two sections or more after its last read, and a wave counts only its own loads: what it waits
+  // for is visible to the others behind the barrier.  MODE 1, 2: the last step but one, the last.
+  auto run = [&](auto HB_) {
+    constexpr int HB = decltype(HB_)::value;
+    bf16x8 fa[HB][2], fb[4][2];
+    auto rows = [&](int st, int h) {
+      const char* s = lds + st * W_STAGE + abase + h * 8192;
+#pragma unroll
+      for (int i = 0; i < HB; ++i) {
+        fa[i][0] = *reinterpret_cast<const bf16x8*>(s + i * 2048 + p0);
+        fa[i][1] = *reinterpret_cast<const bf16x8*>(s + i * 2048 + p1);
+      }
+    };
+    auto mma = [&](int h) {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j][k], fa[i][k], acc[h][i][j], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+    };
+    auto step = [&](int s, auto ST_, auto MODE_) {
+      constexpr int ST = decltype(ST_)::value, MODE = decltype(MODE_)::value;
+      if constexpr (MODE < 2) {
+        gb(s + 1, 0, ST ^ 1); gb(s + 1, 1, ST ^ 1); gb(s + 1, 2, ST ^ 1); gb(s + 1, 3, ST ^ 1);
+        ga(s + 1, 2, ST ^ 1);
+      }
+      const char* bs = lds + ST * W_STAGE + bbase;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        fb[j][0] = *reinterpret_cast<const bf16x8*>(bs + j * 2048 + p0);
+        fb[j][1] = *reinterpret_cast<const bf16x8*>(bs + j * 2048 + p1);
+      }
+      rows(ST, 0);
+      if constexpr (MODE < 2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      barrier();
+      mma(0);
+      barrier();
+      if constexpr (MODE < 2) { ga(s + 1, 3, ST ^ 1); ga(s + 1, 1, ST ^ 1); }
+      if constexpr (MODE == 0) ga(s + 2, 0, ST);
+      rows(ST, 1);
+      if constexpr (MODE == 0) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+      else if constexpr (MODE == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+      barrier();
+      mma(1);
+      barrier();
+    };
+    using Z = std::integral_constant<int, 0>;
+    using O = std::integral_constant<int, 1>;
+    using L = std::integral_constant<int, 2>;
+    ga(0, 0, 0); gb(0, 0, 0); gb(0, 1, 0); gb(0, 2, 0); gb(0, 3, 0); ga(0, 2, 0);
+    ga(0, 3, 0); ga(0, 1, 0); ga(1, 0, 1);
+    asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+    barrier();
+    if (wm == 1) barrier();                            // waves 4-7 run one section behind
+    const int steps = g.K >> 6;                        // even
+    int s = 0;
+    for (; s + 4 <= steps; s += 2) {
+      step(s, Z{}, Z{});
+      step(s + 1, O{}, Z{});
+    }
+    step(s, Z{}, O{});
+    step(s + 1, O{}, L{});
+    if (wm == 0) barrier();                            // the last barrier of waves 4-7
+  };
+  switch (H) {
+    case 1: run(std::integral_constant<int, 1>{}); break;
+    case 2: run(std::integral_constant<int, 2>{}); break;
+    case 3: run(std::integral_constant<int, 3>{}); break;
+    default: run(std::integral_constant<int, 4>{});
+  }
+
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int place = t.lo + (2 * wm + h) * 16 * H + 16 * i + lr;
+      if (i >= H || place >= t.hi) continue;           // the four lanes of a place stay together
+      uint16_t* row = g.out + (size_t)place * g.N;
+      float x[4][4];
+      if constexpr (GLU) {
+        const float ps = g.pair_scale ? g.pair_scale[g.order[place]] : 1.f;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) x[j][r] = glu_f(acc[h][i][j][r] * ps, acc[h][i][j + 2][r] * ps, g.act, g.limit, g.alpha);
+        st_pair(row, n0 + 32 * wn, g.N, lg, x[0], x[1]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) x[j][r] = acc[h][i][j][r];
+        st_pair(row, n0 + 64 * wn, g.N, lg, x[0], x[1]);
+        st_pair(row, n0 + 64 * wn + 32, g.N, lg, x[2], x[3]);
+      }
+    }
+}
+
 template <bool GLU>
 int launch_group(GroupArgs g, int places, int rows_per_tile, hipStream_t s) {
   // worst split of the places over the experts: every non-empty expert may end in a partial tile
   const int nonempty = g.E < places ? g.E : places;
-  const int bm = rows_per_tile;
+  int bm = rows_per_tile;
+  if (bm == WIDE) {
+    // 32-bit byte offsets into A and into an expert's weights, whole steps of 128 of K, 16-byte stores
+    const long long a_bytes = 2ll * g.a_stride * (g.order ? (places + g.top - 1) / g.top : places);
+    const long long b_bytes = 2ll * g.N * g.K * (GLU ? 2 : 1);
+    if (g.K % 128 || g.N % 8 || ((uintptr_t)g.out & 15) || a_bytes >= 1ll << 31 || b_bytes >= 1ll << 31) bm = 128;
+  }
   g.mtiles = places / bm + nonempty;
-  const int no = (bm == 128 ? 128 : 64) / (GLU ? 2 : 1);
+  const int no = (bm >= 128 ? bm : 64) / (GLU ? 2 : 1);
   const int ntn = (g.N + no - 1) / no;
   const long long blocks = (long long)g.mtiles * ntn;
   if (blocks > 0x3fffffff) return -4;
-  if (bm == 128) {
-    const int padded = (int)((blocks + 7) / 8 * 8);
+  const int padded = (int)((blocks + 7) / 8 * 8);
+  if (bm == WIDE) {
+    moe_group_wide_kernel<GLU><<<padded, 512, 0, s>>>(g, ntn);
+  } else if (bm == 128) {
     moe_group_tiles_kernel<GLU><<<padded, 256, 0, s>>>(g, ntn);
   } else if (bm == 64) {
     moe_group_rows_kernel<4, GLU><<<(int)blocks, 256, 0, s>>>(g);
@@ -462,7 +712,7 @@ extern "C" int dgi_moe_plan(const int* idx, int P, int E, int* order, int* where
 }
 
 // glu: b [E, 2 N, K] and order / top (and pair_scale) map a place to its row of a; else b [E, N, K] and row = place.
-// rows_per_tile: 16, 32, 64 (few rows per expert) or 128.  places: the most places seg can hold.
+// rows_per_tile: 16, 32, 64 (few rows per expert), 128 or 256.  places: the most places seg can hold.
 extern "C" int dgi_moe_group(const void* a, int a_stride, const void* b, void* out, const int* seg, const int* order,
                              const float* pair_scale, int places, int E, int N, int K, int top, int glu, int act, float limit,
                              float alpha, int rows_per_tile, hipStream_t s) {

@@ -1,0 +1,60 @@
+"""Grouped expert products on tiles of 256 places: experts of no, few and many places, edges of the weight tiles, the
+shortest inner sizes, widths that fall back to the smaller tile, against the products in 64 bits."""
+import pytest
+import torch
+
+from dgi.ops import moe
+
+F64 = torch.float64
+BF16 = torch.bfloat16
+
+# places per expert around the tile's sizes: whole tiles, one place more, blocks of 64 and of 16
+COUNTS = [0, 1, 16, 63, 64, 65, 128, 130, 192, 200, 255, 256, 257, 512, 513, 0, 700]
+
+
+def draw(*shape, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=g) * scale).to(BF16)
+
+
+def exact(h, idx, w, gu, dn, act, limit, weigh):
+    """The weighed sum in 64 bits, and the sum of its terms' magnitudes."""
+    h, gu, dn, w = h.to(F64), gu.to(F64), dn.to(F64), w.to(F64)
+    y, mag = torch.zeros_like(h), torch.zeros_like(h)
+    for e in range(gu.shape[0]):
+        t, k = torch.nonzero(idx == e, as_tuple=True)
+        ws = w[t, k][:, None]
+        z = (h[t] * ws if weigh == "input" else h[t]) @ gu[e].t()
+        g, u = z.chunk(2, dim=1)
+        if act == "clamped":
+            g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+            mid = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+        else:
+            mid = torch.nn.functional.silu(g) * u
+        f = 1.0 if weigh == "input" else ws
+        y.index_add_(0, t, f * (mid @ dn[e].t()))
+        mag.index_add_(0, t, f * (mid.abs() @ dn[e].abs().t()))
+    return y, mag
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act,weigh", [("silu", "output"), ("clamped", "input")])
+@pytest.mark.parametrize("W,ff", [(128, 128), (256, 72), (384, 640), (72, 256)])
+def test_wide_tiles(monkeypatch, W, ff, act, weigh):
+    E, top = len(COUNTS), 2
+    g = torch.Generator().manual_seed(7)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(COUNTS)])
+    flat = flat[torch.randperm(flat.numel(), generator=g)]
+    flat = flat[: flat.numel() // top * top]
+    idx = flat.reshape(-1, top).to(torch.int32)
+    T = idx.shape[0]
+    h = draw(T, W, seed=1)
+    gu, dn = draw(E, 2 * ff, W, seed=2, scale=W ** -0.5), draw(E, W, ff, seed=3, scale=ff ** -0.5)
+    w = torch.rand(T, top, generator=g)
+    monkeypatch.setattr(moe, "group_tile", lambda *a: 256)
+    got = moe.moe_experts(h.cuda(), idx.cuda(), w.cuda(), gu.cuda(), dn.cuda(), None, act=act, limit=0.8, weigh=weigh)
+    y, mag = exact(h, idx, w, gu, dn, act, 0.8, weigh)
+    # three roundings to bf16 (half an ulp is 2^-9): each term's activation, each expert's row, the sum; fp32 elsewhere
+    bound = 2.0 ** -9 * (2 * mag + y.abs()) + 1e-5 * (1 + mag)
+    worst = ((got.cpu().to(F64) - y).abs() / bound).max().item()
+    assert worst <= 1.0, worst
