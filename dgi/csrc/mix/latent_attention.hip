@@ -223,35 +223,134 @@ __global__ __launch_bounds__(1024) void latent_attn_rows_kernel(
   }
 }
 
-// out[h][row] = sum_z o_z e^(m_z - M) / sum_z l_z e^(m_z - M), M = max_z m_z; grid (rows, H), run 0 is never empty
-template <typename T>
+// out[h][row] = sum_z o_z e^(m_z - M) / sum_z l_z e^(m_z - M), M = max_z m_z; grid (rows, H), run 0 is never empty.
+// V consecutive dims per thread (4: kr a multiple of 4); four runs' sums are loaded together.
+template <typename T, int V>
 __global__ __launch_bounds__(256) void latent_attn_reduce_kernel(const float* __restrict__ part_o,
                                                                  const float* __restrict__ part_ml, int nsplit, int kr,
                                                                  T* __restrict__ out, long long o_hs, long long o_ts,
                                                                  const float* __restrict__ sinks) {
   const int row = blockIdx.x, head = blockIdx.y, rows = gridDim.x, H = gridDim.y;
+  const size_t first = (size_t)head * rows + row, next = (size_t)H * rows;         // slot of run 0, slots from run to run
   float M = -__builtin_inff();
-  for (int z = 0; z < nsplit; ++z) M = fmaxf(M, part_ml[2 * (((size_t)z * H + head) * rows + row)]);
+  for (int z = 0; z < nsplit; ++z) M = fmaxf(M, part_ml[2 * (first + z * next)]);
   float L = 0.f;
-  for (int z = 0; z < nsplit; ++z) {
-    const size_t slot = ((size_t)z * H + head) * rows + row;
-    L += part_ml[2 * slot + 1] * expf(part_ml[2 * slot] - M);
-  }
+  for (int z = 0; z < nsplit; ++z) L += part_ml[2 * (first + z * next) + 1] * expf(part_ml[2 * (first + z * next)] - M);
   const float inv = sinks ? inv_with_sink(M, L, sinks[head]) : 1.f / L;
   T* op = out + (size_t)head * o_hs + (size_t)row * o_ts;
-  for (int e = threadIdx.x; e < kr; e += blockDim.x) {
-    float acc = 0.f;
-    for (int z = 0; z < nsplit; ++z) {
-      const size_t slot = ((size_t)z * H + head) * rows + row;
-      acc += part_o[slot * kr + e] * expf(part_ml[2 * slot] - M);
+  for (int e = threadIdx.x * V; e < kr; e += blockDim.x * V) {
+    float acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
+    for (int z0 = 0; z0 < nsplit; z0 += 4) {
+      float x[4][V], f[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const size_t slot = first + (size_t)min(z0 + u, nsplit - 1) * next;
+        const float* po = part_o + slot * kr + e;
+        if constexpr (V == 4) {
+          const float4 v = *reinterpret_cast<const float4*>(po);
+          x[u][0] = v.x; x[u][1] = v.y; x[u][2] = v.z; x[u][3] = v.w;
+        } else {
+          x[u][0] = po[0];
+        }
+        f[u] = part_ml[2 * slot];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (z0 + u >= nsplit) break;
+        const float fz = expf(f[u] - M);
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] += x[u][i] * fz;
+      }
     }
-    stf<T>(op + e, acc * inv);
+#pragma unroll
+    for (int i = 0; i < V; ++i) stf<T>(op + e + i, acc[i] * inv);
   }
 }
 
+template <typename T>
+void launch_reduce(const float* part_o, const float* part_ml, int nsplit, int rows, int H, int kr, T* out, long long o_hs,
+                   long long o_ts, const float* sinks, hipStream_t s) {
+  if (kr % 4 == 0)
+    latent_attn_reduce_kernel<T, 4><<<dim3(rows, H), kr > 256 ? 128 : 64, 0, s>>>(part_o, part_ml, nsplit, kr, out, o_hs, o_ts, sinks);
+  else
+    latent_attn_reduce_kernel<T, 1><<<dim3(rows, H), kr >= 256 ? 256 : 64, 0, s>>>(part_o, part_ml, nsplit, kr, out, o_hs, o_ts, sinks);
+}
+
+// Queries of one row's heads head0 .. head0 + NH - 1 as bf16 rows of stride DP in LDS, [folded part | rotated part]; heads
+// past H are zero rows.  NT threads, kr <= 16 NM.  All loads go out before the first is waited for (addresses past the end
+// are clamped, not skipped), and meanwhile() runs behind the folded part's.
+template <int NH, int NT, int NM, typename F>
+__device__ __forceinline__ void stage_queries(uint16_t* qs, int DP, const uint16_t* __restrict__ q, int q_stride,
+                                              const uint16_t* __restrict__ q_lat, long long ql_hs, long long ql_ts, int row,
+                                              int head0, int H, int dim, int rd, int kr, int pos,
+                                              const float* __restrict__ cos_sin, int dims, int interleaved, F&& meanwhile) {
+  const bool qvec = ((uintptr_t)q_lat & 15) == 0 && (ql_hs & 7) == 0 && (ql_ts & 7) == 0;
+  if (qvec) {
+    constexpr int NQ = (NH * NM * 2 + NT - 1) / NT;
+    const int cq = kr >> 3;
+    u32x4 v[NQ];
+#pragma unroll
+    for (int it = 0; it < NQ; ++it) {
+      const int idx = min((int)threadIdx.x + NT * it, NH * cq - 1);
+      const int hh = idx / cq, c = idx - hh * cq;
+      v[it] = *reinterpret_cast<const u32x4*>(q_lat + (size_t)min(head0 + hh, H - 1) * ql_hs + (size_t)row * ql_ts + c * 8);
+    }
+    meanwhile();
+#pragma unroll
+    for (int it = 0; it < NQ; ++it) {
+      const int idx = min((int)threadIdx.x + NT * it, NH * cq - 1);
+      const int hh = idx / cq, c = idx - hh * cq;
+      *reinterpret_cast<u32x4*>(qs + (size_t)hh * DP + c * 8) = head0 + hh < H ? v[it] : u32x4{0u, 0u, 0u, 0u};
+    }
+  } else {
+    meanwhile();
+    for (int i = threadIdx.x; i < NH * kr; i += NT) {
+      const int hh = i / kr, e = i - hh * kr;
+      const int head = head0 + hh;
+      qs[(size_t)hh * DP + e] = head < H ? q_lat[(size_t)head * ql_hs + (size_t)row * ql_ts + e] : (uint16_t)0;
+    }
+  }
+  // rotated part
+  constexpr int U = 4;
+  const int half = dims >> 1;
+  const float* cs = dims > 0 ? cos_sin + (size_t)pos * dims : nullptr;
+  for (int i0 = threadIdx.x; i0 < NH * rd; i0 += U * NT) {
+    uint16_t a[U], b[U];
+    float c[U], sn[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = min(i0 + u * NT, NH * rd - 1);
+      const int hh = i / rd, e = i - hh * rd;
+      const uint16_t* qr = q + (size_t)row * q_stride + (size_t)min(head0 + hh, H - 1) * (dim + rd) + dim;
+      int k = 0, partner = e;
+      if (e < dims) {
+        k = interleaved ? e >> 1 : e < half ? e : e - half;
+        partner = interleaved ? e ^ 1 : e < half ? e + half : e - half;
+      }
+      a[u] = qr[e];
+      b[u] = qr[partner];
+      c[u] = sn[u] = 0.f;
+      if (cs) {
+        c[u] = cs[k];
+        sn[u] = cs[half + k];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = min(i0 + u * NT, NH * rd - 1);
+      const int hh = i / rd, e = i - hh * rd;
+      const bool lead = interleaved ? !(e & 1) : e < half;                  // the pair's first element
+      const float x = bf16_to_f32(a[u]), y = bf16_to_f32(b[u]);
+      const uint16_t r = f32_to_bf16(lead ? x * c[u] - y * sn[u] : x * c[u] + y * sn[u]);
+      qs[(size_t)hh * DP + kr + e] = head0 + hh >= H ? (uint16_t)0 : e < dims ? r : a[u];
+    }
+  }
+}
 
 // ---------------------------------------------------------------------------------------------
-// MFMA form (bf16; kr and kr + rd multiples of 16).  A workgroup owns one query row, a group of 16
+// MFMA form (bf16; kr and kr + rd multiples of 16; 512 + 64 dims take the tile form below).  A workgroup owns one query row, a group of 16
 // heads and one run of the row's 64-key tiles; its four waves take 16 keys of every tile each and keep
 // their own running softmax, so nothing is exchanged between waves per tile.  Per tile and wave:
 //
@@ -293,56 +392,8 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
   const int pos = positions[row];
   const int first = window > 0 ? max(0, pos - window + 1) : 0;
 
-  // the group's queries as bf16 rows [folded part | rotated part]; heads past H are zero rows
-  {
-    const int half = dims >> 1;
-    const float* cs = cos_sin ? cos_sin + (size_t)pos * dims : nullptr;
-    // folded part: 16-byte copies where the query tensor allows them (all issued before any lands)
-    const bool qvec = ((uintptr_t)q_lat & 15) == 0 && (ql_hs & 7) == 0 && (ql_ts & 7) == 0;
-    if (qvec) {
-      constexpr int NQ = (16 * NM * 2 + 255) / 256;
-      const int cq = kr >> 3;
-#pragma unroll
-      for (int it = 0; it < NQ; ++it) {
-        const int idx = threadIdx.x + 256 * it;
-        const int hh = idx / cq, c = idx - hh * cq;
-        if (hh < 16) {
-          const int head = g * 16 + hh;
-          u32x4 v = {0u, 0u, 0u, 0u};
-          if (head < H) v = *reinterpret_cast<const u32x4*>(q_lat + (size_t)head * ql_hs + (size_t)row * ql_ts + c * 8);
-          *reinterpret_cast<u32x4*>(qs + (size_t)hh * DP + c * 8) = v;
-        }
-      }
-    } else {
-      for (int i = threadIdx.x; i < 16 * kr; i += 256) {
-        const int hh = i / kr, e = i - hh * kr;
-        const int head = g * 16 + hh;
-        qs[(size_t)hh * DP + e] = head < H ? q_lat[(size_t)head * ql_hs + (size_t)row * ql_ts + e] : (uint16_t)0;
-      }
-    }
-    // rotated part
-#pragma unroll 4
-    for (int i = threadIdx.x; i < 16 * rd; i += 256) {
-      const int hh = i / rd, e2 = i - hh * rd;
-      const int head = g * 16 + hh;
-      uint16_t v = 0;
-      if (head < H) {
-        const uint16_t* qr = q + (size_t)row * q_stride + (size_t)head * (dim + rd) + dim;
-        if (e2 < dims) {
-          int k, partner;
-          bool lead;                                  // the pair's first element
-          if (interleaved) { k = e2 >> 1; partner = e2 ^ 1; lead = !(e2 & 1); }
-          else { lead = e2 < half; k = lead ? e2 : e2 - half; partner = lead ? e2 + half : e2 - half; }
-          const float a = bf16_to_f32(qr[e2]), b = bf16_to_f32(qr[partner]);
-          const float c = cs[k], sn = cs[half + k];
-          v = f32_to_bf16(lead ? a * c - b * sn : a * c + b * sn);
-        } else {
-          v = qr[e2];
-        }
-      }
-      qs[(size_t)hh * DP + kr + e2] = v;
-    }
-  }
+  stage_queries<16, 256, NM>(qs, DP, q, q_stride, q_lat, ql_hs, ql_ts, row, g * 16, H, dim, rd, kr, pos, cos_sin, dims, interleaved,
+                             [] {});
   __syncthreads();
   const uint16_t* qp = qs + (size_t)lr * DP + 4 * lg;   // this lane's operand of Q^T: head lr, dims 16 s + 4 lg .. + 3
 
@@ -524,6 +575,256 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Tile form (bf16; latents and keys of whole 128 bytes): what bounds a decode step over long contexts is reading every cached row once.
+// A workgroup owns one query row, 16 NG heads and one run of the row's 64-key tiles; the tiles go from memory to LDS
+// directly, two of them in turn, so that one (74 KB at 512 + 64 dims) is always under way while the other is computed, and
+// the heads share it: with NG = 2 a cached row is read once for 32 heads.  Wave (group of 16 heads, half of the tile):
+//
+//   S^T [32 keys x 16 heads] = K [32 keys x D] Q^T [D x 16 heads]      16x16x32 products, keys from LDS, queries in registers
+//   O^T [kr x 16 heads]     += C^T [kr x 32 keys] P^T [32 keys x 16 heads]      the same, C^T by transposing LDS reads
+//
+// A lane of S^T holds keys 4 g .. + 3 and 16 + 4 g .. + 3 of one head: taken in that order they are its operand of P^T, so
+// nothing is exchanged, and a wave keeps its own running softmax.  Chunk c (16 bytes) of a tile's row j lies at c ^ (j & 7):
+// neither kind of read meets a bank twice.  At the end the two waves of a group exchange halves of O^T through LDS.
+// Keys past the last are copies of it with weight 0.  The widths are constants of the kernel: with loop bounds read at run
+// time the compiler kept neither the products' order nor the operands in registers.
+//
+// 32 rows x 32 heads over about 2000 keys each: 123 us (the form above, every row read for each 16 heads, C^T gathered in
+// single elements) -> 35, 2.1 TB/s; at four to five tiles a workgroup what is left is its first loads, one behind the
+// other (position, page, tile), and the partial sums' 17 MB.
+__device__ __forceinline__ void load_lds16(const char* src, char* lds) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+// Eight operands C^T: blocks of 16 latent dims m .. m + 7, rows 4 g .. + 3 (v[2 i]) and 16 rows on (v[2 i + 1]).  Four
+// neighbouring blocks lie in the same 128 bytes of a row, the next four in the next.  In assembly with its own wait: before
+// the builtin's first read the compiler waits for all loads to LDS under way, the next tile's too.
+template <int RB>
+__device__ __forceinline__ void read_tr8(u32x2 (&v)[16], unsigned a0, unsigned a1, unsigned a2, unsigned a3) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %16\n\t"
+      "ds_read_b64_tr_b16 %1, %16 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %2, %17\n\t"
+      "ds_read_b64_tr_b16 %3, %17 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %4, %18\n\t"
+      "ds_read_b64_tr_b16 %5, %18 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %6, %19\n\t"
+      "ds_read_b64_tr_b16 %7, %19 offset:%20\n\t"
+      "ds_read_b64_tr_b16 %8, %16 offset:128\n\t"
+      "ds_read_b64_tr_b16 %9, %16 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %10, %17 offset:128\n\t"
+      "ds_read_b64_tr_b16 %11, %17 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %12, %18 offset:128\n\t"
+      "ds_read_b64_tr_b16 %13, %18 offset:%21\n\t"
+      "ds_read_b64_tr_b16 %14, %19 offset:128\n\t"
+      "ds_read_b64_tr_b16 %15, %19 offset:%21\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]),
+        "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11]), "=&v"(v[12]), "=&v"(v[13]), "=&v"(v[14]), "=&v"(v[15])
+      : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "n"(16 * RB), "n"(16 * RB + 128)
+      : "memory");
+}
+
+template <int KR, int RD, int NG>
+__global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
+    const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ q_lat, long long ql_hs, long long ql_ts,
+    const uint16_t* __restrict__ cache, const int* __restrict__ block_tables, int bt_stride,
+    const int* __restrict__ cu_seqlens, int n_seqs, const int* __restrict__ positions, int H, int dim,
+    int bs, float scale, int window, const float* __restrict__ cos_sin, int dims, int interleaved,
+    uint16_t* __restrict__ out, long long o_hs, long long o_ts, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const float* __restrict__ sinks) {
+  constexpr int KT = 64, NW = 2 * NG, RPW = KT / NW;                     // keys per tile, waves, rows a wave loads
+  constexpr int D = KR + RD, NK = D / 32, NM = KR / 16, CPR = D / 8, row_bytes = 2 * D, stage = KT * row_bytes;
+  static_assert(KR % 128 == 0 && RD % 64 == 0 && RPW * CPR % 64 == 0, "tiles of whole 128-byte blocks, loads of whole waves");
+  extern __shared__ __attribute__((aligned(16))) char lds[];            // [2][KT][D] bf16
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int kw = w & 1, grp = w >> 1;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int row = blockIdx.x, rows = gridDim.x, head0 = blockIdx.y * 16 * NG;
+
+  int seq = row;
+  if (cu_seqlens) {
+    int lo = 0, hi = n_seqs - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (cu_seqlens[mid] <= row) lo = mid; else hi = mid - 1;
+    }
+    seq = lo;
+  }
+  const int* bt = block_tables + (size_t)seq * bt_stride;
+  const int pos = positions[row];
+  const int first = window > 0 ? max(0, pos - window + 1) : 0;
+  const int ntiles = (pos - first + KT) / KT;
+  const int tps = (ntiles + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int t_lo = blockIdx.z * tps, t_hi = min(ntiles, t_lo + tps);
+
+  // loads of a tile: lane j knows the slot of its row j; load `it` of a wave brings chunks 64 it + lane of the wave's rows
+  auto key_of = [&](int ti) { return min(first + ti * KT + lane, pos); };
+  auto issue = [&](int st, int slots) {
+#pragma unroll
+    for (int it = 0; it < RPW * CPR / 64; ++it) {
+      const int idx = 64 * it + lane, j = idx / CPR, c = idx - j * CPR;
+      const int sl = __shfl(slots, w * RPW + j, 64);
+      load_lds16(reinterpret_cast<const char*>(cache) + (long long)sl * row_bytes + (c ^ (j & 7)) * 16,        // RPW is a multiple of 8
+                 lds + st * stage + w * RPW * row_bytes + it * 1024);
+    }
+  };
+  int key = key_of(t_lo + 1), page = bt[key / bs];     // of the tile loaded next
+  const int key0 = key_of(t_lo), page0 = bt[key0 / bs];
+
+  // queries through the second stage into registers: head lr of the group, dims 32 s + 8 lg .. + 7
+  bf16x8 qf[NK];
+  {
+    const int DP = D + 8;
+    uint16_t* qs = reinterpret_cast<uint16_t*>(lds + stage);
+    stage_queries<16 * NG, 128 * NG, NM>(qs, DP, q, q_stride, q_lat, ql_hs, ql_ts, row, head0, H, dim, RD, KR, pos, cos_sin, dims,
+                                         interleaved, [&] { if (t_lo < t_hi) issue(0, page0 * bs + key0 % bs); });
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NK; ++s)
+      qf[s] = *reinterpret_cast<const bf16x8*>(qs + (size_t)(grp * 16 + lr) * DP + 32 * s + 8 * lg);
+  }
+
+  float m_run = -__builtin_inff(), l_run = 0.f;        // of head lr, over this wave's keys
+  f32x4 acc[NM];                                       // O^T: latent dims 16 m + 4 lg + i of head lr
+#pragma unroll
+  for (int m = 0; m < NM; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int k0off = (32 * kw + lr) * row_bytes + (lg ^ (lr & 7)) * 16, k1off = (32 * kw + lr) * row_bytes + ((4 + lg) ^ (lr & 7)) * 16;
+  const int tq = lr >> 2, tp = lr & 3;
+  int voff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    voff[i] = (32 * kw + 4 * lg + tq) * row_bytes + ((2 * i + (tp >> 1)) ^ ((4 * lg + tq) & 7)) * 16 + (tp & 1) * 8;
+
+  int st = 0;
+  for (int ti = t_lo; ti < t_hi; ++ti, st ^= 1) {
+    // this wave's loads of tile ti have landed, and its reads of the other stage; behind the barrier everybody's
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int slots = page * bs + key % bs;
+    key = key_of(ti + 2);
+    page = bt[key / bs];                               // not waited for before the next tile's turn
+    if (ti + 1 < t_hi) issue(st ^ 1, slots);
+    const int n = min(KT, pos - (first + ti * KT) + 1);
+    if (32 * kw >= n) continue;                        // none of this wave's keys exists (wave-uniform; no barrier follows)
+    const char* tile = lds + st * stage;
+    f32x4 sp[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) sp[u][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NK; ++s) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const bf16x8 a = *reinterpret_cast<const bf16x8*>(tile + ((s & 1) ? k1off : k0off) + u * 16 * row_bytes + (s >> 1) * 128);
+          sp[u][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[s], sp[u][s & 1], 0, 0, 0);
+        }
+    }
+    // x[u][i]: key 32 kw + 16 u + 4 lg + i, head lr
+    float x[2][4], mx = -__builtin_inff();
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[u][i] = (32 * kw + 16 * u + 4 * lg + i < n) ? (sp[u][0][i] + sp[u][1][i]) * scale : -__builtin_inff();
+        mx = fmaxf(mx, x[u][i]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));            // key 32 kw exists: finite
+    const float m_new = fmaxf(m_run, mx);
+    const float corr = expf(m_run - m_new);            // first tile: exp(-inf) = 0
+    float sum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        x[u][i] = expf(x[u][i] - m_new);
+        sum += x[u][i];
+      }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    l_run = l_run * corr + sum;
+    m_run = m_new;
+    u32x4 pf;
+    pf[0] = pack_bf16x2(x[0][0], x[0][1]);
+    pf[1] = pack_bf16x2(x[0][2], x[0][3]);
+    pf[2] = pack_bf16x2(x[1][0], x[1][1]);
+    pf[3] = pack_bf16x2(x[1][2], x[1][3]);
+    if (__any(corr != 1.f)) {                          // else no head's maximum moved: the sums keep their scale
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[m][i] *= corr;
+    }
+    const unsigned tl = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)tile;
+#pragma unroll
+    for (int m = 0; m < NM; m += 8) {
+      u32x2 v[16];
+      read_tr8<row_bytes>(v, tl + voff[0] + m * 32, tl + voff[1] + m * 32, tl + voff[2] + m * 32, tl + voff[3] + m * 32);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const u32x4 vf = {v[2 * i][0], v[2 * i][1], v[2 * i + 1][0], v[2 * i + 1][1]};
+        acc[m + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), acc[m + i], 0, 0, 0);
+      }
+    }
+  }
+
+  // the two waves of a group: (max, sum) of every head, then each gives the other half of its O^T and keeps the rest
+  __syncthreads();                                     // the last tile is fully read
+  float* ml = reinterpret_cast<float*>(lds);           // [NW][16][2]
+  f32x4* ex = reinterpret_cast<f32x4*>(lds + NW * 128);      // [NW][NM / 2][64]
+  if (lg == 0) {
+    ml[(w * 16 + lr) * 2] = m_run;
+    ml[(w * 16 + lr) * 2 + 1] = l_run;
+  }
+#pragma unroll
+  for (int mm = 0; mm < NM / 2; ++mm) {                // wave 0 of a group keeps the first half, wave 1 the second
+    const f32x4 lo = acc[mm], hi = acc[mm + NM / 2];
+    ex[(w * (NM / 2) + mm) * 64 + lane] = kw ? lo : hi;
+    acc[mm] = kw ? hi : lo;
+  }
+  __syncthreads();
+  const float m2 = ml[((w ^ 1) * 16 + lr) * 2], l2 = ml[((w ^ 1) * 16 + lr) * 2 + 1];
+  const float M = fmaxf(m_run, m2);
+  const float f1 = m_run == -__builtin_inff() ? 0.f : expf(m_run - M);   // a wave (or a whole run) without keys adds nothing
+  const float f2 = m2 == -__builtin_inff() ? 0.f : expf(m2 - M);
+  const float L = l_run * f1 + l2 * f2;
+  const int head = head0 + grp * 16 + lr;
+  if (head >= H) return;
+  const size_t slot = ((size_t)blockIdx.z * H + head) * rows + row;
+  if (part_o && kw == 0 && lg == 0) {
+    part_ml[2 * slot] = M;
+    part_ml[2 * slot + 1] = L;
+  }
+  const float inv = part_o ? 1.f : sinks ? inv_with_sink(M, L, sinks[head]) : 1.f / L;
+  uint16_t* op = out + (size_t)head * o_hs + (size_t)row * o_ts;
+  const bool ovec = ((uintptr_t)out & 7) == 0 && (o_hs & 3) == 0 && (o_ts & 3) == 0;
+  auto kept = [&](auto put) {                          // put(latent dim, its four sums) for the half this wave keeps
+#pragma unroll
+    for (int mm = 0; mm < NM / 2; ++mm) {
+      const f32x4 y = ex[((w ^ 1) * (NM / 2) + mm) * 64 + lane];
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (acc[mm][i] * f1 + y[i] * f2) * inv;
+      put(16 * (kw * (NM / 2) + mm) + 4 * lg, v);
+    }
+  };
+  if (part_o)
+    kept([&](int e, const float* v) { *reinterpret_cast<float4*>(part_o + slot * KR + e) = make_float4(v[0], v[1], v[2], v[3]); });
+  else if (ovec)
+    kept([&](int e, const float* v) { *reinterpret_cast<uint2*>(op + e) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])); });
+  else
+    kept([&](int e, const float* v) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) op[e + i] = f32_to_bf16(v[i]);
+    });
+}
+
 template <typename K>
 int allow_lds(K kernel, size_t lds) {
   return (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -568,7 +869,7 @@ int launch(const void* q, int q_stride, const void* q_lat, long long ql_hs, long
       positions, H, dim, rd, kr, bs, scale, window, cos_sin, dims, interleaved, (T*)out, o_hs, o_ts, DP, DQ,
       nsplit > 1 ? part_o : nullptr, part_ml, sinks);
   if (nsplit > 1)
-    latent_attn_reduce_kernel<T><<<dim3(rows, H), kr >= 256 ? 256 : 64, 0, s>>>(part_o, part_ml, nsplit, kr, (T*)out, o_hs, o_ts, sinks);
+    launch_reduce<T>(part_o, part_ml, nsplit, rows, H, kr, (T*)out, o_hs, o_ts, sinks, s);
   return 0;
 }
 
@@ -598,8 +899,31 @@ int launch_mfma(const void* q, int q_stride, const void* q_lat, long long ql_hs,
       cu_seqlens, n_seqs, positions, H, dim, rd, kr, bs, scale, window, cos_sin, dims, interleaved, DP, (uint16_t*)out, o_hs,
       o_ts, nsplit > 1 ? part_o : nullptr, part_ml, magic, sinks);
   if (nsplit > 1)
-    latent_attn_reduce_kernel<uint16_t><<<dim3(rows, H), kr >= 256 ? 256 : 64, 0, s>>>(part_o, part_ml, nsplit, kr,
-                                                                                      (uint16_t*)out, o_hs, o_ts, sinks);
+    launch_reduce<uint16_t>(part_o, part_ml, nsplit, rows, H, kr, (uint16_t*)out, o_hs, o_ts, sinks, s);
+  return 0;
+}
+
+template <int KR, int RD, int NG>
+int launch_tiles(const void* q, int q_stride, const void* q_lat, long long ql_hs, long long ql_ts, const void* cache,
+                 const int* block_tables, int bt_stride, const int* cu_seqlens, int n_seqs, const int* positions, int rows,
+                 int H, int dim, int bs, float scale, int window, const float* cos_sin, int dims,
+                 int interleaved, void* out, long long o_hs, long long o_ts, int nsplit, float* part_o, float* part_ml,
+                 const float* sinks, hipStream_t s) {
+  constexpr int D = KR + RD;
+  // two tiles; the queries (rows of D + 8) fit in the second, the exchange at the end takes the place of both
+  constexpr size_t lds = std::max(2 * 64 * D * 2, 2 * NG * (128 + KR / 32 * 64 * 16));
+  static_assert(16 * NG * (D + 8) <= 64 * D, "queries in one stage");
+  if (lds > lds_max()) return -6;
+  static int allowed = -1;
+  if (allowed != 0 && lds > 64 * 1024) {
+    allowed = allow_lds(latent_attn_tiles_kernel<KR, RD, NG>, lds_max());
+    if (allowed != 0) return allowed;
+  }
+  latent_attn_tiles_kernel<KR, RD, NG><<<dim3(rows, (H + 16 * NG - 1) / (16 * NG), nsplit), 128 * NG, lds, s>>>(
+      (const uint16_t*)q, q_stride, (const uint16_t*)q_lat, ql_hs, ql_ts, (const uint16_t*)cache, block_tables, bt_stride,
+      cu_seqlens, n_seqs, positions, H, dim, bs, scale, window, cos_sin, dims, interleaved, (uint16_t*)out, o_hs, o_ts,
+      nsplit > 1 ? part_o : nullptr, part_ml, sinks);
+  if (nsplit > 1) launch_reduce<uint16_t>(part_o, part_ml, nsplit, rows, H, KR, (uint16_t*)out, o_hs, o_ts, sinks, s);
   return 0;
 }
 
@@ -627,6 +951,10 @@ extern "C" int dgi_latent_attn_rows(const void* q, int q_stride, const void* q_l
       rc = launch_mfma<8, 12>(q, q_stride, q_lat, ql_hs, ql_ts, cache, block_tables, bt_stride, cu_seqlens, n_seqs, positions,
                               rows, H, dim, rd, kr, block_size, scale, window, cos_sin, dims, interleaved, out, o_hs, o_ts,
                               nsplit, part_o, part_ml, sinks, s);
+    else if (kr == 512 && rd == 64)
+      rc = (H <= 16 ? launch_tiles<512, 64, 1> : launch_tiles<512, 64, 2>)(
+          q, q_stride, q_lat, ql_hs, ql_ts, cache, block_tables, bt_stride, cu_seqlens, n_seqs, positions, rows, H, dim, block_size,
+          scale, window, cos_sin, dims, interleaved, out, o_hs, o_ts, nsplit, part_o, part_ml, sinks, s);
     else
       rc = launch_mfma<32, 36>(q, q_stride, q_lat, ql_hs, ql_ts, cache, block_tables, bt_stride, cu_seqlens, n_seqs, positions,
                                rows, H, dim, rd, kr, block_size, scale, window, cos_sin, dims, interleaved, out, o_hs, o_ts,

@@ -194,6 +194,15 @@ def split_runs(rows: int, heads: int, max_keys: int) -> int:
     return int(max(1, min(16, SPLIT_WAVES // (rows * heads), max_keys // 128)))
 
 
+def tile_runs(rows: int, heads: int, max_keys: int) -> int:
+    """Runs of keys per row for the tile kernel (512 + 64 dims): its workgroups take a row, up to 32 heads and one run, one
+    to a compute unit (two tiles are most of its LDS), so as many as fill the 256 of them, every run at least two 64-key tiles
+    long.  32 rows of 32 heads over 2000 keys: 8 runs 35 us and 8 to combine them."""
+    if max_keys <= 0 or rows <= 0:
+        return 1
+    return int(max(1, min(64, 256 // (rows * ((heads + 31) // 32)), max_keys // 128)))
+
+
 def latent_attn_rows(q: torch.Tensor, q_lat: torch.Tensor, cache: torch.Tensor, block_tables: torch.Tensor,
                      cu_seqlens: Optional[torch.Tensor], positions: torch.Tensor, H: int, dim: int, rot_dim: int,
                      kv_rank: int, scale: float, window: int, cos_sin: Optional[torch.Tensor], interleaved: bool,
@@ -212,9 +221,12 @@ def latent_attn_rows(q: torch.Tensor, q_lat: torch.Tensor, cache: torch.Tensor, 
     if _native(q):
         T = q.shape[0]
         mfma = mfma_rows_ok(q.dtype, kv_rank, rot_dim)
-        # the MFMA kernel's workgroups (16 heads, 4 waves) are best at about one per compute unit
-        nsplit = split_runs(T, (H + 15) // 16 * 16 if mfma else H,
-                            min(max_keys, window) if window > 0 and max_keys > 0 else max_keys)
+        bound = min(max_keys, window) if window > 0 and max_keys > 0 else max_keys
+        if mfma and kv_rank == 512 and rot_dim == 64:
+            nsplit = tile_runs(T, H, bound)
+        else:
+            # the MFMA kernel's workgroups (16 heads, 4 waves) are best at about one per compute unit
+            nsplit = split_runs(T, (H + 15) // 16 * 16 if mfma else H, bound)
         po = pm = None
         if nsplit > 1:
             po = torch.empty(nsplit * H * T * kv_rank, dtype=torch.float32, device=q.device)

@@ -54,7 +54,7 @@ def test_wide_tiles(monkeypatch, W, ff, act, weigh):
     monkeypatch.setattr(moe, "group_tile", lambda *a: 256)
     got = moe.moe_experts(h.cuda(), idx.cuda(), w.cuda(), gu.cuda(), dn.cuda(), None, act=act, limit=0.8, weigh=weigh)
     y, mag = exact(h, idx, w, gu, dn, act, 0.8, weigh)
-    # three roundings to bf16 (half an ulp is 2^-9): each term's activation, each expert's row, the sum; fp32 elsewhere
-    bound = 2.0 ** -9 * (2 * mag + y.abs()) + 1e-5 * (1 + mag)
+    # three roundings to bf16 (at most 2^-8 of the value): each term's activation, each expert's row, the sum; fp32 elsewhere
+    bound = 2.0 ** -8 * (2 * mag + y.abs()) + 1e-5 * (1 + mag)
     worst = ((got.cpu().to(F64) - y).abs() / bound).max().item()
     assert worst <= 1.0, worst
