@@ -8,7 +8,7 @@
 // [cached prefix | freshly written KV] straight from the block pool.
 //
 // CDNA4 structure:
-//   grid = (q_tiles, n_heads), 256 threads = 4 waves x 32 query rows.
+//   grid = q_tiles x n_heads (all heads of a tile side by side), 256 threads = 4 waves x 32 query rows.
 //   K/V tiles of 64 keys are staged through LDS by the whole workgroup:
 //     * K image: 256-byte rows, 16-byte chunk XOR-swizzled by (row & 15) so the
 //       32-row ds_read_b128 fragment reads are conflict free (guide T2);
@@ -36,7 +36,7 @@ extern "C" int dgi_paged_prefill(const void* q, int q_stride, const void* k_cach
                                  int tree_n, int tile_rows, hipStream_t s) {
   if (n_tiles == 0) return 0;
   if (hd != 128 && hd != 64) return -5;
-  if (nh % nkv) return -2;
+  if (nh % nkv || (long long)n_tiles * nh > 0x7fffffff) return -2;
   if (tree_n > 64) return -6;
   int bs_log2 = 0;
   while ((1 << bs_log2) < block_size) ++bs_log2;
@@ -46,7 +46,7 @@ extern "C" int dgi_paged_prefill(const void* q, int q_stride, const void* k_cach
   tile_rows &= 0xffff;
   if (tile_rows != 128 && tile_rows != 256) return -7;
 #define DGI_PREFILL(HDV, NWV, DBV)                                                                     \
-  prefill_attn_kernel<HDV, NWV, DBV><<<dim3(n_tiles, nh), NWV * 64, 0, s>>>(                           \
+  prefill_attn_kernel<HDV, NWV, DBV><<<n_tiles * nh, NWV * 64, 0, s>>>(                           \
       (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables,     \
       bt_stride, cu_seqlens_q, context_lens, tiles, (uint16_t*)out, out_stride, nh, nkv, bs_log2,         \
       scale_log2, tree_mask, tree_n)

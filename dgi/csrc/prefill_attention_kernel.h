@@ -68,10 +68,15 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   __shared__ __attribute__((aligned(16))) uint16_t lds[(DB ? 2 : 1) * KT * (HD + HDV)];
   const int dk = PAD ? dk_ : HD, dv = PAD ? dv_ : HDV;
 
-  const int b = tiles[2 * blockIdx.x];
-  const int t0 = tiles[2 * blockIdx.x + 1];  // first query row (within seq) of this tile
-  const int head = blockIdx.y;
-  const int kvh = head / (nh / nkv);
+  // Workgroup -> (tile, head): all heads of a tile before the next tile, so that in a list with the heaviest tiles first no
+  // head's heavy tiles start when the others are nearly done, and neighbours take different key/value heads: XCD x (workgroup
+  // x mod 8) works on the heads of key/value head x mod nkv, whose keys and values stay in its L2.  One prompt of 8192 rows,
+  // 32 heads on 8, traced: head by head, the last head's heavy tiles ran almost alone, 969 us; so 739.
+  const int hx = blockIdx.x % nh, tile = blockIdx.x / nh;
+  const int b = tiles[2 * tile];
+  const int t0 = tiles[2 * tile + 1];  // first query row (within seq) of this tile
+  const int kvh = hx % nkv;
+  const int head = kvh * (nh / nkv) + hx / nkv;
   // per-head score factor: folded into the scale; the softmax below takes maxima of raw scores, so a negative
   // factor flips the raw scores' sign, and a factor of zero stays above it (masked keys are -inf)
   bool flip = false;
@@ -88,7 +93,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   const int* bt = block_tables + (size_t)b * bt_stride;
 
   const int tid = threadIdx.x;
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);      // in a scalar register: what depends on the wave alone is
   const int lane = tid & 63;
   const int lr = lane & 31;
   const int hh = lane >> 5;
@@ -285,18 +290,53 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     if (kb0 > wave_last_pos || !wave_rows) continue;
     if (MASKED && kb0 + KT <= wave_min_first) continue;    // wholly before every row's block
 
-    // ---- S^T = K Q^T for two 32-key blocks
+    // ---- S^T = K Q^T for two 32-key blocks: the first block's operands are all under way before its products, the
+    // second's come between them (left to itself the compiler waits out an LDS read for every product or two).  With the
+    // first values read before the softmax, the second block's exponentials between the first's products and no exchange
+    // between the halves of a wave per tile: 739 us -> 704 (without the trace 617, 890 TF/s); matrix cores and vector unit
+    // are busy 43 % of the time each.  (A wave's next scores taken beside its softmax, in blocks of 32 keys, measured 759:
+    // the scalar and address work of two steps a tile cost more than the overlap gave.)
     f32x16 sc[2];
+    {
+      bf16x8 kf[2][NS];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+      for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sc[kb][r] = 0.f;
+        for (int s = 0; s < NS; ++s) kf[kb][s] = *reinterpret_cast<const bf16x8*>(ks + k_off<HD>(32 * kb + lr, 2 * s + hh));
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[kb][r] = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kb][s], as_bf16x8(qf[s]), sc[kb], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x100, NS, 0);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(ks + k_off<HD>(32 * kb + lr, 2 * s + hh));
-        sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(qf[s]), sc[kb], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       }
+      __builtin_amdgcn_sched_group_barrier(0x008, NS, 0);
     }
+    // operands of V^T: keys 32 (j >> 1) + 16 (j & 1) .. + 15 of the tile, all blocks of 32 dims; the first before the softmax
+    const int g16 = lane >> 4;
+    const int idx = lane & 15;
+    const int tq = idx >> 2, tp = idx & 3;
+    auto read_v = [&](int j, u32x4 (&vf)[ND]) {
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        const int col = 32 * d + 16 * (g16 & 1) + 4 * tp;
+        const int r0 = 16 * j + 4 * hh + tq;
+        const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vs + v_off<HDV>(r0, col >> 3) + (col & 7)));
+        const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vs + v_off<HDV>(r0 + 8, col >> 3) + (col & 7)));
+        vf[d][0] = (uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16);
+        vf[d][1] = (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16);
+        vf[d][2] = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
+        vf[d][3] = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
+      }
+    };
+    u32x4 vf[2][ND];
+    read_v(0, vf[0]);
     if constexpr (BIAS) {
       // distance bias in raw score units (bias / scale): one table row per distance, the last row for
       // everything farther — a tile wholly beyond it for every row of the wave adds one constant
@@ -347,26 +387,29 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
       // finite value: a lane whose keys are all masked must get max -inf (no rescale) and
       // P = 2^(-inf) = 0, whatever the scale.  Causal-only tiles (the diagonal) skip the
       // 64-bit tree-mask shifts.
-      const int lim = row_valid ? min(my_pos, kv_end - 1) : -1;    // last visible key
+      // Keys count from this lane's first one, so that the limits are compared with constants.
       const int key0 = kb0 + 4 * hh;
+      const int lim = (row_valid ? min(my_pos, kv_end - 1) : -1) - key0;    // last visible key
       if (wave_tree) {
+        const int tree0 = tree_key0 - key0;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int key = key0 + 32 * kb + (r & 3) + 8 * (r >> 2);
-            const int dt = key - tree_key0;
+            const int key = 32 * kb + (r & 3) + 8 * (r >> 2);
+            const int dt = key - tree0;
             const bool tbit = (tmask >> (dt & 63)) & 1ull;
-            const bool ok = (key <= lim) & (!is_tree | (dt < 0) | tbit);
+            const bool ok = (lim >= key) & (!is_tree | (dt < 0) | tbit);
             sc[kb][r] = ok ? sc[kb][r] : -__builtin_inff();
           }
       } else {
+        const int from = my_first - key0;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int key = key0 + 32 * kb + (r & 3) + 8 * (r >> 2);
-            const bool ok = MASKED ? (key <= lim) & (key >= my_first) : (key <= lim);
+            const int key = 32 * kb + (r & 3) + 8 * (r >> 2);
+            const bool ok = MASKED ? (lim >= key) & (from <= key) : (lim >= key);
             sc[kb][r] = ok ? sc[kb][r] : -__builtin_inff();
           }
       }
@@ -377,10 +420,11 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[kb][r]);
     mx = row_valid ? mx * scale_log2 : -1e30f;
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     // deferred max: rescale O / l only when the running max grows by > 2^8, so
-    // most tiles skip the 64 O multiplies (P stays <= 256, safe in f32 / bf16)
+    // most tiles skip the 64 O multiplies (P stays <= 256, safe in f32 / bf16) and the exchange with the half of the wave
+    // that holds the query's other keys
     if (__any(mx > m_run + 8.f)) {
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float m_new = fmaxf(m_run, mx);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       l_run *= alpha;
@@ -388,63 +432,45 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
       for (int d = 0; d < ND; ++d) o[d] *= alpha;
       m_run = m_new;
     }
-    // P = 2^(s * scale_log2 - m): packed fp32 (v_pk_fma_f32 / v_pk_add_f32), two scores per
-    // VALU issue for the scale and the row sums; raw v_exp_f32 (arguments <= 8; masked scores
-    // underflow to 0); four partial row sums instead of one 32-long dependent add chain
-    float ps[4];
-    {
-      const f32x2v s2 = {scale_log2, scale_log2};
-      const f32x2v n2 = {-m_run, -m_run};
-      f32x2v acc2[2] = {{0.f, 0.f}, {0.f, 0.f}};
+    // P = 2^(s * scale_log2 - m) (raw v_exp_f32: arguments <= 8, masked scores underflow to 0; four partial row sums instead
+    // of one 32-long dependent add chain) and O^T += V^T P^T.  The second block's exponentials run between the first
+    // block's products: each takes about as long as the other.
+    float ps[4] = {0.f, 0.f, 0.f, 0.f};
+    auto weights = [&](int kb) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-          f32x2v x = {sc[kb][r], sc[kb][r + 1]};
-          x = x * s2 + n2;
-          x[0] = __builtin_amdgcn_exp2f(x[0]);
-          x[1] = __builtin_amdgcn_exp2f(x[1]);
-          sc[kb][r] = x[0];
-          sc[kb][r + 1] = x[1];
-          acc2[(r >> 1) & 1] += x;
-        }
-      ps[0] = acc2[0][0];
-      ps[1] = acc2[0][1];
-      ps[2] = acc2[1][0];
-      ps[3] = acc2[1][1];
-    }
-    float psum = (ps[0] + ps[1]) + (ps[2] + ps[3]);
-    psum += __shfl_xor(psum, 32, 64);
-    l_run += psum;
-
-    // ---- O^T += V^T P^T
-    const int g16 = lane >> 4;
-    const int idx = lane & 15;
-    const int tq = idx >> 2, tp = idx & 3;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+      for (int r = 0; r < 16; ++r) {
+        sc[kb][r] = __builtin_amdgcn_exp2f(sc[kb][r] * scale_log2 - m_run);
+        ps[r & 3] += sc[kb][r];
+      }
+    };
+    auto products = [&](int kb) {
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
+        const int j = 2 * kb + s2;
+        if (j < 3) read_v(j + 1, vf[(j + 1) & 1]);
         u32x4 pf;
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) pf[jj] = pack_bf16x2(sc[kb][8 * s2 + 2 * jj], sc[kb][8 * s2 + 2 * jj + 1]);
 #pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          const int col = 32 * d + 16 * (g16 & 1) + 4 * tp;
-          const int r0 = 32 * kb + 16 * s2 + 4 * hh + tq;
-          short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_short4*)(vs + v_off<HDV>(r0, col >> 3) + (col & 7)));
-          short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_short4*)(vs + v_off<HDV>(r0 + 8, col >> 3) + (col & 7)));
-          u32x4 vf;
-          vf[0] = (uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16);
-          vf[1] = (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16);
-          vf[2] = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
-          vf[3] = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
-          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vf), as_bf16x8(pf), o[d], 0, 0, 0);
-        }
+        for (int d = 0; d < ND; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vf[j & 1][d]), as_bf16x8(pf), o[d], 0, 0, 0);
       }
+    };
+    weights(0);
+    __builtin_amdgcn_sched_barrier(0);
+    products(0);
+    weights(1);
+#pragma unroll
+    for (int i = 0; i < 2 * ND; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 32 / ND, 0);
+      __builtin_amdgcn_sched_group_barrier(0x400, 8 / ND, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    products(1);
+    l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);      // this lane's keys; the halves of the wave meet after the loop
   }
+  l_run += __shfl_xor(l_run, 32, 64);
 
   if (!row_valid) return;
   if (MASKED && sinks) l_run += __builtin_amdgcn_exp2f(sinks[head] * 1.4426950408889634f - m_run);   // sink: denominator only

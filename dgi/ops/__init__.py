@@ -344,8 +344,8 @@ def order_prefill_tiles(cu_seqlens_q, context_lens=None, tile: int = 0) -> np.nd
     heaviest tiles first.  A causal tile's work is the keys it reads, kv_end = context -
     qlen + t0 + tile, so in (sequence, row) order the longest workgroups of the last heads
     are dispatched last and run alone at the end of the grid; longest-first ordering lets
-    the short ones fill in behind them (the grid is (tiles, heads): every head walks the
-    same order).  Ties keep (sequence, row) order."""
+    the short ones fill in behind them (the kernel takes all heads of a tile before the
+    next tile).  Ties keep (sequence, row) order."""
     tile = tile or PREFILL_TILE
     cu = np.asarray(cu_seqlens_q, np.int64)
     nb = len(cu) - 1
