@@ -897,19 +897,37 @@ extern "C" int dgi_chunk_scan_decay(float* y, int light, const void* q, int q_st
 constexpr int SHORT = 16;            // rows up to which a sequence stays with this file's kernel beside a chunked launch (one chunk)
 constexpr int APART_FROM = 8;        // sequences of a step above which those are looked for
 
+// Rows a portion has to have for chunk_scan.hip to be the faster, where all portions of the step are alike.  It takes a third to a quarter of
+// this file's time per row, but the time of some 80 rows more per portion (its pipeline fills): 64 rows, below which delta and mlstm, whose
+// token loops are long, still gain (72 rows, 16 portions, 64 heads of 64: 99 -> 70 and 113 -> 94 us).  wkv's loop is short, and once the
+// workgroups (16 columns) outnumber the places its pipelines find on the chip they also wait for each other (64-wide heads; units, rows, this
+// file's time, chunk_scan.hip's: 256, 72, 23, 19 us; 1024, 100, 38, 44; 2816, 140, 144, 140; 4096, 140, 154, 185; 128-wide heads: 2048, 72,
+// 90, 103; 4096, 100, 362, 335).  light is up against chunk_scan_decay.hip (512 units, 300 rows: 33, 29; 704, 200: 37, 41; 1408, 200: 64, 60;
+// 256, 231: 21, 24).
+static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
+  const long units = (long)n_seq * H * ((dv + 15) / 16);
+  if (mode == LIGHT) return units > 768 ? 160 : units > 256 ? 320 : 1l << 40;
+  if (mode != WKV || units <= 512) return 64;
+  return dk > 64 ? 104 : units <= 3072 ? 136 : 224;
+}
+
 // The kernel of a step's prompt portions: 0 this file's (no portions, or shapes the others do not take), 1 chunk_scan.hip, 2 chunk_scan_decay.hip.
-// chunk_scan.hip takes a third to a quarter of this file's time per row, but the time of some 80 rows more per portion (its pipeline fills) and
-// a second launch beside decode rows (measured, 32 heads: 4 of 5 steps with portions of 46 rows and less are slower there).  Known here are
-// the step's rows and sequences: on average more than 64 rows a sequence, or 256 rows more than sequences.
+// Known here are the step's rows and sequences: with at least chunk_from() rows a sequence on average the portions are long enough; few rows on
+// average and yet many rows are decode rows beside long portions.  Among many sequences both kernels are launched and each
+// sequence is taken by its own length; in between the launch of chunk_scan.hip would mostly be in vain.
 // gla and light have chunk_scan_decay.hip too, with little to fill: better than this file's kernel from some four rows a sequence on, or 128 rows
-// beside decode rows.  light leaves it for chunk_scan.hip where its workgroups (16 columns) outnumber the compute units (2 prompts
-// of 4096 rows in all, 64 heads of 64: 214 against 167 us; 2 prompts of 462 rows, 32 heads: 21 against 24).
+// beside decode rows.
 static int chunk_form(int mode, int dk, int dv, int G, int H, const void* q, int q_stride, const void* k, int k_stride, int in_f32, int n_seq,
                       int rows) {
-  const bool portions = rows > 64 * n_seq || rows - n_seq >= 256;
+  const long from = chunk_from(mode, dk, dv, H, n_seq);
+  bool portions = rows > from * n_seq;
+  if (mode != GLA && mode != LIGHT) {
+    if (from <= 64) portions |= rows - n_seq >= 256;
+    else if (n_seq > APART_FROM) portions = 4l * rows > 3 * from * n_seq || (rows - n_seq >= 512 && rows <= 48l * n_seq);
+  }
   const bool ok = portions && dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32);
   if ((mode == GLA || mode == LIGHT) && dk <= 256 && G == H) {
-    if (ok && rows > 64 * n_seq && (long)n_seq * H * ((dv + 15) / 16) > compute_units()) return 1;
+    if (ok) return 1;
     return rows > 4 * n_seq || rows - n_seq >= 128 ? 2 : 0;
   }
   return ok;
@@ -944,9 +962,10 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   bool short_rows = rows <= 4 * n_seq;             // rows of the step: at most four per sequence on average
   const bool staged = mode == MLSTM && norm_new && mx_new;
   // Prompt portions: sixteen tokens at a time on the matrix cores (chunk_scan.hip).  Among many sequences there are decode
-  // rows beside the portions: those of at most SHORT rows stay with this kernel, in a launch of their own.
+  // rows and short portions beside the long ones: they stay with this kernel, in a launch of their own.
   const int form = chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows);
-  const int apart = n_seq > APART_FROM && (form == 1 || (form == 2 && rows <= 4 * n_seq)) ? SHORT : 0;
+  const int apart = n_seq > APART_FROM && (form == 1 || (form == 2 && rows <= 4 * n_seq))
+                        ? (mode == WKV && chunk_from(mode, dk, dv, H, n_seq) > 64 ? (int)chunk_from(mode, dk, dv, H, n_seq) : SHORT) : 0;
   if (form) {
     const int rc = form == 1 ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
                                               aux2, aux2_stride, 0, par1, par2, nullptr, cap, state, norm, mx, norm_new, mx_new, positions,
@@ -955,7 +974,7 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
                                                    mode == LIGHT ? 0 : aux1_stride, state, positions, seq_row0, seq_slots, n_seq, H, dk, dv,
                                                    apart, st);
     if (rc) return rc;
-    short_rows = true;
+    if (apart <= SHORT) short_rows = true;
   }
   if (!form || apart) {
     const int R = short_rows ? scan_channels(dk, dv, H, n_seq, n_seq) : scan_channels(dk, dv, H, n_seq, rows);

@@ -253,9 +253,15 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 
 // chunked: portions go sixteen tokens at a time through the matrix cores (chunk_scan.hip, where the shapes allow it).  Its workgroups have a
-// compute unit to themselves and a pipeline to fill, so among more than APART_FROM sequences those of at most SHORT rows stay with this
-// file's kernel (12 portions of 39 rows, 32 heads: 31 us against 51 there).
-constexpr int SHORT = 48, APART_FROM = 8;
+// compute unit to themselves and a pipeline to fill, so among more than APART_FROM sequences the short ones stay with this file's kernel: those
+// of at most 48 rows while the workgroups find a place each (12 portions of 39 rows, 32 heads: 31 us against 51 there), longer ones when they
+// wait for each other (64 columns, this file's time and that one's: 11 portions of 100 rows, 16 heads 35, 41; 128 rows 42, 41; 16 portions of 128
+// rows, 64 heads 158, 162; 200 rows 242, 222).
+constexpr int APART_FROM = 8;
+static int apart_rows(int n_seq, int heads, int dv) {
+  const long units = (long)n_seq * heads * ((dv + 63) / 64);
+  return n_seq <= APART_FROM ? 0 : units <= 128 ? 48 : units <= 256 ? 112 : 144;
+}
 
 // Segments (of *seg_rows rows) that a chunked step's portions are cut into (1: whole portions).  rows - n_seq + 1 bounds the longest portion.
 // Two passes over a segment take 2 (seg_rows / 16 + 5) chunks' time and the state pass some 10 us, one over a whole portion
@@ -284,7 +290,7 @@ extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const vo
   int most = 0;
   const float* B = xbc + (size_t)heads * dv;
   if (chunked && dgi_chunk_scan_ok(5, N, B + (size_t)G * N, xbc_stride, B, xbc_stride, 1)) {
-    most = n_seq > APART_FROM ? SHORT : 0;
+    most = apart_rows(n_seq, heads, dv);
     const int rc = dgi_chunk_scan(y, 5, B + (size_t)G * N, xbc_stride, B, xbc_stride, xbc, xbc_stride, 1, dt_raw, dt_stride, nullptr, 0,
                                   !dt_f32, a_log, dt_bias, d_skip, 0.f, state, nullptr, nullptr, nullptr, nullptr, positions, seq_row0,
                                   seq_slots, n_seq, heads, G, N, dv, most, segs, seg_rows, ws, wsd, s);

@@ -194,9 +194,21 @@ def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, se
         T, n_seq = xbc.shape[0], seq_slots.shape[0]
         y = torch.empty(T, heads * dv, dtype=torch.float32, device=xbc.device)
         if chunked is None:
-            # a third of the time per row, but some 80 rows' time more per portion and a second launch beside decode rows (12
-            # portions of 39 rows, 32 heads: 51 us against 32 row by row); known here are the step's rows and sequences only
-            chunked = SCAN_CHUNK > 0 and (T > 64 * n_seq or T - n_seq >= 512)
+            # a third of the time per row, but some 80 rows' time more per portion, and once the heads outnumber the
+            # pipelines that find a place on the chip they wait for each other: 64 columns, row by row against chunks, 4
+            # portions, 16 heads, 72 rows 21, 18 us; 64 heads, 72 rows 32, 36, 128 rows 50, 43; 11 portions, 64 heads, 128
+            # rows 114, 122, 200 rows 180, 171.  Known here are the step's rows and sequences only; among more than eight
+            # each sequence is taken by its own length, and few rows on average but many rows are decode rows beside
+            # long portions
+            units = n_seq * heads * -(-dv // 64)
+            rows = 64 if units <= 128 else 112 if units <= 256 else 144
+            if rows == 64:
+                chunked = T > 64 * n_seq or T - n_seq >= 512
+            elif n_seq <= 8:
+                chunked = T > rows * n_seq
+            else:
+                chunked = 4 * T > 3 * rows * n_seq or (T - n_seq >= 512 and T <= 48 * n_seq)
+            chunked = chunked and SCAN_CHUNK > 0
         _call("ssm_scan", y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G, bool(chunked))
         return y
     return ssm_scan_ref(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G)

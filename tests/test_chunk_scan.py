@@ -145,7 +145,7 @@ MODES = ["wkv", "delta", "mlstm", "light", "ssm"]
 def test_lengths(mode, lens):
     """Ends inside a chunk, at its edge and after an odd number of chunks; short sequences beside long ones in one launch (up to eight
     sequences) and in one of their own; every second sequence continues a state."""
-    H = 12 if mode == "light" and len(lens) < 3 else 6          # light: enough workgroups (or rows) for either of its kernels
+    H = (200 if len(lens) < 3 else 70) if mode == "light" else 6        # light: enough workgroups (or rows) for either of its kernels
     d = make(mode, lens, H, 64, 64, torch.float32, [3 * (i % 2) for i in range(len(lens))])
     check(call(d, **({"chunked": True} if mode == "ssm" else {})), oracle(d))
 
@@ -156,8 +156,9 @@ def test_sizes(mode, D, V):
     """Key sizes below, at and above a 64-channel group, value sizes of one, two and three 16-column blocks and odd ones; bf16 rows."""
     if mode == "wkv":
         V = D
-    H = 96 if mode == "light" else 4
-    d = make(mode, [70, 66], H, D, V, torch.bfloat16, [5, 0])
+    light = mode == "light"
+    H = 400 // -(-V // 16) + 1 if light else 4
+    d = make(mode, [170, 166] if light else [70, 66], H, D, V, torch.bfloat16, [5, 0])
     check(call(d, **({"chunked": True} if mode == "ssm" else {})), oracle(d))
 
 
@@ -206,8 +207,8 @@ def test_delta_repeated_keys():
 @pytest.mark.parametrize("mode", MODES)
 def test_non_finite_values_stay_behind(mode):
     """An infinity or NaN in a token's value reaches that token's column from that token on, and nothing before it."""
-    lens, t = [130], 71                                  # inside a chunk
-    H = 96 if mode == "light" else 4
+    lens, t = [170 if mode == "light" else 130], 71      # inside a chunk
+    H = 200 if mode == "light" else 4
     kw = {"chunked": True} if mode == "ssm" else {}
     clean = make(mode, lens, H, 64, 64, torch.float32, [0])
     want = call(clean, **kw)[0]
