@@ -115,6 +115,9 @@ int dgi_latent_attn_rows(const void* q, int q_stride, const void* q_lat, long lo
                          int window, const float* cos_sin, int dims, int interleaved, void* out, long long o_hs,
                          long long o_ts, int is_f32, int nsplit, float* part_o, float* part_ml, int mfma, const float* sinks,
                          hipStream_t s);
+int dgi_latent_fold(void* q_lat, const void* q, int q_stride, const void* uk, int T, int H, int dim, int qk, int kr, hipStream_t s);
+int dgi_latent_values(void* out, const void* o_lat, const float* part, const float* ml, int runs, const float* sinks,
+                      const void* uv, const void* gate, int gate_stride, int per_head, int T, int H, int vdim, hipStream_t s);
 int dgi_glu_silu(void* out, const void* gu, int gu_stride, int rows, int I, int is_f32, hipStream_t s);
 int dgi_moe_expert_gate_up(float* mid, const void* h, int h_stride, const int* idx, const void* gate_up, int T, int E,
                            int top, int ff, int W, const float* pair_scale, int act, float limit, float alpha, int is_f32,
@@ -723,7 +726,7 @@ void latent_attn_rows(at::Tensor out, const at::Tensor& q, const at::Tensor& q_l
                       int64_t H, int64_t dim, int64_t rot_dim, int64_t kv_rank, double scale, int64_t window,
                       const c10::optional<at::Tensor>& cos_sin, bool interleaved, int64_t nsplit,
                       c10::optional<at::Tensor> part_o, c10::optional<at::Tensor> part_ml, bool mfma,
-                      const c10::optional<at::Tensor>& sinks) {
+                      const c10::optional<at::Tensor>& sinks, bool combine) {
   const int f = act_kind(q, "q");
   float *pop = nullptr, *pmp = nullptr;
   TORCH_CHECK(nsplit >= 1, "latent_attn_rows: nsplit >= 1");
@@ -766,8 +769,49 @@ void latent_attn_rows(at::Tensor out, const at::Tensor& q, const at::Tensor& q_l
                                 (long long)q_lat.stride(1), cache.data_ptr(), block_tables.data_ptr<int>(),
                                 (int)block_tables.stride(0), cu, n_seqs, i32p(positions, "positions", T), T, (int)H, (int)dim,
                                 (int)rot_dim, (int)kv_rank, (int)cache.size(2), (float)scale, (int)window, csp, dims,
-                                interleaved ? 1 : 0, out.data_ptr(), (long long)out.stride(0), (long long)out.stride(1), f,
+                                interleaved ? 1 : 0, combine || nsplit == 1 ? out.data_ptr() : nullptr, (long long)out.stride(0),
+                                (long long)out.stride(1), f,
                                 (int)nsplit, pop, pmp, mfma ? 1 : 0, f32p(sinks, "sinks", H), cur_stream()), "latent_attn_rows");
+}
+
+void latent_fold(at::Tensor q_lat, const at::Tensor& q, const at::Tensor& uk) {
+  TORCH_CHECK(act_kind(q, "q") == 0 && act_kind(uk, "uk") == 0 && act_kind(q_lat, "q_lat") == 0, "latent_fold: bfloat16 only");
+  check_rows(q, "q");
+  TORCH_CHECK(uk.dim() == 3 && uk.is_contiguous(), "latent_fold: uk must be contiguous [H, dim, kv_rank]");
+  const int64_t H = uk.size(0), dim = uk.size(1), kr = uk.size(2), T = q.size(0);
+  TORCH_CHECK(q.size(1) % H == 0 && q.size(1) / H >= dim, "latent_fold: q must be [T, H * (dim + rot_dim)]");
+  TORCH_CHECK(q_lat.is_contiguous() && q_lat.dim() == 3 && q_lat.size(0) == H && q_lat.size(1) == T && q_lat.size(2) == kr);
+  check_rc(dgi_latent_fold(q_lat.data_ptr(), q.data_ptr(), (int)q.stride(0), uk.data_ptr(), (int)T, (int)H, (int)dim,
+                           (int)(q.size(1) / H), (int)kr, cur_stream()), "latent_fold");
+}
+
+void latent_values(at::Tensor out, const c10::optional<at::Tensor>& o_lat, const c10::optional<at::Tensor>& part_o,
+                   const c10::optional<at::Tensor>& part_ml, int64_t runs, const c10::optional<at::Tensor>& sinks, const at::Tensor& uv,
+                   const c10::optional<at::Tensor>& gate, bool per_head) {
+  TORCH_CHECK(act_kind(out, "out") == 0 && act_kind(uv, "uv") == 0, "latent_values: bfloat16 only");
+  TORCH_CHECK(uv.dim() == 3 && uv.is_contiguous() && uv.size(2) == 512, "latent_values: uv must be contiguous [H, vdim, 512]");
+  const int64_t H = uv.size(0), vdim = uv.size(1), T = out.size(0);
+  TORCH_CHECK(out.dim() == 2 && out.is_contiguous() && out.size(1) == H * vdim, "latent_values: out must be [T, H * vdim]");
+  const void *op = nullptr, *gp = nullptr;
+  const float *pp = nullptr, *mp = nullptr;
+  int gs = 0;
+  if (runs > 1) {
+    TORCH_CHECK(part_o.has_value() && part_ml.has_value(), "latent_values: runs need their sums");
+    check_f32(*part_o, "part_o", runs * H * T * 512);
+    check_f32(*part_ml, "part_ml", runs * H * T * 2);
+    pp = part_o->data_ptr<float>(); mp = part_ml->data_ptr<float>();
+  } else {
+    TORCH_CHECK(o_lat.has_value() && act_kind(*o_lat, "o_lat") == 0 && o_lat->is_contiguous() && o_lat->numel() == H * T * 512);
+    op = o_lat->data_ptr();
+  }
+  if (gate.has_value()) {
+    check_rows(*gate, "gate");
+    TORCH_CHECK(act_kind(*gate, "gate") == 0 && gate->size(0) == T && gate->size(1) == (per_head ? H : H * vdim),
+                "latent_values: gate must be [T, H] (per head) or [T, H * vdim]");
+    gp = gate->data_ptr(); gs = (int)gate->stride(0);
+  }
+  check_rc(dgi_latent_values(out.data_ptr(), op, pp, mp, (int)runs, runs > 1 ? f32p(sinks, "sinks", H) : nullptr, uv.data_ptr(), gp, gs,
+                             per_head ? 1 : 0, (int)T, (int)H, (int)vdim, cur_stream()), "latent_values");
 }
 
 void rotate_heads(at::Tensor x, const at::Tensor& positions, const at::Tensor& cos_sin, bool interleaved, int64_t H,
@@ -1182,7 +1226,11 @@ TORCH_LIBRARY_FRAGMENT(dgi, m) {
         "Tensor positions, Tensor slots, Tensor? cos_sin, bool interleaved, Tensor(b!)? cache) -> ()");
   m.def("latent_attn_rows(Tensor(a!) out, Tensor q, Tensor q_lat, Tensor cache, Tensor block_tables, Tensor? cu_seqlens, "
         "Tensor positions, int H, int dim, int rot_dim, int kv_rank, float scale, int window, Tensor? cos_sin, "
-        "bool interleaved, int nsplit=1, Tensor(b!)? part_o=None, Tensor(c!)? part_ml=None, bool mfma=False, Tensor? sinks=None) -> ()");
+        "bool interleaved, int nsplit=1, Tensor(b!)? part_o=None, Tensor(c!)? part_ml=None, bool mfma=False, Tensor? sinks=None, "
+        "bool combine=True) -> ()");
+  m.def("latent_fold(Tensor(a!) q_lat, Tensor q, Tensor uk) -> ()");
+  m.def("latent_values(Tensor(a!) out, Tensor? o_lat, Tensor? part_o, Tensor? part_ml, int runs, Tensor? sinks, Tensor uv, Tensor? gate, "
+        "bool per_head) -> ()");
   m.def("rotate_heads(Tensor(a!) x, Tensor positions, Tensor cos_sin, bool interleaved, int H, int head_size, int offset) -> ()");
   m.def("latent_pages(Tensor(a!) kt, Tensor(b!) vt, Tensor kv, Tensor lat, int rd) -> ()");
   m.def("gate_heads(Tensor(a!) out, Tensor ov, Tensor? gate, bool per_head) -> ()");
@@ -1231,6 +1279,8 @@ TORCH_LIBRARY_IMPL(dgi, CUDA, m) {
   m.impl("stream_add_norm", &stream_add_norm);
   m.impl("latent_prep", &latent_prep);
   m.impl("latent_attn_rows", &latent_attn_rows);
+  m.impl("latent_fold", &latent_fold);
+  m.impl("latent_values", &latent_values);
   m.impl("rotate_heads", &rotate_heads);
   m.impl("latent_pages", &latent_pages);
   m.impl("gate_heads", &gate_heads);

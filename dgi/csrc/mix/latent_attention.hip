@@ -868,7 +868,7 @@ int launch(const void* q, int q_stride, const void* q_lat, long long ql_hs, long
       (const T*)q, q_stride, (const T*)q_lat, ql_hs, ql_ts, (const T*)cache, block_tables, bt_stride, cu_seqlens, n_seqs,
       positions, H, dim, rd, kr, bs, scale, window, cos_sin, dims, interleaved, (T*)out, o_hs, o_ts, DP, DQ,
       nsplit > 1 ? part_o : nullptr, part_ml, sinks);
-  if (nsplit > 1)
+  if (nsplit > 1 && out)
     launch_reduce<T>(part_o, part_ml, nsplit, rows, H, kr, (T*)out, o_hs, o_ts, sinks, s);
   return 0;
 }
@@ -898,7 +898,7 @@ int launch_mfma(const void* q, int q_stride, const void* q_lat, long long ql_hs,
       (const uint16_t*)q, q_stride, (const uint16_t*)q_lat, ql_hs, ql_ts, (const uint16_t*)cache, block_tables, bt_stride,
       cu_seqlens, n_seqs, positions, H, dim, rd, kr, bs, scale, window, cos_sin, dims, interleaved, DP, (uint16_t*)out, o_hs,
       o_ts, nsplit > 1 ? part_o : nullptr, part_ml, magic, sinks);
-  if (nsplit > 1)
+  if (nsplit > 1 && out)
     launch_reduce<uint16_t>(part_o, part_ml, nsplit, rows, H, kr, (uint16_t*)out, o_hs, o_ts, sinks, s);
   return 0;
 }
@@ -923,7 +923,7 @@ int launch_tiles(const void* q, int q_stride, const void* q_lat, long long ql_hs
       (const uint16_t*)q, q_stride, (const uint16_t*)q_lat, ql_hs, ql_ts, (const uint16_t*)cache, block_tables, bt_stride,
       cu_seqlens, n_seqs, positions, H, dim, bs, scale, window, cos_sin, dims, interleaved, (uint16_t*)out, o_hs, o_ts,
       nsplit > 1 ? part_o : nullptr, part_ml, sinks);
-  if (nsplit > 1) launch_reduce<uint16_t>(part_o, part_ml, nsplit, rows, H, KR, (uint16_t*)out, o_hs, o_ts, sinks, s);
+  if (nsplit > 1 && out) launch_reduce<uint16_t>(part_o, part_ml, nsplit, rows, H, KR, (uint16_t*)out, o_hs, o_ts, sinks, s);
   return 0;
 }
 
@@ -933,7 +933,7 @@ int launch_tiles(const void* q, int q_stride, const void* q_lat, long long ql_hs
 // cache [NB, 1, bs, kr + rd]; cu_seqlens (n_seqs + 1 row offsets) maps rows to block-table rows, nullptr: row i
 // uses table row i.  Workgroups are sized so that the grid covers the chip where the step allows; nsplit > 1 cuts
 // every row's keys into that many runs (steps of few rows over long contexts) whose partial results, in
-// part_o [nsplit, H, rows, kr] and part_ml [nsplit, H, rows, 2] (fp32), a second kernel combines.
+// part_o [nsplit, H, rows, kr] and part_ml [nsplit, H, rows, 2] (fp32), a second kernel combines (out nullptr: the caller does).
 extern "C" int dgi_latent_attn_rows(const void* q, int q_stride, const void* q_lat, long long ql_hs, long long ql_ts,
                                     const void* cache, const int* block_tables, int bt_stride, const int* cu_seqlens,
                                     int n_seqs, const int* positions, int rows, int H, int dim, int rd, int kr,
@@ -942,6 +942,7 @@ extern "C" int dgi_latent_attn_rows(const void* q, int q_stride, const void* q_l
                                     float* part_o, float* part_ml, int mfma, const float* sinks, hipStream_t s) {
   if (rows == 0) return 0;
   if (H <= 0 || kr <= 0 || rd < 0 || dim < 0 || window < 0) return -2;
+  if (!out && nsplit == 1) return -7;
   if (nsplit < 1 || nsplit > 65535 || (nsplit > 1 && (!part_o || !part_ml)) || H > 65535) return -7;
   if (mfma) {
     if (is_f32 || kr % 16 || (kr + rd) % 16 || kr > 512 || kr + rd > 576 || ((uintptr_t)cache & 15)) return -8;

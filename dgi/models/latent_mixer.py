@@ -5,7 +5,8 @@ rows ``[c | r]`` of the layer that owns the latent, and returns the heads' outpu
 
 * decode rows, short portions, fp32 and geometries the matrix kernel does not take: the unrotated query part is
   folded through the key up-projection by a batched product over heads, ``latent_attn_rows`` (HIP) attends over
-  the cached rows themselves and a batched product takes the weighted latent sums to values;
+  the cached rows themselves and a batched product takes the weighted latent sums to values (decode rows in bf16 on 512 + 64
+  dims: ``latent_decode_heads``, the same three parts with kernels of their own around the attention);
 * long portions in bf16: the pages a portion can see (its window, or its whole context) are expanded once into
   per-head keys ``[U_k c | r]`` and values ``U_v c`` (one GEMM, ``latent_pages``), and the MFMA flash kernel runs on
   them: (dim + rot_dim + vdim) MACs per query, key and head instead of the 2 kv_rank + rot_dim of the folded form.
@@ -117,9 +118,13 @@ def latent_heads(m, up: LatentUp, q: torch.Tensor, cache: torch.Tensor, meta: At
     def put(ov, lo, hi):
         latent.gate_heads(ov, None if gate is None else gate[lo:hi], per_head, out=out[lo:hi])
 
-    if nd > 0:
+    max_keys = meta.dec_block_tables.shape[1] * cache.shape[2] if nd > 0 else 0
+    if nd > 0 and latent.decode_heads_ok(q, nd, m.dim, m.rot_dim, m.kv_rank, m.vdim, gate):
+        latent.latent_decode_heads(q[:nd], up.uk, up.uv, cache, meta.dec_block_tables, meta.positions[:nd], m.rot_dim, m.scale, m.window,
+                                   cos_sin, inter, out[:nd], max_keys, sinks, None if gate is None else gate[:nd], per_head)
+    elif nd > 0:
         put(_rows(m, up, q[:nd], cache, meta.dec_block_tables, None, meta.positions[:nd], cos_sin, inter, sinks,
-                  meta.dec_block_tables.shape[1] * cache.shape[2]), 0, nd)
+                  max_keys), 0, nd)
     if meta.num_prefill_tokens >= MFMA_PROMPT_ROWS and mfma_prompt_ok(m, q):
         prompt_heads(m, up, q[nd:], cache, meta, cos_sin, inter, sinks, None if gate is None else gate[nd:], per_head, out[nd:])
     elif meta.num_prefill_tokens > 0:

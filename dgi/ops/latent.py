@@ -240,6 +240,41 @@ def latent_attn_rows(q: torch.Tensor, q_lat: torch.Tensor, cache: torch.Tensor, 
     return out
 
 
+# rows up to which latent_decode_heads is the faster form: every 16 rows read uv again (32 heads over 300 keys, the layer's part: 1 row
+# 29 us against 41, 256 rows 56 and 60, 384 rows 89 and 87)
+DECODE_HEADS_ROWS = 256
+
+
+def decode_heads_ok(q: torch.Tensor, rows: int, dim: int, rot_dim: int, kv_rank: int, vdim: int, gate=None) -> bool:
+    """Whether ``rows`` decode rows of this geometry take ``latent_decode_heads``: few of them, bf16, 512 + 64 dims, rows and
+    heads in whole 16-byte chunks."""
+    return (q.is_cuda and q.dtype == torch.bfloat16 and MFMA_ROWS and 0 < rows <= DECODE_HEADS_ROWS and kv_rank == 512 and rot_dim == 64
+            and dim % 32 == 0 and 0 < dim <= 128 and vdim % 16 == 0 and 0 < vdim <= 128 and q.stride(1) == 1 and q.stride(0) % 8 == 0
+            and q.data_ptr() % 16 == 0 and (gate is None or gate.dtype == torch.bfloat16))
+
+
+def latent_decode_heads(q, uk, uv, cache, block_tables, positions, rot_dim: int, scale: float, window: int, cos_sin, interleaved: bool,
+                        out, max_keys: int = 0, sinks=None, gate=None, per_head: bool = False) -> torch.Tensor:
+    """Head outputs ``out`` [T, H * vdim] of decode rows on cached latents (``decode_heads_ok``): ``q`` [T, H * (dim + rot_dim)], the key
+    and value up-projections ``uk`` [H, dim, 512] and ``uv`` [H, vdim, 512], the rest as ``latent_attn_rows`` and ``gate_heads``.  Three
+    launches: queries folded, attention in runs of keys, and one that combines the runs, takes the sums to values and applies
+    the gate.  32 rows of 32 heads, 8 runs: 4.5 and 10.8 us around the attention's 35; the library's products, the combining pass
+    and the one that puts the heads side by side took 28."""
+    _native(q)
+    T, (H, dim, kr) = q.shape[0], uk.shape
+    q_lat, o_lat = (torch.empty(H, T, kr, dtype=q.dtype, device=q.device) for _ in range(2))
+    runs = tile_runs(T, H, min(max_keys, window) if window > 0 and max_keys > 0 else max_keys)
+    po = pm = None
+    if runs > 1:
+        po = torch.empty(runs * H * T * kr, dtype=torch.float32, device=q.device)
+        pm = torch.empty(runs * H * T * 2, dtype=torch.float32, device=q.device)
+    _call("latent_fold", q_lat, q, uk)
+    _call("latent_attn_rows", o_lat, q, q_lat, cache, block_tables, None, positions, H, dim, int(rot_dim), kr, float(scale), int(window),
+          cos_sin, bool(interleaved), runs, po, pm, True, sinks, False)
+    _call("latent_values", out, o_lat, po, pm, runs, sinks, uv, gate, bool(per_head))
+    return out
+
+
 def latent_pages_ref(kv, lat, bs, H, dim, rot_dim, vdim):
     n = lat.shape[0] // bs
     k = kv[:, :H * dim].view(n, bs, H, dim).permute(0, 2, 1, 3)
