@@ -662,7 +662,7 @@ __global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
   const int t_lo = blockIdx.z * tps, t_hi = min(ntiles, t_lo + tps);
 
   // loads of a tile: lane j knows the slot of its row j; load `it` of a wave brings chunks 64 it + lane of the wave's rows
-  auto key_of = [&](int ti) { return min(first + ti * KT + lane, pos); };
+  auto key_of = [&](int ti) { return max(0, min(first + ti * KT + lane, pos)); };
   auto issue = [&](int st, int slots) {
 #pragma unroll
     for (int it = 0; it < RPW * CPR / 64; ++it) {
