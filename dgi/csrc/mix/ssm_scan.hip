@@ -21,6 +21,8 @@
 //
 // gated_group_norm: g = y * silu(z), each of `groups` equal parts of a row divided by its own root
 // mean square (eps inside the root), times w.
+#include <algorithm>
+
 #include "../common.h"
 
 using namespace dgi;
@@ -265,18 +267,21 @@ static int apart_rows(int n_seq, int heads, int dv) {
 
 // Segments (of *seg_rows rows) that a chunked step's portions are cut into (1: whole portions).  rows - n_seq + 1 bounds the longest portion.
 // Two passes over a segment take 2 (seg_rows / 16 + 5) chunks' time and the state pass some 10 us, one over a whole portion
-// rows / 16 + 5: worth it from about 512 rows on while the workgroups (32 columns of a head) leave half of the chip idle (1444 rows, 16 heads of
-// 48 columns, state 128: see chunk_scan.hip).
+// rows / 16 + 5: worth it from about 512 rows on while the workgroups (32 columns of a head) leave half of the chip idle.  Every segment's
+// workgroups have a compute unit to themselves, so the rows are shared out over 256 of them, less one segment for each portion that may end in a
+// part of one; a second round of workgroups costs more than shorter segments give (1444 rows, 16 heads of 64: whole 123 us, 11 segments
+// 82, 8 segments 50; 2 x 2000 rows whole 166, 6 of 672 117, 7 of 576 101).  At most 24 segments, of 64 rows at least: the state pass goes through them one by one.
 extern "C" int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg_rows) {
-  const long groups = (long)n_seq * heads * ((dv + 31) / 32);
+  const long one = (long)heads * ((dv + 31) / 32), groups = n_seq * one;
   const int longest = rows - n_seq + 1;
   *seg_rows = 0;
   if (groups <= 0 || groups > 128 || longest < 512) return 1;
-  const long fit = 384 / groups, most = longest / 128;
-  const int segs = (int)(fit < most ? fit : most);
+  const long places = 256 - (n_seq - 1) * one;
+  const long share = std::max({64l, (rows * one + places - 1) / places, (longest + 23l) / 24});
+  const int each = (int)((share + 15) / 16 * 16), segs = (longest + each - 1) / each;
   if (segs < 3) return 1;
-  *seg_rows = (longest / segs + 15) / 16 * 16;
-  return (longest + *seg_rows - 1) / *seg_rows;
+  *seg_rows = each;
+  return segs;
 }
 
 extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const void* dt_raw, int dt_f32, int dt_stride,
