@@ -127,8 +127,10 @@ struct Lay {
   static constexpr int SETS = CH && NT == 4 ? 2 : 1;           // channel decays: one set of preparing waves for the scores, one for the state
   static constexpr int PREPS = (TURNS ? 2 : 1) * NS * SETS;    // preparing waves, EARLY of them before the scores waves
   static constexpr int EARLY = NC == 1 ? 0 : (CH ? 2 : (MODE == MLSTM ? 0 : 1));
-  static constexpr int OUT = NC, GATES = 2 * NC, NORM = GATES + 1, SCORES = NC == 1 ? 4 : 6, PREP = SCORES + W2;
+  static constexpr int OUT = NC, GATES = 2 * NC, NORM = GATES + 1, SCORES = NC == 1 ? 3 : 6, PREP = SCORES + W2;
   static constexpr int WAVES = PREP + PREPS - EARLY;
+  // every wave has one role: a wave left over would run as an output wave of columns that are another workgroup's
+  static_assert(SCORES - EARLY == (CH ? GATES : MODE == MLSTM ? NORM + 1 : GATES + 1), "state, output, gates, normaliser, preparing, scores");
   static constexpr int LEAD = 2 + W2 + (TURNS ? 1 : 0);        // steps before the first output
   static constexpr int DP = 16 * NT, QR = DP + 4, ROWS = C * QR;
   static constexpr int QB = 3 + W2, KB = 2 + W2;               // buffers of q and k

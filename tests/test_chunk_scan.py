@@ -221,3 +221,12 @@ def test_non_finite_values_stay_behind(mode):
         cols[3] = False
         assert torch.isfinite(got[:, cols]).all()
         assert not torch.isfinite(got[t, 3])
+
+
+@pytest.mark.parametrize("D,V", [(132, 33), (200, 48), (256, 64), (256, 100)])
+def test_ssm_large_states(D, V):
+    """Key sizes of 129 to 256 (one column block per workgroup, so every wave beyond the roles of one would write another's columns):
+    one, two and more blocks of columns, whole portions, segments, and short sequences in a launch of their own."""
+    for lens in ([70, 66], [700, 33], [1] * 9 + [120]):
+        d = make("ssm", lens, 2, D, V, torch.float32, [3 * (i % 2) for i in range(len(lens))], seed=D + V)
+        check(call(d, chunked=True), oracle(d))
