@@ -498,6 +498,7 @@ void ssm_scan(at::Tensor y, const at::Tensor& xbc, const at::Tensor& dt_raw, con
   at::Tensor ws, wsd;
   if (chunked && n_seq > 0) segs = dgi_ssm_segments(n_seq, (int)heads, (int)dv, T, &seg_rows);
   if (segs > 1) {
+    TORCH_CHECK((int64_t)segs * seg_rows >= T, "ssm_scan: the segments must cover the longest portion");
     ws = at::empty({n_seq, segs, heads, dv, N}, state.options());
     wsd = at::empty({n_seq, segs, heads}, state.options());
   }

@@ -265,7 +265,8 @@ static int apart_rows(int n_seq, int heads, int dv) {
   return n_seq <= APART_FROM ? 0 : units <= 128 ? 48 : units <= 256 ? 112 : 144;
 }
 
-// Segments (of *seg_rows rows) that a chunked step's portions are cut into (1: whole portions).  rows - n_seq + 1 bounds the longest portion.
+// Segments (of *seg_rows rows) that a chunked step's portions are cut into (1: whole portions).  Together they are as long as the step: a portion
+// may have all of its rows, beside sequences without any.
 // Two passes over a segment take 2 (seg_rows / 16 + 5) chunks' time and the state pass some 10 us, one over a whole portion
 // rows / 16 + 5: worth it from about 512 rows on while the workgroups (32 columns of a head) leave half of the chip idle.  Every segment's
 // workgroups have a compute unit to themselves, so the rows are shared out over 256 of them, less one segment for each portion that may end in a
@@ -273,12 +274,11 @@ static int apart_rows(int n_seq, int heads, int dv) {
 // 82, 8 segments 50; 2 x 2000 rows whole 166, 6 of 672 117, 7 of 576 101).  At most 24 segments, of 64 rows at least: the state pass goes through them one by one.
 extern "C" int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg_rows) {
   const long one = (long)heads * ((dv + 31) / 32), groups = n_seq * one;
-  const int longest = rows - n_seq + 1;
   *seg_rows = 0;
-  if (groups <= 0 || groups > 128 || longest < 512) return 1;
+  if (groups <= 0 || groups > 128 || rows - n_seq + 1 < 512) return 1;
   const long places = 256 - (n_seq - 1) * one;
-  const long share = std::max({64l, (rows * one + places - 1) / places, (longest + 23l) / 24});
-  const int each = (int)((share + 15) / 16 * 16), segs = (longest + each - 1) / each;
+  const long share = std::max({64l, (rows * one + places - 1) / places, (rows + 23l) / 24});
+  const int each = (int)((share + 15) / 16 * 16), segs = (rows + each - 1) / each;
   if (segs < 3) return 1;
   *seg_rows = each;
   return segs;

@@ -230,3 +230,11 @@ def test_ssm_large_states(D, V):
     for lens in ([70, 66], [700, 33], [1] * 9 + [120]):
         d = make("ssm", lens, 2, D, V, torch.float32, [3 * (i % 2) for i in range(len(lens))], seed=D + V)
         check(call(d, chunked=True), oracle(d))
+
+
+@pytest.mark.parametrize("lens", [[0, 577], [577, 0], [0, 0, 1500, 0], [600, 0, 70]])
+def test_ssm_segments_beside_sequences_without_rows(lens):
+    """Empty sequences leave a portion longer than rows - sequences + 1: its last rows and its state are there all the same, and the
+    empty ones keep their states."""
+    d = make("ssm", lens, 1, 128, 32, torch.bfloat16, [4 if n == 0 else 0 for n in lens], seed=len(lens))
+    check(call(d, chunked=True), oracle(d))
