@@ -29,7 +29,13 @@
 // by k, substitution, update) or a preparing wave's arithmetic (wkv): a wave issues an instruction every four to five cycles at best, so
 // addresses are lane offsets kept in registers, and rows past the end a branch of their own.  Measured, a step of 2 prompts of 4096 rows in
 // all, 64 heads, states 64 x 64 (ssm 128 x 64), against the same token by token on the vector ALUs (linear_scan.hip, ssm_scan.hip):
-// delta 173 us (726), ssm 196 (637), wkv 250 (some 630), light 167 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 92 (322).
+// delta 178 us (726), ssm 209 (637), wkv 230 (some 630), light 158 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 105 (322).
+//
+// Precision: results and states are no further from 64 bits than the token loop's (2-norm over 1300 to 4096 rows: ssm 7.8e-8, the loop 8.0e-8;
+// delta 1.17e-7, 1.18e-7; wkv 9.8e-8, 1.01e-7).  Regrouping alone does not do that: with the sums over channels in two running sums, P and the decays
+// rounded product by product and P u in 32 bits the same were 1.25e-7, 1.57e-7 and 1.30e-7.  So sums over channels are added as trees, a sum over
+// tokens starts with the oldest, the per-token decays and wkv's suffix products carry their rounding errors along, and P and P u are 64-bit
+// (four v_mfma_f64_16x16x4_f64 per chunk and output wave).  It costs 3 (delta) to 13 % (mlstm) of the time; wkv's was not the longest role.
 //
 // Half-chunk products of channel decays below 1e-28 leave the range of the scaled operands; the wave that prepares such channels
 // then sums their scores token by token instead.  An infinity or NaN among a chunk's u takes a path that keeps it from the tokens
@@ -43,8 +49,10 @@ namespace {
 
 constexpr int WKV = 0, DELTA = 1, MLSTM = 2, LIGHT = 4, SSM = 5;      // 3: gla, chunk_scan_decay.hip
 constexpr int C = 16;              // tokens per chunk
-constexpr int TR = 20;             // padded row of sixteen tokens
+constexpr int TR = 20, PR = 18;    // padded rows of sixteen tokens; in 64 bits
 constexpr float SAFE = 1e-28f;
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 struct ChunkArgs {
   float* y;                        // [T, H * dv]
@@ -122,6 +130,8 @@ struct Lay {
   static constexpr bool TURNS = CH || MODE == LIGHT;           // two sets of preparing waves take turns, two steps a chunk
   static constexpr int NC = NT <= 8 ? 2 : 1, W2 = NT <= 8 ? 2 : 1;
   static constexpr int NS = NT / 4;                            // preparing waves of 64 channels
+  static constexpr int NA = NT == 4 ? 4 : 8;                   // sums side by side of a sum over the channels: state waves
+  static constexpr int NO = MODE == WKV ? 8 : 4;               // output waves
   // Waves: state, output, then gates and normaliser (or preparing waves), scores, (more) preparing waves: waves four apart share a SIMD,
   // and the scores' products are best beside the output waves', the fewest.
   static constexpr int SETS = CH && NT == 4 ? 2 : 1;           // channel decays: one set of preparing waves for the scores, one for the state
@@ -135,14 +145,14 @@ struct Lay {
   static constexpr int DP = 16 * NT, QR = DP + 4, ROWS = C * QR;
   static constexpr int QB = 3 + W2, KB = 2 + W2;               // buffers of q and k
   static constexpr int Q = 0;                                  // [QB][16][QR] q (channel decays: times the prefix products)
-  static constexpr int K = Q + QB * ROWS;                      // [KB][16][QR] k; channel decays: [2][16][QR] scaled for the scores
+  static constexpr int K = Q + QB * ROWS;                      // [KB][16][QR] k, rows by place (read by its tokens: no bank twice); channel decays: [2][16][QR] scaled for the scores
   static constexpr int QT = K + (CH ? 2 : KB) * ROWS;          // CH: [2][16][QR] q scaled for the scores
   static constexpr int KT = QT + (CH ? 2 * ROWS : 0);          // CH: [KB][DP][TR] k times the suffix products, by channel
   static constexpr int DEC = KT + (CH ? KB * DP * TR : 0);     // CH: [KB][DP] decay of the whole chunk
   static constexpr int ST = DEC + (CH ? KB * DP : 0);          // [2][NC][NT][64][4] state before the chunk, as the state wave holds it
   static constexpr int U = ST + 2 * NC * DP * 16;              // DELTA: [2][NC][64][4] u
-  static constexpr int P = U + (MODE == DELTA ? 2 * NC * 256 : 0);     // [4][16][TR]
-  static constexpr int M = P + 4 * C * TR;                     // DELTA: [2][16][TR]
+  static constexpr int P = U + (MODE == DELTA ? 2 * NC * 256 : 0);     // [3][16][PR] in 64 bits
+  static constexpr int M = P + 6 * C * PR;                     // DELTA: [2][16][TR]
   static constexpr int T = M + (MODE == DELTA ? 2 * C * TR : 0);       // DELTA: [2][16][TR]
   static constexpr int SC = T + (MODE == DELTA ? 2 * C * TR : 0);      // [4][96] per-token factors, see below
   static constexpr int GT = SC + (CH ? 0 : 4 * 96);            // [2][3][64] gates of 64 tokens
@@ -153,7 +163,10 @@ struct Lay {
   static constexpr int END = RAW + (CH ? 2 * NS * RAWN : 0);
 };
 // per-token factors [16] each: 0 of the state read-out, 16 of the state update, 32 delta: beta, mlstm: row sums of P, then 1 / normaliser,
-// 48 delta: -beta A / |k|, mlstm: exp(-maximum), 64 mlstm: A, 80 (one number) decay of the chunk
+// 48 delta: -beta A / |k|, mlstm: exp(-maximum), 64 mlstm: A, 80 (one number) decay of the chunk.  Where they meet the registers of u or of
+// an output they lie as those do, token t at place(t), so do the columns of P: register r of lane group g holds token 4 r + g, and a sum
+// over the tokens starts with the oldest, which under a decay are the small ones.
+__device__ __forceinline__ constexpr int place(int t) { return 4 * (t & 3) + (t >> 2); }      // its own inverse
 
 // two waves per SIMD at least: within 256 registers the products take ordinary registers, without moves to accumulation ones
 template <int MODE, typename TI, int NT>
@@ -189,6 +202,27 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
   // chunks: a load behind a branch, or one whose registers are renamed at the end of a loop, would be waited for on the spot.
   auto barriers = [&](int m) {
     for (int i = 0; i < m; ++i) __syncthreads();
+  };
+  // Products over the channels 16 i .. + 15.  A sum over all channels runs in several sums side by side that are added as a tree at the
+  // end, so that its error is a tree's.
+  auto channels = [](auto& acc, int i, const float4& x, const f32x4& y) {
+    constexpr int N = sizeof(acc) / sizeof(acc[0]);
+    const float xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[(4 * i + r) % N] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[r], y[r], acc[(4 * i + r) % N], 0, 0, 0);
+  };
+  auto zero = [](auto& acc) {
+    constexpr int N = sizeof(acc) / sizeof(acc[0]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  auto total = [](auto& acc) {
+    constexpr int N = sizeof(acc) / sizeof(acc[0]);
+#pragma unroll
+    for (int h = N / 2; h > 0; h /= 2)
+#pragma unroll
+      for (int i = 0; i < h; ++i) acc[i] += acc[i + h];
+    return acc[0];
   };
   const int prep = wave >= L::PREP ? wave - L::PREP + L::EARLY : (wave < L::SCORES && wave >= L::SCORES - L::EARLY ? wave - (L::SCORES - L::EARLY) : -1);
   if (prep >= 0) {
@@ -266,16 +300,18 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
         }
         float s[C];
         if (L::SETS == 1 || set == 1) {
-          // suffix products: the state's update
-          float run = 1.f;
+          // suffix products: the state's update (their rounding errors carried along: they would stay in the state)
+          float run = 1.f, low = 0.f;
 #pragma unroll
           for (int t = C - 1; t >= 0; --t) {
-            s[t] = k[t] * run;
-            run *= d[t];
+            s[t] = k[t] * (run + low);
+            const float next = run * d[t];
+            low = fmaf(low, d[t], fmaf(run, d[t], -next));
+            run = next;
           }
 #pragma unroll
-          for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(KT + 4 * i) = make_float4(s[4 * i], s[4 * i + 1], s[4 * i + 2], s[4 * i + 3]);
-          sm[L::DEC + (c % L::KB) * DP + ch] = run;
+          for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(KT + 4 * i) = make_float4(s[i], s[4 + i], s[8 + i], s[12 + i]);      // by place
+          sm[L::DEC + (c % L::KB) * DP + ch] = run + low;
           // prefix products: the state's read-out, before the token's own decay
           float f = 1.f;
 #pragma unroll
@@ -394,7 +430,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
             for (int x = 0; x < 4; ++x) k[i][x] = silu(k[i][x]);
         }
         float* Q = sm + L::Q + (c % L::QB) * L::ROWS + t * QR + 64 * w + 4 * j;
-        float* K = sm + L::K + (c % L::KB) * L::ROWS + t * QR + 64 * w + 4 * j;
+        float* K = sm + L::K + (c % L::KB) * L::ROWS + place(t) * QR + 64 * w + 4 * j;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           *reinterpret_cast<float4*>(Q + 16 * i) = make_float4(q[i][0], q[i][1], q[i][2], q[i][3]);
@@ -450,54 +486,79 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
     const int turn = wave - L::SCORES;
     f32x4 pa, ka;                                    // keys s = 4 g + r by queries (delta: also keys) t = n16
     float bon;
-    auto products = [&](int c) {
-      const float* Q = sm + (L::CH ? L::QT + (c & 1) * L::ROWS : L::Q + (c % L::QB) * L::ROWS);
-      const float* K = sm + L::K + (L::CH ? c & 1 : c % L::KB) * L::ROWS;
-      f32x4 pb = {0.f, 0.f, 0.f, 0.f}, kk = {0.f, 0.f, 0.f, 0.f};
-      pa = pb;
-      ka = pb;
-      bon = 0.f;
+    // delta: 1 / |k_t|, dk^-1/2 / |q_t| and 1 / |k_s| of the tokens s (beside the products: the step after is the longer one)
+    float nk, nq, ns[4];
+    auto norms = [&](int c) {
+      float sk = 0.f, sq = 0.f;
+      float* N = sm + L::NRM + (c & 3) * NS * 32;
 #pragma unroll
       for (int w = 0; w < NS; ++w) {
-        const float* R = sm + L::RAW + ((c & 1) * NS + w) * L::RAWN;
-        if constexpr (L::CH) bon += R[4 + n16];
-        if (L::CH && R[0] != 0.f) {
+        sk += N[32 * w + n16];
+        sq += N[32 * w + 16 + n16];
+      }
+      nk = 1.f / sqrtf(sk + 1e-6f);
+      nq = qscale / sqrtf(sq + 1e-6f);
+      __builtin_amdgcn_wave_barrier();
+      if (g == 0) N[n16] = nk;
+      __builtin_amdgcn_wave_barrier();
+      const float4 x = ld4(N + 4 * g);
+      ns[0] = x.x; ns[1] = x.y; ns[2] = x.z; ns[3] = x.w;
+    };
+    // Four channels are one product and the products are added as a tree (delta: two and two): this
+    // error is all columns', and P is what the results of a fast decay consist of.
+    auto products = [&](int c) {
+      const float* Q = sm + (L::CH ? L::QT + (c & 1) * L::ROWS : L::Q + (c % L::QB) * L::ROWS) + n16 * QR + 4 * g;
+      const float* K = sm + L::K + (L::CH ? (c & 1) * L::ROWS + n16 * QR : (c % L::KB) * L::ROWS + place(n16) * QR) + 4 * g;
+      pa = ka = f32x4{0.f, 0.f, 0.f, 0.f};
+      auto tiles = [&](int i0) {
+        constexpr int N = 4, PER = MODE == DELTA ? 2 : 4;
+        f32x4 ps[PER * N], ks[PER * N];
+        zero(ps);
+        zero(ks);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) pa[r] += R[20 + (4 * g + r) * C + n16];
-        } else {
+        for (int i = 0; i < N; ++i) {
+          const float4 qf = ld4(Q + 16 * (i0 + i)), kf = ld4(K + 16 * (i0 + i));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int o = n16 * QR + 64 * w + 16 * i + 4 * g;
-            const float4 qf = ld4(Q + o), kf = ld4(K + o);
-            pa = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf.x, pa, 0, 0, 0);
-            pb = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf.y, pb, 0, 0, 0);
-            pa = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf.z, pa, 0, 0, 0);
-            pb = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf.w, pb, 0, 0, 0);
-            if constexpr (MODE == DELTA) {
-              ka = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, kf.x, ka, 0, 0, 0);
-              kk = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, kf.y, kk, 0, 0, 0);
-              ka = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, kf.z, ka, 0, 0, 0);
-              kk = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, kf.w, kk, 0, 0, 0);
-            }
+          for (int r = 0; r < 4; ++r) {
+            const float qs[4] = {qf.x, qf.y, qf.z, qf.w}, kx[4] = {kf.x, kf.y, kf.z, kf.w};
+            const int o = PER * i + r % PER;
+            ps[o] = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[r], qs[r], ps[o], 0, 0, 0);
+            if constexpr (MODE == DELTA) ks[o] = __builtin_amdgcn_mfma_f32_16x16x4f32(kx[r], kx[r], ks[o], 0, 0, 0);
           }
         }
-      }
+        pa += total(ps);
+        if constexpr (MODE == DELTA) ka += total(ks);
+      };
+      if constexpr (L::CH) {
+        bon = 0.f;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pa[r] += pb[r];
-        ka[r] += kk[r];
+        for (int w = 0; w < NS; ++w) {
+          const float* R = sm + L::RAW + ((c & 1) * NS + w) * L::RAWN;
+          bon += R[4 + n16];
+          if (R[0] != 0.f) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pa[r] += R[20 + (4 * g + r) * C + n16];
+          } else {
+            tiles(4 * w);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int w = 0; w < NS; ++w) {
+          tiles(4 * w);
+          if constexpr (NT == 16) __builtin_amdgcn_sched_barrier(0);       // all tiles' products at once would not fit the registers
+        }
       }
     };
     auto finish = [&](int c) {
-      float* P = sm + L::P + (c & 3) * C * TR;
-      float p[4];
+      double* P = reinterpret_cast<double*>(sm + L::P) + (c % 3 * C + n16) * PR + g;      // s = 4 g + r at place 4 r + g
+      double p[4];
       if constexpr (L::CH) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int s = 4 * g + r;
           p[r] = s < n16 ? pa[r] : (s == n16 ? bon : 0.f);
         }
-        *reinterpret_cast<float4*>(P + n16 * TR + 4 * g) = make_float4(p[0], p[1], p[2], p[3]);
       } else {
         const float* G = sm + L::GT + ((c >> 2) & 1) * 192 + 16 * (c & 3);
         const float* DM = sm + L::DM + (c & 3) * 272;
@@ -506,41 +567,23 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
         float cf[4] = {wr.x, wr.y, wr.z, wr.w}, qs = 1.f, rk = 1.f;
         if constexpr (MODE == MLSTM) qs = qscale;
         if constexpr (MODE == DELTA) {
-          float sk = 0.f, sq = 0.f;
-          float* N = sm + L::NRM + (c & 3) * NS * 32;
+          qs = nq;
+          rk = nk;
 #pragma unroll
-          for (int w = 0; w < NS; ++w) {
-            sk += N[32 * w + n16];
-            sq += N[32 * w + 16 + n16];
-          }
-          rk = 1.f / sqrtf(sk + 1e-6f);              // 1 / |k_t|
-          qs = qscale / sqrtf(sq + 1e-6f);
-          __builtin_amdgcn_wave_barrier();
-          if (g == 0) N[n16] = rk;                   // for the tokens s
-          __builtin_amdgcn_wave_barrier();
-          const float4 x = ld4(N + 4 * g);
-          cf[0] = x.x; cf[1] = x.y; cf[2] = x.z; cf[3] = x.w;
+          for (int r = 0; r < 4; ++r) cf[r] = ns[r];
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) p[r] = 4 * g + r <= n16 ? pa[r] * qs * cf[r] * D[r] : 0.f;
+        for (int r = 0; r < 4; ++r) p[r] = 4 * g + r <= n16 ? (double)pa[r] * ((double)qs * cf[r]) * D[r] : 0.;
         float* S = sm + L::SC + (c & 3) * 96;
-        if (g == 0) S[n16] = A * qs;
-        if (n16 == 15) {                             // delta: the order of u's registers, see below
-          if constexpr (MODE == DELTA) {
+        if (g == 0) S[place(n16)] = A * qs;
+        if (n16 == 15) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) S[16 + 4 * r + g] = D[r] * cf[r];
-          } else {
-            *reinterpret_cast<float4*>(S + 16 + 4 * g) = make_float4(D[0] * cf[0], D[1] * cf[1], D[2] * cf[2], D[3] * cf[3]);
-          }
+          for (int r = 0; r < 4; ++r) S[16 + 4 * r + g] = D[r] * cf[r];
           if (g == 0) S[80] = A;
         }
         if constexpr (MODE == DELTA) {
           const float beta = G[128 + n16];
-          const int place = 4 * (n16 & 3) + (n16 >> 2);
-          if (g == 0) { S[32 + place] = beta; S[48 + place] = -beta * A * rk; }
-          // u is held with register b, lane group g' <-> token 4 b + g': columns of P in that order
-#pragma unroll
-          for (int r = 0; r < 4; ++r) P[n16 * TR + 4 * r + g] = p[r];
+          if (g == 0) { S[32 + place(n16)] = beta; S[48 + place(n16)] = -beta * A * rk; }
           float* T = sm + L::T + (c & 1) * C * TR;
           float tt[4];
 #pragma unroll
@@ -557,21 +600,22 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
           const float m2 = (below ? -row.z : e2) - m3 * t3.z;
           const float m1 = (below ? -row.y : e1) - m2 * t2.y - m3 * t3.y;
           const float m0 = (below ? -row.x : e0) - m1 * t1.x - m2 * t2.x - m3 * t3.x;
-          float* M = sm + L::M + (c & 1) * C * TR + (4 * e + (n16 >> 2)) * TR + g;      // row: the register place of token n16
+          float* M = sm + L::M + (c & 1) * C * TR + place(n16) * TR + g;      // rows and columns by place
           M[0] = m0 - e0; M[4] = m1 - e1; M[8] = m2 - e2; M[12] = m3 - e3;
-        } else {
-          *reinterpret_cast<float4*>(P + n16 * TR + 4 * g) = make_float4(p[0], p[1], p[2], p[3]);
         }
         if constexpr (MODE == MLSTM) {
-          float rs = (p[0] + p[1]) + (p[2] + p[3]);
+          float rs = ((float)p[0] + (float)p[1]) + ((float)p[2] + (float)p[3]);
           rs += __shfl_xor(rs, 16, 64);
           rs += __shfl_xor(rs, 32, 64);
           if (g == 0) { S[32 + n16] = rs; S[48 + n16] = G[128 + n16]; S[64 + n16] = A * qs; }
         }
       }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) P[4 * r] = p[r];
     };
     barriers(LEAD - 1 - L::W2 + turn);
     for (int c = turn; c < chunks; c += L::W2) {
+      if constexpr (MODE == DELTA) norms(c);
       products(c);
       if constexpr (L::W2 == 2) __syncthreads();
       finish(c);
@@ -654,21 +698,32 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
           G[128] = !ok ? 0.f : (MODE == MLSTM ? expf(-m_new) : x);
         }
       };
-      // D[t = n16, s = 4 g + r] and A_t of a chunk: one running product down from t
+      // D[t = n16, s = 4 g + r] and A_t of a chunk: one running product down from t, with its rounding errors carried along (all
+      // channels share these factors, so the errors would not average out over a read-out's sum)
       auto products = [&](int c) {
         const float* G = sm + L::GT + ((c >> 2) & 1) * 192 + 16 * (c & 3);
-        float D[4] = {0.f, 0.f, 0.f, 0.f}, A = 1.f;
+        float D[4], A = 1.f, low = 0.f;
+        auto times = [&](float d) {
+          const float next = A * d;
+          low = fmaf(low, d, fmaf(A, d, -next));
+          A = next;
+        };
+        auto product = [&]() { return MODE == LIGHT && !finite(A) ? A : A + low; };      // light: decays of any size
 #pragma unroll
-        for (int i = 3; i >= 0; --i) {
+        for (int i = 3; i > 0; --i) {                  // the tokens behind this lane's four, up to t
           const float4 d4 = ld4(G + 4 * i);
           const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
 #pragma unroll
-          for (int r = 3; r >= 0; --r) {
-            const int u = 4 * i + r;
-            D[r] = i == g ? (u <= n16 ? A : 0.f) : D[r];
-            A *= u <= n16 ? dd[r] : 1.f;
-          }
+          for (int r = 3; r >= 0; --r) times(i > g && 4 * i + r <= n16 ? dd[r] : 1.f);
         }
+        const float4 d4 = ld4(G + 4 * g);
+        const float dd[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int r = 3; r >= 0; --r) {
+          D[r] = 4 * g + r <= n16 ? product() : 0.f;
+          times(4 * g + r <= n16 ? dd[r] : 1.f);
+        }
+        A = product();                                 // lane group 0: of all tokens
         float* DM = sm + L::DM + (c & 3) * 272;
         *reinterpret_cast<float4*>(DM + 4 * lane) = make_float4(D[0], D[1], D[2], D[3]);
         if (g == 0) DM[256 + n16] = A;
@@ -718,21 +773,21 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
         dot += __shfl_xor(dot, 32, 64);
         const float nq = S[32 + n16] + dot * S[64 + n16];
         const float inv = 1.f / (fmaxf(fabsf(nq), S[48 + n16]) + 1e-6f);
-        float add[NS] = {};
+        const float at = S[80];
+        float f[C];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float4 f4 = ld4(S + 16 + 4 * i);
-          const float f[4] = {f4.x, f4.y, f4.z, f4.w};
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int w = 0; w < NS; ++w) add[w] += f[r] * K[(4 * i + r) * QR + 64 * w + lane];
+          f[place(4 * i)] = f4.x; f[place(4 * i + 1)] = f4.y; f[place(4 * i + 2)] = f4.z; f[place(4 * i + 3)] = f4.w;
         }
-        const float at = S[80];
 #pragma unroll
-        for (int w = 0; w < NS; ++w) nrm[w] = at * nrm[w] + add[w];
+        for (int w = 0; w < NS; ++w) nrm[w] *= at;
+#pragma unroll
+        for (int t = 0; t < C; ++t)
+#pragma unroll
+          for (int w = 0; w < NS; ++w) nrm[w] += f[t] * K[place(t) * QR + 64 * w + lane];
         __builtin_amdgcn_wave_barrier();
-        if (g == 0) S[32 + n16] = inv;
+        if (g == 0) S[32 + place(n16)] = inv;
         __syncthreads();
       }
       __syncthreads();
@@ -751,8 +806,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
   const int col = (zb * L::NC + cw) * 16 + n16, colc = min(col, dv - 1);
   const bool cok = col < dv;
   const TI* vb = (const TI*)a.v + (size_t)row0 * a.v_stride + (size_t)head * dv;
-  // u's register r: token 4 g + r; delta: 4 r + g
-  auto tok = [&](int r) { return MODE == DELTA ? 4 * r + g : 4 * g + r; };
+  auto tok = [&](int r) { return 4 * r + g; };
   TI rv[2][4];
   unsigned vv[4];
 #pragma unroll
@@ -817,49 +871,50 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
       if constexpr (MODE == SSM) all *= at;
       if constexpr (MODE == DELTA) {
         // x = beta v - beta A S^T k / |k|, rows in the order of u's registers
-        f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = {0.f, 0.f, 0.f, 0.f};
-        const float* Kr = K + (4 * (n16 & 3) + (n16 >> 2)) * QR + 4 * g;
+        f32x4 xs[L::NA];
+        zero(xs);
+        const float* Kr = K + n16 * QR + 4 * g;
 #pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          const float4 kf = ld4(Kr + 16 * i);
-          x0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, S[i][0], x0, 0, 0, 0);
-          x1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, S[i][1], x1, 0, 0, 0);
-          x0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, S[i][2], x0, 0, 0, 0);
-          x1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, S[i][3], x1, 0, 0, 0);
-        }
-        f32x4 X;
+        for (int i = 0; i < NT; ++i) channels(xs, i, ld4(Kr + 16 * i), S[i]);
+        const f32x4 kS = total(xs);
+        f32x4 R;                                       // what is to be added to u: first what u lacks of 64 bits
         bool bad = false;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          X[r] = F[32 + 4 * g + r] * u[r] + F[48 + 4 * g + r] * (x0[r] + x1[r]);
-          bad |= !finite(X[r]);
+          const double x = (double)F[32 + 4 * g + r] * u[r] + (double)F[48 + 4 * g + r] * kS[r];
+          u[r] = (float)x;
+          R[r] = (float)(x - u[r]);
+          bad |= !finite(u[r]);
         }
         if (__builtin_expect(!__any(bad), 1)) {
+          // what the substitution adds is summed by itself: added to u product by product it would round at u's size sixteen times
           const float4 mf = ld4(sm + L::M + (c & 1) * C * TR + n16 * TR + 4 * g);
-          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.x, X[0], X, 0, 0, 0);
-          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.y, X[1], X, 0, 0, 0);
-          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.z, X[2], X, 0, 0, 0);
-          X = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.w, X[3], X, 0, 0, 0);
+          R = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.x, u[0] + R[0], R, 0, 0, 0);
+          R = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.y, u[1] + R[1], R, 0, 0, 0);
+          R = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.z, u[2] + R[2], R, 0, 0, 0);
+          R = __builtin_amdgcn_mfma_f32_16x16x4f32(mf.w, u[3] + R[3], R, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) u[r] += R[r];
         } else {
           const float* T = sm + L::T + (c & 1) * C * TR;
 #pragma unroll
           for (int s = 0; s < C; ++s) {
-            const float us = __shfl(X[s >> 2], (s & 3) * 16 + n16, 64);
+            const float us = __shfl(u[s >> 2], (s & 3) * 16 + n16, 64);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              if (4 * r + g > s) X[r] -= T[(4 * r + g) * TR + s] * us;
+              if (tok(r) > s) u[r] -= T[tok(r) * TR + s] * us;
           }
         }
-        *reinterpret_cast<f32x4*>(sm + L::U + ((c & 1) * L::NC + cw) * 256 + 4 * lane) = X;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) u[r] = X[r];
+        *reinterpret_cast<float4*>(sm + L::U + ((c & 1) * L::NC + cw) * 256 + 4 * lane) = make_float4(u[0], u[1], u[2], u[3]);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[r] = L::CH ? u[r] : u[r] * F[16 + 4 * g + r];
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
         float kt[4];
-        f32x4 s = S[i];
+        // delta: the chunk's part by itself, so that the state is rounded once; where decays are short (mlstm, wkv) the state is the
+        // smallest term and comes first
+        f32x4 s = MODE == DELTA ? f32x4{0.f, 0.f, 0.f, 0.f} : S[i];
         if constexpr (L::CH) {
           const float4 k4 = ld4(KT + 16 * i * TR), de = ld4(DE + 16 * i);
           kt[0] = k4.x; kt[1] = k4.y; kt[2] = k4.z; kt[3] = k4.w;
@@ -867,13 +922,14 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
         } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            kt[r] = K[tok(r) * QR + 16 * i + n16];
-            s[r] *= at;
+            kt[r] = K[(4 * g + r) * QR + 16 * i + n16];
+            if (MODE != DELTA) s[r] *= at;
           }
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[r], x[r], s, 0, 0, 0);
-        S[i] = s;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[i][r] = MODE == DELTA ? fmaf(at, S[i][r], s[r]) : s[r];
       }
       __syncthreads();
     };
@@ -902,14 +958,14 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
   float* yb = a.y + (size_t)row0 * H * dv + (size_t)head * dv;
   unsigned vy[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) vy[r] = (unsigned)((4 * g + r) * (H * dv) + colc) * 4u;
+  for (int r = 0; r < 4; ++r) vy[r] = (unsigned)(tok(r) * (H * dv) + colc) * 4u;
   barriers(LEAD);
   auto step = [&](int c, int st) {
     const int left = n - c * C;
-    const float* Q = sm + L::Q + (c % L::QB) * L::ROWS + n16 * QR + 4 * g;
+    const float* Q = sm + L::Q + (c % L::QB) * L::ROWS + place(n16) * QR + 4 * g;
     const float* F = sm + L::SC + (c & 3) * 96 + 4 * g;
     const float* ST = sm + L::ST + ((c & 1) * L::NC + cw) * DP * 16 + 4 * lane;
-    const float* P = sm + L::P + (c & 3) * C * TR;
+    const double* P = reinterpret_cast<const double*>(sm + L::P) + c % 3 * C * PR;
     float u[4];
     if constexpr (MODE == DELTA) {
       const float4 u4 = ld4(sm + L::U + ((c & 1) * L::NC + cw) * 256 + 4 * lane);
@@ -917,36 +973,32 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
     } else {
       take_v(c, st, u);
     }
-    const float4 pf = ld4(P + n16 * TR + 4 * g);
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    // P u in 64 bits (row m of these products comes out as u's token m): sixteen tokens' roundings are the result's otherwise
+    const f64x2 p0 = *reinterpret_cast<const f64x2*>(P + n16 * PR + 4 * g), p1 = *reinterpret_cast<const f64x2*>(P + n16 * PR + 4 * g + 2);
+    f64x4 o = {0., 0., 0., 0.};
     if (__builtin_expect(!__any(!finite(u[0]) || !finite(u[1]) || !finite(u[2]) || !finite(u[3])), 1)) {
-      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.x, u[0], o, 0, 0, 0);
-      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.y, u[1], o, 0, 0, 0);
-      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.z, u[2], o, 0, 0, 0);
-      o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf.w, u[3], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f64_16x16x4f64(p0[0], u[0], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f64_16x16x4f64(p0[1], u[1], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f64_16x16x4f64(p1[0], u[2], o, 0, 0, 0);
+      o = __builtin_amdgcn_mfma_f64_16x16x4f64(p1[1], u[3], o, 0, 0, 0);
     } else {
 #pragma unroll
       for (int s = 0; s < C; ++s) {
-        const float us = MODE == DELTA ? __shfl(u[s >> 2], (s & 3) * 16 + n16, 64) : __shfl(u[s & 3], (s >> 2) * 16 + n16, 64);
-        const int at = MODE == DELTA ? 4 * (s & 3) + (s >> 2) : s;
+        const float us = __shfl(u[s >> 2], (s & 3) * 16 + n16, 64);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          if (4 * g + r >= s) o[r] += P[(4 * g + r) * TR + at] * us;
+          if (tok(r) >= s) o[r] += P[tok(r) * PR + place(s)] * us;
       }
     }
-    f32x4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+    f32x4 os[L::NO];
+    zero(os);
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      const float4 qf = ld4(Q + 16 * i), s = ld4(ST + 256 * i);
-      o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.x, s.x, o0, 0, 0, 0);
-      o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.y, s.y, o1, 0, 0, 0);
-      o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.z, s.z, o0, 0, 0, 0);
-      o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(qf.w, s.w, o1, 0, 0, 0);
-    }
+    for (int i = 0; i < NT; ++i) channels(os, i, ld4(Q + 16 * i), *reinterpret_cast<const f32x4*>(ST + 256 * i));
+    const f32x4 qS = total(os);
     float out[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      out[r] = o[r] + (o0[r] + o1[r]) * (L::CH ? 1.f : F[r]);
+      out[r] = (float)(o[r] + (double)qS[r] * (L::CH ? 1.f : F[r]));
       if constexpr (MODE == MLSTM) out[r] *= F[32 + r];
       if constexpr (MODE == SSM) out[r] += skip * u[r];
     }
@@ -960,7 +1012,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (cok && 4 * g + r < left) *reinterpret_cast<float*>(yc + vy[r]) = out[r];
+        if (cok && tok(r) < left) *reinterpret_cast<float*>(yc + vy[r]) = out[r];
     }
     __syncthreads();
   };

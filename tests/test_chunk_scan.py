@@ -22,7 +22,7 @@ def make(mode, lens, H, D, V, dtype, past, seed=0, pad=0):
     g = torch.Generator().manual_seed(seed + 17)
     T, n = sum(lens), len(lens)
     rn = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
-    d = {"mode": mode, "lens": lens, "H": H, "D": D, "V": V, "past": past, "S": rn(n + 1, H, V, D) if mode == "ssm" else rn(n + 1, H, D, V),
+    d = {"mode": mode, "lens": lens, "H": H, "D": D, "V": V, "pad": pad, "past": past, "S": rn(n + 1, H, V, D) if mode == "ssm" else rn(n + 1, H, D, V),
          "n": rn(n + 1, H, D), "m": rn(n + 1, H)}
     if mode == "ssm":
         G = d["G"] = 2 if H % 2 == 0 else 1
@@ -56,9 +56,9 @@ def call(d, **kw):
         y = recur.ssm_scan(c(d["xbc"]), c(d["dt"]), c(b), c(a), c(s), S, *where, H, V, D, d["G"], **kw)
         return y.cpu(), S.cpu()
     # rows stay strided views
-    base = c(torch.cat([d["q"], d["k"], d["v"]], 1))
-    gd = d["G"] * D
-    q, k, v = base[:, :gd], base[:, gd:2 * gd], base[:, 2 * gd:]
+    gd, hv = d["G"] * D, H * V
+    base = c(torch.cat([d["q"], d["k"], d["v"], d["q"][:, :d["pad"]]], 1))
+    q, k, v = base[:, :gd], base[:, gd:2 * gd], base[:, 2 * gd:2 * gd + hv]
     if d["mode"] == "wkv":
         y = linrec.wkv_scan(q, k, v, c(d["a"]), c(d["par"][0]), c(d["par"][1]), S, *where, H, D)
     elif d["mode"] == "delta":
