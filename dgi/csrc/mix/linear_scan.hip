@@ -412,12 +412,33 @@ __global__ __launch_bounds__(256) void mlstm_commit_kernel(float* __restrict__ n
 // several rows is right too, row after row.
 //
 // 32 sequences, 64 heads of 64 x 64 (67 MB): 30 us (2.2 TB/s) -> 15 (4.4 TB/s).
+// a product that is rounded, never part of a fused one
+__device__ __forceinline__ float mul_rounded(float x, float y) {
+#pragma clang fp contract(off)
+  return x * y;
+}
+// Sums of row_scan_kernel: over four channels at a time, then over those sums, across the workgroup as a tree.  One running
+// sum over a thread's channels and then over the G partial sums was 1.2 times as far from 64 bits as linear_scan_kernel.
+__device__ __forceinline__ void add4(float4& x, const float4& y) { x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w; }
+__device__ __forceinline__ void fma4(float4& x, float f, const float4& y) { x.x += f * y.x; x.y += f * y.y; x.z += f * y.z; x.w += f * y.w; }
+template <int N, typename F>
+__device__ __forceinline__ float tree_sum(F&& at) {
+  float x[N / 4];
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) x[i] = (at(4 * i) + at(4 * i + 1)) + (at(4 * i + 2) + at(4 * i + 3));
+#pragma unroll
+  for (int h = N / 8; h > 0; h /= 2)
+#pragma unroll
+    for (int i = 0; i < h; ++i) x[i] += x[i + h];
+  return x[0];
+}
+
 template <int MODE, typename TI, int Q, int R>
 __global__ __launch_bounds__(256) void row_scan_kernel(const ScanArgs a) {
   constexpr int G = 256 / Q, KMAX = G * R, CMAX = 4 * Q;
   static_assert(KMAX + CMAX <= 256, "one thread per staged element");
   __shared__ __attribute__((aligned(16))) float part[MODE == DELTA ? 2 : 1][G][CMAX];
-  __shared__ __attribute__((aligned(16))) float sk[KMAX], sq[KMAX], sw[KMAX], sx[KMAX], sv[CMAX], tot[CMAX];
+  __shared__ __attribute__((aligned(16))) float sk[KMAX], sq[KMAX], sw[KMAX], sx[KMAX], su[KMAX], sv[CMAX], tot[CMAX];
   __shared__ float sums[3][G];
   const int seq = blockIdx.x, head = blockIdx.y;
   const int row0 = a.seq_row0[seq], n = a.seq_row0[seq + 1] - row0;
@@ -445,21 +466,21 @@ __global__ __launch_bounds__(256) void row_scan_kernel(const ScanArgs a) {
     const size_t row = (size_t)(row0 + t);
     // thread -> key channel, or column behind the KMAX channels
     if (tid < KMAX) {
-      float k = 0.f, q = 0.f, w = 0.f, x = 0.f;
+      float k = 0.f, q = 0.f, w = 0.f, u = 0.f;
       if (tid < dk) {
         k = ldf<TI>((const TI*)a.k + (size_t)kvh * dk + row * a.k_stride + tid);
         q = ldf<TI>((const TI*)a.q + (size_t)kvh * dk + row * a.q_stride + tid);
         if constexpr (MODE == GLA) w = a.aux1[row * a.aux1_stride + head * dk + tid];
         if constexpr (MODE == WKV) {
           w = expf(-expf(a.aux1[row * a.aux1_stride + head * dk + tid] + a.par1[head * dk + tid]));
-          x = q * k * a.par2[head * dk + tid];
+          u = a.par2[head * dk + tid];
         }
         if constexpr (MODE == LIGHT) { k = silu_f(k); q = silu_f(q); }
       }
       sk[tid] = k;
       sq[tid] = q;
       if constexpr (MODE == WKV || MODE == GLA) sw[tid] = w;
-      if constexpr (MODE == WKV) sx[tid] = x;
+      if constexpr (MODE == WKV) { sx[tid] = q * k; su[tid] = u; }
     } else if (tid - KMAX < CMAX) {
       const int col = tid - KMAX;
       float v = 0.f;
@@ -488,16 +509,25 @@ __global__ __launch_bounds__(256) void row_scan_kernel(const ScanArgs a) {
       float4 aq = make_float4(0.f, 0.f, 0.f, 0.f);
       float kk = 0.f, qq = 0.f, kq = 0.f;
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const float k = sk[g + G * i], q = sq[g + G * i];
-        acc.x += S[i].x * k; acc.y += S[i].y * k; acc.z += S[i].z * k; acc.w += S[i].w * k;
-        aq.x += S[i].x * q; aq.y += S[i].y * q; aq.z += S[i].z * q; aq.w += S[i].w * q;
-        kk += k * k; qq += q * q; kq += k * q;
+      for (int j = 0; j < R; j += 4) {
+        float4 pk = make_float4(0.f, 0.f, 0.f, 0.f), pq = pk;
+        float a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll
+        for (int i = j; i < j + 4; ++i) {
+          const float k = sk[g + G * i], q = sq[g + G * i];
+          fma4(pk, k, S[i]);
+          fma4(pq, q, S[i]);
+          a1 += k * k; a2 += q * q; a3 += k * q;
+        }
+        add4(acc, pk);
+        add4(aq, pq);
+        kk += a1; qq += a2; kq += a3;
       }
       *reinterpret_cast<float4*>(&part[1][g][4 * c]) = aq;
       if (c == 0) { sums[0][g] = kk; sums[1][g] = qq; sums[2][g] = kq; }
     } else if constexpr (MODE == MLSTM) {
-      const float i_in = a.cap * tanhf(g1 / a.cap), f_in = logsigmoid_f(a.cap * tanhf(g2 / a.cap));
+      // rounded by itself: where the gate is the new maximum, its factor is exactly 1
+      const float i_in = mul_rounded(a.cap, tanhf(g1 / a.cap)), f_in = logsigmoid_f(a.cap * tanhf(g2 / a.cap));
       const float m_new = fmaxf(f_in + m_run, i_in);
       fa = expf(f_in + m_run - m_new);
       fb = expf(i_in - m_new);
@@ -506,42 +536,48 @@ __global__ __launch_bounds__(256) void row_scan_kernel(const ScanArgs a) {
       const float4 b = make_float4(fb * v4.x, fb * v4.y, fb * v4.z, fb * v4.w);
       float nq = 0.f;
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const float k = sk[g + G * i], q = sq[g + G * i];
-        S[i].x = fa * S[i].x + k * b.x; S[i].y = fa * S[i].y + k * b.y; S[i].z = fa * S[i].z + k * b.z; S[i].w = fa * S[i].w + k * b.w;
-        acc.x += S[i].x * q; acc.y += S[i].y * q; acc.z += S[i].z * q; acc.w += S[i].w * q;
-        N[i] = fa * N[i] + fb * k;
-        nq += N[i] * q;
+      for (int j = 0; j < R; j += 4) {
+        float4 pq = make_float4(0.f, 0.f, 0.f, 0.f);
+        float a1 = 0.f;
+#pragma unroll
+        for (int i = j; i < j + 4; ++i) {
+          const float k = sk[g + G * i], q = sq[g + G * i];
+          S[i].x = fa * S[i].x + k * b.x; S[i].y = fa * S[i].y + k * b.y; S[i].z = fa * S[i].z + k * b.z; S[i].w = fa * S[i].w + k * b.w;
+          fma4(pq, q, S[i]);
+          N[i] = fmaf(fb, k, fa * N[i]);
+          a1 += N[i] * q;
+        }
+        add4(acc, pq);
+        nq += a1;
       }
       if (c == 0) sums[0][g] = nq;
     } else {
       float bonus = 0.f;
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        const float k = sk[g + G * i], q = sq[g + G * i], w = MODE == LIGHT ? decay : sw[g + G * i];
-        if constexpr (MODE == WKV) {
-          bonus += sx[g + G * i];
-          acc.x += S[i].x * q; acc.y += S[i].y * q; acc.z += S[i].z * q; acc.w += S[i].w * q;
+      for (int j = 0; j < R; j += 4) {
+        float4 pq = make_float4(0.f, 0.f, 0.f, 0.f);
+        float b1 = 0.f;
+#pragma unroll
+        for (int i = j; i < j + 4; ++i) {
+          const float k = sk[g + G * i], q = sq[g + G * i], w = MODE == LIGHT ? decay : sw[g + G * i];
+          if constexpr (MODE == WKV) {
+            b1 += sx[g + G * i] * su[g + G * i];
+            fma4(pq, q, S[i]);
+          }
+          S[i].x = fmaf(k, v4.x, w * S[i].x); S[i].y = fmaf(k, v4.y, w * S[i].y); S[i].z = fmaf(k, v4.z, w * S[i].z); S[i].w = fmaf(k, v4.w, w * S[i].w);
+          if constexpr (MODE != WKV) fma4(pq, q, S[i]);
         }
-        S[i].x = w * S[i].x + k * v4.x; S[i].y = w * S[i].y + k * v4.y; S[i].z = w * S[i].z + k * v4.z; S[i].w = w * S[i].w + k * v4.w;
-        if constexpr (MODE != WKV) {
-          acc.x += S[i].x * q; acc.y += S[i].y * q; acc.z += S[i].z * q; acc.w += S[i].w * q;
-        }
+        add4(acc, pq);
+        bonus += b1;
       }
       if (MODE == WKV && c == 0) sums[0][g] = bonus;
     }
     *reinterpret_cast<float4*>(&part[0][g][4 * c]) = acc;
     __syncthreads();
-    auto total = [&](int j) {
-      float x = 0.f;
-#pragma unroll
-      for (int i = 0; i < G; ++i) x += sums[j][i];
-      return x;
-    };
+    auto total = [&](int j) { return tree_sum<G>([&](int i) { return sums[j][i]; }); };
     float o = 0.f;
     if (tid < CMAX) {
-#pragma unroll
-      for (int i = 0; i < G; ++i) o += part[0][i][tid];
+      o = tree_sum<G>([&](int i) { return part[0][i][tid]; });
       if constexpr (MODE == WKV) o += total(0) * sv[tid];
       if constexpr (MODE == GLA) o *= qscale;
       if constexpr (MODE == MLSTM) o = o * qscale / (fmaxf(fabsf(total(0) * qscale), em) + 1e-6f);
@@ -552,9 +588,7 @@ __global__ __launch_bounds__(256) void row_scan_kernel(const ScanArgs a) {
       if (tid < CMAX) {
         const float ku = beta * (sv[tid] - o * ge * rk) * rk;
         tot[tid] = ku;
-        o = 0.f;
-#pragma unroll
-        for (int i = 0; i < G; ++i) o += part[1][i][tid];
+        o = tree_sum<G>([&](int i) { return part[1][i][tid]; });
         o = rq * (ge * o + total(2) * ku);
       }
       __syncthreads();
@@ -562,7 +596,7 @@ __global__ __launch_bounds__(256) void row_scan_kernel(const ScanArgs a) {
 #pragma unroll
       for (int i = 0; i < R; ++i) {
         const float k = sk[g + G * i];
-        S[i].x = ge * S[i].x + k * u.x; S[i].y = ge * S[i].y + k * u.y; S[i].z = ge * S[i].z + k * u.z; S[i].w = ge * S[i].w + k * u.w;
+        S[i].x = fmaf(ge, S[i].x, k * u.x); S[i].y = fmaf(ge, S[i].y, k * u.y); S[i].z = fmaf(ge, S[i].z, k * u.z); S[i].w = fmaf(ge, S[i].w, k * u.w);
       }
     }
     if (tid < dv) a.y[row * ((size_t)H * dv) + (size_t)head * dv + tid] = o;
