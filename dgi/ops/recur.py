@@ -188,8 +188,10 @@ def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, se
     S [N, dv] in fp32 read from / written to ``state`` [slots, heads, dv, N] (value-major; zero at position 0).
     Returns y [T, heads*dv] fp32.
 
-    On the GPU a step with prompt portions takes them sixteen rows at a time on the matrix cores — the same recurrence
-    with its fp32 sums reassociated; steps of single rows, and every step with ``chunked`` False, go row by row."""
+    On the GPU the prompt portions of bf16 models are taken sixteen rows at a time on the matrix cores — the same recurrence
+    with its fp32 sums reassociated, where the step's rows and sequences make that the faster form.  Models in fp32
+    (``dt_raw`` fp32), steps of single rows, and every step with ``chunked`` False go row by row: those results do not depend
+    on how a prompt was cut or on what else is in the step.  ``chunked`` True asks for the chunks."""
     if _native(xbc):
         T, n_seq = xbc.shape[0], seq_slots.shape[0]
         y = torch.empty(T, heads * dv, dtype=torch.float32, device=xbc.device)
@@ -208,7 +210,7 @@ def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, se
                 chunked = T > rows * n_seq
             else:
                 chunked = 4 * T > 3 * rows * n_seq or (T - n_seq >= 512 and T <= 48 * n_seq)
-            chunked = chunked and SCAN_CHUNK > 0
+            chunked = chunked and SCAN_CHUNK > 0 and dt_raw.dtype != torch.float32
         _call("ssm_scan", y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G, bool(chunked))
         return y
     return ssm_scan_ref(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G)

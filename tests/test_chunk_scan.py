@@ -238,3 +238,17 @@ def test_ssm_segments_beside_sequences_without_rows(lens):
     empty ones keep their states."""
     d = make("ssm", lens, 1, 128, 32, torch.bfloat16, [4 if n == 0 else 0 for n in lens], seed=len(lens))
     check(call(d, chunked=True), oracle(d))
+
+
+def test_ssm_of_fp32_models_does_not_depend_on_the_step():
+    """A sequence alone, beside others, and in two parts: the same numbers, bit for bit."""
+    lens, cut = [300, 90, 700], 130
+    d = make("ssm", lens, 8, 64, 64, torch.float32, [0, 5, 0])
+    y, S = call(d)
+    check((y, S), oracle(make("ssm", lens, 8, 64, 64, torch.float32, [0, 5, 0])))
+    only = dict(d, lens=lens[:1], past=[0], xbc=d["xbc"][:300], dt=d["dt"][:300])
+    y1, S1 = call(only)
+    assert torch.equal(y1, y[:300]) and torch.equal(S1[1], S[3])
+    y2, S2 = call(dict(only, lens=[cut], xbc=d["xbc"][:cut], dt=d["dt"][:cut]))
+    y3, S3 = call(dict(only, lens=[300 - cut], past=[cut], S=S2, xbc=d["xbc"][cut:300], dt=d["dt"][cut:300]))
+    assert torch.equal(torch.cat([y2, y3]), y[:300]) and torch.equal(S3[1], S[3])
