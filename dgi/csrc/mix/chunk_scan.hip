@@ -37,8 +37,8 @@
 // tokens starts with the oldest, the per-token decays and wkv's suffix products carry their rounding errors along, and P and P u are 64-bit
 // (four v_mfma_f64_16x16x4_f64 per chunk and output wave).  It costs 3 (delta) to 13 % (mlstm) of the time; wkv's was not the longest role.
 //
-// Half-chunk products of channel decays below 1e-28 leave the range of the scaled operands; the wave that prepares such channels
-// then sums their scores token by token instead.  An infinity or NaN among a chunk's u takes a path that keeps it from the tokens
+// Half-chunk products of channel decays below 1e-28, or q and k so large or small that their scaled values leave the fp32 range: the wave that
+// prepares such channels sums their scores token by token instead.  An infinity or NaN among a chunk's u takes a path that keeps it from the tokens
 // before it (a matrix product multiplies it by their zeros).  A portion at position 0 reads no state.
 #include <type_traits>
 #include "../common.h"
@@ -89,6 +89,12 @@ __device__ __forceinline__ void widen(const Raw4<float>& r, float* f) { f[0] = r
 __device__ __forceinline__ void widen(const Raw4<uint16_t>& r, float* f) {
   f[0] = __uint_as_float(r.v.x << 16); f[1] = __uint_as_float(r.v.x & 0xffff0000u);
   f[2] = __uint_as_float(r.v.y << 16); f[3] = __uint_as_float(r.v.y & 0xffff0000u);
+}
+
+// the largest magnitude (fmaxf would first bring its operands into canonical form: three instructions)
+__device__ __forceinline__ float larger3(float m, float a, float b) {
+  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
+  return m;
 }
 
 template <int CTRL>
@@ -339,7 +345,19 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
           K[t * QR] = k[t] * __builtin_amdgcn_rcpf(hi);
         }
         float* R = sm + L::RAW + ((c & 1) * NS + w) * L::RAWN;
-        const bool raw = __any(!(lo > SAFE && hi > SAFE));
+        // The scaled operands have to stay in the fp32 range.  Those divided are q of the tokens 1 to 7 and k of 8 to 14 (0 and 15 have no
+        // partner in the chunk), those multiplied, and lost where they are small, k of 0 to 6 and q of 9 to 15.
+        const float least = fminf(lo, hi);
+        float top = 0.f;
+#pragma unroll
+        for (int t = 1; t < 8; ++t) top = larger3(top, q[t], k[t + 7]);
+        bool raw = false;
+        if (__builtin_expect(__any(!(least > 1e-8f && top < 1e30f)), 0)) {
+          float low = 1.f;
+#pragma unroll
+          for (int t = 0; t < 7; ++t) low = fminf(low, fminf(q[t + 9] == 0.f ? 1.f : fabsf(q[t + 9]), k[t] == 0.f ? 1.f : fabsf(k[t])));
+          raw = __any(!(least > SAFE && top < 1e38f * least && low * least > 1e-36f));
+        }
         if (lane == 0) R[0] = raw ? 1.f : 0.f;
 #pragma unroll
         for (int t = 0; t < C; ++t) s[t] = q[t] * bonus * k[t];

@@ -252,3 +252,24 @@ def test_ssm_of_fp32_models_does_not_depend_on_the_step():
     y2, S2 = call(dict(only, lens=[cut], xbc=d["xbc"][:cut], dt=d["dt"][:cut]))
     y3, S3 = call(dict(only, lens=[300 - cut], past=[cut], S=S2, xbc=d["xbc"][cut:300], dt=d["dt"][cut:300]))
     assert torch.equal(torch.cat([y2, y3]), y[:300]) and torch.equal(S3[1], S[3])
+
+
+@pytest.mark.parametrize("q,k", [(1e17, 1e-17), (1e-17, 1e17), (1e-15, 1e-3), (1e16, 1e-3)])
+def test_wkv_scales_beside_strong_decays(q, k):
+    """Half a chunk's decays near the edge of what the scaled operands allow, q and k far from 1: scaled they would leave the fp32 range
+    (an overflow, or keys that vanish), the results do not."""
+    d = make("wkv", [130, 40], 3, 64, 64, torch.float32, [0, 7])
+    d["a"][:], d["par"] = 0.0, (torch.full_like(d["par"][0], 2.04), d["par"][1])      # half a chunk: about 1e-27
+    d["a"][:, 1::2] = -6.0
+    d["q"] *= q
+    d["k"] *= k
+    d["S"] *= k
+    y, S = call(d)
+    wy, wS = oracle(d)
+    assert torch.isfinite(wy.float()).all() and torch.isfinite(wS.float()).all()
+    assert (y.to(F64) - wy).abs().max() <= 3e-5 * wy.abs().max()
+    assert (S.to(F64) - wS).abs().max() <= 3e-5 * wS.abs().max()
+    # the strongly decayed channels by themselves: their own sums, not hidden behind the others'
+    d["q"][:, 1::2] = 0.0
+    y, wy = call(d)[0], oracle(d)[0]
+    assert (y.to(F64) - wy).abs().max() <= 3e-5 * wy.abs().max()
