@@ -24,6 +24,8 @@
 // Optional sinks: exp(sinks[head]) joins the softmax denominator of that head (a logit without a key or a value,
 // neither scaled nor cached); it is added once, where the row's result is normalised.
 #include <algorithm>
+#include <cfloat>
+
 #include "../common.h"
 
 using namespace dgi;
@@ -35,6 +37,9 @@ __device__ __forceinline__ float inv_with_sink(float m, float l, float sink) {
   const float top = fmaxf(m, sink), f = expf(m - top);
   return f / (l * f + expf(sink - top));
 }
+
+// The same without a sink.  A row without a position (negative) has no keys, and results of zero.
+__device__ __forceinline__ float inv_sum(float l) { return l == 0.f ? 0.f : 1.f / l; }
 
 template <typename T> __device__ __forceinline__ float ldf(const T* p);
 template <> __device__ __forceinline__ float ldf<float>(const float* p) { return *p; }
@@ -97,7 +102,7 @@ __global__ __launch_bounds__(1024) void latent_attn_rows_kernel(
     for (int e = lane; e < kr; e += 64) qw[e] = ldf<T>(ql + e);
     const T* qr = q + (size_t)row * q_stride + (size_t)head * (dim + rd) + dim;
     const int half = dims >> 1;
-    const float* cs = cos_sin ? cos_sin + (size_t)pos * dims : nullptr;
+    const float* cs = cos_sin ? cos_sin + (size_t)max(pos, 0) * dims : nullptr;
     for (int i = lane; i < half; i += 64) {
       const int i0 = interleaved ? 2 * i : i, i1 = interleaved ? 2 * i + 1 : i + half;
       const float u = ldf<T>(qr + i0), v = ldf<T>(qr + i1);
@@ -211,7 +216,7 @@ __global__ __launch_bounds__(1024) void latent_attn_rows_kernel(
     }
     return;
   }
-  const float inv = sinks ? inv_with_sink(m_run, l_run, sinks[head]) : 1.f / l_run;
+  const float inv = sinks ? inv_with_sink(m_run, l_run, sinks[head]) : inv_sum(l_run);
   T* op = out + (size_t)head * o_hs + (size_t)row * o_ts;
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
@@ -223,7 +228,7 @@ __global__ __launch_bounds__(1024) void latent_attn_rows_kernel(
   }
 }
 
-// out[h][row] = sum_z o_z e^(m_z - M) / sum_z l_z e^(m_z - M), M = max_z m_z; grid (rows, H), run 0 is never empty.
+// out[h][row] = sum_z o_z e^(m_z - M) / sum_z l_z e^(m_z - M), M = max_z m_z (finite also where no run has keys); grid (rows, H).
 // V consecutive dims per thread (4: kr a multiple of 4); four runs' sums are loaded together.
 template <typename T, int V>
 __global__ __launch_bounds__(256) void latent_attn_reduce_kernel(const float* __restrict__ part_o,
@@ -232,11 +237,11 @@ __global__ __launch_bounds__(256) void latent_attn_reduce_kernel(const float* __
                                                                  const float* __restrict__ sinks) {
   const int row = blockIdx.x, head = blockIdx.y, rows = gridDim.x, H = gridDim.y;
   const size_t first = (size_t)head * rows + row, next = (size_t)H * rows;         // slot of run 0, slots from run to run
-  float M = -__builtin_inff();
+  float M = -FLT_MAX;
   for (int z = 0; z < nsplit; ++z) M = fmaxf(M, part_ml[2 * (first + z * next)]);
   float L = 0.f;
   for (int z = 0; z < nsplit; ++z) L += part_ml[2 * (first + z * next) + 1] * expf(part_ml[2 * (first + z * next)] - M);
-  const float inv = sinks ? inv_with_sink(M, L, sinks[head]) : 1.f / L;
+  const float inv = sinks ? inv_with_sink(M, L, sinks[head]) : inv_sum(L);
   T* op = out + (size_t)head * o_hs + (size_t)row * o_ts;
   for (int e = threadIdx.x * V; e < kr; e += blockDim.x * V) {
     float acc[V];
@@ -315,7 +320,7 @@ __device__ __forceinline__ void stage_queries(uint16_t* qs, int DP, const uint16
   // rotated part
   constexpr int U = 4;
   const int half = dims >> 1;
-  const float* cs = dims > 0 ? cos_sin + (size_t)pos * dims : nullptr;
+  const float* cs = dims > 0 ? cos_sin + (size_t)max(pos, 0) * dims : nullptr;
   for (int i0 = threadIdx.x; i0 < NH * rd; i0 += U * NT) {
     uint16_t a[U], b[U];
     float c[U], sn[U];
@@ -560,7 +565,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
       part_ml[2 * slot + 1] = Lh;
     }
   } else {
-    const float inv = sinks ? inv_with_sink(Mh, Lh, sinks[head]) : 1.f / Lh;
+    const float inv = sinks ? inv_with_sink(Mh, Lh, sinks[head]) : inv_sum(Lh);
     uint16_t* op = out + (size_t)head * o_hs + (size_t)row * o_ts;
     const bool ovec = ((uintptr_t)out & 7) == 0 && (o_hs & 3) == 0 && (o_ts & 3) == 0;
     for (int e = part * 4; e < kr; e += 64) {
@@ -801,7 +806,7 @@ __global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
     part_ml[2 * slot] = M;
     part_ml[2 * slot + 1] = L;
   }
-  const float inv = part_o ? 1.f : sinks ? inv_with_sink(M, L, sinks[head]) : 1.f / L;
+  const float inv = part_o ? 1.f : sinks ? inv_with_sink(M, L, sinks[head]) : inv_sum(L);
   uint16_t* op = out + (size_t)head * o_hs + (size_t)row * o_ts;
   const bool ovec = ((uintptr_t)out & 7) == 0 && (o_hs & 3) == 0 && (o_ts & 3) == 0;
   auto kept = [&](auto put) {                          // put(latent dim, its four sums) for the half this wave keeps

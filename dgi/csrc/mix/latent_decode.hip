@@ -7,6 +7,8 @@
 // Both are bounded by launches and latency (2 MB and 4 MB of weights at 32 heads of 64 + 128 dims on 512), not by work: the
 // library's batched products took 12 and 5 us for 32 rows, and between them and after them ran a pass that combines the
 // runs of keys and one that puts the heads side by side.  latent_values reads the runs' partial sums itself.
+#include <cfloat>
+
 #include "../common.h"
 
 using namespace dgi;
@@ -120,10 +122,10 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
       len[idx] = e[i].y;
     }
     __syncthreads();
-    float M = -__builtin_inff(), L = 0.f;                  // of this lane's row
+    float M = -FLT_MAX, L = 0.f;                           // of this lane's row; finite also where no run has keys
     for (int z = 0; z < runs; ++z) M = fmaxf(M, fac[z][lr]);
     for (int z = 0; z < runs; ++z) L += len[z * 16 + lr] * expf(fac[z][lr] - M);
-    float inv = 1.f / L;
+    float inv = L == 0.f ? 0.f : 1.f / L;
     if (sinks) {                                           // one more logit in the denominator, relative to the larger of the two
       const float sink = sinks[head], top = fmaxf(M, sink), f = expf(M - top);
       inv = f / (L * f + expf(sink - top));

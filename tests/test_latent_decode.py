@@ -54,3 +54,21 @@ def test_decode_heads(T, H, dim, vdim, gated):
                                    None if gate is None else gate.to(dev), gated == "head")
         worst = ((out.cpu().to(F64) - want).abs() / slack).max().item()
         assert worst <= 1.0, worst
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("max_keys", [0, 1 << 13])
+def test_rows_without_a_position(gated, max_keys):
+    """A negative position: no key, head outputs of zero, with one run of keys and with several."""
+    g = torch.Generator().manual_seed(5)
+    T, H, dim, vdim, dev = 3, 4, 64, 32, "cuda"
+    cache = torch.randn(20, 1, BS, KR + RD, generator=g).to(BF16).to(dev)
+    q = torch.randn(T, H * (dim + RD), generator=g).to(BF16).to(dev)
+    uk, uv = (torch.randn(H, n, KR, generator=g).to(BF16).to(dev) for n in (dim, vdim))
+    gate = torch.randn(T, H, generator=g).to(BF16).to(dev) if gated else None
+    out = torch.full((T, H * vdim), 7.0, dtype=BF16, device=dev)
+    latent.latent_decode_heads(q, uk, uv, cache, torch.arange(20, dtype=I32, device=dev)[None, :].repeat(T, 1).contiguous(),
+                               torch.tensor([-1, 300, -70], dtype=I32, device=dev), RD, 0.1, 0, torch.randn(320, RD, generator=g).to(dev),
+                               True, out, max_keys, None, gate, True)
+    assert (out[[0, 2]] == 0).all() and torch.isfinite(out).all() and (out[1] != 0).any()

@@ -72,3 +72,33 @@ def test_latent_tiles(H, window, bs, dims, inter):
     latent.latent_attn_rows(qd[order].contiguous(), ql[:, order].contiguous(), cd, tables[:2].contiguous(), cu,
                             pos[order].contiguous(), *args, out, sinks=sd)
     check(out, order)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kr,rd,dtype", [(512, 64, BF16), (128, 64, BF16), (512, 32, BF16), (64, 20, torch.float32)])
+@pytest.mark.parametrize("sinks", [False, True])
+def test_rows_without_a_position(kr, rd, dtype, sinks):
+    """A negative position (a row that pads a step): no key, results of zero in every form, the rows beside it as without it."""
+    g = torch.Generator().manual_seed(kr + rd)
+    H, T, bs, N, dev = 5, 4, 16, 700, "cuda"
+    pos = [699, -1, 300, -70]
+    cache = torch.randn(N // bs + 1, 1, bs, kr + rd, generator=g).to(dtype)
+    tables = torch.arange(N // bs + 1, dtype=I32)[None, :].repeat(T, 1).contiguous()
+    q, q_lat = torch.randn(T, H * (32 + rd), generator=g).to(dtype), (torch.randn(H, T, kr, generator=g) * 0.3).to(dtype)
+    cs = torch.randn(N, rd, generator=g)
+    sk = torch.randn(H, generator=g) if sinks else None
+
+    def run(rows, max_keys, device):
+        o = torch.full((H, len(rows), kr), 7.0, dtype=dtype, device=device)
+        to = lambda t: None if t is None else t.to(device)  # noqa: E731
+        latent.latent_attn_rows(to(q[rows].contiguous()), to(q_lat[:, rows].contiguous()), to(cache), to(tables[rows]), None,
+                                torch.tensor([pos[i] for i in rows], dtype=I32, device=device), H, 32, rd, kr, 0.1, 0, to(cs), True, o,
+                                max_keys=max_keys, sinks=to(sk))
+        return o.cpu().float()
+
+    want = run([0, 2], 0, "cpu")
+    for max_keys in (0, 1 << 14):
+        got = run([0, 1, 2, 3], max_keys, dev)
+        assert (got[:, [1, 3]] == 0).all()
+        # bf16: the query's rotated part, weights and results are rounded, 2^-8 each, and a score is a few units large
+        assert (got[:, [0, 2]] - want).abs().max() <= (2.0 ** -6 if dtype == BF16 else 1e-4) * want.abs().max()
