@@ -1,20 +1,21 @@
 """Decode rows on cached latents, the whole layer part (latent_decode_heads: fold, attention in runs, values with gates) against
-64 bits: one row, rows around sixteen, one run and several, query and value sizes, gates, strided queries."""
+64 bits: one row, rows around sixteen and many, one run and up to 64, query and value sizes, gates, strided queries, windows, rotation."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
+from dgi.models import latent_mixer
 from dgi.ops import latent
 
 F64, BF16, I32 = torch.float64, torch.bfloat16, torch.int32
 KR, RD, BS = 512, 64, 16
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("T", [1, 15, 16, 17, 40])
-@pytest.mark.parametrize("H,dim,vdim,gated", [(4, 64, 128, None), (3, 32, 16, "head"), (33, 96, 48, "element"), (2, 128, 112, None)])
-def test_decode_heads(T, H, dim, vdim, gated):
+def compare(T, H, dim, vdim, gated, keys=(0, 1 << 12), window=0, dims=0, inter=True, N=330, layer=False, pos=None):
+    """latent_decode_heads (or the layer around it) against 64 bits for rows at positions spread over N."""
     g = torch.Generator().manual_seed(T * H)
-    N, qk = 330, dim + RD
+    qk = dim + RD
     rows = torch.randn(N, KR + RD, generator=g).to(BF16)
     nblk = -(-N // BS)
     perm = torch.randperm(nblk, generator=g).to(I32)
@@ -26,17 +27,25 @@ def test_decode_heads(T, H, dim, vdim, gated):
     uk, uv = ((torch.randn(H, n, KR, generator=g) * KR ** -0.5).to(BF16) for n in (dim, vdim))
     sinks = torch.randn(H, generator=g)
     gate = None if gated is None else torch.randn(T, H if gated == "head" else H * vdim, generator=g).to(BF16)
-    pos = [(37 * t + 5) % N for t in range(T)]
+    pos = [(37 * t + 5) % N for t in range(T)] if pos is None else pos
+    ang = torch.arange(N, dtype=F64)[:, None] * torch.exp(-torch.arange(max(dims, 2) // 2, dtype=F64) / 8)
+    cs = torch.cat([ang.cos(), ang.sin()], 1).float() if dims else None
     scale = qk ** -0.5
+    qr = q.view(T, H, qk)[:, :, dim:].float()
+    if dims:
+        qr = latent.rotate_ref(qr, cs[torch.tensor(pos)], dims, inter)
+    qr = qr.to(BF16).to(F64)                                 # the rotated part is rounded once
     want, slack = torch.zeros(T, H * vdim, dtype=F64), torch.zeros(T, H * vdim, dtype=F64)
     e = 2.0 ** -8                                            # a rounding to bf16, at most, of a number's size
     for t, p in enumerate(pos):
-        c, r = rows[:p + 1, :KR].to(F64), rows[:p + 1, KR:].to(F64)
-        qq = q[t].to(F64).view(H, qk)
-        ql = torch.einsum("hd,hdk->hk", qq[:, :dim], uk.to(F64))
-        s = (ql @ c.t() + qq[:, dim:] @ r.t()) * scale
+        lo = max(0, p - window + 1) if window else 0
+        c, r = rows[lo:p + 1, :KR].to(F64), rows[lo:p + 1, KR:].to(F64)
+        ql = torch.einsum("hd,hdk->hk", q[t].to(F64).view(H, qk)[:, :dim], uk.to(F64))
+        s = (ql @ c.t() + qr[t] @ r.t()) * scale
         w = torch.softmax(torch.cat([s, sinks.to(F64)[:, None]], 1), 1)[:, :-1]
         ds = (ql.abs() @ c.abs().t()) * scale * e            # the folded query is rounded: a score moves by this at most
+        if dims:                                             # a rotated value between two bf16 numbers may go either way
+            ds = ds + (qr[t].abs() @ r.abs().t()) * scale * 2 * e
         o, om = w @ c, (w * (e + ds + (w * ds).sum(1, keepdim=True))) @ c.abs()
         y = torch.einsum("hk,hvk->hv", o, uv.to(F64))
         ym = torch.einsum("hk,hvk->hv", om + e * o.abs(), uv.to(F64).abs()) + e * y.abs()
@@ -46,15 +55,55 @@ def test_decode_heads(T, H, dim, vdim, gated):
         want[t], slack[t] = (y * f).reshape(-1), (ym * f).reshape(-1) + 1e-5
     dev = "cuda"
     assert latent.decode_heads_ok(wide.to(dev)[:, :H * qk], T, dim, RD, KR, vdim, gate)
+    to = lambda x: None if x is None else x.to(dev)  # noqa: E731
     tables = perm[None, :].repeat(T, 1).contiguous().to(dev)
-    for max_keys in (0, 1 << 12):
+    positions = torch.tensor(pos, dtype=I32, device=dev)
+    qd = wide.to(dev)[:, :H * qk]
+    for max_keys in keys:
         out = torch.full((T, H * vdim), 7.0, dtype=BF16, device=dev)
-        latent.latent_decode_heads(wide.to(dev)[:, :H * qk], uk.to(dev), uv.to(dev), cache.to(dev), tables,
-                                   torch.tensor(pos, dtype=I32, device=dev), RD, scale, 0, None, True, out, max_keys, sinks.to(dev),
-                                   None if gate is None else gate.to(dev), gated == "head")
+        if layer:
+            m = SimpleNamespace(heads=H, dim=dim, rot_dim=RD, kv_rank=KR, vdim=vdim, qk_dim=qk, scale=scale, window=window, gate=gated,
+                                rot=SimpleNamespace(layout="interleaved" if inter else "half"), o_size=H * vdim, cache_dim=KR + RD)
+            wt = torch.zeros(T, -(-max(max_keys, N) // BS), dtype=I32, device=dev)
+            wt[:, :nblk] = tables
+            meta = SimpleNamespace(num_decode=T, num_prefill_tokens=0, dec_block_tables=wt, positions=positions)
+            out = latent_mixer.latent_heads(m, SimpleNamespace(uk=to(uk), uv=to(uv)), qd, to(cache), meta, to(cs), to(gate), to(sinks))
+        else:
+            latent.latent_decode_heads(qd, to(uk), to(uv), to(cache), tables, positions, RD, scale, window, to(cs), inter, out, max_keys,
+                                       to(sinks), to(gate), gated == "head")
         worst = ((out.cpu().to(F64) - want).abs() / slack).max().item()
         assert worst <= 1.0, worst
 
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 40])
+@pytest.mark.parametrize("H,dim,vdim,gated", [(4, 64, 128, None), (3, 32, 16, "head"), (33, 96, 48, "element"), (2, 128, 112, None)])
+def test_decode_heads(T, H, dim, vdim, gated):
+    compare(T, H, dim, vdim, gated)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H", [(96, 32), (90, 32), (128, 32), (129, 33), (250, 32), (256, 17)])
+def test_decode_heads_rows_per_workgroup(T, H):
+    """Steps whose value product takes eight and sixteen rows a workgroup, the last of them full and not."""
+    compare(T, H, 32, 32, "head")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,max_keys", [(1, 1 << 13), (3, 1 << 14), (7, 1 << 13)])
+def test_decode_heads_many_runs(T, max_keys):
+    """64 runs of keys (the most there are), some and most of them empty, and a number of runs that is no multiple of four."""
+    assert latent.tile_runs(T, 20, max_keys) == {1: 64, 3: 64, 7: 36}[T]
+    compare(T, 20, 64, 48, None, keys=(max_keys,), N=330 if T > 1 else 6)
+    compare(T, 20, 64, 48, None, keys=(max_keys,), N=5000, pos=[4999 - 611 * t for t in range(T)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [5, 100])
+@pytest.mark.parametrize("window,dims,inter,gated", [(0, 64, True, None), (100, 64, False, "head"), (70, 32, True, "element"), (33, 0, True, None)])
+def test_layer_with_windows_and_rotation(T, window, dims, inter, gated):
+    """The layer's part as a model calls it: windows, rotations of all and of some dims in both layouts, tables wider than the contexts."""
+    compare(T, 18, 64, 32, gated, keys=(0, 1 << 12), window=window, dims=dims, inter=inter, layer=True)
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("gated", [False, True])
