@@ -590,7 +590,10 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
 //   O^T [kr x 16 heads]     += C^T [kr x 32 keys] P^T [32 keys x 16 heads]      the same, C^T by transposing LDS reads
 //
 // A lane of S^T holds keys 4 g .. + 3 and 16 + 4 g .. + 3 of one head: taken in that order they are its operand of P^T, so
-// nothing is exchanged, and a wave keeps its own running softmax.  Chunk c (16 bytes) of a tile's row j lies at c ^ (j & 7):
+// nothing is exchanged, and a wave keeps its own running softmax.  P is taken in two bf16 parts, the rounded weights and what the rounding
+// took off: with one, results were further from 64 bits than the form above (32 heads, the layer's part: 60 rows over some 90 keys 3.04e-3
+// against 2.99e-3, 32 rows over 2000 keys 3.041e-3 and 3.034e-3), because fewer, larger groups of keys share a maximum; with two 2.80e-3 and
+// 2.88e-3, for 1.5 us a layer.  Chunk c (16 bytes) of a tile's row j lies at c ^ (j & 7):
 // neither kind of read meets a bank twice.  At the end the two waves of a group exchange halves of O^T through LDS.
 // Keys past the last are copies of it with weight 0.  The widths are constants of the kernel: with loop bounds read at run
 // time the compiler kept neither the products' order nor the operands in registers.
@@ -760,6 +763,14 @@ __global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
     pf[1] = pack_bf16x2(x[0][2], x[0][3]);
     pf[2] = pack_bf16x2(x[1][0], x[1][1]);
     pf[3] = pack_bf16x2(x[1][2], x[1][3]);
+    u32x4 pl;                                          // what the rounding took off
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t hi = pf[2 * u + i];
+        pl[2 * u + i] = pack_bf16x2(x[u][2 * i] - __uint_as_float(hi << 16), x[u][2 * i + 1] - __uint_as_float(hi & 0xffff0000u));
+      }
     if (__any(corr != 1.f)) {                          // else no head's maximum moved: the sums keep their scale
 #pragma unroll
       for (int m = 0; m < NM; ++m)
@@ -774,6 +785,7 @@ __global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const u32x4 vf = {v[2 * i][0], v[2 * i][1], v[2 * i + 1][0], v[2 * i + 1][1]};
+        acc[m + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pl), acc[m + i], 0, 0, 0);
         acc[m + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), acc[m + i], 0, 0, 0);
       }
     }

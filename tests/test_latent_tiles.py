@@ -102,3 +102,33 @@ def test_rows_without_a_position(kr, rd, dtype, sinks):
         assert (got[:, [1, 3]] == 0).all()
         # bf16: the query's rotated part, weights and results are rounded, 2^-8 each, and a score is a few units large
         assert (got[:, [0, 2]] - want).abs().max() <= (2.0 ** -6 if dtype == BF16 else 1e-4) * want.abs().max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,n,max_keys", [(32, 90, 0), (17, 900, 0), (32, 900, 1 << 11)])
+def test_weights_keep_their_precision(monkeypatch, H, n, max_keys):
+    """No further from 64 bits than the form that holds the weights in fp32: what both round is the result.  Two such errors over 2e5
+    values differ by under one per cent; weights rounded to bf16 add two fifths."""
+    g = torch.Generator().manual_seed(H + n)
+    T, bs, dev = 12, 16, "cuda"
+    nblk = -(-n // bs)
+    cache = torch.randn(nblk, 1, bs, KR + RD, generator=g).to(BF16)
+    q, q_lat = torch.randn(T, H * (DIM + RD), generator=g).to(BF16), (torch.randn(H, T, KR, generator=g) * 0.3).to(BF16)
+    pos = torch.tensor([n - 1 - 3 * t for t in range(T)], dtype=I32)
+    scale = (DIM + RD) ** -0.5
+    rows = cache.view(-1, KR + RD).to(F64)
+    want = torch.empty(H, T, KR, dtype=F64)
+    for t, p in enumerate(pos.tolist()):
+        s = torch.cat([q_lat[:, t].to(F64), q[t].to(F64).view(H, DIM + RD)[:, DIM:]], 1) @ rows[:p + 1].t() * scale
+        want[:, t] = torch.softmax(s, 1) @ rows[:p + 1, :KR]
+    tables = torch.arange(nblk, dtype=I32)[None, :].repeat(T, 1).contiguous().to(dev)
+
+    def error():
+        out = torch.empty(H, T, KR, dtype=BF16, device=dev)
+        latent.latent_attn_rows(q.to(dev), q_lat.to(dev), cache.to(dev), tables, None, pos.to(dev), H, DIM, RD, KR, scale, 0, None, True,
+                                out, max_keys=max_keys)
+        return ((out.cpu().to(F64) - want).norm() / want.norm()).item()
+
+    tiles = error()
+    monkeypatch.setattr(latent, "MFMA_ROWS", False)
+    assert tiles <= 1.05 * error()
