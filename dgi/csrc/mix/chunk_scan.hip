@@ -137,7 +137,7 @@ struct Lay {
   static constexpr int NC = NT <= 8 ? 2 : 1, W2 = NT <= 8 ? 2 : 1;
   static constexpr int NS = NT / 4;                            // preparing waves of 64 channels
   static constexpr int NA = NT == 4 ? 4 : 8;                   // sums side by side of a sum over the channels: state waves
-  static constexpr int NO = MODE == WKV ? 8 : 4;               // output waves
+  static constexpr int NO = MODE == WKV || (MODE == DELTA && NT == 8) ? 8 : 4;      // output waves (delta, 128 channels: with 4 results were 2 % further off than the loop's)
   // Waves: state, output, then gates and normaliser (or preparing waves), scores, (more) preparing waves: waves four apart share a SIMD,
   // and the scores' products are best beside the output waves', the fewest.
   static constexpr int SETS = CH && NT == 4 ? 2 : 1;           // channel decays: one set of preparing waves for the scores, one for the state
