@@ -177,7 +177,33 @@ def ssm_scan_ref(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0
     return y.reshape(T, inner)
 
 
-SCAN_CHUNK = int(os.environ.get("DGI_SCAN_CHUNK", "16"))       # 0: portions row by row unless a call asks for chunks
+SCAN_CHUNK = int(os.environ.get("DGI_SCAN_CHUNK", "16"))       # 0: portions row by row in every case (chunks have sixteen rows)
+# workgroups of the row-by-row form (sequence x head x 16 columns) from which steps stay with it, unless a call asks for chunks
+SCAN_CHUNK_BELOW = int(os.environ.get("DGI_SCAN_CHUNK_BELOW", str(1 << 40)))
+
+
+def scan_chunks(T: int, n_seq: int, heads: int, dv: int, dtype, chunked=None) -> bool:
+    """Whether ``ssm_scan`` takes the portions of a step of ``T`` rows in chunks on the GPU.
+
+    A third of the time per row, but some 80 rows' time more per portion, and once the heads outnumber the pipelines that find a
+    place on the chip they wait for each other: 64 columns, row by row against chunks, 4 portions, 16 heads, 72 rows 21, 18 us; 64
+    heads, 72 rows 32, 36, 128 rows 50, 43; 11 portions, 64 heads, 128 rows 114, 122, 200 rows 180, 171.  Known here are the
+    step's rows and sequences only; among more than eight each sequence is taken by its own length, by the lines of
+    ``apart_rows`` in ssm_scan.hip (112 and 144 there and here lie together), and few rows on average but many rows are decode rows
+    beside long portions."""
+    if SCAN_CHUNK <= 0:
+        return False
+    if chunked is not None:
+        return bool(chunked)
+    if dtype == torch.float32 or n_seq * heads * -(-dv // 16) >= SCAN_CHUNK_BELOW:
+        return False
+    units = n_seq * heads * -(-dv // 64)
+    if units <= 128:
+        return T > 64 * n_seq or T - n_seq >= 512
+    rows = 112 if units <= 256 else 144
+    if n_seq <= 8:
+        return T > rows * n_seq
+    return 4 * T > 3 * rows * n_seq or (T - n_seq >= 512 and T <= 48 * n_seq)
 
 
 def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads: int, dv: int,
@@ -195,23 +221,8 @@ def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, se
     if _native(xbc):
         T, n_seq = xbc.shape[0], seq_slots.shape[0]
         y = torch.empty(T, heads * dv, dtype=torch.float32, device=xbc.device)
-        if chunked is None:
-            # a third of the time per row, but some 80 rows' time more per portion, and once the heads outnumber the
-            # pipelines that find a place on the chip they wait for each other: 64 columns, row by row against chunks, 4
-            # portions, 16 heads, 72 rows 21, 18 us; 64 heads, 72 rows 32, 36, 128 rows 50, 43; 11 portions, 64 heads, 128
-            # rows 114, 122, 200 rows 180, 171.  Known here are the step's rows and sequences only; among more than eight
-            # each sequence is taken by its own length, and few rows on average but many rows are decode rows beside
-            # long portions
-            units = n_seq * heads * -(-dv // 64)
-            rows = 64 if units <= 128 else 112 if units <= 256 else 144
-            if rows == 64:
-                chunked = T > 64 * n_seq or T - n_seq >= 512
-            elif n_seq <= 8:
-                chunked = T > rows * n_seq
-            else:
-                chunked = 4 * T > 3 * rows * n_seq or (T - n_seq >= 512 and T <= 48 * n_seq)
-            chunked = chunked and SCAN_CHUNK > 0 and dt_raw.dtype != torch.float32
-        _call("ssm_scan", y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G, bool(chunked))
+        chunked = scan_chunks(T, n_seq, heads, dv, dt_raw.dtype, chunked)
+        _call("ssm_scan", y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G, chunked)
         return y
     return ssm_scan_ref(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, seq_slots, heads, dv, N, G)
 
