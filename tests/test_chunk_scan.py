@@ -165,7 +165,8 @@ def test_sizes(mode, D, V):
 @pytest.mark.parametrize("D,V,pad", [(18, 10, 0), (20, 8, 1), (200, 32, 0)])
 @pytest.mark.parametrize("mode", ["delta", "mlstm", "light", "ssm"])
 def test_rows_the_chunks_do_not_take(mode, D, V, pad):
-    """Key sizes that are no multiple of four or above 128 and rows off a four-element boundary: another kernel, the same result."""
+    """Key sizes that are no multiple of four or above 128 (ssm: 256, so 200 is one of its own) and rows off a four-element boundary: another
+    kernel, the same result."""
     d = make(mode, [70, 66], 4, D, V, torch.bfloat16, [0, 5], pad=pad)
     check(call(d), oracle(d))
 
@@ -273,3 +274,17 @@ def test_wkv_scales_beside_strong_decays(q, k):
     d["q"][:, 1::2] = 0.0
     y, wy = call(d)[0], oracle(d)[0]
     assert (y.to(F64) - wy).abs().max() <= 3e-5 * wy.abs().max()
+
+
+@pytest.mark.parametrize("mode,H,D,line", [("wkv", 52, 16, 136), ("wkv", 310, 16, 224), ("wkv", 11, 68, 104), ("ssm", 2, 20, 48), ("ssm", 14, 20, 112),
+                                           ("ssm", 28, 20, 144)])
+def test_portions_around_the_line_between_the_launches(mode, H, D, line):
+    """Among more than eight sequences portions of at most ``line`` rows go in a launch of their own; the line depends on the number of
+    workgroups (and, wkv, on the key size).  One row to either side of it, on average near it, and decode rows beside one long portion."""
+    V = D if mode == "wkv" else 17
+    for lens, H in (([line, line + 1, line - 1, 1, line, 2 * line + 200, line + 1, 15, line + 7, line + 16], H),
+                    ([1] * 30 + [line + 1, 700, line], -(-10 * H // 33))):
+        d = make(mode, lens, H, D, V, torch.bfloat16, [3 * (i % 2) for i in range(len(lens))], seed=H)
+        if mode == "ssm":
+            assert recur.scan_chunks(sum(lens), len(lens), H, V, torch.bfloat16)
+        check(call(d), oracle(d))

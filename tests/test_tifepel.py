@@ -348,7 +348,7 @@ def test_ssm_scan_portions_and_slots(device, dtype, geom):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("geom", [(4, 24, 20, 2), (2, 16, 130, 1)])
+@pytest.mark.parametrize("geom", [(4, 24, 20, 2), (2, 16, 130, 1), (2, 16, 132, 1)])      # 130: no multiple of four, row by row after all
 def test_chunked_scan_equals_one_pass(geom, monkeypatch):
     """The chunk-parallel form (local chunk states, serial pass over them, outputs per chunk) against
     the oracle: portions that end inside a chunk, a one-row sequence beside them, a continued sequence
