@@ -29,7 +29,7 @@
 // by k, substitution, update) or a preparing wave's arithmetic (wkv): a wave issues an instruction every four to five cycles at best, so
 // addresses are lane offsets kept in registers, and rows past the end a branch of their own.  Measured, a step of 2 prompts of 4096 rows in
 // all, 64 heads, states 64 x 64 (ssm 128 x 64), against the same token by token on the vector ALUs (linear_scan.hip, ssm_scan.hip):
-// delta 178 us (726), ssm 209 (637), wkv 230 (some 630), light 158 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 105 (322).
+// delta 178 us (726), ssm 209 (637), wkv 232 (some 630), light 158 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 103 (322).
 //
 // Precision: results and states are no further from 64 bits than the token loop's (2-norm over 1300 to 4096 rows: ssm 7.8e-8, the loop 8.0e-8;
 // delta 1.17e-7, 1.18e-7; wkv 9.8e-8, 1.01e-7).  Regrouping alone does not do that: with the sums over channels in two running sums, P and the decays
