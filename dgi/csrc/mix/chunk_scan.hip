@@ -32,7 +32,8 @@
 // delta 178 us (726), ssm 209 (637), wkv 232 (some 630), light 158 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 103 (322).
 //
 // Precision: results and states are no further from 64 bits than the token loop's (2-norm over 1300 to 4096 rows: ssm 7.8e-8, the loop 8.0e-8;
-// delta 1.17e-7, 1.18e-7; wkv 9.8e-8, 1.01e-7).  Regrouping alone does not do that: with the sums over channels in two running sums, P and the decays
+// delta 1.17e-7, 1.18e-7; wkv 9.8e-8, 1.01e-7; but states of wkv on bf16 rows 7.34e-8, 7.28e-8: the loop's products of bf16 keys and values
+// are exact, here a decayed key is rounded).  Regrouping alone does not do that: with the sums over channels in two running sums, P and the decays
 // rounded product by product and P u in 32 bits the same were 1.25e-7, 1.57e-7 and 1.30e-7.  So sums over channels are added as trees, a sum over
 // tokens starts with the oldest, the per-token decays and wkv's suffix products carry their rounding errors along, and P and P u are 64-bit
 // (four v_mfma_f64_16x16x4_f64 per chunk and output wave).  It costs 3 (delta) to 13 % (mlstm) of the time; wkv's was not the longest role.

@@ -599,7 +599,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
 // time the compiler kept neither the products' order nor the operands in registers.
 //
 // 32 rows x 32 heads over about 2000 keys each: 123 us (the form above, every row read for each 16 heads, C^T gathered in
-// single elements) -> 35, 2.1 TB/s; at four to five tiles a workgroup what is left is its first loads, one behind the
+// single elements) -> 36, 2.1 TB/s; at four to five tiles a workgroup what is left is its first loads, one behind the
 // other (position, page, tile), and the partial sums' 17 MB.
 __device__ __forceinline__ void load_lds16(const char* src, char* lds) {
   __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
