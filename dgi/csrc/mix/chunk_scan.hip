@@ -187,7 +187,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
   if (n <= a.skip_rows) return;
   const int slot = a.seq_slots[seq];
   // ssm in segments (see below): 1 the state of a segment from nothing, to the workspace; 2 outputs from the state found there
-  bool stored = a.positions[row0] > 0, last = true;
+  bool stored = MODE == SSM ? a.positions[row0] != 0 : a.positions[row0] > 0, last = true;      // as the loops of their files
   if (MODE == SSM && a.pass) {
     row0 += seg * a.seg_rows;
     n -= seg * a.seg_rows;
@@ -1050,7 +1050,7 @@ __global__ __launch_bounds__(256) void ssm_segments_kernel(float* __restrict__ w
   const int seq = blockIdx.x, head = blockIdx.y, e = blockIdx.z * 256 + threadIdx.x;
   const int row0 = seq_row0[seq], n = seq_row0[seq + 1] - row0;
   if (e >= per_head || n <= skip_rows) return;
-  float S = positions[row0] > 0 ? state[((size_t)seq_slots[seq] * H + head) * per_head + e] : 0.f;
+  float S = positions[row0] != 0 ? state[((size_t)seq_slots[seq] * H + head) * per_head + e] : 0.f;
   const int used = (n + seg_rows - 1) / seg_rows;
   for (int i = 0; i < used; ++i) {
     float* p = ws + (((size_t)seq * segs + i) * H + head) * per_head + e;

@@ -288,3 +288,12 @@ def test_portions_around_the_line_between_the_launches(mode, H, D, line):
         if mode == "ssm":
             assert recur.scan_chunks(sum(lens), len(lens), H, V, torch.bfloat16)
         check(call(d), oracle(d))
+
+
+@pytest.mark.parametrize("lens", [[90, 70], [1500, 40]])
+def test_ssm_takes_only_position_zero_as_a_start(lens):
+    """A portion at any other position reads its state, whole or in segments: the same as row by row."""
+    d = make("ssm", lens, 1, 64, 32, torch.bfloat16, [-2000, 0], seed=4)
+    want = call(d, chunked=False)
+    check(call(d, chunked=True), [t.to(F64) for t in want])
+    assert not torch.allclose(want[0][:4], call(dict(d, past=[0, 0]), chunked=False)[0][:4])
