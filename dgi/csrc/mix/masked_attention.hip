@@ -169,7 +169,7 @@ __global__ __launch_bounds__(64) void masked_attn_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
-// Grouped kernel: one workgroup per (row, kv head) serves all R = H / G query heads of the group
+// Grouped kernel (fp32, and bf16 heads of more than 128 dims): one workgroup per (row, kv head) serves all R = H / G query heads of the group
 // from ONE pass over the keys, with 16-byte cache reads.  Eight waves take 64-key tiles round
 // robin; in a tile a 16-lane group owns one key at a time (lane c of the group its 16-byte chunk c,
 // against the same chunk of the R queries in registers), so one wave instruction reads four whole K
@@ -442,7 +442,263 @@ __global__ __launch_bounds__(64 * GNW) void masked_attn_group_kernel(
   }
 }
 
-// combines the runs of masked_attn_group_kernel; grid (rows, H)
+// ---------------------------------------------------------------------------------------------
+// The grouped kernel for bf16 heads of up to 128 dims.  Bounded by the cached rows' bytes, so what counts is how many of them are
+// under way: a wave holds one tile of 64 keys in flight all the time.  The keys' registers are loaded again with the tile's values
+// as the products consume them, those again with the next tile's keys as the values are summed, and the pages of the next tile are
+// looked up a tile ahead.  32 rows of 1500 to 2500 keys, 8 groups of 4 heads of 128 dims, cap, sinks and gate: 56 us (the kernel above with
+// 16 lanes per key on the vector ALUs, each batch of rows waited for: 68), 4.7 TB/s in all, 5.8 while the longest row is read; 100 rows of
+// 600 keys, at most 1024 in a block: 87 -> 57; 1 row of 7000 keys of 64 dims in 13 runs: 31 -> 20.  Scores are matrix products (16 keys by up to 16 heads, products of bf16 numbers exact, sums in fp32);
+// they change to one key per lane through LDS for the softmax, whose weights and the values' sums stay in fp32 on the vector ALUs.
+// NW waves take tiles in turn; runs over gridDim.z as above.
+template <int CTRL>
+__device__ __forceinline__ float row_max_step(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false)));
+}
+// maximum over the wave (every lane gets it)
+__device__ __forceinline__ float wave_max_all(float v) {
+  v = row_max_step<0x128>(v);
+  v = row_max_step<0x124>(v);
+  v = row_max_step<0x122>(v);
+  v = row_max_step<0x121>(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+struct RowsArgs {
+  const uint16_t *q, *k, *v, *gate;
+  uint16_t* out;
+  const int *block_tables, *cu_seqlens, *positions;
+  const float *dist_bias, *sinks, *head_scale;
+  float *part_o, *part_ml;
+  int q_stride, bt_stride, n_seqs, H, dk, dv, bs, mask, gate_stride, out_stride, n_dist, gate_heads;
+  float scale, softcap;
+};
+
+// R: heads of a group, rounded up to 2, 4 or 8; D: dims, rounded up to 64 or 128
+template <int R, int D, int NW>
+__global__ __launch_bounds__(64 * NW, R == 8 ? 2 : 3) void masked_attn_tiles_kernel(const RowsArgs a) {
+  constexpr int KS = D / 32;                         // loads (and products) of a block of 16 keys
+  constexpr int LK = D / 8, KL = 64 / LK;            // lanes of a value row, rows of a load
+  constexpr int VB = 16 / KL;                        // loads of 16 value rows
+  constexpr int QP = D + 8;
+  __shared__ __attribute__((aligned(16))) uint16_t qs[R * QP];
+  __shared__ __attribute__((aligned(16))) float ps[NW][64 * R];        // scores, then weights: [key][head]
+  __shared__ int vs[NW][2][64];                      // cache slot of each key of the wave's tile, and of the next one
+  __shared__ float cm[NW][R], cl[NW][R];
+  __shared__ float co[NW][R][D];
+  const int row = blockIdx.x, kvh = blockIdx.y, G = gridDim.y, r = a.H / G;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int n16 = lane & 15, g = lane >> 4;
+  const int lc = lane & (LK - 1), lg = lane / LK;
+  const int dk = a.dk, dv = a.dv, bs = a.bs;
+
+  int seq = row;
+  if (a.cu_seqlens) {
+    int lo = 0, hi = a.n_seqs - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (a.cu_seqlens[mid] <= row) lo = mid; else hi = mid - 1;
+    }
+    seq = lo;
+  }
+  const int* bt = a.block_tables + (size_t)seq * a.bt_stride;
+  const int pos = a.positions[row];
+  const int first = a.mask > 0 ? (pos / a.mask) * a.mask : (a.mask < 0 ? max(0, pos + a.mask + 1) : 0);
+  const int ntiles = (pos - first) / 64 + 1;
+  const int tpr = (ntiles + (int)gridDim.z - 1) / (int)gridDim.z;      // tiles per run
+  const int t_end = min(ntiles, ((int)blockIdx.z + 1) * tpr);
+  int tile = blockIdx.z * tpr + w;
+  // slot of this lane's key of a tile; lanes past the last key point at it: every load stays in bounds
+  auto slot = [&](int t) {
+    const int kq = min(first + t * 64 + lane, pos);
+    return (bt[kq / bs] * G + kvh) * bs + kq % bs;
+  };
+  const int slot0 = slot(min(tile, ntiles - 1));
+
+  const uint16_t* qp = a.q + (size_t)row * a.q_stride + (size_t)kvh * r * dk;
+  for (int e = tid; e < R * D; e += 64 * NW) {
+    const int i = e / D, c = e % D;
+    qs[i * QP + c] = i < r && c < dk ? qp[i * dk + c] : 0;
+  }
+  __syncthreads();
+  u32x4 qf[KS];                                      // query n16 (0 past R), dims 32 s + 8 g
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+    qf[s] = n16 < R ? *reinterpret_cast<const u32x4*>(&qs[(n16 < R ? n16 : 0) * QP + 32 * s + 8 * g]) : u32x4{0u, 0u, 0u, 0u};
+
+  float m[R], l[R], o[R][8];                         // l: this lane's keys alone
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    m[i] = -__builtin_inff();
+    l[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[i][j] = 0.f;
+  }
+  float* psw = ps[w];
+  auto meet = [] {                                   // the wave's LDS writes before, its reads after
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  static_assert(KS == VB, "16 keys and 16 values take the same registers");
+  u32x4 raw[4][KS];
+  // chunks past a row's end: its last one again (keys: zeros when they are used; values: sums that nobody reads)
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  int ck[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) ck[s] = min(32 * s + 8 * g, dk - 8);
+  const int cv = min(8 * lc, dv - 8);
+  auto load_k = [&](const int* sl, int u) {          // keys 16 u ..
+    const uint16_t* p = a.k + (size_t)sl[16 * u + n16] * dk;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) raw[u][s] = *reinterpret_cast<const u32x4*>(p + ck[s]);
+  };
+  auto load_v = [&](const int* sl, int u) {
+#pragma unroll
+    for (int x = 0; x < VB; ++x)
+      raw[u][x] = *reinterpret_cast<const u32x4*>(a.v + (size_t)sl[16 * u + KL * x + lg] * dv + cv);
+  };
+  auto add_v = [&](int u) {
+#pragma unroll
+    for (int x = 0; x < VB; ++x) {
+      float f[8], p[R];
+      unpack8(raw[u][x], f);
+#pragma unroll
+      for (int i = 0; i < R; ++i) p[i] = psw[(16 * u + KL * x + lg) * R + i];      // 0 past the last key
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[i][j] += p[i] * f[j];
+    }
+  };
+  if (tile < t_end) {
+    vs[w][0][lane] = slot0;
+    meet();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load_k(vs[w][0], u);
+    for (int cur = 0;; cur ^= 1) {
+      const bool more = tile + NW < t_end;
+      const int next = slot(min(tile + NW, ntiles - 1));
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (dk < D) {
+#pragma unroll
+          for (int s = 0; s < KS; ++s) raw[u][s] = 32 * s + 8 * g < dk ? raw[u][s] : zero;
+        }
+        f32x4 sc = {0.f, 0.f, 0.f, 0.f};             // keys 16 u + 4 g + i, head n16
+#pragma unroll
+        for (int s = 0; s < KS; ++s) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(raw[u][s]), as_bf16x8(qf[s]), sc, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);           // a block's values take the place of its keys
+        load_v(vs[w][cur], u);
+        if (n16 < R) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) psw[(16 * u + 4 * g + i) * R + n16] = sc[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      meet();
+      const int key = first + tile * 64 + lane;
+      const bool ok = key <= pos;
+      float p[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        p[i] = 0.f;
+        if (i < r) {
+          float s = -__builtin_inff();
+          if (ok) {
+            s = psw[lane * R + i] * a.scale;
+            if (a.head_scale) s *= a.head_scale[kvh * r + i];
+            if (a.dist_bias) s += a.dist_bias[(size_t)min(pos - key, a.n_dist - 1) * a.H + kvh * r + i];
+            if (a.softcap > 0.f) s = a.softcap * tanhf(s / a.softcap);
+          }
+          const float m_new = fmaxf(m[i], wave_max_all(s));      // the tile's first key (lane 0) is visible: finite
+          const float corr = expf(m[i] - m_new);
+          p[i] = ok ? expf(s - m_new) : 0.f;
+          l[i] = l[i] * corr + p[i];
+          m[i] = m_new;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) o[i][j] *= corr;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < R; ++i) psw[lane * R + i] = p[i];      // over the lane's own scores
+      vs[w][cur ^ 1][lane] = next;
+      meet();
+      if (!more) break;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        add_v(u);
+        __builtin_amdgcn_sched_barrier(0);
+        load_k(vs[w][cur ^ 1], u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      meet();
+      tile += NW;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      add_v(u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // lane groups -> lane group 0, then waves -> LDS
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    l[i] = wave_sum(l[i]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+#pragma unroll
+      for (int s = LK; s < 64; s *= 2) o[i][j] += __shfl_xor(o[i][j], s, 64);
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      cm[w][i] = m[i];
+      cl[w][i] = l[i];
+    }
+  }
+  if (lg == 0) {
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) co[w][i][8 * lc + j] = o[i][j];
+  }
+  __syncthreads();
+  for (int idx = tid; idx < r * dv; idx += 64 * NW) {
+    const int i = idx / dv, d = idx - i * dv;
+    const int head = kvh * r + i;
+    float M = a.sinks && !a.part_o ? a.sinks[head] : -__builtin_inff();
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, cm[ww][i]);
+    float L = a.sinks && !a.part_o ? expf(a.sinks[head] - M) : 0.f, O = 0.f;      // the sink: one more term of the denominator
+    if (M != -__builtin_inff()) {                    // an empty run leaves zeros
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) {
+        const float f = expf(cm[ww][i] - M);         // waves without a tile: exp(-inf) = 0
+        L += cl[ww][i] * f;
+        O += co[ww][i][d] * f;
+      }
+    }
+    if (a.part_o) {
+      const size_t at = ((size_t)blockIdx.z * gridDim.x + row) * a.H + head;
+      a.part_o[at * dv + d] = O;
+      if (d == 0) {
+        a.part_ml[2 * at] = M;
+        a.part_ml[2 * at + 1] = L;
+      }
+      continue;
+    }
+    float v = O / L;
+    if (a.gate) v *= 1.f / (1.f + expf(-bf16_to_f32(a.gate[(size_t)row * a.gate_stride + (a.gate_heads ? (size_t)head : (size_t)head * dv + d)])));
+    a.out[(size_t)row * a.out_stride + (size_t)head * dv + d] = f32_to_bf16(v);
+  }
+}
+
+// combines the runs of the two kernels above; grid (rows, H)
 template <typename T>
 __global__ __launch_bounds__(128) void masked_attn_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                  int nsplit, int dv, const float* __restrict__ sinks,
@@ -467,6 +723,31 @@ __global__ __launch_bounds__(128) void masked_attn_reduce_kernel(const float* __
     if (gate) v *= 1.f / (1.f + expf(-ldf<T>(gate + (size_t)row * gate_stride + (gate_heads ? (size_t)head : (size_t)head * dv + d))));
     stf<T>(out + (size_t)row * out_stride + (size_t)head * dv + d, v);
   }
+}
+
+template <int R, int D>
+void launch_tiles_dims(const RowsArgs& a, int rows, int G, int nsplit, hipStream_t s) {
+  // a workgroup per compute unit or fewer: eight waves each (30 rows of 2000 keys, 8 groups of 4 heads of 64 dims: 14.9 us, with four
+  // waves 16.8); more of them: four, so that more workgroups share a unit (128 rows of 500 keys, groups of 2: 30.4, with eight 30.9)
+  if ((long long)rows * G * nsplit <= 256) masked_attn_tiles_kernel<R, D, 8><<<dim3(rows, G, nsplit), 512, 0, s>>>(a);
+  else masked_attn_tiles_kernel<R, D, 4><<<dim3(rows, G, nsplit), 256, 0, s>>>(a);
+}
+
+template <int R>
+void launch_tiles_heads(const RowsArgs& a, int rows, int G, int nsplit, hipStream_t s) {
+  if (a.dk <= 64 && a.dv <= 64) launch_tiles_dims<R, 64>(a, rows, G, nsplit, s);
+  else launch_tiles_dims<R, 128>(a, rows, G, nsplit, s);
+}
+
+void launch_tiles(RowsArgs a, int rows, int G, int nsplit, hipStream_t s) {
+  const int r = a.H / G;
+  if (nsplit < 2) a.part_o = a.part_ml = nullptr;
+  if (r <= 2) launch_tiles_heads<2>(a, rows, G, nsplit, s);
+  else if (r <= 4) launch_tiles_heads<4>(a, rows, G, nsplit, s);
+  else launch_tiles_heads<8>(a, rows, G, nsplit, s);
+  if (nsplit > 1)
+    masked_attn_reduce_kernel<uint16_t><<<dim3(rows, a.H), 128, 0, s>>>(a.part_o, a.part_ml, nsplit, a.dv, a.sinks, a.gate, a.gate_stride,
+                                                                        a.gate_heads, a.out, a.out_stride);
 }
 
 template <typename T, int R, int VP>
@@ -498,11 +779,13 @@ int dispatch_group(int r, int vpn, const void* q, int q_stride, const void* k_ca
   return launch_group<T, RV, VPV>(q, q_stride, k_cache, v_cache, block_tables, bt_stride, cu_seqlens, n_seqs, \
                                   positions, rows, H, G, dk, dv, bs, scale, mask, gate, gate_stride, out, out_stride, dist_bias, \
                                   n_dist, softcap, sinks, head_scale, gate_heads, nsplit, part_o, part_ml, s)
-  if (vpn == 1) {
-    if (r == 1) DGI_GRP(1, 1);
-    if (r == 2) DGI_GRP(2, 1);
-    if (r <= 4) DGI_GRP(4, 1);
-    DGI_GRP(8, 1);
+  if constexpr (sizeof(T) == 4) {                    // bf16 heads of up to 128 dims: masked_attn_tiles_kernel
+    if (vpn == 1) {
+      if (r == 1) DGI_GRP(1, 1);
+      if (r == 2) DGI_GRP(2, 1);
+      if (r <= 4) DGI_GRP(4, 1);
+      DGI_GRP(8, 1);
+    }
   }
   if (r == 1) DGI_GRP(1, 2);
   if (r == 2) DGI_GRP(2, 2);
@@ -531,10 +814,24 @@ extern "C" int dgi_masked_attn_rows(const void* q, int q_stride, const void* k_c
   if (nsplit < 1 || nsplit > 65535 || (nsplit > 1 && (!part_o || !part_ml))) return -6;
   if (dist_bias && n_dist < 1) return -5;
   {
-    // grouped kernel where the geometry allows (see masked_attn_group_kernel)
+    // grouped kernels where the geometry allows (see masked_attn_tiles_kernel and masked_attn_group_kernel)
     const int E = is_f32 ? 4 : 8, r = H / G;
     const int vpn = (std::max(dk, dv) + 16 * E - 1) / (16 * E);
     const bool aligned = ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0;
+    if (!is_f32 && dk % 8 == 0 && dv % 8 == 0 && r <= 8 && vpn == 1 && aligned && G <= 65535) {
+      RowsArgs a;
+      a.q = (const uint16_t*)q; a.k = (const uint16_t*)k_cache; a.v = (const uint16_t*)v_cache; a.gate = (const uint16_t*)gate;
+      a.out = (uint16_t*)out;
+      a.block_tables = block_tables; a.cu_seqlens = cu_seqlens; a.positions = positions;
+      a.dist_bias = dist_bias; a.sinks = sinks; a.head_scale = head_scale;
+      a.part_o = part_o; a.part_ml = part_ml;
+      a.q_stride = q_stride; a.bt_stride = bt_stride; a.n_seqs = n_seqs; a.H = H; a.dk = dk; a.dv = dv; a.bs = block_size; a.mask = mask;
+      a.gate_stride = gate_stride; a.out_stride = out_stride; a.n_dist = n_dist; a.gate_heads = gate_heads;
+      a.scale = scale; a.softcap = softcap;
+      launch_tiles(a, rows, G, nsplit, s);
+      DGI_CHECK_LAUNCH();
+      return 0;
+    }
     if (dk % E == 0 && dv % E == 0 && r <= 8 && vpn <= 2 && r * dv <= 1024 && aligned && G <= 65535) {
       const int rc = is_f32 ? dispatch_group<float>(r, vpn, q, q_stride, k_cache, v_cache, block_tables, bt_stride, cu_seqlens,
                                                     n_seqs, positions, rows, H, G, dk, dv, block_size, scale, mask, gate,
