@@ -13,11 +13,11 @@
 //                                 of an output sit in the same lane, so the activation is the product's epilogue;
 //                  down:          B = down [E, N, K], A = the rows gate-up left, row(place) = place.
 //
-// Three kernels.  Few rows per expert (decode steps): bounded by the expert weights' bytes.  A workgroup owns 64 weight
-// rows and up to 64 places; its four waves take a quarter of K each, weights and rows go from memory straight into
-// operand registers (16x16x32 products), and the four partial sums meet in LDS.  Many rows: tiles of 128 places by 128
-// weight rows, K in steps of 64 through two LDS stages (32x32x16 products).  Very many: 256 by 256, loaded to LDS
-// directly and multiplied by two groups of waves in turn.
+// Four kernels.  Few rows per expert (decode steps): bounded by the expert weights' bytes, so weights are read once, in whole
+// 128-byte lines, straight to LDS.  Up to 64 places a tile: the workgroups share the weight rows out evenly and stream them with
+// the tile's rows of A kept in registers; where those do not fit (or K is no multiple of 64), a workgroup owns 64 weight rows
+// and both operands come through LDS stages.  Many rows: tiles of 128 places by 128 weight rows, K in steps of 64 through two
+// LDS stages (32x32x16 products).  Very many: 256 by 256, loaded to LDS directly and multiplied by two groups of waves in turn.
 //
 // The tile a workgroup owns is found from seg alone, so the grid is sized for the worst split of the places over the
 // experts and a workgroup past the last tile leaves.  Weights are the A operand: a lane's result is four consecutive
@@ -130,6 +130,10 @@ struct GroupArgs {
   int mtiles;
 };
 
+__device__ __forceinline__ void load_lds16(const char* src, char* lds) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
 __device__ __forceinline__ void st_out4(uint16_t* p, const float* v, int n, bool vec) {
   if (vec && n == 4) {
     *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
@@ -140,93 +144,269 @@ __device__ __forceinline__ void st_out4(uint16_t* p, const float* v, int n, bool
   }
 }
 
-// ---- few rows per expert: MB blocks of 16 places, 64 weight rows (GLU: 32 outputs, gate and up), K over four waves
+// ---- few rows per expert, rows of A that do not fit the registers: up to 16 MB places x 64 weight rows (GLU: 32 outputs, gate and
+// up), a wave 16 of the weight rows, four stages of 64 of K.  16 experts, widths 4096 x 3584, top 4, 128 rows (64 places a tile): the
+// whole feed-forward 299 us, on 128 x 128 tiles 302.
 template <int MB, bool GLU>
 __global__ __launch_bounds__(256) void moe_group_rows_kernel(GroupArgs g) {
-  __shared__ __attribute__((aligned(16))) float part[4][MB * 4][64][4];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int D = 4;                                 // stages, of 64 of K each
+  constexpr int CA = MB == 4 ? 2 : 1;                  // a wave's loads of rows of A per stage
+  constexpr int STAGE = (4 + MB) * 2048;
+  __shared__ __attribute__((aligned(16))) char lds[D * STAGE];       // [stage][weights 64 | rows 16 MB], rows of 128 bytes
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int lr = lane & 15, lg = lane >> 4;
   int e, lo, hi;
   if (!find_tile<16 * MB>(g.seg, g.E, blockIdx.x % g.mtiles, e, lo, hi)) return;
-  const int nt = blockIdx.x / g.mtiles;
+  e = __builtin_amdgcn_readfirstlane(e);
+  const int K = g.K;
   constexpr int NO = GLU ? 32 : 64;                    // outputs per workgroup
-  const int n0 = nt * NO;
-  const uint16_t* B = g.b + (size_t)e * (GLU ? 2 : 1) * g.N * g.K;
-  // this lane's weight rows: block j of 16 (GLU: two gate blocks, then the matching up blocks)
-  const uint16_t* wp[4];
+  const int n0 = (blockIdx.x / g.mtiles) * NO;
+  // A load fills 8 LDS rows of 64 elements; piece c of LDS row r is piece c ^ (r & 7) of the row's 64 elements: reads of 8 rows spread
+  // over all banks.  GLU: LDS row r holds the gate (r & 2: up) row of output 2 (r >> 2) + (r & 1), so both projections of an output
+  // end up in one lane.
+  const int row8 = lane >> 3, c8 = ((lane & 7) ^ row8) * 8;
+  const char* B = reinterpret_cast<const char*>(g.b + (size_t)e * (GLU ? 2 : 1) * g.N * K);
+  const char* bp[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int n = n0 + (GLU ? (j & 1) : j) * 16 + lr;
-    wp[j] = B + ((size_t)min(n, g.N - 1) + (GLU && j >= 2 ? g.N : 0)) * g.K;
+  for (int i = 0; i < 2; ++i) {
+    const int r = 16 * w + 8 * i + row8;
+    const int n = min(n0 + (GLU ? 2 * (r >> 2) + (r & 1) : r), g.N - 1) + (GLU && (r & 2) ? g.N : 0);
+    bp[i] = B + (size_t)n * K * 2;
   }
-  const uint16_t* ap[MB];
+  const char* ap[CA];
+  int ai[CA];                                          // which 8 rows of A
+#pragma unroll
+  for (int i = 0; i < CA; ++i) {
+    ai[i] = (w + 4 * i) % (2 * MB);                    // MB 1: two waves load the same
+    const int place = min(lo + 8 * ai[i] + row8, hi - 1);
+    ap[i] = reinterpret_cast<const char*>(g.a + (size_t)(g.order ? g.order[place] / g.top : place) * g.a_stride);
+  }
+  auto load = [&](int s) {
+    char* st = lds + (s % D) * STAGE;
+    const int k = min(64 * s + c8, K - 8) * 2;         // pieces past the row's end: its last one (zeros when they are used)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) load_lds16(bp[i] + k, st + (2 * w + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < CA; ++i) load_lds16(ap[i] + k, st + 8192 + ai[i] * 1024);
+  };
+  f32x4 acc[MB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = (K + 63) >> 6;
+  auto step = [&](int s, auto LEFT_) {
+    constexpr int LEFT = decltype(LEFT_)::value;       // stages loaded after this one
+    if constexpr (LEFT == 2) { if constexpr (CA == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); }
+    else if constexpr (LEFT == 1) { if constexpr (CA == 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); }
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (LEFT == 2 && s + 3 < steps) load(s + 3);       // into the stage that every wave has read before the barrier
+    const char* st = lds + (s % D) * STAGE;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = lr * 128 + ((4 * h + lg) ^ (lr & 7)) * 16;
+      u32x4 fb = *reinterpret_cast<const u32x4*>(st + w * 2048 + at), fa[MB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) fa[i] = *reinterpret_cast<const u32x4*>(st + 8192 + i * 2048 + at);
+      if (s == steps - 1 && (K & 63)) {
+        const bool in = 64 * s + 32 * h + 8 * lg < K;
+        const u32x4 zero = {0u, 0u, 0u, 0u};
+        fb = in ? fb : zero;
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fa[i] = in ? fa[i] : zero;
+      }
+#pragma unroll
+      for (int i = 0; i < MB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(fb), as_bf16x8(fa[i]), acc[i], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // read, before the barrier after which the stage is loaded again
+  };
+  load(0);
+  if (steps > 1) load(1);
+  if (steps > 2) load(2);
+  int s = 0;
+  for (; s + 2 < steps; ++s) step(s, std::integral_constant<int, 2>{});
+  if (s + 1 < steps) step(s++, std::integral_constant<int, 1>{});
+  step(s, std::integral_constant<int, 0>{});
+  const bool vec = (g.N & 3) == 0 && ((uintptr_t)g.out & 7) == 0;
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
-    const int place = min(lo + 16 * i + lr, hi - 1);
-    const int row = g.order ? g.order[place] / g.top : place;
-    ap[i] = g.a + (size_t)row * g.a_stride;
-  }
-  f32x4 acc[MB][4];
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // K in steps of 32; wave w takes a contiguous quarter of them.  U steps are loaded together.
-  constexpr int U = MB == 1 ? 4 : 2;
-  const int steps = (g.K + 31) >> 5, per = (steps + 3) >> 2;
-  const int s_lo = w * per, s_hi = min(steps, s_lo + per);
-  const u32x4 zero = {0u, 0u, 0u, 0u};
-  for (int s = s_lo; s < s_hi; s += U) {
-    u32x4 wf[U][4], af[U][MB];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = (s + u) * 32 + 8 * lg;
-      const bool ok = s + u < s_hi && k < g.K;         // K is a multiple of 8: a chunk is whole or absent
-#pragma unroll
-      for (int j = 0; j < 4; ++j) wf[u][j] = ok ? *reinterpret_cast<const u32x4*>(wp[j] + k) : zero;
-#pragma unroll
-      for (int i = 0; i < MB; ++i) af[u][i] = ok ? *reinterpret_cast<const u32x4*>(ap[i] + k) : zero;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wf[u][j]), as_bf16x8(af[u][i]), acc[i][j], 0, 0, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(part[w][i * 4 + j][lane]) = acc[i][j];
-  __syncthreads();
-  auto total = [&](int blk) {
-    f32x4 t = *reinterpret_cast<const f32x4*>(part[0][blk][lane]);
-#pragma unroll
-    for (int ww = 1; ww < 4; ++ww) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(part[ww][blk][lane]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) t[r] += v[r];
-    }
-    return t;
-  };
-  constexpr int ITEMS = MB * (GLU ? 2 : 4);            // (block of places, block of 16 outputs)
-  const bool vec = (g.N & 3) == 0 && ((uintptr_t)g.out & 7) == 0;
-  for (int it = w; it < ITEMS; it += 4) {
-    const int i = GLU ? it >> 1 : it >> 2, j = GLU ? it & 1 : it & 3;
-    const int place = lo + 16 * i + lr, n = n0 + 16 * j + 4 * lg;
-    const f32x4 x = total(i * 4 + j);
-    float v[4];
+    const int place = lo + 16 * i + lr;
+    if (place >= hi) continue;
+    uint16_t* row = g.out + (size_t)place * g.N;
     if constexpr (GLU) {
-      const f32x4 y = total(i * 4 + 2 + j);
-      const float ps = g.pair_scale && place < hi ? g.pair_scale[g.order[place]] : 1.f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = glu_f(x[r] * ps, y[r] * ps, g.act, g.limit, g.alpha);
+      const float ps = g.pair_scale ? g.pair_scale[g.order[place]] : 1.f;
+      const int n = n0 + 8 * w + 2 * lg;
+      const float a = glu_f(acc[i][0] * ps, acc[i][2] * ps, g.act, g.limit, g.alpha);
+      const float b = glu_f(acc[i][1] * ps, acc[i][3] * ps, g.act, g.limit, g.alpha);
+      if (vec) {
+        if (n < g.N) *reinterpret_cast<uint32_t*>(row + n) = pack_bf16x2(a, b);
+      } else {
+        if (n < g.N) row[n] = f32_to_bf16(a);
+        if (n + 1 < g.N) row[n + 1] = f32_to_bf16(b);
+      }
     } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = x[r];
+      const int n = n0 + 16 * w + 4 * lg;
+      const float v[4] = {acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+      if (n < g.N) st_out4(row + n, v, min(4, g.N - n), vec);
     }
-    if (place < hi && n < g.N) st_out4(g.out + (size_t)place * g.N + n, v, min(4, g.N - n), vec);
+  }
+}
+
+// ---- few rows per expert: one workgroup per compute unit takes an equal run of the step's blocks (16 weight rows of one tile of places
+// each) and streams them without a gap.  Its eight waves split K; a wave keeps its part of the tile's rows of A in registers (they
+// come through the same ring of LDS stages first), so that all that moves is weights, and no wave waits for another but to add up
+// the partial sums of a block.  A load takes 8 rows x 128 bytes: one compute unit reads 54 GB/s that way, but 37 with the products'
+// own 16 rows x 64 bytes, and needs 22 of the chip's 5.8 TB/s.  Even shares: 64 weight rows a workgroup were 544 for 512 places.
+//
+// 16 experts, top 2, the whole feed-forward (16 to 20 us of it router, plan and combine), against weights straight to registers
+// (64 rows a workgroup, K over its waves; 128 x 128 tiles from 4 or 12 places an expert on):
+//   widths 2048 x 2048: 1 row 36 us -> 28, 8 rows 93 -> 69, 32 rows 110 -> 95 (4.9 TB/s in the products), 128 rows 130 -> 100
+//   widths 4096 x 3584: 1 row 70 -> 56, 8 rows 227 -> 185, 32 rows 285 -> 265 (5.6 TB/s)
+constexpr int STREAM_WGS = 256;
+
+// KS: stages of 64 of K per wave at the most.  K a multiple of 64.
+template <int MB, int KS, bool GLU>
+__global__ __launch_bounds__(512) void moe_group_stream_kernel(GroupArgs g) {
+  constexpr int D = MB == 4 ? 5 : 6;                   // stages of 16 rows x 64 of K, 2 KB each, per wave
+  // one array: with two, the compiler waits for all loads to LDS before every read of it
+  __shared__ __attribute__((aligned(16))) char lds[8 * D * 2048 + 2 * 8 * MB * 1024];      // [wave][stage], partial sums [2][wave][MB][64][4]
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int lr = lane & 15, lg = lane >> 4;
+  const int K = g.K;
+  constexpr int NO = GLU ? 8 : 16;                     // outputs of a block
+  const int nblk = (g.N + NO - 1) / NO;
+  // this workgroup's blocks
+  int tiles = 0;
+  for (int e0 = 0; e0 < g.E; e0 += 64) {
+    const int ee = e0 + lane;
+    tiles += ee < g.E ? (g.seg[ee + 1] - g.seg[ee] + 16 * MB - 1) / (16 * MB) : 0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) tiles += __shfl_xor(tiles, o, 64);
+  const long long total = (long long)__builtin_amdgcn_readfirstlane(tiles) * nblk;
+  int at = (int)(total * blockIdx.x / gridDim.x);
+  const int end = (int)(total * (blockIdx.x + 1) / gridDim.x);
+  // this wave's part of K: stages of 64
+  const int stages = K >> 6, per = (stages + 7) >> 3;
+  const int mine = max(0, min(per, stages - w * per));
+  const int row8 = lane >> 3;
+  const size_t koff = (size_t)w * per * 128 + (((lane & 7) ^ row8) << 4);
+  char* const rg = lds + w * (D * 2048);
+  float* const red = reinterpret_cast<float*>(lds + 8 * D * 2048);
+  auto sums = [&](int par, int ww, int i) { return reinterpret_cast<f32x4*>(red + ((par * 8 + ww) * MB + i) * 256 + 4 * lane); };
+  const int rd0 = lr * 128 + ((lg ^ (lr & 7)) << 4), rd1 = lr * 128 + (((4 + lg) ^ (lr & 7)) << 4);
+  int par = 0;
+  while (at < end) {
+    int e, lo, hi;
+    find_tile<16 * MB>(g.seg, g.E, at / nblk, e, lo, hi);
+    e = __builtin_amdgcn_readfirstlane(e);
+    const int b0 = at % nblk, nb = min(nblk - b0, end - at);
+    at += nb;
+    const char* ap[MB][2];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int place = min(lo + 16 * i + 8 * j + row8, hi - 1);
+        ap[i][j] = reinterpret_cast<const char*>(g.a + (size_t)(g.order ? g.order[place] / g.top : place) * g.a_stride) + koff;
+      }
+    const char* B = reinterpret_cast<const char*>(g.b + (size_t)e * (GLU ? 2 : 1) * g.N * K) + koff;
+    auto wrow = [&](int blk, int j) {                  // GLU: LDS row r holds the gate (r & 2: up) row of output 2 (r >> 2) + (r & 1)
+      const int r = 8 * j + row8;
+      const int n = min((b0 + blk) * NO + (GLU ? 2 * (r >> 2) + (r & 1) : r), g.N - 1) + (GLU && (r & 2) ? g.N : 0);
+      return B + (size_t)n * K * 2;
+    };
+    // stages in order: the rows of A, then the blocks' weights
+    const int all = (MB + nb) * mine;
+    int issued = 0, l_ks = 0, l_blk = 0, l_slot = 0;
+    const char *p0 = ap[0][0], *p1 = ap[0][1];
+    auto load = [&]() {
+      load_lds16(p0 + l_ks * 128, rg + l_slot * 2048);
+      load_lds16(p1 + l_ks * 128, rg + l_slot * 2048 + 1024);
+      ++issued;
+      l_slot = l_slot + 1 == D ? 0 : l_slot + 1;
+      if (++l_ks == mine) {
+        l_ks = 0;
+        ++l_blk;
+        if (l_blk < MB) {
+#pragma unroll
+          for (int i = 1; i < MB; ++i)
+            if (i == l_blk) { p0 = ap[i][0]; p1 = ap[i][1]; }
+        } else {
+          p0 = wrow(l_blk - MB, 0);
+          p1 = wrow(l_blk - MB, 1);
+        }
+      }
+    };
+    for (int i = 0; i < D && i < all; ++i) load();
+    int slot = 0;
+    auto take = [&](u32x4& f0, u32x4& f1) {
+      if (issued < all) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (D - 1)) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      const char* st = rg + slot * 2048;
+      f0 = *reinterpret_cast<const u32x4*>(st + rd0);
+      f1 = *reinterpret_cast<const u32x4*>(st + rd1);
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f0), "+v"(f1)::"memory");      // read, before the stage is loaded again
+      slot = slot + 1 == D ? 0 : slot + 1;
+      if (issued < all) load();
+    };
+    u32x4 af[MB][KS][2];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        if (ks < mine) take(af[i][ks][0], af[i][ks][1]);
+    for (int blk = 0; blk < nb; ++blk) {
+      f32x4 acc[MB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        if (ks < mine) {
+          u32x4 f0, f1;
+          take(f0, f1);
+#pragma unroll
+          for (int i = 0; i < MB; ++i) {
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(f0), as_bf16x8(af[i][ks][0]), acc[i], 0, 0, 0);
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(f1), as_bf16x8(af[i][ks][1]), acc[i], 0, 0, 0);
+          }
+        }
+#pragma unroll
+      for (int i = 0; i < MB; ++i) *sums(par, w, i) = acc[i];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        if (((blk * MB + i) & 7) != w) continue;       // uniform: one wave sums 16 places
+        f32x4 t = *sums(par, 0, i);
+#pragma unroll
+        for (int ww = 1; ww < 8; ++ww) t += *sums(par, ww, i);
+        const int place = lo + 16 * i + lr;
+        if (place < hi) {
+          uint16_t* row = g.out + (size_t)place * g.N;
+          const bool vec = (g.N & 3) == 0 && ((uintptr_t)g.out & 7) == 0;
+          if constexpr (GLU) {
+            const float ps = g.pair_scale ? g.pair_scale[g.order[place]] : 1.f;
+            const int n = (b0 + blk) * NO + 2 * lg;
+            const float x = glu_f(t[0] * ps, t[2] * ps, g.act, g.limit, g.alpha), y = glu_f(t[1] * ps, t[3] * ps, g.act, g.limit, g.alpha);
+            if (vec) {
+              if (n < g.N) *reinterpret_cast<uint32_t*>(row + n) = pack_bf16x2(x, y);
+            } else {
+              if (n < g.N) row[n] = f32_to_bf16(x);
+              if (n + 1 < g.N) row[n + 1] = f32_to_bf16(y);
+            }
+          } else {
+            const int n = (b0 + blk) * NO + 4 * lg;
+            const float v[4] = {t[0], t[1], t[2], t[3]};
+            if (n < g.N) st_out4(row + n, v, min(4, g.N - n), vec);
+          }
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      par ^= 1;
+    }
   }
 }
 
@@ -397,10 +577,6 @@ __device__ __forceinline__ bool find_wide(const int* __restrict__ seg, int E, in
     base += __shfl(inc, 63, 64);
   }
   return false;
-}
-
-__device__ __forceinline__ void load_lds16(const char* src, char* lds) {
-  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
 
 // Two neighbouring blocks of 16 outputs (four of each per lane) as one 16-byte store: lane group g ends up with eight
@@ -598,6 +774,18 @@ int launch_group(GroupArgs g, int places, int rows_per_tile, hipStream_t s) {
     moe_group_wide_kernel<GLU><<<padded, 512, 0, s>>>(g, ntn);
   } else if (bm == 128) {
     moe_group_tiles_kernel<GLU><<<padded, 256, 0, s>>>(g, ntn);
+  } else if (g.K % 64 == 0 && bm * g.K <= 1 << 17) {     // a tile's rows of A fill half the registers of a compute unit at the most
+    const int ks = (g.K / 64 + 7) / 8;                   // at most 16, 8, 4
+    if (bm == 16) {
+      if (ks <= 4) moe_group_stream_kernel<1, 4, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+      else if (ks <= 8) moe_group_stream_kernel<1, 8, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+      else moe_group_stream_kernel<1, 16, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+    } else if (bm == 32) {
+      if (ks <= 4) moe_group_stream_kernel<2, 4, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+      else moe_group_stream_kernel<2, 8, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+    } else {
+      moe_group_stream_kernel<4, 4, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+    }
   } else if (bm == 64) {
     moe_group_rows_kernel<4, GLU><<<(int)blocks, 256, 0, s>>>(g);
   } else if (bm == 32) {

@@ -15,8 +15,8 @@ Two evaluation paths on the GPU, same result up to summation order:
 * bf16: the pairs are sorted by expert on the device (``moe_plan``), two grouped matrix-core products
   (``moe_group``, gate-up with the activation as its epilogue, then down) walk the experts' segments, and a
   combine kernel gathers each token's routes in their fixed order (deterministic, no atomics, no host round
-  trip: the same path inside and outside captured graphs).  Tiles of 16 to 64 places with K split over the
-  waves when experts have few rows (bounded by the weights' bytes), of 128 or 256 places otherwise;
+  trip: the same path inside and outside captured graphs).  Tiles of 16 to 64 places whose weights are streamed
+  when experts have few rows (bounded by the weights' bytes), of 128 or 256 places otherwise;
 * fp32 and widths that are no multiple of 8 — few rows (and every step inside a captured graph): workgroups own
   (expert, output tile) and walk the pairs that chose the expert; many rows: one vendor GEMM pair per
   expert over its sorted segment.
@@ -161,17 +161,22 @@ def grouped_ok(h, gate_up, down) -> bool:
 
 def group_tile(pairs: int, experts: int, weights: int) -> int:
     """Places per tile of the grouped products, by the mean number of pairs of an expert and an expert's ``weights``
-    (elements of one projection: large experts give the big tiles enough workgroups at fewer rows).
+    (elements of one projection: large experts give the biggest tiles enough workgroups at fewer rows).
 
-    256 against 128, 16 experts, the whole feed-forward: widths 4096 x 3584, mean 64 297 us against 293, 128 320 against
-    488, 512 738 against 1157; 2048 x 2048, mean 96 131 against 136, 128 134 against 165; 1024 x 1024 (64 tiles of one
-    product at the least), mean 192 63 against 58, 256 69 against 86."""
+    16 experts, top 2 or 4, the whole feed-forward.  256 against 128, widths 4096 x 3584: mean 128 338 us against 457, 512 738
+    against 1157; 6144 x 2560: mean 64 452 against 417; 2048 x 2048: mean 64 139 against 144, 128 134 against 165; 1024 x 1024 (64
+    tiles of one product at the least), mean 192 63 against 58, 256 69 against 86.  64 against 128: 2048 x 2048 mean 32 108 against
+    136, 64 136 against 144; 4096 x 3584 299 against 302, 481 against 314; but 64 experts of 1024 x 512, mean 32 76 against 73.  32
+    against 64 and 16: 2048 x 2048 mean 16 100 against 104 and 119, mean 4 97 against 101 and 95; 2048 x 4096 mean 16 177 against
+    198 and 220, mean 4 170 against 195 and 167."""
     mean = pairs / max(1, experts)
     if mean >= 256 or (mean >= 96 and experts * weights >= 1 << 26):
         return 256
-    if mean >= 12 or (mean >= 4 and weights >= 1 << 23):
+    if mean > 40 or (mean > 12 and experts > 32 and weights < 1 << 20):
         return 128
-    return 16 if mean <= 2 else 32
+    if mean > 20:
+        return 64
+    return 16 if mean <= 4 else 32
 
 
 def moe_experts(h, idx, wts, gate_up, down, shared=None, act: str = "silu", limit: float = 0.0, alpha: float = 1.702,

@@ -1,0 +1,59 @@
+"""Grouped expert products that stream the weights (dgi/csrc/mix/moe_group.hip: moe_group_stream_kernel, moe_group_rows_kernel): tiles of
+16, 32 and 64 places, blocks of weights that end inside 16 rows, inner sizes around what eight waves share, and too long or ragged for
+the rows of A to stay in registers, against the products in 64 bits."""
+import pytest
+import torch
+
+from dgi.ops import moe
+from test_moe_wide import BF16, F64, draw, exact
+
+COUNTS = [0, 1, 15, 16, 17, 0, 31, 33, 64, 65, 7, 0]
+
+
+def run(monkeypatch, tile, W, ff, counts, act="silu", weigh="output", top=2):
+    E = len(counts)
+    g = torch.Generator().manual_seed(7)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    flat = flat[torch.randperm(flat.numel(), generator=g)]
+    flat = flat[: flat.numel() // top * top]
+    idx = flat.reshape(-1, top).to(torch.int32)
+    T = idx.shape[0]
+    h = draw(T, W, seed=1)
+    gu, dn = draw(E, 2 * ff, W, seed=2, scale=W ** -0.5), draw(E, W, ff, seed=3, scale=ff ** -0.5)
+    w = torch.rand(T, top, generator=g)
+    monkeypatch.setattr(moe, "group_tile", lambda *a: tile)
+    got = moe.moe_experts(h.cuda(), idx.cuda(), w.cuda(), gu.cuda(), dn.cuda(), None, act=act, limit=0.8, weigh=weigh)
+    y, mag = exact(h, idx, w, gu, dn, act, 0.8, weigh)
+    # three roundings to bf16 (at most 2^-8 of the value): each term's activation, each expert's row, the sum; fp32 elsewhere
+    bound = 2.0 ** -8 * (2 * mag + y.abs()) + 1e-5 * (1 + mag)
+    worst = ((got.cpu().to(F64) - y).abs() / bound).max().item()
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [16, 32, 64])
+@pytest.mark.parametrize("W,ff", [(64, 128), (576, 72), (1088, 200), (2048, 64), (72, 104), (8, 16)])
+def test_streamed_experts(monkeypatch, W, ff, tile):
+    """72, 104, 8 and 200 are no multiples of 64 (the other kernel); 576 = 9 stages leave waves without any."""
+    run(monkeypatch, tile, W, ff, COUNTS)
+    run(monkeypatch, tile, W, ff, COUNTS, "clamped", "input")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,W,ff", [(16, 8192, 64), (16, 8256, 128), (32, 4096, 64), (32, 4160, 64), (64, 2112, 64), (16, 2560, 1088)])
+def test_rows_around_what_the_registers_hold(monkeypatch, tile, W, ff):
+    run(monkeypatch, tile, W, ff, [3, 0, 20, 1, 35])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [16, 32, 64])
+def test_one_row_and_more_shares_than_blocks(monkeypatch, tile):
+    run(monkeypatch, tile, 128, 64, [1, 0, 1])
+    run(monkeypatch, tile, 128, 64, [0] * 70 + [5] + [0] * 40 + [70, 3])       # more experts than lanes
+
+
+def test_tiles_by_the_mean_rows_of_an_expert():
+    big, small = 1 << 24, 1 << 19
+    assert [moe.group_tile(16 * m, 16, big) for m in (1, 4, 5, 20, 21, 40, 41, 95, 96)] == [16, 16, 32, 32, 64, 64, 128, 128, 256]
+    assert [moe.group_tile(16 * m, 16, small) for m in (40, 41, 255, 256)] == [64, 128, 128, 256]
+    assert [moe.group_tile(64 * m, 64, small) for m in (12, 13)] == [32, 128]
