@@ -134,6 +134,11 @@ __device__ __forceinline__ void load_lds16(const char* src, char* lds) {
   __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
 
+// the same for data that nothing reads again soon (nt): the chip's caches give it up first
+__device__ __forceinline__ void load_lds16_once(const char* src, char* lds) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 2);
+}
+
 __device__ __forceinline__ void st_out4(uint16_t* p, const float* v, int n, bool vec) {
   if (vec && n == 4) {
     *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
@@ -146,7 +151,7 @@ __device__ __forceinline__ void st_out4(uint16_t* p, const float* v, int n, bool
 
 // ---- few rows per expert, rows of A that do not fit the registers: up to 16 MB places x 64 weight rows (GLU: 32 outputs, gate and
 // up), a wave 16 of the weight rows, four stages of 64 of K.  16 experts, widths 4096 x 3584, top 4, 128 rows (64 places a tile): the
-// whole feed-forward 299 us, on 128 x 128 tiles 302.
+// whole feed-forward 270 us, on 128 x 128 tiles 302.
 template <int MB, bool GLU>
 __global__ __launch_bounds__(256) void moe_group_rows_kernel(GroupArgs g) {
   constexpr int D = 4;                                 // stages, of 64 of K each
@@ -181,18 +186,21 @@ __global__ __launch_bounds__(256) void moe_group_rows_kernel(GroupArgs g) {
     const int place = min(lo + 8 * ai[i] + row8, hi - 1);
     ap[i] = reinterpret_cast<const char*>(g.a + (size_t)(g.order ? g.order[place] / g.top : place) * g.a_stride);
   }
+  // every weight tile starts at a stage of its own: workgroups in step with each other would read the same offset of rows that are
+  // all the same power of two apart, from a few channels of the memory at a time
+  const int steps = (K + 63) >> 6, first = blockIdx.x / g.mtiles % steps;
+  auto stage = [&](int s) { return s + first < steps ? s + first : s + first - steps; };
   auto load = [&](int s) {
     char* st = lds + (s % D) * STAGE;
-    const int k = min(64 * s + c8, K - 8) * 2;         // pieces past the row's end: its last one (zeros when they are used)
+    const int k = min(64 * stage(s) + c8, K - 8) * 2;  // pieces past the row's end: its last one (zeros when they are used)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) load_lds16(bp[i] + k, st + (2 * w + i) * 1024);
+    for (int i = 0; i < 2; ++i) load_lds16_once(bp[i] + k, st + (2 * w + i) * 1024);
 #pragma unroll
     for (int i = 0; i < CA; ++i) load_lds16(ap[i] + k, st + 8192 + ai[i] * 1024);
   };
   f32x4 acc[MB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int steps = (K + 63) >> 6;
   auto step = [&](int s, auto LEFT_) {
     constexpr int LEFT = decltype(LEFT_)::value;       // stages loaded after this one
     if constexpr (LEFT == 2) { if constexpr (CA == 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); }
@@ -209,8 +217,8 @@ __global__ __launch_bounds__(256) void moe_group_rows_kernel(GroupArgs g) {
       u32x4 fb = *reinterpret_cast<const u32x4*>(st + w * 2048 + at), fa[MB];
 #pragma unroll
       for (int i = 0; i < MB; ++i) fa[i] = *reinterpret_cast<const u32x4*>(st + 8192 + i * 2048 + at);
-      if (s == steps - 1 && (K & 63)) {
-        const bool in = 64 * s + 32 * h + 8 * lg < K;
+      if ((K & 63) && stage(s) == steps - 1) {
+        const bool in = 64 * (steps - 1) + 32 * h + 8 * lg < K;
         const u32x4 zero = {0u, 0u, 0u, 0u};
         fb = in ? fb : zero;
 #pragma unroll
@@ -257,12 +265,13 @@ __global__ __launch_bounds__(256) void moe_group_rows_kernel(GroupArgs g) {
 // each) and streams them without a gap.  Its eight waves split K; a wave keeps its part of the tile's rows of A in registers (they
 // come through the same ring of LDS stages first), so that all that moves is weights, and no wave waits for another but to add up
 // the partial sums of a block.  A load takes 8 rows x 128 bytes: one compute unit reads 54 GB/s that way, but 37 with the products'
-// own 16 rows x 64 bytes, and needs 22 of the chip's 5.8 TB/s.  Even shares: 64 weight rows a workgroup were 544 for 512 places.
+// own 16 rows x 64 bytes.  Weights are read as what nothing reads again soon (nt): 6.9 TB/s in all for reads alone, without it 6.3.
+// Even shares: 64 weight rows a workgroup were 544 for 512 places.
 //
 // 16 experts, top 2, the whole feed-forward (16 to 20 us of it router, plan and combine), against weights straight to registers
 // (64 rows a workgroup, K over its waves; 128 x 128 tiles from 4 or 12 places an expert on):
-//   widths 2048 x 2048: 1 row 36 us -> 28, 8 rows 93 -> 69, 32 rows 110 -> 95 (4.9 TB/s in the products), 128 rows 130 -> 100
-//   widths 4096 x 3584: 1 row 70 -> 56, 8 rows 227 -> 185, 32 rows 285 -> 265 (5.6 TB/s)
+//   widths 2048 x 2048: 1 row 36 us -> 30, 8 rows 93 -> 62, 32 rows 110 -> 84 (6.0 TB/s in the products), 128 rows 130 -> 88
+//   widths 4096 x 3584: 1 row 70 -> 52, 8 rows 227 -> 165, 32 rows 285 -> 232 (6.5 TB/s)
 constexpr int STREAM_WGS = 256;
 
 // KS: stages of 64 of K per wave at the most.  K a multiple of 64.
@@ -322,8 +331,8 @@ __global__ __launch_bounds__(512) void moe_group_stream_kernel(GroupArgs g) {
     int issued = 0, l_ks = 0, l_blk = 0, l_slot = 0;
     const char *p0 = ap[0][0], *p1 = ap[0][1];
     auto load = [&]() {
-      load_lds16(p0 + l_ks * 128, rg + l_slot * 2048);
-      load_lds16(p1 + l_ks * 128, rg + l_slot * 2048 + 1024);
+      load_lds16_once(p0 + l_ks * 128, rg + l_slot * 2048);
+      load_lds16_once(p1 + l_ks * 128, rg + l_slot * 2048 + 1024);
       ++issued;
       l_slot = l_slot + 1 == D ? 0 : l_slot + 1;
       if (++l_ks == mine) {

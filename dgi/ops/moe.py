@@ -165,10 +165,10 @@ def group_tile(pairs: int, experts: int, weights: int) -> int:
 
     16 experts, top 2 or 4, the whole feed-forward.  256 against 128, widths 4096 x 3584: mean 128 338 us against 457, 512 738
     against 1157; 6144 x 2560: mean 64 452 against 417; 2048 x 2048: mean 64 139 against 144, 128 134 against 165; 1024 x 1024 (64
-    tiles of one product at the least), mean 192 63 against 58, 256 69 against 86.  64 against 128: 2048 x 2048 mean 32 108 against
-    136, 64 136 against 144; 4096 x 3584 299 against 302, 481 against 314; but 64 experts of 1024 x 512, mean 32 76 against 73.  32
-    against 64 and 16: 2048 x 2048 mean 16 100 against 104 and 119, mean 4 97 against 101 and 95; 2048 x 4096 mean 16 177 against
-    198 and 220, mean 4 170 against 195 and 167."""
+    tiles of one product at the least), mean 192 63 against 58, 256 69 against 86.  64 against 128: 2048 x 2048 mean 32 96 against
+    136, 64 144 against 144; 4096 x 3584 270 against 302, 510 against 314; but 64 experts of 1024 x 512, mean 32 76 against 73.  32
+    against 64 and 16: 2048 x 2048 mean 16 89 against 93 and 116; 2048 x 4096 mean 16 149 against 169 and 203, mean 4 144 against
+    164 and 142."""
     mean = pairs / max(1, experts)
     if mean >= 256 or (mean >= 96 and experts * weights >= 1 << 26):
         return 256
