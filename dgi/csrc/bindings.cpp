@@ -27,6 +27,14 @@ int dgi_paged_prefill(const void* q, int q_stride, const void* k_cache, const vo
                       int out_stride, int nh, int nkv, int hd, int block_size, float scale,
                       const unsigned long long* tree_mask, int tree_n, int tile_rows, hipStream_t s);
 int dgi_silu_mul(const void* gu, void* out, int T, int I, hipStream_t s);
+int dgi_stream_gemm(const void* x, long long ldx, const void* w, const void* bias, void* out, long long ldo, int M, int N, int K,
+                    int mode, int parts, hipStream_t s);
+int dgi_add_rmsnorm_parts(void* out, const float* parts, int nparts, void* residual, const void* gamma, int T, int H, float eps,
+                          hipStream_t s);
+int dgi_sum_parts(void* out, const float* parts, int nparts, const void* bias, int M, int N, hipStream_t s);
+int dgi_rope_cache_parts(void* out, const float* parts, int nparts, const void* bias, int T, const int* positions, const float* cos_sin,
+                         int nh, int nkv, int hd, int rd, int mode, const int* slot_mapping, void* k_cache, void* v_cache,
+                         int block_size, hipStream_t s);
 int dgi_skinny_gemm(const void* x, int ldx, const void* w, const void* bias, void* y, int ldy, int M,
                     int N, int K, int nw, hipStream_t s);
 int dgi_mfma_gemm(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int epi,
@@ -221,6 +229,78 @@ void skinny_gemm(at::Tensor out, const at::Tensor& x, const at::Tensor& w,
   check_rc(dgi_skinny_gemm(x.data_ptr(), (int)x.stride(0), w.data_ptr(), b, out.data_ptr(), (int)out.stride(0),
                            (int)M, (int)N, (int)K, (int)cfg, cur_stream()),
            "skinny_gemm");
+}
+
+const void* opt_bias(const c10::optional<at::Tensor>& bias, int64_t N) {
+  if (!bias.has_value()) return nullptr;
+  check_bf16(*bias, "bias");
+  TORCH_CHECK(bias->is_contiguous() && bias->numel() == N && ((uintptr_t)bias->data_ptr() & 15) == 0, "bias: one per output");
+  return bias->data_ptr();
+}
+
+void check_parts(const at::Tensor& parts, int64_t M, int64_t N) {
+  check_dev(parts, "parts");
+  TORCH_CHECK(parts.scalar_type() == at::kFloat && parts.is_contiguous() && parts.dim() == 3 && parts.size(0) >= 1 && parts.size(1) == M &&
+                  parts.size(2) == N && ((uintptr_t)parts.data_ptr() & 15) == 0,
+              "parts: fp32 [parts, rows, outputs]");
+}
+
+// few rows, weights read once: mode 0 out = x w^T (+ bias); 1 out = SwiGLU with w = [gate; up]; 2 out = fp32 parts [parts, M, N]
+void stream_gemm(at::Tensor out, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t mode) {
+  check_bf16(x, "x"); check_bf16(w, "w");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.stride(1) == 1 && w.is_contiguous() && x.device() == w.device() && x.device() == out.device(),
+              "stream_gemm: row-major operands on one device");
+  const int64_t M = x.size(0), K = x.size(1), N = mode == 1 ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(mode >= 0 && mode <= 2 && w.size(1) == K && (mode != 1 || w.size(0) % 2 == 0) && M <= 128 && K < (1 << 30) && N < (1 << 30),
+              "stream_gemm: shape mismatch");
+  TORCH_CHECK(mode == 0 || !bias.has_value(), "stream_gemm: a bias goes with whole rows");
+  int64_t ldo = N;
+  int parts = 1;
+  if (mode == 2) {
+    check_parts(out, M, N);
+    parts = (int)out.size(0);
+  } else {
+    check_bf16(out, "out");
+    TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == N && out.stride(1) == 1, "stream_gemm: out is [rows, outputs]");
+    ldo = out.stride(0);
+  }
+  check_rc(dgi_stream_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), opt_bias(bias, N), out.data_ptr(), ldo, (int)M, (int)N, (int)K, (int)mode,
+                           parts, cur_stream()), "stream_gemm");
+}
+
+void add_rmsnorm_parts(at::Tensor out, const at::Tensor& parts, at::Tensor residual, const at::Tensor& w, double eps) {
+  check_bf16(out, "out"); check_bf16(residual, "residual"); check_bf16(w, "w");
+  TORCH_CHECK(out.dim() == 2 && out.is_contiguous() && residual.is_contiguous() && w.is_contiguous() && out.sizes() == residual.sizes() &&
+                  w.numel() == out.size(1), "add_rmsnorm_parts: rows");
+  check_parts(parts, out.size(0), out.size(1));
+  check_rc(dgi_add_rmsnorm_parts(out.data_ptr(), parts.data_ptr<float>(), (int)parts.size(0), residual.data_ptr(), w.data_ptr(),
+                                 (int)out.size(0), (int)out.size(1), (float)eps, cur_stream()), "add_rmsnorm_parts");
+}
+
+void sum_parts(at::Tensor out, const at::Tensor& parts, const c10::optional<at::Tensor>& bias) {
+  check_bf16(out, "out");
+  TORCH_CHECK(out.dim() == 2 && out.is_contiguous(), "sum_parts: rows");
+  check_parts(parts, out.size(0), out.size(1));
+  check_rc(dgi_sum_parts(out.data_ptr(), parts.data_ptr<float>(), (int)parts.size(0), opt_bias(bias, out.size(1)), (int)out.size(0),
+                         (int)out.size(1), cur_stream()), "sum_parts");
+}
+
+void rope_cache_parts(at::Tensor out, const at::Tensor& parts, const c10::optional<at::Tensor>& bias, const at::Tensor& positions,
+                      const at::Tensor& cos_sin, int64_t nh, int64_t nkv, int64_t hd, const at::Tensor& slot_mapping, at::Tensor k_cache,
+                      at::Tensor v_cache, int64_t mode) {
+  check_bf16(out, "out"); check_i32(positions, "positions"); check_i32(slot_mapping, "slot_mapping");
+  check_bf16(k_cache, "k_cache"); check_bf16(v_cache, "v_cache");
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous() && cos_sin.dim() == 2 && cos_sin.size(1) <= hd);
+  TORCH_CHECK(out.dim() == 2 && out.is_contiguous() && out.size(1) == nh * hd);
+  TORCH_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() && k_cache.sizes() == v_cache.sizes());
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.size(1) == nkv && k_cache.size(3) == hd);
+  const int T = (int)out.size(0);
+  check_parts(parts, T, (nh + 2 * nkv) * hd);
+  TORCH_CHECK(positions.numel() == T && slot_mapping.numel() == T);
+  check_rc(dgi_rope_cache_parts(out.data_ptr(), parts.data_ptr<float>(), (int)parts.size(0), opt_bias(bias, (nh + 2 * nkv) * hd), T,
+                                positions.data_ptr<int>(), cos_sin.data_ptr<float>(), (int)nh, (int)nkv, (int)hd, (int)cos_sin.size(1),
+                                (int)mode, slot_mapping.data_ptr<int>(), k_cache.data_ptr(), v_cache.data_ptr(), (int)k_cache.size(2),
+                                cur_stream()), "rope_cache_parts");
 }
 
 // LDS-tiled MFMA GEMM (prefill / mixed steps): epi 0 out = x w^T; epi 1 out = SwiGLU with w = [gate; up].
@@ -594,6 +674,11 @@ TORCH_LIBRARY(dgi, m) {
         "Tensor cu_seqlens_q, Tensor context_lens, Tensor tiles, int nh, int nkv, float scale, "
         "Tensor? tree_mask, int tree_n, int tile_rows=128) -> ()");
   m.def("silu_mul(Tensor(a!) out, Tensor gu) -> ()");
+  m.def("stream_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int mode) -> ()");
+  m.def("add_rmsnorm_parts(Tensor(a!) out, Tensor parts, Tensor(b!) residual, Tensor w, float eps) -> ()");
+  m.def("sum_parts(Tensor(a!) out, Tensor parts, Tensor? bias) -> ()");
+  m.def("rope_cache_parts(Tensor(a!) out, Tensor parts, Tensor? bias, Tensor positions, Tensor cos_sin, int nh, int nkv, int hd, "
+        "Tensor slot_mapping, Tensor(b!) k_cache, Tensor(c!) v_cache, int mode) -> ()");
   m.def("skinny_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int cfg=0) -> ()");
   m.def("mfma_gemm(Tensor(a!) out, Tensor x, Tensor w, int epi=0) -> ()");
   m.def("mfma_gemm_norm(Tensor(a!) out, Tensor x, Tensor w, int kind, Tensor(b!) ss, float inv_k, float eps, "
@@ -627,6 +712,10 @@ TORCH_LIBRARY_IMPL(dgi, CUDA, m) {
   m.impl("paged_decode", &paged_decode);
   m.impl("paged_prefill", &paged_prefill);
   m.impl("silu_mul", &silu_mul);
+  m.impl("stream_gemm", &stream_gemm);
+  m.impl("add_rmsnorm_parts", &add_rmsnorm_parts);
+  m.impl("sum_parts", &sum_parts);
+  m.impl("rope_cache_parts", &rope_cache_parts);
   m.impl("skinny_gemm", &skinny_gemm);
   m.impl("mfma_gemm", &mfma_gemm);
   m.impl("mfma_gemm_norm", &mfma_gemm_norm);

@@ -456,6 +456,47 @@ class LlamaModel:
                 self.layer_hook(self.layer_start + i)
         return h, residual
 
+    # ------------------------------------------------------------------ layers of few rows
+    def _stream_ok(self, h: torch.Tensor) -> bool:
+        """Whether the layers run on the streaming products (``ops.stream_parts``): up to 128 rows of a model wide enough that the
+        weights' bytes are what a step takes."""
+        if self.reduce is not None or self.capture_layers or h.shape[1] < 2048:
+            return False
+        L = self.layers[0]
+        return (ops.stream_ok(h, L.qkv) and L.gate_up.shape[0] % 16 == 0 and L.o.shape[1] % 64 == 0 and L.down.shape[1] % 64 == 0
+                and all(t.is_contiguous() and t.dtype == h.dtype and t.data_ptr() % 16 == 0
+                        for K in self.layers for t in (K.qkv, K.o, K.gate_up, K.down, K.in_norm, K.post_norm, K.qkv_bias) if t is not None))
+
+    def _forward_layers_stream(self, h: torch.Tensor, meta: AttnMeta, residual: Optional[torch.Tensor],
+                               trim_last: Optional[torch.Tensor]):
+        """Layers of few rows: qkv, o and down leave fp32 parts that the rotary, the norms (and their residual adds) sum up as they
+        read them, gate_up has SwiGLU as its epilogue: seven kernels a layer beside the attention's.  Rounded where ``forward_layers``
+        rounds; its contract."""
+        c = self.cfg
+        eps = c.rms_eps
+        parts = None
+        for i, L in enumerate(self.layers):
+            if parts is not None:
+                x = ops.add_rmsnorm_parts(parts, residual, L.in_norm, eps)
+            elif residual is None:
+                residual = h
+                x = ops.rmsnorm(h, L.in_norm, eps)
+            else:
+                ops.fused_add_rmsnorm(h, residual, L.in_norm, eps)
+                x = h
+            q = ops.rope_cache_parts(ops.stream_parts(x, L.qkv), L.qkv_bias, meta.positions, self.cos_sin, c.num_heads, c.num_kv_heads,
+                                     c.head_dim, meta.slot_mapping, self.kv_cache[i, 0], self.kv_cache[i, 1], self.rope_mode)
+            attn = self.attention(i, q, meta, rope=False)
+            if trim_last is not None and i == len(self.layers) - 1:
+                attn, residual = attn.index_select(0, trim_last), residual.index_select(0, trim_last)
+            x = ops.add_rmsnorm_parts(ops.stream_parts(attn, L.o), residual, L.post_norm, eps)
+            # past 96 rows the rows of x are read so often that only the narrower weights gain
+            act = ops.stream_glu(x, L.gate_up) if x.shape[0] <= 96 or x.shape[1] <= 4096 else ops.silu_mul(ops.linear(x, L.gate_up))
+            parts = ops.stream_parts(act, L.down)
+            if self.layer_hook is not None:
+                self.layer_hook(self.layer_start + i)
+        return ops.sum_parts(parts), residual
+
     # ------------------------------------------------------------------ fused-norm layers
     def _fold_ok(self, h: torch.Tensor) -> bool:
         if NORM_FOLD == "0" or self.reduce is not None:
@@ -658,6 +699,8 @@ class LlamaModel:
                 if trim_last is not None:     # same contract as the unfused path: only the logits rows
                     h, residual = h.index_select(0, trim_last), residual.index_select(0, trim_last)
                 return h, residual
+            if self._stream_ok(h):
+                return self._forward_layers_stream(h, meta, residual, trim_last)
         Mp = self._mlp_rows(T, h) if self.layers else T
         # hand-written MFMA GEMMs where the start-up table measured them faster (dgi.runtime.gemm_pad)
         mfma_gu, mfma_dn = self.mlp_impl(Mp) if (self.mlp_impl is not None and self.layers) else (False, False)

@@ -427,6 +427,105 @@ def _skinny_cfg(M: int, N: int) -> int:
     return 5 if (M > 8 and N >= 16384) else 0
 
 
+# Products of few rows that read their weights once (dgi/csrc/stream_gemm.hip, where both sides' times are).
+# DGI_STREAM_MAX_M=0 turns them off.
+STREAM_MAX_M = int(os.environ.get("DGI_STREAM_MAX_M", "128"))
+
+
+def stream_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Operands that the streaming products take: bf16 rows of a multiple of 64, weights [N, K] with N a multiple of 8, everything at
+    16-byte boundaries, at most 128 rows."""
+    return (x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= min(STREAM_MAX_M, 128)
+            and w.dim() == 2 and w.is_contiguous() and w.shape[0] % 8 == 0 and w.shape[1] == x.shape[1] and x.shape[1] % 64 == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def stream_part_count(N: int, K: int) -> int:
+    """Parts that K is cut into so that some 256 workgroups (one per compute unit) share N outputs, 128 at a time; a part is at least
+    four stages of 64 of K, and none is empty."""
+    stages = K // 64
+    parts = max(1, min(256 // max(1, -(-N // 128)), stages // 4))
+    return -(-stages // -(-stages // parts))
+
+
+def stream_parts_ref(x, w):
+    return (x.float() @ w.float().t())[None]
+
+
+def stream_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w.T as fp32 partial sums over parts of K [parts, M, N], for ``add_rmsnorm_parts``, ``rope_cache_parts`` or ``sum_parts``."""
+    if _native(x):
+        N, K = w.shape
+        out = torch.empty(stream_part_count(N, K), x.shape[0], N, dtype=torch.float32, device=x.device)
+        _call("stream_gemm", out, x, w, None, 2)
+        return out
+    return stream_parts_ref(x, w)
+
+
+def stream_glu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up over w = [gate; up], rounded like ``silu_mul(linear(x, w))``."""
+    if _native(x):
+        out = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype, device=x.device)
+        _call("stream_gemm", out, x, w, None, 1)
+        return out
+    return silu_mul_ref((x.float() @ w.float().t()).to(x.dtype))
+
+
+def sum_parts(parts: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The product that ``stream_parts`` left in parts (+ bias), in bf16."""
+    if _native(parts):
+        out = torch.empty(parts.shape[1], parts.shape[2], dtype=torch.bfloat16, device=parts.device)
+        _call("sum_parts", out, parts, bias)
+        return out
+    y = parts.sum(0)
+    return (y if bias is None else y + bias.float()).to(torch.bfloat16)
+
+
+def add_rmsnorm_parts(parts: torch.Tensor, residual: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """``fused_add_rmsnorm`` of the product in ``parts``: residual is updated in place, the normalised rows are returned."""
+    if _native(parts):
+        out = torch.empty_like(residual)
+        _call("add_rmsnorm_parts", out, parts, residual, w, eps)
+        return out
+    x = parts.sum(0).to(residual.dtype)
+    fused_add_rmsnorm_ref(x, residual, w, eps)
+    return x
+
+
+def rope_cache_parts(parts, bias, positions, cos_sin, nh, nkv, hd, slot_mapping, k_cache, v_cache, mode: int = 0) -> torch.Tensor:
+    """``rope_cache`` of the fused q | k | v product in ``parts`` (+ bias): rotated q rows [T, nh * hd] are returned, k and v go to the
+    cache."""
+    if _native(parts):
+        out = torch.empty(parts.shape[1], nh * hd, dtype=k_cache.dtype, device=parts.device)
+        _call("rope_cache_parts", out, parts, bias, positions, cos_sin, nh, nkv, hd, slot_mapping, k_cache, v_cache, mode)
+        return out
+    y = parts.sum(0)
+    qkv = (y if bias is None else y + bias.float()).to(k_cache.dtype)
+    rope_cache_ref(qkv, positions, cos_sin, nh, nkv, hd, slot_mapping, k_cache, v_cache, mode)
+    return qkv[:, : nh * hd]
+
+
+def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:
+    """``linear`` as a streaming product where that is the faster: outputs that fill the chip by themselves up to 96 rows, narrow and
+    large weights (96 MB; the sum over the parts is a launch of its own) up to 128."""
+    N, K = w.shape
+    if not stream_ok(x, w) or (bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_contiguous() or bias.data_ptr() % 16)):
+        return None
+    if not load_native(False):
+        return None
+    if N >= 160 * 128 and x.shape[0] <= 96:
+        if out is None:
+            out = torch.empty(x.shape[0], N, dtype=x.dtype, device=x.device)
+        elif out.dim() != 2 or out.stride(1) != 1 or out.stride(0) % 4 or out.data_ptr() % 8 or out.dtype != x.dtype:
+            return None
+        _call("stream_gemm", out, x, w, bias, 0)
+        return out
+    if N < 160 * 128 and N * K >= 48 << 20:
+        y = sum_parts(stream_parts(x, w), bias)
+        return y if out is None else out.copy_(y)
+    return None
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x @ w.T (+ bias) for a 2-D activation; [N, K] weights as stored."""
@@ -441,6 +540,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _call("skinny_gemm", out, x, w, bias, _skinny_cfg(M, N))
         return out
+    if x.is_cuda and x.shape[0] <= STREAM_MAX_M:
+        y = _linear_stream(x, w, bias, out)
+        if y is not None:
+            return y
     r = torch.nn.functional.linear(x, w, bias)
     if out is not None:
         out.copy_(r)
