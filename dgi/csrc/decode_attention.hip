@@ -6,12 +6,15 @@
 // the paged pool written by rope_cache.hip.
 //
 // Work decomposition (CDNA4, wave64):
-//   grid = (max_splits, n_kv_heads, batch), 4 waves (8 when a short-context,
-//   small-batch step runs one split per sequence: no partials, no reduce kernel).
+//   grid = (n_kv_heads, batch, max_splits), 8 waves, or 4 where there are more
+//   workgroups than compute units.
 //   A workgroup owns one (sequence, kv-head, KV split) and all G = nh/nkv
 //   query heads of that kv head, so each K/V byte is read from HBM once per
 //   decode step regardless of the GQA ratio.
-//   Each wave walks 32-token tiles.  Scores are computed "swapped":
+//   Each wave walks 32-token tiles; bounded by the cached rows' bytes, it keeps
+//   a tile under way all the time (the next tile's keys and values are asked for
+//   as the products and the LDS writes free their registers: 350 rows of 576 tokens,
+//   64 heads on 8, 168 us -> 149, 5.5 TB/s).  Scores are computed "swapped":
 //     S^T[token][query] = K[token][:] . Q[query][:]   (mfma_f32_16x16x32_bf16,
 //   K fragments straight from HBM into VGPRs, Q fragments resident), so a lane
 //   owns one query column and the online softmax needs only two xor-shuffles.
@@ -26,6 +29,8 @@
 //   partials, one relaxed ticket, one acquire on the last arriver) or a small
 //   reduce kernel does.
 #include "common.h"
+
+#include <type_traits>
 
 using namespace dgi;
 
@@ -53,13 +58,21 @@ constexpr int decode_wave_lds() {
   return (32 * HD * 2 > 16 * (HD + 4) * 4 ? 32 * HD * 2 : 16 * (HD + 4) * 4) + 128;
 }
 
-template <int HD, int NW>
+// ONCE: nothing reads it again soon, the chip's caches give it up first
+template <bool ONCE>
+__device__ __forceinline__ u32x4 load_row(const uint16_t* p) {
+  if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  return *reinterpret_cast<const u32x4*>(p);
+}
+
+// P16: pages of 16 tokens (the engine's)
+template <int HD, int NW, bool P16>
 __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
     const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_cache,
     const uint16_t* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ context_lens, uint16_t* __restrict__ out, int out_stride,
     float* __restrict__ part_o, float* __restrict__ part_lse, int* __restrict__ counters, int max_splits, int nh,
-    int nkv, int bs_log2, int part_size, float scale_log2, bool page16) {
+    int nkv, int bs_log2, int part_size, float scale_log2) {
   constexpr int KS = HD / 32;   // k-steps of the QK^T product
   constexpr int NC = HD / 16;   // 16-wide dim blocks of the PV product
   constexpr int VCH = HD / 8;   // 16-byte chunks per V row
@@ -72,15 +85,15 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
   constexpr int NT = 64 * NW;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
-  const int split = blockIdx.x;
-  const int h = blockIdx.y;
-  const int b = blockIdx.z;
+  const int split = blockIdx.z;
+  const int h = blockIdx.x;
+  const int b = blockIdx.y;
   const int ctx = context_lens[b];
   // write-through views of the split workspace (fused reduce); byte ranges cover the launch
   const __amdgpu_buffer_rsrc_t po_rs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)part_o, 0, (int)min((size_t)gridDim.z * nh * max_splits * HD * 4, (size_t)0x7fffffff), kRsrcWord3);
+      (void*)part_o, 0, (int)min((size_t)gridDim.y * nh * max_splits * HD * 4, (size_t)0x7fffffff), kRsrcWord3);
   const __amdgpu_buffer_rsrc_t pl_rs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)part_lse, 0, (int)min((size_t)gridDim.z * nh * max_splits * 4, (size_t)0x7fffffff), kRsrcWord3);
+      (void*)part_lse, 0, (int)min((size_t)gridDim.y * nh * max_splits * 4, (size_t)0x7fffffff), kRsrcWord3);
   // part_size <= 0: device-side split plan from this sequence's own context —
   // up to max_splits parts of at least -part_size tokens (32-token multiples),
   // so a graph captured for the longest context does not leave short ones
@@ -107,9 +120,8 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
   const int g = lane >> 4;
   uint16_t* vt = reinterpret_cast<uint16_t*>(smem + w * WREG);
 
-  // Q fragments (B operand): B[k = 8g + j][col = query qi] = Q[qi][32 s + 8 g + j].  The 8-wave
-  // one-split variant (small batch, short context: one or two tiles per wave) issues them after
-  // its first tile's K/V loads, so the two round trips overlap instead of running back to back.
+  // Q fragments (B operand): B[k = 8g + j][col = query qi] = Q[qi][32 s + 8 g + j], asked for after the first tile's keys and
+  // values, so that the two round trips overlap.
   u32x4 qf[KS];
   auto load_q = [&]() {
 #pragma unroll
@@ -121,8 +133,6 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
       }
     }
   };
-  constexpr bool LATE_Q = NW == 8;
-  if (!LATE_Q) load_q();
 
   const int* bt = block_tables + (size_t)b * bt_stride;
   const size_t head_stride = (size_t)bs * HD;
@@ -133,62 +143,40 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
   for (int c = 0; c < NC; ++c) o[c] = f32x4{0, 0, 0, 0};
 
   const int ntiles = (end - start + 31) >> 5;
-  for (int t = w; t < ntiles; t += NW) {
-    const int tb = start + (t << 5);
-    u32x4 kf[2][KS];
-    u32x4 vr[VCH / 2];
-    if (page16 && tb + 32 <= end) {
-      // full tile of 16-token pages (the engine's page size): its two pages come from two
-      // scalar block-table reads, every lane's offset inside a page is a constant, so each
-      // load is an SGPR base + a fixed VGPR offset (no per-load 64-bit address arithmetic:
-      // at small batch the tile loop is VALU-issue-bound)
-      const int fb = tb >> 4;
-      const uint16_t* kp[2];
-      const uint16_t* vp[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const size_t page = ((size_t)bt[fb + j] * nkv + h) * head_stride;
-        kp[j] = k_cache + page;
-        vp[j] = v_cache + page;
-      }
-      // ---- K fragments straight to VGPRs (A operand: row = token, k = dims)
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-          kf[u][s] = *reinterpret_cast<const u32x4*>(kp[u] + qi * HD + 32 * s + 8 * g);
-      // ---- V tile -> registers (row 4k + lane / VCH of the tile; rows 16-31 on the second page)
-#pragma unroll
-      for (int k = 0; k < VCH / 2; ++k) {
-        const int idx = k * 64 + lane;
-        const int row = idx / VCH;
-        vr[k] = *reinterpret_cast<const u32x4*>(vp[row >> 4] + (row & 15) * HD + (idx % VCH) * 8);
-      }
-    } else {
-      // ---- K fragments straight to VGPRs (A operand: row = token, k = dims)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        int tok = tb + 16 * u + qi;
-        tok = min(tok, end - 1);
-        const int blk = bt[tok >> bs_log2];
-        const uint16_t* kpl = k_cache + ((size_t)blk * nkv + h) * head_stride + (size_t)(tok & (bs - 1)) * HD;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) kf[u][s] = *reinterpret_cast<const u32x4*>(kpl + 32 * s + 8 * g);
-      }
-      // ---- V tile -> registers -> swizzled LDS
-#pragma unroll
-      for (int k = 0; k < VCH / 2; ++k) {
-        // 32 rows x VCH chunks; each pass covers 64/VCH rows
-        const int idx = k * 64 + lane;
-        const int row = idx / VCH;
-        const int ch = idx % VCH;
-        int tok = min(tb + row, end - 1);
-        const int blk = bt[tok >> bs_log2];
-        const uint16_t* vpl = v_cache + ((size_t)blk * nkv + h) * head_stride + (size_t)(tok & (bs - 1)) * HD;
-        vr[k] = *reinterpret_cast<const u32x4*>(vpl + ch * 8);
-      }
+  u32x4 kf[2][KS], vr[VCH / 2];
+  // P16: a tile's two pages come from scalar reads of the block table (made a tile ahead), a load is a scalar base + a lane's
+  // offset.  Tokens past the end are the last one again: their products are masked, but what lies there may be no number.
+  int pg[2];
+  auto pages = [&](int t) {
+    if constexpr (P16) {
+      const int fb = (start >> 4) + 2 * t, lastp = (end - 1) >> 4;
+      pg[0] = bt[min(fb, lastp)];
+      pg[1] = bt[min(fb + 1, lastp)];
     }
-    if (LATE_Q && t == w) load_q();
+  };
+  auto load_k = [&](int t) {       // K fragments (A operand: row = token, k = dims)
+    const int tb = start + (t << 5);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int tok = min(tb + 16 * u + qi, end - 1);
+      const uint16_t* p;
+      if constexpr (P16) p = k_cache + ((size_t)pg[u] * nkv + h) * head_stride + ((tok & 15) * HD + 8 * g);
+      else p = k_cache + ((size_t)bt[tok >> bs_log2] * nkv + h) * head_stride + (size_t)(tok & (bs - 1)) * HD + 8 * g;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) kf[u][s] = load_row<NW == 4>(p + 32 * s);
+    }
+  };
+  auto load_v = [&](int t) {       // rows k * 64 / VCH + lane / VCH of the tile
+    const int tb = start + (t << 5);
+#pragma unroll
+    for (int k = 0; k < VCH / 2; ++k) {
+      const int tok = min(tb + k * (64 / VCH) + lane / VCH, end - 1), col = lane % VCH * 8;
+      if constexpr (P16) vr[k] = load_row<NW == 4>(v_cache + ((size_t)pg[(k * (64 / VCH)) >> 4] * nkv + h) * head_stride + ((tok & 15) * HD + col));
+      else vr[k] = load_row<NW == 4>(v_cache + ((size_t)bt[tok >> bs_log2] * nkv + h) * head_stride + (size_t)(tok & (bs - 1)) * HD + col);
+    }
+  };
+  auto tile = [&](int t, auto LAST) {
+    const int tb = start + (t << 5);
     // ---- S^T = K Q^T
     f32x4 sacc[2];
 #pragma unroll
@@ -198,21 +186,26 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
       for (int s = 0; s < KS; ++s)
         sacc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kf[u][s]), as_bf16x8(qf[s]), sacc[u], 0, 0, 0);
     }
+    if constexpr (!LAST.value) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_k(t + NW);              // into the registers that the products have read
+      __builtin_amdgcn_sched_barrier(0);
+    }
     // write V (the previous tile's transposed reads are complete: in-order LDS per wave)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int k = 0; k < VCH / 2; ++k) {
-      const int idx = k * 64 + lane;
-      const int row = idx / VCH;
-      const int ch = idx % VCH;
-      *reinterpret_cast<u32x4*>(vt + v_lds_off<HD>(row, ch * 8)) = vr[k];
+    for (int k = 0; k < VCH / 2; ++k) *reinterpret_cast<u32x4*>(vt + v_lds_off<HD>(k * (64 / VCH) + lane / VCH, lane % VCH * 8)) = vr[k];
+    if constexpr (!LAST.value) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(t + NW);
+      pages(t + 2 * NW);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // ---- online softmax (lane owns query qi; tokens 16u + 4g + i); only the sequence's last
     // tile has tokens past its end to mask
-    const bool full = tb + 32 <= end;
     float x[2][4];
     float mx = -1e30f;
-    if (full) {
+    if (tb + 32 <= end) {
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -273,6 +266,17 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
       vf[3] = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
       o[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(vf), as_bf16x8(pf), o[c], 0, 0, 0);
     }
+  };
+  // A tile's keys and values are always under way while the one before is multiplied.
+  if (w < ntiles) {
+    pages(w);
+    load_k(w);
+    load_v(w);
+    load_q();
+    pages(w + NW);
+    int t = w;
+    for (; t + NW < ntiles; t += NW) tile(t, std::false_type{});
+    tile(t, std::true_type{});
   }
 
   // ---- merge the NW waves through LDS
@@ -409,56 +413,35 @@ extern "C" int dgi_paged_decode(const void* q, int q_stride, const void* k_cache
   while ((1 << bs_log2) < block_size) ++bs_log2;
   if ((1 << bs_log2) != block_size) return -4;
   const float scale_log2 = scale * 1.4426950408889634f;
-  // full tiles of 16-token pages take the scalar-page-base load path (DGI_DECODE_PAGE16=0: off)
-  static const bool page16_on = [] {
-    const char* e = getenv("DGI_DECODE_PAGE16");
-    return !(e && e[0] == '0');
-  }();
-  const bool page16 = page16_on && bs_log2 == 4;
-  dim3 grid(max_splits, nkv, B);
-  // few workgroups (small batch, one split: every (sequence, kv head) walks its whole
-  // context): 8 waves per workgroup halve the serial tile chain of each wave
-  const bool wide = max_splits == 1 && B * nkv <= 128;
-  if (hd == 128) {
-    if (wide) {
-      paged_decode_kernel<128, 8><<<grid, 512, 8 * decode_wave_lds<128>(), s>>>(
-          (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache,
-          block_tables, bt_stride, context_lens, (uint16_t*)out, out_stride, part_o, part_lse,
-          counters, max_splits, nh, nkv, bs_log2, part_size, scale_log2, page16);
-    } else {
-      paged_decode_kernel<128, 4><<<grid, 256, 4 * decode_wave_lds<128>(), s>>>(
-          (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache,
-          block_tables, bt_stride, context_lens, (uint16_t*)out, out_stride, part_o, part_lse,
-          counters, max_splits, nh, nkv, bs_log2, part_size, scale_log2, page16);
-    }
+  // splits slowest: consecutive workgroups go to different XCDs, and where short contexts leave all but the first splits empty the
+  // others would have all the work (64 rows of 1024 in up to 4 splits of 2048 at the least, splits fastest: 133 us, not 51)
+  dim3 grid(nkv, B, max_splits);
+  // up to a workgroup per compute unit: eight waves each, half the serial chain of tiles (8 rows of 1000 tokens, 8 kv heads, in 4 splits
+  // 12.9 us, with four 15.3); more of them: four, so that several share a unit, and rows marked as read once (64 rows of 1024: 50.6,
+  // with eight 52.6; without the mark 53.4)
+  const bool wide = (long long)B * nkv * max_splits <= 256;
+  auto launch = [&](auto HD_, auto NW_, auto P16_) {
+    constexpr int HD = decltype(HD_)::value, NW = decltype(NW_)::value;
+    paged_decode_kernel<HD, NW, decltype(P16_)::value><<<grid, 64 * NW, NW * decode_wave_lds<HD>(), s>>>(
+        (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables, bt_stride, context_lens,
+        (uint16_t*)out, out_stride, part_o, part_lse, counters, max_splits, nh, nkv, bs_log2, part_size, scale_log2);
+  };
+  auto launch_pages = [&](auto HD_, auto NW_) {
+    if (bs_log2 == 4) launch(HD_, NW_, std::true_type{});
+    else launch(HD_, NW_, std::false_type{});
+  };
+  auto launch_dims = [&](auto HD_) {
+    constexpr int HD = decltype(HD_)::value;
+    if (wide) launch_pages(HD_, std::integral_constant<int, 8>{});
+    else launch_pages(HD_, std::integral_constant<int, 4>{});
     DGI_CHECK_LAUNCH();
     if (max_splits > 1 && counters == nullptr) {
-      decode_reduce_kernel<128><<<dim3(B, nh), 128, 0, s>>>(part_o, part_lse, context_lens,
-                                                            (uint16_t*)out, out_stride, max_splits,
-                                                            nh, part_size);
+      decode_reduce_kernel<HD><<<dim3(B, nh), HD, 0, s>>>(part_o, part_lse, context_lens, (uint16_t*)out, out_stride, max_splits, nh, part_size);
       DGI_CHECK_LAUNCH();
     }
-  } else if (hd == 64) {
-    if (wide) {
-      paged_decode_kernel<64, 8><<<grid, 512, 8 * decode_wave_lds<64>(), s>>>(
-          (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache,
-          block_tables, bt_stride, context_lens, (uint16_t*)out, out_stride, part_o, part_lse,
-          counters, max_splits, nh, nkv, bs_log2, part_size, scale_log2, page16);
-    } else {
-      paged_decode_kernel<64, 4><<<grid, 256, 4 * decode_wave_lds<64>(), s>>>(
-          (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache,
-          block_tables, bt_stride, context_lens, (uint16_t*)out, out_stride, part_o, part_lse,
-          counters, max_splits, nh, nkv, bs_log2, part_size, scale_log2, page16);
-    }
-    DGI_CHECK_LAUNCH();
-    if (max_splits > 1 && counters == nullptr) {
-      decode_reduce_kernel<64><<<dim3(B, nh), 64, 0, s>>>(part_o, part_lse, context_lens,
-                                                          (uint16_t*)out, out_stride, max_splits,
-                                                          nh, part_size);
-      DGI_CHECK_LAUNCH();
-    }
-  } else {
-    return -5;
-  }
-  return 0;
+    return 0;
+  };
+  if (hd == 128) return launch_dims(std::integral_constant<int, 128>{});
+  if (hd == 64) return launch_dims(std::integral_constant<int, 64>{});
+  return -5;
 }

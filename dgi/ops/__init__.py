@@ -244,17 +244,15 @@ def paged_decode_ref(q, k_cache, v_cache, block_tables, context_lens, nh, nkv, s
 
 
 def decode_split_plan(batch: int, max_ctx: int, nkv: int, num_cus: int = 256) -> tuple[int, int]:
-    """(max_splits, part_size) for the split-KV decode kernel.
+    """(max_splits, part_size) for the split-KV decode kernel, as its device-side plan (``part_size`` < 0).
 
-    Aim for >= 4 workgroups per CU; part_size is a multiple of 128 tokens
-    (4 waves x 32-token tiles)."""
-    want = max(1, (4 * num_cus + batch * nkv - 1) // max(1, batch * nkv))
-    max_parts = max(1, (max_ctx + 127) // 128)
-    splits = min(want, max_parts)
-    part = ((max_ctx + splits - 1) // splits + 127) // 128 * 128
-    part = max(part, 128)
-    splits = (max_ctx + part - 1) // part
-    return max(1, splits), part
+    One workgroup of eight waves per CU: more splits cost more than they bring (8 kv heads of 128 dims, us a layer with the
+    reduce kernel: 8 rows of 4000 tokens in 2 / 4 / 8 / 16 splits 43.7 / 29.7 / 31.4 / 35.1, 1 row of 8000 in 16 / 32 / 64
+    18.5 / 19.0 / 27.7).  Rows that fill the chip by themselves are not split (64 rows of 1024 in 1 / 2 splits 50.6 / 52.6,
+    of 300 17.6 / 24.1) but past 2048 tokens, so that a few long ones do not hold up the step."""
+    seqs = max(1, batch * nkv)
+    splits, part = (8, 2048) if 2 * seqs > num_cus else (num_cus // seqs, 128)
+    return max(1, min(splits, -(-max_ctx // part))), -part
 
 
 def paged_decode(q, k_cache, v_cache, block_tables, context_lens, nh, nkv, scale,

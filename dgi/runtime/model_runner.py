@@ -433,19 +433,16 @@ class GraphRunner:
 
     def split_plan(self, b: int) -> tuple:
         """(max_splits, part_size) captured for bucket ``b``.  Dynamic (the
-        default): the kernel splits each sequence's own context into up to
-        ~4 workgroups per CU worth of parts of >= 64 tokens, so one graph serves
-        every context length without idle splits; DGI_DECODE_DYNAMIC=0 keeps the
+        default): the kernel splits each sequence's own context
+        (``ops.decode_split_plan``), so one graph serves every context
+        length without idle splits; DGI_DECODE_DYNAMIC=0 keeps the
         fixed max_model_len / part_size plan."""
         r = self.r
         if os.environ.get("DGI_DECODE_DYNAMIC", "1") == "0":
             return r.graph_splits, r.graph_part
-        nkv = r.model.cfg.num_kv_heads
-        want = max(1, -(-4 * r.num_cus // max(1, b * nkv)))
-        # minimum part: 128 tokens (one 32-token tile per wave) below batch 8, 64 above
-        # (profiles/r2_fused_decode_bench.md: best or within 0.3 us at ctx 256-4096)
-        mp = int(os.environ.get("DGI_DECODE_MIN_PART", "0")) or (128 if b < 8 else 64)
-        return min(r.ws_splits, want), -mp
+        want, part = ops.decode_split_plan(b, r.max_model_len, r.model.cfg.num_kv_heads, r.num_cus)
+        part = -int(os.environ.get("DGI_DECODE_MIN_PART", "0")) or part
+        return min(r.ws_splits, want), part
 
     def views(self, b: int) -> dict:
         """Bucket ``b``'s inputs: views into the staging image ``dev_in``."""

@@ -1,0 +1,57 @@
+"""Decode attention's tiles of 32 cached tokens: contexts at the edges of tiles, pages and splits, with no numbers in the
+cache past each context's end; and the plan of the splits."""
+import math
+
+import pytest
+import torch
+
+from dgi import ops
+
+CTX = [1, 15, 16, 17, 31, 32, 33, 64, 127, 129, 255, 257, 289, 640, 1025, 2049]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bs", [16, 32])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("nh,nkv", [(8, 2), (64, 8), (16, 16)])
+@pytest.mark.parametrize("splits,part", [(1, 1 << 20), (3, -128), (20, -64), (8, -2048), (17, 128)])
+def test_contexts_at_edges(bs, hd, nh, nkv, splits, part):
+    g = torch.Generator().manual_seed(bs + hd + nh)
+    need = [-(-c // bs) for c in CTX]
+    pages = sum(need) + 1
+    perm = torch.randperm(pages - 1, generator=g) + 1
+    bt = torch.zeros(len(CTX), max(need), dtype=torch.int32)
+    cache = torch.randn(2, pages, nkv, bs, hd, generator=g).bfloat16()
+    cache[:, 0] = math.nan                                     # nobody's page
+    at = 0
+    for i, (c, n) in enumerate(zip(CTX, need)):
+        bt[i, :n] = perm[at: at + n]
+        at += n
+        if c % bs:
+            cache[:, bt[i, n - 1].long(), :, c % bs:] = math.nan
+    q = torch.randn(len(CTX), nh * hd, generator=g).bfloat16()
+    cache, bt, q = cache.cuda(), bt.cuda(), q.cuda()
+    ctx = torch.tensor(CTX, dtype=torch.int32, device="cuda")
+    scale = hd ** -0.5
+    ref = ops.paged_decode_ref(q, cache[0], cache[1], bt, ctx, nh, nkv, scale)
+    out = ops.paged_decode(q, cache[0], cache[1], bt, ctx, nh, nkv, scale, splits, part)
+    # weights and results are rounded to bf16 (2^-9 each) against values of unit size
+    torch.testing.assert_close(out.float(), ref.float(), atol=2e-2, rtol=2e-2)
+    if splits > 1:
+        ws = (torch.empty(len(CTX) * nh * splits * hd, device="cuda"), torch.empty(len(CTX) * nh * splits, device="cuda"))
+        again = ops.paged_decode(q, cache[0], cache[1], bt, ctx, nh, nkv, scale, splits, part, workspace=ws)
+        torch.testing.assert_close(again.float(), ref.float(), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("batch,ctx,nkv", [(1, 1, 8), (1, 8000, 8), (2, 600, 8), (8, 4000, 8), (12, 900, 8), (17, 9000, 8), (64, 1024, 8),
+                                           (350, 40000, 8), (300, 100, 1), (1, 1 << 17, 1), (3, 5000, 7)])
+def test_plan_of_splits(batch, ctx, nkv):
+    """At least one split, none that a longest context would leave empty, a workspace of 128-token parts holds them, and no
+    more than one workgroup per unit but for long contexts of many rows."""
+    splits, part = ops.decode_split_plan(batch, ctx, nkv)
+    assert part < 0 and part % 32 == 0
+    assert 1 <= splits <= max(1, -(-ctx // 128))
+    if splits > 1:
+        assert (splits - 1) * -part < ctx
+    if batch * nkv * splits > 256:
+        assert splits <= 8 and (splits == 1 or ctx > 2048)
