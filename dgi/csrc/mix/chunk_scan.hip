@@ -14,7 +14,7 @@
 // substitution with blocks of four tokens, each block one matrix product with M_b = [inverse of its diagonal block - I;
 // - T below it times that inverse].  (gla: chunk_scan_decay.hip.)
 //
-// A workgroup owns (sequence, head, NC blocks of 16 value columns) and is a pipeline of waves that hand chunks on through LDS, one
+// A workgroup owns (sequence, head, NC blocks of 16 value columns: two, or four, see four_blocks) and is a pipeline of waves that hand chunks on through LDS, one
 // barrier per chunk:
 //   preparing waves  load q / k (and the channel decays) two chunks ahead in registers and write them (scaled) to LDS;
 //   gates wave       gates of 64 tokens at a time (in four steps, so that none is long), D and A of each chunk;
@@ -29,7 +29,7 @@
 // by k, substitution, update) or a preparing wave's arithmetic (wkv): a wave issues an instruction every four to five cycles at best, so
 // addresses are lane offsets kept in registers, and rows past the end a branch of their own.  Measured, a step of 2 prompts of 4096 rows in
 // all, 64 heads, states 64 x 64 (ssm 128 x 64), against the same token by token on the vector ALUs (linear_scan.hip, ssm_scan.hip):
-// delta 178 us (726), ssm 209 (637), wkv 232 (some 630), light 158 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 103 (322).
+// delta 178 us (726), ssm 209 (637), wkv 232 (some 630), light 158 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 83 (322; 103 in two column blocks a workgroup).
 //
 // Precision: results and states are no further from 64 bits than the token loop's (2-norm over 1300 to 4096 rows: ssm 7.8e-8, the loop 8.0e-8;
 // delta 1.17e-7, 1.18e-7; wkv 9.8e-8, 1.01e-7; but states of wkv on bf16 rows 7.34e-8, 7.28e-8: the loop's products of bf16 keys and values
@@ -131,11 +131,11 @@ __device__ __forceinline__ float sum16(const float* v, int lane) {
 
 // LDS (floats) and roles of a workgroup.  NT: 16-channel tiles (dk <= 16 NT).  A chunk's steps, in order: q / k written, scores (two
 // steps; one for NT 16, whose buffers must be fewer), state, output: an array read d steps after it is written has d + 1 buffers.
-template <int MODE, int NT>
+template <int MODE, int NT, int COLS>
 struct Lay {
   static constexpr bool CH = MODE == WKV;                      // decays per key channel
   static constexpr bool TURNS = CH || MODE == LIGHT;           // two sets of preparing waves take turns, two steps a chunk
-  static constexpr int NC = NT <= 8 ? 2 : 1, W2 = NT <= 8 ? 2 : 1;
+  static constexpr int NC = COLS / 16, W2 = NT <= 8 ? 2 : 1;         // column blocks, scores waves
   static constexpr int NS = NT / 4;                            // preparing waves of 64 channels
   static constexpr int NA = NT == 4 ? 4 : 8;                   // sums side by side of a sum over the channels: state waves
   static constexpr int NO = MODE == WKV || (MODE == DELTA && NT == 8) ? 8 : 4;      // output waves (delta, 128 channels: with 4 results were 2 % further off than the loop's)
@@ -144,7 +144,7 @@ struct Lay {
   static constexpr int SETS = CH && NT == 4 ? 2 : 1;           // channel decays: one set of preparing waves for the scores, one for the state
   static constexpr int PREPS = (TURNS ? 2 : 1) * NS * SETS;    // preparing waves, EARLY of them before the scores waves
   static constexpr int EARLY = NC == 1 ? 0 : (CH ? 2 : (MODE == MLSTM ? 0 : 1));
-  static constexpr int OUT = NC, GATES = 2 * NC, NORM = GATES + 1, SCORES = NC == 1 ? 3 : 6, PREP = SCORES + W2;
+  static constexpr int OUT = NC, GATES = 2 * NC, NORM = GATES + 1, SCORES = NC == 1 ? 3 : 2 * NC + 2, PREP = SCORES + W2;
   static constexpr int WAVES = PREP + PREPS - EARLY;
   // every wave has one role: a wave left over would run as an output wave of columns that are another workgroup's
   static_assert(SCORES - EARLY == (CH ? GATES : MODE == MLSTM ? NORM + 1 : GATES + 1), "state, output, gates, normaliser, preparing, scores");
@@ -175,15 +175,65 @@ struct Lay {
 // over the tokens starts with the oldest, which under a decay are the small ones.
 __device__ __forceinline__ constexpr int place(int t) { return 4 * (t & 3) + (t >> 2); }      // its own inverse
 
-// two waves per SIMD at least: within 256 registers the products take ordinary registers, without moves to accumulation ones
+// Whether workgroups of four column blocks are there for a kernel: not where its waves (thirteen, so 128 registers each) would spill (ssm, wkv, mlstm
+// on fp32 rows or over 128 channels: 1 prompt of 1000 and 5 decode rows, 64 heads, 219 us -> 268), or its LDS would not suffice.
 template <int MODE, typename TI, int NT>
-__global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_kernel(const ChunkArgs a) {
-  using L = Lay<MODE, NT>;
+constexpr bool has_four() {
+  return MODE == LIGHT || (NT == 4 && (MODE == DELTA || (MODE == MLSTM && sizeof(TI) == 2)));
+}
+
+// Steps whose workgroups of two column blocks do not find a compute unit each: four blocks share what does not depend on the columns
+// (q, k, gates, scores), at SLOW hundredths of two blocks' time per chunk.  Only the lengths say which is the faster (decode rows and short portions
+// take no place for long), so the workgroups decide: all chunks over 256 units and a part of the longest sequence's for the last round, or the longest
+// sequence's if that is more.  seq, the seq-th longest before, becomes the sequence itself.
+//   us before (two blocks, sequences in their order) and now, 64-wide heads       mlstm        light       delta
+//   5 prompts of 3001 bf16 rows in all, 32 heads                                  104, 84      95, 80      97, 91
+//   12 prompts of 4000, 64 heads                                                  198, 140     176, 130    173, 158
+//   9 prompts of 1500, 32 heads                                                   62, 54       56, 50      51, 54
+//   1 prompt of 2048 and 3 decode rows, 64 heads (stays at two blocks)            172, 167     147, 150    242, 157
+constexpr int MOST_SEQ = 16;       // more would be decode rows mostly, whose workgroups should be gone soon
+template <int MODE, int NT>
+__device__ __forceinline__ bool four_blocks(const ChunkArgs& a, int& seq, int& row0, int& n) {
+  constexpr int SLOW = MODE == DELTA ? 150 : MODE == MLSTM ? 130 : NT == 4 ? 135 : 155;
+  const int lane = threadIdx.x & 63, i = min(lane, a.n_seq - 1);
+  const int from = a.seq_row0[i], len = lane < a.n_seq ? max(a.seq_row0[i + 1] - from, 0) : -1;
+  int before = 0;                                    // sequences that are longer, or as long and earlier
+  for (int j = 0; j < a.n_seq; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    before += other > len || (other == len && j < lane);
+  }
+  seq = __ffsll((unsigned long long)__ballot(lane < a.n_seq && before == seq)) - 1;
+  row0 = __builtin_amdgcn_readlane(from, seq);
+  n = __builtin_amdgcn_readlane(len, seq);
+  const float own = len > a.skip_rows ? (float)((len + C - 1) / C + 5) : 0.f;      // the pipeline fills in some five
+  float sum = own, most = own;
+#pragma unroll
+  for (int o = MOST_SEQ / 2; o > 0; o >>= 1) {
+    sum += __shfl_xor(sum, o, 64);
+    most = fmaxf(most, __shfl_xor(most, o, 64));
+  }
+  const float units = (float)__popcll(__ballot(own > 0.f)) * a.H, part = sum * a.H / 256.f;
+  auto time = [&](int blocks) { return fmaxf(most, part * blocks + (units * blocks > 256.f ? most * 0.5f : 0.f)); };
+  return __builtin_amdgcn_readfirstlane(time((a.dv + 31) / 32) * 100.f > time((a.dv + 63) / 64) * SLOW);
+}
+
+// two waves per SIMD at least: within 256 registers the products take ordinary registers, without moves to accumulation ones
+template <int MODE, typename TI, int NT, int COLS>
+__global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_scan_kernel(const ChunkArgs a) {
+  using L = Lay<MODE, NT, COLS>;
   constexpr int QR = L::QR, DP = L::DP, NS = L::NS, LEAD = L::LEAD;
   extern __shared__ __attribute__((aligned(16))) float sm[];
   // consecutive workgroups (which go to different XCDs) own consecutive heads; a head's workgroups come n_seq * H later
-  const int head = blockIdx.x % a.H, seq = blockIdx.x / a.H % a.n_seq, zb = blockIdx.x / a.H / a.n_seq, seg = MODE == SSM ? blockIdx.y : 0;
-  int row0 = a.seq_row0[seq], n = a.seq_row0[seq + 1] - row0;
+  const int head = blockIdx.x % a.H, zb = blockIdx.x / a.H / a.n_seq, seg = MODE == SSM ? blockIdx.y : 0;
+  int seq = blockIdx.x / a.H % a.n_seq, blocks = L::NC;      // blocks: of columns, this workgroup's
+  int row0, n;
+  if constexpr (COLS == 64) {
+    blocks = four_blocks<MODE, NT>(a, seq, row0, n) ? 4 : 2;       // the same in every workgroup
+    if (zb * blocks * 16 >= a.dv) return;            // the grid is that of two blocks each
+  } else {
+    row0 = a.seq_row0[seq];
+    n = a.seq_row0[seq + 1] - row0;
+  }
   if (n <= a.skip_rows) return;
   const int slot = a.seq_slots[seq];
   // ssm in segments (see below): 1 the state of a segment from nothing, to the workspace; 2 outputs from the state found there
@@ -821,8 +871,13 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT>::WAVES), 2) void chunk_scan_ker
   }
 
   const bool outputs = wave >= L::OUT;
-  const int cw = outputs ? wave - L::OUT : wave;     // column block of the workgroup
-  const int col = (zb * L::NC + cw) * 16 + n16, colc = min(col, dv - 1);
+  // column block of the workgroup (two of four: those of the outputs beside other SIMDs than those of the state)
+  const int cw = outputs ? wave - L::OUT - (COLS == 64 && blocks == 2 ? 2 : 0) : wave;
+  if (COLS == 64 && (cw < 0 || cw >= blocks)) {
+    barriers(chunks + LEAD);
+    return;
+  }
+  const int col = (zb * blocks + cw) * 16 + n16, colc = min(col, dv - 1);
   const bool cok = col < dv;
   const TI* vb = (const TI*)a.v + (size_t)row0 * a.v_stride + (size_t)head * dv;
   auto tok = [&](int r) { return 4 * r + g; };
@@ -1060,12 +1115,12 @@ __global__ __launch_bounds__(256) void ssm_segments_kernel(float* __restrict__ w
   }
 }
 
-template <int MODE, typename TI, int NT>
+template <int MODE, typename TI, int NT, int COLS>
 int launch_one(const ChunkArgs& a, dim3 grid, hipStream_t st) {
-  using L = Lay<MODE, NT>;
+  using L = Lay<MODE, NT, COLS>;
   constexpr size_t lds = (size_t)L::END * 4;
   static_assert(lds <= 160 * 1024, "LDS");
-  auto kernel = chunk_scan_kernel<MODE, TI, NT>;
+  auto kernel = chunk_scan_kernel<MODE, TI, NT, COLS>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
@@ -1075,16 +1130,24 @@ int launch_one(const ChunkArgs& a, dim3 grid, hipStream_t st) {
 }
 
 template <int MODE, typename TI>
-int launch_dims(const ChunkArgs& a, dim3 grid, hipStream_t st) {
-  if (a.dk <= 64) return launch_one<MODE, TI, 4>(a, grid, st);
-  if (a.dk <= 128) return launch_one<MODE, TI, 8>(a, grid, st);
+int launch_dims(const ChunkArgs& a, bool four, dim3 grid, hipStream_t st) {
+  if (a.dk <= 64) {
+    if constexpr (has_four<MODE, TI, 4>())
+      if (four) return launch_one<MODE, TI, 4, 64>(a, grid, st);
+    return launch_one<MODE, TI, 4, 32>(a, grid, st);
+  }
+  if (a.dk <= 128) {
+    if constexpr (has_four<MODE, TI, 8>())
+      if (four) return launch_one<MODE, TI, 8, 64>(a, grid, st);
+    return launch_one<MODE, TI, 8, 32>(a, grid, st);
+  }
   if constexpr (MODE != SSM) return -3;
-  else return launch_one<MODE, TI, 16>(a, grid, st);
+  else return launch_one<MODE, TI, 16, 16>(a, grid, st);
 }
 
 template <int MODE>
-int launch_mode(const ChunkArgs& a, int in_f32, dim3 grid, hipStream_t st) {
-  return in_f32 ? launch_dims<MODE, float>(a, grid, st) : launch_dims<MODE, uint16_t>(a, grid, st);
+int launch_mode(const ChunkArgs& a, int in_f32, bool four, dim3 grid, hipStream_t st) {
+  return in_f32 ? launch_dims<MODE, float>(a, four, grid, st) : launch_dims<MODE, uint16_t>(a, four, grid, st);
 }
 
 }  // namespace
@@ -1110,7 +1173,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
                               int segs, int seg_rows, float* ws, float* wsd, hipStream_t st) {
   if (n_seq == 0) return 0;
-  const int cols = dk <= 128 ? 32 : 16;            // value columns of a workgroup
+  const int cols = dk <= 128 ? 32 : 16;            // value columns of a workgroup (or twice as many, see four_blocks)
   const long long nz = (dv + cols - 1) / cols;
   if (!dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32) || dv <= 0 || H <= 0 || G <= 0 || H % G) return -3;
   if (mode == MLSTM && nz > 1 && (!norm_new || !mx_new)) return -7;
@@ -1126,8 +1189,10 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
   a.n_seq = n_seq; a.seg_rows = seg_rows; a.ws = ws; a.wsd = wsd;
   a.pass = segs > 1 ? 1 : 0;
   const dim3 grid((unsigned)(n_seq * nz * H), segs > 1 ? segs : 1);
+  // more workgroups than compute units: possibly of four column blocks each
+  const bool four = dv > 32 && n_seq <= MOST_SEQ && n_seq * nz * H > 256;
   if (a.pass) {
-    int rc = launch_dims<SSM, float>(a, grid, st);
+    int rc = launch_dims<SSM, float>(a, false, grid, st);
     if (rc) return rc;
     ssm_segments_kernel<<<dim3(n_seq, H, (dk * dv + 255) / 256), 256, 0, st>>>(ws, wsd, state, positions, seq_row0, seq_slots, H, dk * dv, segs,
                                                                                seg_rows, skip_rows);
@@ -1135,11 +1200,11 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
   }
   int rc = -2;
   switch (mode) {
-    case WKV: rc = launch_mode<WKV>(a, in_f32, grid, st); break;
-    case DELTA: rc = launch_mode<DELTA>(a, in_f32, grid, st); break;
-    case MLSTM: rc = launch_mode<MLSTM>(a, in_f32, grid, st); break;
-    case LIGHT: rc = launch_mode<LIGHT>(a, in_f32, grid, st); break;
-    case SSM: rc = in_f32 ? launch_dims<SSM, float>(a, grid, st) : -2; break;
+    case WKV: rc = launch_mode<WKV>(a, in_f32, four, grid, st); break;
+    case DELTA: rc = launch_mode<DELTA>(a, in_f32, four, grid, st); break;
+    case MLSTM: rc = launch_mode<MLSTM>(a, in_f32, four, grid, st); break;
+    case LIGHT: rc = launch_mode<LIGHT>(a, in_f32, four, grid, st); break;
+    case SSM: rc = in_f32 ? launch_dims<SSM, float>(a, false, grid, st) : -2; break;
   }
   if (rc) return rc;
   DGI_CHECK_LAUNCH();
