@@ -130,6 +130,9 @@ int dgi_moe_plan(const int* idx, int P, int E, int* order, int* where, int* seg,
 int dgi_moe_group(const void* a, int a_stride, const void* b, void* out, const int* seg, const int* order,
                   const float* pair_scale, int places, int E, int N, int K, int top, int glu, int act, float limit, float alpha,
                   int rows_per_tile, hipStream_t s);
+int dgi_moe_plan_group(const int* idx, int P, int* order, int* where, int* seg, const void* a, int a_stride, const void* b, void* out,
+                       const float* pair_scale, int E, int N, int K, int top, int act, float limit, float alpha, int rows_per_tile,
+                       hipStream_t s);
 int dgi_moe_combine(void* out, const void* ys, const int* where, const void* h, int h_stride, const int* idx,
                     const float* wts, const void* shared, int shared_stride, int T, int E, int top, int W, int is_f32,
                     hipStream_t s);
@@ -606,6 +609,22 @@ void moe_group(at::Tensor out, const at::Tensor& a, const at::Tensor& b, const a
   check_rc(dgi_moe_group(a.data_ptr(), (int)a.stride(0), b.data_ptr(), out.data_ptr(), seg.data_ptr<int>(), op,
                          f32p(pair_scale, "pair_scale", places), (int)places, (int)E, (int)N, (int)K, (int)top, glu ? 1 : 0, (int)act,
                          (float)limit, (float)alpha, (int)rows_per_tile, cur_stream()), "moe_group");
+}
+
+// moe_plan, then moe_group with its order: out [pairs, N], a [rows, K], idx [rows, top], b [E, 2 N, K]
+void moe_plan_group(at::Tensor out, at::Tensor order, at::Tensor where, at::Tensor seg, const at::Tensor& idx, const at::Tensor& a,
+                    const at::Tensor& b, const c10::optional<at::Tensor>& pair_scale, int64_t top, int64_t act, double limit, double alpha,
+                    int64_t rows_per_tile) {
+  TORCH_CHECK(act_kind(a, "a") == 0 && act_kind(b, "b") == 0 && act_kind(out, "out") == 0, "moe_plan_group: bfloat16 only");
+  check_rows(a, "a");
+  TORCH_CHECK(b.is_contiguous() && b.dim() == 3 && out.is_contiguous() && out.dim() == 2 && a.size(1) == b.size(2));
+  const int64_t P = idx.numel(), E = b.size(0), N = out.size(1), K = a.size(1);
+  TORCH_CHECK(b.size(1) == 2 * N && out.size(0) == P && P < (int64_t(1) << 31) && top >= 1 && a.size(0) * top >= P, "moe_plan_group: shapes");
+  check_i32(order, "order"); check_i32(where, "where"); check_i32(seg, "seg");
+  TORCH_CHECK(order.numel() == P && where.numel() == P && seg.numel() == E + 1);
+  check_rc(dgi_moe_plan_group(i32p(idx, "idx"), (int)P, order.data_ptr<int>(), where.data_ptr<int>(), seg.data_ptr<int>(), a.data_ptr(),
+                              (int)a.stride(0), b.data_ptr(), out.data_ptr(), f32p(pair_scale, "pair_scale", P), (int)E, (int)N, (int)K, (int)top,
+                              (int)act, (float)limit, (float)alpha, (int)rows_per_tile, cur_stream()), "moe_plan_group");
 }
 
 void moe_combine(at::Tensor out, const at::Tensor& ys, const c10::optional<at::Tensor>& where, const at::Tensor& h, const at::Tensor& idx,
@@ -1247,6 +1266,8 @@ TORCH_LIBRARY_FRAGMENT(dgi, m) {
   m.def("moe_plan(Tensor(a!) order, Tensor(b!) where, Tensor(c!) seg, Tensor idx) -> ()");
   m.def("moe_group(Tensor(a!) out, Tensor a, Tensor b, Tensor seg, Tensor? order, Tensor? pair_scale, int top, int act, float limit, "
         "float alpha, int rows_per_tile) -> ()");
+  m.def("moe_plan_group(Tensor(a!) out, Tensor(b!) order, Tensor(c!) where, Tensor(d!) seg, Tensor idx, Tensor a, Tensor b, Tensor? pair_scale, "
+        "int top, int act, float limit, float alpha, int rows_per_tile) -> ()");
   m.def("moe_combine(Tensor(a!) out, Tensor ys, Tensor? where, Tensor h, Tensor idx, Tensor? wts, Tensor? shared, int E) -> ()");
 }
 
@@ -1294,5 +1315,6 @@ TORCH_LIBRARY_IMPL(dgi, CUDA, m) {
   m.impl("moe_router", &moe_router);
   m.impl("moe_plan", &moe_plan);
   m.impl("moe_group", &moe_group);
+  m.impl("moe_plan_group", &moe_plan_group);
   m.impl("moe_combine", &moe_combine);
 }

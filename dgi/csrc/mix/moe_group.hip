@@ -79,13 +79,13 @@ __global__ __launch_bounds__(PLAN_NT) void moe_plan_kernel(const int* __restrict
 }
 
 // The m-tile `tile` of BM places: its expert and places [lo, hi); false past the last tile.  Uniform over the wave.
-template <int BM>
-__device__ __forceinline__ bool find_tile(const int* __restrict__ seg, int E, int tile, int& e, int& lo, int& hi) {
+template <int BM, typename Seg>
+__device__ __forceinline__ bool find_tile(const Seg& seg, int E, int tile, int& e, int& lo, int& hi) {
   const int lane = threadIdx.x & 63;
   int base = 0;                                        // tiles of the experts before this round's 64
   for (int e0 = 0; e0 < E; e0 += 64) {
     const int ee = e0 + lane;
-    const int s0 = ee < E ? seg[ee] : 0, s1 = ee < E ? seg[ee + 1] : 0;
+    const int s0 = ee < E ? seg(ee) : 0, s1 = ee < E ? seg(ee + 1) : 0;
     const int n = (s1 - s0 + BM - 1) / BM;
     int inc = n;                                       // inclusive prefix over the lanes
 #pragma unroll
@@ -128,6 +128,9 @@ struct GroupArgs {
   int E, N, K, top, act;
   float limit, alpha;
   int mtiles;
+  const int* idx;             // the pairs' experts where the kernel sorts them itself; to order, where and seg for the kernels that follow
+  int pairs;
+  int *order_out, *where_out, *seg_out;
 };
 
 __device__ __forceinline__ void load_lds16(const char* src, char* lds) {
@@ -161,7 +164,7 @@ __global__ __launch_bounds__(256) void moe_group_rows_kernel(GroupArgs g) {
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int lr = lane & 15, lg = lane >> 4;
   int e, lo, hi;
-  if (!find_tile<16 * MB>(g.seg, g.E, blockIdx.x % g.mtiles, e, lo, hi)) return;
+  if (!find_tile<16 * MB>([&](int i) { return g.seg[i]; }, g.E, blockIdx.x % g.mtiles, e, lo, hi)) return;
   e = __builtin_amdgcn_readfirstlane(e);
   const int K = g.K;
   constexpr int NO = GLU ? 32 : 64;                    // outputs per workgroup
@@ -270,26 +273,82 @@ __global__ __launch_bounds__(256) void moe_group_rows_kernel(GroupArgs g) {
 //
 // 16 experts, top 2, the whole feed-forward (16 to 20 us of it router, plan and combine), against weights straight to registers
 // (64 rows a workgroup, K over its waves; 128 x 128 tiles from 4 or 12 places an expert on):
-//   widths 2048 x 2048: 1 row 36 us -> 30, 8 rows 93 -> 62, 32 rows 110 -> 84 (6.0 TB/s in the products), 128 rows 130 -> 88
+//   widths 2048 x 2048: 1 row 36 us -> 30, 8 rows 93 -> 62, 32 rows 110 -> 84 (6.0 TB/s in the products), 128 rows 130 -> 88 (a plan kernel before them)
 //   widths 4096 x 3584: 1 row 70 -> 52, 8 rows 227 -> 165, 32 rows 285 -> 232 (6.5 TB/s)
 constexpr int STREAM_WGS = 256;
 
+// PLAN (gate-up of a step of at most PLAN_PAIRS pairs and PLAN_EXPERTS experts): every workgroup sorts the pairs itself, a pair per thread, where it
+// would have read seg and order; the first one writes them for the kernels that follow.  A launch less: the whole feed-forward,
+// 16 experts of 2048 x 2048, 1 row 31.0 us -> 28.7, 32 rows 86.0 -> 83.2.
+//
 // KS: stages of 64 of K per wave at the most.  K a multiple of 64.
-template <int MB, int KS, bool GLU>
+constexpr int PLAN_PAIRS = 512, PLAN_EXPERTS = 64;
+
+template <int MB, int KS, bool GLU, bool PLAN>
 __global__ __launch_bounds__(512) void moe_group_stream_kernel(GroupArgs g) {
   constexpr int D = MB == 4 ? 5 : 6;                   // stages of 16 rows x 64 of K, 2 KB each, per wave
   // one array: with two, the compiler waits for all loads to LDS before every read of it
-  __shared__ __attribute__((aligned(16))) char lds[8 * D * 2048 + 2 * 8 * MB * 1024];      // [wave][stage], partial sums [2][wave][MB][64][4]
+  constexpr int RED = 8 * D * 2048, TAB = RED + 2 * 8 * MB * 1024;
+  __shared__ __attribute__((aligned(16))) char lds[TAB + (PLAN ? 4 * (PLAN_PAIRS + PLAN_EXPERTS + 1) : 0)];      // [wave][stage], partial sums [2][wave][MB][64][4], order and seg
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int lr = lane & 15, lg = lane >> 4;
   const int K = g.K;
   constexpr int NO = GLU ? 8 : 16;                     // outputs of a block
   const int nblk = (g.N + NO - 1) / NO;
+  int* const order_lds = reinterpret_cast<int*>(lds + TAB);
+  int* const seg_lds = order_lds + PLAN_PAIRS;
+  auto pair_of = [&](int place) { return PLAN ? order_lds[place] : g.order[place]; };
+  if constexpr (PLAN) {
+    // pairs of a wave's 64 threads by expert, then the experts' sums over the waves; a pair's place: those of lower experts, and of its own before it
+    const int tid = threadIdx.x, r = tid < g.pairs ? g.idx[tid] : -1;
+    const bool ok = r >= 0 && r < g.E;
+    int* const cnt = reinterpret_cast<int*>(lds);      // [wave][expert]
+    cnt[tid] = 0;
+    unsigned long long same = __ballot(ok);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      const unsigned long long m = __ballot((r >> b) & 1);
+      same &= (r >> b) & 1 ? m : ~m;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    __syncthreads();
+    if (ok && rank == 0) cnt[w * 64 + r] = __popcll(same);
+    __syncthreads();
+    int all = 0, before = 0;                           // of expert `lane`, and of the waves before this one
+#pragma unroll
+    for (int ww = 0; ww < 8; ++ww) {
+      const int c = cnt[ww * 64 + lane];
+      all += c;
+      before += ww < w ? c : 0;
+    }
+    int upto = all;                                    // inclusive over the experts
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += v;
+    }
+    const int place = __shfl(upto - all + before, ok ? r : 0, 64) + rank;
+    if (ok) order_lds[place] = tid;
+    if (w == 0) {
+      seg_lds[lane + 1] = upto;
+      if (lane == 0) seg_lds[0] = 0;
+    }
+    if (blockIdx.x == 0) {
+      if (ok) {
+        g.order_out[place] = tid;
+        g.where_out[tid] = place;
+      }
+      if (w == 0 && lane < g.E) g.seg_out[lane + 1] = upto;
+      if (tid == 0) g.seg_out[0] = 0;
+    }
+    __syncthreads();                                   // the counts are read: the waves load over them
+  }
+  auto seg_of = [&](int e) { return PLAN ? seg_lds[e] : g.seg[e]; };
   // this workgroup's blocks
   int tiles = 0;
   for (int e0 = 0; e0 < g.E; e0 += 64) {
     const int ee = e0 + lane;
-    tiles += ee < g.E ? (g.seg[ee + 1] - g.seg[ee] + 16 * MB - 1) / (16 * MB) : 0;
+    tiles += ee < g.E ? (seg_of(ee + 1) - seg_of(ee) + 16 * MB - 1) / (16 * MB) : 0;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) tiles += __shfl_xor(tiles, o, 64);
@@ -302,13 +361,13 @@ __global__ __launch_bounds__(512) void moe_group_stream_kernel(GroupArgs g) {
   const int row8 = lane >> 3;
   const size_t koff = (size_t)w * per * 128 + (((lane & 7) ^ row8) << 4);
   char* const rg = lds + w * (D * 2048);
-  float* const red = reinterpret_cast<float*>(lds + 8 * D * 2048);
+  float* const red = reinterpret_cast<float*>(lds + RED);
   auto sums = [&](int par, int ww, int i) { return reinterpret_cast<f32x4*>(red + ((par * 8 + ww) * MB + i) * 256 + 4 * lane); };
   const int rd0 = lr * 128 + ((lg ^ (lr & 7)) << 4), rd1 = lr * 128 + (((4 + lg) ^ (lr & 7)) << 4);
   int par = 0;
   while (at < end) {
     int e, lo, hi;
-    find_tile<16 * MB>(g.seg, g.E, at / nblk, e, lo, hi);
+    find_tile<16 * MB>(seg_of, g.E, at / nblk, e, lo, hi);
     e = __builtin_amdgcn_readfirstlane(e);
     const int b0 = at % nblk, nb = min(nblk - b0, end - at);
     at += nb;
@@ -318,7 +377,7 @@ __global__ __launch_bounds__(512) void moe_group_stream_kernel(GroupArgs g) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int place = min(lo + 16 * i + 8 * j + row8, hi - 1);
-        ap[i][j] = reinterpret_cast<const char*>(g.a + (size_t)(g.order ? g.order[place] / g.top : place) * g.a_stride) + koff;
+        ap[i][j] = reinterpret_cast<const char*>(g.a + (size_t)(GLU ? pair_of(place) / g.top : place) * g.a_stride) + koff;
       }
     const char* B = reinterpret_cast<const char*>(g.b + (size_t)e * (GLU ? 2 : 1) * g.N * K) + koff;
     auto wrow = [&](int blk, int j) {                  // GLU: LDS row r holds the gate (r & 2: up) row of output 2 (r >> 2) + (r & 1)
@@ -397,7 +456,7 @@ __global__ __launch_bounds__(512) void moe_group_stream_kernel(GroupArgs g) {
           uint16_t* row = g.out + (size_t)place * g.N;
           const bool vec = (g.N & 3) == 0 && ((uintptr_t)g.out & 7) == 0;
           if constexpr (GLU) {
-            const float ps = g.pair_scale ? g.pair_scale[g.order[place]] : 1.f;
+            const float ps = g.pair_scale ? g.pair_scale[pair_of(place)] : 1.f;
             const int n = (b0 + blk) * NO + 2 * lg;
             const float x = glu_f(t[0] * ps, t[2] * ps, g.act, g.limit, g.alpha), y = glu_f(t[1] * ps, t[3] * ps, g.act, g.limit, g.alpha);
             if (vec) {
@@ -434,7 +493,7 @@ __global__ __launch_bounds__(256, 2) void moe_group_tiles_kernel(GroupArgs g, in
   const int id = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
   if (id >= total) return;
   int e, lo, hi;
-  if (!find_tile<128>(g.seg, g.E, id % g.mtiles, e, lo, hi)) return;
+  if (!find_tile<128>([&](int i) { return g.seg[i]; }, g.E, id % g.mtiles, e, lo, hi)) return;
   constexpr int NO = GLU ? 64 : 128;
   const int n0 = (id / g.mtiles) * NO;
   const uint16_t* B = g.b + (size_t)e * (GLU ? 2 : 1) * g.N * g.K;
@@ -762,6 +821,19 @@ __global__ __launch_bounds__(512) void moe_group_wide_kernel(GroupArgs g, int nt
     }
 }
 
+template <int MB, int KS, bool GLU>
+void launch_stream(const GroupArgs& g, hipStream_t s) {
+  if constexpr (GLU)
+    if (g.idx) {
+      moe_group_stream_kernel<MB, KS, true, true><<<STREAM_WGS, 512, 0, s>>>(g);
+      return;
+    }
+  moe_group_stream_kernel<MB, KS, GLU, false><<<STREAM_WGS, 512, 0, s>>>(g);
+}
+
+// a tile's rows of A fill half the registers of a compute unit at the most
+bool streams(int bm, int K) { return bm <= 64 && K % 64 == 0 && bm * K <= 1 << 17; }
+
 template <bool GLU>
 int launch_group(GroupArgs g, int places, int rows_per_tile, hipStream_t s) {
   // worst split of the places over the experts: every non-empty expert may end in a partial tile
@@ -783,17 +855,17 @@ int launch_group(GroupArgs g, int places, int rows_per_tile, hipStream_t s) {
     moe_group_wide_kernel<GLU><<<padded, 512, 0, s>>>(g, ntn);
   } else if (bm == 128) {
     moe_group_tiles_kernel<GLU><<<padded, 256, 0, s>>>(g, ntn);
-  } else if (g.K % 64 == 0 && bm * g.K <= 1 << 17) {     // a tile's rows of A fill half the registers of a compute unit at the most
+  } else if (streams(bm, g.K)) {
     const int ks = (g.K / 64 + 7) / 8;                   // at most 16, 8, 4
     if (bm == 16) {
-      if (ks <= 4) moe_group_stream_kernel<1, 4, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
-      else if (ks <= 8) moe_group_stream_kernel<1, 8, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
-      else moe_group_stream_kernel<1, 16, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+      if (ks <= 4) launch_stream<1, 4, GLU>(g, s);
+      else if (ks <= 8) launch_stream<1, 8, GLU>(g, s);
+      else launch_stream<1, 16, GLU>(g, s);
     } else if (bm == 32) {
-      if (ks <= 4) moe_group_stream_kernel<2, 4, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
-      else moe_group_stream_kernel<2, 8, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+      if (ks <= 4) launch_stream<2, 4, GLU>(g, s);
+      else launch_stream<2, 8, GLU>(g, s);
     } else {
-      moe_group_stream_kernel<4, 4, GLU><<<STREAM_WGS, 512, 0, s>>>(g);
+      launch_stream<4, 4, GLU>(g, s);
     }
   } else if (bm == 64) {
     moe_group_rows_kernel<4, GLU><<<(int)blocks, 256, 0, s>>>(g);
@@ -916,8 +988,26 @@ extern "C" int dgi_moe_group(const void* a, int a_stride, const void* b, void* o
   if (places == 0 || N == 0) return 0;
   if (K <= 0 || K % 8 || a_stride % 8 || (((uintptr_t)a | (uintptr_t)b) & 15) || E <= 0 || (glu && (!order || top <= 0))) return -2;
   GroupArgs g{(const uint16_t*)a, a_stride, (const uint16_t*)b, (uint16_t*)out, seg, glu ? order : nullptr, pair_scale,
-              E, N, K, top, act, limit, alpha, 0};
+              E, N, K, top, act, limit, alpha, 0, nullptr, 0, nullptr, nullptr, nullptr};
   const int rc = glu ? launch_group<true>(g, places, rows_per_tile, s) : launch_group<false>(g, places, rows_per_tile, s);
+  if (rc) return rc;
+  DGI_CHECK_LAUNCH();
+  return 0;
+}
+
+// moe_plan and the gate-up product: in one launch where the product's workgroups can sort the pairs themselves
+extern "C" int dgi_moe_plan_group(const int* idx, int P, int* order, int* where, int* seg, const void* a, int a_stride, const void* b, void* out,
+                                  const float* pair_scale, int E, int N, int K, int top, int act, float limit, float alpha, int rows_per_tile,
+                                  hipStream_t s) {
+  if (P == 0 || N == 0 || P > PLAN_PAIRS || E > PLAN_EXPERTS || !streams(rows_per_tile, K)) {
+    const int rc = dgi_moe_plan(idx, P, E, order, where, seg, s);
+    return rc ? rc : dgi_moe_group(a, a_stride, b, out, seg, order, pair_scale, P, E, N, K, top, 1, act, limit, alpha, rows_per_tile, s);
+  }
+  if (K <= 0 || a_stride % 8 || (((uintptr_t)a | (uintptr_t)b) & 15) || E <= 0 || top <= 0) return -2;
+  if (rows_per_tile != 16 && rows_per_tile != 32 && rows_per_tile != 64) return -3;
+  const GroupArgs g{(const uint16_t*)a, a_stride, (const uint16_t*)b, (uint16_t*)out, seg, order, pair_scale,
+                    E, N, K, top, act, limit, alpha, 0, idx, P, order, where, seg};
+  const int rc = launch_group<true>(g, P, rows_per_tile, s);
   if (rc) return rc;
   DGI_CHECK_LAUNCH();
   return 0;

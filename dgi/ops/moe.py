@@ -12,11 +12,12 @@ stacked: ``gate_up`` [E, 2 ff, W] (gate rows, then up rows) and ``down`` [E, W, 
 
 Two evaluation paths on the GPU, same result up to summation order:
 
-* bf16: the pairs are sorted by expert on the device (``moe_plan``), two grouped matrix-core products
-  (``moe_group``, gate-up with the activation as its epilogue, then down) walk the experts' segments, and a
-  combine kernel gathers each token's routes in their fixed order (deterministic, no atomics, no host round
-  trip: the same path inside and outside captured graphs).  Tiles of 16 to 64 places whose weights are streamed
-  when experts have few rows (bounded by the weights' bytes), of 128 or 256 places otherwise;
+* bf16: the pairs are sorted by expert on the device (``moe_plan``, or in small steps by the gate-up product
+  itself: ``moe_plan_group``), two grouped matrix-core products (``moe_group``, gate-up with the activation as
+  its epilogue, then down) walk the experts' segments, and a combine kernel gathers each token's routes in their
+  fixed order (deterministic, no atomics, no host round trip: the same path inside and outside captured graphs).
+  Tiles of 16 to 64 places whose weights are streamed when experts have few rows (bounded by the weights' bytes),
+  of 128 or 256 places otherwise;
 * fp32 and widths that are no multiple of 8 — few rows (and every step inside a captured graph): workgroups own
   (expert, output tile) and walk the pairs that chose the expert; many rows: one vendor GEMM pair per
   expert over its sorted segment.
@@ -201,9 +202,8 @@ def moe_experts(h, idx, wts, gate_up, down, shared=None, act: str = "silu", limi
         if T > 0:
             tile = group_tile(P, E, W * ff)
             kind = 1 if act == "clamped" else 0
-            _call("moe_plan", order, where, seg, idx)
-            _call("moe_group", mid, h, gate_up, seg, order, None if w_in is None else w_in.reshape(-1), top, kind, float(limit),
-                  float(alpha), tile)
+            _call("moe_plan_group", mid, order, where, seg, idx, h, gate_up, None if w_in is None else w_in.reshape(-1), top, kind,
+                  float(limit), float(alpha), tile)
             _call("moe_group", ys, mid, down, seg, None, None, top, 0, 0.0, 0.0, tile)
             _call("moe_combine", out, ys, where, h, idx, w_out, shared, E)
         return out

@@ -57,3 +57,31 @@ def test_tiles_by_the_mean_rows_of_an_expert():
     assert [moe.group_tile(16 * m, 16, big) for m in (1, 4, 5, 20, 21, 40, 41, 95, 96)] == [16, 16, 32, 32, 64, 64, 128, 128, 256]
     assert [moe.group_tile(16 * m, 16, small) for m in (40, 41, 255, 256)] == [64, 128, 128, 256]
     assert [moe.group_tile(64 * m, 64, small) for m in (12, 13)] == [32, 128]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", [16, 32, 64])
+@pytest.mark.parametrize("T,top,E", [(1, 1, 1), (1, 2, 16), (31, 2, 3), (32, 2, 16), (63, 1, 64), (128, 4, 64), (171, 3, 64), (129, 4, 16), (40, 2, 65)])
+def test_pairs_sorted_by_the_product(T, top, E, tile):
+    """Up to 512 pairs and 64 experts the gate-up product sorts the pairs itself: the plan that ``moe_plan`` makes, identity routes
+    (E and beyond) left out, and the same product."""
+    from dgi.ops import _call
+    W, ff = 128, 72
+    g = torch.Generator().manual_seed(T + E)
+    idx = torch.randint(0, E + 2, (T, top), generator=g, dtype=torch.int32).cuda()
+    h, gu = draw(T, W, seed=4).cuda(), draw(E, 2 * ff, W, seed=5, scale=W ** -0.5).cuda()
+    scale = torch.rand(T * top, generator=g).cuda()
+    P = T * top
+    for weights in (None, scale):
+        made = []
+        for fused in (False, True):
+            order, where, seg = (torch.full((n,), -7, dtype=torch.int32, device="cuda") for n in (P, P, E + 1))
+            out = torch.full((P, ff), 3.0, dtype=BF16, device="cuda")
+            if fused:
+                _call("moe_plan_group", out, order, where, seg, idx, h, gu, weights, top, 0, 0.0, 0.0, tile)
+            else:
+                _call("moe_plan", order, where, seg, idx)
+                _call("moe_group", out, h, gu, seg, order, weights, top, 0, 0.0, 0.0, tile)
+            made.append((order, where, seg, out))
+        for a, b in zip(*made):
+            assert torch.equal(a, b)
