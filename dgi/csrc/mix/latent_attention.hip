@@ -285,12 +285,54 @@ void launch_reduce(const float* part_o, const float* part_ml, int nsplit, int ro
 
 // Queries of one row's heads head0 .. head0 + NH - 1 as bf16 rows of stride DP in LDS, [folded part | rotated part]; heads
 // past H are zero rows.  NT threads, kr <= 16 NM.  All loads go out before the first is waited for (addresses past the end
-// are clamped, not skipped), and meanwhile() runs behind the folded part's.
-template <int NH, int NT, int NM, typename F>
+// are clamped, not skipped), and meanwhile() runs behind the folded part's, or where rd is RD behind both parts'.
+template <int NH, int NT, int NM, int RD, typename F>
 __device__ __forceinline__ void stage_queries(uint16_t* qs, int DP, const uint16_t* __restrict__ q, int q_stride,
                                               const uint16_t* __restrict__ q_lat, long long ql_hs, long long ql_ts, int row,
                                               int head0, int H, int dim, int rd, int kr, int pos,
                                               const float* __restrict__ cos_sin, int dims, int interleaved, F&& meanwhile) {
+  // rotated part, U elements of a thread at a time; with RD they are the same element of U heads
+  static_assert(RD == 0 || (NT % RD == 0 && NH * RD % NT == 0), "whole heads");
+  constexpr int U = RD > 0 ? NH * RD / NT : 4, UC = RD > 0 ? 1 : U;
+  const int half = dims >> 1;
+  const float* cs = dims > 0 ? cos_sin + (size_t)max(pos, 0) * dims : nullptr;
+  uint16_t a[U], b[U];
+  float c[UC], sn[UC];
+  auto load_rot = [&](int i0) {
+    int k = 0, partner = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = RD > 0 ? i0 + u * NT : min(i0 + u * NT, NH * rd - 1);
+      const int hh = RD > 0 ? i / RD : i / rd, e = RD > 0 ? i0 % RD : i - hh * rd;
+      const uint16_t* qr = q + (size_t)row * q_stride + (size_t)min(head0 + hh, H - 1) * (dim + rd) + dim;
+      if (RD == 0 || u == 0) {
+        k = 0;
+        partner = e;
+        if (e < dims) {
+          k = interleaved ? e >> 1 : e < half ? e : e - half;
+          partner = interleaved ? e ^ 1 : e < half ? e + half : e - half;
+        }
+        c[u] = sn[u] = 0.f;
+        if (cs) {
+          c[u] = cs[k];
+          sn[u] = cs[half + k];
+        }
+      }
+      a[u] = qr[e];
+      b[u] = qr[partner];
+    }
+  };
+  auto put_rot = [&](int i0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = RD > 0 ? i0 + u * NT : min(i0 + u * NT, NH * rd - 1);
+      const int hh = RD > 0 ? i / RD : i / rd, e = RD > 0 ? i0 % RD : i - hh * rd;
+      const bool lead = interleaved ? !(e & 1) : e < half;                  // the pair's first element
+      const float x = bf16_to_f32(a[u]), y = bf16_to_f32(b[u]), co = c[RD > 0 ? 0 : u], si = sn[RD > 0 ? 0 : u];
+      const uint16_t r = f32_to_bf16(lead ? x * co - y * si : x * co + y * si);
+      qs[(size_t)hh * DP + kr + e] = head0 + hh >= H ? (uint16_t)0 : e < dims ? r : a[u];
+    }
+  };
   const bool qvec = ((uintptr_t)q_lat & 15) == 0 && (ql_hs & 7) == 0 && (ql_ts & 7) == 0;
   if (qvec) {
     constexpr int NQ = (NH * NM * 2 + NT - 1) / NT;
@@ -299,17 +341,19 @@ __device__ __forceinline__ void stage_queries(uint16_t* qs, int DP, const uint16
 #pragma unroll
     for (int it = 0; it < NQ; ++it) {
       const int idx = min((int)threadIdx.x + NT * it, NH * cq - 1);
-      const int hh = idx / cq, c = idx - hh * cq;
-      v[it] = *reinterpret_cast<const u32x4*>(q_lat + (size_t)min(head0 + hh, H - 1) * ql_hs + (size_t)row * ql_ts + c * 8);
+      const int hh = idx / cq, ch = idx - hh * cq;
+      v[it] = *reinterpret_cast<const u32x4*>(q_lat + (size_t)min(head0 + hh, H - 1) * ql_hs + (size_t)row * ql_ts + ch * 8);
     }
+    if constexpr (RD > 0) load_rot(threadIdx.x);
     meanwhile();
 #pragma unroll
     for (int it = 0; it < NQ; ++it) {
       const int idx = min((int)threadIdx.x + NT * it, NH * cq - 1);
-      const int hh = idx / cq, c = idx - hh * cq;
-      *reinterpret_cast<u32x4*>(qs + (size_t)hh * DP + c * 8) = head0 + hh < H ? v[it] : u32x4{0u, 0u, 0u, 0u};
+      const int hh = idx / cq, ch = idx - hh * cq;
+      *reinterpret_cast<u32x4*>(qs + (size_t)hh * DP + ch * 8) = head0 + hh < H ? v[it] : u32x4{0u, 0u, 0u, 0u};
     }
   } else {
+    if constexpr (RD > 0) load_rot(threadIdx.x);
     meanwhile();
     for (int i = threadIdx.x; i < NH * kr; i += NT) {
       const int hh = i / kr, e = i - hh * kr;
@@ -317,39 +361,12 @@ __device__ __forceinline__ void stage_queries(uint16_t* qs, int DP, const uint16
       qs[(size_t)hh * DP + e] = head < H ? q_lat[(size_t)head * ql_hs + (size_t)row * ql_ts + e] : (uint16_t)0;
     }
   }
-  // rotated part
-  constexpr int U = 4;
-  const int half = dims >> 1;
-  const float* cs = dims > 0 ? cos_sin + (size_t)max(pos, 0) * dims : nullptr;
-  for (int i0 = threadIdx.x; i0 < NH * rd; i0 += U * NT) {
-    uint16_t a[U], b[U];
-    float c[U], sn[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int i = min(i0 + u * NT, NH * rd - 1);
-      const int hh = i / rd, e = i - hh * rd;
-      const uint16_t* qr = q + (size_t)row * q_stride + (size_t)min(head0 + hh, H - 1) * (dim + rd) + dim;
-      int k = 0, partner = e;
-      if (e < dims) {
-        k = interleaved ? e >> 1 : e < half ? e : e - half;
-        partner = interleaved ? e ^ 1 : e < half ? e + half : e - half;
-      }
-      a[u] = qr[e];
-      b[u] = qr[partner];
-      c[u] = sn[u] = 0.f;
-      if (cs) {
-        c[u] = cs[k];
-        sn[u] = cs[half + k];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int i = min(i0 + u * NT, NH * rd - 1);
-      const int hh = i / rd, e = i - hh * rd;
-      const bool lead = interleaved ? !(e & 1) : e < half;                  // the pair's first element
-      const float x = bf16_to_f32(a[u]), y = bf16_to_f32(b[u]);
-      const uint16_t r = f32_to_bf16(lead ? x * c[u] - y * sn[u] : x * c[u] + y * sn[u]);
-      qs[(size_t)hh * DP + kr + e] = head0 + hh >= H ? (uint16_t)0 : e < dims ? r : a[u];
+  if constexpr (RD > 0) {
+    put_rot(threadIdx.x);
+  } else {
+    for (int i0 = threadIdx.x; i0 < NH * rd; i0 += U * NT) {
+      load_rot(i0);
+      put_rot(i0);
     }
   }
 }
@@ -397,7 +414,7 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
   const int pos = positions[row];
   const int first = window > 0 ? max(0, pos - window + 1) : 0;
 
-  stage_queries<16, 256, NM>(qs, DP, q, q_stride, q_lat, ql_hs, ql_ts, row, g * 16, H, dim, rd, kr, pos, cos_sin, dims, interleaved,
+  stage_queries<16, 256, NM, 0>(qs, DP, q, q_stride, q_lat, ql_hs, ql_ts, row, g * 16, H, dim, rd, kr, pos, cos_sin, dims, interleaved,
                              [] {});
   __syncthreads();
   const uint16_t* qp = qs + (size_t)lr * DP + 4 * lg;   // this lane's operand of Q^T: head lr, dims 16 s + 4 lg .. + 3
@@ -582,25 +599,24 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
 
 // ---------------------------------------------------------------------------------------------
 // Tile form (bf16; latents and keys of whole 128 bytes): what bounds a decode step over long contexts is reading every cached row once.
-// A workgroup owns one query row, 16 NG heads and one run of the row's 64-key tiles; the tiles go from memory to LDS
-// directly, two of them in turn, so that one (74 KB at 512 + 64 dims) is always under way while the other is computed, and
-// the heads share it: with NG = 2 a cached row is read once for 32 heads.  Wave (group of 16 heads, half of the tile):
+// A workgroup owns one query row, 16 NG heads and one run of the row's 32-key tiles; the tiles go from memory to LDS directly, four of them
+// in turn (37 KB each at 512 + 64 dims), two always under way, and the heads share them: with NG = 2 a cached row is read once for 32 heads.
+// A group of 16 heads has four waves:
 //
-//   S^T [32 keys x 16 heads] = K [32 keys x D] Q^T [D x 16 heads]      16x16x32 products, keys from LDS, queries in registers
-//   O^T [kr x 16 heads]     += C^T [kr x 32 keys] P^T [32 keys x 16 heads]      the same, C^T by transposing LDS reads
+//   S^T [16 keys x 16 heads] = K [16 keys x D / 2] Q^T [D / 2 x 16 heads]      each wave half the keys and half the dims; through LDS to all four
+//   O^T [kr / 4 x 16 heads] += C^T [kr / 4 x 32 keys] P^T [32 keys x 16 heads]      each wave a quarter of the latent dims, C^T by transposing LDS reads
 //
-// A lane of S^T holds keys 4 g .. + 3 and 16 + 4 g .. + 3 of one head: taken in that order they are its operand of P^T, so
-// nothing is exchanged, and a wave keeps its own running softmax.  P is taken in two bf16 parts, the rounded weights and what the rounding
-// took off: with one, results were further from 64 bits than the form above (32 heads, the layer's part: 60 rows over some 90 keys 3.04e-3
-// against 2.99e-3, 32 rows over 2000 keys 3.041e-3 and 3.034e-3), because fewer, larger groups of keys share a maximum; with two 2.80e-3 and
-// 2.88e-3, for 1.5 us a layer.  Chunk c (16 bytes) of a tile's row j lies at c ^ (j & 7):
-// neither kind of read meets a bank twice.  At the end the two waves of a group exchange halves of O^T through LDS.
-// Keys past the last are copies of it with weight 0.  The widths are constants of the kernel: with loop bounds read at run
-// time the compiler kept neither the products' order nor the operands in registers.
+// (16x16x32 products, keys from LDS, queries in registers).  The scores of a tile are formed behind the same barrier as the values of the one
+// before it.  A lane of S^T holds keys 4 g .. + 3 and 16 + 4 g .. + 3 of one head: taken in that order they are its operand of P^T; every wave
+// keeps the running softmax of all its group's keys.  P is taken in two bf16 parts, the rounded weights and what the rounding took off: with one,
+// results were further from 64 bits than the form above (32 heads, 32 rows over 2000 keys 3.041e-3 and 3.034e-3).  Chunk c (16 bytes) of a tile's
+// row j lies at c ^ (j & 7): neither kind of read meets a bank twice.  Keys past the last are copies of it with weight 0.  The widths are
+// constants of the kernel: with loop bounds read at run time the compiler kept neither the products' order nor the operands in registers.
 //
-// 32 rows x 32 heads over about 2000 keys each: 123 us (the form above, every row read for each 16 heads, C^T gathered in
-// single elements) -> 36, 2.1 TB/s; at four to five tiles a workgroup what is left is its first loads, one behind the
-// other (position, page, tile), and the partial sums' 17 MB.
+// 32 rows x 32 heads over about 2000 keys each: 123 us (the form above, every row read for each 16 heads, C^T gathered in single elements) ->
+// 28.8, 2.6 TB/s; over 4000 47, 4 TB/s while the longest runs last.  Four waves with tiles of 64 keys, a 32 x 16 block of scores each, took 35.4
+// and 57.6: one wave a SIMD issues too slowly; eight that each form all scores of their heads 33.3 and 56.3: 460 KB through LDS a tile, not 215.
+// What is left: some 14 us of first loads, one behind the other (position, page, tile), and of the partial sums' 17 MB.
 __device__ __forceinline__ void load_lds16(const char* src, char* lds) {
   __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
@@ -637,19 +653,24 @@ __device__ __forceinline__ void read_tr8(u32x2 (&v)[16], unsigned a0, unsigned a
 }
 
 template <int KR, int RD, int NG>
-__global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
+__global__ __launch_bounds__(256 * NG, NG) void latent_attn_tiles_kernel(
     const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ q_lat, long long ql_hs, long long ql_ts,
     const uint16_t* __restrict__ cache, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ cu_seqlens, int n_seqs, const int* __restrict__ positions, int H, int dim,
     int bs, float scale, int window, const float* __restrict__ cos_sin, int dims, int interleaved,
     uint16_t* __restrict__ out, long long o_hs, long long o_ts, float* __restrict__ part_o, float* __restrict__ part_ml,
     const float* __restrict__ sinks) {
-  constexpr int KT = 64, NW = 2 * NG, RPW = KT / NW;                     // keys per tile, waves, rows a wave loads
-  constexpr int D = KR + RD, NK = D / 32, NM = KR / 16, CPR = D / 8, row_bytes = 2 * D, stage = KT * row_bytes;
-  static_assert(KR % 128 == 0 && RD % 64 == 0 && RPW * CPR % 64 == 0, "tiles of whole 128-byte blocks, loads of whole waves");
-  extern __shared__ __attribute__((aligned(16))) char lds[];            // [2][KT][D] bf16
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int kw = w & 1, grp = w >> 1;
+  constexpr int KT = 32, ST = 4, NW = 4 * NG;                           // keys per tile, tiles in LDS, waves
+  constexpr int D = KR + RD, NK = D / 32, NM = KR / 16, NA = NM / 4, CPR = D / 8, row_bytes = 2 * D, stage = KT * row_bytes;
+  constexpr int SCORES = ST * stage, PAGES = SCORES + NG * 4096;        // [NG][4][64] f32x4, [NW][4][64] int
+  static_assert(16 * NG * (D + 8) * 2 <= stage + NG * 4096, "queries in the last tile's place and the scores'");
+  constexpr int LOADS = KT * CPR / 64, LP = LOADS / NW;                 // 64 chunks each; a wave's: LP, the first LOADS % NW waves' one more
+  static_assert(KR % 512 == 0 && RD % 64 == 0 && KT * CPR % 64 == 0, "whole 128-byte blocks, loads of whole waves");
+  constexpr int NH = NK / 2;                                            // steps of half the dims
+  static_assert(NH % 2 == 1, "a half's steps start at an odd one");
+  extern __shared__ __attribute__((aligned(16))) char lds[];            // [ST][KT][D] bf16
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int kq = w & 3, grp = w >> 2, u16 = kq & 1, part = kq >> 1;      // scores: 16 keys of a tile, half of the dims; values: a quarter of the dims
   const int lr = lane & 15, lg = lane >> 4;
   const int row = blockIdx.x, rows = gridDim.x, head0 = blockIdx.y * 16 * NG;
 
@@ -667,83 +688,126 @@ __global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
   const int first = window > 0 ? max(0, pos - window + 1) : 0;
   const int ntiles = (pos - first + KT) / KT;
   const int tps = (ntiles + (int)gridDim.z - 1) / (int)gridDim.z;
-  const int t_lo = blockIdx.z * tps, t_hi = min(ntiles, t_lo + tps);
+  const int t_lo = blockIdx.z * tps, count = min(ntiles, t_lo + tps) - t_lo;      // this run's tiles (none: 0 or less)
 
-  // loads of a tile: lane j knows the slot of its row j; load `it` of a wave brings chunks 64 it + lane of the wave's rows
-  auto key_of = [&](int ti) { return max(0, min(first + ti * KT + lane, pos)); };
-  auto issue = [&](int st, int slots) {
+  // Slots of a tile's rows, two tiles at a time: lane l has row l % 32 of tile l / 32 of the pair.  A pair's pages are looked up, straight to
+  // LDS, four tiles ahead, before loads that have been waited for when they are used: read to a register, the compiler would
+  // wait for everything under way.
+  auto key_of = [&](int pair) { return max(0, min(first + (t_lo + pair * 2) * KT + lane, pos)); };
+  char* const pages = lds + PAGES + w * 1024;          // [4][64]
+  auto look_up = [&](int pair) {
+    __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(bt + key_of(pair) / bs),
+                                     (__attribute__((address_space(3))) void*)(pages + (pair & 3) * 256), 4, 0, 0);
+  };
+  int slots = 0;
+  auto load = [&](int i) {                             // tiles in order, with the pair's slots
 #pragma unroll
-    for (int it = 0; it < RPW * CPR / 64; ++it) {
-      const int idx = 64 * it + lane, j = idx / CPR, c = idx - j * CPR;
-      const int sl = __shfl(slots, w * RPW + j, 64);
-      load_lds16(reinterpret_cast<const char*>(cache) + (long long)sl * row_bytes + (c ^ (j & 7)) * 16,        // RPW is a multiple of 8
-                 lds + st * stage + w * RPW * row_bytes + it * 1024);
+    for (int it = 0; it <= LP; ++it) {
+      if (it == LP && (LOADS % NW == 0 || w >= LOADS % NW)) break;
+      const int idx = 64 * (w + NW * it) + lane, j = idx / CPR, c = idx - j * CPR;
+      const int sl = __shfl(slots, (i & 1) * 32 + j, 64);
+      load_lds16(reinterpret_cast<const char*>(cache) + (long long)sl * row_bytes + (c ^ (j & 7)) * 16,
+                 lds + (i & (ST - 1)) * stage + (w + NW * it) * 1024);
     }
   };
-  int key = key_of(t_lo + 1), page = bt[key / bs];     // of the tile loaded next
-  const int key0 = key_of(t_lo), page0 = bt[key0 / bs];
+  auto issue = [&](int i) {
+    if ((i & 1) == 0) {
+      slots = reinterpret_cast<const int*>(pages + (i / 2 & 3) * 256)[lane] * bs + key_of(i / 2) % bs;
+      look_up(i / 2 + 2);
+    }
+    load(i);
+  };
+  const int page0 = bt[key_of(0) / bs], page1 = bt[key_of(1) / bs];
 
-  // queries through the second stage into registers: head lr of the group, dims 32 s + 8 lg .. + 7
-  bf16x8 qf[NK];
+  // queries through the last stage into registers: head lr of the group, this wave's half of the dims, 32 s + 8 lg .. + 7
+  bf16x8 qf[NH];
   {
     const int DP = D + 8;
-    uint16_t* qs = reinterpret_cast<uint16_t*>(lds + stage);
-    stage_queries<16 * NG, 128 * NG, NM>(qs, DP, q, q_stride, q_lat, ql_hs, ql_ts, row, head0, H, dim, RD, KR, pos, cos_sin, dims,
-                                         interleaved, [&] { if (t_lo < t_hi) issue(0, page0 * bs + key0 % bs); });
-    __syncthreads();
+    uint16_t* qs = reinterpret_cast<uint16_t*>(lds + (ST - 1) * stage);
+    stage_queries<16 * NG, 256 * NG, NM, RD>(qs, DP, q, q_stride, q_lat, ql_hs, ql_ts, row, head0, H, dim, RD, KR, pos, cos_sin, dims,
+                                         interleaved, [&] {
+                                           // also where the run has fewer (copies of its last row): the waits are counted
+                                           look_up(2);
+                                           look_up(3);
+                                           slots = count > 0 ? page0 * bs + key_of(0) % bs : 0;      // no keys, possibly no pages: any row that is there
+                                           load(0);
+                                           load(1);
+                                           slots = count > 0 ? page1 * bs + key_of(1) % bs : 0;
+                                           load(2);
+                                         });
+    // not __syncthreads(): that would wait for the tiles under way
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 #pragma unroll
-    for (int s = 0; s < NK; ++s)
-      qf[s] = *reinterpret_cast<const bf16x8*>(qs + (size_t)(grp * 16 + lr) * DP + 32 * s + 8 * lg);
+    for (int s = 0; s < NH; ++s)
+      qf[s] = *reinterpret_cast<const bf16x8*>(qs + (size_t)(grp * 16 + lr) * DP + 32 * (part * NH + s) + 8 * lg);
   }
 
-  float m_run = -__builtin_inff(), l_run = 0.f;        // of head lr, over this wave's keys
-  f32x4 acc[NM];                                       // O^T: latent dims 16 m + 4 lg + i of head lr
+  float m_run = -__builtin_inff(), l_run = 0.f;        // of head lr
+  f32x4 acc[NA];                                       // O^T: latent dims 16 (kq NA + m) + 4 lg + i of head lr
 #pragma unroll
-  for (int m = 0; m < NM; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int k0off = (32 * kw + lr) * row_bytes + (lg ^ (lr & 7)) * 16, k1off = (32 * kw + lr) * row_bytes + ((4 + lg) ^ (lr & 7)) * 16;
+  for (int m = 0; m < NA; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // steps of even and odd dims 32 s of the half: 64-byte halves of 128-byte blocks
+  const int klow = (lg ^ (lr & 7)) * 16, khigh = ((4 + lg) ^ (lr & 7)) * 16, krow = (16 * u16 + lr) * row_bytes + part * (NH / 2) * 128;
+  const int k0off = krow + (part ? khigh : klow), k1off = krow + (part ? klow + 128 : khigh);
+  // this wave's scores of a tile, keys 16 u16 + 4 lg + i of head lr, summed over its half of the dims; waves of the group read all four
+  f32x4* const scores = reinterpret_cast<f32x4*>(lds + SCORES) + grp * 256 + lane;
+  auto score = [&](int i) {
+    const char* tile = lds + (i & (ST - 1)) * stage;
+    f32x4 sp[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int s = 0; s < NH; ++s) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(tile + ((s & 1) ? k1off : k0off) + (s >> 1) * 128);
+      sp[s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[s], sp[s & 1], 0, 0, 0);
+    }
+    scores[kq * 64] = sp[0] + sp[1];
+  };
   const int tq = lr >> 2, tp = lr & 3;
   int voff[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    voff[i] = (32 * kw + 4 * lg + tq) * row_bytes + ((2 * i + (tp >> 1)) ^ ((4 * lg + tq) & 7)) * 16 + (tp & 1) * 8;
+    voff[i] = (4 * lg + tq) * row_bytes + ((2 * i + (tp >> 1)) ^ ((4 * lg + tq) & 7)) * 16 + (tp & 1) * 8 + kq * NA * 32;
 
-  int st = 0;
-  for (int ti = t_lo; ti < t_hi; ++ti, st ^= 1) {
-    // this wave's loads of tile ti have landed, and its reads of the other stage; behind the barrier everybody's
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  auto landed = [&](int later) {                       // this wave's loads but those of the `later` newest tiles
+    if (later == 2) {
+      if (LOADS % NW == 0 || w >= LOADS % NW) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * LP) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * LP + 2) : "memory");
+    } else if (later == 1) {
+      if (LOADS % NW == 0 || w >= LOADS % NW) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LP) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LP + 1) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const int slots = page * bs + key % bs;
-    key = key_of(ti + 2);
-    page = bt[key / bs];                               // not waited for before the next tile's turn
-    if (ti + 1 < t_hi) issue(st ^ 1, slots);
-    const int n = min(KT, pos - (first + ti * KT) + 1);
-    if (32 * kw >= n) continue;                        // none of this wave's keys exists (wave-uniform; no barrier follows)
-    const char* tile = lds + st * stage;
-    f32x4 sp[2][2];
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) sp[u][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s = 0; s < NK; ++s) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const bf16x8 a = *reinterpret_cast<const bf16x8*>(tile + ((s & 1) ? k1off : k0off) + u * 16 * row_bytes + (s >> 1) * 128);
-          sp[u][s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[s], sp[u][s & 1], 0, 0, 0);
-        }
-    }
-    // x[u][i]: key 32 kw + 16 u + 4 lg + i, head lr
+  };
+  if (count > 0) {
+    landed(2);                                         // the first three tiles are loaded in any case
+    score(0);
+  }
+  for (int ti = 0; ti < count; ++ti) {
+    // behind the barrier: the scores of tile ti, tile ti + 1 whole, and everybody's reads of the tile before
+    landed(ti + 2 < max(count, ST - 1) ? 1 : 0);
+    const f32x4 sp[2][2] = {{scores[0], scores[128]}, {scores[64], scores[192]}};
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // everybody has read them: the next tile's take their place
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (ti + ST - 1 < count) issue(ti + ST - 1);       // over the tile before
+    if (ti + 1 < count) score(ti + 1);
+    const int n = min(KT, pos - (first + (t_lo + ti) * KT) + 1);
+    const char* tile = lds + (ti & (ST - 1)) * stage;
+    // x[u][i]: key 16 u + 4 lg + i, head lr
     float x[2][4], mx = -__builtin_inff();
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        x[u][i] = (32 * kw + 16 * u + 4 * lg + i < n) ? (sp[u][0][i] + sp[u][1][i]) * scale : -__builtin_inff();
+        x[u][i] = (16 * u + 4 * lg + i < n) ? (sp[u][0][i] + sp[u][1][i]) * scale : -__builtin_inff();
         mx = fmaxf(mx, x[u][i]);
       }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));            // key 32 kw exists: finite
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));            // the tile's first key exists: finite
     const float m_new = fmaxf(m_run, mx);
     const float corr = expf(m_run - m_new);            // first tile: exp(-inf) = 0
     float sum = 0.f;
@@ -773,13 +837,13 @@ __global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
       }
     if (__any(corr != 1.f)) {                          // else no head's maximum moved: the sums keep their scale
 #pragma unroll
-      for (int m = 0; m < NM; ++m)
+      for (int m = 0; m < NA; ++m)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[m][i] *= corr;
     }
     const unsigned tl = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)tile;
 #pragma unroll
-    for (int m = 0; m < NM; m += 8) {
+    for (int m = 0; m < NA; m += 8) {
       u32x2 v[16];
       read_tr8<row_bytes>(v, tl + voff[0] + m * 32, tl + voff[1] + m * 32, tl + voff[2] + m * 32, tl + voff[3] + m * 32);
 #pragma unroll
@@ -791,55 +855,29 @@ __global__ __launch_bounds__(128 * NG, 1) void latent_attn_tiles_kernel(
     }
   }
 
-  // the two waves of a group: (max, sum) of every head, then each gives the other half of its O^T and keeps the rest
-  __syncthreads();                                     // the last tile is fully read
-  float* ml = reinterpret_cast<float*>(lds);           // [NW][16][2]
-  f32x4* ex = reinterpret_cast<f32x4*>(lds + NW * 128);      // [NW][NM / 2][64]
-  if (lg == 0) {
-    ml[(w * 16 + lr) * 2] = m_run;
-    ml[(w * 16 + lr) * 2 + 1] = l_run;
-  }
-#pragma unroll
-  for (int mm = 0; mm < NM / 2; ++mm) {                // wave 0 of a group keeps the first half, wave 1 the second
-    const f32x4 lo = acc[mm], hi = acc[mm + NM / 2];
-    ex[(w * (NM / 2) + mm) * 64 + lane] = kw ? lo : hi;
-    acc[mm] = kw ? hi : lo;
-  }
-  __syncthreads();
-  const float m2 = ml[((w ^ 1) * 16 + lr) * 2], l2 = ml[((w ^ 1) * 16 + lr) * 2 + 1];
-  const float M = fmaxf(m_run, m2);
-  const float f1 = m_run == -__builtin_inff() ? 0.f : expf(m_run - M);   // a wave (or a whole run) without keys adds nothing
-  const float f2 = m2 == -__builtin_inff() ? 0.f : expf(m2 - M);
-  const float L = l_run * f1 + l2 * f2;
   const int head = head0 + grp * 16 + lr;
   if (head >= H) return;
   const size_t slot = ((size_t)blockIdx.z * H + head) * rows + row;
-  if (part_o && kw == 0 && lg == 0) {
-    part_ml[2 * slot] = M;
-    part_ml[2 * slot + 1] = L;
+  if (part_o && kq == 0 && lg == 0) {                  // a run without keys: -inf, 0 and zeros
+    part_ml[2 * slot] = m_run;
+    part_ml[2 * slot + 1] = l_run;
   }
-  const float inv = part_o ? 1.f : sinks ? inv_with_sink(M, L, sinks[head]) : inv_sum(L);
+  const float inv = part_o ? 1.f : sinks ? inv_with_sink(m_run, l_run, sinks[head]) : inv_sum(l_run);
   uint16_t* op = out + (size_t)head * o_hs + (size_t)row * o_ts;
   const bool ovec = ((uintptr_t)out & 7) == 0 && (o_hs & 3) == 0 && (o_ts & 3) == 0;
-  auto kept = [&](auto put) {                          // put(latent dim, its four sums) for the half this wave keeps
 #pragma unroll
-    for (int mm = 0; mm < NM / 2; ++mm) {
-      const f32x4 y = ex[((w ^ 1) * (NM / 2) + mm) * 64 + lane];
-      float v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (acc[mm][i] * f1 + y[i] * f2) * inv;
-      put(16 * (kw * (NM / 2) + mm) + 4 * lg, v);
-    }
-  };
-  if (part_o)
-    kept([&](int e, const float* v) { *reinterpret_cast<float4*>(part_o + slot * KR + e) = make_float4(v[0], v[1], v[2], v[3]); });
-  else if (ovec)
-    kept([&](int e, const float* v) { *reinterpret_cast<uint2*>(op + e) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])); });
-  else
-    kept([&](int e, const float* v) {
+  for (int m = 0; m < NA; ++m) {
+    const int e = 16 * (kq * NA + m) + 4 * lg;
+    const float v[4] = {acc[m][0] * inv, acc[m][1] * inv, acc[m][2] * inv, acc[m][3] * inv};
+    if (part_o) {
+      *reinterpret_cast<float4*>(part_o + slot * KR + e) = make_float4(v[0], v[1], v[2], v[3]);
+    } else if (ovec) {
+      *reinterpret_cast<uint2*>(op + e) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+    } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) op[e + i] = f32_to_bf16(v[i]);
-    });
+    }
+  }
 }
 
 template <typename K>
@@ -927,16 +965,15 @@ int launch_tiles(const void* q, int q_stride, const void* q_lat, long long ql_hs
                  int interleaved, void* out, long long o_hs, long long o_ts, int nsplit, float* part_o, float* part_ml,
                  const float* sinks, hipStream_t s) {
   constexpr int D = KR + RD;
-  // two tiles; the queries (rows of D + 8) fit in the second, the exchange at the end takes the place of both
-  constexpr size_t lds = std::max(2 * 64 * D * 2, 2 * NG * (128 + KR / 32 * 64 * 16));
-  static_assert(16 * NG * (D + 8) <= 64 * D, "queries in one stage");
+  // four tiles (the queries, rows of D + 8, take the last one's place and a little more), scores, pages: all there is
+  constexpr size_t lds = 4 * 32 * D * 2 + NG * 8192;
   if (lds > lds_max()) return -6;
   static int allowed = -1;
   if (allowed != 0 && lds > 64 * 1024) {
     allowed = allow_lds(latent_attn_tiles_kernel<KR, RD, NG>, lds_max());
     if (allowed != 0) return allowed;
   }
-  latent_attn_tiles_kernel<KR, RD, NG><<<dim3(rows, (H + 16 * NG - 1) / (16 * NG), nsplit), 128 * NG, lds, s>>>(
+  latent_attn_tiles_kernel<KR, RD, NG><<<dim3(rows, (H + 16 * NG - 1) / (16 * NG), nsplit), 256 * NG, lds, s>>>(
       (const uint16_t*)q, q_stride, (const uint16_t*)q_lat, ql_hs, ql_ts, (const uint16_t*)cache, block_tables, bt_stride,
       cu_seqlens, n_seqs, positions, H, dim, bs, scale, window, cos_sin, dims, interleaved, (uint16_t*)out, o_hs, o_ts,
       nsplit > 1 ? part_o : nullptr, part_ml, sinks);

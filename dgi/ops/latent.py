@@ -197,7 +197,7 @@ def split_runs(rows: int, heads: int, max_keys: int) -> int:
 def tile_runs(rows: int, heads: int, max_keys: int) -> int:
     """Runs of keys per row for the tile kernel (512 + 64 dims): its workgroups take a row, up to 32 heads and one run, one
     to a compute unit (two tiles are most of its LDS), so as many as fill the 256 of them, every run at least two 64-key tiles
-    long.  32 rows of 32 heads over 2000 keys: 8 runs 36 us and 8 to combine them."""
+    long.  32 rows of 32 heads over 2000 keys: 8 runs 29 us and 8 to combine them."""
     if max_keys <= 0 or rows <= 0:
         return 1
     return int(max(1, min(64, 256 // (rows * ((heads + 31) // 32)), max_keys // 128)))
@@ -258,7 +258,7 @@ def latent_decode_heads(q, uk, uv, cache, block_tables, positions, rot_dim: int,
     """Head outputs ``out`` [T, H * vdim] of decode rows on cached latents (``decode_heads_ok``): ``q`` [T, H * (dim + rot_dim)], the key
     and value up-projections ``uk`` [H, dim, 512] and ``uv`` [H, vdim, 512], the rest as ``latent_attn_rows`` and ``gate_heads``.  Three
     launches: queries folded, attention in runs of keys, and one that combines the runs, takes the sums to values and applies
-    the gate.  32 rows of 32 heads, 8 runs: 4.5 and 10.8 us around the attention's 36; the library's products, the combining pass
+    the gate.  32 rows of 32 heads, 8 runs: 4.5 and 10.5 us around the attention's 29; the library's products, the combining pass
     and the one that puts the heads side by side took 28."""
     _native(q)
     T, (H, dim, kr) = q.shape[0], uk.shape

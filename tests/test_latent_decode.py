@@ -121,3 +121,35 @@ def test_rows_without_a_position(gated, max_keys):
                                torch.tensor([-1, 300, -70], dtype=I32, device=dev), RD, 0.1, 0, torch.randn(320, RD, generator=g).to(dev),
                                True, out, max_keys, None, gate, True)
     assert (out[[0, 2]] == 0).all() and torch.isfinite(out).all() and (out[1] != 0).any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [4, 32])
+def test_contexts_around_the_tiles(H):
+    """Contexts around tiles of 32 keys and what is loaded ahead of them, runs without keys, and rows without a position whose pages are
+    nobody's, against the same rows one by one in a single run."""
+    g = torch.Generator().manual_seed(H)
+    pos = [0, 14, 30, 31, 32, 62, 63, 64, 95, 96, 127, 128, 300, -1, 2049]
+    T, dim, vdim, dev = len(pos), 64, 32, "cuda"
+    cols = 2100 // BS + 1
+    cache = torch.randn(cols, 1, BS, KR + RD, generator=g).to(BF16).to(dev)
+    tables = torch.stack([torch.randperm(cols, generator=g) if p >= 0 else torch.full((cols,), 1 << 30) for p in pos]).to(I32).to(dev)
+    q = torch.randn(T, H * (dim + RD), generator=g).to(BF16).to(dev)
+    uk, uv = ((torch.randn(H, n, KR, generator=g) * KR ** -0.5).to(BF16).to(dev) for n in (dim, vdim))
+    cs = torch.randn(2100, RD, generator=g).to(dev)
+    positions = torch.tensor(pos, dtype=I32, device=dev)
+
+    def run(rows, max_keys):
+        out = torch.full((len(rows), H * vdim), 7.0, dtype=BF16, device=dev)
+        latent.latent_decode_heads(q[rows].contiguous(), uk, uv, cache, tables[rows].contiguous(), positions[rows].contiguous(), RD, 0.08, 0, cs,
+                                   True, out, max_keys, None, None, False)
+        return out.float()
+
+    many = run(list(range(T)), 1 << 14)
+    for i, p in enumerate(pos):
+        if p < 0:
+            assert (many[i] == 0).all()
+            continue
+        one = run([i], 0)[0]
+        # weights relative to another maximum, sums and the head's value rounded to bf16
+        assert (many[i] - one).abs().max() <= 2.0 ** -7 * one.abs().max()
