@@ -66,12 +66,15 @@ __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__
 }
 
 // A workgroup owns a head and rb rows: 16, fewer where the step has few rows, so that 256 workgroups share the partial sums
-// (32 rows of 32 heads, 8 runs: 64 workgroups that also read the runs' maxima one by one took 15.7 us, 256 so 10.8); its eight waves take 64 of the 512 latent dims each (operands straight from
+// (32 rows of 32 heads, 8 runs: 64 workgroups that also read the runs' maxima one by one took 15.7 us, 256 so 10.5), and more than eight
+// runs are shared out over the lanes that have no row of their own (8 rows of 32 runs 20.6 us -> 11.0, 1 row of 31 runs 15.4 -> 10.4; 8 runs 10.5,
+// so 11.2); its eight waves take 64 of the 512 latent dims each (operands straight from
 // memory), and their sums meet in LDS.  runs > 1: o comes as the partial sums of that many runs of keys (at most 64),
 // [runs, H, T, 512] relative to each run's maximum (ml: maximum and sum of weights), else as o_lat [H, T, 512].  The loads of
 // the weights and of the first four runs are under way while the runs' factors are formed.
-constexpr int KR = 512, VMAX = 8, RUNS = 64;
+constexpr int KR = 512, VMAX = 8, RUNS = 64, SHARE = 8;
 
+template <bool SHARED>
 __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ o_lat,
                                                             const float* __restrict__ part, const float* __restrict__ ml, int runs,
                                                             const float* __restrict__ sinks, const uint16_t* __restrict__ uv,
@@ -80,7 +83,9 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
   __shared__ __attribute__((aligned(16))) float sums[8][VMAX][64][4];
   const int head = blockIdx.x, t0 = blockIdx.y * rb, t1 = min(t0 + rb, T);
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
-  const int t = min(t0 + lr, t1 - 1), nv = vdim >> 4, k = w * 64 + 8 * lg;
+  // SHARED: lanes past the rows take part of the runs, lane lr row lr % rb and every (16 / rb)-th run
+  const int r = SHARED ? lr & (rb - 1) : lr, grp = SHARED ? lr / rb : 0, ng = SHARED ? 16 / rb : 1;
+  const int t = min(t0 + r, t1 - 1), nv = vdim >> 4, k = w * 64 + 8 * lg;
   u32x4 a[VMAX][2];
   auto load_uv = [&]() {
 #pragma unroll
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
     auto load_runs = [&](int z0) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const float* src = part + (first + (size_t)min(z0 + u, runs - 1) * next) * KR + k;
+        const float* src = part + (first + (size_t)min(z0 + u * ng + grp, runs - 1) * next) * KR + k;
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -123,8 +128,12 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
     }
     __syncthreads();
     float M = -FLT_MAX, L = 0.f;                           // of this lane's row; finite also where no run has keys
-    for (int z = 0; z < runs; ++z) M = fmaxf(M, fac[z][lr]);
-    for (int z = 0; z < runs; ++z) L += len[z * 16 + lr] * expf(fac[z][lr] - M);
+    for (int z = grp; z < runs; z += ng) M = fmaxf(M, fac[z][r]);
+    if constexpr (SHARED)
+      for (int o = rb; o < 16; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+    for (int z = grp; z < runs; z += ng) L += len[z * 16 + r] * expf(fac[z][r] - M);
+    if constexpr (SHARED)
+      for (int o = rb; o < 16; o <<= 1) L += __shfl_xor(L, o, 64);
     float inv = L == 0.f ? 0.f : 1.f / L;
     if (sinks) {                                           // one more logit in the denominator, relative to the larger of the two
       const float sink = sinks[head], top = fmaxf(M, sink), f = expf(M - top);
@@ -135,10 +144,11 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[s][i] = 0.f;
-    for (int z0 = 0; z0 < runs; z0 += 4) {
+    for (int z0 = 0; z0 < runs; z0 += 4 * ng) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const float f = z0 + u < runs ? expf(fac[min(z0 + u, runs - 1)][lr] - M) : 0.f;
+        const int z = z0 + u * ng + grp;
+        const float f = z < runs ? expf(fac[min(z, runs - 1)][r] - M) : 0.f;
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -147,8 +157,14 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
             x[s][4 * i + 2] += p[u][s][i].z * f; x[s][4 * i + 3] += p[u][s][i].w * f;
           }
       }
-      if (z0 + 4 < runs) load_runs(z0 + 4);
+      if (z0 + 4 * ng < runs) load_runs(z0 + 4 * ng);
     }
+    if constexpr (SHARED)
+      for (int o = rb; o < 16; o <<= 1)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[s][i] += __shfl_xor(x[s][i], o, 64);
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
@@ -217,11 +233,11 @@ extern "C" int dgi_latent_values(void* out, const void* o_lat, const float* part
   if (H <= 0 || vdim % 16 || vdim < 16 || vdim > 16 * VMAX || runs < 1 || runs > RUNS || (runs > 1 ? !part || !ml : !o_lat)) return -2;
   if ((((uintptr_t)uv | (uintptr_t)o_lat | (uintptr_t)part) & 15) || ((uintptr_t)out & 7) || ((uintptr_t)ml & 7)) return -3;
   int rb = 16;
-  while (rb > 4 && (long long)H * ((T + rb - 1) / rb) < 256) rb >>= 1;       // fewer rows each while compute units are left over
+  while (rb > 1 && ((long long)H * ((T + rb - 1) / rb) < 256 || rb / 2 >= T)) rb >>= 1;       // fewer rows each while compute units are left over
   if ((T + rb - 1) / rb > 65535) return -4;
-  latent_values_kernel<<<dim3(H, (T + rb - 1) / rb), 512, 0, s>>>((uint16_t*)out, (const uint16_t*)o_lat, part, ml, runs, sinks,
-                                                              (const uint16_t*)uv, (const uint16_t*)gate, gate_stride, per_head, T, H,
-                                                              vdim, rb);
+  auto kernel = runs > SHARE && rb < 16 ? latent_values_kernel<true> : latent_values_kernel<false>;
+  kernel<<<dim3(H, (T + rb - 1) / rb), 512, 0, s>>>((uint16_t*)out, (const uint16_t*)o_lat, part, ml, runs, sinks, (const uint16_t*)uv,
+                                                    (const uint16_t*)gate, gate_stride, per_head, T, H, vdim, rb);
   DGI_CHECK_LAUNCH();
   return 0;
 }
