@@ -82,13 +82,22 @@ __global__ __launch_bounds__(COLS * NL) void ssm_scan_kernel(
   float* sp = state + (((size_t)seq_slots[seq] * heads + h) * dv + v) * N;     // [..][head][v][n]
   const bool fresh = positions[r0] == 0;
   float S[NQ][4];
+  const bool vec = (N & 3) == 0 && ((uintptr_t)state & 15) == 0;
 #pragma unroll
-  for (int q = 0; q < NQ; ++q)
+  for (int q = 0; q < NQ; ++q) {
+    const int n = 4 * l + 64 * q;
+    if (vec) {
+      // read and written once a step, and the other layers' come in between: marked so, the chip's caches give it up first, and whole
+      // quads are one access (four layers, 64 x 128: 32 rows of 64 heads 189 us -> 122, 4.4 TB/s; of 16 heads 64 -> 40; 4 rows 39 -> 25)
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+      if (!fresh && vok && n < N) s = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(sp + n));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = 4 * l + 64 * q + j;
-      S[q][j] = (!fresh && vok && n < N) ? sp[n] : 0.f;
+      for (int j = 0; j < 4; ++j) S[q][j] = s[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) S[q][j] = (!fresh && vok && n + j < N) ? sp[n + j] : 0.f;
     }
+  }
   const float na = -expf(a_log[h]), bias = dt_bias[h], dsk = d_skip[h];
 
   float rb[PB], rc[PB], rx = 0.f, rdt = 0.f;
@@ -146,12 +155,16 @@ __global__ __launch_bounds__(COLS * NL) void ssm_scan_kernel(
   }
   if (vok) {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q)
+    for (int q = 0; q < NQ; ++q) {
+      const int n = 4 * l + 64 * q;
+      if (vec) {
+        if (n < N) __builtin_nontemporal_store(f32x4{S[q][0], S[q][1], S[q][2], S[q][3]}, reinterpret_cast<f32x4*>(sp + n));
+      } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int n = 4 * l + 64 * q + j;
-        if (n < N) sp[n] = S[q][j];
+        for (int j = 0; j < 4; ++j)
+          if (n + j < N) sp[n + j] = S[q][j];
       }
+    }
   }
 }
 
