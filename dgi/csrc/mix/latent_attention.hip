@@ -617,8 +617,10 @@ __global__ __launch_bounds__(256) void latent_attn_mfma_kernel(
 // 28.8, 2.6 TB/s; over 4000 47, 4 TB/s while the longest runs last.  Four waves with tiles of 64 keys, a 32 x 16 block of scores each, took 35.4
 // and 57.6: one wave a SIMD issues too slowly; eight that each form all scores of their heads 33.3 and 56.3: 460 KB through LDS a tile, not 215.
 // What is left: some 14 us of first loads, one behind the other (position, page, tile), and of the partial sums' 17 MB.
+// ONCE: nothing reads it again soon (nt), the chip's caches give it up first
+template <bool ONCE>
 __device__ __forceinline__ void load_lds16(const char* src, char* lds) {
-  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, ONCE ? 2 : 0);
 }
 
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -652,7 +654,7 @@ __device__ __forceinline__ void read_tr8(u32x2 (&v)[16], unsigned a0, unsigned a
       : "memory");
 }
 
-template <int KR, int RD, int NG>
+template <int KR, int RD, int NG, bool ONCE>
 __global__ __launch_bounds__(256 * NG, NG) void latent_attn_tiles_kernel(
     const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ q_lat, long long ql_hs, long long ql_ts,
     const uint16_t* __restrict__ cache, const int* __restrict__ block_tables, int bt_stride,
@@ -706,7 +708,7 @@ __global__ __launch_bounds__(256 * NG, NG) void latent_attn_tiles_kernel(
       if (it == LP && (LOADS % NW == 0 || w >= LOADS % NW)) break;
       const int idx = 64 * (w + NW * it) + lane, j = idx / CPR, c = idx - j * CPR;
       const int sl = __shfl(slots, (i & 1) * 32 + j, 64);
-      load_lds16(reinterpret_cast<const char*>(cache) + (long long)sl * row_bytes + (c ^ (j & 7)) * 16,
+      load_lds16<ONCE>(reinterpret_cast<const char*>(cache) + (long long)sl * row_bytes + (c ^ (j & 7)) * 16,
                  lds + (i & (ST - 1)) * stage + (w + NW * it) * 1024);
     }
   };
@@ -968,12 +970,17 @@ int launch_tiles(const void* q, int q_stride, const void* q_lat, long long ql_hs
   // four tiles (the queries, rows of D + 8, take the last one's place and a little more), scores, pages: all there is
   constexpr size_t lds = 4 * 32 * D * 2 + NG * 8192;
   if (lds > lds_max()) return -6;
-  static int allowed = -1;
-  if (allowed != 0 && lds > 64 * 1024) {
-    allowed = allow_lds(latent_attn_tiles_kernel<KR, RD, NG>, lds_max());
-    if (allowed != 0) return allowed;
+  // a step that fills the chip marks the cached rows as read once (32 rows of 32 heads over 2000 keys, the layer 44.6 us -> 43.6; 2 rows
+  // over 500 26.1, marked 26.5), unless other groups of heads read them too
+  const dim3 grid(rows, (H + 16 * NG - 1) / (16 * NG), nsplit);
+  const bool once = grid.y == 1 && (long long)rows * nsplit >= 256;
+  auto kernel = once ? latent_attn_tiles_kernel<KR, RD, NG, true> : latent_attn_tiles_kernel<KR, RD, NG, false>;
+  static int allowed[2] = {-1, -1};
+  if (allowed[once] != 0 && lds > 64 * 1024) {
+    allowed[once] = allow_lds(kernel, lds_max());
+    if (allowed[once] != 0) return allowed[once];
   }
-  latent_attn_tiles_kernel<KR, RD, NG><<<dim3(rows, (H + 16 * NG - 1) / (16 * NG), nsplit), 256 * NG, lds, s>>>(
+  kernel<<<grid, 256 * NG, lds, s>>>(
       (const uint16_t*)q, q_stride, (const uint16_t*)q_lat, ql_hs, ql_ts, (const uint16_t*)cache, block_tables, bt_stride,
       cu_seqlens, n_seqs, positions, H, dim, bs, scale, window, cos_sin, dims, interleaved, (uint16_t*)out, o_hs, o_ts,
       nsplit > 1 ? part_o : nullptr, part_ml, sinks);

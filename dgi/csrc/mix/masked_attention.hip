@@ -446,7 +446,7 @@ __global__ __launch_bounds__(64 * GNW) void masked_attn_group_kernel(
 // The grouped kernel for bf16 heads of up to 128 dims.  Bounded by the cached rows' bytes, so what counts is how many of them are
 // under way: a wave holds one tile of 64 keys in flight all the time.  The keys' registers are loaded again with the tile's values
 // as the products consume them, those again with the next tile's keys as the values are summed, and the pages of the next tile are
-// looked up a tile ahead.  32 rows of 1500 to 2500 keys, 8 groups of 4 heads of 128 dims, cap, sinks and gate: 56 us (the kernel above with
+// looked up a tile ahead.  32 rows of 1500 to 2500 keys, 8 groups of 4 heads of 128 dims, cap, sinks and gate: 54.4 us (the kernel above with
 // 16 lanes per key on the vector ALUs, each batch of rows waited for: 68), 4.7 TB/s in all, 5.8 while the longest row is read; 100 rows of
 // 600 keys, at most 1024 in a block: 87 -> 57; 1 row of 7000 keys of 64 dims in 13 runs: 31 -> 20.  Scores are matrix products (16 keys by up to 16 heads, products of bf16 numbers exact, sums in fp32);
 // they change to one key per lane through LDS for the softmax, whose weights and the values' sums stay in fp32 on the vector ALUs.
@@ -467,6 +467,12 @@ __device__ __forceinline__ float wave_max_all(float v) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
+template <bool ONCE>
+__device__ __forceinline__ u32x4 cached_row(const uint16_t* p) {
+  if constexpr (ONCE) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  return *reinterpret_cast<const u32x4*>(p);
+}
+
 struct RowsArgs {
   const uint16_t *q, *k, *v, *gate;
   uint16_t* out;
@@ -477,8 +483,9 @@ struct RowsArgs {
   float scale, softcap;
 };
 
-// R: heads of a group, rounded up to 2, 4 or 8; D: dims, rounded up to 64 or 128
-template <int R, int D, int NW>
+// R: heads of a group, rounded up to 2, 4 or 8; D: dims, rounded up to 64 or 128; ONCE: cached rows are marked as what nothing reads again
+// soon, so that the chip's caches give them up first
+template <int R, int D, int NW, bool ONCE>
 __global__ __launch_bounds__(64 * NW, R == 8 ? 2 : 3) void masked_attn_tiles_kernel(const RowsArgs a) {
   constexpr int KS = D / 32;                         // loads (and products) of a block of 16 keys
   constexpr int LK = D / 8, KL = 64 / LK;            // lanes of a value row, rows of a load
@@ -554,12 +561,12 @@ __global__ __launch_bounds__(64 * NW, R == 8 ? 2 : 3) void masked_attn_tiles_ker
   auto load_k = [&](const int* sl, int u) {          // keys 16 u ..
     const uint16_t* p = a.k + (size_t)sl[16 * u + n16] * dk;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) raw[u][s] = *reinterpret_cast<const u32x4*>(p + ck[s]);
+    for (int s = 0; s < KS; ++s) raw[u][s] = cached_row<ONCE>(p + ck[s]);
   };
   auto load_v = [&](const int* sl, int u) {
 #pragma unroll
     for (int x = 0; x < VB; ++x)
-      raw[u][x] = *reinterpret_cast<const u32x4*>(a.v + (size_t)sl[16 * u + KL * x + lg] * dv + cv);
+      raw[u][x] = cached_row<ONCE>(a.v + (size_t)sl[16 * u + KL * x + lg] * dv + cv);
   };
   auto add_v = [&](int u) {
 #pragma unroll
@@ -728,9 +735,14 @@ __global__ __launch_bounds__(128) void masked_attn_reduce_kernel(const float* __
 template <int R, int D>
 void launch_tiles_dims(const RowsArgs& a, int rows, int G, int nsplit, hipStream_t s) {
   // a workgroup per compute unit or fewer: eight waves each (30 rows of 2000 keys, 8 groups of 4 heads of 64 dims: 14.9 us, with four
-  // waves 16.8); more of them: four, so that more workgroups share a unit (128 rows of 500 keys, groups of 2: 30.4, with eight 30.9)
-  if ((long long)rows * G * nsplit <= 256) masked_attn_tiles_kernel<R, D, 8><<<dim3(rows, G, nsplit), 512, 0, s>>>(a);
-  else masked_attn_tiles_kernel<R, D, 4><<<dim3(rows, G, nsplit), 256, 0, s>>>(a);
+  // waves 16.8); more of them: four, so that more workgroups share a unit (128 rows of 500 keys, groups of 2: 30.4, with eight 30.9).
+  // From 256 on cached rows are marked as read once (32 rows of 2000 keys 56 us -> 54.4, 128 of 500 59 -> 55.5); smaller steps, whose
+  // rows the caches may still hold, gain nothing (4 rows of 300 keys 12.2, marked 12.7)
+  const long long units = (long long)rows * G * nsplit;
+  const dim3 grid(rows, G, nsplit);
+  if (units > 256) masked_attn_tiles_kernel<R, D, 4, true><<<grid, 256, 0, s>>>(a);
+  else if (units == 256) masked_attn_tiles_kernel<R, D, 8, true><<<grid, 512, 0, s>>>(a);
+  else masked_attn_tiles_kernel<R, D, 8, false><<<grid, 512, 0, s>>>(a);
 }
 
 template <int R>
