@@ -349,18 +349,38 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
   }
   __syncthreads();
   if (!s_last) return;
+  // the splits' sums first, all of a head's in LDS, then the partial results, SB of them under way at a time
+  constexpr int SB = 16;
+  float* lse = reinterpret_cast<float*>(smem);          // [G][nsplit]
+  const bool staged = G * nsplit * 4 <= NW * WREG;
+  if (staged) {
+    for (int idx = tid; idx < G * nsplit; idx += NT)
+      lse[idx] = part_lse[((size_t)b * nh + h * G + idx / nsplit) * max_splits + idx % nsplit];
+    __syncthreads();
+  }
   for (int idx = tid; idx < G * HD; idx += NT) {
     const int qq = idx / HD;
     const int d = idx - qq * HD;
     const int head = h * G + qq;
     const size_t base = ((size_t)b * nh + head) * max_splits;
+    const float* l = staged ? lse + qq * nsplit : part_lse + base;
+    float v[SB];
+    auto load = [&](int s0) {
+#pragma unroll
+      for (int i = 0; i < SB; ++i) v[i] = part_o[(base + min(s0 + i, nsplit - 1)) * HD + d];
+    };
+    load(0);
     float M = -1e30f;
-    for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, part_lse[base + sp]);
+    for (int sp = 0; sp < nsplit; ++sp) M = fmaxf(M, l[sp]);
     float W = 0.f, acc = 0.f;
-    for (int sp = 0; sp < nsplit; ++sp) {
-      const float wgt = exp2f(part_lse[base + sp] - M);
-      W += wgt;
-      acc += wgt * part_o[(base + sp) * HD + d];
+    for (int s0 = 0; s0 < nsplit; s0 += SB) {
+#pragma unroll
+      for (int i = 0; i < SB; ++i) {
+        const float wgt = s0 + i < nsplit ? exp2f(l[min(s0 + i, nsplit - 1)] - M) : 0.f;
+        W += wgt;
+        acc += wgt * v[i];
+      }
+      if (s0 + SB < nsplit) load(s0 + SB);
     }
     out[(size_t)b * out_stride + head * HD + d] = f32_to_bf16(acc / W);
   }
@@ -420,6 +440,9 @@ extern "C" int dgi_paged_decode(const void* q, int q_stride, const void* k_cache
   // 12.9 us, with four 15.3); more of them: four, so that several share a unit, and rows marked as read once (64 rows of 1024: 50.6,
   // with eight 52.6; without the mark 53.4)
   const bool wide = (long long)B * nkv * max_splits <= 256;
+  // there the last workgroup of a (sequence, kv head) combines its splits (1 row of 600 tokens 8.3 us, with a reduce kernel 9.1, of 8000
+  // in 32 splits 16.0 and 19.3); among more workgroups than that the last arriver's work is the tail of the launch
+  if (!wide) counters = nullptr;
   auto launch = [&](auto HD_, auto NW_, auto P16_) {
     constexpr int HD = decltype(HD_)::value, NW = decltype(NW_)::value;
     paged_decode_kernel<HD, NW, decltype(P16_)::value><<<grid, 64 * NW, NW * decode_wave_lds<HD>(), s>>>(

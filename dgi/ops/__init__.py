@@ -248,8 +248,9 @@ def decode_split_plan(batch: int, max_ctx: int, nkv: int, num_cus: int = 256) ->
 
     One workgroup of eight waves per CU: more splits cost more than they bring (8 kv heads of 128 dims, us a layer with the
     reduce kernel: 8 rows of 4000 tokens in 2 / 4 / 8 / 16 splits 43.7 / 29.7 / 31.4 / 35.1, 1 row of 8000 in 16 / 32 / 64
-    18.5 / 19.0 / 27.7).  Rows that fill the chip by themselves are not split (64 rows of 1024 in 1 / 2 splits 50.6 / 52.6,
-    of 300 17.6 / 24.1) but past 2048 tokens, so that a few long ones do not hold up the step."""
+    18.5 / 19.0 / 27.7; combined in the kernel 1 row of 8000 in 32 16.0).  Rows that fill the chip by themselves are not split
+    (64 rows of 1024 in 1 / 2 splits 50.6 / 52.6, of 300 17.6 / 24.1) but past 2048 tokens, so that a few long ones do not
+    hold up the step."""
     seqs = max(1, batch * nkv)
     splits, part = (8, 2048) if 2 * seqs > num_cus else (num_cus // seqs, 128)
     return max(1, min(splits, -(-max_ctx // part))), -part

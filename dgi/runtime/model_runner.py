@@ -130,14 +130,11 @@ class ModelRunner:
         self.dec_ws = None
         if self.is_cuda:
             # partial O / log-sum-exp per split + one ticket counter per (sequence, kv-head) for the
-            # in-kernel split reduce (write-through partials, one acquire on the last arriver; round 3's
-            # form fenced every workgroup, which wrote back L2 and cost more than a reduce kernel).
-            # Opt-in (DGI_DECODE_FUSED_REDUCE=1): 8B TPOT ties the reduce kernel at batch 1-4 and
-            # loses 0.09-0.23 ms at batch 16-64, where the last arriver's serial combine is the
-            # tail of the launch (profiles/r4_decode/README.md)
+            # in-kernel split reduce of steps of up to a workgroup per CU (write-through partials, one
+            # acquire on the last arriver); DGI_DECODE_FUSED_REDUCE=0: a reduce kernel always
             self.dec_ws = (torch.empty(maxb * nh * self.ws_splits * hd, dtype=torch.float32, device=self.device),
                            torch.empty(maxb * nh * self.ws_splits, dtype=torch.float32, device=self.device))
-            if os.environ.get("DGI_DECODE_FUSED_REDUCE", "0") == "1":
+            if os.environ.get("DGI_DECODE_FUSED_REDUCE", "1") == "1":
                 self.dec_ws += (torch.zeros(maxb * model.cfg.num_kv_heads, dtype=torch.int32, device=self.device),)
         # called while the host waits for a step's sampled tokens (P/D ranks keep
         # their KV handshakes moving instead of blocking in a stream synchronize)
@@ -404,10 +401,10 @@ class GraphRunner:
         self.max_bucket = self.buckets[-1] if self.buckets else 0
         self.graphs: dict[int, torch.cuda.CUDAGraph] = {}
         # small buckets also get a one-split variant (8-wave workgroups walk each
-        # sequence's whole context: no partials, no reduce kernel) replayed when
-        # every context is short (DGI_DECODE_SHORT_CTX tokens, 0 = off; the one-split plan wins up to
-        # ~700 tokens, the split plan from ~1k: profiles/r4_decode/attn8b_p16_1.jsonl)
-        self.short_ctx = int(os.environ.get("DGI_DECODE_SHORT_CTX", "640"))
+        # sequence's whole context: no partials, no reduce) replayed when
+        # every context is short (DGI_DECODE_SHORT_CTX tokens, 0 = off).  8 kv heads of 128 dims, us a layer, one split against
+        # the plan's: 1 row of 150 tokens 5.4, 7.6, of 600 9.2, 8.3; 2 of 400 8.8, 8.4; 4 of 100 5.2, 5.4, of 500 11.3, 9.2
+        self.short_ctx = int(os.environ.get("DGI_DECODE_SHORT_CTX", "384"))
         self.short_max_b = int(os.environ.get("DGI_DECODE_SHORT_B", "8"))
         self.short_graphs: dict[int, torch.cuda.CUDAGraph] = {}
         self._short = False
