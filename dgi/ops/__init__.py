@@ -525,6 +525,18 @@ def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:
     return None
 
 
+def tile_gemm_rows(N: int, K: int) -> int:
+    """Rows past 128 up to which ``linear`` runs on the ping-pong kernel (``mfma_gemm``): the logits of large vocabularies, whose 384 tiles of
+    columns or more come in a few whole rounds of the chip, and products of long rows, which it splits along K.  Vendor's product
+    and this one, us, at 129 / 256 / 353 / 512 / 1024 rows: 128256 x 4096 289, 224 / 299, 235 / 433, 398 / 510, 402 / 860, 766; x 8192
+    527, 465 / 541, 451 / 813, 765 / 975, 786 / 1710, 1471; 8192 x 28672 309, 173 / 323, 195 / 197, 195 / 310, 201 / 384, 330 (but
+    640: 264, 310).  Narrower ones are the vendor's: 32000 x 4096 64, 80 / 74, 85 / 88, 101; 4096 x 14336 57, 97; 57344 x 8192
+    192, 204 / 218, 220 / 313, 363."""
+    if N >= 384 * 256:
+        return 1024
+    return 512 if K >= 16384 and N * K >= 1 << 27 else 0
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
            out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = x @ w.T (+ bias) for a 2-D activation; [N, K] weights as stored."""
@@ -543,6 +555,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
         y = _linear_stream(x, w, bias, out)
         if y is not None:
             return y
+    if 128 < M <= tile_gemm_rows(N, K) and bias is None and out is None and mfma_gemm_ok(x, w) and load_native(False):
+        return mfma_gemm(x, w)
     r = torch.nn.functional.linear(x, w, bias)
     if out is not None:
         out.copy_(r)
