@@ -85,3 +85,22 @@ def test_pairs_sorted_by_the_product(T, top, E, tile):
             made.append((order, where, seg, out))
         for a, b in zip(*made):
             assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("skip", [0, 1])
+@pytest.mark.parametrize("P,E", [(1, 1), (3, 5), (4, 2), (1023, 16), (1024, 16), (1025, 3), (4096, 64), (4097, 65), (8190, 16), (20000, 130)])
+def test_plan_of_many_pairs(P, E, skip):
+    """The places of the pairs by expert in their order, identity routes left out, also from an index at no 16-byte boundary."""
+    from dgi.ops import _call
+    idx = torch.randint(-1, E + 1, (P + skip,), generator=torch.Generator().manual_seed(P), dtype=torch.int32).cuda()[skip:]
+    order, where, seg = (torch.full((n,), -7, dtype=torch.int32, device="cuda") for n in (P, P, E + 1))
+    _call("moe_plan", order, where, seg, idx)
+    i = idx.cpu().long()
+    pairs = torch.nonzero((i >= 0) & (i < E))[:, 0]
+    pairs = pairs[torch.argsort(i[pairs], stable=True)]
+    counts = torch.bincount(i[pairs], minlength=E)
+    assert seg.tolist() == [0] + counts.cumsum(0).tolist()
+    n = pairs.numel()
+    assert torch.equal(order[:n].cpu().long(), pairs) and (order[n:] == -7).all()
+    assert torch.equal(where.cpu().long()[pairs], torch.arange(n))
