@@ -12,6 +12,7 @@
 
 extern "C" {
 int dgi_rmsnorm(void* out, const void* x, const void* w, int T, int H, float eps, hipStream_t s);
+int dgi_row_sumsq(float* out, int ldo, int cols, const void* x, long long ldx, int T, int H, hipStream_t s);
 int dgi_fused_add_rmsnorm(void* x, void* residual, const void* w, int T, int H, float eps,
                           hipStream_t s);
 int dgi_rope_cache(void* qkv, int T, int qkv_stride, const int* positions, const float* cos_sin,
@@ -106,6 +107,14 @@ void rmsnorm(at::Tensor out, const at::Tensor& x, const at::Tensor& w, double ep
   TORCH_CHECK(w.numel() == H && out.numel() == x.numel());
   check_rc(dgi_rmsnorm(out.data_ptr(), x.data_ptr(), w.data_ptr(), (int)(x.numel() / H), H,
                        (float)eps, cur_stream()), "rmsnorm");
+}
+
+void row_sumsq(at::Tensor out, const at::Tensor& x) {
+  check_bf16(x, "x"); check_dev(out, "out");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && out.scalar_type() == at::kFloat && out.dim() == 2 && out.stride(1) == 1 &&
+                  out.size(0) == x.size(0) && out.size(1) >= 1 && x.size(1) < (1 << 30) && out.device() == x.device(), "row_sumsq: rows");
+  check_rc(dgi_row_sumsq(out.data_ptr<float>(), (int)out.stride(0), (int)out.size(1), x.data_ptr(), x.stride(0), (int)x.size(0),
+                         (int)x.size(1), cur_stream()), "row_sumsq");
 }
 
 void fused_add_rmsnorm(at::Tensor x, at::Tensor residual, const at::Tensor& w, double eps) {
@@ -673,6 +682,7 @@ TORCH_LIBRARY(dgi, m) {
   m.def("paged_prefill(Tensor(a!) out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, "
         "Tensor cu_seqlens_q, Tensor context_lens, Tensor tiles, int nh, int nkv, float scale, "
         "Tensor? tree_mask, int tree_n, int tile_rows=128) -> ()");
+  m.def("row_sumsq(Tensor(a!) out, Tensor x) -> ()");
   m.def("silu_mul(Tensor(a!) out, Tensor gu) -> ()");
   m.def("stream_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int mode) -> ()");
   m.def("add_rmsnorm_parts(Tensor(a!) out, Tensor parts, Tensor(b!) residual, Tensor w, float eps) -> ()");
@@ -711,6 +721,7 @@ TORCH_LIBRARY_IMPL(dgi, CUDA, m) {
   m.impl("rope_cache", &rope_cache);
   m.impl("paged_decode", &paged_decode);
   m.impl("paged_prefill", &paged_prefill);
+  m.impl("row_sumsq", &row_sumsq);
   m.impl("silu_mul", &silu_mul);
   m.impl("stream_gemm", &stream_gemm);
   m.impl("add_rmsnorm_parts", &add_rmsnorm_parts);
