@@ -497,6 +497,14 @@ class LlamaModel:
                 self.layer_hook(self.layer_start + i)
         return ops.sum_parts(parts), residual
 
+    @staticmethod
+    def _last_mlp(h: torch.Tensor, L: LlamaLayerWeights) -> torch.Tensor:
+        """gate_up, SwiGLU and down of the rows that logits are asked for."""
+        act = ops.silu_mul(ops.linear(h, L.gate_up))
+        if ops.split_gemm(act.shape[0], *L.down.shape) and ops.mfma_gemm_ok(act, L.down):
+            return ops.mfma_gemm(act, L.down)
+        return ops.linear(act, L.down)
+
     # ------------------------------------------------------------------ fused-norm layers
     def _fold_ok(self, h: torch.Tensor) -> bool:
         if NORM_FOLD == "0" or self.reduce is not None:
@@ -568,7 +576,7 @@ class LlamaModel:
                 Rs = R.index_select(0, trim_last)
                 ho = ops.linear(attn, L.o)
                 ops.fused_add_rmsnorm(ho, Rs, L.post_norm, eps)
-                out = ops.linear(ops.silu_mul(ops.linear(ho, L.gate_up)), L.down)
+                out = self._last_mlp(ho, L)
                 if self.layer_hook is not None:
                     self.layer_hook(self.layer_start + i)
                 return out, Rs
@@ -731,7 +739,7 @@ class LlamaModel:
                 if self.reduce is not None:
                     self.reduce(h)
                 ops.fused_add_rmsnorm(h, residual, L.post_norm, eps)
-                h = ops.linear(ops.silu_mul(ops.linear(h, L.gate_up)), L.down)
+                h = self._last_mlp(h, L)
                 if self.reduce is not None:
                     self.reduce(h)
                 if self.layer_hook is not None:

@@ -525,16 +525,21 @@ def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:
     return None
 
 
-def tile_gemm_rows(N: int, K: int) -> int:
-    """Rows past 128 up to which ``linear`` runs on the ping-pong kernel (``mfma_gemm``): the logits of large vocabularies, whose 384 tiles of
-    columns or more come in a few whole rounds of the chip, and products of long rows, which it splits along K.  Vendor's product
+def tile_gemm(M: int, N: int) -> bool:
+    """Whether ``linear`` runs on the ping-pong kernel (``mfma_gemm``, whole tiles: its split-K workspace belongs to one stream at a
+    time): the logits of large vocabularies for 129 to 1024 rows, where the tiles nearly fill whole rounds of the chip.  Vendor's product
     and this one, us, at 129 / 256 / 353 / 512 / 1024 rows: 128256 x 4096 289, 224 / 299, 235 / 433, 398 / 510, 402 / 860, 766; x 8192
-    527, 465 / 541, 451 / 813, 765 / 975, 786 / 1710, 1471; 8192 x 28672 309, 173 / 323, 195 / 197, 195 / 310, 201 / 384, 330 (but
-    640: 264, 310).  Narrower ones are the vendor's: 32000 x 4096 64, 80 / 74, 85 / 88, 101; 4096 x 14336 57, 97; 57344 x 8192
-    192, 204 / 218, 220 / 313, 363."""
-    if N >= 384 * 256:
-        return 1024
-    return 512 if K >= 16384 and N * K >= 1 << 27 else 0
+    527, 465 / 541, 451 / 813, 765 / 975, 786 / 1710, 1471.  Narrower ones are the vendor's: 32000 x 4096 64, 80 / 74, 85 / 88,
+    101; 57344 x 8192 192, 204 / 218, 220 / 313, 363."""
+    tiles = -(-M // 256) * (N // 256)
+    return 128 < M <= 1024 and N >= 384 * 256 and 8 * tiles >= 7 * -(-tiles // 256) * 256
+
+
+def split_gemm(M: int, N: int, K: int) -> bool:
+    """Whether a product of long rows, 129 to 512 of them, is better split along K by ``mfma_gemm`` (8192 x 28672, vendor's product and
+    this one, us: 129 rows 309, 173; 200 311, 185; 256 323, 195; 353 197, 195; 512 310, 201; but 640 264, 310; 4096 x 14336 at
+    200 60, 98).  For callers that issue such products on one stream at a time: they share a workspace per device."""
+    return 128 < M <= 512 and K >= 16384 and N * K >= 1 << 27
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -555,8 +560,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
         y = _linear_stream(x, w, bias, out)
         if y is not None:
             return y
-    if 128 < M <= tile_gemm_rows(N, K) and bias is None and out is None and mfma_gemm_ok(x, w) and load_native(False):
-        return mfma_gemm(x, w)
+    if tile_gemm(M, N) and bias is None and out is None and mfma_gemm_ok(x, w) and load_native(False):
+        return mfma_gemm(x, w, streamk=1)
     r = torch.nn.functional.linear(x, w, bias)
     if out is not None:
         out.copy_(r)

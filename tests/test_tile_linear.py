@@ -1,5 +1,5 @@
-"""``ops.linear`` past 128 rows where it runs on the ping-pong kernel: the logits of large vocabularies and products of long rows, around the
-rows and sizes at which the rule changes, against the product in fp32."""
+"""Products past 128 rows that run on the ping-pong kernel: the logits of large vocabularies (``ops.linear``) and products of long rows, around
+the rows and sizes at which the rules change, against the product in fp32."""
 import pytest
 import torch
 
@@ -8,7 +8,7 @@ from dgi import ops
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [129, 255, 256, 257, 353, 512, 513, 1024, 1025])
-@pytest.mark.parametrize("N,K", [(384 * 256, 128), (384 * 256 - 256, 128), (501 * 256, 192), (384 * 256 + 8, 64), (8192, 16384), (8192, 16448)])
+@pytest.mark.parametrize("N,K", [(384 * 256, 128), (384 * 256 - 256, 128), (501 * 256, 192), (384 * 256 + 8, 64), (448 * 256, 64), (8192, 16384)])
 def test_linear_past_the_streamed_rows(M, N, K):
     g = torch.Generator(device="cuda")
     g.manual_seed(M + N)
@@ -21,7 +21,19 @@ def test_linear_past_the_streamed_rows(M, N, K):
     assert ((y - ref).norm() / ref.norm()) <= 2.0 ** -8
 
 
-def test_rows_of_the_rule():
-    assert [ops.tile_gemm_rows(n, k) for n, k in [(128256, 4096), (128256, 8192), (384 * 256, 64), (384 * 256 - 8, 64), (32000, 4096),
-                                                  (8192, 28672), (4096, 14336), (8192, 16384), (8192, 16383), (57344, 8192)]] == \
-        [1024, 1024, 1024, 0, 0, 512, 0, 512, 0, 0]
+def test_rows_of_the_rules():
+    assert [ops.tile_gemm(m, 128256) for m in (128, 129, 256, 257, 512, 1024, 1025)] == [False, True, True, True, True, True, False]
+    assert [ops.tile_gemm(200, n) for n in (32000, 384 * 256 - 256, 384 * 256, 448 * 256, 512 * 256, 594 * 256)] == [False, False, False, True, True, False]
+    assert [ops.split_gemm(m, 8192, 28672) for m in (128, 129, 512, 513)] == [False, True, True, False]
+    assert [ops.split_gemm(200, n, k) for n, k in [(4096, 14336), (8192, 16384), (8192, 16383), (4096, 16384)]] == [False, True, False, False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [129, 300, 512])
+def test_split_product(M):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    x = torch.randn(M, 16448, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(8192, 16448, device="cuda", generator=g) * 16448 ** -0.5).bfloat16()
+    ref = x.float() @ w.float().t()
+    assert ((ops.mfma_gemm(x, w).float() - ref).norm() / ref.norm()) <= 2.0 ** -8
