@@ -556,12 +556,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _call("skinny_gemm", out, x, w, bias, _skinny_cfg(M, N))
         return out
-    if x.is_cuda and x.shape[0] <= STREAM_MAX_M:
-        y = _linear_stream(x, w, bias, out)
-        if y is not None:
-            return y
-    if tile_gemm(M, N) and bias is None and out is None and mfma_gemm_ok(x, w) and load_native(False):
-        return mfma_gemm(x, w, streamk=1)
+    if x.is_cuda and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):      # these kernels have no derivatives
+        if M <= STREAM_MAX_M:
+            y = _linear_stream(x, w, bias, out)
+            if y is not None:
+                return y
+        if tile_gemm(M, N) and bias is None and out is None and mfma_gemm_ok(x, w) and load_native(False):
+            return mfma_gemm(x, w, streamk=1)
     r = torch.nn.functional.linear(x, w, bias)
     if out is not None:
         out.copy_(r)

@@ -37,3 +37,17 @@ def test_split_product(M):
     w = (torch.randn(8192, 16448, device="cuda", generator=g) * 16448 ** -0.5).bfloat16()
     ref = x.float() @ w.float().t()
     assert ((ops.mfma_gemm(x, w).float() - ref).norm() / ref.norm()) <= 2.0 ** -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [64, 200])
+def test_linear_keeps_its_derivatives(M):
+    """Rows that want a gradient stay with the differentiable product, whatever its size."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    x = torch.randn(M, 64, device="cuda", generator=g).bfloat16().requires_grad_()
+    w = torch.randn(501 * 256, 64, device="cuda", generator=g).bfloat16()
+    up = torch.randn(M, 501 * 256, device="cuda", generator=g).bfloat16()
+    ops.linear(x, w).backward(up)
+    ref = up.float() @ w.float()
+    assert ((x.grad.float() - ref).norm() / ref.norm()) <= 2.0 ** -7
