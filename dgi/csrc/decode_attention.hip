@@ -1,4 +1,4 @@
-// dgi/csrc/decode_attention.hip — paged GQA decode attention, split-KV (SURVEY K7).
+// dgi/csrc/decode_attention.hip — paged GQA decode attention, split-KV.
 //
 // The reference decodes through HF `model.generate` with a dense per-request
 // cache (worker/engines/llm.py:61-69) and its shard path drops the KV
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_kernel(
     }
   }
   if (nsplit == 1 || counters == nullptr) return;
-  // ---- fused split reduce (MI355X_MICROARCH "Valid forms"): every wave drains its sc1 stores,
+  // ---- fused split reduce: every wave drains its sc1 stores,
   // the workgroup meets at a barrier, one lane takes a relaxed agent-scope ticket; the workgroup
   // that draws nsplit - 1 acquires once (invalidates its CU's L1) and combines every split in
   // split order (deterministic).  No workgroup waits for another: placement-independent.

@@ -1,4 +1,4 @@
-// dgi/csrc/rmsnorm.hip — RMSNorm and fused residual-add + RMSNorm (SURVEY K2/K10).
+// dgi/csrc/rmsnorm.hip — RMSNorm and fused residual-add + RMSNorm.
 //
 // Replaces the RMSNorm modules that the reference executes inside HF Llama
 // layers (worker/distributed/model_shard.py:209-226).  One 256-thread
