@@ -18,6 +18,7 @@ from typing import Optional
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 _LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "_C.so")
 _loaded = False
@@ -504,25 +505,43 @@ def rope_cache_parts(parts, bias, positions, cos_sin, nh, nkv, hd, slot_mapping,
     return qkv[:, : nh * hd]
 
 
+def plain_values(*tensors) -> bool:
+    """Whether only the operands' values are wanted, so that a kernel without derivatives, batching and meta rules may take them: nothing
+    records history or carries tangents through them, none is a transform's or a trace's stand-in, and no dispatch mode looks on."""
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack():
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is None:
+            continue
+        if ((grad and t.requires_grad) or type(t) not in (torch.Tensor, torch.nn.Parameter)
+                or torch._C._functorch.is_functorch_wrapped_tensor(t) or forward_ad.unpack_dual(t).tangent is not None):
+            return False
+    return True
+
+
+def _stream_sizes(M: int, N: int, K: int) -> bool:
+    """Where ``linear`` is the faster as a streaming product: outputs that fill the chip by themselves up to 96 rows, narrow and large
+    weights (96 MB; the sum over the parts is a launch of its own) up to 128."""
+    return M <= STREAM_MAX_M and (M <= 96 if N >= 160 * 128 else N * K >= 48 << 20)
+
+
 def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:
-    """``linear`` as a streaming product where that is the faster: outputs that fill the chip by themselves up to 96 rows, narrow and
-    large weights (96 MB; the sum over the parts is a launch of its own) up to 128."""
+    """``linear`` as a streaming product (``_stream_sizes``); None for operands that it does not take."""
     N, K = w.shape
     if not stream_ok(x, w) or (bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_contiguous() or bias.data_ptr() % 16)):
         return None
     if not load_native(False):
         return None
-    if N >= 160 * 128 and x.shape[0] <= 96:
+    if N >= 160 * 128:
         if out is None:
             out = torch.empty(x.shape[0], N, dtype=x.dtype, device=x.device)
         elif out.dim() != 2 or out.stride(1) != 1 or out.stride(0) % 4 or out.data_ptr() % 8 or out.dtype != x.dtype:
             return None
         _call("stream_gemm", out, x, w, bias, 0)
         return out
-    if N < 160 * 128 and N * K >= 48 << 20:
-        y = sum_parts(stream_parts(x, w), bias)
-        return y if out is None else out.copy_(y)
-    return None
+    y = sum_parts(stream_parts(x, w), bias)
+    return y if out is None else out.copy_(y)
 
 
 def tile_gemm(M: int, N: int) -> bool:
@@ -550,14 +569,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     M, K = x.shape
     N = w.shape[0]
     if (x.is_cuda and _use_skinny(M, N, K) and x.dtype == torch.bfloat16
-            and w.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w.is_contiguous()
-            and load_native(False)):     # a process that built only another kernel group keeps the vendor GEMM
+            and w.dtype == torch.bfloat16 and plain_values(x, w, bias, out) and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and load_native(False)):     # a process that built only another kernel group keeps the vendor GEMM
         if out is None:
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _call("skinny_gemm", out, x, w, bias, _skinny_cfg(M, N))
         return out
-    if x.is_cuda and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):      # these kernels have no derivatives
-        if M <= STREAM_MAX_M:
+    if x.is_cuda and M <= 1024 and (_stream_sizes(M, N, K) or tile_gemm(M, N)) and plain_values(x, w, bias, out):
+        if _stream_sizes(M, N, K):
             y = _linear_stream(x, w, bias, out)
             if y is not None:
                 return y

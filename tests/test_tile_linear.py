@@ -51,3 +51,54 @@ def test_linear_keeps_its_derivatives(M):
     ops.linear(x, w).backward(up)
     ref = up.float() @ w.float()
     assert ((x.grad.float() - ref).norm() / ref.norm()) <= 2.0 ** -7
+
+
+def test_what_is_plain():
+    """Operands of a transform, of a trace or with history are not for kernels that know values alone."""
+    from torch._subclasses import FakeTensorMode
+    from torch.autograd import forward_ad
+    seen = []
+    look = lambda t: (seen.append(ops.plain_values(t)), t * 2)[1]  # noqa: E731
+    x, p = torch.randn(3, 4), torch.nn.Parameter(torch.randn(3, 4))
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    torch.func.grad(lambda t: look(t).sum())(x)
+    with FakeTensorMode() as mode:
+        look(torch.empty(3, 4))
+    look(mode.from_tensor(x))
+    with forward_ad.dual_level():
+        look(forward_ad.make_dual(x, x))
+        assert ops.plain_values(x)
+    look(p)
+    look(x * p)
+    assert seen == [False] * 8
+    with torch.no_grad():
+        assert ops.plain_values(x, None, p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(8, 4096, 1024), (64, 20480, 64), (128, 4096, 12288), (200, 501 * 256, 64)])
+@pytest.mark.parametrize("of", ["x", "w", "bias"])
+def test_linear_keeps_every_derivative(M, N, K, of):
+    """Backward and forward derivatives of each operand alone, at the sizes of each kernel, and operands without data."""
+    from torch._subclasses import FakeTensorMode
+    from torch.autograd import forward_ad
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    a = {"x": rnd(M, K), "w": rnd(N, K) * K ** -0.5, "bias": rnd(N) if M <= 128 else None}
+    if a[of] is None:
+        pytest.skip("no bias at this size")
+    up, tan = rnd(M, N), rnd(*a[of].shape)
+    f = {k: None if v is None else v.float() for k, v in a.items()}
+    want = {"x": up.float() @ f["w"], "w": up.float().t() @ f["x"], "bias": up.float().sum(0)}[of]
+    leaf = a[of].clone().requires_grad_()
+    ops.linear(**{**a, of: leaf}).backward(up)
+    # sums in fp32, rounded to bf16 on both ways
+    assert ((leaf.grad.float() - want).norm() / want.norm()) <= 2.0 ** -7
+    want = {"x": lambda t: t @ f["w"].t(), "w": lambda t: f["x"] @ t.t(), "bias": lambda t: t.expand(M, N)}[of](tan.float())
+    with forward_ad.dual_level():
+        got = forward_ad.unpack_dual(ops.linear(**{**a, of: forward_ad.make_dual(a[of], tan)})).tangent
+        assert ((got.float() - want).norm() / want.norm()) <= 2.0 ** -7
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        assert ops.linear(**{**a, of: mode.from_tensor(a[of])}).shape == (M, N)
