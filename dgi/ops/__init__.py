@@ -527,21 +527,24 @@ def _stream_sizes(M: int, N: int, K: int) -> bool:
 
 
 def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:
-    """``linear`` as a streaming product (``_stream_sizes``); None for operands that it does not take."""
-    N, K = w.shape
-    if not stream_ok(x, w) or (bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_contiguous() or bias.data_ptr() % 16)):
+    """``linear`` as a streaming product (``_stream_sizes``); None for operands that it does not take.  ``out`` gets the rows as they are
+    where it lies as they do and apart from what is still read, else a copy."""
+    if not stream_ok(x, w) or w.device != x.device or not load_native(False):
         return None
-    if not load_native(False):
+    N = w.shape[0]
+    if bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (N,) or not bias.is_contiguous() or bias.data_ptr() % 16
+                             or bias.device != x.device):
         return None
-    if N >= 160 * 128:
-        if out is None:
-            out = torch.empty(x.shape[0], N, dtype=x.dtype, device=x.device)
-        elif out.dim() != 2 or out.stride(1) != 1 or out.stride(0) % 4 or out.data_ptr() % 8 or out.dtype != x.dtype:
-            return None
-        _call("stream_gemm", out, x, w, bias, 0)
-        return out
-    y = sum_parts(stream_parts(x, w), bias)
-    return y if out is None else out.copy_(y)
+    if N < 160 * 128:
+        y = sum_parts(stream_parts(x, w), bias)
+    else:
+        y = out
+        if (out is None or out.shape != (x.shape[0], N) or out.dtype != x.dtype or out.device != x.device or out.stride(1) != 1
+                or out.stride(0) % 4 or out.stride(0) < N or out.data_ptr() % 8
+                or any(t is not None and t.untyped_storage().data_ptr() == out.untyped_storage().data_ptr() for t in (x, w, bias))):
+            y = torch.empty(x.shape[0], N, dtype=x.dtype, device=x.device)
+        _call("stream_gemm", y, x, w, bias, 0)
+    return y if out is None or y is out else out.copy_(y)
 
 
 def tile_gemm(M: int, N: int) -> bool:
@@ -580,7 +583,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
             y = _linear_stream(x, w, bias, out)
             if y is not None:
                 return y
-        if tile_gemm(M, N) and bias is None and out is None and mfma_gemm_ok(x, w) and load_native(False):
+        if (tile_gemm(M, N) and bias is None and out is None and w.dim() == 2 and w.shape[1] == K and w.device == x.device
+                and w.data_ptr() % 16 == 0 and mfma_gemm_ok(x, w) and load_native(False)):
             return mfma_gemm(x, w, streamk=1)
     r = torch.nn.functional.linear(x, w, bias)
     if out is not None:

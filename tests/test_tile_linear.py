@@ -102,3 +102,40 @@ def test_linear_keeps_every_derivative(M, N, K, of):
         assert ((got.float() - want).norm() / want.norm()) <= 2.0 ** -7
     with FakeTensorMode(allow_non_fake_inputs=True) as mode:
         assert ops.linear(**{**a, of: mode.from_tensor(a[of])}).shape == (M, N)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(64, 20480, 64), (20, 4096, 12288), (20, 20480, 20480), (200, 501 * 256, 64)])
+def test_linear_takes_what_the_plain_product_takes(M, N, K):
+    """Biases and results of other shapes, types and places, results over the operands, weights off their 16 bytes and of one row."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    x, flat = rnd(M, K), rnd(N * K + 1) * K ** -0.5
+    w = flat[:-1].view(N, K)
+    y = x.float() @ w.float().t()
+
+    def check(got, want):
+        # one rounding to bf16; sums of K products in fp32, in another order
+        assert got.shape == want.shape and ((got.float() - want).norm() / want.norm()) <= 2.0 ** -8
+
+    for bias in (rnd(1), rnd(M, N), rnd(1, N)):
+        check(ops.linear(x, w, bias), y + bias.float())
+    for out in (torch.empty(M, N, device="cuda"), torch.empty(M, N, dtype=torch.bfloat16), torch.empty(2, M, N, device="cuda"),
+                torch.empty(N, M, device="cuda").bfloat16().t(), rnd(M, N + 4)[:, :N]):
+        assert ops.linear(x, w, out=out) is out
+        check(out.cuda(), y.expand_as(out))
+    if N == K:
+        both = x.clone()
+        assert ops.linear(both, w, out=both) is both
+        check(both, y)
+        del both
+        one = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        check(ops.linear(x[:1].expand(M, K), w, out=one), y[:1].expand(M, N))
+    off = flat[1:].view(N, K)
+    check(ops.linear(x, off), x.float() @ off.float().t())
+    check(ops.linear(x, w[0]), x.float() @ w[0].float())
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w.new_zeros(N, K + 64))
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w, out=torch.empty(M + 1, N, device="cuda").bfloat16())
