@@ -882,8 +882,9 @@ def row_sumsq(x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """out[:, 0] = sum of squares of each row of x (fp32), the other columns zero: the
     statistics the fused-norm GEMM reads for a stream no residual epilogue produced (the
     first layer's input)."""
-    if (x.dtype == torch.bfloat16 and x.shape == (out.shape[0], x.shape[1]) and x.shape[1] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and out.dtype == torch.float32 and out.stride(1) == 1 and _native(x)):
+    if (x.is_cuda and x.dtype == torch.bfloat16 and out.dtype == torch.float32 and out.device == x.device and out.dim() == 2
+            and x.shape == (out.shape[0], x.shape[1]) and plain_values(x, out) and x.shape[1] % 8 == 0 and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and out.stride(1) == 1 and load_native(False)):
         _call("row_sumsq", out, x)
         return out
     out.zero_()

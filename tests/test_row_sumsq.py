@@ -16,3 +16,14 @@ def test_row_sumsq(T, H, pad, cols):
     # a tree over the row: well under 64 roundings of 2^-24
     assert ((out[:, 0].cpu().double() - ref).abs() <= 64 * 2.0 ** -24 * ref).all()
     assert (out[:, 1:cols] == 0).all() and (out[:, cols:] == 7.0).all()
+
+
+@pytest.mark.gpu
+def test_history_and_other_places():
+    """Rows that want a gradient keep it; statistics may lie elsewhere."""
+    x = torch.randn(5, 64, generator=torch.Generator().manual_seed(2)).bfloat16().cuda()
+    leaf = x.clone().requires_grad_()
+    ops.row_sumsq(leaf, torch.empty(5, 3, device="cuda"))[:, 0].sum().backward()
+    assert torch.equal(leaf.grad, (2 * x.float()).bfloat16())
+    out = ops.row_sumsq(x, torch.empty(5, 3))
+    assert out.device.type == "cpu" and torch.allclose(out[:, 0], x.float().pow(2).sum(-1).cpu(), rtol=1e-5) and not out[:, 1:].any()
