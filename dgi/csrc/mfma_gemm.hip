@@ -36,6 +36,8 @@
 // on load and skipped on store.
 #include "common.h"
 
+#include <atomic>
+#include <mutex>
 #include <type_traits>
 
 using namespace dgi;
@@ -1196,53 +1198,66 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
              });
 }
 
+// Compute units of the current device that persistent launches use (a multiple of the 8 XCDs), 0 if unknown.
+int gemm_units() {
+  static std::atomic<int> units[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int n = units[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 8) return 0;
+    units[dev].store(n &= ~7, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 // Per-device split-K workspace (one fp32 slab per block + two counters per tile),
 // allocated on first use outside stream capture.  Shared by every stream of
 // the process: the engine issues its projection GEMMs on one stream at a time.
 struct SkWorkspace {
   float* ws = nullptr;
   int* cnt = nullptr;   // 2 P counters, preceded by the error word cnt[-1] (timed-out waits)
-  int P = 0;
 };
 
+std::mutex g_sk_mutex;
 SkWorkspace g_sk_per_dev[64];
 
-SkWorkspace* sk_peek(int dev) { return g_sk_per_dev[dev].ws ? &g_sk_per_dev[dev] : nullptr; }
+SkWorkspace sk_peek(int dev) {
+  std::lock_guard<std::mutex> lock(g_sk_mutex);
+  return g_sk_per_dev[dev];
+}
 
-SkWorkspace* sk_workspace(hipStream_t s) {
+SkWorkspace sk_workspace(int P, hipStream_t s) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return {};
+  std::lock_guard<std::mutex> lock(g_sk_mutex);
   SkWorkspace& w = g_sk_per_dev[dev];
-  if (w.ws) return &w;
+  if (w.ws) return w;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return nullptr;
-  int cus = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8) return nullptr;
-  const int P = cus & ~7;
+  if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return {};
   float* ws = nullptr;
   int* cnt = nullptr;
-  if (hipMalloc(&ws, (size_t)P * 65536 * sizeof(float)) != hipSuccess) return nullptr;
+  if (hipMalloc(&ws, (size_t)P * 65536 * sizeof(float)) != hipSuccess) return {};
   if (hipMalloc(&cnt, (size_t)(2 * P + 1) * sizeof(int)) != hipSuccess ||
-      hipMemset(cnt, 0, (size_t)(2 * P + 1) * sizeof(int)) != hipSuccess) {
+      hipMemset(cnt, 0, (size_t)(2 * P + 1) * sizeof(int)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     hipFree(ws);
-    return nullptr;
+    return {};
   }
   w.ws = ws;
   w.cnt = cnt + 1;
-  w.P = P;
-  return &w;
+  return w;
 }
 
 // Split-K waits of this device that ran out since the last reset (0 unless a counter broke).
 int sk_timeouts(bool reset) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return -1;
-  SkWorkspace* w = sk_peek(dev);
-  if (!w) return 0;
+  const SkWorkspace w = sk_peek(dev);
+  if (!w.ws) return 0;
   int v = 0;
-  if (hipDeviceSynchronize() != hipSuccess || hipMemcpy(&v, w->cnt - 1, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
+  if (hipDeviceSynchronize() != hipSuccess || hipMemcpy(&v, w.cnt - 1, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
     return -1;
-  if (reset && v && hipMemset(w->cnt - 1, 0, sizeof(int)) != hipSuccess) return -1;
+  if (reset && v && hipMemset(w.cnt - 1, 0, sizeof(int)) != hipSuccess) return -1;
   return v;
 }
 
@@ -1285,20 +1300,23 @@ void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, i
            0, 0, 0, 0, !(prio & 8) && EPI != 2 && EPI != 5, na.ss, na.ss_ld, na.inv_k, na.eps,
            na.pos, na.cs, na.slots, na.kc, na.vc, na.qcols, na.kvcols, na.nkv, na.bs};
   const int nt = K / kBK;
-  SkWorkspace* sk = ((skmode || a.ovl) && nt >= 8) ? sk_workspace(s) : nullptr;
-  if (sk) {
-    const int P = (g_cu_limit >= 8 && g_cu_limit < sk->P) ? (g_cu_limit & ~7) : sk->P;
+  const int units = (skmode || a.ovl) && nt >= 8 ? gemm_units() : 0;
+  if (units) {
+    const int P = (g_cu_limit >= 8 && g_cu_limit < units) ? (g_cu_limit & ~7) : units;
     const int full = total / P, rem = total % P;
     const int splits = rem ? min(4, P / rem) : 0;
     if (skmode && splits >= 2 && (full < 8 || skmode == 2)) {
-      a.ws = sk->ws;
-      a.cnt = sk->cnt;
-      a.rem = rem;
-      a.splits = splits;
-      a.full = full;
-      a.P = P;
-      kern<<<dim3(P), 512, 0, s>>>(a);
-      return;
+      const SkWorkspace sk = sk_workspace(units, s);
+      if (sk.ws) {
+        a.ws = sk.ws;
+        a.cnt = sk.cnt;
+        a.rem = rem;
+        a.splits = splits;
+        a.full = full;
+        a.P = P;
+        kern<<<dim3(P), 512, 0, s>>>(a);
+        return;
+      }
     }
     if (a.ovl && rem == 0 && full >= 2) {
       // whole waves of tiles: persistent, so each block's next tile loads under this one's epilogue

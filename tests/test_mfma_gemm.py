@@ -265,3 +265,28 @@ def test_mfma_gemm_norm_rope_matches_fp32(M, nh, nkv, K, phases):
         err = (g.float() - w.float()).abs()
         tol = 2e-2 * w.float().abs().max().item() + 1e-3
         assert err.max().item() <= tol, (err.max().item(), tol)
+
+
+@pytest.mark.gpu
+def test_mfma_gemm_first_used_by_several_threads():
+    """Threads that meet in the first products of a process (whole tiles, the launch sized for the device's units)."""
+    import threading
+    ops.load_native(required=True)
+    x, w = _rand(300, 512, device="cuda", seed=1), _rand(256 * 256, 512, device="cuda", scale=0.05, seed=2)
+    start, got = threading.Barrier(4), [None] * 4
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            start.wait()
+            got[i] = ops.mfma_gemm(x, w, streamk=1)
+            torch.cuda.current_stream().synchronize()
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    ref = ops.mfma_gemm_ref(x, w).float()
+    assert all(torch.equal(a, got[0]) for a in got[1:])
+    assert (got[0].float() - ref).abs().max().item() <= 2e-2 * ref.abs().max().item() + 1e-3
