@@ -38,10 +38,11 @@ int dgi_rope_cache_parts(void* out, const float* parts, int nparts, const void* 
                          int block_size, hipStream_t s);
 int dgi_skinny_gemm(const void* x, int ldx, const void* w, const void* bias, void* y, int ldy, int M,
                     int N, int K, int nw, hipStream_t s);
-int dgi_mfma_gemm(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int epi,
-                  hipStream_t s);
+int dgi_mfma_gemm(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int epi, float* slabs,
+                  int* counters, hipStream_t s);
 void dgi_set_gemm_cus(int cus);
 int dgi_gemm_split_timeouts(int reset);
+int dgi_gemm_units();
 int dgi_mfma_gemm_norm(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, int kind,
                        float* ss, int ss_ld, float inv_k, float eps, int phases, hipStream_t s);
 int dgi_mfma_gemm_norm_rope(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K, float* ss,
@@ -313,7 +314,9 @@ void rope_cache_parts(at::Tensor out, const at::Tensor& parts, const c10::option
 }
 
 // LDS-tiled MFMA GEMM (prefill / mixed steps): epi 0 out = x w^T; epi 1 out = SwiGLU with w = [gate; up].
-void mfma_gemm(at::Tensor out, const at::Tensor& x, const at::Tensor& w, int64_t epi) {
+// slabs / counters: split-K workspace of this call alone (gemm_units() slabs of 256 x 256, 1 + 2 gemm_units() zeros), else the device's.
+void mfma_gemm(at::Tensor out, const at::Tensor& x, const at::Tensor& w, int64_t epi, const c10::optional<at::Tensor>& slabs,
+               const c10::optional<at::Tensor>& counters) {
   check_bf16(out, "out"); check_bf16(x, "x"); check_bf16(w, "w");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2, "mfma_gemm: 2-D operands");
   TORCH_CHECK(x.device() == w.device() && x.device() == out.device(), "mfma_gemm: operands on one device");
@@ -329,8 +332,17 @@ void mfma_gemm(at::Tensor out, const at::Tensor& x, const at::Tensor& w, int64_t
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(out.data_ptr()) % 8 == 0, "mfma_gemm: operand alignment");
   TORCH_CHECK((int64_t)M * x.stride(0) < (1LL << 31), "mfma_gemm: activation too large for 32-bit offsets");
+  TORCH_CHECK(slabs.has_value() == counters.has_value(), "mfma_gemm: slabs and counters go together");
+  if (slabs.has_value()) {
+    check_dev(*slabs, "slabs"); check_i32(*counters, "counters");
+    TORCH_CHECK(slabs->scalar_type() == at::kFloat && slabs->is_contiguous() && counters->is_contiguous() && slabs->device() == x.device() &&
+                    counters->device() == x.device() && ((uintptr_t)slabs->data_ptr() & 15) == 0 &&
+                    slabs->numel() >= (int64_t)dgi_gemm_units() * 65536 && counters->numel() >= 1 + 2 * (int64_t)dgi_gemm_units(),
+                "mfma_gemm: a slab and two counters per compute unit, and one more");
+  }
   check_rc(dgi_mfma_gemm(x.data_ptr(), (int)x.stride(0), w.data_ptr(), out.data_ptr(), (int)out.stride(0), (int)M,
-                         (int)N, (int)K, (int)epi, cur_stream()),
+                         (int)N, (int)K, (int)epi, slabs.has_value() ? slabs->data_ptr<float>() : nullptr,
+                         counters.has_value() ? counters->data_ptr<int>() : nullptr, cur_stream()),
            "mfma_gemm");
 }
 
@@ -665,6 +677,7 @@ void tree_verify(at::Tensor accept_len, at::Tensor path, at::Tensor out_tokens,
 // CUs the MFMA GEMM's persistent launches size their grid for (0 = the device's; a CU-masked
 // two-batch-overlap step sets the GEMM stream's share)
 void set_gemm_cus(int64_t cus) { dgi_set_gemm_cus(static_cast<int>(cus)); }
+int64_t gemm_units() { return dgi_gemm_units(); }
 int64_t gemm_split_timeouts(bool reset) { return dgi_gemm_split_timeouts(reset ? 1 : 0); }
 
 }  // namespace
@@ -672,6 +685,7 @@ int64_t gemm_split_timeouts(bool reset) { return dgi_gemm_split_timeouts(reset ?
 TORCH_LIBRARY(dgi, m) {
   m.def("set_gemm_cus(int cus) -> ()", &set_gemm_cus);
   m.def("gemm_split_timeouts(bool reset) -> int", &gemm_split_timeouts);
+  m.def("gemm_units() -> int", &gemm_units);
   m.def("rmsnorm(Tensor(a!) out, Tensor x, Tensor w, float eps) -> ()");
   m.def("fused_add_rmsnorm(Tensor(a!) x, Tensor(b!) residual, Tensor w, float eps) -> ()");
   m.def("rope_cache(Tensor(a!) qkv, Tensor positions, Tensor cos_sin, int nh, int nkv, int hd, "
@@ -690,7 +704,7 @@ TORCH_LIBRARY(dgi, m) {
   m.def("rope_cache_parts(Tensor(a!) out, Tensor parts, Tensor? bias, Tensor positions, Tensor cos_sin, int nh, int nkv, int hd, "
         "Tensor slot_mapping, Tensor(b!) k_cache, Tensor(c!) v_cache, int mode) -> ()");
   m.def("skinny_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int cfg=0) -> ()");
-  m.def("mfma_gemm(Tensor(a!) out, Tensor x, Tensor w, int epi=0) -> ()");
+  m.def("mfma_gemm(Tensor(a!) out, Tensor x, Tensor w, int epi=0, Tensor(b!)? slabs=None, Tensor(c!)? counters=None) -> ()");
   m.def("mfma_gemm_norm(Tensor(a!) out, Tensor x, Tensor w, int kind, Tensor(b!) ss, float inv_k, float eps, "
         "int phases=0) -> ()");
   m.def("mfma_gemm_norm_rope(Tensor(a!) out, Tensor x, Tensor w, Tensor ss, float inv_k, float eps, "

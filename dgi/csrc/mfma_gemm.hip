@@ -1211,9 +1211,9 @@ int gemm_units() {
   return n;
 }
 
-// Per-device split-K workspace (one fp32 slab per block + two counters per tile),
-// allocated on first use outside stream capture.  Shared by every stream of
-// the process: the engine issues its projection GEMMs on one stream at a time.
+// Split-K workspace: one fp32 slab per block, two counters per tile.  A caller's own (one call at a time), or the
+// device's, allocated on first use outside stream capture and shared by every stream of the process: for callers that
+// issue such products on one stream at a time, as the fused-norm layers of an engine do.
 struct SkWorkspace {
   float* ws = nullptr;
   int* cnt = nullptr;   // 2 P counters, preceded by the error word cnt[-1] (timed-out waits)
@@ -1283,7 +1283,7 @@ struct NormArgs {
 
 template <int EPI>
 void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, int I, int K, int tiles_m, int total,
-               int skmode, int prio, hipStream_t s, const NormArgs& na = NormArgs{}) {
+               int skmode, int prio, hipStream_t s, const NormArgs& na = NormArgs{}, const SkWorkspace& own = SkWorkspace{}) {
   decltype(&mfma_gemm_pp_kernel<EPI, 0, 2>) kern;
   if constexpr (EPI >= 2)       // the fused-norm epilogues: default priority scheme only
     kern = (prio & 4) ? mfma_gemm_pp_kernel<EPI, 0, 2> : mfma_gemm_pp_kernel<EPI, 0, 4>;
@@ -1306,7 +1306,7 @@ void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, i
     const int full = total / P, rem = total % P;
     const int splits = rem ? min(4, P / rem) : 0;
     if (skmode && splits >= 2 && (full < 8 || skmode == 2)) {
-      const SkWorkspace sk = sk_workspace(units, s);
+      const SkWorkspace sk = own.ws ? own : sk_workspace(units, s);
       if (sk.ws) {
         a.ws = sk.ws;
         a.cnt = sk.cnt;
@@ -1331,9 +1331,9 @@ void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, i
 
 template <int EPI, int SCHED>
 void launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int I, int K, int tiles_m, int total,
-            int skmode, int prio, hipStream_t s) {
+            int skmode, int prio, hipStream_t s, const SkWorkspace& own) {
   if (SCHED == 3)
-    launch_pp<EPI>(x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s);
+    launch_pp<EPI>(x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s, NormArgs{}, own);
   else if (SCHED == 2)
     mfma_gemm_ring_kernel<EPI><<<dim3(total), 512, 0, s>>>((const uint16_t*)x, ldx, (const uint16_t*)w,
                                                           (uint16_t*)y, ldy, M, I, K, tiles_m, total);
@@ -1351,7 +1351,11 @@ void launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int 
 // s_setprio variant of schedule 3, (epi >> 12) & 1: two 32-MFMA phases per K tile, (epi >> 13) & 1:
 // four 16-MFMA phases (default: two up to M = 2560, see mfma_gemm_pp_kernel), (epi >> 14) & 1: no
 // cross-tile overlap (next tile's prologue after the epilogue; whole waves of tiles not persistent).
+// slabs / counters: the call's own split-K workspace (gemm_units() * 65536 floats, 1 + 2 * gemm_units() zeros, the first the error
+// word), or nullptr for the device's.
 extern "C" void dgi_set_gemm_cus(int cus) { g_cu_limit = cus; }
+
+extern "C" int dgi_gemm_units() { return gemm_units(); }
 
 extern "C" int dgi_gemm_split_timeouts(int reset) { return sk_timeouts(reset != 0); }
 
@@ -1420,7 +1424,7 @@ extern "C" int dgi_mfma_gemm_norm_rope(const void* x, int ldx, const void* w, vo
 }
 
 extern "C" int dgi_mfma_gemm(const void* x, int ldx, const void* w, void* y, int ldy, int M, int N, int K,
-                             int epi, hipStream_t s) {
+                             int epi, float* slabs, int* counters, hipStream_t s) {
   if (M <= 0) return 0;
   const int swiglu = epi & 15;
   int sched = (epi >> 4) & 15;
@@ -1445,12 +1449,15 @@ extern "C" int dgi_mfma_gemm(const void* x, int ldx, const void* w, void* y, int
   const int tiles_n = swiglu ? I / 128 : N / 256;
   const int tiles_m = (M + kBM - 1) / kBM;
   const int total = tiles_m * tiles_n;
+  SkWorkspace own;
+  own.ws = slabs;
+  own.cnt = slabs ? counters + 1 : nullptr;
   if (swiglu)
     (sched == 3 ? launch<1, 3> : sched == 2 ? launch<1, 2> : sched ? launch<1, 1> : launch<1, 0>)(
-        x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s);
+        x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s, own);
   else
     (sched == 3 ? launch<0, 3> : sched == 2 ? launch<0, 2> : sched ? launch<0, 1> : launch<0, 0>)(
-        x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s);
+        x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s, own);
   DGI_CHECK_LAUNCH();
   return 0;
 }

@@ -501,8 +501,8 @@ class LlamaModel:
     def _last_mlp(h: torch.Tensor, L: LlamaLayerWeights) -> torch.Tensor:
         """gate_up, SwiGLU and down of the rows that logits are asked for."""
         act = ops.silu_mul(ops.linear(h, L.gate_up))
-        if ops.split_gemm(act.shape[0], *L.down.shape) and ops.mfma_gemm_ok(act, L.down):
-            return ops.mfma_gemm(act, L.down)
+        if ops.split_gemm(act.shape[0], *L.down.shape) and ops.mfma_gemm_ok(act, L.down) and L.down.data_ptr() % 16 == 0:
+            return ops.mfma_gemm(act, L.down, own_space=True)      # other models may do so on other streams
         return ops.linear(act, L.down)
 
     # ------------------------------------------------------------------ fused-norm layers

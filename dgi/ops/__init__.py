@@ -560,7 +560,7 @@ def tile_gemm(M: int, N: int) -> bool:
 def split_gemm(M: int, N: int, K: int) -> bool:
     """Whether a product of long rows, 129 to 512 of them, is better split along K by ``mfma_gemm`` (8192 x 28672, vendor's product and
     this one, us: 129 rows 309, 173; 200 311, 185; 256 323, 195; 353 197, 195; 512 310, 201; but 640 264, 310; 4096 x 14336 at
-    200 60, 98).  For callers that issue such products on one stream at a time: they share a workspace per device."""
+    200 60, 98)."""
     return 128 < M <= 512 and K >= 16384 and N * K >= 1 << 27
 
 
@@ -765,9 +765,16 @@ def gemm_split_timeouts(reset: bool = False) -> int:
     return int(torch.ops.dgi.gemm_split_timeouts(bool(reset)))
 
 
+def _split_space(device) -> tuple:
+    """Split-K workspace of one product: a slab of 256 x 256 per compute unit, and the error word and two counters for each, zeros."""
+    with torch.cuda.device(device):
+        units = torch.ops.dgi.gemm_units()
+    return (torch.empty(units * 65536, dtype=torch.float32, device=device), torch.zeros(1 + 2 * units, dtype=torch.int32, device=device))
+
+
 def mfma_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: Optional[torch.Tensor] = None,
               sched: Optional[int] = None, streamk: int = 0, prio: int = 0, phases: int = 0,
-              overlap: bool = True) -> torch.Tensor:
+              overlap: bool = True, own_space: bool = False) -> torch.Tensor:
     """Hand-written LDS-tiled MFMA GEMM (256x256 tiles, global_load_lds
     staging, XCD-aware tile order): ``epi`` 0 -> x @ w.T; 1 -> the fused
     SwiGLU of the MLP, silu(x @ gate.T) * (x @ up.T) with w = [gate; up],
@@ -776,7 +783,10 @@ def mfma_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: Optional[torc
     last partial wave) policy: 0 auto, 1 off, 2 whenever it applies;
     ``phases`` per K tile: 0 auto (2 up to M = 2560, else 4), 2 or 4;
     ``prio``: s_setprio variant (benchmarking); ``overlap`` False: no
-    cross-tile prologue / epilogue overlap (A/B)."""
+    cross-tile prologue / epilogue overlap (A/B).  Split-K goes through a
+    workspace that all streams of a device share, for callers that issue such
+    products on one stream at a time; ``own_space`` True: through one of this
+    call's (64 MB of torch's pool)."""
     M = x.shape[0]
     N = w.shape[0] // 2 if epi == 1 else w.shape[0]
     if mfma_gemm_ok(x, w):
@@ -785,7 +795,7 @@ def mfma_gemm(x: torch.Tensor, w: torch.Tensor, epi: int = 0, out: Optional[torc
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _call("mfma_gemm", out, x, w, epi | ((MFMA_SCHED if sched is None else sched) << 4) | (streamk << 8)
               | (prio << 10) | ((1 if phases == 2 else 0) << 12) | ((1 if phases == 4 else 0) << 13)
-              | ((0 if overlap else 1) << 14))
+              | ((0 if overlap else 1) << 14), *(_split_space(x.device) if own_space else ()))
         return out
     r = mfma_gemm_ref(x, w, epi)
     if out is not None:

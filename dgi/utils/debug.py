@@ -61,7 +61,7 @@ def after_op(name: str, *tensors) -> None:
         raise RuntimeError(f"dgi op {name} failed (inputs {shapes}): {e}") from e
     if name.startswith("mfma_gemm"):
         from dgi import ops
-        n = ops.gemm_split_timeouts(reset=True)
+        n = ops.gemm_split_timeouts(reset=True) + (int(tensors[5][0]) if name == "mfma_gemm" and len(tensors) > 5 else 0)
         if n:  # pragma: no cover - needs a broken split-K counter
             shapes = [tuple(t.shape) for t in tensors if isinstance(t, torch.Tensor)]
             raise RuntimeError(f"dgi op {name}: {n} split-K wait(s) timed out (inputs {shapes}): wrong tiles")

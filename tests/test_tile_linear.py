@@ -139,3 +139,59 @@ def test_linear_takes_what_the_plain_product_takes(M, N, K):
         ops.linear(x, w.new_zeros(N, K + 64))
     with pytest.raises(RuntimeError):
         ops.linear(x, w, out=torch.empty(M + 1, N, device="cuda").bfloat16())
+
+
+def test_the_last_mlp_has_a_workspace_of_its_own(monkeypatch):
+    """Models stepped from several threads or streams share a device: their split products must not share partial sums."""
+    from types import SimpleNamespace
+    from dgi.models.llama import LlamaModel
+    seen = []
+    monkeypatch.setattr(ops, "split_gemm", lambda *a: True)
+    monkeypatch.setattr(ops, "mfma_gemm_ok", lambda *a: True)
+    monkeypatch.setattr(ops, "mfma_gemm", lambda x, w, **k: (seen.append(k), x @ w.t())[1])
+    layer = SimpleNamespace(gate_up=torch.randn(16, 8), down=torch.randn(8, 8))
+    LlamaModel._last_mlp(torch.randn(3, 8), layer)
+    assert seen == [{"own_space": True}]
+
+
+@pytest.mark.gpu
+def test_split_products_of_two_streams():
+    """Two threads, each with a stream and operands of its own: every product has the bits that it has alone; and captured."""
+    import threading
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    sets = []
+    for i, M in enumerate((129, 300)):
+        x = torch.randn(M, 16384, device="cuda", generator=g).bfloat16()
+        w = (torch.randn(8192, 16384, device="cuda", generator=g) * 2 ** -7).bfloat16()
+        v = torch.randn(448 * 256, 16384, device="cuda", generator=g).bfloat16() if i else None
+        sets.append((x, w, v, ops.mfma_gemm(x, w, own_space=True)))
+        assert torch.equal(ops.mfma_gemm(x, w), sets[-1][3])
+        ref = x.float() @ w.float().t()
+        assert ((sets[-1][3].float() - ref).norm() / ref.norm()) <= 2.0 ** -8
+    torch.cuda.synchronize()
+    wrong = [0, 0]
+
+    def work(i):
+        x, w, v, want = sets[i]
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(30):
+                got = ops.mfma_gemm(x, w, own_space=True)
+                if v is not None and _ % 8 == 0:
+                    ops.linear(x, v)
+                wrong[i] += int(not torch.equal(got, want))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == [0, 0]
+    x, w, _, want = sets[0]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.mfma_gemm(x, w, own_space=True)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(got, want) and torch.equal(ops.mfma_gemm(x, w), want)
