@@ -514,13 +514,13 @@ __global__ __launch_bounds__(64 * NW, R == 8 ? 2 : 3) void masked_attn_tiles_ker
   const int* bt = a.block_tables + (size_t)seq * a.bt_stride;
   const int pos = a.positions[row];
   const int first = a.mask > 0 ? (pos / a.mask) * a.mask : (a.mask < 0 ? max(0, pos + a.mask + 1) : 0);
-  const int ntiles = (pos - first) / 64 + 1;
+  const int ntiles = pos < 0 ? 0 : (pos - first) / 64 + 1;       // a row without a position sees no keys
   const int tpr = (ntiles + (int)gridDim.z - 1) / (int)gridDim.z;      // tiles per run
   const int t_end = min(ntiles, ((int)blockIdx.z + 1) * tpr);
   int tile = blockIdx.z * tpr + w;
   // slot of this lane's key of a tile; lanes past the last key point at it: every load stays in bounds
   auto slot = [&](int t) {
-    const int kq = min(first + t * 64 + lane, pos);
+    const int kq = max(min(first + t * 64 + lane, pos), 0);
     return (bt[kq / bs] * G + kvh) * bs + kq % bs;
   };
   const int slot0 = slot(min(tile, ntiles - 1));
@@ -682,7 +682,10 @@ __global__ __launch_bounds__(64 * NW, R == 8 ? 2 : 3) void masked_attn_tiles_ker
 #pragma unroll
     for (int ww = 0; ww < NW; ++ww) M = fmaxf(M, cm[ww][i]);
     float L = a.sinks && !a.part_o ? expf(a.sinks[head] - M) : 0.f, O = 0.f;      // the sink: one more term of the denominator
-    if (M != -__builtin_inff()) {                    // an empty run leaves zeros
+    if (pos < 0) {                                   // no keys at all: zeros
+      M = 0.f;
+      L = 1.f;
+    } else if (M != -__builtin_inff()) {             // an empty run leaves zeros
 #pragma unroll
       for (int ww = 0; ww < NW; ++ww) {
         const float f = expf(cm[ww][i] - M);         // waves without a tile: exp(-inf) = 0

@@ -72,3 +72,17 @@ def test_an_infinite_key_and_value_stay_theirs():
     kc[int(table[0, 5]), 0, 3, 7] = -float("inf")        # position 83 of row 0
     vc[int(table[1, 5]), 0, 10:] = float("inf")          # positions 90 on of row 1: past its end
     check(q, kc, vc, table, pos, 2, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("runs", [1, 3])
+def test_rows_without_a_position(runs):
+    """Position -1: no key is read, the result is zero; the rows beside it keep theirs."""
+    q, kc, vc, table, pos, gate = case([700, 1, 33], 4, 2, 64, 64, 16, 9)
+    pos[1] = -1
+    check(q, kc, vc, table, pos, 4, 2, gate=gate, runs=runs)
+    check(q, kc, vc, table, pos, 4, 2, runs=runs, sinks=torch.linspace(-2.0, 3.0, 4), window=20)
+    kept = [0, 2]
+    want = mix.masked_attn_rows(q.cuda()[kept], kc.cuda(), vc.cuda(), table.cuda()[kept], None, pos.cuda()[kept], 4, 2, 0.125, 1)
+    got = mix.masked_attn_rows(q.cuda(), kc.cuda(), vc.cuda(), table.cuda(), None, pos.cuda(), 4, 2, 0.125, 1)
+    assert torch.equal(got[kept], want) and not got[1].any()
