@@ -86,3 +86,14 @@ def test_rows_without_a_position(runs):
     want = mix.masked_attn_rows(q.cuda()[kept], kc.cuda(), vc.cuda(), table.cuda()[kept], None, pos.cuda()[kept], 4, 2, 0.125, 1)
     got = mix.masked_attn_rows(q.cuda(), kc.cuda(), vc.cuda(), table.cuda(), None, pos.cuda(), 4, 2, 0.125, 1)
     assert torch.equal(got[kept], want) and not got[1].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 32, 33, 63, 64, 96, 600])
+def test_an_infinite_value_at_the_row_s_own_position(n):
+    """What stands in for keys past the last one is that key: its infinite value must not meet their zero weights."""
+    q, kc, vc, table, pos, _ = case([n, 20], 2, 1, 64, 64, 16, 10)
+    vc[int(table[0, (n - 1) // 16]), 0, (n - 1) % 16, 5] = float("inf")
+    args = (table.cuda(), None, pos.cuda(), 2, 1, 0.125)
+    got = mix.masked_attn_rows(q.cuda(), kc.cuda(), vc.cuda(), *args)
+    assert torch.isposinf(got.view(2, 2, 64)[0, :, 5]).all() and int(torch.isfinite(got).sum()) == got.numel() - 2
