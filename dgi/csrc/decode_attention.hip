@@ -436,12 +436,15 @@ extern "C" int dgi_paged_decode(const void* q, int q_stride, const void* k_cache
   // splits slowest: consecutive workgroups go to different XCDs, and where short contexts leave all but the first splits empty the
   // others would have all the work (64 rows of 1024 in up to 4 splits of 2048 at the least, splits fastest: 133 us, not 51)
   dim3 grid(nkv, B, max_splits);
-  // up to a workgroup per compute unit: eight waves each, half the serial chain of tiles (8 rows of 1000 tokens, 8 kv heads, in 4 splits
+  // Up to a workgroup per compute unit: eight waves each, half the serial chain of tiles (8 rows of 1000 tokens, 8 kv heads, in 4 splits
   // 12.9 us, with four 15.3); more of them: four, so that several share a unit, and rows marked as read once (64 rows of 1024: 50.6,
-  // with eight 52.6; without the mark 53.4)
-  const bool wide = (long long)B * nkv * max_splits <= 256;
+  // with eight 52.6; without the mark 53.4).  A device-side plan counts as unsplit: how many of its splits there are depends on the contexts
+  // (24 rows of 1000 in up to 4 splits of 2048 at the least 22.9, with four waves 27.5), and where it cuts such steps in earnest eight
+  // waves are as good (17 rows of 4000 in 3 splits 59.9, with four 61.9).
+  const bool wide = (long long)B * nkv * (part_size > 0 ? max_splits : 1) <= 256;
   // there the last workgroup of a (sequence, kv head) combines its splits (1 row of 600 tokens 8.3 us, with a reduce kernel 9.1, of 8000
-  // in 32 splits 16.0 and 19.3); among more workgroups than that the last arriver's work is the tail of the launch
+  // in 32 splits 16.0 and 19.3); among more workgroups than that the ticket's round trip holds places that others wait for (64 rows
+  // of 4000 in 2 splits 187, with a reduce kernel 176)
   if (!wide) counters = nullptr;
   auto launch = [&](auto HD_, auto NW_, auto P16_) {
     constexpr int HD = decltype(HD_)::value, NW = decltype(NW_)::value;

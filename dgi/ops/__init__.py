@@ -244,16 +244,39 @@ def paged_decode_ref(q, k_cache, v_cache, block_tables, context_lens, nh, nkv, s
     return out
 
 
-def decode_split_plan(batch: int, max_ctx: int, nkv: int, num_cus: int = 256) -> tuple[int, int]:
-    """(max_splits, part_size) for the split-KV decode kernel, as its device-side plan (``part_size`` < 0).
+def decode_whole(batch: int, nkv: int, num_cus: int = 256) -> int:
+    """Contexts up to which decode attention leaves rows whole (``decode_split_plan``); 0: they are split from 128 tokens on."""
+    seqs = batch * nkv
+    if 2 * seqs <= num_cus:
+        return 0
+    if 4 * seqs <= 3 * num_cus:
+        return 2048
+    return 8192 if seqs <= num_cus else 1024 if 2 * seqs <= 3 * num_cus else 2048
 
-    One workgroup of eight waves per CU: more splits cost more than they bring (8 kv heads of 128 dims, us a layer with the
-    reduce kernel: 8 rows of 4000 tokens in 2 / 4 / 8 / 16 splits 43.7 / 29.7 / 31.4 / 35.1, 1 row of 8000 in 16 / 32 / 64
-    18.5 / 19.0 / 27.7; combined in the kernel 1 row of 8000 in 32 16.0).  Rows that fill the chip by themselves are not split
-    (64 rows of 1024 in 1 / 2 splits 50.6 / 52.6, of 300 17.6 / 24.1) but past 2048 tokens, so that a few long ones do not
-    hold up the step."""
-    seqs = max(1, batch * nkv)
-    splits, part = (8, 2048) if 2 * seqs > num_cus else (num_cus // seqs, 128)
+
+def decode_split_plan(batch: int, max_ctx: int, nkv: int, num_cus: int = 256) -> tuple[int, int]:
+    """(max_splits, part_size) for the split-KV decode kernel, as its device-side plan (``part_size`` < 0): workgroups own a (row, kv head,
+    split).  8 kv heads of 128 dims, us a layer:
+
+    * up to half a workgroup per CU: as many splits as give every CU one, of eight waves; more cost more than they bring (8 rows of
+      4000 tokens in 2 / 4 / 8 / 16 splits 43.7 / 29.7 / 31.4 / 35.1, 1 row of 8000 in 16 / 32 / 64 18.5 / 19.0 / 27.7).
+    * up to three quarters (24 rows; a captured step may have as few as 17 of them): whole while all contexts are short (17 rows of 1600
+      32, in two splits 35; 24 rows 35 and 41), then three splits: two would take as many rounds of the chip (17 of 4000 72 whole, in
+      two 74, in three 60; 24 rows 80, 83, 85).
+    * up to one per CU: whole (32 rows of 2000 / 4000 53 / 101, in two splits 56 / 101, in three 61 / 103), but past 8192 tokens, so
+      that a few long ones do not hold up the step.
+    * more: workgroups of four waves, three to a CU.  Up to 48 rows 1024 tokens a split keep the chip busy to the end (40 rows of 1600 / 3000
+      64 / 117 whole, 55 / 95 in splits; 2048 a split 66 / 95); past that they cost more than whole rows (64 rows of 1000 47.9
+      whole, 54.3; of 3000 137, 134), and 2048 it is (49.7 and 135.5)."""
+    seqs, whole = max(1, batch * nkv), decode_whole(batch, nkv, num_cus)
+    if max_ctx <= whole:
+        return 1, -whole
+    if whole == 0:
+        splits, part = num_cus // seqs, 128
+    elif 4 * seqs <= 3 * num_cus:
+        splits, part = max(3, min(8, -(-max_ctx // 16384))), 1024
+    else:
+        splits, part = 8, whole
     return max(1, min(splits, -(-max_ctx // part))), -part
 
 

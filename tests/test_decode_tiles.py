@@ -55,3 +55,22 @@ def test_plan_of_splits(batch, ctx, nkv):
         assert (splits - 1) * -part < ctx
     if batch * nkv * splits > 256:
         assert splits <= 8 and (splits == 1 or ctx > 2048)
+
+
+def live_splits(ctx, splits, part):
+    """Splits of one context as the kernel's device-side plan makes them."""
+    n = max(1, min(splits, -(-ctx // -part)))
+    part = -(-(-(-ctx // n)) // 32) * 32
+    return -(-ctx // part)
+
+
+@pytest.mark.parametrize("nkv", [4, 8])
+@pytest.mark.parametrize("limit", [4096, 8192, 32768])
+def test_plans_keep_the_units_busy(nkv, limit):
+    """Steps of up to a workgroup per unit, which run one at a time on each: long contexts take rounds of the chip that are two
+    thirds full at least, whatever the longest context that may come."""
+    for seqs in range(96, 257, nkv):
+        splits, part = ops.decode_split_plan(seqs // nkv, limit, nkv)
+        for ctx in (3400, 4096):
+            n = seqs * live_splits(ctx, splits, part)
+            assert n / (-(-n // 256) * 256) >= 0.66, (seqs, ctx)
