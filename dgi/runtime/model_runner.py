@@ -407,6 +407,7 @@ class GraphRunner:
         self.short_ctx = int(os.environ.get("DGI_DECODE_SHORT_CTX", "384"))
         self.short_max_b = int(os.environ.get("DGI_DECODE_SHORT_B", "8"))
         self.short_graphs: dict[int, torch.cuda.CUDAGraph] = {}
+        self.short_limits: dict[int, int] = {}
         self._short = False
         self.pool_handle = None
         dev = runner.device
@@ -432,14 +433,26 @@ class GraphRunner:
         """(max_splits, part_size) captured for bucket ``b``.  Dynamic (the
         default): the kernel splits each sequence's own context
         (``ops.decode_split_plan``), so one graph serves every context
-        length without idle splits; DGI_DECODE_DYNAMIC=0 keeps the
-        fixed max_model_len / part_size plan."""
+        length; DGI_DECODE_DYNAMIC=0 keeps the fixed max_model_len /
+        part_size plan."""
         r = self.r
         if os.environ.get("DGI_DECODE_DYNAMIC", "1") == "0":
             return r.graph_splits, r.graph_part
         want, part = ops.decode_split_plan(b, r.max_model_len, r.model.cfg.num_kv_heads, r.num_cus)
         part = -int(os.environ.get("DGI_DECODE_MIN_PART", "0")) or part
         return min(r.ws_splits, want), part
+
+    def short_limit(self, b: int) -> int:
+        """Context up to which bucket ``b`` replays a one-split graph of its own (0: it has none): few rows, and buckets whose rows are best
+        left whole while all contexts are short (8 kv heads of 128 dims, the splits of longer ones captured and whole, us a layer: 17 rows in
+        a bucket of 24, 1600 tokens 35 and 32; 48 rows of 300 tokens 18.1 and 16.4, 128 of 1000 96.7 and 92)."""
+        c = self.r.model.cfg
+        if self.short_ctx <= 0 or c.head_dim not in (64, 128):
+            return 0
+        if b <= self.short_max_b:
+            return self.short_ctx
+        splits, part = self.split_plan(b)
+        return ops.decode_whole(b, c.num_kv_heads, self.r.num_cus) if splits > 1 and part < 0 else 0
 
     def views(self, b: int) -> dict:
         """Bucket ``b``'s inputs: views into the staging image ``dev_in``."""
@@ -496,7 +509,8 @@ class GraphRunner:
             if self.pool_handle is None:
                 self.pool_handle = g.pool()
             self.graphs[b] = g
-            if self.short_ctx > 0 and b <= self.short_max_b and self.r.model.cfg.head_dim in (64, 128):
+            self.short_limits[b] = self.short_limit(b)
+            if self.short_limits[b] > 0:
                 self._short = True
                 try:
                     self._body(b)
@@ -553,7 +567,7 @@ class GraphRunner:
         if ahead:
             self.dev_in[:n].copy_(self.out[:n])        # the previous launch's tokens (same rows, same order)
         gs = self.short_graphs.get(b)
-        short = gs is not None and max_ctx <= self.short_ctx
+        short = gs is not None and max_ctx <= self.short_limits[b]
         (gs if short else self.graphs[b]).replay()
         self.last_bucket = b
         self.last_key = (b, short)

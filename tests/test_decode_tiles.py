@@ -74,3 +74,53 @@ def test_plans_keep_the_units_busy(nkv, limit):
         for ctx in (3400, 4096):
             n = seqs * live_splits(ctx, splits, part)
             assert n / (-(-n // 256) * 256) >= 0.66, (seqs, ctx)
+
+
+def test_captured_plans_serve_short_contexts(monkeypatch):
+    """A bucket's plan is that of the longest context that may come.  Where it would split contexts that are best left whole, or leave a second
+    kernel to combine nothing, a graph of whole rows goes with it."""
+    from types import SimpleNamespace
+    from dgi.runtime.model_runner import GraphRunner
+    for name in ("DGI_DECODE_DYNAMIC", "DGI_DECODE_MIN_PART"):
+        monkeypatch.delenv(name, raising=False)
+    for limit in (1024, 2048, 8192, 131072):
+        r = GraphRunner.__new__(GraphRunner)
+        cfg = SimpleNamespace(num_kv_heads=8, head_dim=128)
+        r.r = SimpleNamespace(model=SimpleNamespace(cfg=cfg), num_cus=256, max_model_len=limit, ws_splits=limit // 128)
+        r.short_ctx, r.short_max_b = 384, 8
+        assert [r.short_limit(b) for b in (1, 8, 9, 16)] == [384, 384, 0, 0]
+        for b in (17, 24, 32, 40, 48, 64, 512):
+            splits, part = r.split_plan(b)
+            whole = ops.decode_whole(b, 8)
+            assert whole in (1024, 2048, 8192) and (splits > 1) == (limit > whole)
+            assert r.short_limit(b) == (whole if splits > 1 else 0)
+            assert ops.decode_split_plan(b, whole, 8)[0] == 1 and ops.decode_split_plan(b, whole + 1, 8)[0] > 1
+        r.short_ctx = 0
+        assert not any(r.short_limit(b) for b in (1, 24, 64))
+
+
+@pytest.mark.gpu
+def test_both_graphs_of_a_large_bucket(monkeypatch):
+    """Contexts that grow past the line between the two graphs of a bucket: the same tokens as with one graph."""
+    from dgi.engine import EngineConfig, LLMEngine
+    from dgi.models.config import get_config
+    from dgi.models.llama import LlamaModel
+    from dgi.runtime.model_runner import GraphRunner
+    from dgi.sched.request import SamplingParams
+    monkeypatch.setattr(ops, "decode_whole", lambda b, nkv, num_cus=256: 64)
+    cfg = get_config("llama3-8b@L2")
+    cfg.hidden_size, cfg.intermediate_size, cfg.num_heads, cfg.num_kv_heads, cfg.vocab_size = 1024, 1024, 8, 8, 1024
+    m = LlamaModel(cfg, "cuda", torch.bfloat16, init="random", seed=5)
+    keys, outs = [], []
+    launch = GraphRunner.launch
+    monkeypatch.setattr(GraphRunner, "launch", lambda self, *a, **k: (launch(self, *a, **k), keys.append(self.last_key))[0])
+    for short in ("384", "0"):
+        monkeypatch.setenv("DGI_DECODE_SHORT_CTX", short)
+        eng = LLMEngine(EngineConfig(model=cfg.name, device="cuda", num_blocks=256, max_num_seqs=40, max_model_len=4096,
+                                     max_num_batched_tokens=512, graph_buckets=(40,)), model_cfg=cfg, model=m)
+        reqs = eng.generate([[(7 * i + j) % 1000 for j in range(52 + i)] for i in range(3)],
+                            SamplingParams(max_tokens=20, temperature=0.0, ignore_eos=True))
+        outs.append([r.output for r in reqs])
+        assert {k for k in keys} == ({(40, True), (40, False)} if short != "0" else {(40, False)})
+        keys.clear()
+    assert outs[0] == outs[1]
