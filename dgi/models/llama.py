@@ -124,13 +124,31 @@ def _ss_cols(hidden: int) -> int:
     return (hidden // 256 + 7) // 8 * 8
 
 
-class LlamaLayerWeights:
+class _Looked:
+    __slots__ = ("_plain",)      # not among a layer's weights
+
+
+class LlamaLayerWeights(_Looked):
     __slots__ = ("in_norm", "qkv", "o", "post_norm", "gate_up", "down", "qkv_bias")
 
     def __init__(self, in_norm, qkv, o, post_norm, gate_up, down, qkv_bias=None):
         self.in_norm, self.qkv, self.o = in_norm, qkv, o
         self.post_norm, self.gate_up, self.down = post_norm, gate_up, down
         self.qkv_bias = qkv_bias   # [qkv_size] for Qwen2, else None (fused into the QKV GEMM epilogue)
+
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        object.__setattr__(self, "_plain", None)
+
+    def plain(self, dtype) -> bool:
+        """Whether all weights are whole rows of ``dtype`` at 16-byte boundaries: looked up once after any is assigned (the look costs some
+        200 us a step of 80 layers)."""
+        if self._plain is None:
+            ts = [t for t in (getattr(self, k) for k in LlamaLayerWeights.__slots__) if t is not None]
+            kinds = {t.dtype for t in ts}
+            ok = len(kinds) == 1 and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in ts)
+            object.__setattr__(self, "_plain", (kinds.pop() if ok else None,))
+        return self._plain[0] == dtype
 
 
 def _rand(shape, gen, device, dtype, std):
@@ -464,8 +482,7 @@ class LlamaModel:
             return False
         L = self.layers[0]
         return (ops.stream_ok(h, L.qkv) and L.gate_up.shape[0] % 16 == 0 and L.o.shape[1] % 64 == 0 and L.down.shape[1] % 64 == 0
-                and all(t.is_contiguous() and t.dtype == h.dtype and t.data_ptr() % 16 == 0
-                        for K in self.layers for t in (K.qkv, K.o, K.gate_up, K.down, K.in_norm, K.post_norm, K.qkv_bias) if t is not None))
+                and all(K.plain(h.dtype) for K in self.layers))
 
     def _forward_layers_stream(self, h: torch.Tensor, meta: AttnMeta, residual: Optional[torch.Tensor],
                                trim_last: Optional[torch.Tensor]):

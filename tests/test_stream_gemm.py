@@ -5,7 +5,7 @@ import torch
 
 from dgi import ops
 from dgi.models.config import get_config
-from dgi.models.llama import LlamaModel
+from dgi.models.llama import LlamaLayerWeights, LlamaModel
 from dgi.runtime.batch import AttnMeta
 
 BF16, F64 = torch.bfloat16, torch.float64
@@ -204,3 +204,40 @@ def test_a_step_takes_them_and_replays(monkeypatch):
         outs.append([r.output for r in reqs])
     assert "add_rmsnorm_parts" in names and "rope_cache_parts" in names
     assert outs[0] == outs[1]
+
+
+def test_weights_are_looked_at_once(monkeypatch):
+    """The look at every weight of every layer is not repeated at each step, but is after a weight is replaced."""
+    looks = []
+
+    class Weight:
+        dtype = BF16
+
+        def __init__(self, *shape, at=0):
+            self.shape, self.at = shape, at
+
+        def is_contiguous(self):
+            looks.append(self)
+            return True
+
+        def data_ptr(self):
+            return self.at
+
+    def layer():
+        return LlamaLayerWeights(Weight(2048), Weight(3072, 2048), Weight(2048, 2048), Weight(2048), Weight(8192, 2048), Weight(2048, 4096))
+
+    monkeypatch.setattr(ops, "stream_ok", lambda x, w: True)
+    m = LlamaModel.__new__(LlamaModel)
+    m.reduce, m.capture_layers, m.layers = None, (), [layer() for _ in range(3)]
+    h = torch.zeros(20, 2048, dtype=BF16)
+    assert m._stream_ok(h) and len(looks) == 18
+    assert m._stream_ok(h) and not m._stream_ok(h.float()) and len(looks) == 18
+    m.layers[1].down = Weight(2048, 4096, at=8)
+    assert not m._stream_ok(h)
+    m.layers[1].down = Weight(2048, 4096)
+    assert m._stream_ok(h)
+    m.layers[2].qkv_bias = Weight(3072)
+    m.layers[2].qkv_bias.dtype = torch.float32
+    assert not m._stream_ok(h)
+    m.layers[2] = layer()
+    assert m._stream_ok(h)
