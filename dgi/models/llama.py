@@ -487,7 +487,7 @@ class LlamaModel:
     def _forward_layers_stream(self, h: torch.Tensor, meta: AttnMeta, residual: Optional[torch.Tensor],
                                trim_last: Optional[torch.Tensor]):
         """Layers of few rows: qkv, o and down leave fp32 parts that the rotary, the norms (and their residual adds) sum up as they
-        read them, gate_up has SwiGLU as its epilogue: seven kernels a layer beside the attention's.  Rounded where ``forward_layers``
+        read them, gate_up has SwiGLU as its epilogue where that is the faster: seven kernels a layer beside the attention's.  Rounded where ``forward_layers``
         rounds; its contract."""
         c = self.cfg
         eps = c.rms_eps
@@ -507,8 +507,8 @@ class LlamaModel:
             if trim_last is not None and i == len(self.layers) - 1:
                 attn, residual = attn.index_select(0, trim_last), residual.index_select(0, trim_last)
             x = ops.add_rmsnorm_parts(ops.stream_parts(attn, L.o), residual, L.post_norm, eps)
-            # past 96 rows the rows of x are read so often that only the narrower weights gain
-            act = ops.stream_glu(x, L.gate_up) if x.shape[0] <= 96 or x.shape[1] <= 4096 else ops.silu_mul(ops.linear(x, L.gate_up))
+            act = ops.stream_glu(x, L.gate_up) if ops.glu_streams(x.shape[0], L.gate_up.shape[0] // 2, x.shape[1]) else \
+                ops.silu_mul(ops.linear(x, L.gate_up))
             parts = ops.stream_parts(act, L.down)
             if self.layer_hook is not None:
                 self.layer_hook(self.layer_start + i)

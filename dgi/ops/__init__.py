@@ -543,10 +543,43 @@ def plain_values(*tensors) -> bool:
     return True
 
 
+def _rounds_filled(units: int) -> float:
+    """How much of the chip's rounds units of 128 weight rows fill, one to a compute unit."""
+    return units / (-(-units // 256) * 256)
+
+
 def _stream_sizes(M: int, N: int, K: int) -> bool:
-    """Where ``linear`` is the faster as a streaming product: outputs that fill the chip by themselves up to 96 rows, narrow and large
-    weights (96 MB; the sum over the parts is a launch of its own) up to 128."""
-    return M <= STREAM_MAX_M and (M <= 96 if N >= 160 * 128 else N * K >= 48 << 20)
+    """Where ``linear`` is the faster as a streaming product.  Time of the vendor's product over this one's at 32, 64, 80, 96 rows:
+
+    * whole rows (N >= 20480).  One round of the chip: 28672 x 5120 1.06, 1.10, 1.36, 1.00; but a poorly filled one reads too slowly past
+      64 rows, 20480 x 3584 1.10, 1.15, 1.00, 0.95 (x 512 1.43 to 1.24).  Several, three quarters full at least: 50304 x 3584 1.07, 1.07,
+      0.98, 1.02, not 37888 x 3584 0.92, 0.98, 0.84, 0.87; past 64 rows full ones of up to 4096 of K: 128256 x 4096 1.23, 1.17, 1.10, 1.08, not
+      65536 x 5120 1.09, 1.07, 0.98, 0.94.
+    * narrower ones of 96 MB and more in parts, whose sum is a launch of its own.  Three parts and more, at 64 and 128 rows: 10240 x 5120 1.23,
+      1.14, 4096 x 14336 1.43, 2.07.  Two 16384 x 4608 1.09, 1.02, but 16384 x 3584 1.02, 0.93.  One 18944 x 3584 1.04, 0.80."""
+    if M > STREAM_MAX_M:
+        return False
+    if N >= 160 * 128:
+        units = -(-N // 128)
+        fill = _rounds_filled(units)
+        if units <= 256:
+            return M <= 64 or (M <= 96 and (fill >= 0.85 or K <= 2048))
+        return fill >= 0.75 and (M <= 64 or (M <= 96 and fill >= 0.9 and K <= 4096))
+    if N * K < 48 << 20:
+        return False
+    parts = stream_part_count(N, K)
+    return M <= 64 or parts >= 3 or (parts == 2 and N * K >= 64 << 20)
+
+
+def glu_streams(M: int, I: int, K: int) -> bool:
+    """Where gate_up and SwiGLU of up to 128 rows are the faster as ``stream_glu`` (units of 64 outputs).  Time of the vendor's product and
+    ``silu_mul`` over its, at 32, 64, 96, 128 rows: 13824 x 5120 1.11, 1.09, 1.04, 1.09, 8960 x 3584 (140 units) 1.23, 1.19, 1.07, 1.05,
+    8192 x 4096 (128) 1.17, 1.06, 0.93, 0.88, 4096 x 2048 (64) 1.07, 0.89, 0.76, 0.74; several rounds of the chip: 28672 x 8192 1.19, 1.17,
+    1.02, 0.93, 26624 x 5120 0.99, 1.01, 0.93, 0.93, not 18944 x 3584 (296 units) 0.98, 0.98, 0.94, 0.89."""
+    units = -(-I // 64)
+    if units > 256:
+        return M <= 64 and _rounds_filled(units) >= 0.75
+    return M <= (128 if units >= 140 else 64 if units >= 88 else 32)
 
 
 def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:

@@ -241,3 +241,18 @@ def test_weights_are_looked_at_once(monkeypatch):
     assert not m._stream_ok(h)
     m.layers[2] = layer()
     assert m._stream_ok(h)
+
+
+def test_sizes_that_stream():
+    """Rounds of the chip that are mostly idle, wide rows many times over and parts of two large pieces stay with the vendor's product."""
+    rows = lambda N, K: [M for M in (17, 64, 65, 96, 97, 128, 129) if ops._stream_sizes(M, N, K)]  # noqa: E731
+    assert rows(37888, 3584) == rows(34816, 4096) == rows(45056, 5120) == []
+    assert rows(65536, 5120) == rows(20480, 3584) == rows(128256, 8192) == rows(17408, 5120) == rows(16384, 3584) == [17, 64]
+    assert rows(32000, 8192) == rows(128256, 4096) == rows(20480, 512) == [17, 64, 65, 96]
+    assert rows(4096, 14336) == rows(16384, 4096) == rows(520, 98304) == [17, 64, 65, 96, 97, 128]
+    assert rows(4096, 4096) == []
+    glu = lambda I, K: [M for M in (1, 32, 33, 64, 65, 96, 97, 128) if ops.glu_streams(M, I, K)]  # noqa: E731
+    assert glu(18944, 3584) == glu(17408, 5120) == []
+    assert glu(14336, 4096) == glu(13824, 5120) == glu(8960, 1536) == [1, 32, 33, 64, 65, 96, 97, 128]
+    assert glu(8192, 4096) == glu(28672, 8192) == glu(24576, 6144) == [1, 32, 33, 64]
+    assert glu(4096, 2048) == [1, 32]
