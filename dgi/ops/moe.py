@@ -180,6 +180,16 @@ def group_tile(pairs: int, experts: int, weights: int) -> int:
     return 16 if mean <= 4 else 32
 
 
+def expert_tile(pairs: int, experts: int, W: int, ff: int) -> int:
+    """``group_tile`` for experts of widths W and ff.  Widths that are no multiples of 64, whose weights go through LDS stages in tiles of up to 64,
+    take tiles of 128 from a mean of 25 pairs on where those give every compute unit work: 16 experts of 2040 x 2040 mean 28 130 us against 132, 36
+    136 against 142; 8 of 4104 x 3592 mean 36 231 against 236; but 16 of 1000 x 1000 mean 36 62 against 50, 4 of 1032 x 4104 106 against 62."""
+    tile = group_tile(pairs, experts, W * ff)
+    if tile == 64 and (W % 64 or ff % 64) and pairs > 24 * experts and experts * W >= 32000:
+        return 128
+    return tile
+
+
 def moe_experts(h, idx, wts, gate_up, down, shared=None, act: str = "silu", limit: float = 0.0, alpha: float = 1.702,
                 weigh: str = "output") -> torch.Tensor:
     """sum_k route_{idx[t, k]}(h_t) weighed by wts[t, k] on the output or (``weigh="input"``) on the
@@ -200,7 +210,7 @@ def moe_experts(h, idx, wts, gate_up, down, shared=None, act: str = "silu", limi
         mid = torch.empty(P, ff, dtype=h.dtype, device=h.device)
         ys = torch.empty(P, W, dtype=h.dtype, device=h.device)        # places past the last real route are never read
         if T > 0:
-            tile = group_tile(P, E, W * ff)
+            tile = expert_tile(P, E, W, ff)
             kind = 1 if act == "clamped" else 0
             _call("moe_plan_group", mid, order, where, seg, idx, h, gate_up, None if w_in is None else w_in.reshape(-1), top, kind,
                   float(limit), float(alpha), tile)

@@ -104,3 +104,10 @@ def test_plan_of_many_pairs(P, E, skip):
     n = pairs.numel()
     assert torch.equal(order[:n].cpu().long(), pairs) and (order[n:] == -7).all()
     assert torch.equal(where.cpu().long()[pairs], torch.arange(n))
+
+
+def test_tiles_of_ragged_widths():
+    assert [moe.expert_tile(16 * m, 16, 2040, 2040) for m in (20, 24, 25, 40, 41)] == [32, 64, 128, 128, 128]
+    assert [moe.expert_tile(16 * m, 16, 2048, 2048) for m in (24, 25, 40, 41)] == [64, 64, 64, 128]
+    assert moe.expert_tile(16 * 36, 16, 1000, 1000) == moe.expert_tile(4 * 36, 4, 1032, 4104) == 64
+    assert moe.expert_tile(8 * 36, 8, 4104, 3592) == moe.expert_tile(8 * 36, 8, 4096, 4104) == 128
