@@ -741,14 +741,17 @@ __global__ __launch_bounds__(128) void masked_attn_reduce_kernel(const float* __
 
 template <int R, int D>
 void launch_tiles_dims(const RowsArgs& a, int rows, int G, int nsplit, hipStream_t s) {
-  // a workgroup per compute unit or fewer: eight waves each (30 rows of 2000 keys, 8 groups of 4 heads of 64 dims: 14.9 us, with four
+  // A workgroup per compute unit or fewer: eight waves each (30 rows of 2000 keys, 8 groups of 4 heads of 64 dims: 14.9 us, with four
   // waves 16.8); more of them: four, so that more workgroups share a unit (128 rows of 500 keys, groups of 2: 30.4, with eight 30.9).
-  // From 256 on cached rows are marked as read once (32 rows of 2000 keys 56 us -> 54.4, 128 of 500 59 -> 55.5); smaller steps, whose
-  // rows the caches may still hold, gain nothing (4 rows of 300 keys 12.2, marked 12.7)
+  // Where nearly all units have work to the end, cached rows are marked as read once (8 groups of 4 heads of 128 dims, us marked and not: 32
+  // rows of 2000 keys 54.9, 56.6, 31 rows 54.2, 55.8, 64 of 1000 52.2, 54.3, 100 of 300 30.6, 32.2).  Where some wait for others, each
+  // reads faster without the mark (20 rows of 2000 49.0, 44.2, 28 of 1000 28.0, 27.3; 36 rows of 2000, 64 heads 93.8, 85.4, 40 of 64 dims 47.7,
+  // 43.6), and smaller steps' rows the caches may still hold (4 rows of 300 11.9, 11.4).
   const long long units = (long long)rows * G * nsplit;
   const dim3 grid(rows, G, nsplit);
-  if (units > 256) masked_attn_tiles_kernel<R, D, 4, true><<<grid, 256, 0, s>>>(a);
-  else if (units == 256) masked_attn_tiles_kernel<R, D, 8, true><<<grid, 512, 0, s>>>(a);
+  if (units >= 448) masked_attn_tiles_kernel<R, D, 4, true><<<grid, 256, 0, s>>>(a);
+  else if (units > 256) masked_attn_tiles_kernel<R, D, 4, false><<<grid, 256, 0, s>>>(a);
+  else if (units >= 240) masked_attn_tiles_kernel<R, D, 8, true><<<grid, 512, 0, s>>>(a);
   else masked_attn_tiles_kernel<R, D, 8, false><<<grid, 512, 0, s>>>(a);
 }
 

@@ -97,3 +97,12 @@ def test_an_infinite_value_at_the_row_s_own_position(n):
     args = (table.cuda(), None, pos.cuda(), 2, 1, 0.125)
     got = mix.masked_attn_rows(q.cuda(), kc.cuda(), vc.cuda(), *args)
     assert torch.isposinf(got.view(2, 2, 64)[0, :, 5]).all() and int(torch.isfinite(got).sum()) == got.numel() - 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [119, 120, 128, 129, 223, 224])
+def test_workgroups_around_the_lines_of_the_launch(rows):
+    """Two groups: 238 to 448 workgroups, of eight waves and four, cached rows marked as read once and not."""
+    ctx = [1 + (53 * i) % 260 for i in range(rows)]
+    q, kc, vc, table, pos, gate = case(ctx, 8, 2, 64, 64, 16, rows)
+    check(q, kc, vc, table, pos, 8, 2, 0, gate)
