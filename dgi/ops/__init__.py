@@ -614,10 +614,12 @@ def tile_gemm(M: int, N: int) -> bool:
 
 
 def split_gemm(M: int, N: int, K: int) -> bool:
-    """Whether a product of long rows, 129 to 512 of them, is better split along K by ``mfma_gemm`` (8192 x 28672, vendor's product and
-    this one, us: 129 rows 309, 173; 200 311, 185; 256 323, 195; 353 197, 195; 512 310, 201; but 640 264, 310; 4096 x 14336 at
-    200 60, 98)."""
-    return 128 < M <= 512 and K >= 16384 and N * K >= 1 << 27
+    """Whether a product of long rows, 129 to 512 of them, is better split along K by ``mfma_gemm``: where its tiles of 256 x 256 give 96 to 256
+    blocks in four pieces.  Vendor's product and this one, us, at 129 / 256 / 353 / 512 rows: 8192 x 28672 299, 197 / 312, 195 / 199, 196 / 315, 201; 6144 x
+    24576 184, 166 / 279, 172 / 215, 170 / 285, 175; 8192 x 16384 94, 130 / 157, 139 / 129, 126 / 160, 128.  Not 4096 x 32768 up to 256 rows (64 blocks:
+    160, 187 / 191, 194), 16384 x 53248 from 257 on (two pieces: 257 rows 508, 635), 640 rows of 8192 x 28672 (264, 310)."""
+    tiles = -(-M // 256) * (N // 256)
+    return 128 < M <= 512 and K >= 16384 and N * K >= 1 << 27 and 24 <= tiles <= 64 and (M > 160 or K >= 24576)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,

@@ -195,3 +195,11 @@ def test_split_products_of_two_streams():
         got.zero_()
         graph.replay()
         assert torch.equal(got, want) and torch.equal(ops.mfma_gemm(x, w), want)
+
+
+def test_rows_that_are_split():
+    """Four pieces of 24 to 64 tiles; short sums of few rows stay with the vendor's product."""
+    split = lambda N, K: [M for M in (129, 160, 161, 256, 257, 512) if ops.split_gemm(M, N, K)]  # noqa: E731
+    assert split(8192, 28672) == split(6144, 24576) == [129, 160, 161, 256, 257, 512]
+    assert split(8192, 16384) == [161, 256, 257, 512] and split(16384, 16384) == [161, 256] and split(16384, 53248) == [129, 160, 161, 256]
+    assert split(4096, 32768) == [257, 512] and split(5120, 27648) == [257, 512]
