@@ -604,13 +604,18 @@ def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:
 
 
 def tile_gemm(M: int, N: int) -> bool:
-    """Whether ``linear`` runs on the ping-pong kernel (``mfma_gemm``, whole tiles: its split-K workspace belongs to one stream at a
-    time): the logits of large vocabularies for 129 to 1024 rows, where the tiles nearly fill whole rounds of the chip.  Vendor's product
-    and this one, us, at 129 / 256 / 353 / 512 / 1024 rows: 128256 x 4096 289, 224 / 299, 235 / 433, 398 / 510, 402 / 860, 766; x 8192
-    527, 465 / 541, 451 / 813, 765 / 975, 786 / 1710, 1471.  Narrower ones are the vendor's: 32000 x 4096 64, 80 / 74, 85 / 88,
-    101; 57344 x 8192 192, 204 / 218, 220 / 313, 363."""
+    """Rows and outputs whose tiles nearly fill whole rounds of the chip on the ping-pong kernel (``mfma_gemm``, whole tiles: its split-K
+    workspace belongs to one stream at a time): large vocabularies and 129 to 1024 rows.  ``linear`` takes it where ``tile_pays`` too."""
     tiles = -(-M // 256) * (N // 256)
     return 128 < M <= 1024 and N >= 384 * 256 and 8 * tiles >= 7 * -(-tiles // 256) * 256
+
+
+def tile_pays(M: int, N: int) -> bool:
+    """Where the vendor's product is the slower of the two: outputs that are no multiple of 512, the last rows more than a third of a tile.  Its
+    time over this one's at 129, 256, 300, 353, 400, 512, 1024 rows: 128256 x 4096 1.32, 1.15, 0.92, 1.04, 1.18, 1.16, 1.07, 115968 x 3584 1.32, 1.25,
+    0.97, 1.06, 1.20, 1.23, 0.95, 256256 x 2048 1.26, 1.16, 0.84, 0.94, 1.11, 1.12, 1.02; but 128512 x 3584 0.90, 0.93, 0.78, 0.87, 0.98, 0.96, 0.91,
+    131072 x 2304 0.95, 0.90, 0.85, 0.89, -, 0.93, 0.94."""
+    return N % 512 == 256 and (M - 1) % 256 >= 96
 
 
 def split_gemm(M: int, N: int, K: int) -> bool:
@@ -636,12 +641,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _call("skinny_gemm", out, x, w, bias, _skinny_cfg(M, N))
         return out
-    if x.is_cuda and M <= 1024 and (_stream_sizes(M, N, K) or tile_gemm(M, N)) and plain_values(x, w, bias, out):
+    if x.is_cuda and M <= 1024 and (_stream_sizes(M, N, K) or (tile_gemm(M, N) and tile_pays(M, N))) and plain_values(x, w, bias, out):
         if _stream_sizes(M, N, K):
             y = _linear_stream(x, w, bias, out)
             if y is not None:
                 return y
-        if (tile_gemm(M, N) and bias is None and out is None and w.dim() == 2 and w.shape[1] == K and w.device == x.device
+        if (tile_gemm(M, N) and tile_pays(M, N) and bias is None and out is None and w.dim() == 2 and w.shape[1] == K and w.device == x.device
                 and w.data_ptr() % 16 == 0 and mfma_gemm_ok(x, w) and load_native(False)):
             return mfma_gemm(x, w, streamk=1)
     r = torch.nn.functional.linear(x, w, bias)

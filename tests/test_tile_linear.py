@@ -203,3 +203,17 @@ def test_rows_that_are_split():
     assert split(8192, 28672) == split(6144, 24576) == [129, 160, 161, 256, 257, 512]
     assert split(8192, 16384) == [161, 256, 257, 512] and split(16384, 16384) == [161, 256] and split(16384, 53248) == [129, 160, 161, 256]
     assert split(4096, 32768) == [257, 512] and split(5120, 27648) == [257, 512]
+
+
+@pytest.mark.gpu
+def test_linear_leaves_outputs_in_whole_vendor_tiles(monkeypatch):
+    """The ping-pong kernel only where it is the faster: outputs that are no multiple of 512, rows that fill a third of their last tile."""
+    calls = []
+    real = ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    for M, N, want in [(129, 501 * 256, True), (353, 501 * 256, True), (352, 501 * 256, False), (257, 501 * 256, False), (512, 1001 * 256, True),
+                       (200, 512 * 256, False), (512, 500 * 256, False), (129, 592 * 256, False)]:
+        x, w = torch.randn(M, 64, device="cuda").bfloat16(), torch.randn(N, 64, device="cuda").bfloat16()
+        calls.clear()
+        ops.linear(x, w)
+        assert calls == (["mfma_gemm"] if want else []), (M, N)
