@@ -6,8 +6,8 @@
 // the paged pool written by rope_cache.hip.
 //
 // Work decomposition (CDNA4, wave64):
-//   grid = (n_kv_heads, batch, max_splits), 8 waves, or 4 where there are more
-//   workgroups than compute units.
+//   grid = (n_kv_heads, batch, max_splits), 8 waves, or 4 where rows and kv heads
+//   (fixed parts: splits too) alone are more workgroups than compute units.
 //   A workgroup owns one (sequence, kv-head, KV split) and all G = nh/nkv
 //   query heads of that kv head, so each K/V byte is read from HBM once per
 //   decode step regardless of the GQA ratio.
@@ -22,7 +22,7 @@
 //   directly from the accumulator registers; V^T comes from a per-wave LDS
 //   tile through ds_read_b64_tr_b16 (hardware transpose) with an XOR swizzle
 //   that makes the transposed reads bank-conflict free.
-//   The 4 waves merge (m, l, O) through LDS; with more than one split the
+//   The waves merge (m, l, O) through LDS; with more than one split the
 //   partial results (normalised O and log2-sum-exp) go to a workspace and
 //   either the last-arriving split of each (sequence, kv head) combines them
 //   in the same launch (ticket counters in the workspace: write-through

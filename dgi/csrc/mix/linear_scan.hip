@@ -433,8 +433,10 @@ __device__ __forceinline__ float tree_sum(F&& at) {
   return x[0];
 }
 
-// States are read and written once a step, and the other layers' come in between: marked so, the chip's caches give them up first (32 rows of 64 heads
-// of 64 x 64, four layers: wkv 77.5 us -> 64.1, delta 86.5 -> 66.7, mlstm 84.5 -> 70, gla 80 -> 61.5; 8 rows of 16 heads 21.9 -> 21.0).
+// States are read and written once a step, and the other layers' come in between: marked so, the chip's caches give them up first.  32 rows of 64
+// heads of 64 x 64, us a layer: sixteen layers (540 MB of states, more than the caches hold) wkv 18.6 -> 15.2, delta 21.0 -> 16.1, mlstm 20.5 -> 16.8,
+// gla 19.5 -> 14.5.  Where the caches hold them there is little to gain: four layers, the same states again and again, 16.6 -> 15.7, 18.6 -> 17.0,
+// 17.4 -> 17.5, 15.2 -> 15.4; four layers of wkv right after something else wrote the states 78.8 and 78.8 in all.
 __device__ __forceinline__ float4 ld_state(const float* p) {
   const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
   return make_float4(v[0], v[1], v[2], v[3]);

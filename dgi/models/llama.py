@@ -3,13 +3,17 @@
 Replaces the HF modules the reference executes (worker/engines/llm.py:22-69,
 worker/distributed/model_shard.py:28-246).  Per layer the step runs
 
-    fused_add_rmsnorm (HIP) -> QKV GEMM (hipBLASLt) -> RoPE + paged KV write (HIP)
-    -> paged decode / prefill attention (HIP, MFMA) -> O GEMM
-    -> fused_add_rmsnorm (HIP) -> gate|up GEMM -> SiLU*mul (HIP) -> down GEMM
+    fused_add_rmsnorm -> QKV GEMM -> RoPE + paged KV write -> paged decode / prefill attention
+    -> O GEMM -> fused_add_rmsnorm -> gate|up GEMM -> SiLU*mul -> down GEMM
 
-with fused QKV and gate|up weights so each layer issues 4 GEMMs.  Qwen2's biased
-q/k/v projections ride in the QKV GEMM's bias epilogue (hipBLASLt), so the
-family adds no kernel; GLM-4 adds biased QKV and half-dim interleaved RoPE
+with fused QKV and gate|up weights, in one of four forms by the step's rows
+(``forward_layers``): up to 16 with norm, rotary and SwiGLU inside the products
+(``_forward_layers_fused``); up to 128 on products that stream their weights and leave
+partial sums to the norm or the rotary (``_forward_layers_stream``); larger steps of models
+with a routing table on MFMA products with the norm in their epilogue
+(``_forward_layers_folded``); all others as above, with the library's or our own
+products.  Qwen2's biased q/k/v projections ride in the QKV GEMM's bias epilogue or
+in the rotary's sums, so the family adds no kernel; GLM-4 adds biased QKV and half-dim interleaved RoPE
 (``rope_cache`` mode 1 over the first ``rotary_dim`` dims).  A model
 object may hold any contiguous layer range (pipeline stage): stage 0 owns the
 embedding, the last stage the final norm and LM head, exactly like the

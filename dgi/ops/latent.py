@@ -196,7 +196,7 @@ def split_runs(rows: int, heads: int, max_keys: int) -> int:
 
 def tile_runs(rows: int, heads: int, max_keys: int) -> int:
     """Runs of keys per row for the tile kernel (512 + 64 dims): its workgroups take a row, up to 32 heads and one run, one
-    to a compute unit (two tiles are most of its LDS), so as many as fill the 256 of them, every run at least two 64-key tiles
+    to a compute unit (its four tiles of 32 keys are nearly all of the LDS), so as many as fill the 256 of them, every run at least 128 keys
     long.  32 rows of 32 heads over 2000 keys: 8 runs 29 us and 8 to combine them."""
     if max_keys <= 0 or rows <= 0:
         return 1

@@ -127,7 +127,7 @@ def test_rows_without_a_position(gated, max_keys):
 @pytest.mark.parametrize("H", [4, 32])
 def test_contexts_around_the_tiles(H):
     """Contexts around tiles of 32 keys and what is loaded ahead of them, runs without keys, and rows without a position whose pages are
-    nobody's, against the same rows one by one in a single run."""
+    nobody's, against the same rows one by one in a single run, and those against 64 bits."""
     g = torch.Generator().manual_seed(H)
     pos = [0, 14, 30, 31, 32, 62, 63, 64, 95, 96, 127, 128, 300, -1, 2049]
     T, dim, vdim, dev = len(pos), 64, 32, "cuda"
@@ -146,6 +146,7 @@ def test_contexts_around_the_tiles(H):
         return out.float()
 
     many = run(list(range(T)), 1 << 14)
+    wide, kinds = cache.cpu(), [x.cpu().to(F64) for x in (uk, uv)]
     for i, p in enumerate(pos):
         if p < 0:
             assert (many[i] == 0).all()
@@ -153,3 +154,12 @@ def test_contexts_around_the_tiles(H):
         one = run([i], 0)[0]
         # weights relative to another maximum, sums and the head's value rounded to bf16
         assert (many[i] - one).abs().max() <= 2.0 ** -7 * one.abs().max()
+        rows = wide[tables[i].long().cpu(), 0].reshape(-1, KR + RD)[: p + 1].to(F64)
+        qi = q[i].cpu().view(H, dim + RD)
+        qr = latent.rotate_ref(qi[None, :, dim:].float(), cs[p: p + 1].cpu(), RD, True)[0].to(BF16).to(F64)
+        folded = torch.einsum("hd,hdk->hk", qi[:, :dim].to(F64), kinds[0]).to(BF16).to(F64)
+        w = torch.softmax((folded @ rows[:, :KR].t() + qr @ rows[:, KR:].t()) * 0.08, 1)
+        want = torch.einsum("hk,hvk->hv", w @ rows[:, :KR], kinds[1]).reshape(-1)
+        # both roundings that move a score (the folded query, a rotated value between two bf16 numbers) are the reference's up to their ties; the
+        # values and the result are rounded once each
+        assert ((one.cpu().to(F64) - want).norm() / want.norm()) <= 2.0 ** -6, p

@@ -179,9 +179,14 @@ def test_layers_compose_on_the_cpu(monkeypatch):
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,prompts", [(17, []), (64, []), (100, []), (9, [20, 1, 33]), (0, [70])])
 def test_layers_on_the_gpu(monkeypatch, T, prompts):
-    assert real_stream_ok is not None
+    names, real = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (names.append(name), real(name, *a))[1])
     plain, stream = layers("cuda", T, prompts, monkeypatch, hidden_size=2048, intermediate_size=4160, num_heads=16, num_kv_heads=4)
     close(stream, plain)
+    # both forms ran, one after the other
+    first = names.index("rope_cache_parts")
+    assert "rope_cache" in names[:first] and "add_rmsnorm_parts" not in names[:first]
+    assert names[first:].count("rope_cache_parts") == 2 and "rope_cache" not in names[first:] and names[first:].count("add_rmsnorm_parts") == 3
 
 
 @pytest.mark.gpu
