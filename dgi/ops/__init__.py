@@ -543,6 +543,11 @@ def plain_values(*tensors) -> bool:
     return True
 
 
+def _device_is_current(t: torch.Tensor) -> bool:
+    """Kernels go to the current device's stream, torch's own operations to their operands' device."""
+    return t.is_cuda and t.device.index == torch.cuda.current_device()
+
+
 def _rounds_filled(units: int) -> float:
     """How much of the chip's rounds units of 128 weight rows fill, one to a compute unit."""
     return units / (-(-units // 256) * 256)
@@ -635,13 +640,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     M, K = x.shape
     N = w.shape[0]
     if (x.is_cuda and _use_skinny(M, N, K) and x.dtype == torch.bfloat16
-            and w.dtype == torch.bfloat16 and plain_values(x, w, bias, out) and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.is_contiguous() and load_native(False)):     # a process that built only another kernel group keeps the vendor GEMM
+            and w.dtype == torch.bfloat16 and plain_values(x, w, bias, out) and _device_is_current(x) and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and w.is_contiguous() and load_native(False)):     # a process that built only another kernel group keeps the vendor GEMM
         if out is None:
             out = torch.empty(M, N, dtype=x.dtype, device=x.device)
         _call("skinny_gemm", out, x, w, bias, _skinny_cfg(M, N))
         return out
-    if x.is_cuda and M <= 1024 and (_stream_sizes(M, N, K) or (tile_gemm(M, N) and tile_pays(M, N))) and plain_values(x, w, bias, out):
+    if (x.is_cuda and M <= 1024 and (_stream_sizes(M, N, K) or (tile_gemm(M, N) and tile_pays(M, N))) and plain_values(x, w, bias, out)
+            and _device_is_current(x)):
         if _stream_sizes(M, N, K):
             y = _linear_stream(x, w, bias, out)
             if y is not None:
@@ -956,7 +962,7 @@ def row_sumsq(x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     statistics the fused-norm GEMM reads for a stream no residual epilogue produced (the
     first layer's input)."""
     if (x.is_cuda and x.dtype == torch.bfloat16 and out.dtype == torch.float32 and out.device == x.device and out.dim() == 2
-            and x.shape == (out.shape[0], x.shape[1]) and plain_values(x, out) and x.shape[1] % 8 == 0 and x.stride(1) == 1
+            and x.shape == (out.shape[0], x.shape[1]) and plain_values(x, out) and _device_is_current(x) and x.shape[1] % 8 == 0 and x.stride(1) == 1
             and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and out.stride(1) == 1 and load_native(False)):
         _call("row_sumsq", out, x)
         return out

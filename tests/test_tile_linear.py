@@ -217,3 +217,21 @@ def test_linear_leaves_outputs_in_whole_vendor_tiles(monkeypatch):
         calls.clear()
         ops.linear(x, w)
         assert calls == (["mfma_gemm"] if want else []), (M, N)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(8, 4096, 1024), (64, 20480, 64), (128, 4096, 12288), (200, 501 * 256, 64)])
+def test_operands_of_another_device(monkeypatch, M, N, K):
+    """Kernels are launched on the current device: operands of another one stay with torch's product, which goes to theirs."""
+    calls = []
+    monkeypatch.setattr(ops, "_call", lambda name, *a: calls.append(name))
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), torch.randn(N, K, device="cuda").bfloat16()
+    ops.linear(x, w)
+    assert calls
+    calls.clear()
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
+    y = ops.linear(x, w)
+    ops.row_sumsq(x, torch.empty(M, 2, device="cuda"))
+    assert not calls
+    ref = x.float() @ w.float().t()
+    assert ((y.float() - ref).norm() / ref.norm()) <= 2.0 ** -8
