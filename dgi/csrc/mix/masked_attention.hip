@@ -647,10 +647,14 @@ __global__ __launch_bounds__(64 * NW, R == 8 ? 2 : 3) void masked_attn_tiles_ker
     }
     // only a wave's last tile can end early: what is there instead of its missing values may be infinite, and 0 times that is no number
     const int n = pos - (first + tile * 64) + 1;
+    if (n < 64) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int x = 0; x < VB; ++x) raw[u][x] = 16 * u + KL * x + lg < n ? raw[u][x] : zero;
+    }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-#pragma unroll
-      for (int x = 0; x < VB; ++x) raw[u][x] = 16 * u + KL * x + lg < n ? raw[u][x] : zero;
       add_v(u);
       __builtin_amdgcn_sched_barrier(0);
     }
