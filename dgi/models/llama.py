@@ -164,6 +164,8 @@ def _rand(shape, gen, device, dtype, std):
 class LlamaModel:
     """Layer range [layer_start, layer_end) of a Llama causal LM."""
 
+    decode_splits = True        # decode attention follows the step's plan of splits (``AttnMeta.dec_max_splits``)
+
     def __init__(self, cfg: ModelConfig, device: torch.device | str = "cpu", dtype=torch.bfloat16,
                  layer_start: int = 0, layer_end: Optional[int] = None, has_embed: Optional[bool] = None,
                  has_head: Optional[bool] = None, seed: int = 0, init: str = "random",

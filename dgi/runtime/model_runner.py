@@ -451,6 +451,8 @@ class GraphRunner:
             return 0
         if b <= self.short_max_b:
             return self.short_ctx
+        if not getattr(self.r.model, "decode_splits", False):
+            return 0
         splits, part = self.split_plan(b)
         return ops.decode_whole(b, c.num_kv_heads, self.r.num_cus) if splits > 1 and part < 0 else 0
 

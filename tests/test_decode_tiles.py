@@ -86,7 +86,7 @@ def test_captured_plans_serve_short_contexts(monkeypatch):
     for limit in (1024, 2048, 8192, 131072):
         r = GraphRunner.__new__(GraphRunner)
         cfg = SimpleNamespace(num_kv_heads=8, head_dim=128)
-        r.r = SimpleNamespace(model=SimpleNamespace(cfg=cfg), num_cus=256, max_model_len=limit, ws_splits=limit // 128)
+        r.r = SimpleNamespace(model=SimpleNamespace(cfg=cfg, decode_splits=True), num_cus=256, max_model_len=limit, ws_splits=limit // 128)
         r.short_ctx, r.short_max_b = 384, 8
         assert [r.short_limit(b) for b in (1, 8, 9, 16)] == [384, 384, 0, 0]
         for b in (17, 24, 32, 40, 48, 64, 512):
@@ -95,6 +95,8 @@ def test_captured_plans_serve_short_contexts(monkeypatch):
             assert whole in (1024, 2048, 8192) and (splits > 1) == (limit > whole)
             assert r.short_limit(b) == (whole if splits > 1 else 0)
             assert ops.decode_split_plan(b, whole, 8)[0] == 1 and ops.decode_split_plan(b, whole + 1, 8)[0] > 1
+        r.r.model.decode_splits = False                  # models whose attention has no such plan
+        assert [r.short_limit(b) for b in (8, 24, 64)] == [384, 0, 0]
         r.short_ctx = 0
         assert not any(r.short_limit(b) for b in (1, 24, 64))
 
