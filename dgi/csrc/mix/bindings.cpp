@@ -68,7 +68,8 @@ int dgi_causal_conv(void* out, int out_f32, const void* x, int x_f32, int x_stri
 int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const void* dt_raw, int dt_f32, int dt_stride,
                  const float* dt_bias, const float* a_log, const float* d_skip, float* state, const int* positions,
                  const int* seq_row0, const int* seq_slots, int n_seq, int heads, int dv, int N, int G, int chunked, int segs,
-                 int seg_rows, float* ws, float* wsd, hipStream_t s);
+                 int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t s);
+long long dgi_ssm_parts_floats(int dk, int H, int G, int T, int n_seq, int* chunks);
 int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg_rows);
 int dgi_gated_group_norm(void* out, int out_f32, const float* y, const void* z, int z_f32, int z_stride, const float* w,
                          int T, int C, int groups, float eps, hipStream_t s);
@@ -498,8 +499,14 @@ void ssm_scan(at::Tensor y, const at::Tensor& xbc, const at::Tensor& dt_raw, con
   check_f32(dt_bias, "dt_bias", heads); check_f32(a_log, "a_log", heads); check_f32(d_skip, "d_skip", heads);
   const int n_seq = (int)seq_slots.numel();
   int segs = 1, seg_rows = 0;
-  at::Tensor ws, wsd;
-  if (chunked && n_seq > 0) segs = dgi_ssm_segments(n_seq, (int)heads, (int)dv, T, &seg_rows);
+  int parts_chunks = 0;
+  at::Tensor ws, wsd, parts;
+  if (chunked && n_seq > 0) {
+    segs = dgi_ssm_segments(n_seq, (int)heads, (int)dv, T, &seg_rows);
+    // what the heads of a group share (chunk_parts.hip)
+    const long long floats = G > 0 ? dgi_ssm_parts_floats((int)N, (int)heads, (int)G, T, n_seq, &parts_chunks) : 0;
+    if (floats > 0) parts = at::empty({floats}, state.options());
+  }
   if (segs > 1) {
     TORCH_CHECK((int64_t)segs * seg_rows >= T, "ssm_scan: the segments must cover the longest portion");
     ws = at::empty({n_seq, segs, heads, dv, N}, state.options());
@@ -509,7 +516,8 @@ void ssm_scan(at::Tensor y, const at::Tensor& xbc, const at::Tensor& dt_raw, con
                         (int)dt_raw.stride(0), dt_bias.data_ptr<float>(), a_log.data_ptr<float>(), d_skip.data_ptr<float>(),
                         state.data_ptr<float>(), i32p(positions, "positions", T), i32p(seq_row0, "seq_row0", n_seq + 1),
                         i32p(seq_slots, "seq_slots"), n_seq, (int)heads, (int)dv, (int)N, (int)G, chunked, segs, seg_rows,
-                        segs > 1 ? ws.data_ptr<float>() : nullptr, segs > 1 ? wsd.data_ptr<float>() : nullptr, cur_stream()), "ssm_scan");
+                        segs > 1 ? ws.data_ptr<float>() : nullptr, segs > 1 ? wsd.data_ptr<float>() : nullptr,
+                        parts.defined() ? parts.data_ptr<float>() : nullptr, parts_chunks, cur_stream()), "ssm_scan");
 }
 
 void gated_group_norm(at::Tensor out, const at::Tensor& y, const at::Tensor& z, const at::Tensor& w, int64_t groups,

@@ -1,12 +1,13 @@
 // dgi/csrc/mix/chunk_scan.hip — prompt portions of the recurrences that carry a matrix S [dk, dv] per head (linear_scan.hip has
-// their definitions, ssm_scan.hip that of ssm), sixteen tokens at a time in fp32 matrix products (v_mfma_f32_16x16x4_f32).
+// their definitions, ssm_scan.hip that of ssm), sixteen tokens at a time in fp32 matrix products (v_mfma_f32_16x16x4_f32).  Those that chunk_parts.hip
+// takes (light; mlstm, but for fp32 rows of more than 64 channels; ssm of groups of four heads) go there.
 //
 // For tokens t, s of a chunk that starts from the state S, with D[t, s] the product of the decays of the tokens after s up to t
 // and A_t that of all tokens up to t:
 //
 //     o_t = A_t S^T q_t + sum_(s <= t) P[t, s] u_s,   P[t, s] = D[t, s] (q_t . k_s) c_s          S <- A_15 S + sum_s D[15, s] c_s k_s u_s^T
 //
-// light: u = v, c = 1;  ssm: q = C, k = B, u = x, c = dt;  mlstm: c = the input gate, o divided by the normaliser;
+// ssm: q = C, k = B, u = x, c = dt;  mlstm: c = the input gate, o divided by the normaliser;
 // wkv: the decays are per key channel, so they sit inside the products: q_t and k_s are scaled by the decays between them and
 // the middle of the chunk (so chunk halves, not chunks, have to stay in the fp32 range), the state products use prefix and suffix
 // products and no division;  it reads before it writes: s < t, and the bonus on the diagonal;
@@ -29,74 +30,32 @@
 // by k, substitution, update) or a preparing wave's arithmetic (wkv): a wave issues an instruction every four to five cycles at best, so
 // addresses are lane offsets kept in registers, and rows past the end a branch of their own.  Measured, a step of 2 prompts of 4096 rows in
 // all, 64 heads, states 64 x 64 (ssm 128 x 64), against the same token by token on the vector ALUs (linear_scan.hip, ssm_scan.hip):
-// delta 178 us (726), ssm 209 (637), wkv 232 (some 630), light 158 (chunk_scan_decay.hip: 214); mlstm, 5 prompts of 3001 rows, 32 heads: 83 (322; 103 in two column blocks a workgroup).
+// delta 178 us (726), ssm 199 (637), wkv 232 (some 630).
 //
 // Precision: results and states are no further from 64 bits than the token loop's (2-norm over 1300 to 4096 rows: ssm 7.8e-8, the loop 8.0e-8;
 // delta 1.17e-7, 1.18e-7; wkv 9.8e-8, 1.01e-7; but states of wkv on bf16 rows 7.34e-8, 7.28e-8: the loop's products of bf16 keys and values
 // are exact, here a decayed key is rounded).  Regrouping alone does not do that: with the sums over channels in two running sums, P and the decays
 // rounded product by product and P u in 32 bits the same were 1.25e-7, 1.57e-7 and 1.30e-7.  So sums over channels are added as trees, a sum over
 // tokens starts with the oldest, the per-token decays and wkv's suffix products carry their rounding errors along, and P and P u are 64-bit
-// (four v_mfma_f64_16x16x4_f64 per chunk and output wave).  It costs 3 (delta) to 13 % (mlstm) of the time; wkv's was not the longest role.
+// (four v_mfma_f64_16x16x4_f64 per chunk and output wave).  It costs 3 % of delta's time; wkv's was not the longest role.
 //
 // Half-chunk products of channel decays below 1e-28, or q and k so large or small that their scaled values leave the fp32 range: the wave that
 // prepares such channels sums their scores token by token instead.  An infinity or NaN among a chunk's u takes a path that keeps it from the tokens
 // before it (a matrix product multiplies it by their zeros).  A portion at position 0 reads no state.
 #include <type_traits>
-#include "../common.h"
+#include "chunk_args.h"
 
 using namespace dgi;
 
 namespace {
 
-constexpr int WKV = 0, DELTA = 1, MLSTM = 2, LIGHT = 4, SSM = 5;      // 3: gla, chunk_scan_decay.hip
 constexpr int C = 16;              // tokens per chunk
 constexpr int TR = 20, PR = 18;    // padded rows of sixteen tokens; in 64 bits
 constexpr float SAFE = 1e-28f;
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
-struct ChunkArgs {
-  float* y;                        // [T, H * dv]
-  const void *q, *k, *v;           // rows with their own strides (elements); wkv: q the receptance; ssm: C, B, x
-  int q_stride, k_stride, v_stride;
-  const void *aux1, *aux2;         // per token: w_raw [T, H*dk] | b_raw | i_raw | - | dt_raw;  - | a_raw | f_raw | - | -
-  int aux1_stride, aux2_stride, aux_bf16;
-  const float *par1, *par2, *par3; // w0 | a_log | - | decay [H] | a_log;  u | dt_bias | - | - | dt_bias;  ssm: d_skip
-  float *state, *norm, *mx;        // state [slots, H, dk, dv] (ssm: [slots, H, dv, dk])
-  float *norm_new, *mx_new;        // mlstm with several workgroups per head: staged, as in linear_scan
-  const int *positions, *seq_row0, *seq_slots;
-  int H, G, dk, dv;
-  int n_seq;
-  int pass, seg_rows;              // ssm in segments: 0 whole portions, 1 and 2 the two passes
-  float *ws, *wsd;                 // [n_seq, segments, H, dv, dk] states, [n_seq, segments, H] decays
-  int skip_rows;                   // sequences of at most this many rows are not this launch's
-  float cap;
-};
-
-template <typename T> __device__ __forceinline__ float ldf(const T* p);
-template <> __device__ __forceinline__ float ldf<float>(const float* p) { return *p; }
-template <> __device__ __forceinline__ float ldf<uint16_t>(const uint16_t* p) { return bf16_to_f32(*p); }
-__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float silu(float x) { return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f)); }
 __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
-__device__ __forceinline__ float logsigmoid_f(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
-__device__ __forceinline__ bool finite(float x) { return fabsf(x) < __builtin_inff(); }
-
-// four consecutive elements as they lie in memory
-template <typename T> struct Raw4;
-template <> struct Raw4<float> { float4 v; };
-template <> struct Raw4<uint16_t> { uint2 v; };
-__device__ __forceinline__ void widen(const Raw4<float>& r, float* f) { f[0] = r.v.x; f[1] = r.v.y; f[2] = r.v.z; f[3] = r.v.w; }
-__device__ __forceinline__ void widen(const Raw4<uint16_t>& r, float* f) {
-  f[0] = __uint_as_float(r.v.x << 16); f[1] = __uint_as_float(r.v.x & 0xffff0000u);
-  f[2] = __uint_as_float(r.v.y << 16); f[3] = __uint_as_float(r.v.y & 0xffff0000u);
-}
-
-// the largest magnitude (fmaxf would first bring its operands into canonical form: three instructions)
-__device__ __forceinline__ float larger3(float m, float a, float b) {
-  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a), "v"(b));
-  return m;
-}
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
@@ -134,7 +93,7 @@ __device__ __forceinline__ float sum16(const float* v, int lane) {
 template <int MODE, int NT, int COLS>
 struct Lay {
   static constexpr bool CH = MODE == WKV;                      // decays per key channel
-  static constexpr bool TURNS = CH || MODE == LIGHT;           // two sets of preparing waves take turns, two steps a chunk
+  static constexpr bool TURNS = CH;                            // two sets of preparing waves take turns, two steps a chunk
   static constexpr int NC = COLS / 16, W2 = NT <= 8 ? 2 : 1;         // column blocks, scores waves
   static constexpr int NS = NT / 4;                            // preparing waves of 64 channels
   static constexpr int NA = NT == 4 ? 4 : 8;                   // sums side by side of a sum over the channels: state waves
@@ -175,26 +134,25 @@ struct Lay {
 // over the tokens starts with the oldest, which under a decay are the small ones.
 __device__ __forceinline__ constexpr int place(int t) { return 4 * (t & 3) + (t >> 2); }      // its own inverse
 
-// Whether workgroups of four column blocks are there for a kernel: not where its waves (thirteen, so 128 registers each) would spill (ssm, wkv, mlstm
-// on fp32 rows or over 128 channels: 1 prompt of 1000 and 5 decode rows, 64 heads, 219 us -> 268), or its LDS would not suffice.
-template <int MODE, typename TI, int NT>
+// Whether workgroups of four column blocks are there for a kernel: not where its waves (thirteen, so 128 registers each) would spill (ssm, wkv, mlstm:
+// 1 prompt of 1000 and 5 decode rows, 64 heads, 219 us -> 268), or its LDS would not suffice.
+template <int MODE, int NT>
 constexpr bool has_four() {
-  return MODE == LIGHT || (NT == 4 && (MODE == DELTA || (MODE == MLSTM && sizeof(TI) == 2)));
+  return NT == 4 && MODE == DELTA;
 }
 
 // Steps whose workgroups of two column blocks do not find a compute unit each: four blocks share what does not depend on the columns
 // (q, k, gates, scores), at SLOW hundredths of two blocks' time per chunk.  Only the lengths say which is the faster (decode rows and short portions
 // take no place for long), so the workgroups decide: all chunks over 256 units and a part of the longest sequence's for the last round, or the longest
 // sequence's if that is more.  seq, the seq-th longest before, becomes the sequence itself.
-//   us before (two blocks, sequences in their order) and now, 64-wide heads       mlstm        light       delta
-//   5 prompts of 3001 bf16 rows in all, 32 heads                                  104, 84      95, 80      97, 91
-//   12 prompts of 4000, 64 heads                                                  198, 140     176, 130    173, 158
-//   9 prompts of 1500, 32 heads                                                   62, 54       56, 50      51, 54
-//   1 prompt of 2048 and 3 decode rows, 64 heads (stays at two blocks)            172, 167     147, 150    242, 157
+//   us before (two blocks, sequences in their order) and now, 64-wide heads       delta
+//   5 prompts of 3001 bf16 rows in all, 32 heads                                  97, 91
+//   12 prompts of 4000, 64 heads                                                  173, 158
+//   9 prompts of 1500, 32 heads                                                   51, 54
+//   1 prompt of 2048 and 3 decode rows, 64 heads (stays at two blocks)            242, 157
 constexpr int MOST_SEQ = 16;       // more would be decode rows mostly, whose workgroups should be gone soon
-template <int MODE, int NT>
 __device__ __forceinline__ bool four_blocks(const ChunkArgs& a, int& seq, int& row0, int& n) {
-  constexpr int SLOW = MODE == DELTA ? 150 : MODE == MLSTM ? 130 : NT == 4 ? 135 : 155;
+  constexpr int SLOW = 150;
   const int lane = threadIdx.x & 63, i = min(lane, a.n_seq - 1);
   const int from = a.seq_row0[i], len = lane < a.n_seq ? max(a.seq_row0[i + 1] - from, 0) : -1;
   int before = 0;                                    // sequences that are longer, or as long and earlier
@@ -228,7 +186,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
   int seq = blockIdx.x / a.H % a.n_seq, blocks = L::NC;      // blocks: of columns, this workgroup's
   int row0, n;
   if constexpr (COLS == 64) {
-    blocks = four_blocks<MODE, NT>(a, seq, row0, n) ? 4 : 2;       // the same in every workgroup
+    blocks = four_blocks(a, seq, row0, n) ? 4 : 2;       // the same in every workgroup
     if (zb * blocks * 16 >= a.dv) return;            // the grid is that of two blocks each
   } else {
     row0 = a.seq_row0[seq];
@@ -305,32 +263,32 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
       }
       auto load_d = [&](int c) {
         const int first = min(c * C, n - 1);
-        const char* p = db + (size_t)first * a.aux1_stride * 4;
+        global_in p = (global_in)db + (size_t)first * a.aux1_stride * 4;
         asm volatile("" : "+s"(p));
         if (first + C <= n) {
 #pragma unroll
-          for (int t = 0; t < C; ++t) rd[t] = *reinterpret_cast<const float*>(p + vd[t]);
+          for (int t = 0; t < C; ++t) rd[t] = gload<float>(p + vd[t]);
         } else {
 #pragma unroll
-          for (int t = 0; t < C; ++t) rd[t] = *reinterpret_cast<const float*>(p + ((unsigned)min(t, n - 1 - first) * a.aux1_stride * 4u + od));
+          for (int t = 0; t < C; ++t) rd[t] = gload<float>(p + ((unsigned)min(t, n - 1 - first) * a.aux1_stride * 4u + od));
         }
       };
       auto load_qk = [&](int c) {
         const int first = min(c * C, n - 1);
-        const char *q = (const char*)(qb + (size_t)first * a.q_stride), *k = (const char*)(kb + (size_t)first * a.k_stride);
+        global_in q = (global_in)(qb + (size_t)first * a.q_stride), k = (global_in)(kb + (size_t)first * a.k_stride);
         asm volatile("" : "+s"(q), "+s"(k));
         if (first + C <= n) {
 #pragma unroll
           for (int t = 0; t < C; ++t) {
-            rq[t] = *reinterpret_cast<const TI*>(q + vq[t]);
-            rk[t] = *reinterpret_cast<const TI*>(k + vk[t]);
+            rq[t] = gload<TI>(q + vq[t]);
+            rk[t] = gload<TI>(k + vk[t]);
           }
         } else {
 #pragma unroll
           for (int t = 0; t < C; ++t) {
             const unsigned r = (unsigned)min(t, n - 1 - first) * (unsigned)sizeof(TI);
-            rq[t] = *reinterpret_cast<const TI*>(q + (r * a.q_stride + oq));
-            rk[t] = *reinterpret_cast<const TI*>(k + (r * a.k_stride + oq));
+            rq[t] = gload<TI>(q + (r * a.q_stride + oq));
+            rk[t] = gload<TI>(k + (r * a.k_stride + oq));
           }
         }
       };
@@ -454,7 +412,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
       const unsigned vq = (unsigned)t * a.q_stride * (unsigned)sizeof(TI), vk = (unsigned)t * a.k_stride * (unsigned)sizeof(TI);
       auto load = [&](int c, int st) {
         const int first = min(c * C, n - 1);
-        const char *pq = (const char*)(qb + (size_t)first * a.q_stride), *pk = (const char*)(kb + (size_t)first * a.k_stride);
+        global_in pq = (global_in)(qb + (size_t)first * a.q_stride), pk = (global_in)(kb + (size_t)first * a.k_stride);
         asm volatile("" : "+s"(pq), "+s"(pk));
         unsigned oq = vq, ok = vk;
         if (first + C > n) {
@@ -464,8 +422,8 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          rq[st][i] = *reinterpret_cast<const Raw4<TI>*>(pq + (oq + vx[i]));
-          rk[st][i] = *reinterpret_cast<const Raw4<TI>*>(pk + (ok + vx[i]));
+          rq[st][i] = gload<Raw4<TI>>(pq + (oq + vx[i]));
+          rk[st][i] = gload<Raw4<TI>>(pk + (ok + vx[i]));
         }
       };
       float q[4][4], k[4][4];
@@ -474,10 +432,6 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
         for (int i = 0; i < 4; ++i) {
           widen(rq[st][i], q[i]);
           widen(rk[st][i], k[i]);
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            if (MODE == LIGHT) q[i][x] = silu(q[i][x]);
-          }
         }
         if (n - c * C < C || dk < DP) {                      // rows past the portion, channels past dk: zeros
           const bool ok = c * C + t < n;
@@ -492,12 +446,6 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
         }
       };
       auto put = [&](int c) {
-        if constexpr (MODE == LIGHT) {                       // zeros stay zeros
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int x = 0; x < 4; ++x) k[i][x] = silu(k[i][x]);
-        }
         float* Q = sm + L::Q + (c % L::QB) * L::ROWS + t * QR + 64 * w + 4 * j;
         float* K = sm + L::K + (c % L::KB) * L::ROWS + place(t) * QR + 64 * w + 4 * j;
 #pragma unroll
@@ -700,7 +648,6 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
       float ga = 0.f, gb = 0.f;                      // raw gates of the next 64 tokens
       float p1 = 0.f, p2 = 0.f;
       if constexpr (MODE == DELTA || MODE == SSM) { p1 = -expf(a.par1[head]); p2 = a.par2[head]; }
-      if constexpr (MODE == LIGHT) p1 = a.par1[head];
       float m_run = 0.f, m_old = 0.f, m_new = 0.f, x = 0.f, z = 0.f;       // mlstm: running maximum, input gate, forget gate
       if constexpr (MODE == MLSTM) {
         if (stored) m_run = a.mx[(size_t)slot * H + head];
@@ -719,9 +666,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
       // 3: to LDS
       auto gates = [&](int b, int phase) {
         if (phase == 0) {
-          if constexpr (MODE == LIGHT) {
-            x = p1;
-          } else if constexpr (MODE == SSM) {
+          if constexpr (MODE == SSM) {
             x = softplus_f(ga + p2);
             z = expf(p1 * x);
           } else if constexpr (MODE == DELTA) {
@@ -762,8 +707,8 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
           // decay | write factor | mlstm: exp(-maximum), delta: write strength; tokens past the portion: no decay, nothing written
           const bool ok = b * 64 + lane < n;
           float* G = sm + L::GT + (b & 1) * 192 + lane;
-          G[0] = !ok ? 1.f : (MODE == LIGHT ? x : (MODE == MLSTM ? expf(z + m_old - m_new) : z));
-          G[64] = !ok ? 0.f : (MODE == LIGHT ? 1.f : (MODE == MLSTM ? expf(x - m_new) : x));
+          G[0] = !ok ? 1.f : (MODE == MLSTM ? expf(z + m_old - m_new) : z);
+          G[64] = !ok ? 0.f : (MODE == MLSTM ? expf(x - m_new) : x);
           G[128] = !ok ? 0.f : (MODE == MLSTM ? expf(-m_new) : x);
         }
       };
@@ -777,7 +722,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
           low = fmaf(low, d, fmaf(A, d, -next));
           A = next;
         };
-        auto product = [&]() { return MODE == LIGHT && !finite(A) ? A : A + low; };      // light: decays of any size
+        auto product = [&]() { return A + low; };
 #pragma unroll
         for (int i = 3; i > 0; --i) {                  // the tokens behind this lane's four, up to t
           const float4 d4 = ld4(G + 4 * i);
@@ -887,15 +832,15 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
   for (int r = 0; r < 4; ++r) vv[r] = (unsigned)(tok(r) * a.v_stride + colc) * (unsigned)sizeof(TI);
   auto load_v = [&](int c, int st) {
     const int first = min(c * C, n - 1);
-    const char* p = (const char*)(vb + (size_t)first * a.v_stride);
+    global_in p = (global_in)(vb + (size_t)first * a.v_stride);
     asm volatile("" : "+s"(p));
     if (first + C <= n) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) rv[st][r] = *reinterpret_cast<const TI*>(p + vv[r]);
+      for (int r = 0; r < 4; ++r) rv[st][r] = gload<TI>(p + vv[r]);
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        rv[st][r] = *reinterpret_cast<const TI*>(p + (unsigned)(min(tok(r), n - 1 - first) * a.v_stride + colc) * (unsigned)sizeof(TI));
+        rv[st][r] = gload<TI>(p + (unsigned)(min(tok(r), n - 1 - first) * a.v_stride + colc) * (unsigned)sizeof(TI));
     }
   };
   auto take_v = [&](int c, int st, float* u) {
@@ -904,10 +849,6 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
     if ((c + 1) * C > n) {                           // rows past the portion
 #pragma unroll
       for (int r = 0; r < 4; ++r) u[r] = c * C + tok(r) < n ? u[r] : 0.f;
-    }
-    if constexpr (MODE == LIGHT) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) u[r] = silu(u[r]);
     }
     load_v(c + 2, st);
   };
@@ -1076,17 +1017,17 @@ __global__ __launch_bounds__((64 * Lay<MODE, NT, COLS>::WAVES), 2) void chunk_sc
       if constexpr (MODE == MLSTM) out[r] *= F[32 + r];
       if constexpr (MODE == SSM) out[r] += skip * u[r];
     }
-    char* yc = (char*)(yb + (size_t)c * C * H * dv);
+    global_out yc = (global_out)(yb + (size_t)c * C * H * dv);
     asm volatile("" : "+s"(yc));
     if (left >= C) {
       if (cok) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) *reinterpret_cast<float*>(yc + vy[r]) = out[r];
+        for (int r = 0; r < 4; ++r) gstore(yc + vy[r], out[r]);
       }
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (cok && tok(r) < left) *reinterpret_cast<float*>(yc + vy[r]) = out[r];
+        if (cok && tok(r) < left) gstore(yc + vy[r], out[r]);
     }
     __syncthreads();
   };
@@ -1132,12 +1073,12 @@ int launch_one(const ChunkArgs& a, dim3 grid, hipStream_t st) {
 template <int MODE, typename TI>
 int launch_dims(const ChunkArgs& a, bool four, dim3 grid, hipStream_t st) {
   if (a.dk <= 64) {
-    if constexpr (has_four<MODE, TI, 4>())
+    if constexpr (has_four<MODE, 4>())
       if (four) return launch_one<MODE, TI, 4, 64>(a, grid, st);
     return launch_one<MODE, TI, 4, 32>(a, grid, st);
   }
   if (a.dk <= 128) {
-    if constexpr (has_four<MODE, TI, 8>())
+    if constexpr (has_four<MODE, 8>())
       if (four) return launch_one<MODE, TI, 8, 64>(a, grid, st);
     return launch_one<MODE, TI, 8, 32>(a, grid, st);
   }
@@ -1161,17 +1102,17 @@ extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, 
   return dk % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && (((uintptr_t)q | (uintptr_t)k) & piece) == 0;
 }
 
-// mode as above (light: par1 the decays; ssm: q = C, k = B, v = x, aux1 = dt_raw (aux_bf16), par1 a_log, par2 dt_bias, par3 d_skip).
+// mode as above (and light: par1 the decays; ssm: q = C, k = B, v = x, aux1 = dt_raw (aux_bf16), par1 a_log, par2 dt_bias, par3 d_skip).
 // Needs dgi_chunk_scan_ok.  skip_rows: sequences of at most that many rows are left to another launch.  segs > 1 (ssm): portions are
-// cut into segments of seg_rows rows (a multiple of 16, segs of them at least as long as the longest portion) that run side by side: each one's
+// cut into segments of seg_rows rows (a multiple of 32, segs of them at least as long as the longest portion) that run side by side: each one's
 // state from nothing, a short serial pass over those states, then the outputs from each segment's incoming state.  About
-// twice the work, for steps whose heads leave most of the chip idle.
+// twice the work, for steps whose heads leave most of the chip idle.  parts (ssm): dgi_ssm_parts_floats of workspace for chunk_parts.hip, or null.
 extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                               int v_stride, int in_f32, const void* aux1, int aux1_stride, const void* aux2, int aux2_stride,
                               int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
                               float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
-                              int segs, int seg_rows, float* ws, float* wsd, hipStream_t st) {
+                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st) {
   if (n_seq == 0) return 0;
   const int cols = dk <= 128 ? 32 : 16;            // value columns of a workgroup (or twice as many, see four_blocks)
   const long long nz = (dv + cols - 1) / cols;
@@ -1186,24 +1127,26 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
   a.positions = positions; a.seq_row0 = seq_row0; a.seq_slots = seq_slots;
   a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.skip_rows = skip_rows;
   if (n_seq * nz * H > 0x3fffffff || segs > 65535 || (segs > 1 && (mode != SSM || !ws || !wsd || seg_rows <= 0))) return -3;
-  a.n_seq = n_seq; a.seg_rows = seg_rows; a.ws = ws; a.wsd = wsd;
+  a.n_seq = n_seq; a.seg_rows = seg_rows; a.ws = ws; a.wsd = wsd; a.parts = parts; a.parts_chunks = parts_chunks;
   a.pass = segs > 1 ? 1 : 0;
   const dim3 grid((unsigned)(n_seq * nz * H), segs > 1 ? segs : 1);
   // more workgroups than compute units: possibly of four column blocks each
   const bool four = dv > 32 && n_seq <= MOST_SEQ && n_seq * nz * H > 256;
+  const bool by_parts = mode == SSM ? parts != nullptr : dgi_chunk_parts_takes(mode, dk, in_f32);
+  if (mode == SSM && parts && segs > 1 && seg_rows % 32) return -3;
   if (a.pass) {
-    int rc = launch_dims<SSM, float>(a, false, grid, st);
+    int rc = by_parts ? dgi_chunk_parts(a, mode, in_f32, grid, st) : launch_dims<SSM, float>(a, false, grid, st);
     if (rc) return rc;
     ssm_segments_kernel<<<dim3(n_seq, H, (dk * dv + 255) / 256), 256, 0, st>>>(ws, wsd, state, positions, seq_row0, seq_slots, H, dk * dv, segs,
                                                                                seg_rows, skip_rows);
     a.pass = 2;
   }
   int rc = -2;
-  switch (mode) {
+  if (by_parts) rc = dgi_chunk_parts(a, mode, in_f32, grid, st);
+  else switch (mode) {
     case WKV: rc = launch_mode<WKV>(a, in_f32, four, grid, st); break;
     case DELTA: rc = launch_mode<DELTA>(a, in_f32, four, grid, st); break;
-    case MLSTM: rc = launch_mode<MLSTM>(a, in_f32, four, grid, st); break;
-    case LIGHT: rc = launch_mode<LIGHT>(a, in_f32, four, grid, st); break;
+    case MLSTM: rc = in_f32 && dk > 64 ? launch_one<MLSTM, float, 8, 32>(a, grid, st) : -2; break;
     case SSM: rc = in_f32 ? launch_dims<SSM, float>(a, false, grid, st) : -2; break;
   }
   if (rc) return rc;

@@ -1124,7 +1124,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
                               float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
-                              int segs, int seg_rows, float* ws, float* wsd, hipStream_t st);
+                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st);
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 extern "C" int dgi_chunk_scan_decay(float* y, int light, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                                    int v_stride, int in_f32, const float* decay, int decay_stride, float* state,
@@ -1139,11 +1139,12 @@ constexpr int APART_FROM = 8;        // sequences of a step above which those ar
 // token loops are long, still gain (72 rows, 16 portions, 64 heads of 64: 99 -> 70 and 113 -> 94 us).  wkv's loop is short, and once the
 // workgroups (16 columns) outnumber the places its pipelines find on the chip they also wait for each other (64-wide heads; units, rows, this
 // file's time, chunk_scan.hip's: 256, 72, 23, 19 us; 1024, 100, 38, 44; 2816, 140, 144, 140; 4096, 140, 154, 185; 128-wide heads: 2048, 72,
-// 90, 103; 4096, 100, 362, 335).  light is up against chunk_scan_decay.hip (512 units, 300 rows: 33, 29; 704, 200: 37, 41; 1408, 200: 64, 60;
-// 256, 231: 21, 24).
+// 90, 103; 4096, 100, 362, 335).  light is up against chunk_scan_decay.hip (that one's time and chunk_parts.hip's: 256 units, 100 rows 11, 12; 160 rows 14,
+// 13; 400 rows 31, 25; 512 units, 100 rows 16, 12; 1024 units, 64 rows 20, 17; 2048 units, 64 rows 36, 35; 128-wide heads: 128 units, 100 rows 15, 15;
+// 1024 units, 64 rows 30, 25; 4096 units, 64 rows 108, 91).
 static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
   const long units = (long)n_seq * H * ((dv + 15) / 16);
-  if (mode == LIGHT) return units > 768 ? 160 : units > 256 ? 320 : 1l << 40;
+  if (mode == LIGHT) return units > 256 ? 64 : 128;
   if (mode != WKV || units <= 512) return 64;
   return dk > 64 ? 104 : units <= 3072 ? 136 : 224;
 }
@@ -1198,7 +1199,7 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   if ((mode == LIGHT && !par1) || (mode != LIGHT && !aux1)) return -4;
   bool short_rows = rows <= 4 * n_seq;             // rows of the step: at most four per sequence on average
   const bool staged = mode == MLSTM && norm_new && mx_new;
-  // Prompt portions: sixteen tokens at a time on the matrix cores (chunk_scan.hip).  Among many sequences there are decode
+  // Prompt portions: sixteen tokens at a time on the matrix cores (chunk_scan.hip, chunk_parts.hip).  Among many sequences there are decode
   // rows and short portions beside the long ones: they stay with this kernel, in a launch of their own.
   const int form = chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows);
   const int apart = n_seq > APART_FROM && (form == 1 || (form == 2 && rows <= 4 * n_seq))
@@ -1206,7 +1207,7 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   if (form) {
     const int rc = form == 1 ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
                                               aux2, aux2_stride, 0, par1, par2, nullptr, cap, state, norm, mx, norm_new, mx_new, positions,
-                                              seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, 0, nullptr, nullptr, st)
+                                              seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, 0, nullptr, nullptr, nullptr, 0, st)
                              : dgi_chunk_scan_decay(y, mode == LIGHT, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? par1 : aux1,
                                                    mode == LIGHT ? 0 : aux1_stride, state, positions, seq_row0, seq_slots, n_seq, H, dk, dv,
                                                    apart, st);

@@ -264,7 +264,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
                               float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
-                              int segs, int seg_rows, float* ws, float* wsd, hipStream_t st);
+                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st);
 
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 
@@ -292,7 +292,7 @@ extern "C" int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg
   if (groups <= 0 || groups > 128 || rows - n_seq + 1 < 512) return 1;
   const long places = 256 - (n_seq - 1) * one;
   const long share = std::max({64l, (rows * one + places - 1) / places, (rows + 23l) / 24});
-  const int each = (int)((share + 15) / 16 * 16), segs = (rows + each - 1) / each;
+  const int each = (int)((share + 31) / 32 * 32), segs = (rows + each - 1) / each;
   if (segs < 3) return 1;
   *seg_rows = each;
   return segs;
@@ -301,7 +301,8 @@ extern "C" int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg
 extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const void* dt_raw, int dt_f32, int dt_stride,
                             const float* dt_bias, const float* a_log, const float* d_skip, float* state,
                             const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int heads,
-                            int dv, int N, int G, int chunked, int segs, int seg_rows, float* ws, float* wsd, hipStream_t s) {
+                            int dv, int N, int G, int chunked, int segs, int seg_rows, float* ws, float* wsd, float* parts,
+                            int parts_chunks, hipStream_t s) {
   if (n_seq == 0) return 0;
   if (G <= 0 || heads % G) return -2;
   if (N > 256 || N <= 0 || dv <= 0) return -3;
@@ -312,7 +313,7 @@ extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const vo
     most = apart_rows(n_seq, heads, dv);
     const int rc = dgi_chunk_scan(y, 5, B + (size_t)G * N, xbc_stride, B, xbc_stride, xbc, xbc_stride, 1, dt_raw, dt_stride, nullptr, 0,
                                   !dt_f32, a_log, dt_bias, d_skip, 0.f, state, nullptr, nullptr, nullptr, nullptr, positions, seq_row0,
-                                  seq_slots, n_seq, heads, G, N, dv, most, segs, seg_rows, ws, wsd, s);
+                                  seq_slots, n_seq, heads, G, N, dv, most, segs, seg_rows, ws, wsd, parts, parts_chunks, s);
     if (rc || !most) return rc;
   }
   const int nq = (N + 63) / 64;

@@ -1,0 +1,82 @@
+"""Prompt portions in chunks of 32 tokens on the bf16 matrix cores (dgi/csrc/mix/chunk_parts.hip): lengths around a chunk and around the 64 tokens
+whose gates are made together, key and value sizes around its tiles, state-space groups (what their heads share is prepared in a pass of its own), segments,
+and values that are not finite, which leave the matrix cores and go token by token.
+
+Tolerance: as test_chunk_scan's, 3e-5 of the largest output."""
+import pytest
+import torch
+
+from test_chunk_scan import F64, call, check, make, oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def run(d):
+    return call(d, **({"chunked": True} if d["mode"] == "ssm" else {}))
+
+
+def heads(mode, V):
+    return 8 if mode == "ssm" else 400 // -(-V // 16) + 1 if mode == "light" else 4      # light: enough workgroups for this kernel
+
+
+@pytest.mark.parametrize("mode", ["mlstm", "light", "ssm"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,V", [(64, 64), (4, 16), (36, 17), (100, 48), (128, 33)])
+@pytest.mark.parametrize("lens", [[97], [128, 65, 160, 31, 32, 33, 1], [95, 129]], ids=lambda x: "-".join(map(str, x)))
+def test_sizes(mode, dtype, D, V, lens):
+    if mode == "light":
+        lens = [n + 96 if n > 90 else n for n in lens]
+    d = make(mode, lens, heads(mode, V), D, V, dtype, [3 * (i % 2) for i in range(len(lens))], seed=D + V)
+    check(run(d), oracle(d))
+
+
+@pytest.mark.parametrize("H,D,lens", [(8, 128, [1500, 40]), (8, 60, [700]), (12, 64, [600, 0, 70])])
+def test_segments(H, D, lens):
+    """Few heads: segments (of whole chunks) side by side, with the prepared parts shared by both passes."""
+    for past in (0, 40):
+        d = make("ssm", lens, H, D, 24, torch.bfloat16, [past or (0 if n else 4) for n in lens], seed=H + D)      # an empty sequence keeps its state
+        check(run(d), oracle(d))
+
+
+def where_finite(got, want):
+    """The same values are finite, and they agree."""
+    for a, b in zip(got, want):
+        fa, fb = torch.isfinite(a), torch.isfinite(b)
+        assert torch.equal(fa, fb)
+        if fb.any():
+            assert (a[fa] - b[fb]).abs().max() <= 1e-4 * max(1.0, b[fb].abs().max().item())
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v", "gate", "state", "large"])
+@pytest.mark.parametrize("mode", ["mlstm", "ssm"])
+def test_not_finite(mode, what):
+    """Infinities and NaN in what a token brings, or in the state: the same results are finite as row by row.  Values too large for three parts."""
+    for bad in (float("inf"), float("nan")) if what != "large" else (3.39e38,):
+        d = make(mode, [130], 8, 64, 32, torch.float32, [3])
+        t = 71
+        if mode == "ssm":
+            G, x = d["G"], d["xbc"]
+            at = {"v": 3, "k": 8 * 32 + 5, "q": 8 * 32 + G * 64 + 5, "large": 8 * 32 + 5}.get(what)
+            if at is not None:
+                x[t, at] = bad
+        elif what in ("q", "k", "v", "large"):
+            d["k" if what == "large" else what][t, 5] = bad
+        if what == "gate":
+            (d["dt"] if mode == "ssm" else d["a"])[t, 2] = bad
+        if what == "state":
+            d["S"][1, 2, 3, 4] = bad
+        slow = call(d, chunked=False) if mode == "ssm" else call(dict(d, pad=1))
+        where_finite(run(d)[:2], slow[:2])
+
+
+def test_light_decays_that_are_none():
+    """Decays of 0, below 0 and above 1 (whose powers may leave the fp32 range)."""
+    d = make("light", [200], 104, 64, 32, torch.float32, [3])
+    d["par"][0][:6] = torch.tensor([0.0, -0.5, 1.0, 1.01, 1e-30, 100.0])
+    got, want = run(d), oracle(d)
+    for h in range(104):
+        g, w = got[0].view(200, 104, 32)[:, h].to(F64), want[0].view(200, 104, 32)[:, h]
+        for t in range(200):                                   # up to where a state of fp32 values would overflow
+            if w[t].abs().max() > 1e30:
+                break
+            assert (g[t] - w[t]).abs().max() <= 3e-5 * max(1.0, w[: t + 1].abs().max().item())
