@@ -33,7 +33,7 @@ extern "C" int dgi_paged_prefill_masked(const void* q, int q_stride, const void*
   if ((1 << bs_log2) != block_size) return -4;
   const float scale_log2 = scale * 1.4426950408889634f;
 #define DGI_PREFILL_MASKED(HDV_, BIASV, HDVV, PADV)                                                      \
-  prefill_attn_kernel<HDV_, 4, 1, true, BIASV, HDVV, PADV><<<n_tiles * nh, 256, 0, s>>>(              \
+  prefill_attn_kernel<HDV_, 4, true, BIASV, HDVV, PADV><<<n_tiles * nh, 256, 0, s>>>(              \
       (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables,     \
       bt_stride, cu_seqlens_q, context_lens, tiles, (uint16_t*)out, out_stride, nh, nkv, bs_log2,         \
       scale_log2, nullptr, 0, mask, (const uint16_t*)gate, gate_stride, dist_bias, n_dist, 1.f / scale,   \

@@ -42,20 +42,19 @@ extern "C" int dgi_paged_prefill(const void* q, int q_stride, const void* k_cach
   while ((1 << bs_log2) < block_size) ++bs_log2;
   if ((1 << bs_log2) != block_size) return -4;
   const float scale_log2 = scale * 1.4426950408889634f;
-  const int db = (tile_rows >> 16) & 1;          // bit 16: two LDS stages (prefill_attn_kernel DB)
   tile_rows &= 0xffff;
   if (tile_rows != 128 && tile_rows != 256) return -7;
-#define DGI_PREFILL(HDV, NWV, DBV)                                                                     \
-  prefill_attn_kernel<HDV, NWV, DBV><<<n_tiles * nh, NWV * 64, 0, s>>>(                           \
+#define DGI_PREFILL(HDV, NWV)                                                                          \
+  prefill_attn_kernel<HDV, NWV><<<n_tiles * nh, NWV * 64, 0, s>>>(                                \
       (const uint16_t*)q, q_stride, (const uint16_t*)k_cache, (const uint16_t*)v_cache, block_tables,     \
       bt_stride, cu_seqlens_q, context_lens, tiles, (uint16_t*)out, out_stride, nh, nkv, bs_log2,         \
       scale_log2, tree_mask, tree_n)
   if (hd == 128) {
-    if (tile_rows == 256) { if (db) DGI_PREFILL(128, 8, 1); else DGI_PREFILL(128, 8, 0); }
-    else { if (db) DGI_PREFILL(128, 4, 1); else DGI_PREFILL(128, 4, 0); }
+    if (tile_rows == 256) DGI_PREFILL(128, 8);
+    else DGI_PREFILL(128, 4);
   } else {
-    if (tile_rows == 256) { if (db) DGI_PREFILL(64, 8, 1); else DGI_PREFILL(64, 8, 0); }
-    else { if (db) DGI_PREFILL(64, 4, 1); else DGI_PREFILL(64, 4, 0); }
+    if (tile_rows == 256) DGI_PREFILL(64, 8);
+    else DGI_PREFILL(64, 4);
   }
 #undef DGI_PREFILL
   DGI_CHECK_LAUNCH();

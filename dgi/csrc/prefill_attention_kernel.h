@@ -24,21 +24,44 @@ namespace dgi {
 namespace prefill {
 
 
-// Element offset of 16-byte chunk `ch` of LDS row `row`.
+// Where the 16-byte chunk `ch` of an LDS row lies in it (and which chunk lies at `ch`), and its element offset.
 // HD=128 (256-B rows): K chunk ^ (row & 15) — 16 consecutive rows at one chunk
 // hit 16 distinct slots (ds_read_b128); V chunk ^ ((row & 3) << 2) for the
 // transposed reads.  HD=64 (128-B rows, two rows per 64-bank line): row & 1
 // already picks the bank half, so K XORs (row >> 1) & 7 and V shifts rows
 // 2-3 of each 4-row block by 4 chunks.
 template <int HD>
-__device__ __forceinline__ int k_off(int row, int ch) {
-  if constexpr (HD == 128) return row * 128 + (((ch) ^ (row & 15)) << 3);
-  else return row * 64 + (((ch) ^ ((row >> 1) & 7)) << 3);
+__device__ __forceinline__ int k_slot(int row, int ch) {
+  return HD == 128 ? ch ^ (row & 15) : ch ^ ((row >> 1) & 7);
 }
 template <int HD>
-__device__ __forceinline__ int v_off(int row, int ch) {
-  if constexpr (HD == 128) return row * 128 + (((ch) ^ ((row & 3) << 2)) << 3);
-  else return row * 64 + (((ch) ^ (((row >> 1) & 1) << 2)) << 3);
+__device__ __forceinline__ int v_slot(int row, int ch) {
+  return HD == 128 ? ch ^ ((row & 3) << 2) : ch ^ (((row >> 1) & 1) << 2);
+}
+template <int HD>
+__device__ __forceinline__ int k_off(int row, int ch) { return row * HD + (k_slot<HD>(row, ch) << 3); }
+template <int HD>
+__device__ __forceinline__ int v_off(int row, int ch) { return row * HD + (v_slot<HD>(row, ch) << 3); }
+
+// One 16-byte chunk a lane from memory to LDS (`at` + 16 lane)
+typedef __attribute__((address_space(3))) char* lds_ptr;
+__device__ __forceinline__ void load_chunk(const char* src, lds_ptr at) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)at, 16, 0, 0);
+}
+// The same from `lane_at` bytes into the rows of a page; OFF bytes on on both sides.
+template <int OFF>
+__device__ __forceinline__ void load_chunk(__amdgpu_buffer_rsrc_t rows, int lane_at, lds_ptr at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (__attribute__((address_space(3))) void*)at, 16, lane_at, 0, OFF, 0);
+}
+
+template <int V> struct ic { static constexpr int value = V; };
+
+template <int A, int B, class F>
+__device__ __forceinline__ void each(F f) {
+  if constexpr (A < B) {
+    f(ic<A>{});
+    each<A + 1, B>(f);
+  }
 }
 
 constexpr int KT = 64;  // keys per tile
@@ -49,12 +72,15 @@ __device__ __forceinline__ float inv_scale_cap(float scale_log2) { return 1.4426
 // NW waves x 32 query rows per workgroup (one K/V tile staging shared by all of them):
 // NW = 4 -> 128-row tiles, 2 workgroups per CU; NW = 8 -> 256-row tiles, 1 per CU
 // (same 2 waves per SIMD, half the K/V staging per query row).
-// DB = 1: two LDS stages.  Tile i+1 is written into the idle stage right after the one
-// barrier of iteration i (its registers were loaded during iteration i-1), tile i+2's
-// global loads are issued, then tile i is consumed — one barrier per 64 keys instead of
-// two, and a wave's LDS write no longer waits for every other wave before its MFMAs
-// (round 5: 24 % MFMA busy with DB = 0, profiles/r5_pmc/).
-template <int HD, int NW, int DB, bool MASKED = false, bool BIAS = false, int HDV = HD, bool PAD = false>
+//
+// Two LDS stages: a tile goes from memory to one of them (no registers between) while the tile in the other is multiplied,
+// one barrier per 64 keys.  One prompt of 8192 rows, 32 heads on 8 of 128 dims: 589 us -> 524 (1050 TF/s), 64 dims and 4096
+// rows 107 -> 90, a tile 3830 cycles a SIMD against 4700, of which its products take 2048.  What the staging registers, the
+// block ids' scalar loads, the addresses of each load and read and the copies around the mask cost went into it: 256
+// registers with every operand waited for as it was read, now 214 with reads a product or more ahead, 185 -> 143 vector and
+// 88 -> 50 scalar instructions a tile.  What is left: the clock falls to 1.85 GHz under it, a wave waits some 600 cycles a
+// tile while the loads of all four are issued, and one wave's products and exponentials overlap the other's in part.
+template <int HD, int NW, bool MASKED = false, bool BIAS = false, int HDV = HD, bool PAD = false>
 __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     const uint16_t* __restrict__ q, int q_stride, const uint16_t* __restrict__ k_cache,
     const uint16_t* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
@@ -65,7 +91,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     const float* __restrict__ dist_bias = nullptr, int n_dist = 0, float inv_scale = 0.f,
     float softcap = 0.f, const float* __restrict__ sinks = nullptr, const float* __restrict__ head_scale = nullptr,
     int dk_ = HD, int dv_ = HDV, int gate_heads = 0) {
-  __shared__ __attribute__((aligned(16))) uint16_t lds[(DB ? 2 : 1) * KT * (HD + HDV)];
+  __shared__ __attribute__((aligned(16))) uint16_t lds[2 * KT * (HD + HDV)];
   const int dk = PAD ? dk_ : HD, dv = PAD ? dv_ : HDV;
 
   // Workgroup -> (tile, head): all heads of a tile before the next tile, so that in a list with the heaviest tiles first no
@@ -110,8 +136,6 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   constexpr int NS = HD / 16;   // k-steps of S^T = K Q^T
   constexpr int ND = HDV / 32;  // 32-dim blocks of O^T
   constexpr int CH = HD / 8, CHV = HDV / 8;    // 16-byte chunks per K / V row
-  constexpr int NT = NW * 64;        // threads
-  constexpr int NP = KT * CH / NT, NPV = KT * CHV / NT;   // staging passes per tile (one chunk per thread per pass)
   // Q fragments (B operand): lane holds Q[row lr][16 s + 8 hh + j]
   u32x4 qf[NS];
   {
@@ -122,7 +146,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     // Q lands before any K/V load is issued.  Without this wait the compiler's waitcnt pass
     // merges "Q pending" from the preheader into the loop header and, to reach the older Q
     // loads, emits vmcnt(0) before the first QK^T MFMA of EVERY tile — which also waits for
-    // the K/V loads of tile i+2 issued a few instructions earlier: one full HBM round trip
+    // the next tile's loads issued a few instructions earlier: one full HBM round trip
     // per tile and no load/compute overlap at all.
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), expcnt / lgkmcnt untouched (gfx9 encoding)
   }
@@ -150,105 +174,83 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   // offset of chunk ch inside a key / value row
   auto kch = [&](int ch) { return PAD ? min(ch * 8, dk - 8) : ch * 8; };
   auto vch = [&](int ch) { return PAD ? min(ch * 8, dv - 8) : ch * 8; };
-  // K/V tile loads are software-pipelined one tile ahead through registers:
-  // the global loads of tile i+1 are in flight while tile i is consumed from
-  // LDS (1 workgroup per CU at this register budget, so latency must be hidden
-  // inside the wave, not by occupancy).
-  constexpr bool ONE = HD == HDV && !PAD;      // keys and values share row addresses
-  u32x4 kr[NP], vr[NPV];
-  auto load_tile = [&](int kb0) {
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int row = p * (NT / CH) + tid / CH;
-      const int ch = tid % CH;
-      const int key = min(kb0 + row, kv_end - 1);
-      const int blk = bt[key >> bs_log2];
-      const size_t base = ((size_t)blk * nkv + kvh) * head_stride + (size_t)(key & (bs - 1)) * dk + kch(ch);
-      kr[p] = *reinterpret_cast<const u32x4*>(k_cache + base);
-      if constexpr (ONE) vr[p] = *reinterpret_cast<const u32x4*>(v_cache + base);
-    }
-    if constexpr (!ONE) {
-#pragma unroll
-      for (int p = 0; p < NPV; ++p) {
-        const int key = min(kb0 + p * (NT / CHV) + tid / CHV, kv_end - 1);
-        const int blk = bt[key >> bs_log2];
-        vr[p] = *reinterpret_cast<const u32x4*>(v_cache + ((size_t)blk * nkv + kvh) * v_head_stride +
-                                                (size_t)(key & (bs - 1)) * dv + vch(tid % CHV));
-      }
-    }
-  };
-  auto store_tile = [&](uint16_t* kst, uint16_t* vst) {
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      const int row = p * (NT / CH) + tid / CH;
-      const int ch = tid % CH;
-      *reinterpret_cast<u32x4*>(kst + k_off<HD>(row, ch)) = kr[p];
-      if constexpr (HD == HDV) *reinterpret_cast<u32x4*>(vst + v_off<HD>(row, ch)) = vr[p];
-    }
-    if constexpr (HD != HDV) {
-#pragma unroll
-      for (int p = 0; p < NPV; ++p)
-        *reinterpret_cast<u32x4*>(vst + v_off<HDV>(p * (NT / CHV) + tid / CHV, tid % CHV)) = vr[p];
-    }
-  };
-  // Full tiles of 16-token pages (the engine's page size): the rows one wave stages in one
-  // pass lie in ONE page (a wave covers 64 / CH consecutive rows, 4 or 8, and passes are
-  // whole pages apart), so that page's block id is a wave-uniform scalar load and every
-  // lane's offset inside the page is a constant — no per-lane block-table gather and no
-  // 64-bit address arithmetic per load (the decode kernel's page16 path, round 4).
-  constexpr int RP = NT / CH;                  // tile rows per staging pass (16, 32 or 64)
-  static_assert(RP % 16 == 0 && 16 % (64 / CH) == 0, "passes are whole pages");
-  const int wsub = __builtin_amdgcn_readfirstlane(w) * (64 / CH);   // first row of this wave in a pass
-  const int lane_off = ((wsub & 15) + lane / CH) * dk + kch(lane % CH);
-  const int wpage = wsub >> 4;
-  // the same for value rows of another size
-  constexpr int RPV = NT / CHV;
-  static_assert(RPV % 16 == 0 && 16 % (64 / CHV) == 0, "passes are whole pages");
-  const int vsub = __builtin_amdgcn_readfirstlane(w) * (64 / CHV);
-  const int v_lane_off = ((vsub & 15) + lane / CHV) * dv + vch(lane % CHV);
-  const int vpage = vsub >> 4;
+  // RW rows of a tile are staged by each wave, 1 KB (64 / CH rows) a load, one behind the other in LDS; of full tiles of
+  // 16-token pages (the engine's page size) they lie in one page, one behind the other there too, so that its loads share
+  // one id and one address and differ in their instruction's offset.  The swizzle is in which chunk of its row a lane loads.
+  constexpr int RW = KT / NW;                                      // rows of a tile a wave stages
+  constexpr int NP = RW * CH / 64, NPV = RW * CHV / 64;            // its loads of keys and of values
+  static_assert(16 % RW == 0 && NP >= 1 && NPV >= 1, "a wave's rows lie in one page");
+  const int row0 = w * RW;
   const bool page16 = bs_log2 == 4;
-  // Block ids of a fast tile: wave-uniform scalar loads (s_load), issued at the top of the
-  // iteration that issues the tile's K/V loads so their latency overlaps the LDS stores.  (A
-  // vector-load prefetch one iteration ahead was tried: vmcnt is in-order, so waiting for it
-  // waited for the K/V loads issued after it — the stall the prefetch was meant to remove.)
-  int nbt[NP], nbv[HD == HDV ? 1 : NPV];
-  auto fast = [&](int kb0) { return page16 && kb0 + KT <= kv_end; };
-  auto fetch_bt = [&](int kb0) {
+  int k_at[NP], v_at[PAD ? NPV : 1];       // bytes from the wave's first row (whole rows: less the load's offset)
 #pragma unroll
-    for (int p = 0; p < NP; ++p) nbt[p] = bt[(kb0 >> 4) + p * (RP / 16) + wpage];
-    if constexpr (HD != HDV) {
+  for (int p = 0; p < NP; ++p) {
+    const int row = p * (64 / CH) + lane / CH;
+    k_at[p] = 2 * (row * dk + kch(k_slot<HD>(row0 + row, lane % CH))) - (PAD ? 0 : 1024 * p);
+  }
 #pragma unroll
-      for (int p = 0; p < NPV; ++p) nbv[p] = bt[(kb0 >> 4) + p * (RPV / 16) + vpage];
-    }
+  for (int p = 0; p < (PAD ? NPV : 1); ++p) {
+    const int row = p * (64 / CHV) + lane / CHV;
+    v_at[p] = 2 * (row * dv + vch(v_slot<HDV>(row0 + row, lane % CHV))) - (PAD ? 0 : 1024 * p);
+  }
+  int none = 0;
+  asm("" : "+v"(none));                   // a vector load: a scalar one's wait would be one for all reads of LDS
+  auto read_id = [&](int kb0) __attribute__((always_inline)) { return bt[(min(kb0 + row0, kv_end - 1) >> 4) + none]; };
+  auto full = [&](int kb0) __attribute__((always_inline)) { return page16 && kb0 + KT <= kv_end; };
+  // the page of a full tile's rows, and load l of its NP + NPV
+  __amdgpu_buffer_rsrc_t k_rows, v_rows;
+  auto at_page = [&](int id) __attribute__((always_inline)) {
+    const size_t blk = (size_t)__builtin_amdgcn_readfirstlane(id) * nkv + kvh;
+    k_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(k_cache + blk * head_stride + (row0 & 15) * dk), 0, RW * dk * 2, 0x00027000);
+    v_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(v_cache + blk * v_head_stride + (row0 & 15) * dv), 0, RW * dv * 2, 0x00027000);
   };
-  auto load_tile_fast = [&]() {
-#pragma unroll
+  auto load = [&](auto l_, int stage) __attribute__((always_inline)) {
+    constexpr int l = decltype(l_)::value, p = l < NP ? l : l - NP;
+    const lds_ptr at = (lds_ptr)(lds + stage * KT * (HD + HDV) + (l < NP ? row0 * HD : KT * HD + row0 * HDV));
+    if constexpr (PAD) load_chunk<0>(l < NP ? k_rows : v_rows, l < NP ? k_at[l < NP ? p : 0] : v_at[l < NP ? 0 : p], at + 1024 * p);
+    else load_chunk<1024 * p>(l < NP ? k_rows : v_rows, l < NP ? k_at[p] : v_at[0], at);
+  };
+  // rows of a tile that ends early, or of pages of another size: each lane finds its own
+  auto load_part = [&](int kb0, int stage) __attribute__((always_inline)) {
+    const lds_ptr kl = (lds_ptr)(lds + stage * KT * (HD + HDV) + row0 * HD), vl = (lds_ptr)(lds + stage * KT * (HD + HDV) + KT * HD + row0 * HDV);
+    int part = lane;
+    asm volatile("" : "+v"(part));      // computed here: kept from before the loop its addresses would cost registers
+#pragma unroll 1
     for (int p = 0; p < NP; ++p) {
-      const size_t base = ((size_t)nbt[p] * nkv + kvh) * head_stride;
-      kr[p] = *reinterpret_cast<const u32x4*>(k_cache + base + lane_off);
-      if constexpr (ONE) vr[p] = *reinterpret_cast<const u32x4*>(v_cache + base + lane_off);
+      const int row = row0 + p * (64 / CH) + part / CH, key = min(kb0 + row, kv_end - 1);
+      load_chunk((const char*)(k_cache + ((size_t)bt[key >> bs_log2] * nkv + kvh) * head_stride + (size_t)(key & (bs - 1)) * dk +
+                               kch(k_slot<HD>(row, part % CH))), kl + p * 1024);
     }
-    if constexpr (!ONE) {
+#pragma unroll 1
+    for (int p = 0; p < NPV; ++p) {
+      const int row = row0 + p * (64 / CHV) + part / CHV, key = min(kb0 + row, kv_end - 1);
+      load_chunk((const char*)(v_cache + ((size_t)bt[key >> bs_log2] * nkv + kvh) * v_head_stride + (size_t)(key & (bs - 1)) * dv +
+                               vch(v_slot<HDV>(row, part % CHV))), vl + p * 1024);
+    }
+  };
+  int id = 0;
+  if (kv_end > kv_begin) {
+    if (page16) id = read_id(kv_begin);
+    if (full(kv_begin)) {
+      at_page(id);
+      each<0, NP + NPV>([&](auto l) __attribute__((always_inline)) { load(l, 0); });
+    } else load_part(kv_begin, 0);
+    if (page16) id = read_id(kv_begin + KT);
+  }
+  // LDS addresses of this lane's operands in stage 0: keys lr (the second 32 are 64 HD bytes on), dims 16 s + 8 hh ..; values
+  // of dims 32 d .., keys 4 hh + tq (16 j + 8 more are 32 HDV j and 16 HDV bytes on)
+  typedef __attribute__((address_space(3))) const char* lds_at;
+  lds_at ka[NS], va[ND];
 #pragma unroll
-      for (int p = 0; p < NPV; ++p) {
-        const int blk = HD == HDV ? nbt[HD == HDV ? p : 0] : nbv[HD == HDV ? 0 : p];
-        vr[p] = *reinterpret_cast<const u32x4*>(v_cache + ((size_t)blk * nkv + kvh) * v_head_stride + v_lane_off);
-      }
-    }
-  };
-  auto load_any = [&](int kb0) {
-    if (fast(kb0)) {
-      fetch_bt(kb0);
-      load_tile_fast();
-    } else {
-      load_tile(kb0);
-    }
-  };
-  if (kv_end > kv_begin) load_any(kv_begin);
-  if (DB && kv_end > kv_begin) {
-    store_tile(lds, lds + KT * HD);             // stage 0 <- tile 0
-    if (kv_begin + KT < kv_end) load_any(kv_begin + KT);   // registers <- tile 1
+  for (int s = 0; s < NS; ++s) {
+    ka[s] = (lds_at)(lds + k_off<HD>(lr, 2 * s + hh));
+    asm("" : "+v"(ka[s]));
+  }
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    const int col = 32 * d + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    va[d] = (lds_at)(lds + KT * HD + v_off<HDV>(4 * hh + ((lane & 15) >> 2), col >> 3) + (col & 7));
+    asm("" : "+v"(va[d]));
   }
   // last key this wave can see (causal); tiles beyond it are skipped
   const int wave_last_pos = pos_base + min(t0 + 32 * w + 31, qlen - 1);
@@ -258,85 +260,58 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   const bool wave_rows = t0 + 32 * w < qlen;
   const int wave_min_first = first_key(wave_first_pos);   // first block start among this wave's rows
   const int wave_max_first = first_key(wave_last_pos);    // last block start among them
-  int it = 0;
-  for (int kb0 = kv_begin; kb0 < kv_end; kb0 += KT, ++it) {
-    uint16_t* ks;
-    uint16_t* vs;
-    if (DB) {
-      // stage it&1 holds tile it (written last iteration, or before the loop); every wave has
-      // finished reading stage (it+1)&1 (tile it-1) once it is past this barrier
-      __syncthreads();
-      ks = lds + (it & 1) * KT * (HD + HDV);
-      vs = ks + KT * HD;
-      if (kb0 + KT < kv_end) {
-        const bool nxt = kb0 + 2 * KT < kv_end;
-        const bool nfast = nxt && fast(kb0 + 2 * KT);
-        if (nfast) fetch_bt(kb0 + 2 * KT);
-        uint16_t* kn = lds + ((it + 1) & 1) * KT * (HD + HDV);
-        store_tile(kn, kn + KT * HD);           // tile it+1, loaded during the previous iteration
-        if (nfast) load_tile_fast();
-        else if (nxt) load_tile(kb0 + 2 * KT);
-      }
-    } else {
-      ks = lds;
-      vs = lds + KT * HD;
-      __syncthreads();  // previous tile fully consumed
-      store_tile(ks, vs);
-      __syncthreads();
-      if (kb0 + KT < kv_end) load_any(kb0 + KT);
-    }
-    // whole tile above this wave's diagonal, or no valid query row in this wave
-    // (it still stages K/V for the others)
-    if (kb0 > wave_last_pos || !wave_rows) continue;
-    if (MASKED && kb0 + KT <= wave_min_first) continue;    // wholly before every row's block
-
+  auto step = [&](int kb0, auto stage_) __attribute__((always_inline)) {
+    constexpr int stage = decltype(stage_)::value, at = stage * KT * (HD + HDV) * 2;
+    // this stage holds the tile once every wave's loads have landed; every wave has finished with the tile before, whose
+    // stage the next tile goes to
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+    __syncthreads();
+    const bool next = full(kb0 + KT);
+    if (next) {
+      at_page(id);
+      each<0, NP + NPV>([&](auto l) __attribute__((always_inline)) { load(l, 1 - stage); });
+    } else if (kb0 + KT < kv_end) load_part(kb0 + KT, 1 - stage);
+    if (page16) id = read_id(kb0 + 2 * KT);
+    if (kb0 > wave_last_pos || !wave_rows || (MASKED && kb0 + KT <= wave_min_first)) return;
     // ---- S^T = K Q^T for two 32-key blocks: the first block's operands are all under way before its products, the
-    // second's come between them (left to itself the compiler waits out an LDS read for every product or two).  With the
-    // first values read before the softmax, the second block's exponentials between the first's products and no exchange
-    // between the halves of a wave per tile: 739 us -> 704 (without the trace 617, 890 TF/s); matrix cores and vector unit
-    // are busy 43 % of the time each.  (A wave's next scores taken beside its softmax, in blocks of 32 keys, measured 759:
-    // the scalar and address work of two steps a tile cost more than the overlap gave.)
+    // second's come between them, the first values between the second's (left to itself the compiler waits out an LDS read
+    // for every product or two, hence the fences).  The values' first read waits for the next tile's loads, too: the
+    // compiler cannot tell the stages apart.  Read after the maxima instead 546 us for 538; all of them before the
+    // exponentials, the loads among the products after them, 860 (64 more registers, they spill); the softmax in blocks of
+    // 32 keys, each beside the other's products, 547 for 542.
     f32x16 sc[2];
+    // operands of V^T: keys 32 (j >> 1) + 16 (j & 1) .. + 15 of the tile, dims 32 d ..
+    auto read_v = [&](int j, int d) __attribute__((always_inline)) {
+      const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(va[d] + (at + 32 * HDV * j)));
+      const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(va[d] + (at + 32 * HDV * j + 16 * HDV)));
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto read_k = [&](int kb, int s) __attribute__((always_inline)) {
+      return *(const __attribute__((address_space(3))) bf16x8*)(ka[s] + (at + 64 * HD * kb));
+    };
+    typedef short short8v __attribute__((ext_vector_type(8)));
+    short8v vf[2][ND];
     {
-      bf16x8 kf[2][NS];
+      bf16x8 kf[NS];
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int s = 0; s < NS; ++s) kf[kb][s] = *reinterpret_cast<const bf16x8*>(ks + k_off<HD>(32 * kb + lr, 2 * s + hh));
+      for (int s = 0; s < NS; ++s) kf[s] = read_k(0, s);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[kb][r] = 0.f;
 #pragma unroll
-        for (int s = 0; s < NS; ++s) sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kb][s], as_bf16x8(qf[s]), sc[kb], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x100, NS, 0);
+        for (int s = 0; s < NS; ++s) {
+          sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[s], as_bf16x8(qf[s]), sc[kb], 0, 0, 0);
+          if (kb == 0) kf[s] = read_k(1, s);
+          else {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            for (int f = s * 2 * ND / NS; f < (s + 1) * 2 * ND / NS; ++f) vf[f / ND][f % ND] = read_v(f / ND, f % ND);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
-      __builtin_amdgcn_sched_group_barrier(0x008, NS, 0);
     }
-    // operands of V^T: keys 32 (j >> 1) + 16 (j & 1) .. + 15 of the tile, all blocks of 32 dims; the first before the softmax
-    const int g16 = lane >> 4;
-    const int idx = lane & 15;
-    const int tq = idx >> 2, tp = idx & 3;
-    auto read_v = [&](int j, u32x4 (&vf)[ND]) {
-#pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        const int col = 32 * d + 16 * (g16 & 1) + 4 * tp;
-        const int r0 = 16 * j + 4 * hh + tq;
-        const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vs + v_off<HDV>(r0, col >> 3) + (col & 7)));
-        const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vs + v_off<HDV>(r0 + 8, col >> 3) + (col & 7)));
-        vf[d][0] = (uint32_t)(uint16_t)lo[0] | ((uint32_t)(uint16_t)lo[1] << 16);
-        vf[d][1] = (uint32_t)(uint16_t)lo[2] | ((uint32_t)(uint16_t)lo[3] << 16);
-        vf[d][2] = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
-        vf[d][3] = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
-      }
-    };
-    u32x4 vf[2][ND];
-    read_v(0, vf[0]);
     if constexpr (BIAS) {
       // distance bias in raw score units (bias / scale): one table row per distance, the last row for
       // everything farther — a tile wholly beyond it for every row of the wave adds one constant
@@ -377,49 +352,35 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
         }
     }
     // ---- online softmax; lane owns query lr, keys kb0 + 32kb + (r&3) + 8(r>>2) + 4hh.
-    // Interior tiles (every key visible to every row of this wave, no tree rows) skip the
-    // per-element mask; both kinds then share one exponent path.
+    // Interior tiles (every key visible to every row of this wave, no tree rows) skip the mask.
     const bool interior = (kb0 + KT <= kv_end) && (kb0 + KT - 1 <= wave_first_pos) && !wave_tree &&
                           (!MASKED || kb0 >= wave_max_first);
     if (!interior) {
-      // masked keys -> -inf in raw score units, in place (one select per element, no branches:
-      // the tree bit is read with a clamped shift and applied by mask).  -inf, not a large
-      // finite value: a lane whose keys are all masked must get max -inf (no rescale) and
-      // P = 2^(-inf) = 0, whatever the scale.  Causal-only tiles (the diagonal) skip the
-      // 64-bit tree-mask shifts.
-      // Keys count from this lane's first one, so that the limits are compared with constants.
+      // masked keys -> -inf in raw score units.  -inf, not a large finite value: a lane whose keys are all masked must get
+      // max -inf (no rescale) and P = 2^(-inf) = 0, whatever the scale.  Bit i of `see`: this lane's row sees key key0 + i.
       const int key0 = kb0 + 4 * hh;
       const int lim = (row_valid ? min(my_pos, kv_end - 1) : -1) - key0;    // last visible key
-      if (wave_tree) {
-        const int tree0 = tree_key0 - key0;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = 32 * kb + (r & 3) + 8 * (r >> 2);
-            const int dt = key - tree0;
-            const bool tbit = (tmask >> (dt & 63)) & 1ull;
-            const bool ok = (lim >= key) & (!is_tree | (dt < 0) | tbit);
-            sc[kb][r] = ok ? sc[kb][r] : -__builtin_inff();
-          }
-      } else {
+      unsigned long long see = lim < 0 ? 0 : lim >= 63 ? ~0ull : (2ull << lim) - 1;
+      if (MASKED) {
         const int from = my_first - key0;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int key = 32 * kb + (r & 3) + 8 * (r >> 2);
-            const bool ok = MASKED ? (lim >= key) & (from <= key) : (lim >= key);
-            sc[kb][r] = ok ? sc[kb][r] : -__builtin_inff();
-          }
+        see = from <= 0 ? see : from > 63 ? 0 : see & (~0ull << from);
       }
+      if (is_tree) {
+        const int t = tree_key0 - key0;                                       // keys before t are seen, after it as the mask says
+        see &= t >= 64 ? ~0ull : t >= 0 ? (tmask << t) | ((1ull << t) - 1) : t > -64 ? tmask >> -t : 0ull;
+      }
+      const unsigned see_lo = (unsigned)see, see_hi = (unsigned)(see >> 32);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[kb][r] = (kb ? see_hi : see_lo) >> ((r & 3) + 8 * (r >> 2)) & 1 ? sc[kb][r] : -__builtin_inff();
     }
     float mx = -1e30f;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[kb][r]);
-    mx = row_valid ? mx * scale_log2 : -1e30f;
+    mx *= scale_log2;
     // deferred max: rescale O / l only when the running max grows by > 2^8, so
     // most tiles skip the 64 O multiplies (P stays <= 256, safe in f32 / bf16) and the exchange with the half of the wave
     // that holds the query's other keys
@@ -434,41 +395,37 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     }
     // P = 2^(s * scale_log2 - m) (raw v_exp_f32: arguments <= 8, masked scores underflow to 0; four partial row sums instead
     // of one 32-long dependent add chain) and O^T += V^T P^T.  The second block's exponentials run between the first
-    // block's products: each takes about as long as the other.
-    float ps[4] = {0.f, 0.f, 0.f, 0.f};
-    auto weights = [&](int kb) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        sc[kb][r] = __builtin_amdgcn_exp2f(sc[kb][r] * scale_log2 - m_run);
-        ps[r & 3] += sc[kb][r];
-      }
+    // block's products: each takes about as long as the other.  Values are read two groups of products ahead.
+    float ps[4];
+    u32x4 pf;
+    auto weight = [&](int kb, int r) __attribute__((always_inline)) {
+      sc[kb][r] = __builtin_amdgcn_exp2f(sc[kb][r] * scale_log2 - m_run);
+      ps[r & 3] = kb == 0 && r < 4 ? sc[kb][r] : ps[r & 3] + sc[kb][r];
     };
-    auto products = [&](int kb) {
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        const int j = 2 * kb + s2;
-        if (j < 3) read_v(j + 1, vf[(j + 1) & 1]);
-        u32x4 pf;
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) pf[jj] = pack_bf16x2(sc[kb][8 * s2 + 2 * jj], sc[kb][8 * s2 + 2 * jj + 1]);
-#pragma unroll
-        for (int d = 0; d < ND; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(vf[j & 1][d]), as_bf16x8(pf), o[d], 0, 0, 0);
-      }
-    };
-    weights(0);
-    __builtin_amdgcn_sched_barrier(0);
-    products(0);
-    weights(1);
-#pragma unroll
-    for (int i = 0; i < 2 * ND; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 32 / ND, 0);
-      __builtin_amdgcn_sched_group_barrier(0x400, 8 / ND, 0);
+    for (int r = 0; r < 16; ++r) {
+      weight(0, r);
     }
     __builtin_amdgcn_sched_barrier(0);
-    products(1);
+    each<0, 4 * ND>([&](auto i_) __attribute__((always_inline)) {
+      constexpr int i = decltype(i_)::value, j = i / ND, d = i % ND;
+      if constexpr (d == 0) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) pf[jj] = pack_bf16x2(sc[j >> 1][8 * (j & 1) + 2 * jj], sc[j >> 1][8 * (j & 1) + 2 * jj + 1]);
+      }
+      o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vf[j & 1][d]), as_bf16x8(pf), o[d], 0, 0, 0);
+      if constexpr (j < 2) {
+        vf[j][d] = read_v(j + 2, d);
+#pragma unroll
+        for (int r = i * 8 / ND; r < (i + 1) * 8 / ND; ++r) weight(1, r);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
     l_run += (ps[0] + ps[1]) + (ps[2] + ps[3]);      // this lane's keys; the halves of the wave meet after the loop
+  };
+  for (int kb0 = kv_begin; kb0 < kv_end; kb0 += 2 * KT) {
+    step(kb0, ic<0>{});
+    if (kb0 + KT < kv_end) step(kb0 + KT, ic<1>{});
   }
   l_run += __shfl_xor(l_run, 32, 64);
 

@@ -358,7 +358,7 @@ def paged_prefill_ref(q, k_cache, v_cache, block_tables, cu_seqlens_q, context_l
 # each staged K/V tile).  Every producer of ``tiles`` (model runner, EAGLE verify /
 # draft metadata, ops.paged_prefill) cuts sequences at this size.
 PREFILL_TILE = int(os.environ.get("DGI_PREFILL_TILE", "128"))
-# two LDS stages in the prefill attention kernel (one barrier per K/V tile); 0 = the round-4 loop
+# bit 16 of the native call's tile size: kept for its callers, the kernel has two LDS stages either way
 PREFILL_DB = int(os.environ.get("DGI_PREFILL_DB", "1"))
 
 

@@ -1,0 +1,89 @@
+"""Prompt attention at the edges of its tiles of 64 keys: last tiles of every kind, pages of other sizes, tree rows that
+start anywhere in a tile; against 64 bits."""
+import math
+
+import pytest
+import torch
+
+from dgi import ops
+from dgi.ops import mix
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(nh, nkv, hd, page, qlens, ctxs, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda", generator=g).bfloat16()
+
+    width = max(-(-c // page) for c in ctxs) + 1
+    pages = len(ctxs) * width
+    kc, vc = rand(pages, nkv, page, hd), rand(pages, nkv, page, hd)
+    table = torch.randperm(pages, device="cuda", generator=g).int().view(len(ctxs), width)
+    for b, c in enumerate(ctxs):                       # what lies past a sequence's end is never part of a result
+        for p in range(c // page, width):
+            kc[table[b, p], :, c - p * page if p == c // page else 0:] = float("nan")
+            vc[table[b, p], :, c - p * page if p == c // page else 0:] = float("nan")
+    cu = torch.tensor([sum(qlens[:i]) for i in range(len(qlens) + 1)], dtype=torch.int32, device="cuda")
+    return rand(sum(qlens), nh * hd), kc, vc, table, cu, torch.tensor(ctxs, dtype=torch.int32, device="cuda")
+
+
+def _check(out, q, kc, vc, table, cu, ctx, nh, nkv, hd, visible):
+    """|error| <= 2^-8 (sum p |v| + |o|): weights and results are rounded to bf16 (2^-9 each), the rest is fp32."""
+    page, scale = kc.shape[2], hd ** -0.5
+    for b in range(len(ctx)):
+        n, lo, hi = int(ctx[b]), int(cu[b]), int(cu[b + 1])
+        rows = torch.arange(n, device="cuda")
+        k, v = (c[table[b].long()[rows // page], :, rows % page].double().repeat_interleave(nh // nkv, 1) for c in (kc, vc))
+        s = torch.einsum("qhd,khd->hqk", q[lo:hi].double().view(-1, nh, hd), k) * scale
+        p = torch.softmax(s.masked_fill(~visible(b, hi - lo, n)[None], -math.inf), -1)
+        want, size = torch.einsum("hqk,khd->qhd", p, v), torch.einsum("hqk,khd->qhd", p, v.abs())
+        off = (out[lo:hi].double().view(-1, nh, hd) - want).abs()
+        assert bool((off <= 2.0 ** -8 * (size + want.abs())).all()), (b, float(off.max()))
+
+
+def _causal(_, m, n):
+    return torch.arange(n, device="cuda")[None] <= torch.arange(n - m, n, device="cuda")[:, None]
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("page", [8, 16, 32])
+@pytest.mark.parametrize("tile", [128, 256])
+def test_ends_of_tiles(hd, page, tile, monkeypatch):
+    monkeypatch.setattr(ops, "PREFILL_TILE", tile)
+    qlens, ctxs = [1, 63, 64, 65, 128, 129, 33, 300], [1, 63, 64, 65, 128, 129, 190, 449]
+    case = _case(6, 3, hd, page, qlens, ctxs, 5)
+    _check(ops.paged_prefill(*case, 6, 3, hd ** -0.5), *case, 6, 3, hd, _causal)
+
+
+@pytest.mark.parametrize("ctx", [64, 65, 96, 100, 127, 128, 131, 160, 200])
+def test_tree_rows_anywhere_in_a_tile(ctx):
+    """64 tree rows, the last ones of a sequence, whose keys begin at any offset of a tile and of a lane's keys."""
+    hd, n = 128, 64
+    par = torch.tensor([[-1] + [(i - 1) // 2 if i % 3 else max(0, i - 5) for i in range(1, n)]] * 2, dtype=torch.int32)
+    anc, _ = ops.tree_mask_ref(par)
+    case = _case(4, 2, hd, 16, [n, n], [ctx, ctx + 7], ctx)
+    out = ops.paged_prefill(*case, 4, 2, hd ** -0.5, tree_mask=anc.cuda(), tree_n=n)
+
+    def visible(b, m, keys):
+        see = torch.ones(m, keys, dtype=torch.bool)
+        for i in range(n):
+            bits = int(anc[b, i]) & (1 << 64) - 1
+            see[i, keys - n:] = torch.tensor([bool(bits >> j & 1) for j in range(n)])
+        return see.cuda() & _causal(b, m, keys)
+
+    _check(out, *case, 4, 2, hd, visible)
+
+
+@pytest.mark.parametrize("window,block", [(1, 0), (31, 0), (64, 0), (65, 0), (0, 1), (0, 32), (0, 100)])
+def test_first_keys_anywhere_in_a_tile(window, block):
+    hd = 64
+    case = _case(4, 2, hd, 16, [200, 70], [200, 333], 9)
+    out = mix.paged_prefill_masked(*case, 4, 2, hd ** -0.5, block, None, window=window)
+
+    def visible(b, m, n):
+        p, j = torch.arange(n - m, n, device="cuda")[:, None], torch.arange(n, device="cuda")[None]
+        return (j <= p) & (j > p - window if window else j >= p // block * block)
+
+    _check(out, *case, 4, 2, hd, visible)
