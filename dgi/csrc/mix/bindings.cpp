@@ -85,7 +85,9 @@ int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, const void*
                     int v_stride, int in_f32, const float* aux1, int aux1_stride, const float* aux2, int aux2_stride,
                     const float* par1, const float* par2, float* state, float* norm, float* mx, const int* positions,
                     const int* seq_row0, const int* seq_slots, int n_seq, int H, int G, int dk, int dv, float cap,
-                    int rows, float* norm_new, float* mx_new, hipStream_t st);
+                    int rows, float* norm_new, float* mx_new, float* parts, int parts_chunks, hipStream_t st);
+long long dgi_linear_scan_parts(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
+                                int in_f32, int* parts_chunks);
 int dgi_token_shift(void* out, int out_f32, const void* h, int h_f32, int h_stride, const float* mu, int nmix, float* tail,
                     const int* positions, const int* row_seq, const int* seq_row0, const int* seq_slots, int n_seq, int T,
                     int W, hipStream_t st);
@@ -965,12 +967,17 @@ void linear_scan(at::Tensor y, int64_t mode, const at::Tensor& q, const at::Tens
     mx_new = at::empty({n_seq, H}, state.options());
     nn = norm_new.data_ptr<float>(); mn = mx_new.data_ptr<float>();
   }
+  at::Tensor parts;
+  int parts_chunks = 0;
+  const long long floats = dgi_linear_scan_parts((int)mode, (int)dk, (int)dv, (int)H, (int)G, n_seq, T, q.data_ptr(), (int)q.stride(0), k.data_ptr(),
+                                                 (int)k.stride(0), f, &parts_chunks);
+  if (floats > 0) parts = at::empty({floats}, state.options());
   check_rc(dgi_linear_scan(y.data_ptr<float>(), (int)mode, q.data_ptr(), (int)q.stride(0), k.data_ptr(), (int)k.stride(0),
                            v.data_ptr(), (int)v.stride(0), f, a1, a1s, a2, a2s,
                            f32p(par1, "par1", np), f32p(par2, "par2", np), state.data_ptr<float>(), nrm, mxp,
                            i32p(positions, "positions", T), i32p(seq_row0, "seq_row0", n_seq + 1),
                            i32p(seq_slots, "seq_slots"), n_seq, (int)H, (int)G, (int)dk, (int)dv, (float)cap, T,
-                           nn, mn, cur_stream()), "linear_scan");
+                           nn, mn, parts.defined() ? parts.data_ptr<float>() : nullptr, parts_chunks, cur_stream()), "linear_scan");
 }
 
 // paged caches of one attention layer: k [NB, G, bs, dk], v [NB, G, bs, dv]

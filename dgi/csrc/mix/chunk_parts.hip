@@ -29,116 +29,16 @@
 //   ssm, 2 prompts of 4096 rows, 64 heads of 128 x 64     210 us -> 170 (of it 20 the pass before)
 //   mlstm, 5 prompts of 3001 bf16 rows, 32 heads of 64     83 -> 49;  of 128 197 -> 137;  fp32 rows 105 -> 74
 //   light, 2 prompts of 4096 bf16 rows, 64 heads of 64    158 -> 113
-// mlstm on fp32 rows of 128 channels stays there (its waves would spill: 213 -> 230 us), delta too (four chunks of q and k would have to be kept).
+// mlstm on fp32 rows of 128 channels stays there (its waves would spill: 213 -> 230 us); delta: chunk_delta.hip.
 //
 // Precision: results and states are no further from 64 bits than the token loop's (2-norm, 512 rows: ssm 7.9e-8, the loop 1.03e-7; states of mlstm
 // 3.1e-8, 4.4e-8): decays are summed as logarithms in 64 bits and a running maximum is kept in 64 bits, since its rounding would be the state's.
 #include <type_traits>
-#include "chunk_args.h"
+#include "chunk_split.h"
 
 using namespace dgi;
 
 namespace {
-
-constexpr int C = 32;              // tokens per chunk
-typedef double f64x2 __attribute__((ext_vector_type(2)));
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-constexpr float MOST = 3.38e38f;   // beyond, a first part would round to infinity
-constexpr double LOG2E = 1.4426950408889634;
-
-__device__ __forceinline__ double softplus_d(double x) { return fmax(x, 0.) + log1p(exp(-fabs(x))); }
-
-__device__ __forceinline__ short4v read_tr(const char* p) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)p); }
-
-// two values in three bf16 parts each; x becomes what is left for the next
-__device__ __forceinline__ uint32_t part_of(float& x0, float& x1) {
-  const uint32_t p = pack_bf16x2(x0, x1);
-  x0 -= __uint_as_float(p << 16);
-  x1 -= __uint_as_float(p & 0xffff0000u);
-  return p;
-}
-template <int PARTS>
-__device__ __forceinline__ void split8(const float* x, u32x4* p) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float a = x[2 * i], b = x[2 * i + 1];
-    if constexpr (PARTS == 1) {
-      p[0][i] = pack_bf16x2(a, b);
-    } else {
-      p[0][i] = part_of(a, b);
-      p[1][i] = part_of(a, b);
-      p[2][i] = pack_bf16x2(a, b);
-    }
-  }
-}
-// 3 / 2 2^(16 + the exponent of the largest): added and taken off again, it rounds to multiples of 2^-7 of it
-__device__ __forceinline__ float grid_of(float most) { return __uint_as_float(((__float_as_uint(most) & 0x7f800000u) + 0x08000000u) | 0x00400000u); }
-// Parts of products x f (l: what f lacks of more bits), with what they lack in 32 bits.  GRID: the first part is a multiple of what grid says.
-template <bool GRID>
-__device__ __forceinline__ void split2_of(const float* x, const float* f, const float* l, float grid, int i, u32x4* p) {
-  float a = x[2 * i] * f[2 * i], b = x[2 * i + 1] * f[2 * i + 1];
-  float ea = fmaf(x[2 * i], f[2 * i], -a), eb = fmaf(x[2 * i + 1], f[2 * i + 1], -b);
-  if constexpr (GRID) {
-    ea = fmaf(x[2 * i], l[2 * i], ea);
-    eb = fmaf(x[2 * i + 1], l[2 * i + 1], eb);
-    const float a0 = (a + grid) - grid, b0 = (b + grid) - grid;
-    p[0][i] = pack_bf16x2(a0, b0);
-    a = (a - a0) + ea;
-    b = (b - b0) + eb;
-    p[1][i] = part_of(a, b);
-    p[2][i] = part_of(a, b);
-    p[3][i] = pack_bf16x2(a, b);
-  } else {
-    p[0][i] = part_of(a, b);
-    p[1][i] = part_of(a, b);
-    p[2][i] = pack_bf16x2(a + ea, b + eb);
-  }
-}
-
-__device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
-}
-// products of N operands' parts by one's (or its own: BN = N), for sums of their own: the first two parts' to hi, the smaller ones, smallest first, to lo.
-// Sums take turns, none waits for its own last product.
-template <int PA, int PB, int N, int BN>
-__device__ __forceinline__ void multiply(const u32x4 (&a)[N][PA], const u32x4 (&b)[BN][PB], f32x4 (&lo)[N], f32x4 (&hi)[N]) {
-#pragma unroll
-  for (int x = 2; x > 0; --x)                        // parts that together are x smaller than the first
-#pragma unroll
-    for (int p = x; p >= 0; --p)
-      if (p < PA && x - p < PB) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) lo[i] = mfma(a[i][p], b[i % BN][x - p], lo[i]);
-      }
-#pragma unroll
-  for (int i = 0; i < N; ++i) hi[i] = mfma(a[i][0], b[i % BN][0], hi[i]);
-}
-
-// 2^(whole + part), part within [-2, 2]
-__device__ __forceinline__ float power(float whole, float part) {
-  return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(part), (int)whole);
-}
-__device__ __forceinline__ void whole_and_part(double x, float& whole, float& part) {
-  x = fmin(fmax(x, -1e6), 1e6);
-  const double i = rint(x);
-  whole = (float)i;
-  part = (float)(x - i);
-}
-// 2^x, rounded about once, and what it lacks: 2^part - 1 by its series, part within [-0.5, 0.5] (the first term left out is 4e-9)
-__device__ __forceinline__ float power_once(double x, float* rest = nullptr) {
-  float i, f;
-  whole_and_part(x, i, f);
-  const float y = f * 0.693147181f;
-  float p = 1.f / 5040.f;
-  p = fmaf(p, y, 1.f / 720.f);
-  p = fmaf(p, y, 1.f / 120.f);
-  p = fmaf(p, y, 1.f / 24.f);
-  p = fmaf(p, y, 1.f / 6.f);
-  p = fmaf(p, y, 0.5f);
-  const float t = fmaf(p * y, y, y), r = 1.f + t;
-  if (rest) *rest = __builtin_amdgcn_ldexpf((1.f - r) + t, (int)i);
-  return __builtin_amdgcn_ldexpf(r, (int)i);
-}
 
 template <int MODE, typename TI, int NK_>
 struct Lay {
@@ -170,23 +70,8 @@ struct Lay {
 // factor; mlstm: exp(-maximum), what F lacks of more bits; then A of the last token, whether something is not finite
 constexpr int EI = 0, EF = 32, BI = 64, BF = 96, GA = 128, GF = 160, RA = 192, RC = 224, GX = 256, GL = 288, ALL = 320, BAD = 321;
 
-// ssm: chunks of all sequences one after the other; of each and every group the parts, three score tiles and a flag (a multiple of 16 bytes)
-__device__ __forceinline__ int first_chunk(int row0, int seq) { return row0 / C + seq; }
+// ssm, of each chunk and group: the parts, three score tiles and a flag (a multiple of 16 bytes)
 __host__ __device__ constexpr int parts_floats(int DP) { return 2 * 3 * C * DP / 2 + 3 * 256 + 4; }
-
-// longest sequences first among at most 16
-constexpr int MOST_SEQ = 16;
-__device__ __forceinline__ int ranked(const ChunkArgs& a, int seq) {
-  if (a.n_seq > MOST_SEQ || a.n_seq == 1) return seq;
-  const int lane = threadIdx.x & 63, i = min(lane, a.n_seq - 1);
-  const int len = lane < a.n_seq ? max(a.seq_row0[i + 1] - a.seq_row0[i], 0) : -1;
-  int before = 0;                                    // sequences that are longer, or as long and earlier
-  for (int j = 0; j < a.n_seq; ++j) {
-    const int other = __builtin_amdgcn_readlane(len, j);
-    before += other > len || (other == len && j < lane);
-  }
-  return __ffsll((unsigned long long)__ballot(lane < a.n_seq && before == seq)) - 1;
-}
 
 template <int MODE, typename TI, int NK>
 __global__ __launch_bounds__((64 * Lay<MODE, TI, NK>::WAVES), (Lay<MODE, TI, NK>::PER_SIMD)) void chunk_parts_kernel(const ChunkArgs a) {

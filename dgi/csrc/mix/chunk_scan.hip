@@ -1106,7 +1106,8 @@ extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, 
 // Needs dgi_chunk_scan_ok.  skip_rows: sequences of at most that many rows are left to another launch.  segs > 1 (ssm): portions are
 // cut into segments of seg_rows rows (a multiple of 32, segs of them at least as long as the longest portion) that run side by side: each one's
 // state from nothing, a short serial pass over those states, then the outputs from each segment's incoming state.  About
-// twice the work, for steps whose heads leave most of the chip idle.  parts (ssm): dgi_ssm_parts_floats of workspace for chunk_parts.hip, or null.
+// twice the work, for steps whose heads leave most of the chip idle.  parts: ssm: dgi_ssm_parts_floats of workspace for chunk_parts.hip, delta:
+// dgi_chunk_delta_floats for chunk_delta.hip, or null.
 extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                               int v_stride, int in_f32, const void* aux1, int aux1_stride, const void* aux2, int aux2_stride,
                               int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
@@ -1145,7 +1146,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
   if (by_parts) rc = dgi_chunk_parts(a, mode, in_f32, grid, st);
   else switch (mode) {
     case WKV: rc = launch_mode<WKV>(a, in_f32, four, grid, st); break;
-    case DELTA: rc = launch_mode<DELTA>(a, in_f32, four, grid, st); break;
+    case DELTA: rc = parts ? dgi_chunk_delta(a, in_f32, grid, st) : launch_mode<DELTA>(a, in_f32, four, grid, st); break;
     case MLSTM: rc = in_f32 && dk > 64 ? launch_one<MLSTM, float, 8, 32>(a, grid, st) : -2; break;
     case SSM: rc = in_f32 ? launch_dims<SSM, float>(a, false, grid, st) : -2; break;
   }

@@ -1125,6 +1125,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
                               int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st);
+long long dgi_chunk_delta_floats(int dk, int H, int T, int n_seq, int in_f32, int* chunks);
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 extern "C" int dgi_chunk_scan_decay(float* y, int light, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                                    int v_stride, int in_f32, const float* decay, int decay_stride, float* state,
@@ -1183,13 +1184,27 @@ extern "C" int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows
   return KS <= 16 && scan_columns(KS, dv) < dv;
 }
 
+// Floats of workspace (`parts`, `parts_chunks` chunks) that a step of delta layers needs for chunk_delta.hip; 0: it does not go there.  Its chain takes 32
+// tokens in little more than chunk_scan.hip takes for 16, but what it prepares costs 0.2 ns a row and head, and a compute unit has one workgroup of
+// it: up to 64 channels it is the faster for long portions whose workgroups find a unit each (us there, here, 64 channels: heads, sequences x rows: 64, 1 x 512
+// 46, 42; 64, 2 x 512 48, 50; 16, 8 x 512 48, 52; 64, 1 x 1024 82, 60; 32, 4 x 1024 85, 77; 16, 8 x 1024 87, 76; 64, 4 x 1024 125, 160), of 128 (bf16 rows) from
+// some 300 rows on (32 heads: 2 x 256 44, 45; 8 x 384 218, 141; 8 x 1024 507, 412).
+extern "C" long long dgi_linear_scan_parts(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k,
+                                           int k_stride, int in_f32, int* parts_chunks) {
+  if (mode != DELTA || n_seq == 0 || chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows) != 1) return 0;
+  const long units = (long)n_seq * H * ((dv + 31) / 32);
+  if (dk <= 64 ? rows < 768l * n_seq || units > 256 : rows < 320l * n_seq || units > 512) return 0;
+  return dgi_chunk_delta_floats(dk, H, rows, n_seq, in_f32, parts_chunks);
+}
+
 // mode 0 wkv, 1 delta, 2 mlstm, 3 gla, 4 light; q / k / v bf16 or fp32 (in_f32) with row strides in elements; rows: rows of the step.
 // norm_new / mx_new: mlstm's staged normaliser / maximum (needed where a head spans several workgroups).
 extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                                int v_stride, int in_f32, const float* aux1, int aux1_stride, const float* aux2,
                                int aux2_stride, const float* par1, const float* par2, float* state, float* norm, float* mx,
                                const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int H, int G,
-                               int dk, int dv, float cap, int rows, float* norm_new, float* mx_new, hipStream_t st) {
+                               int dk, int dv, float cap, int rows, float* norm_new, float* mx_new, float* parts, int parts_chunks,
+                               hipStream_t st) {
   if (n_seq == 0) return 0;
   if (mode < 0 || mode > 4 || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0) return -2;
   if (dk > 512) return -3;
@@ -1207,7 +1222,7 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   if (form) {
     const int rc = form == 1 ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
                                               aux2, aux2_stride, 0, par1, par2, nullptr, cap, state, norm, mx, norm_new, mx_new, positions,
-                                              seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, 0, nullptr, nullptr, nullptr, 0, st)
+                                              seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, 0, nullptr, nullptr, parts, parts_chunks, st)
                              : dgi_chunk_scan_decay(y, mode == LIGHT, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? par1 : aux1,
                                                    mode == LIGHT ? 0 : aux1_stride, state, positions, seq_row0, seq_slots, n_seq, H, dk, dv,
                                                    apart, st);
