@@ -776,7 +776,10 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK>::WAVES), (Lay<MODE, TI, NK>
         odd = big(u);
         split8<PU>(u, up);
       }
-      multiply<PQ, 3, 2, 1>(qf[b % QK], sp[b & 1], lo, hi);
+      // the last block's first parts start from the small ones' sum: one rounding less at the sum's size
+      small<PQ, 3, 2, 1>(qf[b % QK], sp[b & 1], lo);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) (b + 1 < NK ? hi : lo)[h] = mfma(qf[b % QK][h][0], sp[b & 1][0][0], (b + 1 < NK ? hi : lo)[h]);
       if constexpr (L::PRE) read_q(c + 1, b, qf[b % QK]);
       if (!L::PRE) __builtin_amdgcn_sched_group_barrier(0x100, 2 * PQ, 0);      // reads, then a product and some of the next parts in turn
       constexpr int M = 2 * (PQ == 1 ? 3 : 6);
