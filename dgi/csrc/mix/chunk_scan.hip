@@ -1,6 +1,6 @@
 // dgi/csrc/mix/chunk_scan.hip — prompt portions of the recurrences that carry a matrix S [dk, dv] per head (linear_scan.hip has
 // their definitions, ssm_scan.hip that of ssm), sixteen tokens at a time in fp32 matrix products (v_mfma_f32_16x16x4_f32).  Those that chunk_parts.hip
-// takes (light; mlstm, but for fp32 rows of more than 64 channels; ssm of groups of four heads) go there.
+// takes (light; mlstm, but for fp32 rows of more than 64 channels; ssm of groups of four heads) go there, long portions of delta to chunk_delta.hip.
 //
 // For tokens t, s of a chunk that starts from the state S, with D[t, s] the product of the decays of the tokens after s up to t
 // and A_t that of all tokens up to t:

@@ -28,7 +28,7 @@
 // running maximum is a serial pass of one thread (adds and maxima; its exponentials are parallel again).
 // The token loop reads LDS only.  Everything is fp32; q / k / v arrive as bf16 or fp32.
 // A portion that starts at position 0 reads no state; the state is written back at the end of the portion.
-// Prompt portions run in chunks of sixteen tokens on the matrix cores instead (chunk_scan.hip): what is left here are steps of
+// Prompt portions run in chunks of tokens on the matrix cores instead (chunk_scan.hip, chunk_parts.hip, chunk_delta.hip): what is left here are steps of
 // single rows and short portions, key sizes above 128 (gla, light: 256), and rows of delta and mlstm that cannot be read in fours.
 #include "../common.h"
 
@@ -1214,7 +1214,7 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   if ((mode == LIGHT && !par1) || (mode != LIGHT && !aux1)) return -4;
   bool short_rows = rows <= 4 * n_seq;             // rows of the step: at most four per sequence on average
   const bool staged = mode == MLSTM && norm_new && mx_new;
-  // Prompt portions: sixteen tokens at a time on the matrix cores (chunk_scan.hip, chunk_parts.hip).  Among many sequences there are decode
+  // Prompt portions: sixteen or 32 tokens at a time on the matrix cores (chunk_scan.hip, chunk_parts.hip, chunk_delta.hip).  Among many sequences there are decode
   // rows and short portions beside the long ones: they stay with this kernel, in a launch of their own.
   const int form = chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows);
   const int apart = n_seq > APART_FROM && (form == 1 || (form == 2 && rows <= 4 * n_seq))

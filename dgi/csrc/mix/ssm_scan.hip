@@ -268,7 +268,8 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
 
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 
-// chunked: portions go sixteen tokens at a time through the matrix cores (chunk_scan.hip, where the shapes allow it).  Its workgroups have a
+// chunked: portions go 32 tokens at a time through the matrix cores (chunk_parts.hip; sixteen, chunk_scan.hip, where groups have fewer than four heads or
+// channels are more than 128).  Its workgroups have a
 // compute unit to themselves and a pipeline to fill, so among more than APART_FROM sequences the short ones stay with this file's kernel: those
 // of at most 48 rows while the workgroups find a place each (12 portions of 39 rows, 32 heads: 31 us against 51 there), longer ones when they
 // wait for each other (64 columns, this file's time and that one's: 11 portions of 100 rows, 16 heads 35, 41; 128 rows 42, 41; 16 portions of 128

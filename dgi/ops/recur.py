@@ -177,7 +177,7 @@ def ssm_scan_ref(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0
     return y.reshape(T, inner)
 
 
-SCAN_CHUNK = int(os.environ.get("DGI_SCAN_CHUNK", "16"))       # 0: portions row by row in every case (chunks have sixteen rows)
+SCAN_CHUNK = int(os.environ.get("DGI_SCAN_CHUNK", "16"))       # 0: portions row by row in every case
 # workgroups of the row-by-row form (sequence x head x 16 columns) from which steps stay with it, unless a call asks for chunks
 SCAN_CHUNK_BELOW = int(os.environ.get("DGI_SCAN_CHUNK_BELOW", str(1 << 40)))
 
@@ -214,7 +214,7 @@ def ssm_scan(xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, seq_row0, se
     S [N, dv] in fp32 read from / written to ``state`` [slots, heads, dv, N] (value-major; zero at position 0).
     Returns y [T, heads*dv] fp32.
 
-    On the GPU the prompt portions of bf16 models are taken sixteen rows at a time on the matrix cores — the same recurrence
+    On the GPU the prompt portions of bf16 models are taken in chunks of 32 rows (sixteen where groups have fewer than four heads) on the matrix cores — the same recurrence
     with its fp32 sums reassociated, where the step's rows and sequences make that the faster form.  Models in fp32
     (``dt_raw`` fp32), steps of single rows, and every step with ``chunked`` False go row by row: those results do not depend
     on how a prompt was cut or on what else is in the step.  ``chunked`` True asks for the chunks."""
