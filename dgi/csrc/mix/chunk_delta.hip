@@ -15,9 +15,10 @@
 // parts each (chunk_parts.hip).
 //
 // What bounds it: a chunk of the chain takes 1.4 us (chunk_scan.hip: 1.2 for sixteen tokens), 48 products of 16 cycles and 230 vector instructions, which
-// one wave does not overlap (alone on its unit the state waves would take 1.03); preparing 4096 rows of 64 heads 51 us, 150 MB of G and P M to memory.  Two
-// prompts of 4096 rows in all, 64 heads of 64 x 64: 178 us -> 170 on inputs that change from pass to pass, 159 on the same; one of 2048 rows 154 -> 101, one of
-// 4000 rows and 16 heads 290 -> 160; bf16 rows of 128 channels, 4 of 1024 rows, 32 heads, 255 -> 155.  Only long portions are taken, see
+// one wave does not overlap (alone on its unit the state waves would take 1.03); preparing 4096 rows of 64 heads 51 us, 150 MB of G and P M to memory, which
+// nothing reads soon, and then once: stores and loads say so (without, they take the place of q, k and v in the caches, 170 us for 149).  Two
+// prompts of 4096 rows in all, 64 heads of 64 x 64: 178 us -> 149; one of 2048 rows 154 -> 103; bf16 rows of
+// 128 channels, 4 of 1024 rows, 32 heads, 255 -> 157.  Only long portions are taken, see
 // dgi_linear_scan_parts.  Tried: M and P themselves prepared, u by a product more in the chain: 122 us a chain for 105; two state waves a block of columns, half
 // the channels each: 138 for 142 without the rest (x is both's, and the unit has no instructions to spare).
 //
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(const ChunkArgs a
       four(v[0] + l[0], p0);
       four(v[1] + l[1], p1);
 #pragma unroll
-      for (int j = 0; j < 3; ++j) *reinterpret_cast<u32x4*>(to + (3 * i + j) * 1024 + 16 * lane) = u32x4{p0[j][0], p0[j][1], p1[j][0], p1[j][1]};
+      for (int j = 0; j < 3; ++j) __builtin_nontemporal_store(u32x4{p0[j][0], p0[j][1], p1[j][0], p1[j][1]}, reinterpret_cast<u32x4*>(to + (3 * i + j) * 1024 + 16 * lane));
     }
     u32x4 P[2][3];                                     // rows t = 16 ht + n16
 #pragma unroll
@@ -358,8 +359,8 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(const ChunkArgs a
     char* const pm = to + g_bytes(NT);
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      *reinterpret_cast<u32x2*>(pm + j * PART + 8 * lane) = p[0][j];
-      *reinterpret_cast<u32x4*>(pm + j * PART + 512 + 16 * lane) = u32x4{p[1][j][0], p[1][j][1], p[2][j][0], p[2][j][1]};
+      __builtin_nontemporal_store(p[0][j], reinterpret_cast<u32x2*>(pm + j * PART + 8 * lane));
+      __builtin_nontemporal_store(u32x4{p[1][j][0], p[1][j][1], p[2][j][0], p[2][j][1]}, reinterpret_cast<u32x4*>(pm + j * PART + 512 + 16 * lane));
     }
   }
 }
@@ -412,12 +413,12 @@ __global__ __launch_bounds__((64 * Lay<TI, NK>::WAVES), 2) void delta_chain_kern
       if (g) {
 #pragma unroll
         for (int i = 0; i < g_bytes(NT); i += 2048)
-          __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(p + i), (__attribute__((address_space(3))) void*)(to + i), 16, 0, 0);
+          __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(p + i), (__attribute__((address_space(3))) void*)(to + i), 16, 0, 2);
       }
       const char* r = ws + (size_t)min(cr, chunks - 1) * H * EACH + g_bytes(NT) + 1024 * odd + 16 * lane;
 #pragma unroll
       for (int i = 0; i < REST; i += 2048)
-        __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(r + i), (__attribute__((address_space(3))) void*)(rest(cr) + 1024 * odd + i), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(r + i), (__attribute__((address_space(3))) void*)(rest(cr) + 1024 * odd + i), 16, 0, 2);
     };
     fetch(0, true, 0);
     if (L::RN == 4) fetch(0, false, 1);

@@ -1186,14 +1186,14 @@ extern "C" int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows
 
 // Floats of workspace (`parts`, `parts_chunks` chunks) that a step of delta layers needs for chunk_delta.hip; 0: it does not go there.  Its chain takes 32
 // tokens in little more than chunk_scan.hip takes for 16, but what it prepares costs 0.2 ns a row and head, and a compute unit has one workgroup of
-// it: up to 64 channels it is the faster for long portions whose workgroups find a unit each (us there, here, 64 channels: heads, sequences x rows: 64, 1 x 512
-// 46, 42; 64, 2 x 512 48, 50; 16, 8 x 512 48, 52; 64, 1 x 1024 82, 60; 32, 4 x 1024 85, 77; 16, 8 x 1024 87, 76; 64, 4 x 1024 125, 160), of 128 (bf16 rows) from
-// some 300 rows on (32 heads: 2 x 256 44, 45; 8 x 384 218, 141; 8 x 1024 507, 412).
+// it: up to 64 channels it is the faster for long portions whose workgroups find a unit each (us there, here, heads, sequences x rows: fp32 64, 1 x 512
+// 45, 40; 64, 2 x 512 47, 50; 16, 8 x 512 47, 50; 64, 1 x 1024 82, 60; 32, 4 x 1024 83, 75; 16, 8 x 1024 84, 74; 64, 4 x 1024 125, 151; bf16 64, 1 x 384 36, 33;
+// 16, 8 x 384 39, 35; 64, 4 x 384 55, 62), of 128 (bf16 rows) from some 300 rows on (32 heads: 2 x 256 44, 45; 2 x 384 58, 47; 8 x 384 216, 149; 8 x 1024 506, 352).
 extern "C" long long dgi_linear_scan_parts(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k,
                                            int k_stride, int in_f32, int* parts_chunks) {
   if (mode != DELTA || n_seq == 0 || chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows) != 1) return 0;
   const long units = (long)n_seq * H * ((dv + 31) / 32);
-  if (dk <= 64 ? rows < 768l * n_seq || units > 256 : rows < 320l * n_seq || units > 512) return 0;
+  if (dk <= 64 ? rows < (in_f32 ? 768l : 384l) * n_seq || units > 256 : rows < 320l * n_seq || units > 512) return 0;
   return dgi_chunk_delta_floats(dk, H, rows, n_seq, in_f32, parts_chunks);
 }
 
