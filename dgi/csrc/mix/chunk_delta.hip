@@ -17,12 +17,12 @@
 // What bounds it: a chunk of the chain takes 1.4 us (chunk_scan.hip: 1.2 for sixteen tokens), 48 products of 16 cycles and 230 vector instructions, which
 // one wave does not overlap (alone on its unit the state waves would take 1.03); preparing 4096 rows of 64 heads 51 us, 150 MB of G and P M to memory, which
 // nothing reads soon, and then once: stores and loads say so (without, they take the place of q, k and v in the caches, 170 us for 149).  Two
-// prompts of 4096 rows in all, 64 heads of 64 x 64: 178 us -> 149; one of 2048 rows 154 -> 103; bf16 rows of
+// prompts of 4096 rows in all, 64 heads of 64 x 64: 178 us -> 144; one of 2048 rows 154 -> 103; bf16 rows of
 // 128 channels, 4 of 1024 rows, 32 heads, 255 -> 157.  Only long portions are taken, see
 // dgi_linear_scan_parts.  Tried: M and P themselves prepared, u by a product more in the chain: 122 us a chain for 105; two state waves a block of columns, half
 // the channels each: 138 for 142 without the rest (x is both's, and the unit has no instructions to spare).
 //
-// Precision: outputs and states are closer to 64 bits than the token loop's and chunk_scan.hip's (2-norm, 512 fp32 rows: 1.14e-7 and 1.9e-8; the loop 1.36e-7,
+// Precision: outputs and states are closer to 64 bits than the token loop's and chunk_scan.hip's (2-norm, 512 fp32 rows: 1.12e-7 and 1.9e-8; the loop 1.36e-7,
 // 2.1e-8).
 #include <type_traits>
 #include "chunk_split.h"
@@ -155,8 +155,14 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(const ChunkArgs a
         kf[2][p] = kt[1][p] = kt[2][p] = kp[b][1][p];
         qt[1][p] = qt[2][p];
       }
-      multiply<PQ, PQ, 3, 3>(kf, kt, kl, kk);
-      multiply<PQ, PQ, 3, 3>(kf, qt, ql, qk);
+      // the last block's first parts start from the small ones' sum: one rounding less at the sum's size
+      small<PQ, PQ, 3, 3>(kf, kt, kl);
+      small<PQ, PQ, 3, 3>(kf, qt, ql);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        (b + 1 < NK ? kk : kl)[i] = mfma(kf[i][0], kt[i][0], (b + 1 < NK ? kk : kl)[i]);
+        (b + 1 < NK ? qk : ql)[i] = mfma(kf[i][0], qt[i][0], (b + 1 < NK ? qk : ql)[i]);
+      }
     }
 #pragma unroll
     for (int p = 0; p < PQ; ++p) {
@@ -555,7 +561,9 @@ __global__ __launch_bounds__((64 * Lay<TI, NK>::WAVES), 2) void delta_chain_kern
         read_rows(sm + L::Q + (c & 1) * L::ARRB, b, x);
 #pragma unroll
         for (int j = 0; j < 3; ++j) sp[0][j] = *parts_at(c, b, j);
-        multiply<PQ, 3, 2, 1>(x, sp, lo, hi);
+        small<PQ, 3, 2, 1>(x, sp, lo);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) (b + 1 < NK ? hi : lo)[h] = mfma(x[h][0], sp[0][0], (b + 1 < NK ? hi : lo)[h]);
       }
 #pragma unroll
       for (int h = 0; h < 2; ++h) qS[h] = hi[h] + lo[h];

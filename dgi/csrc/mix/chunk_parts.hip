@@ -26,12 +26,12 @@
 // wave's own products (16 cycles) and vector instructions do not overlap, only those of two waves of a SIMD do, in part.  So state and read-out are two
 // waves', parts of the next operand are made between the products, what goes token by token is kept out of the loops' registers, and operands
 // are asked for a chunk ahead (as buffers: a row is a scalar offset).  Measured against chunk_scan.hip, sixteen tokens at a time in fp32 products, on inputs that change from pass to pass:
-//   ssm, 2 prompts of 4096 rows, 64 heads of 128 x 64     210 us -> 170 (of it 20 the pass before)
+//   ssm, 2 prompts of 4096 rows, 64 heads of 128 x 64     210 us -> 168 (of it 20 the pass before)
 //   mlstm, 5 prompts of 3001 bf16 rows, 32 heads of 64     83 -> 49;  of 128 197 -> 137;  fp32 rows 105 -> 74
 //   light, 2 prompts of 4096 bf16 rows, 64 heads of 64    158 -> 113
 // mlstm on fp32 rows of 128 channels stays there (its waves would spill: 213 -> 230 us); delta: chunk_delta.hip.
 //
-// Precision: results and states are no further from 64 bits than the token loop's (2-norm, 512 rows: ssm 7.9e-8, the loop 1.03e-7; states of mlstm
+// Precision: results and states are no further from 64 bits than the token loop's (2-norm, 512 rows: ssm 7.3e-8, the loop 1.03e-7; states of mlstm
 // 3.1e-8, 4.4e-8): decays are summed as logarithms in 64 bits and a running maximum is kept in 64 bits, since its rounding would be the state's.
 #include <type_traits>
 #include "chunk_split.h"
@@ -209,7 +209,9 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK>::WAVES), (Lay<MODE, TI, NK>
           }
 #pragma unroll
         for (int p = 0; p < PQ; ++p) { kf[1][p] = kf[0][p]; qf[1][p] = qf[2][p]; }
-        multiply<PQ, PQ, 3, 3>(kf, qf, lo, hi);
+        small<PQ, PQ, 3, 3>(kf, qf, lo);             // as read_out's sums
+#pragma unroll
+        for (int i = 0; i < 3; ++i) (b + 1 < NK ? hi : lo)[i] = mfma(kf[i][0], qf[i][0], (b + 1 < NK ? hi : lo)[i]);
       }
 #pragma unroll
       for (int i = 0; i < 3; ++i) qk[i] = hi[i] + lo[i];
@@ -1082,7 +1084,8 @@ __global__ __launch_bounds__(256) void ssm_parts_kernel(const ChunkArgs a) {
       kf[0][p] = *reinterpret_cast<const u32x4*>(sm + L::ARRB + p * L::PARTB + place(16 * s + n16, 4 * b + g));
       qf[0][p] = *reinterpret_cast<const u32x4*>(sm + p * L::PARTB + place(16 * t + n16, 4 * b + g));
     }
-    multiply<3, 3, 1, 1>(kf, qf, l1, h1);
+    small<3, 3, 1, 1>(kf, qf, l1);                     // as read_out's sums: the last block's first parts start from the small ones'
+    (b + 1 < NK ? h1 : l1)[0] = mfma(kf[0][0], qf[0][0], (b + 1 < NK ? h1 : l1)[0]);
   }
   *reinterpret_cast<f32x4*>(to + 2 * L::ARRB + 1024 * wave + 16 * lane) = h1[0] + l1[0];
 }
