@@ -14,8 +14,8 @@
 // the barrier), output waves a chunk behind them, waves that fetch what was prepared and waves that bring k and q in parts.  fp32 operands are three bf16
 // parts each (chunk_parts.hip).
 //
-// What bounds it: a chunk of the chain takes 1.4 us (chunk_scan.hip: 1.2 for sixteen tokens), 48 products of 16 cycles and 230 vector instructions, which
-// one wave does not overlap (alone on its unit the state waves would take 1.03); preparing 4096 rows of 64 heads 51 us, 150 MB of G and P M to memory, which
+// What bounds it: a chunk of the chain takes 1.3 us (chunk_scan.hip: 1.2 for sixteen tokens), 48 products of 16 cycles and 230 vector instructions, which
+// one wave does not overlap (alone on its unit the state waves would take 1.03); preparing 4096 rows of 64 heads 50 us, 150 MB of G and P M to memory, which
 // nothing reads soon, and then once: stores and loads say so (without, they take the place of q, k and v in the caches, 170 us for 149).  Two
 // prompts of 4096 rows in all, 64 heads of 64 x 64: 178 us -> 144; one of 2048 rows 154 -> 103; bf16 rows of
 // 128 channels, 4 of 1024 rows, 32 heads, 255 -> 157.  Only long portions are taken, see
