@@ -174,14 +174,14 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   // offset of chunk ch inside a key / value row
   auto kch = [&](int ch) { return PAD ? min(ch * 8, dk - 8) : ch * 8; };
   auto vch = [&](int ch) { return PAD ? min(ch * 8, dv - 8) : ch * 8; };
-  // RW rows of a tile are staged by each wave, 1 KB (64 / CH rows) a load, one behind the other in LDS; of full tiles of
-  // 16-token pages (the engine's page size) they lie in one page, one behind the other there too, so that its loads share
-  // one id and one address and differ in their instruction's offset.  The swizzle is in which chunk of its row a lane loads.
+  // RW rows of a tile are staged by each wave, 1 KB (64 / CH rows) a load, one behind the other in LDS; in pages of at least RW tokens (the
+  // engine's have 16) they lie in one page, one behind the other there too, so that its loads share one id and one address and
+  // differ in their instruction's offset.  The swizzle is in which chunk of its row a lane loads.
   constexpr int RW = KT / NW;                                      // rows of a tile a wave stages
   constexpr int NP = RW * CH / 64, NPV = RW * CHV / 64;            // its loads of keys and of values
   static_assert(16 % RW == 0 && NP >= 1 && NPV >= 1, "a wave's rows lie in one page");
   const int row0 = w * RW;
-  const bool page16 = bs_log2 == 4;
+  const bool whole_rows = bs >= RW;
   int k_at[NP], v_at[PAD ? NPV : 1];       // bytes from the wave's first row (whole rows: less the load's offset)
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -195,14 +195,17 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   }
   int none = 0;
   asm("" : "+v"(none));                   // a vector load: a scalar one's wait would be one for all reads of LDS
-  auto read_id = [&](int kb0) __attribute__((always_inline)) { return bt[(min(kb0 + row0, kv_end - 1) >> 4) + none]; };
-  auto full = [&](int kb0) __attribute__((always_inline)) { return page16 && kb0 + KT <= kv_end; };
-  // the page of a full tile's rows, and load l of its NP + NPV
+  // the page of the wave's rows of a tile, or of this lane's row of them where they have several
+  auto read_id = [&](int kb0) __attribute__((always_inline)) {
+    return whole_rows ? bt[(min(kb0 + row0, kv_end - 1) >> bs_log2) + none] : bt[min(kb0 + row0 + lane % RW, kv_end - 1) >> bs_log2];
+  };
+  auto full = [&](int kb0) __attribute__((always_inline)) { return whole_rows && kb0 + KT <= kv_end; };
+  // rows of the page from a key on, and load l of the NP + NPV of a full tile
   __amdgpu_buffer_rsrc_t k_rows, v_rows;
-  auto at_page = [&](int id) __attribute__((always_inline)) {
+  auto at_page = [&](int id, int key) __attribute__((always_inline)) {
     const size_t blk = (size_t)__builtin_amdgcn_readfirstlane(id) * nkv + kvh;
-    k_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(k_cache + blk * head_stride + (row0 & 15) * dk), 0, RW * dk * 2, 0x00027000);
-    v_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(v_cache + blk * v_head_stride + (row0 & 15) * dv), 0, RW * dv * 2, 0x00027000);
+    k_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(k_cache + blk * head_stride + (key & (bs - 1)) * dk), 0, RW * dk * 2, 0x00027000);
+    v_rows = __builtin_amdgcn_make_buffer_rsrc((void*)(v_cache + blk * v_head_stride + (key & (bs - 1)) * dv), 0, RW * dv * 2, 0x00027000);
   };
   auto load = [&](auto l_, int stage) __attribute__((always_inline)) {
     constexpr int l = decltype(l_)::value, p = l < NP ? l : l - NP;
@@ -210,32 +213,50 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     if constexpr (PAD) load_chunk<0>(l < NP ? k_rows : v_rows, l < NP ? k_at[l < NP ? p : 0] : v_at[l < NP ? 0 : p], at + 1024 * p);
     else load_chunk<1024 * p>(l < NP ? k_rows : v_rows, l < NP ? k_at[p] : v_at[0], at);
   };
-  // rows of a tile that ends early, or of pages of another size: each lane finds its own
-  auto load_part = [&](int kb0, int stage) __attribute__((always_inline)) {
+  // A tile that ends early, or whose rows have several pages: each lane finds its own, no row is after the last key.  The ids
+  // are there by now: read here, each load would wait for its id and so for all loads before it (32 heads of 128, pages of
+  // 32: 8192 rows 798 us, so 511; 3000 rows behind 5000 636, so 338; pages of 8: 816, 568 and 654, 355).
+  auto load_part = [&](int kb0, int stage, int id) __attribute__((always_inline)) {
     const lds_ptr kl = (lds_ptr)(lds + stage * KT * (HD + HDV) + row0 * HD), vl = (lds_ptr)(lds + stage * KT * (HD + HDV) + KT * HD + row0 * HDV);
+    const int first = min(kb0 + row0, kv_end - 1), last = kv_end - 1 - first;
     int part = lane;
     asm volatile("" : "+v"(part));      // computed here: kept from before the loop its addresses would cost registers
+    if (whole_rows) {
+      at_page(id, first);
 #pragma unroll 1
-    for (int p = 0; p < NP; ++p) {
-      const int row = row0 + p * (64 / CH) + part / CH, key = min(kb0 + row, kv_end - 1);
-      load_chunk((const char*)(k_cache + ((size_t)bt[key >> bs_log2] * nkv + kvh) * head_stride + (size_t)(key & (bs - 1)) * dk +
-                               kch(k_slot<HD>(row, part % CH))), kl + p * 1024);
+      for (int p = 0; p < NP; ++p) {
+        const int row = p * (64 / CH) + part / CH;
+        load_chunk<0>(k_rows, 2 * (min(row, last) * dk + kch(k_slot<HD>(row0 + row, part % CH))), kl + p * 1024);
+      }
+#pragma unroll 1
+      for (int p = 0; p < NPV; ++p) {
+        const int row = p * (64 / CHV) + part / CHV;
+        load_chunk<0>(v_rows, 2 * (min(row, last) * dv + vch(v_slot<HDV>(row0 + row, part % CHV))), vl + p * 1024);
+      }
+      return;
     }
-#pragma unroll 1
+    // rows of keys and of values of load p: the page and the row in it
+    auto at = [&](int row) __attribute__((always_inline)) { return (size_t)__shfl(id, row, 64) * nkv + kvh; };
+    auto in = [&](int row) __attribute__((always_inline)) { return min(kb0 + row0 + row, kv_end - 1) & (bs - 1); };
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int row = p * (64 / CH) + part / CH;
+      load_chunk((const char*)(k_cache + at(row) * head_stride + (size_t)in(row) * dk + kch(k_slot<HD>(row0 + row, part % CH))), kl + p * 1024);
+    }
+#pragma unroll
     for (int p = 0; p < NPV; ++p) {
-      const int row = row0 + p * (64 / CHV) + part / CHV, key = min(kb0 + row, kv_end - 1);
-      load_chunk((const char*)(v_cache + ((size_t)bt[key >> bs_log2] * nkv + kvh) * v_head_stride + (size_t)(key & (bs - 1)) * dv +
-                               vch(v_slot<HDV>(row, part % CHV))), vl + p * 1024);
+      const int row = p * (64 / CHV) + part / CHV;
+      load_chunk((const char*)(v_cache + at(row) * v_head_stride + (size_t)in(row) * dv + vch(v_slot<HDV>(row0 + row, part % CHV))), vl + p * 1024);
     }
   };
   int id = 0;
   if (kv_end > kv_begin) {
-    if (page16) id = read_id(kv_begin);
+    id = read_id(kv_begin);
     if (full(kv_begin)) {
-      at_page(id);
+      at_page(id, kv_begin + row0);
       each<0, NP + NPV>([&](auto l) __attribute__((always_inline)) { load(l, 0); });
-    } else load_part(kv_begin, 0);
-    if (page16) id = read_id(kv_begin + KT);
+    } else load_part(kv_begin, 0, id);
+    id = read_id(kv_begin + KT);
   }
   // LDS addresses of this lane's operands in stage 0: keys lr (the second 32 are 64 HD bytes on), dims 16 s + 8 hh ..; values
   // of dims 32 d .., keys 4 hh + tq (16 j + 8 more are 32 HDV j and 16 HDV bytes on)
@@ -268,10 +289,10 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     __syncthreads();
     const bool next = full(kb0 + KT);
     if (next) {
-      at_page(id);
+      at_page(id, kb0 + KT + row0);
       each<0, NP + NPV>([&](auto l) __attribute__((always_inline)) { load(l, 1 - stage); });
-    } else if (kb0 + KT < kv_end) load_part(kb0 + KT, 1 - stage);
-    if (page16) id = read_id(kb0 + 2 * KT);
+    } else if (kb0 + KT < kv_end) load_part(kb0 + KT, 1 - stage, id);
+    id = read_id(kb0 + 2 * KT);
     if (kb0 > wave_last_pos || !wave_rows || (MASKED && kb0 + KT <= wave_min_first)) return;
     // ---- S^T = K Q^T for two 32-key blocks: the first block's operands are all under way before its products, the
     // second's come between them, the first values between the second's (left to itself the compiler waits out an LDS read

@@ -87,3 +87,36 @@ def test_first_keys_anywhere_in_a_tile(window, block):
         return (j <= p) & (j > p - window if window else j >= p // block * block)
 
     _check(out, *case, 4, 2, hd, visible)
+
+
+@pytest.mark.parametrize("hd,vd", [(64, 64), (128, 128), (96, 40)])
+@pytest.mark.parametrize("page", [2, 8, 64, 256])
+def test_pages_of_any_size(hd, vd, page):
+    """A wave's rows of a tile have several pages, or lie anywhere in one; ends in the middle of a wave's rows and before them."""
+    q, kc, vc, table, cu, ctx = _case(4, 2, hd, page, [1, 40, 129, 200], [300, 40, 263, 500], 3)
+    out = mix.paged_prefill_masked(q, kc, vc[..., :vd].contiguous(), table, cu, ctx, 4, 2, hd ** -0.5, 0, None)
+    padded = torch.zeros(*out.shape[:-1], 4 * hd, dtype=out.dtype, device="cuda").view(-1, 4, hd)
+    padded[..., :vd] = out.view(-1, 4, vd)
+    vc[..., vd:] = torch.where(vc[..., vd:].isnan(), vc[..., vd:], 0)
+    _check(padded.view(-1, 4 * hd), q, kc, vc, table, cu, ctx, 4, 2, hd, _causal)
+
+
+@pytest.mark.parametrize("page", [8, 32, 64])
+def test_pages_cost_the_same(page):
+    """Blocks' ids are there before the rows they name are asked for: pages of other sizes take little longer than those of 16 (half as long
+    again where every load waits for its own id)."""
+    def best(page):
+        case = _case(32, 8, 128, page, [2000], [4000], 1)
+        tiles = torch.from_numpy(ops.order_prefill_tiles([0, 2000], [4000])).cuda()
+        times = []
+        for i in range(8):
+            e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            e[0].record()
+            for _ in range(10):
+                ops.paged_prefill(*case, 32, 8, 128 ** -0.5, tiles=tiles)
+            e[1].record()
+            e[1].synchronize()
+            times.append(e[0].elapsed_time(e[1]))
+        return min(times)
+
+    assert best(page) <= 1.25 * best(16)
