@@ -185,6 +185,9 @@ void paged_decode(at::Tensor out, const at::Tensor& q, const at::Tensor& k_cache
            "paged_decode");
 }
 
+// prompt attention loads a cache straight to LDS, 16 bytes a lane: one that lies off such a boundary is copied
+at::Tensor by_16_bytes(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t; }
+
 void paged_prefill(at::Tensor out, const at::Tensor& q, const at::Tensor& k_cache,
                    const at::Tensor& v_cache, const at::Tensor& block_tables,
                    const at::Tensor& cu_seqlens_q, const at::Tensor& context_lens,
@@ -204,7 +207,8 @@ void paged_prefill(at::Tensor out, const at::Tensor& q, const at::Tensor& k_cach
     TORCH_CHECK(tree_mask->size(-1) == 64 && tree_mask->numel() >= 64 * (cu_seqlens_q.numel() - 1));
     tm = reinterpret_cast<const unsigned long long*>(tree_mask->data_ptr<int64_t>());
   }
-  check_rc(dgi_paged_prefill(q.data_ptr(), (int)q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
+  const at::Tensor k_at = by_16_bytes(k_cache), v_at = by_16_bytes(v_cache);
+  check_rc(dgi_paged_prefill(q.data_ptr(), (int)q.stride(0), k_at.data_ptr(), v_at.data_ptr(),
                              block_tables.data_ptr<int>(), (int)block_tables.stride(0),
                              cu_seqlens_q.data_ptr<int>(), context_lens.data_ptr<int>(),
                              tiles.data_ptr<int>(), (int)tiles.size(0), out.data_ptr(),

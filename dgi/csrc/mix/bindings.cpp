@@ -310,6 +310,9 @@ void masked_attn_rows(at::Tensor out, const at::Tensor& q, const at::Tensor& k_c
 
 // bf16, key size == value size in {64, 128}: packed prompt portions (cu_seqlens_q) over
 // [cached prefix | new keys]; tiles [n, 2] = (sequence, first row of a 128-row tile)
+// prompt attention loads a cache straight to LDS, 16 bytes a lane: one that lies off such a boundary is copied
+at::Tensor by_16_bytes(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t; }
+
 void paged_prefill_masked(at::Tensor out, const at::Tensor& q, const at::Tensor& k_cache, const at::Tensor& v_cache,
                           const at::Tensor& block_tables, const at::Tensor& cu_seqlens_q, const at::Tensor& context_lens,
                           const at::Tensor& tiles, int64_t nh, int64_t nkv, double scale, int64_t mask,
@@ -358,7 +361,8 @@ void paged_prefill_masked(at::Tensor out, const at::Tensor& q, const at::Tensor&
     dbp = dist_bias->data_ptr<float>();
     ndist = (int)dist_bias->size(0);
   }
-  check_rc(dgi_paged_prefill_masked(q.data_ptr(), (int)q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
+  const at::Tensor k_at = by_16_bytes(k_cache), v_at = by_16_bytes(v_cache);
+  check_rc(dgi_paged_prefill_masked(q.data_ptr(), (int)q.stride(0), k_at.data_ptr(), v_at.data_ptr(),
                                     block_tables.data_ptr<int>(), (int)block_tables.stride(0), cu_seqlens_q.data_ptr<int>(),
                                     context_lens.data_ptr<int>(), tiles.data_ptr<int>(), (int)tiles.size(0), out.data_ptr(),
                                     (int)out.stride(0), (int)nh, (int)nkv, hd, hv, (int)k_cache.size(2), (float)scale, (int)mask,

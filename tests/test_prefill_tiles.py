@@ -120,3 +120,22 @@ def test_pages_cost_the_same(page):
         return min(times)
 
     assert best(page) <= 1.25 * best(16)
+
+
+@pytest.mark.parametrize("form", ["plain", "masked"])
+def test_caches_off_sixteen_bytes(form):
+    """Caches that start between two 16-byte boundaries, which loads straight to LDS cannot take."""
+    case = list(_case(4, 2, 64, 16, [70, 200], [100, 200], 7))
+
+    def call(c):
+        if form == "plain":
+            return ops.paged_prefill(*c, 4, 2, 0.125)
+        return mix.paged_prefill_masked(*c, 4, 2, 0.125, 0, None)
+
+    want = call(case)
+    for i in (1, 2):
+        x = torch.empty(case[i].numel() + 8, dtype=torch.bfloat16, device="cuda")[i:][: case[i].numel()].view(case[i].shape)
+        assert x.data_ptr() % 16 and x.is_contiguous()
+        x.copy_(case[i])
+        case[i] = x
+    assert torch.equal(call(case), want)
