@@ -46,6 +46,9 @@ typedef const __attribute__((address_space(1))) char* global_in;
 typedef __attribute__((address_space(1))) char* global_out;
 template <typename V> __device__ __forceinline__ V gload(global_in p) { return *reinterpret_cast<const __attribute__((address_space(1))) V*>(p); }
 __device__ __forceinline__ void gstore(global_out p, float v) { *reinterpret_cast<__attribute__((address_space(1))) float*>(p) = v; }
+// the same as flat accesses, where those measured faster (chunk_scan.hip)
+template <typename V> __device__ __forceinline__ V gload(const char* p) { return *reinterpret_cast<const V*>(p); }
+__device__ __forceinline__ void gstore(char* p, float v) { *reinterpret_cast<float*>(p) = v; }
 
 // Rows of a chunk as a buffer: the first row's address and the rows' offsets are scalars, a lane's offset is kept; lane offsets beyond the bytes read
 // zeros and write nothing (a row offset is not looked at, so it is added to the lane's where rows may be missing).
