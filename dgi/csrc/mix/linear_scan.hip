@@ -1143,9 +1143,15 @@ constexpr int APART_FROM = 8;        // sequences of a step above which those ar
 // 90, 103; 4096, 100, 362, 335).  light is up against chunk_scan_decay.hip (that one's time and chunk_parts.hip's: 256 units, 100 rows 11, 12; 160 rows 14,
 // 13; 400 rows 31, 25; 512 units, 100 rows 16, 12; 1024 units, 64 rows 20, 17; 2048 units, 64 rows 36, 35; 128-wide heads: 128 units, 100 rows 15, 15;
 // 1024 units, 64 rows 30, 25; 4096 units, 64 rows 108, 91).
+// Among more than APART_FROM sequences it has a launch more to lose (64-wide heads: 9 x 80 rows, 16 heads 17, 20; 12 x 112 22, 24; 12 x 128 24, 24; 9 x 80, 32
+// heads 24, 28; 9 x 96 28, 28; 24 x 65, 32 heads 52, 49; 128-wide: 9 x 80, 8 heads 24, 27; 9 x 96 28, 27).
 static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
   const long units = (long)n_seq * H * ((dv + 15) / 16);
-  if (mode == LIGHT) return units > 256 ? 64 : 128;
+  if (mode == LIGHT) {
+    if (n_seq <= APART_FROM) return units > 256 ? 64 : 128;
+    if (units <= 768) return dk <= 64 ? 112 : 88;
+    return dk <= 64 && (units <= 1280 || n_seq <= 16) ? 88 : 64;
+  }
   if (mode != WKV || units <= 512) return 64;
   return dk > 64 ? 104 : units <= 3072 ? 136 : 224;
 }
