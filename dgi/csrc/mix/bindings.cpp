@@ -71,6 +71,7 @@ int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const void* dt_raw,
                  int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t s);
 long long dgi_ssm_parts_floats(int dk, int H, int G, int T, int n_seq, int* chunks);
 int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg_rows);
+int dgi_ssm_whole(int n_seq, int heads, int dv, int N, int G, int rows, int segs);
 int dgi_gated_group_norm(void* out, int out_f32, const float* y, const void* z, int z_f32, int z_stride, const float* w,
                          int T, int C, int groups, float eps, hipStream_t s);
 int dgi_moe_route(int* idx, float* wts, const float* logits, int l_stride, const float* corr, int T, int R, int top,
@@ -509,7 +510,8 @@ void ssm_scan(at::Tensor y, const at::Tensor& xbc, const at::Tensor& dt_raw, con
   at::Tensor ws, wsd, parts;
   if (chunked && n_seq > 0) {
     segs = dgi_ssm_segments(n_seq, (int)heads, (int)dv, T, &seg_rows);
-    // what the heads of a group share (chunk_parts.hip)
+    if (G > 0 && dgi_ssm_whole(n_seq, (int)heads, (int)dv, (int)N, (int)G, T, segs)) segs = 1;
+    // what the heads of a group share, where a pass before makes it (chunk_parts.hip)
     const long long floats = G > 0 ? dgi_ssm_parts_floats((int)N, (int)heads, (int)G, T, n_seq, &parts_chunks) : 0;
     if (floats > 0) parts = at::empty({floats}, state.options());
   }

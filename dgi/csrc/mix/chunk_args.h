@@ -87,6 +87,6 @@ __device__ __forceinline__ float larger3(float m, float a, float b) {
 
 }  // namespace
 
-bool dgi_chunk_parts_takes(int mode, int dk, int in_f32);
+bool dgi_chunk_parts_takes(int mode, int dk, int H, int G, int in_f32);
 int dgi_chunk_parts(const ChunkArgs& a, int mode, int in_f32, dim3 grid, hipStream_t st);
 int dgi_chunk_delta(const ChunkArgs& a, int in_f32, dim3 grid, hipStream_t st);

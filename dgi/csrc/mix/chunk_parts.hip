@@ -14,8 +14,8 @@
 //
 // A workgroup owns (sequence, head, two blocks of 16 value columns) and is a pipeline of waves that hand chunks on through LDS, one barrier
 // per chunk:
-//   preparing waves  load q and k a chunk ahead in registers and write their parts to LDS (ssm: parts and scores come from a pass before, as the heads
-//                    of a group and their columns share them);
+//   preparing waves  load q and k a chunk ahead in registers and write their parts to LDS (ssm of more than 64 channels, long steps: parts and scores come
+//                    from a pass before, as the heads of a group and their columns share them);
 //   gates wave       sums of log2 decays of 64 tokens at a time (in 64 bits), as whole number and fraction, A and F;
 //   scores wave      q . k and P in parts;
 //   state waves      one per block of 16 columns: the state's rows of all channels in registers, in the layout the products leave them, which is
@@ -26,7 +26,7 @@
 // wave's own products (16 cycles) and vector instructions do not overlap, only those of two waves of a SIMD do, in part.  So state and read-out are two
 // waves', parts of the next operand are made between the products, what goes token by token is kept out of the loops' registers, and operands
 // are asked for a chunk ahead (as buffers: a row is a scalar offset).  Measured against chunk_scan.hip, sixteen tokens at a time in fp32 products, on inputs that change from pass to pass:
-//   ssm, 2 prompts of 4096 rows, 64 heads of 128 x 64     210 us -> 168 (of it 20 the pass before)
+//   ssm, 2 prompts of 4096 rows, 64 heads of 128 x 64     210 us -> 168 (of it 15 the pass before)
 //   mlstm, 5 prompts of 3001 bf16 rows, 32 heads of 64     83 -> 49;  of 128 197 -> 137;  fp32 rows 105 -> 74
 //   light, 2 prompts of 4096 bf16 rows, 64 heads of 64    158 -> 113
 // mlstm on fp32 rows of 128 channels stays there (its waves would spill: 213 -> 230 us); delta: chunk_delta.hip.
@@ -40,10 +40,10 @@ using namespace dgi;
 
 namespace {
 
-template <int MODE, typename TI, int NK_>
+template <int MODE, typename TI, int NK_, bool PRE_ = false>
 struct Lay {
   static constexpr int NK = NK_, DP = 32 * NK, NT = 2 * NK, NB = 2;       // dk <= DP, 16-channel tiles, column blocks
-  static constexpr bool PRE = MODE == SSM;                     // parts and scores were made before
+  static constexpr bool PRE = PRE_;                            // ssm: parts and scores were made before
   static constexpr int PQ = sizeof(TI) == 2 && MODE != LIGHT ? 1 : 3, PU = sizeof(TI) == 2 && MODE == MLSTM ? 1 : 3;      // parts of q and k, of u
   // Waves: state, output, normaliser, gates, scores, preparing; waves four apart share a SIMD
   static constexpr int NP = PRE ? 0 : PQ == 1 ? (NK == 2 ? 1 : 2) : MODE == MLSTM ? (NK == 2 ? 2 : 4) : 4;
@@ -73,9 +73,9 @@ constexpr int EI = 0, EF = 32, BI = 64, BF = 96, GA = 128, GF = 160, RA = 192, R
 // ssm, of each chunk and group: the parts, three score tiles and a flag (a multiple of 16 bytes)
 __host__ __device__ constexpr int parts_floats(int DP) { return 2 * 3 * C * DP / 2 + 3 * 256 + 4; }
 
-template <int MODE, typename TI, int NK>
-__global__ __launch_bounds__((64 * Lay<MODE, TI, NK>::WAVES), (Lay<MODE, TI, NK>::PER_SIMD)) void chunk_parts_kernel(const ChunkArgs a) {
-  using L = Lay<MODE, TI, NK>;
+template <int MODE, typename TI, int NK, bool PRE>
+__global__ __launch_bounds__((64 * Lay<MODE, TI, NK, PRE>::WAVES), (Lay<MODE, TI, NK, PRE>::PER_SIMD)) void chunk_parts_kernel(const ChunkArgs a) {
+  using L = Lay<MODE, TI, NK, PRE>;
   constexpr int DP = L::DP, NT = L::NT, PQ = L::PQ, PU = L::PU, LEAD = L::LEAD;
   extern __shared__ __attribute__((aligned(16))) char sm[];
   // consecutive workgroups go to different XCDs: ssm: so that the heads of a group share one's cache (a multiple of 8 heads)
@@ -315,7 +315,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK>::WAVES), (Lay<MODE, TI, NK>
       } else if constexpr (MODE == SSM) {
         const size_t at = t * a.aux1_stride + head;
         ga = a.aux_bf16 ? bf16_to_f32(((const uint16_t*)a.aux1)[at]) : ((const float*)a.aux1)[at];
-        flag = *(const int*)((const char*)a.parts + ((size_t)(chunk0 + min(2 * b + (lane >> 5), chunks - 1)) * a.G + kvh) * parts_floats(DP) * 4 + 2 * L::ARRB + 3 * 1024);
+        if constexpr (L::PRE) flag = *(const int*)((const char*)a.parts + ((size_t)(chunk0 + min(2 * b + (lane >> 5), chunks - 1)) * a.G + kvh) * parts_floats(DP) * 4 + 2 * L::ARRB + 3 * 1024);
       }
     };
     double ld = 0., lc = 0.;                         // log2 of the decay;  mlstm: forget and input gate, natural
@@ -1003,9 +1003,9 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK>::WAVES), (Lay<MODE, TI, NK>
 
 // What the heads of a state-space group and their columns share, for every chunk: the parts of C and B as the waves' operands, the scores as the scores
 // wave holds them, whether something is not finite.  A workgroup owns (chunk, group).
-template <int NK>
 __global__ __launch_bounds__(256) void ssm_parts_kernel(const ChunkArgs a) {
-  using L = Lay<SSM, float, NK>;
+  constexpr int NK = 4;
+  using L = Lay<SSM, float, NK, true>;
   constexpr int DP = L::DP, PER = DP / 8, TASKS = 2 * C * PER / 256;
   extern __shared__ __attribute__((aligned(16))) char sm[];
   __shared__ int any_bad;
@@ -1092,26 +1092,27 @@ __global__ __launch_bounds__(256) void ssm_parts_kernel(const ChunkArgs a) {
 
 }  // namespace
 
-template <int MODE, typename TI, int NK>
+template <int MODE, typename TI, int NK, bool PRE = false>
 static int launch(const ChunkArgs& a, dim3 grid, hipStream_t st) {
-  constexpr int lds = Lay<MODE, TI, NK>::END;
+  constexpr int lds = Lay<MODE, TI, NK, PRE>::END;
   static_assert(lds <= 160 * 1024, "LDS");
-  auto kernel = chunk_parts_kernel<MODE, TI, NK>;
+  auto kernel = chunk_parts_kernel<MODE, TI, NK, PRE>;
   if (lds > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return (int)e;
   }
-  kernel<<<grid, 64 * Lay<MODE, TI, NK>::WAVES, lds, st>>>(a);
+  kernel<<<grid, 64 * Lay<MODE, TI, NK, PRE>::WAVES, lds, st>>>(a);
   return 0;
 }
 
-template <int NK>
 static int launch_ssm(const ChunkArgs& a, dim3 grid, hipStream_t st) {
+  if (a.dk <= 64) return launch<SSM, float, 2>(a, grid, st);
+  if (!a.parts) return launch<SSM, float, 4>(a, grid, st);
   if (a.pass != 2) {
-    constexpr int lds = 2 * Lay<SSM, float, NK>::ARRB;
-    ssm_parts_kernel<NK><<<dim3(a.G, a.parts_chunks), 256, lds, st>>>(a);
+    constexpr int lds = 2 * Lay<SSM, float, 4, true>::ARRB;
+    ssm_parts_kernel<<<dim3(a.G, a.parts_chunks), 256, lds, st>>>(a);
   }
-  return launch<SSM, float, NK>(a, grid, st);
+  return launch<SSM, float, 4, true>(a, grid, st);
 }
 
 template <int MODE>
@@ -1124,21 +1125,28 @@ static int launch_mode(const ChunkArgs& a, int in_f32, dim3 grid, hipStream_t st
   return a.dk <= 64 ? launch<MODE, uint16_t, 2>(a, grid, st) : launch<MODE, uint16_t, 4>(a, grid, st);
 }
 
-// Floats of workspace that state-space portions of dk channels in G groups need here (0: they are not taken), for T rows of n_seq sequences.
+// Floats of workspace of a state-space step whose parts and scores are made in a pass before (0: there is none), for T rows of n_seq sequences: steps of
+// 65 to 128 channels that are long, or may have a portion of 1500 rows (512 beside many decode rows).  The pass costs 3 us and its operands come from the L2s; without it every
+// workgroup makes them, on waves of their own.  us without and with, 128 channels (16, 64 heads): 4 x 256 rows 49, 54 and 48, 52; 4 x 400 61, 69 and 57, 69;
+// 8 x 192 24, 45 and 28, 47 (16, 32 heads); 600 beside 16 53, 67 and 50, 62; 2000 142, 144 and 120, 122 (16 heads beside 7 rows; 64 heads alone); 8 x 1000 of 64 heads 317 and 303.  Of 64 channels:
+// 8 x 80 rows, 16 heads 12 and 16; 4 x 1000, 32 heads 49 and 57; 2000, 64 heads 87 and 93; 4 x 2000, 16 heads 142 and 134.
 extern "C" long long dgi_ssm_parts_floats(int dk, int H, int G, int T, int n_seq, int* chunks) {
   *chunks = T / C + n_seq;
-  const long long floats = (long long)*chunks * G * parts_floats(dk <= 64 ? 64 : 128);
-  return dk > 128 || H < 4 * G || *chunks > 65535 || floats > 1ll << 28 ? 0 : floats;
+  if (dk <= 64 || !dgi_chunk_parts_takes(SSM, dk, H, G, 1) || !(T >= 320l * n_seq || T - n_seq >= 1536 || (T - n_seq >= 512 && T <= 48l * n_seq))) return 0;
+  const long long floats = (long long)*chunks * G * parts_floats(128);
+  return *chunks > 65535 || floats > 1ll << 28 ? 0 : floats;
 }
 
-bool dgi_chunk_parts_takes(int mode, int dk, int in_f32) { return mode == LIGHT ? dk <= 128 : mode == MLSTM && dk <= (in_f32 ? 64 : 128); }
+bool dgi_chunk_parts_takes(int mode, int dk, int H, int G, int in_f32) {
+  return mode == SSM ? dk <= 128 && H >= 4 * G : mode == LIGHT ? dk <= 128 : mode == MLSTM && dk <= (in_f32 ? 64 : 128);
+}
 
 // one launch of chunk_scan.hip's dgi_chunk_scan; grid: n_seq * H * (blocks of 32 value columns), segments
 int dgi_chunk_parts(const ChunkArgs& a, int mode, int in_f32, dim3 grid, hipStream_t st) {
   switch (mode) {
     case MLSTM: return launch_mode<MLSTM>(a, in_f32, grid, st);
     case LIGHT: return launch_mode<LIGHT>(a, in_f32, grid, st);
-    case SSM: return a.dk <= 64 ? launch_ssm<2>(a, grid, st) : launch_ssm<4>(a, grid, st);
+    case SSM: return launch_ssm(a, grid, st);
   }
   return -2;
 }

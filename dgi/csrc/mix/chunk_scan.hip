@@ -1137,8 +1137,8 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
   const dim3 grid((unsigned)(n_seq * nz * H), segs > 1 ? segs : 1);
   // more workgroups than compute units: possibly of four column blocks each
   const bool four = dv > 32 && n_seq <= MOST_SEQ && n_seq * nz * H > 256;
-  const bool by_parts = mode == SSM ? parts != nullptr : dgi_chunk_parts_takes(mode, dk, in_f32);
-  if (mode == SSM && parts && segs > 1 && seg_rows % 32) return -3;
+  const bool by_parts = dgi_chunk_parts_takes(mode, dk, H, G, in_f32);
+  if (by_parts && segs > 1 && seg_rows % 32) return -3;
   if (a.pass) {
     int rc = by_parts ? dgi_chunk_parts(a, mode, in_f32, grid, st) : launch_dims<SSM, float>(a, false, grid, st);
     if (rc) return rc;

@@ -115,6 +115,7 @@ __device__ __forceinline__ int ranked(const ChunkArgs& a, int seq) {
   if (a.n_seq > MOST_SEQ || a.n_seq == 1) return seq;
   const int lane = threadIdx.x & 63, i = min(lane, a.n_seq - 1);
   const int len = lane < a.n_seq ? max(a.seq_row0[i + 1] - a.seq_row0[i], 0) : -1;
+  if (!__any(len > a.skip_rows)) return seq;         // none is this launch's
   int before = 0;                                    // sequences that are longer, or as long and earlier
   for (int j = 0; j < a.n_seq; ++j) {
     const int other = __builtin_amdgcn_readlane(len, j);

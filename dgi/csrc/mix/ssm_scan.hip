@@ -267,6 +267,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st);
 
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
+bool dgi_chunk_parts_takes(int mode, int dk, int H, int G, int in_f32);
 
 // chunked: portions go 32 tokens at a time through the matrix cores (chunk_parts.hip; sixteen, chunk_scan.hip, where groups have fewer than four heads or
 // channels are more than 128).  Its workgroups have a
@@ -275,9 +276,10 @@ extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, 
 // wait for each other (64 columns, this file's time and that one's: 11 portions of 100 rows, 16 heads 35, 41; 128 rows 42, 41; 16 portions of 128
 // rows, 64 heads 158, 162; 200 rows 242, 222).  recur.scan_chunks decides for whole steps by the same lines: a change of one is a change of both.
 constexpr int APART_FROM = 8;
-static int apart_rows(int n_seq, int heads, int dv) {
+// In chunks of 32: 88 rows there (12 portions of 96 rows of 128 channels, 64 heads 88, 89; 128 rows 114, 104).
+static int apart_rows(int n_seq, int heads, int dv, int N, int G) {
   const long units = (long)n_seq * heads * ((dv + 63) / 64);
-  return n_seq <= APART_FROM ? 0 : units <= 128 ? 48 : units <= 256 ? 112 : 144;
+  return n_seq <= APART_FROM ? 0 : units <= 128 ? 48 : dgi_chunk_parts_takes(5, N, heads, G, 1) ? 88 : units <= 256 ? 112 : 144;
 }
 
 // Segments (of *seg_rows rows) that a chunked step's portions are cut into (1: whole portions).  Together they are as long as the step: a portion
@@ -299,6 +301,13 @@ extern "C" int dgi_ssm_segments(int n_seq, int heads, int dv, int rows, int* seg
   return segs;
 }
 
+// Whether such a step goes whole all the same: in chunks of 32 (chunk_parts.hip) a portion takes half to two thirds of the above, so three segments are too
+// few, and with more than 64 workgroups segments are worth it from 1024 rows on (us in segments, whole, 64 channels: 8 heads, 8 x 65 rows 25, 11; 600 rows
+// beside 7 45, 31; 16 heads, 4 x 192 29, 16; 600 beside 3 36, 31; 32 heads, 2 x 400 40, 26; 2 x 2000 120, 92).
+extern "C" int dgi_ssm_whole(int n_seq, int heads, int dv, int N, int G, int rows, int segs) {
+  return dgi_chunk_parts_takes(5, N, heads, G, 1) && (segs <= 3 || ((long)n_seq * heads * ((dv + 31) / 32) > 64 && rows - n_seq + 1 < 1024));
+}
+
 extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const void* dt_raw, int dt_f32, int dt_stride,
                             const float* dt_bias, const float* a_log, const float* d_skip, float* state,
                             const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int heads,
@@ -311,7 +320,7 @@ extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const vo
   int most = 0;
   const float* B = xbc + (size_t)heads * dv;
   if (chunked && dgi_chunk_scan_ok(5, N, B + (size_t)G * N, xbc_stride, B, xbc_stride, 1)) {
-    most = apart_rows(n_seq, heads, dv);
+    most = apart_rows(n_seq, heads, dv, N, G);
     const int rc = dgi_chunk_scan(y, 5, B + (size_t)G * N, xbc_stride, B, xbc_stride, xbc, xbc_stride, 1, dt_raw, dt_stride, nullptr, 0,
                                   !dt_f32, a_log, dt_bias, d_skip, 0.f, state, nullptr, nullptr, nullptr, nullptr, positions, seq_row0,
                                   seq_slots, n_seq, heads, G, N, dv, most, segs, seg_rows, ws, wsd, parts, parts_chunks, s);

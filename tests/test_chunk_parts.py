@@ -38,6 +38,24 @@ def test_segments(H, D, lens):
         check(run(d), oracle(d))
 
 
+@pytest.mark.parametrize("D,V", [(128, 33), (100, 48), (68, 16)])
+@pytest.mark.parametrize("lens", [[320], [333, 311], [319], [1027, 1, 0], [1025, 1]], ids=lambda x: "-".join(map(str, x)))
+def test_ssm_pass(D, V, lens):
+    """Long state-space steps of more than 64 channels: the parts come from a pass before, on either side of the lines from which they do; H = 8 in segments where one
+    portion may have 512 rows, H = 72 in whole portions."""
+    for H in (8, 72) if lens[0] > 1000 else (8,):
+        d = make("ssm", lens, H, D, V, torch.bfloat16, [3 * (i % 2) if n else 4 for i, n in enumerate(lens)], seed=D + H)
+        check(run(d), oracle(d))
+
+
+def test_ssm_same_with_and_without_the_pass():
+    """Beside an empty sequence the same 400 rows are a step without it: the same numbers, bit for bit."""
+    d = make("ssm", [400], 8, 128, 64, torch.bfloat16, [5])
+    y, S = run(d)
+    y2, S2 = run(dict(d, lens=[400, 0], past=[5, 5], S=torch.cat([d["S"][:1], d["S"]])))
+    assert torch.equal(y, y2) and torch.equal(S[1], S2[2])
+
+
 def where_finite(got, want):
     """The same values are finite, and they agree."""
     for a, b in zip(got, want):
@@ -67,6 +85,21 @@ def test_not_finite(mode, what):
             d["S"][1, 2, 3, 4] = bad
         slow = call(d, chunked=False) if mode == "ssm" else call(dict(d, pad=1))
         where_finite(run(d)[:2], slow[:2])
+
+
+@pytest.mark.parametrize("what", ["q", "k", "v", "gate", "state", "large"])
+def test_ssm_pass_not_finite(what):
+    """The same where the parts come from a pass before."""
+    for bad in (float("inf"), float("nan")) if what != "large" else (3.39e38,):
+        d = make("ssm", [330], 8, 128, 32, torch.float32, [3])
+        at = {"v": 3, "k": 8 * 32 + 5, "q": 8 * 32 + d["G"] * 128 + 5, "large": 8 * 32 + 5}.get(what)
+        if at is not None:
+            d["xbc"][171, at] = bad
+        elif what == "gate":
+            d["dt"][171, 2] = bad
+        else:
+            d["S"][1, 2, 3, 4] = bad
+        where_finite(run(d)[:2], call(d, chunked=False)[:2])
 
 
 def test_light_decays_that_are_none():

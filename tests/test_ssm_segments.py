@@ -39,3 +39,24 @@ def test_which_steps_go_in_chunks(monkeypatch):
     assert recur.scan_chunks(4096, 2, 64, 64, bf16, True)
     monkeypatch.setattr(recur, "SCAN_CHUNK", 0)
     assert not recur.scan_chunks(4096, 1, 64, 64, bf16) and not recur.scan_chunks(4096, 1, 64, 64, bf16, True)
+
+
+def test_short_portions_need_no_pass():
+    """Steps of short portions, and of up to 64 channels, have no launch before the one that does the work; with more than 64 workgroups only portions that may
+    have 1024 rows are cut."""
+    import torch  # noqa: F401
+    lib = ctypes.CDLL(dgi.build.build(group="mix"))
+    lib.dgi_ssm_parts_floats.restype = ctypes.c_longlong
+    chunks = ctypes.c_int()
+
+    def floats(dk, heads, groups, rows, n_seq):
+        return lib.dgi_ssm_parts_floats(dk, heads, groups, rows, n_seq, ctypes.byref(chunks))
+
+    for rows, n_seq in ((65, 1), (319, 1), (640, 8), (1030, 12), (530, 24)):
+        assert floats(128, 16, 2, rows, n_seq) == 0 and floats(64, 16, 2, rows, n_seq) == 0
+    for rows, n_seq in ((320, 1), (8192, 2), (2032, 33), (616, 17)):
+        assert floats(128, 16, 2, rows, n_seq) > 0 and floats(64, 16, 2, rows, n_seq) == 0
+    assert floats(128, 6, 2, 8192, 2) == 0 and floats(132, 16, 2, 8192, 2) == 0
+    assert lib.dgi_ssm_whole(8, 8, 64, 64, 1, 520, 9) and not lib.dgi_ssm_whole(8, 8, 64, 64, 1, 2007, 9)
+    assert not lib.dgi_ssm_whole(1, 8, 64, 64, 1, 600, 10) and not lib.dgi_ssm_whole(8, 8, 64, 64, 4, 520, 9)
+    assert lib.dgi_ssm_whole(2, 32, 64, 64, 1, 4000, 3) and not lib.dgi_ssm_whole(2, 24, 64, 64, 1, 4000, 5)
