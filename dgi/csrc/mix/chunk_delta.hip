@@ -127,10 +127,10 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(const ChunkArgs a
   u32x4 kT[NT][PQ];                                    // k, channels by tokens, as the chain's tiles have them
   {
     u32x4 kp[NK][2][PQ];
-    f32x4 kl[3], ql[3];
+    f32x4 kl[3], ql[3], kb[3], qb[3];
     float k2[2] = {0.f, 0.f}, q2[2] = {0.f, 0.f};      // squared norms
 #pragma unroll
-    for (int i = 0; i < 3; ++i) kk[i] = kl[i] = qk[i] = ql[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 3; ++i) kk[i] = kl[i] = qk[i] = ql[i] = kb[i] = qb[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int b = 0; b < NK; ++b) {
       u32x4 kf[3][PQ], kt[3][PQ], qt[3][PQ];           // early, early, late by early, late, late
@@ -160,8 +160,10 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(const ChunkArgs a
       small<PQ, PQ, 3, 3>(kf, qt, ql);
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        (b + 1 < NK ? kk : kl)[i] = mfma(kf[i][0], kt[i][0], (b + 1 < NK ? kk : kl)[i]);
-        (b + 1 < NK ? qk : ql)[i] = mfma(kf[i][0], qt[i][0], (b + 1 < NK ? qk : ql)[i]);
+        const bool second = NK == 4 && b == 2;
+        f32x4 &k = second ? kb[i] : b + 1 < NK ? kk[i] : kl[i], &q = second ? qb[i] : b + 1 < NK ? qk[i] : ql[i];
+        k = mfma(kf[i][0], kt[i][0], k);
+        q = mfma(kf[i][0], qt[i][0], q);
       }
     }
 #pragma unroll
@@ -182,7 +184,7 @@ __global__ __launch_bounds__(256, 3) void delta_prepare_kernel(const ChunkArgs a
       __builtin_amdgcn_wave_barrier();
     }
 #pragma unroll
-    for (int i = 0; i < 3; ++i) { kk[i] += kl[i]; qk[i] += ql[i]; }
+    for (int i = 0; i < 3; ++i) { kk[i] += kb[i] + kl[i]; qk[i] += qb[i] + ql[i]; }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       k2[h] += __shfl_xor(k2[h], 16, 64);
@@ -535,15 +537,15 @@ __global__ __launch_bounds__((64 * Lay<TI, NK>::WAVES), 2) void delta_chain_kern
       cold = __any(none != 0.f);
     };
     auto finish = [&](int c) __attribute__((always_inline)) {
-      f32x4 o[2];
+      f32x4 o[2], oh[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) o[h] = f32x4{0.f, 0.f, 0.f, 0.f};
       small<3, 3, 2, 1>(P, up, o);
 #pragma unroll
-      for (int h = 0; h < 2; ++h) o[h] = mfma(P[h][0], up[0][0], o[h]);
+      for (int h = 0; h < 2; ++h) oh[h] = mfma(P[h][0], up[0][0], f32x4{0.f, 0.f, 0.f, 0.f});
       const Rows p = rows_at(yb + (size_t)c * C * H * dv, cold ? 0 : min(n - c * C, C) * sy);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) row_store(p, fmaf(fo[i >> 2][i & 3], qS[i >> 2][i & 3], o[i >> 2][i & 3]), vy[i], 0);
+      for (int i = 0; i < 8; ++i) row_store(p, oh[i >> 2][i & 3] + fmaf(fo[i >> 2][i & 3], qS[i >> 2][i & 3], o[i >> 2][i & 3]), vy[i], 0);
     };
     __syncthreads();
     for (int c = 0; c < chunks; ++c) {

@@ -56,8 +56,8 @@ struct Lay {
   // bytes
   static constexpr int Q = 0, K = Q + (PRE ? 0 : 2 * ARRB), P = K + (PRE ? 0 : 2 * ARRB);
   static constexpr int ST = P + 2 * PB;                        // [2][NB][NT][64][4] state before the chunk, as the state wave holds it
-  static constexpr int NRM = ST + 2 * NB * SB;                 // mlstm: [4][32] 1 / normaliser
-  static constexpr int NX = NRM + (MODE == MLSTM ? 4 * 32 * 4 : 0);       // mlstm: [GR][4][32] bf16 parts of F (the normaliser's x)
+  static constexpr int NRM = ST + 2 * NB * SB;                 // mlstm: [4][2][32] 1 / normaliser, and what that lacks of it
+  static constexpr int NX = NRM + (MODE == MLSTM ? 4 * 64 * 4 : 0);       // mlstm: [GR][4][32] bf16 parts of F (the normaliser's x)
   static constexpr int GT = NX + (MODE == MLSTM ? GR * 256 : 0);
   static constexpr int FLAG = GT + GR * GN * 4;                // [2][NP] something not finite among q and k
   static constexpr int SBAD = FLAG + 32;                       // [2][NB] something not finite in the state
@@ -193,9 +193,9 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, PRE>::WAVES), (Lay<MODE, TI
     auto products = [&](int c) {
       const char* Q = sm + L::Q + (c & 1) * L::ARRB;
       const char* K = sm + L::K + (c & 1) * L::ARRB;
-      f32x4 hi[3], lo[3];
+      f32x4 hi[3], lo[3], mid[3];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) hi[i] = lo[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < 3; ++i) hi[i] = lo[i] = mid[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int b = 0; b < NK; ++b) {
         u32x4 kf[3][PQ], qf[3][PQ];                  // early, early, late by early, late, late
@@ -209,12 +209,15 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, PRE>::WAVES), (Lay<MODE, TI
           }
 #pragma unroll
         for (int p = 0; p < PQ; ++p) { kf[1][p] = kf[0][p]; qf[1][p] = qf[2][p]; }
-        small<PQ, PQ, 3, 3>(kf, qf, lo);             // as read_out's sums
+        small<PQ, PQ, 3, 3>(kf, qf, lo);             // as read_out's sums; of four blocks a tree
 #pragma unroll
-        for (int i = 0; i < 3; ++i) (b + 1 < NK ? hi : lo)[i] = mfma(kf[i][0], qf[i][0], (b + 1 < NK ? hi : lo)[i]);
+        for (int i = 0; i < 3; ++i) {
+          f32x4& sum = NK == 4 && b == 2 ? mid[i] : b + 1 < NK ? hi[i] : lo[i];
+          sum = mfma(kf[i][0], qf[i][0], sum);
+        }
       }
 #pragma unroll
-      for (int i = 0; i < 3; ++i) qk[i] = hi[i] + lo[i];
+      for (int i = 0; i < 3; ++i) qk[i] = NK == 4 ? hi[i] + (mid[i] + lo[i]) : hi[i] + lo[i];
     };
     float wl[3][4];                                  // light: W is every chunk's
     const float skip = MODE == SSM ? a.par3[head] : 0.f;
@@ -530,6 +533,13 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, PRE>::WAVES), (Lay<MODE, TI
     return __builtin_amdgcn_readfirstlane(f) != 0;
   };
 
+  // 1 / x, and what it lacks (0 of one that is not finite): an output is rounded once by its division
+  auto put_quotient = [&](int c, int t, float x) {
+    float* to = reinterpret_cast<float*>(sm + L::NRM) + (c & 3) * 64 + t;
+    const float f = 1.f / x, rest = f * fmaf(-x, f, 1.f);
+    to[0] = f;
+    to[32] = finite(rest) ? rest : 0.f;
+  };
   // A chunk with something that is not finite goes token by token, as the recurrence is written: parts of an infinity are no numbers, and a matrix
   // product multiplies a token's values by the zeros of those before it.  Each wave decides for itself: the state's for S, the outputs' (on
   // a copy of the state before the chunk) for their rows.
@@ -567,7 +577,7 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, PRE>::WAVES), (Lay<MODE, TI
       o += __shfl_xor(o, 32, 64);
       if constexpr (MODE == SSM) o += a.par3[head] * own;
       if constexpr (MODE == MLSTM) o *= qscale;
-      if (ones) reinterpret_cast<float*>(sm + L::NRM)[(c & 3) * 32 + t] = 1.f / (fmaxf(fabsf(o), G[GX + t]) + 1e-6f);
+      if (ones) put_quotient(c, t, fmaxf(fabsf(o), G[GX + t]) + 1e-6f);
       else if (writes && g == 0 && cok) yb[(size_t)(c * C + t) * H * dv + colc] = o;      // mlstm: still to be divided
     }
   };
@@ -842,8 +852,8 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, PRE>::WAVES), (Lay<MODE, TI
           o = (n16 & 7) == i ? x : o;
         }
         const int t = tok(n16 & 7);
-        o = 1.f / (fmaxf(fabsf(o), gates_of(c)[GX + t]) + 1e-6f);
-        if (n16 < 8 && !was_cold && c >= 0) reinterpret_cast<float*>(sm + L::NRM)[(c & 3) * 32 + t] = o;
+        o = fmaxf(fabsf(o), gates_of(c)[GX + t]) + 1e-6f;
+        if (n16 < 8 && !was_cold && c >= 0) put_quotient(c, t, o);
       };
       read_x(0);
       next_gates(0);
@@ -953,14 +963,15 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, PRE>::WAVES), (Lay<MODE, TI
   };
   auto divide = [&](int c) __attribute__((always_inline)) {    // and divided by the normaliser in step c + 3
     if constexpr (MODE == MLSTM) {
-      float f[8], o[8];
-      from_gates(reinterpret_cast<const float*>(sm + L::NRM) + (c & 3) * 32, f);
+      float f[8], rest[8], o[8];
+      from_gates(reinterpret_cast<const float*>(sm + L::NRM) + (c & 3) * 64, f);
+      from_gates(reinterpret_cast<const float*>(sm + L::NRM) + (c & 3) * 64 + 32, rest);
       if (__builtin_expect(cold_out && c >= 0, 0)) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) out[i] = yb[(size_t)min(c * C + tok(i), n - 1) * H * dv + colc];
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = out[i] * f[i];
+      for (int i = 0; i < 8; ++i) o[i] = fmaf(out[i], f[i], __builtin_amdgcn_fmed3f(out[i], -MOST, MOST) * rest[i]);      // an infinite one stays one
       store(c, o, c >= 0);
     }
   };
@@ -1075,7 +1086,7 @@ __global__ __launch_bounds__(256) void ssm_parts_kernel(const ChunkArgs a) {
   }
   if (wave == 3) return;
   const int s = wave == 2, t = wave > 0;
-  f32x4 h1[1] = {{0.f, 0.f, 0.f, 0.f}}, l1[1] = {{0.f, 0.f, 0.f, 0.f}};
+  f32x4 h1[1] = {{0.f, 0.f, 0.f, 0.f}}, m1 = h1[0], l1[1] = {{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
   for (int b = 0; b < NK; ++b) {
     u32x4 kf[1][3], qf[1][3];
@@ -1084,10 +1095,11 @@ __global__ __launch_bounds__(256) void ssm_parts_kernel(const ChunkArgs a) {
       kf[0][p] = *reinterpret_cast<const u32x4*>(sm + L::ARRB + p * L::PARTB + place(16 * s + n16, 4 * b + g));
       qf[0][p] = *reinterpret_cast<const u32x4*>(sm + p * L::PARTB + place(16 * t + n16, 4 * b + g));
     }
-    small<3, 3, 1, 1>(kf, qf, l1);                     // as read_out's sums: the last block's first parts start from the small ones'
-    (b + 1 < NK ? h1 : l1)[0] = mfma(kf[0][0], qf[0][0], (b + 1 < NK ? h1 : l1)[0]);
+    small<3, 3, 1, 1>(kf, qf, l1);                     // as the scores wave's sums
+    f32x4& sum = b == 2 ? m1 : b + 1 < NK ? h1[0] : l1[0];
+    sum = mfma(kf[0][0], qf[0][0], sum);
   }
-  *reinterpret_cast<f32x4*>(to + 2 * L::ARRB + 1024 * wave + 16 * lane) = h1[0] + l1[0];
+  *reinterpret_cast<f32x4*>(to + 2 * L::ARRB + 1024 * wave + 16 * lane) = h1[0] + (m1 + l1[0]);
 }
 
 }  // namespace

@@ -277,7 +277,7 @@ def test_wkv_scales_beside_strong_decays(q, k):
 
 
 @pytest.mark.parametrize("mode,H,D,line", [("wkv", 52, 16, 136), ("wkv", 310, 16, 224), ("wkv", 11, 68, 104), ("ssm", 2, 20, 48), ("ssm", 14, 20, 112),
-                                           ("ssm", 28, 20, 144)])
+                                           ("ssm", 28, 20, 144), ("ssm", 14, 20, 88)])
 def test_portions_around_the_line_between_the_launches(mode, H, D, line):
     """Among more than eight sequences portions of at most ``line`` rows go in a launch of their own; the line depends on the number of
     workgroups (and, wkv, on the key size).  One row to either side of it, on average near it, and decode rows beside one long portion."""

@@ -5,9 +5,12 @@ are no further off than the loop, in results and in states.
 The measure is the 2-norm of the difference over that of the result, over 2e5 to 5e5 values.  Errors of the two forms are independent
 roundings, so the ratio of two such norms has a spread of under one per cent (a few per cent where a sequence's values share a factor): 1.05.
 The quotient of a matrix memory is dominated by its few smallest denominators and varies by tens of per cent: it is not compared."""
+import ctypes
+
 import pytest
 import torch
 
+import dgi.build
 from dgi.ops import linrec
 from test_chunk_scan import F64, call, make, oracle
 
@@ -100,3 +103,70 @@ def test_delta_chunks_of_128_channels():
     want = oracle(d)
     fast, loop = errors(call(d), want)[0], errors(call(dict(d, pad=1)), want)[0]      # rows off a four-element boundary stay with the loop
     assert fast <= 1.01 * loop, (fast, loop)
+
+
+def taken(d):
+    """Floats of workspace that long portions of delta get: 0, and their chunks would have sixteen tokens."""
+    lib = ctypes.CDLL(dgi.build.build(group="mix"))
+    lib.dgi_linear_scan_parts.restype = ctypes.c_longlong
+    row = 2 * d["G"] * d["D"] + d["H"] * d["V"]
+    at = ctypes.c_void_p(4096)
+    return lib.dgi_linear_scan_parts(1, d["D"], d["V"], d["H"], d["G"], len(d["lens"]), sum(d["lens"]), at, row, at, row, int(d["q"].dtype == torch.float32),
+                                     ctypes.byref(ctypes.c_int()))
+
+
+def of_kind(d, kind, seed):
+    """Rows as a convolution leaves them (SiLU); rows that share a direction twice as large as what they differ in; decays near 1."""
+    g = torch.Generator().manual_seed(seed)
+    for n in "qkv":
+        x = d[n].float()
+        if kind == "silu":
+            x = torch.nn.functional.silu(x)
+        if "share" in kind and n != "v":
+            x = x + 2 * torch.randn(1, x.shape[1], generator=g)
+        d[n] = x.to(d[n].dtype)
+    if "slow" in kind:
+        if d["mode"] == "delta":
+            d["par"] = (d["par"][0] - 5, d["par"][1])
+        elif d["mode"] == "mlstm":
+            d["b"] = d["b"] + 6
+        else:
+            d["par"] = (1 - torch.rand(d["H"], generator=g) * 1e-3,)
+    return d
+
+
+@pytest.mark.parametrize("D,dtype,rows", [(64, torch.float32, 800), (64, torch.bfloat16, 400), (128, torch.bfloat16, 400)])
+@pytest.mark.parametrize("kind", ["plain", "silu", "share", "slow", "share slow"])
+def test_long_portions_of_delta(kind, D, dtype, rows):
+    """Chunks of 32 tokens with a prepared inverse (dgi/csrc/mix/chunk_delta.hip).  Where decays are near 1 the loop is five times further off (it rounds every
+    decay); keys that share a direction make the inverse's terms large beside their sum: there states may be up to a quarter further off than the loop's."""
+    d = of_kind(make("delta", [rows], 16, D, 64, dtype, [7], seed=D), kind, 3)
+    assert taken(d) > 0
+    want = oracle(d)
+    a, b = errors(call(d), want), errors(call(dict(d, pad=1)), want)
+    assert a[0] <= 1.05 * b[0] and a[1] <= (1.25 if kind == "share" else 1.05) * b[1], (a, b)
+    if "slow" in kind:
+        assert a[0] <= 0.4 * b[0] and a[1] <= 0.4 * b[1], (a, b)
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float32), (128, torch.bfloat16), (128, torch.float32)])
+@pytest.mark.parametrize("kind", ["plain", "slow"])
+def test_chunks_of_light(kind, D, dtype):
+    """Light layers in chunks of 32 (dgi/csrc/mix/chunk_parts.hip) against the loop, which takes steps of up to four rows."""
+    d = of_kind(make("light", [300], 16, D, 64, dtype, [7], seed=D), kind, 3)
+    compare("light", call(d), in_short_portions(d, 4), oracle(d))
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float32), (128, torch.bfloat16)])
+@pytest.mark.parametrize("kind", ["plain", "silu", "share", "slow"])
+def test_outputs_of_a_matrix_memory(kind, D, dtype):
+    """Its outputs by the geometric mean of the errors of tokens and heads, which a few small denominators do not decide (8192 of them: a spread of one per
+    cent)."""
+    d = of_kind(make("mlstm", [512], 16, D, 64, dtype, [7], seed=D), kind, 3)
+    want = oracle(d)[0].view(512 * 16, 64)
+
+    def mean(y):
+        return ((y.to(F64).view_as(want) - want).norm(dim=1) / want.norm(dim=1)).clamp_min(1e-12).log().mean().exp().item()
+
+    fast, loop = mean(call(d)[0]), mean(call(dict(d, pad=1))[0])
+    assert fast <= 1.05 * loop, (fast, loop)
