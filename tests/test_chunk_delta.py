@@ -8,6 +8,7 @@ import torch
 
 from test_chunk_parts import where_finite
 from test_chunk_scan import call, check, make, oracle
+from test_scan_precision import taken
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +42,40 @@ def test_not_finite(what):
         else:
             d["v" if what == "large" else what][71, 2] = bad
         where_finite(call(d)[:2], call(dict(d, pad=1))[:2])
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float32), (128, torch.bfloat16)])
+@pytest.mark.parametrize("what", ["value", "state", "nan"])
+def test_too_large_for_parts(what, D, dtype):
+    """Finite values whose first bf16 part is an infinity, as x = beta (v - A k S) or by way of the state; and bf16 rows with a NaN.  What is finite row by row is
+    finite here, and agrees (the products of the row loop overflow earlier in places)."""
+    d = make("delta", [800], 4, D, 32, dtype, [3])
+    big = 3.4e38 if dtype == torch.float32 else torch.finfo(dtype).max
+    if what == "value":
+        d["v"][71, 2] = big
+        d["a"][71, 0] = 40.0
+        x = torch.sigmoid(d["a"][71, 0]) * d["v"][71, 2].float()
+        assert torch.isfinite(x)
+        if dtype == torch.float32:
+            assert not torch.isfinite(x.to(torch.bfloat16))
+    elif what == "state":
+        d["S"][1, 2, 3, 4] = 3.4e38
+    else:
+        for n in "qkv":
+            d[n][71 + 90 * "qkv".index(n), 2] = float("nan")
+    for got, want in zip(call(d), call(dict(d, pad=1))):
+        ok = torch.isfinite(want)
+        assert ok.any() and (got[ok] - want[ok]).abs().max() <= 1e-4 * max(1.0, want[ok].abs().max().item())
+    if what == "nan":
+        where_finite(call(d)[:2], call(dict(d, pad=1))[:2])
+
+
+@pytest.mark.parametrize("H,D,V,dtype,lens", [(4, 64, 32, torch.bfloat16, [1, 16, 17, 0, 700, 801, 650, 700, 640]),
+                                              (3, 128, 20, torch.bfloat16, [1, 16, 17, 0, 600, 801, 650, 700, 640]),
+                                              (3, 64, 16, torch.bfloat16, [505, 1, 16, 17, 0] + [540] * 11 + [577]),
+                                              (2, 36, 16, torch.float32, [1700, 1, 16, 17, 0, 1533, 2000, 1800, 64])], ids=lambda x: str(x)[:14])
+def test_many_sequences(H, D, V, dtype, lens):
+    """More than eight sequences: those of up to 16 rows in a launch of their own; more than sixteen: not ordered by length."""
+    d = make("delta", lens, H, D, V, dtype, [3 * (i % 2) if n else 4 for i, n in enumerate(lens)], seed=D)
+    assert taken(d) > 0
+    check(call(d), oracle(d))

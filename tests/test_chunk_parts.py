@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from test_chunk_scan import F64, call, check, make, oracle
+from test_scan_precision import in_short_portions
 
 pytestmark = pytest.mark.gpu
 
@@ -100,6 +101,22 @@ def test_ssm_pass_not_finite(what):
         else:
             d["S"][1, 2, 3, 4] = bad
         where_finite(run(d)[:2], call(d, chunked=False)[:2])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mode", ["mlstm", "light"])
+@pytest.mark.parametrize("what", ["q", "k", "v", "state", "large"])
+def test_not_finite_bf16(what, mode, D):
+    """bf16 rows, and light layers; beside the loop, which light layers have for steps of up to four rows."""
+    for dtype in (torch.bfloat16, torch.float32) if mode == "light" else (torch.bfloat16,):
+        for bad in (float("inf"), float("nan")) if what != "large" else (3.39e38,):
+            d = make(mode, [130], 8, D, 32, dtype, [3])
+            if what == "state":
+                d["S"][1, 2, 3, 4] = bad
+            else:
+                d["k" if what == "large" else what][71, 5] = bad
+            slow = call(dict(d, pad=1)) if mode == "mlstm" else in_short_portions(d, 4)
+            where_finite(call(d)[:2], slow[:2])
 
 
 def test_light_decays_that_are_none():
