@@ -1,4 +1,4 @@
-// dgi/csrc/mix/chunk_args.h — what the kernels of prompt portions in chunks share (chunk_scan.hip, chunk_parts.hip).
+// dgi/csrc/mix/chunk_args.h — what the kernels of prompt portions in chunks share (chunk_scan.hip, chunk_parts.hip, chunk_delta.hip).
 #pragma once
 #include "../common.h"
 
@@ -26,7 +26,7 @@ struct ChunkArgs {
   float *ws, *wsd;                 // [n_seq, segments, H, dv, dk] states, [n_seq, segments, H] decays
   int skip_rows;                   // sequences of at most this many rows are not this launch's
   float cap;
-  float* parts;                    // ssm: what chunk_parts.hip keeps for the launch's chunks (parts_chunks of them), or null
+  float* parts;                    // what a pass before keeps for the launch's chunks (parts_chunks of them): ssm chunk_parts.hip, delta chunk_delta.hip; or null
   int parts_chunks;
 };
 

@@ -30,7 +30,7 @@
 // by k, substitution, update) or a preparing wave's arithmetic (wkv): a wave issues an instruction every four to five cycles at best, so
 // addresses are lane offsets kept in registers, and rows past the end a branch of their own.  Measured, a step of 2 prompts of 4096 rows in
 // all, 64 heads, states 64 x 64 (ssm 128 x 64), against the same token by token on the vector ALUs (linear_scan.hip, ssm_scan.hip):
-// delta 178 us (726), ssm 199 (637), wkv 232 (some 630).
+// delta 178 us (726), ssm 199 (637; 210 with flat loads), wkv 232 (some 630).
 //
 // Precision: results and states are no further from 64 bits than the token loop's (2-norm over 1300 to 4096 rows: ssm 7.8e-8, the loop 8.0e-8;
 // delta 1.17e-7, 1.18e-7; wkv 9.8e-8, 1.01e-7; but states of wkv on bf16 rows 7.34e-8, 7.28e-8: the loop's products of bf16 keys and values
@@ -133,13 +133,6 @@ struct Lay {
 // an output they lie as those do, token t at place(t), so do the columns of P: register r of lane group g holds token 4 r + g, and a sum
 // over the tokens starts with the oldest, which under a decay are the small ones.
 __device__ __forceinline__ constexpr int place(int t) { return 4 * (t & 3) + (t >> 2); }      // its own inverse
-
-// Whether workgroups of four column blocks are there for a kernel: not where its waves (thirteen, so 128 registers each) would spill (ssm, wkv, mlstm:
-// 1 prompt of 1000 and 5 decode rows, 64 heads, 219 us -> 268), or its LDS would not suffice.
-template <int MODE, int NT>
-constexpr bool has_four() {
-  return NT == 4 && MODE == DELTA;
-}
 
 // Steps whose workgroups of two column blocks do not find a compute unit each: four blocks share what does not depend on the columns
 // (q, k, gates, scores), at SLOW hundredths of two blocks' time per chunk.  Only the lengths say which is the faster (decode rows and short portions
@@ -1077,15 +1070,12 @@ int launch_one(const ChunkArgs& a, dim3 grid, hipStream_t st) {
 template <int MODE, typename TI>
 int launch_dims(const ChunkArgs& a, bool four, dim3 grid, hipStream_t st) {
   if (a.dk <= 64) {
-    if constexpr (has_four<MODE, 4>())
+    // not where its waves (thirteen, so 128 registers each) would spill: ssm, wkv, 1 prompt of 1000 and 5 decode rows, 64 heads, 219 us -> 268
+    if constexpr (MODE == DELTA)
       if (four) return launch_one<MODE, TI, 4, 64>(a, grid, st);
     return launch_one<MODE, TI, 4, 32>(a, grid, st);
   }
-  if (a.dk <= 128) {
-    if constexpr (has_four<MODE, 8>())
-      if (four) return launch_one<MODE, TI, 8, 64>(a, grid, st);
-    return launch_one<MODE, TI, 8, 32>(a, grid, st);
-  }
+  if (a.dk <= 128) return launch_one<MODE, TI, 8, 32>(a, grid, st);
   if constexpr (MODE != SSM) return -3;
   else return launch_one<MODE, TI, 16, 16>(a, grid, st);
 }

@@ -60,7 +60,7 @@ __device__ __forceinline__ void split2_of(const float* x, const float* f, const 
 __device__ __forceinline__ f32x4 mfma(const u32x4& a, const u32x4& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
 }
-// products of N operands' parts by one's (or its own: BN = N), for sums of their own: the first two parts' to hi, the smaller ones, smallest first, to lo.
+// products of N operands' parts by one's (or its own: BN = N), for sums of their own: all but the first two parts', smallest first, to lo; multiply: those to hi, too.
 // Sums take turns, none waits for its own last product.
 template <int PA, int PB, int N, int BN>
 __device__ __forceinline__ void small(const u32x4 (&a)[N][PA], const u32x4 (&b)[BN][PB], f32x4 (&lo)[N]) {
@@ -90,7 +90,7 @@ __device__ __forceinline__ void whole_and_part(double x, float& whole, float& pa
   whole = (float)i;
   part = (float)(x - i);
 }
-// 2^x, rounded about once, and what it lacks: 2^part - 1 by its series, part within [-0.5, 0.5] (the first term left out is 4e-9)
+// 2^x, rounded about once, and what it lacks: 2^part - 1 by its series, part within [-0.5, 0.5] (the first term left out is 5.2e-9)
 __device__ __forceinline__ float power_once(double x, float* rest = nullptr) {
   float i, f;
   whole_and_part(x, i, f);

@@ -274,7 +274,7 @@ bool dgi_chunk_parts_takes(int mode, int dk, int H, int G, int in_f32);
 // compute unit to themselves and a pipeline to fill, so among more than APART_FROM sequences the short ones stay with this file's kernel: those
 // of at most 48 rows while the workgroups find a place each (12 portions of 39 rows, 32 heads: 31 us against 51 there), longer ones when they
 // wait for each other (64 columns, this file's time and that one's: 11 portions of 100 rows, 16 heads 35, 41; 128 rows 42, 41; 16 portions of 128
-// rows, 64 heads 158, 162; 200 rows 242, 222).  recur.scan_chunks decides for whole steps by the same lines: a change of one is a change of both.
+// rows, 64 heads 158, 162; 200 rows 242, 222).  recur.scan_chunks decides for whole steps, by the last two of these lines.
 constexpr int APART_FROM = 8;
 // In chunks of 32: 88 rows there (12 portions of 96 rows of 128 channels, 64 heads 88, 89; 128 rows 114, 104).
 static int apart_rows(int n_seq, int heads, int dv, int N, int G) {

@@ -42,7 +42,7 @@ extern "C" int dgi_paged_prefill(const void* q, int q_stride, const void* k_cach
   while ((1 << bs_log2) < block_size) ++bs_log2;
   if ((1 << bs_log2) != block_size) return -4;
   const float scale_log2 = scale * 1.4426950408889634f;
-  tile_rows &= 0xffff;
+  tile_rows &= 0xffff;      // bit 16 once chose the number of LDS stages: calls that set it stay valid
   if (tile_rows != 128 && tile_rows != 256) return -7;
 #define DGI_PREFILL(HDV, NWV)                                                                          \
   prefill_attn_kernel<HDV, NWV><<<n_tiles * nh, NWV * 64, 0, s>>>(                                \

@@ -74,7 +74,7 @@ __device__ __forceinline__ float inv_scale_cap(float scale_log2) { return 1.4426
 // (same 2 waves per SIMD, half the K/V staging per query row).
 //
 // Two LDS stages: a tile goes from memory to one of them (no registers between) while the tile in the other is multiplied,
-// one barrier per 64 keys.  One prompt of 8192 rows, 32 heads on 8 of 128 dims: 589 us -> 524 (1050 TF/s), 64 dims and 4096
+// one barrier per 64 keys.  One prompt of 8192 rows, 32 heads on 8 of 128 dims: 576 us -> 506 (1086 TF/s), 64 dims and 4096
 // rows 107 -> 90, a tile 3830 cycles a SIMD against 4700, of which its products take 2048.  What the staging registers, the
 // block ids' scalar loads, the addresses of each load and read and the copies around the mask cost went into it: 256
 // registers with every operand waited for as it was read, now 214 with reads a product or more ahead, 185 -> 143 vector and

@@ -358,8 +358,6 @@ def paged_prefill_ref(q, k_cache, v_cache, block_tables, cu_seqlens_q, context_l
 # each staged K/V tile).  Every producer of ``tiles`` (model runner, EAGLE verify /
 # draft metadata, ops.paged_prefill) cuts sequences at this size.
 PREFILL_TILE = int(os.environ.get("DGI_PREFILL_TILE", "128"))
-# bit 16 of the native call's tile size: kept for its callers, the kernel has two LDS stages either way
-PREFILL_DB = int(os.environ.get("DGI_PREFILL_DB", "1"))
 
 
 def order_prefill_tiles(cu_seqlens_q, context_lens=None, tile: int = 0) -> np.ndarray:
@@ -405,8 +403,7 @@ def paged_prefill(q, k_cache, v_cache, block_tables, cu_seqlens_q, context_lens,
             tl = prefill_tiles(cu_seqlens_q.tolist(), context_lens=context_lens.tolist())
             tiles = torch.tensor(tl if tl else [[0, 0]], dtype=torch.int32, device=q.device)[: len(tl)]
         _call("paged_prefill", out, q, k_cache, v_cache, block_tables, cu_seqlens_q, context_lens,
-              tiles, nh, nkv, scale, tree_mask, tree_n,
-              PREFILL_TILE | ((PREFILL_DB & 1) << 16))
+              tiles, nh, nkv, scale, tree_mask, tree_n, PREFILL_TILE)
         return out
     r = paged_prefill_ref(q, k_cache, v_cache, block_tables, cu_seqlens_q, context_lens, nh, nkv, scale,
                           tree_mask, tree_n)

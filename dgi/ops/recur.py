@@ -189,7 +189,7 @@ def scan_chunks(T: int, n_seq: int, heads: int, dv: int, dtype, chunked=None) ->
     place on the chip they wait for each other: 64 columns, row by row against chunks, 4 portions, 16 heads, 72 rows 21, 18 us; 64
     heads, 72 rows 32, 36, 128 rows 50, 43; 11 portions, 64 heads, 128 rows 114, 122, 200 rows 180, 171.  Known here are the
     step's rows and sequences only; among more than eight each sequence is taken by its own length, by the lines of
-    ``apart_rows`` in ssm_scan.hip (112 and 144 there and here lie together), and few rows on average but many rows are decode rows
+    ``apart_rows`` in ssm_scan.hip, and few rows on average but many rows are decode rows
     beside long portions."""
     if SCAN_CHUNK <= 0:
         return False

@@ -302,13 +302,13 @@ def test_ssm_takes_only_position_zero_as_a_start(lens):
 @pytest.mark.parametrize("mode,dtype", [("delta", torch.bfloat16), ("delta", torch.float32), ("mlstm", torch.bfloat16), ("mlstm", torch.float32),
                                         ("light", torch.bfloat16), ("light", torch.float32)])
 @pytest.mark.parametrize("D,V", [(64, 64), (48, 33), (64, 72), (60, 130)])
-@pytest.mark.parametrize("lens", [[70, 71, 96, 65, 80, 64, 81, 66, 79],             # four column blocks a workgroup
+@pytest.mark.parametrize("lens", [[70, 71, 96, 65, 80, 64, 81, 66, 79],             # four column blocks a workgroup (delta of up to 64 channels)
                                   [500] + [17, 20, 18, 33, 19, 17, 21, 18],         # two: one portion is most of the step
                                   [1, 300, 1, 1, 17, 290, 1, 16, 1, 310, 305, 1, 1, 1, 1, 299]])      # decode rows beside portions
 def test_more_workgroups_than_units(mode, dtype, D, V, lens):
-    """Steps of more than 256 workgroups, which take two or four blocks of value columns each, longest sequences first."""
+    """Steps of more than 256 workgroups, which take two blocks of value columns each, or four, longest sequences first."""
     if mode == "light":
-        lens = [n * 5 if n > 16 else n for n in lens]           # its chunks are taken from 320 rows a sequence on
+        lens = [n * 5 if n > 16 else n for n in lens]           # its chunks are taken from up to 112 rows a sequence on
     H = 16 if len(lens) * 16 * -(-V // 32) > 256 else 32
     d = make(mode, lens, H, D, V, dtype, [0 if i % 3 else 40 for i in range(len(lens))], seed=len(lens) + V, pad=8)
     check(call(d), oracle(d))

@@ -137,10 +137,9 @@ def _paged_decode_case(nh, nkv, hd, ctx_lens, bs=16):
                                        (14, 2, 64)])
 @pytest.mark.parametrize("qlens,ctxs", [([5], [5]), ([130, 1, 64], [130, 40, 600]), ([512], [512]),
                                         ([300, 77], [1000, 77])])
-@pytest.mark.parametrize("tile,db", [(128, 1), (128, 0), (256, 1)])
-def test_paged_prefill(nh, nkv, hd, qlens, ctxs, tile, db, monkeypatch):
+@pytest.mark.parametrize("tile", [128, 256])
+def test_paged_prefill(nh, nkv, hd, qlens, ctxs, tile, monkeypatch):
     monkeypatch.setattr(ops, "PREFILL_TILE", tile)
-    monkeypatch.setattr(ops, "PREFILL_DB", db)
     bs = 16
     maxw = 80
     nblocks = sum((c + bs - 1) // bs for c in ctxs) + 4
