@@ -8,10 +8,10 @@
 //
 // light: u = v;  ssm: q = C, k = B, u = x, the skip factor on P's diagonal;  mlstm: o divided by the normaliser, itself such a recurrence with u = 1.
 //
-// fp32 operands of a product are three bf16 parts each, x = x0 + x1 + x2 (each rounded to nearest, so together all 24 bits, of values from 2^-110 on; below, what the third lacks of the
-// smallest bf16 number is lost, 2^-134 at most): the six products of
-// parts that reach into 24 bits (three where the other operand is bf16 as it is) run at sixteen times the rate of an fp32 product.  The five
-// small ones are summed by themselves, so that a sum over channels or tokens is rounded at its own size once per 32 of them.
+// fp32 operands of a product are three bf16 parts each, x = x0 + x1 + x2 (each rounded to nearest, so together all 24 bits of values from 2^-110 on;
+// below, what is smaller than the smallest bf16 number is lost): the six products of parts that reach into 24 bits (three where the other
+// operand is bf16 as it is) run at sixteen times the rate of an fp32 product.  The five small ones are summed by themselves, so that a sum over
+// channels or tokens is rounded at its own size once per 32 of them; scores of 128 channels are summed as a tree.
 //
 // A workgroup owns (sequence, head, two blocks of 16 value columns) and is a pipeline of waves that hand chunks on through LDS, one barrier
 // per chunk:
@@ -34,7 +34,8 @@
 //
 // Precision: results and states are no further from 64 bits than the token loop's, nor (2-norm) by more than a hundredth than in chunk_scan.hip, whose P u is in
 // 64 bits.  512 rows, 16 heads, errors over that kernel's of outputs and states: ssm 0.78, 0.92 (7.0e-8; the loop 1.03e-7); light 0.46, 0.31; mlstm 0.94, 0.76 (64
-// channels), 0.95, 0.84 (128); with decays near 1 at most 0.4.  mlstm's outputs by the geometric mean of tokens: bf16 rows 1.03, fp32 0.92.  What gives that: decays are summed as logarithms in 64 bits and a running maximum is kept in 64 bits, since its rounding would be the state's.
+// channels), 0.95, 0.84 (128); with decays near 1 at most 0.4.  mlstm's outputs by the geometric mean of tokens: bf16 rows 1.03, fp32 0.92.  What gives that:
+// decays are summed as logarithms in 64 bits and a running maximum is kept in 64 bits, since its rounding would be the state's.
 #include <type_traits>
 #include "chunk_split.h"
 
