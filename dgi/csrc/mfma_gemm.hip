@@ -115,19 +115,19 @@ __device__ __forceinline__ void swap_pair(const float (&a)[4], const float (&b)[
 }
 
 // rs: the tile's 256 per-row rstd values (LDS) for EPI 3 / 4
-template <int EPI>
-__device__ __forceinline__ void epilogue(const f32x4 (&acc)[8][4], uint16_t* __restrict__ Y, int ldy, int M, int m0,
+template <int EPI, int IT>
+__device__ __forceinline__ void epilogue(const f32x4 (&acc)[IT][4], uint16_t* __restrict__ Y, int ldy, int M, int m0,
                                          int tn, int wm, int wn, int lane, const float* rs = nullptr) {
   const int r16 = lane & 15;
   const int g = lane >> 4;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + wm * 128 + i * 16 + r16;
+  for (int i = 0; i < IT; ++i) {
+    const int m = m0 + wm * (16 * IT) + i * 16 + r16;
     // the swap partners (lanes l, l ^ 16) hold the same row, so a row past M drops both together
     if (m >= M) continue;
     uint16_t* yrow = Y + (size_t)m * ldy;
     float sc = 1.f;
-    if constexpr (EpiKind<EPI>::norm) sc = rs[wm * 128 + i * 16 + r16];
+    if constexpr (EpiKind<EPI>::norm) sc = rs[wm * (16 * IT) + i * 16 + r16];
     if constexpr (EpiKind<EPI>::swiglu) {
       float o[2][4];
 #pragma unroll
@@ -161,7 +161,8 @@ __device__ __forceinline__ void epilogue(const f32x4 (&acc)[8][4], uint16_t* __r
 // values squared.  Per row: each lane sums its 16 columns, the 4 lane groups of a wave combine by
 // shuffles, the 4 waves of a row band through LDS (ssl: 4 x 256 floats), in a fixed order.
 // Every wave of the block must call it (one barrier).
-__device__ __forceinline__ void epilogue_res(const f32x4 (&acc)[8][4], uint16_t* __restrict__ Y, int ldy, int M,
+template <int IT>
+__device__ __forceinline__ void epilogue_res(const f32x4 (&acc)[IT][4], uint16_t* __restrict__ Y, int ldy, int M,
                                              int m0, int tn, int wm, int wn, int lane, float* ssl,
                                              float* __restrict__ ss, int ss_ld) {
   const int r16 = lane & 15;
@@ -170,19 +171,19 @@ __device__ __forceinline__ void epilogue_res(const f32x4 (&acc)[8][4], uint16_t*
   // rows in batches of 4: the batch's 8 residual loads are all issued before the first is used
   // (a load-use per 16-byte chunk would serialise 16 memory round trips per lane)
 #pragma unroll
-  for (int i0 = 0; i0 < 8; i0 += 4) {
+  for (int i0 = 0; i0 < IT; i0 += 4) {
     uint4 old[4][2];
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-      const int m = m0 + wm * 128 + (i0 + ii) * 16 + r16;
+    for (int ii = 0; ii < 4 && i0 + ii < IT; ++ii) {
+      const int m = m0 + wm * (16 * IT) + (i0 + ii) * 16 + r16;
       const uint16_t* yrow = Y + (size_t)min(m, M - 1) * ldy + cbase;
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) old[ii][jj] = *(const uint4*)(yrow + jj * 32);
     }
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
+    for (int ii = 0; ii < 4 && i0 + ii < IT; ++ii) {
       const int i = i0 + ii;
-      const int m = m0 + wm * 128 + i * 16 + r16;
+      const int m = m0 + wm * (16 * IT) + i * 16 + r16;
       float part = 0.f;
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
@@ -207,12 +208,12 @@ __device__ __forceinline__ void epilogue_res(const f32x4 (&acc)[8][4], uint16_t*
       }
       part += __shfl_xor(part, 16, 64);
       part += __shfl_xor(part, 32, 64);
-      if (g == 0) ssl[wn * 256 + wm * 128 + i * 16 + r16] = part;
+      if (g == 0) ssl[wn * 256 + wm * (16 * IT) + i * 16 + r16] = part;
     }
   }
   __syncthreads();
   const int t = threadIdx.x;
-  if (t < 256 && m0 + t < M)
+  if (t < 32 * IT && m0 + t < M)
     ss[(size_t)(m0 + t) * ss_ld + tn] = ((ssl[t] + ssl[256 + t]) + ssl[512 + t]) + ssl[768 + t];
 }
 
@@ -705,13 +706,14 @@ struct PPArgs {
 
 // EPI 5 (see EpiKind): T is the LDS tile image (256 rows x kRopeLd), rs the tile's rstd.  Every wave
 // of the block calls it (two barriers).
-__device__ __forceinline__ void epilogue_rope(const f32x4 (&acc)[8][4], const PPArgs& a, int m0, int tn, int wm,
+template <int IT>
+__device__ __forceinline__ void epilogue_rope(const f32x4 (&acc)[IT][4], const PPArgs& a, int m0, int tn, int wm,
                                               int wn, int lane, const float* rs, uint16_t* T) {
   const int r16 = lane & 15;
   const int g = lane >> 4;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int rl = wm * 128 + i * 16 + r16;
+  for (int i = 0; i < IT; ++i) {
+    const int rl = wm * (16 * IT) + i * 16 + r16;
     const float sc = rs[rl];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -727,8 +729,9 @@ __device__ __forceinline__ void epilogue_rope(const f32x4 (&acc)[8][4], const PP
   const int m = m0 + rl;
   const int col0 = tn * 256;
   const int kind = col0 < a.qcols ? 0 : col0 < a.qcols + a.kvcols ? 1 : 2;    // q, k or v heads
-  const int slot = (m < a.M && kind) ? a.slots[m] : 0;
-  if (m < a.M && slot >= 0) {
+  const bool in = rl < 32 * IT && m < a.M;
+  const int slot = (in && kind) ? a.slots[m] : 0;
+  if (in && slot >= 0) {
     const int blk = kind ? slot / a.bs : 0;
     const int off = kind ? slot - blk * a.bs : 0;
     const float* cs = a.cs + (size_t)a.pos[m] * 128;
@@ -788,7 +791,7 @@ constexpr int kSc1 = 16;
 // the next whole tile's prologue is issued before the current whole tile's epilogue
 // (which does not touch LDS: the body ends with every LDS read retired), so its first
 // K tiles load while the stores drain.
-template <int NT, class Pro, class Body, class Store, class Sum, class Epi>
+template <int NT, int TM, class Pro, class Body, class Store, class Sum, class Epi>
 __device__ __forceinline__ void drive(const PPArgs& a, char* smem, Pro&& prologue, Body&& body, Store&& slab_store,
                                       Sum&& slab_sum, Epi&& epi) {
   const int tid = threadIdx.x;
@@ -829,7 +832,7 @@ __device__ __forceinline__ void drive(const PPArgs& a, char* smem, Pro&& prologu
     body(tm, tn, cur.kb, cur.L, ov);
     const Item nx = next();
     // overlap only between whole tiles whose epilogue stores every row (fixed store count)
-    ov = a.ovl && nx.t >= 0 && !cur.piece && !nx.piece && (tm + 1) * kBM <= a.M;
+    ov = a.ovl && nx.t >= 0 && !cur.piece && !nx.piece && (tm + 1) * TM <= a.M;
     if (ov) prologue(nx.t % a.tiles_m, nx.t / a.tiles_m, nx.kb);
     bool store = true;
     if (cur.piece) {
@@ -904,8 +907,12 @@ __device__ __forceinline__ void drive(const PPArgs& a, char* smem, Pro&& prologu
 //   phase  reads             MFMAs          staging                       wait before the barrier
 //   0      Xa, Wa, Wb (16)   Xa x (Wa, Wb)  W0-3, X2 of t+1               vmcnt(6): X1, X3 of t landed
 //   1      Xb (8)            Xb x (Wa, Wb)  X3, X1 of t+1, X0 of t+2      vmcnt(3): all but X3, X1 of t+1
-template <int EPI, int PRIO, int PH>
+// IT: row tiles of 16 of a wave group, a work item is 32 IT rows (see row_tiles).  The first H0 of them lie in the first slab of the
+// group's 128 LDS rows, the others in the second, so that a slab is one phase's whatever IT; its other rows repeat the tile's first.
+template <int EPI, int PRIO, int PH, int IT = 8>
 __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
+  static_assert(IT == 8 || PH == 2, "phases");
+  constexpr int TM = 32 * IT, H0 = (IT + 1) / 2, H1 = IT - H0;
   // EPI 2: per-wave row partials of the sum of squares; EPI 3 / 4: two slots of the tile's rstd
   // (slot per work item: a fast wave may start the next item while others still store this one).
   // Carved from the one LDS array: with a second __shared__ object hipcc's waitcnt pass can no
@@ -931,13 +938,13 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
   const int xbase = (wm * 128 + r16) * 128;
   const int wbase = kTileBytes + (wn * 64 + r16) * 128;
 
-  f32x4 acc[8][4];
-  bf16x8 xa[4][2], xb[4][2], wa[2][2], wb[2][2];
-  // x fragments of row tiles i0 .. i0 + 3, w fragments of row tiles j0, j0 + 1; both k halves
-  auto rx = [&](int st, int i0, bf16x8 (&f)[4][2]) {
-    const char* s = smem + st * kStageBytes + xbase + i0 * 2048;
+  f32x4 acc[IT][4];
+  bf16x8 xa[H0][2], xb[H1][2], wa[2][2], wb[2][2];
+  // x fragments of the row tiles of slab `half`, w fragments of row tiles j0, j0 + 1; both k halves
+  auto rx = [&](int st, int half, auto& f) {
+    const char* s = smem + st * kStageBytes + xbase + half * 8192;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < (int)(sizeof(f) / sizeof(f[0])); ++i) {
       f[i][0] = *(const bf16x8*)(s + i * 2048 + ph0);
       f[i][1] = *(const bf16x8*)(s + i * 2048 + ph1);
     }
@@ -950,12 +957,12 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
       f[j][1] = *(const bf16x8*)(s + j * 2048 + ph1);
     }
   };
-  auto mma = [&](int i0, int j0, const bf16x8 (&xf)[4][2], const bf16x8 (&wf)[2][2]) {
+  auto mma = [&](int i0, int j0, const auto& xf, const bf16x8 (&wf)[2][2]) {
     if constexpr (PRIO == 0) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < (int)(sizeof(xf) / sizeof(xf[0])); ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
           acc[i0 + i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][h], xf[i][h], acc[i0 + i][j0 + j], 0, 0, 0);
@@ -991,11 +998,14 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
     return t;
   };
   auto set_src = [&](int tm, int tn, int kb) {
-    const int m0 = tm * kBM;
+    const int m0 = tm * TM;
     const int tq = fresh_tid();
     const int q = tq >> 3, lc = (tq & 7) ^ ((tq >> 4) & 7);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) xs[i] = a.X + (size_t)min(m0 + q + i * 64, M - 1) * ldx + lc * 8 + kb * kBK;
+    for (int i = 0; i < 4; ++i) {
+      const int row = q < 16 * (i & 1 ? H1 : H0) ? (i >> 1) * (16 * IT) + (i & 1) * (16 * H0) + q : 0;
+      xs[i] = a.X + (size_t)min(m0 + row, M - 1) * ldx + lc * 8 + kb * kBK;
+    }
     int wrow0, wstep;
     if (EpiKind<EPI>::swiglu) {
       wrow0 = tn * 128 + (q < 32 ? q : a.I + q - 32);
@@ -1022,13 +1032,13 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
   // prologue(tm, tn, kb); the sources are recomputed here so that they are not live across an
   // overlapped epilogue (whose register pressure otherwise makes hipcc reuse store-data
   // registers, each reuse a vmcnt(0)).
-  // ov: the previous tile's epilogue (8 16-byte stores per thread for EPI 1, 16 for EPI 0; all its rows inside M) was
+  // ov: the previous tile's epilogue (IT 16-byte stores per thread for SwiGLU, 2 IT for plain ones; all its rows inside M) was
   // issued between the prologue and this call, so the first wait counts those stores too
   // (vector memory operations retire in issue order)
   auto body = [&](int tm, int tn, int kb, int L, bool ov) {
     set_src(tm, tn, kb);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < IT; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     if constexpr (EpiKind<EPI>::norm) {
@@ -1038,7 +1048,7 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
       const int t = fresh_tid();
       // two lanes per row, each summing half of its partials (float4 loads, all in flight
       // together: ss_ld % 8 == 0, <= 32), then one exchange — a fixed order on every run
-      const int m = min(tm * kBM + (t >> 1), M - 1);
+      const int m = min(tm * TM + (t >> 1), M - 1);
       const int per = a.ss_ld >> 3;
       const f32x4* sp = (const f32x4*)(a.ss + (size_t)m * a.ss_ld) + (t & 1) * per;
       f32x4 v[4];
@@ -1075,16 +1085,16 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
       // phase 2
       if constexpr (MODE < 2) gx(t + 1, 1, ST ^ 1);
       if constexpr (MODE == 0) gx(t + 2, 2, ST);
-      rx(ST, 4, xb);
+      rx(ST, 1, xb);
       barrier();
-      mma(4, 2, xb, wb);
+      mma(H0, 2, xb, wb);
       barrier();
       // phase 3
       if constexpr (MODE == 0) { gw(t + 2, 0, ST); gw(t + 2, 1, ST); }
       if constexpr (MODE == 0) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
       else if constexpr (MODE == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
       barrier();
-      mma(4, 0, xb, wa);
+      mma(H0, 0, xb, wa);
       barrier();
     };
 
@@ -1108,12 +1118,12 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
       // phase 1
       if constexpr (MODE < 2) { gx(t + 1, 3, ST ^ 1); gx(t + 1, 1, ST ^ 1); }
       if constexpr (MODE == 0) gx(t + 2, 0, ST);
-      rx(ST, 4, xb);
+      rx(ST, 1, xb);
       if constexpr (MODE == 0) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
       else if constexpr (MODE == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
       barrier();
-      mma(4, 0, xb, wa);
-      mma(4, 2, xb, wb);
+      mma(H0, 0, xb, wa);
+      mma(H0, 2, xb, wb);
       barrier();
     };
 
@@ -1122,8 +1132,8 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
     using T2 = std::integral_constant<int, 2>;
     if constexpr (PH == 2) {
       if (!ov) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-      else if constexpr (EpiKind<EPI>::swiglu) asm volatile("s_waitcnt vmcnt(11)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(19)" ::: "memory");
+      else if constexpr (EpiKind<EPI>::swiglu) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 + IT) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 + 2 * IT) : "memory");
       barrier();
       if (wm == 1) barrier();     // stagger: waves 4-7 run one section behind
       int t = 0;
@@ -1150,10 +1160,10 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
     if (wm == 0) barrier();     // pairs with the last barrier of waves 4-7: every LDS read retired
   };
 
-  drive<512>(a, smem, prologue, body,
+  drive<512, TM>(a, smem, prologue, body,
              [&](auto&& store16) {
 #pragma unroll
-               for (int i = 0; i < 8; ++i)
+               for (int i = 0; i < IT; ++i)
 #pragma unroll
                  for (int j = 0; j < 4; ++j) store16(i * 4 + j, acc[i][j]);
              },
@@ -1164,21 +1174,21 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
                // fragment registers are free here).  A prefix register set for own >= 2 spills (hipcc).
                if (own < 0) {
 #pragma unroll
-                 for (int i = 0; i < 8; ++i)
+                 for (int i = 0; i < IT; ++i)
 #pragma unroll
                    for (int j = 0; j < 4; ++j) acc[i][j] = load16(0, i * 4 + j);
                }
                for (int jj = own == 1 ? 0 : 1; jj < n; ++jj) {
                  if (jj == own) continue;
 #pragma unroll
-                 for (int i0 = 0; i0 < 8; i0 += 4) {
+                 for (int i0 = 0; i0 < IT; i0 += 4) {
                    f32x4 v[4][4];
 #pragma unroll
-                   for (int i = 0; i < 4; ++i)
+                   for (int i = 0; i < 4 && i0 + i < IT; ++i)
 #pragma unroll
                      for (int j = 0; j < 4; ++j) v[i][j] = load16(jj, (i0 + i) * 4 + j);
 #pragma unroll
-                   for (int i = 0; i < 4; ++i)
+                   for (int i = 0; i < 4 && i0 + i < IT; ++i)
 #pragma unroll
                      for (int j = 0; j < 4; ++j) acc[i0 + i][j] += v[i][j];
                  }
@@ -1187,13 +1197,13 @@ __global__ __launch_bounds__(512) void mfma_gemm_pp_kernel(PPArgs a) {
              [&](int tm, int tn) {
                const int te = fresh_tid();
                if constexpr (EpiKind<EPI>::res)
-                 epilogue_res(acc, a.Y, a.ldy, M, tm * kBM, tn, (te >> 8) & 1, (te >> 6) & 3, te & 63, ep_lds, a.ss,
+                 epilogue_res(acc, a.Y, a.ldy, M, tm * TM, tn, (te >> 8) & 1, (te >> 6) & 3, te & 63, ep_lds, a.ss,
                               a.ss_ld);
                else if constexpr (EpiKind<EPI>::rope)
-                 epilogue_rope(acc, a, tm * kBM, tn, (te >> 8) & 1, (te >> 6) & 3, te & 63, ep_lds + rs_slot * 256,
+                 epilogue_rope(acc, a, tm * TM, tn, (te >> 8) & 1, (te >> 6) & 3, te & 63, ep_lds + rs_slot * 256,
                                (uint16_t*)smem);
                else
-                 epilogue<EPI>(acc, a.Y, a.ldy, M, tm * kBM, tn, (te >> 8) & 1, (te >> 6) & 3, te & 63,
+                 epilogue<EPI>(acc, a.Y, a.ldy, M, tm * TM, tn, (te >> 8) & 1, (te >> 6) & 3, te & 63,
                                ep_lds + rs_slot * 256);
              });
 }
@@ -1281,11 +1291,50 @@ struct NormArgs {
   int qcols = 0, kvcols = 0, nkv = 0, bs = 0;
 };
 
+// How a launch shares out its tiles: hybrid split-K (rem tiles in `splits` pieces, then `full` whole ones for each of the P blocks), or whole tiles.
+struct Shares {
+  int full, rem, splits;
+  bool hybrid;
+};
+Shares shares(int total, int P, int skmode) {
+  Shares r{total / P, total % P, 0, false};
+  r.splits = r.rem ? min(4, P / r.rem) : 0;
+  r.hybrid = skmode && r.splits >= 2 && (r.full < 8 || skmode == 2);
+  return r;
+}
+
+// Row tiles of 16 per wave group (IT, tiles of 32 IT rows) of M rows: the fewest rows of padding are not the least time, since a round of the chip
+// takes (5.4 + IT) / 13.4 of one of 256 rows (its weights come through at 3 TB/s whatever the rows: 57344 x 8192, 896 tiles in 3.5 rounds, 677 us of
+// 256 rows, 614 of 224, 571 of 192, 524 of 160), lower tiles are more of them, and pieces along K take some 25 us to add up (28672 x 4096, 900 rows: 448 tiles of
+// 256 180 us, 560 of 192, the last 48 in pieces, 199).  So the least of rounds times that, 256 rows unless others gain 2 %.  us of 256 rows and of the rule's: 57344 x 8192, 319 rows 362, 321 (160), 435 375, 347 (224), 576 528, 473 (192), 802 670, 617 (224), 512 372 (224: 494); 8192 x 28672
+// in pieces, 319 196, 172; 435 200, 191; 659 312, 293; 8192 x 8192, 319 79, 65; 435 86, 77; 10240 x 8192, 435 92, 88.
+int row_tiles(int M, int tiles_n, int K, int P, int skmode) {
+  int best = 8;
+  double least = 0.;
+  for (int it = 8; it >= 5; --it) {
+    const Shares sh = shares((M + 32 * it - 1) / (32 * it) * tiles_n, P, skmode);
+    const double rounds = sh.full + (sh.hybrid ? 1. / sh.splits + 20. * kBK / K : sh.rem ? 1. : 0.), cost = rounds * (5.4 + it) * (it == 8 ? 0.98 : 1.);
+    if (it == 8 || cost < least) {
+      best = it;
+      least = cost;
+    }
+  }
+  return best;
+}
+
 template <int EPI>
-void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, int I, int K, int tiles_m, int total,
+void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, int I, int K, int tiles_n,
                int skmode, int prio, hipStream_t s, const NormArgs& na = NormArgs{}, const SkWorkspace& own = SkWorkspace{}) {
+  const int nt = K / kBK;
+  const int units = gemm_units();
+  const int P = (g_cu_limit >= 8 && g_cu_limit < units) ? (g_cu_limit & ~7) : units;
+  if (nt < 8) skmode = 0;
   decltype(&mfma_gemm_pp_kernel<EPI, 0, 2>) kern;
-  if constexpr (EPI >= 2)       // the fused-norm epilogues: default priority scheme only
+  int it = 8;
+  if ((prio & 7) == 4 && P) it = row_tiles(M, tiles_n, K, P, skmode);
+  if (it < 8)
+    kern = it == 5 ? mfma_gemm_pp_kernel<EPI, 0, 2, 5> : it == 6 ? mfma_gemm_pp_kernel<EPI, 0, 2, 6> : mfma_gemm_pp_kernel<EPI, 0, 2, 7>;
+  else if constexpr (EPI >= 2)       // the fused-norm epilogues: default priority scheme only
     kern = (prio & 4) ? mfma_gemm_pp_kernel<EPI, 0, 2> : mfma_gemm_pp_kernel<EPI, 0, 4>;
   else
     kern = (prio & 4) ? (prio & 3) == 1   ? mfma_gemm_pp_kernel<EPI, 1, 2>
@@ -1294,33 +1343,30 @@ void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, i
                       : (prio & 3) == 1   ? mfma_gemm_pp_kernel<EPI, 1, 4>
                       : (prio & 3) == 2   ? mfma_gemm_pp_kernel<EPI, 2, 4>
                                           : mfma_gemm_pp_kernel<EPI, 0, 4>;
+  const int tiles_m = (M + 32 * it - 1) / (32 * it), total = tiles_m * tiles_n;
   // EPI 2 reads the tile it stores (in place) and EPI 5 stages its tile through the staging LDS: no
   // overlap of the next tile's loads with their epilogues
   PPArgs a{(const uint16_t*)x, (const uint16_t*)w, (uint16_t*)y, nullptr, nullptr, ldx, ldy, M, I, K, tiles_m, total,
            0, 0, 0, 0, !(prio & 8) && EPI != 2 && EPI != 5, na.ss, na.ss_ld, na.inv_k, na.eps,
            na.pos, na.cs, na.slots, na.kc, na.vc, na.qcols, na.kvcols, na.nkv, na.bs};
-  const int nt = K / kBK;
-  const int units = (skmode || a.ovl) && nt >= 8 ? gemm_units() : 0;
-  if (units) {
-    const int P = (g_cu_limit >= 8 && g_cu_limit < units) ? (g_cu_limit & ~7) : units;
-    const int full = total / P, rem = total % P;
-    const int splits = rem ? min(4, P / rem) : 0;
-    if (skmode && splits >= 2 && (full < 8 || skmode == 2)) {
+  if (P && nt >= 8) {
+    const Shares sh = shares(total, P, skmode);
+    if (sh.hybrid) {
       const SkWorkspace sk = own.ws ? own : sk_workspace(units, s);
       if (sk.ws) {
         a.ws = sk.ws;
         a.cnt = sk.cnt;
-        a.rem = rem;
-        a.splits = splits;
-        a.full = full;
+        a.rem = sh.rem;
+        a.splits = sh.splits;
+        a.full = sh.full;
         a.P = P;
         kern<<<dim3(P), 512, 0, s>>>(a);
         return;
       }
     }
-    if (a.ovl && rem == 0 && full >= 2) {
+    if (a.ovl && sh.rem == 0 && sh.full >= 2) {
       // whole waves of tiles: persistent, so each block's next tile loads under this one's epilogue
-      a.full = full;
+      a.full = sh.full;
       a.P = P;
       kern<<<dim3(P), 512, 0, s>>>(a);
       return;
@@ -1330,10 +1376,11 @@ void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, i
 }
 
 template <int EPI, int SCHED>
-void launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int I, int K, int tiles_m, int total,
+void launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int I, int K, int tiles_n,
             int skmode, int prio, hipStream_t s, const SkWorkspace& own) {
+  const int tiles_m = (M + kBM - 1) / kBM, total = tiles_m * tiles_n;
   if (SCHED == 3)
-    launch_pp<EPI>(x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s, NormArgs{}, own);
+    launch_pp<EPI>(x, ldx, w, y, ldy, M, I, K, tiles_n, skmode, prio, s, NormArgs{}, own);
   else if (SCHED == 2)
     mfma_gemm_ring_kernel<EPI><<<dim3(total), 512, 0, s>>>((const uint16_t*)x, ldx, (const uint16_t*)w,
                                                           (uint16_t*)y, ldy, M, I, K, tiles_m, total);
@@ -1372,19 +1419,17 @@ extern "C" int dgi_mfma_gemm_norm(const void* x, int ldx, const void* w, void* y
   int prio = (phases == 2 || (phases == 0 && M <= 2560)) ? 4 : 0;
   const int I = kind == 4 ? N / 2 : 0;
   const int tiles_n = kind == 4 ? I / 128 : N / 256;
-  const int tiles_m = (M + kBM - 1) / kBM;
-  const int total = tiles_m * tiles_n;
   NormArgs na;
   na.ss = ss;
   na.ss_ld = ss_ld;
   na.inv_k = inv_k;
   na.eps = eps;
   if (kind == 2)
-    launch_pp<2>(x, ldx, w, y, ldy, M, I, K, tiles_m, total, 1, prio, s, na);
+    launch_pp<2>(x, ldx, w, y, ldy, M, I, K, tiles_n, 1, prio, s, na);
   else if (kind == 3)
-    launch_pp<3>(x, ldx, w, y, ldy, M, I, K, tiles_m, total, 1, prio, s, na);
+    launch_pp<3>(x, ldx, w, y, ldy, M, I, K, tiles_n, 1, prio, s, na);
   else
-    launch_pp<4>(x, ldx, w, y, ldy, M, I, K, tiles_m, total, 1, prio, s, na);
+    launch_pp<4>(x, ldx, w, y, ldy, M, I, K, tiles_n, 1, prio, s, na);
   DGI_CHECK_LAUNCH();
   return 0;
 }
@@ -1402,8 +1447,6 @@ extern "C" int dgi_mfma_gemm_norm_rope(const void* x, int ldx, const void* w, vo
     return -3;
   if ((nh * 128) % 256 || (nkv * 128) % 256 || N != (nh + 2 * nkv) * 128 || block_size <= 0) return -3;
   int prio = (phases == 2 || (phases == 0 && M <= 2560)) ? 4 : 0;
-  const int tiles_m = (M + kBM - 1) / kBM;
-  const int total = tiles_m * (N / 256);
   NormArgs na;
   na.ss = ss;
   na.ss_ld = ss_ld;
@@ -1418,7 +1461,7 @@ extern "C" int dgi_mfma_gemm_norm_rope(const void* x, int ldx, const void* w, vo
   na.kvcols = nkv * 128;
   na.nkv = nkv;
   na.bs = block_size;
-  launch_pp<5>(x, ldx, w, y, ldy, M, 0, K, tiles_m, total, 1, prio, s, na);
+  launch_pp<5>(x, ldx, w, y, ldy, M, 0, K, N / 256, 1, prio, s, na);
   DGI_CHECK_LAUNCH();
   return 0;
 }
@@ -1447,17 +1490,15 @@ extern "C" int dgi_mfma_gemm(const void* x, int ldx, const void* w, void* y, int
   if (sched == 3 && (K % (2 * kBK) || K < 4 * kBK)) sched = 1;   // ping-pong needs an even count of >= 4 K tiles
   const int I = swiglu ? N / 2 : 0;
   const int tiles_n = swiglu ? I / 128 : N / 256;
-  const int tiles_m = (M + kBM - 1) / kBM;
-  const int total = tiles_m * tiles_n;
   SkWorkspace own;
   own.ws = slabs;
   own.cnt = slabs ? counters + 1 : nullptr;
   if (swiglu)
     (sched == 3 ? launch<1, 3> : sched == 2 ? launch<1, 2> : sched ? launch<1, 1> : launch<1, 0>)(
-        x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s, own);
+        x, ldx, w, y, ldy, M, I, K, tiles_n, skmode, prio, s, own);
   else
     (sched == 3 ? launch<0, 3> : sched == 2 ? launch<0, 2> : sched ? launch<0, 1> : launch<0, 0>)(
-        x, ldx, w, y, ldy, M, I, K, tiles_m, total, skmode, prio, s, own);
+        x, ldx, w, y, ldy, M, I, K, tiles_n, skmode, prio, s, own);
   DGI_CHECK_LAUNCH();
   return 0;
 }

@@ -290,3 +290,25 @@ def test_mfma_gemm_first_used_by_several_threads():
     ref = ops.mfma_gemm_ref(x, w).float()
     assert all(torch.equal(a, got[0]) for a in got[1:])
     assert (got[0].float() - ref).abs().max().item() <= 2e-2 * ref.abs().max().item() + 1e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [129, 320, 321, 384, 385, 448, 449])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3, 4, 5])
+def test_mfma_gemm_tiles_of_fewer_rows(M, kind):
+    """Two phases a K tile take tiles of 160, 192 or 224 rows where that saves time (here: 128 column tiles, 160 up to 320 rows, then 192
+    up to 384, 224 up to 448), four phases always 256: whole tiles sum in the same order, so every bit is the same."""
+    ops.load_native(required=True)
+    K = 384
+    if kind == 5:
+        two, four = (_rope_case(M, 224, 16, K, "cuda", phases)[0] for phases in (2, 4))
+    elif kind >= 2:
+        N = 128 * 256 if kind != 4 else 256 * 128
+        two, four = (_norm_case(M, N, K, kind, "cuda", phases)[0] for phases in (2, 4))
+    else:
+        x, w = _rand(M, K, device="cuda", seed=M), _rand(128 * 256, K, device="cuda", scale=0.05, seed=1)
+        two, four = ((ops.mfma_gemm(x, w, kind, sched=3, phases=phases),) for phases in (2, 4))
+        ref = ops.mfma_gemm_ref(x, w, kind).float()
+        assert (two[0].float() - ref).abs().max().item() <= 2e-2 * ref.abs().max().item() + 1e-3
+    for a, b in zip(two, four):
+        assert torch.equal(a, b)
