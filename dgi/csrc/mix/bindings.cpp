@@ -81,12 +81,14 @@ int dgi_glu_rows(void* out, const void* gu, int gu_stride, int rows, int I, int 
 int dgi_stream_add_norm(float* x, int T, int W, const void* y, int y_stride, int y_f32, const float* post_w,
                         const float* next_w, float eps, void* out, int out_f32, const void* y2, int y2_stride, int y2_f32,
                         float mult, hipStream_t s);
-int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
+int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride, int in_f32, int seg_rows);
+int dgi_linear_scan_segments(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
+                             int in_f32, const float* aux1, int aux1_stride, long long* floats);
 int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                     int v_stride, int in_f32, const float* aux1, int aux1_stride, const float* aux2, int aux2_stride,
                     const float* par1, const float* par2, float* state, float* norm, float* mx, const int* positions,
                     const int* seq_row0, const int* seq_slots, int n_seq, int H, int G, int dk, int dv, float cap,
-                    int rows, float* norm_new, float* mx_new, float* parts, int parts_chunks, hipStream_t st);
+                    int rows, float* norm_new, float* mx_new, float* parts, int parts_chunks, float* seg, int seg_rows, hipStream_t st);
 long long dgi_linear_scan_parts(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
                                 int in_f32, int* parts_chunks);
 int dgi_token_shift(void* out, int out_f32, const void* h, int h_f32, int h_stride, const float* mu, int nmix, float* tail,
@@ -964,11 +966,17 @@ void linear_scan(at::Tensor y, int64_t mode, const at::Tensor& q, const at::Tens
     nrm = norm->data_ptr<float>(); mxp = mx->data_ptr<float>();
   }
   const int n_seq = (int)seq_slots.numel();
+  // states between the segments of long portions
+  at::Tensor seg;
+  long long between = 0;
+  const int seg_rows = dgi_linear_scan_segments((int)mode, (int)dk, (int)dv, (int)H, (int)G, n_seq, T, q.data_ptr(), (int)q.stride(0), k.data_ptr(),
+                                                (int)k.stride(0), f, a1, a1s, &between);
+  if (between > 0) seg = at::empty({between}, state.options());
   // a matrix memory whose heads span several workgroups stages its new normaliser / maximum (committed by a second launch)
   at::Tensor norm_new, mx_new;
   float *nn = nullptr, *mn = nullptr;
   if (mode == 2 && n_seq > 0 && dgi_linear_scan_staged((int)dk, (int)dv, (int)H, n_seq, T, q.data_ptr(), (int)q.stride(0), k.data_ptr(),
-                                                      (int)k.stride(0), f)) {
+                                                      (int)k.stride(0), f, seg_rows)) {
     norm_new = at::empty({n_seq, H, dk}, state.options());
     mx_new = at::empty({n_seq, H}, state.options());
     nn = norm_new.data_ptr<float>(); mn = mx_new.data_ptr<float>();
@@ -983,7 +991,8 @@ void linear_scan(at::Tensor y, int64_t mode, const at::Tensor& q, const at::Tens
                            f32p(par1, "par1", np), f32p(par2, "par2", np), state.data_ptr<float>(), nrm, mxp,
                            i32p(positions, "positions", T), i32p(seq_row0, "seq_row0", n_seq + 1),
                            i32p(seq_slots, "seq_slots"), n_seq, (int)H, (int)G, (int)dk, (int)dv, (float)cap, T,
-                           nn, mn, parts.defined() ? parts.data_ptr<float>() : nullptr, parts_chunks, cur_stream()), "linear_scan");
+                           nn, mn, parts.defined() ? parts.data_ptr<float>() : nullptr, parts_chunks,
+                           seg.defined() ? seg.data_ptr<float>() : nullptr, seg_rows, cur_stream()), "linear_scan");
 }
 
 // paged caches of one attention layer: k [NB, G, bs, dk], v [NB, G, bs, dv]

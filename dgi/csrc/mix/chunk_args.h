@@ -23,9 +23,11 @@ struct ChunkArgs {
   int H, G, dk, dv;
   int n_seq;
   int pass, seg_rows;              // ssm in segments: 0 whole portions, 1 and 2 the two passes
-  float *ws, *wsd;                 // [n_seq, segments, H, dv, dk] states, [n_seq, segments, H] decays
+  float *ws, *wsd;                 // [n_seq, segments, H, dv, dk] states, [n_seq, segments, H] decays (chunk_segments.h: as said there)
   int skip_rows;                   // sequences of at most this many rows are not this launch's
   float cap;
+  int blocks;                      // chunk_segments.h: of 16 columns, of a head in ws
+  float share;                     // workgroups of a portion over those the chip has at once
   float* parts;                    // what a pass before keeps for the launch's chunks (parts_chunks of them): ssm chunk_parts.hip, delta chunk_delta.hip; or null
   int parts_chunks;
 };
@@ -87,6 +89,10 @@ __device__ __forceinline__ float larger3(float m, float a, float b) {
 
 }  // namespace
 
+int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows, int in_f32, long long* floats);
+int dgi_chunk_segments_groups(int mode, int dv);
+float dgi_chunk_segments_share(int mode, int dk, int dv, int H);
+int dgi_chunk_segments(ChunkArgs a, int mode, int in_f32, int rows, float* ws, hipStream_t st);
 bool dgi_chunk_parts_takes(int mode, int dk, int H, int G, int in_f32);
 int dgi_chunk_parts(const ChunkArgs& a, int mode, int in_f32, dim3 grid, hipStream_t st);
 int dgi_chunk_delta(const ChunkArgs& a, int in_f32, dim3 grid, hipStream_t st);

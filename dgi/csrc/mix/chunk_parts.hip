@@ -30,7 +30,8 @@
 //   ssm, 2 prompts of 4096 rows, 64 heads of 128 x 64     210 us -> 168 (of it 15 the pass before)
 //   mlstm, 5 prompts of 3001 bf16 rows, 32 heads of 64     83 -> 49;  of 128 197 -> 137;  fp32 rows 105 -> 74
 //   light, 2 prompts of 4096 bf16 rows, 64 heads of 64    158 -> 113
-// mlstm on fp32 rows of 128 channels stays there (its waves would spill: 213 -> 230 us); delta: chunk_delta.hip.
+// mlstm on fp32 rows of 128 channels stays there (its waves would spill: 213 -> 230 us); delta: chunk_delta.hip; steps of mlstm and light of many short portions
+// or few long ones: chunk_segments.h.
 //
 // Precision: results and states are no further from 64 bits than the token loop's, nor (2-norm) by more than a hundredth than in chunk_scan.hip, whose P u is in
 // 64 bits.  512 rows, 16 heads, errors over that kernel's of outputs and states: ssm 0.78, 0.92 (7.0e-8; the loop 1.03e-7); light 0.46, 0.31; mlstm 0.94, 0.76 (64

@@ -1,6 +1,7 @@
 // dgi/csrc/mix/chunk_scan.hip — prompt portions of the recurrences that carry a matrix S [dk, dv] per head (linear_scan.hip has
 // their definitions, ssm_scan.hip that of ssm), sixteen tokens at a time in fp32 matrix products (v_mfma_f32_16x16x4_f32).  Those that chunk_parts.hip
-// takes (light; mlstm, but for fp32 rows of more than 64 channels; ssm of groups of four heads) go there, long portions of delta to chunk_delta.hip.
+// takes (light; mlstm, but for fp32 rows of more than 64 channels; ssm of groups of four heads) go there, long portions of delta to chunk_delta.hip, steps of gla,
+// light and mlstm that dgi_chunk_segments_plan says to chunk_segments.h.
 //
 // For tokens t, s of a chunk that starts from the state S, with D[t, s] the product of the decays of the tokens after s up to t
 // and A_t that of all tokens up to t:
@@ -13,7 +14,7 @@
 // products and no division;  it reads before it writes: s < t, and the bonus on the diagonal;
 // delta: u solves (I + T) u = beta (v - A S^T k), T[t, s] = beta_t D[t, s] (k_t . k_s) below the diagonal: block forward
 // substitution with blocks of four tokens, each block one matrix product with M_b = [inverse of its diagonal block - I;
-// - T below it times that inverse].  (gla: chunk_scan_decay.hip.)
+// - T below it times that inverse].  (gla: chunk_segments.h, chunk_scan_decay.hip.)
 //
 // A workgroup owns (sequence, head, NC blocks of 16 value columns: two, or four, see four_blocks) and is a pipeline of waves that hand chunks on through LDS, one
 // barrier per chunk:
@@ -1090,14 +1091,15 @@ int launch_mode(const ChunkArgs& a, int in_f32, bool four, dim3 grid, hipStream_
 // Whether prompt portions of these shapes run here: key sizes of at most 128 (ssm: 256), and, but for wkv,
 // rows of q and k that can be read four elements at a time.
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32) {
-  if (mode == 3 || dk <= 0 || dk > (mode == SSM ? 256 : 128)) return 0;
+  if (dk <= 0 || dk > (mode == SSM ? 256 : 128)) return 0;
   if (mode == WKV) return 1;
   const int piece = in_f32 ? 15 : 7;               // bytes of four elements, less one
   return dk % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && (((uintptr_t)q | (uintptr_t)k) & piece) == 0;
 }
 
 // mode as above (and light: par1 the decays; ssm: q = C, k = B, v = x, aux1 = dt_raw (aux_bf16), par1 a_log, par2 dt_bias, par3 d_skip).
-// Needs dgi_chunk_scan_ok.  skip_rows: sequences of at most that many rows are left to another launch.  segs > 1 (ssm): portions are
+// Needs dgi_chunk_scan_ok.  skip_rows: sequences of at most that many rows are left to another launch.  gla, light, mlstm with seg_rows: by chunk_segments.h, seg_rows
+// and ws as dgi_chunk_segments_plan says, rows: of the step.  segs > 1 (ssm): portions are
 // cut into segments of seg_rows rows (a multiple of 32, segs of them at least as long as the longest portion) that run side by side: each one's
 // state from nothing, a short serial pass over those states, then the outputs from each segment's incoming state.  About
 // twice the work, for steps whose heads leave most of the chip idle.  parts: ssm: dgi_ssm_parts_floats of workspace for chunk_parts.hip, delta:
@@ -1107,10 +1109,11 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
                               float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
-                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st) {
+                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, int rows, hipStream_t st) {
   if (n_seq == 0) return 0;
   const int cols = dk <= 128 ? 32 : 16;            // value columns of a workgroup (or twice as many, see four_blocks)
-  const long long nz = (dv + cols - 1) / cols;
+  const bool beside = mode != SSM && seg_rows > 0;      // chunk_segments.h
+  const long long nz = beside ? dgi_chunk_segments_groups(mode, dv) : (dv + cols - 1) / cols;
   if (!dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32) || dv <= 0 || H <= 0 || G <= 0 || H % G) return -3;
   if (mode == MLSTM && nz > 1 && (!norm_new || !mx_new)) return -7;
   ChunkArgs a;
@@ -1123,6 +1126,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
   a.H = H; a.G = G; a.dk = dk; a.dv = dv; a.skip_rows = skip_rows;
   if (n_seq * nz * H > 0x3fffffff || segs > 65535 || (segs > 1 && (mode != SSM || !ws || !wsd || seg_rows <= 0))) return -3;
   a.n_seq = n_seq; a.seg_rows = seg_rows; a.ws = ws; a.wsd = wsd; a.parts = parts; a.parts_chunks = parts_chunks;
+  if (beside) return dgi_chunk_segments(a, mode, in_f32, rows, ws, st);
   a.pass = segs > 1 ? 1 : 0;
   const dim3 grid((unsigned)(n_seq * nz * H), segs > 1 ? segs : 1);
   // more workgroups than compute units: possibly of four column blocks each

@@ -1,5 +1,5 @@
-// dgi/csrc/mix/chunk_scan_decay.hip — gla and light (see linear_scan.hip) for the prompt portions that chunk_scan.hip does not take: steps of
-// few workgroups, key sizes of 129 to 256 (its buffers would not fit LDS) and rows of light that cannot be read four elements at
+// dgi/csrc/mix/chunk_scan_decay.hip — gla and light (see linear_scan.hip) for the prompt portions that chunk_segments.h and chunk_parts.hip do not take: steps of
+// few workgroups, key sizes of 129 to 256 (their buffers would not fit LDS) and rows that cannot be read four elements at
 // a time.  Sixteen tokens at a time in fp32 matrix products (v_mfma_f32_16x16x4_f32):
 //
 //     S_t = diag(a_t) S_(t-1) + k_t v_t^T,   o_t = S_t^T q_t                       S [dk, dv] fp32

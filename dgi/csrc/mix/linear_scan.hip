@@ -28,7 +28,7 @@
 // running maximum is a serial pass of one thread (adds and maxima; its exponentials are parallel again).
 // The token loop reads LDS only.  Everything is fp32; q / k / v arrive as bf16 or fp32.
 // A portion that starts at position 0 reads no state; the state is written back at the end of the portion.
-// Prompt portions run in chunks of tokens on the matrix cores instead (chunk_scan.hip, chunk_parts.hip, chunk_delta.hip): what is left here are steps of
+// Prompt portions run in chunks of tokens on the matrix cores instead (chunk_scan.hip, chunk_parts.hip, chunk_segments.h, chunk_delta.hip): what is left here are steps of
 // single rows and short portions, key sizes above 128 (gla, light: 256), and rows of delta and mlstm that cannot be read in fours.
 #include "../common.h"
 
@@ -1124,8 +1124,11 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
                               float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
-                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st);
+                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, int rows, hipStream_t st);
 long long dgi_chunk_delta_floats(int dk, int H, int T, int n_seq, int in_f32, int* chunks);
+int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows, int in_f32, long long* floats);
+int dgi_chunk_segments_groups(int mode, int dv);
+float dgi_chunk_segments_share(int mode, int dk, int dv, int H);
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 extern "C" int dgi_chunk_scan_decay(float* y, int light, const void* q, int q_stride, const void* k, int k_stride, const void* v,
                                    int v_stride, int in_f32, const float* decay, int decay_stride, float* state,
@@ -1144,7 +1147,8 @@ constexpr int APART_FROM = 8;        // sequences of a step above which those ar
 // 13; 400 rows 31, 25; 512 units, 100 rows 16, 12; 1024 units, 64 rows 20, 17; 2048 units, 64 rows 36, 35; 128-wide heads: 128 units, 100 rows 15, 15;
 // 1024 units, 64 rows 30, 25; 4096 units, 64 rows 108, 91).
 // Among more than APART_FROM sequences it has a launch more to lose (64-wide heads: 9 x 80 rows, 16 heads 17, 20; 12 x 112 22, 24; 12 x 128 24, 24; 9 x 80, 32
-// heads 24, 28; 9 x 96 28, 28; 24 x 65, 32 heads 52, 49; 128-wide: 9 x 80, 8 heads 24, 27; 9 x 96 28, 27).
+// heads 24, 28; 9 x 96 28, 28; 24 x 65, 32 heads 52, 49; 128-wide: 9 x 80, 8 heads 24, 27; 9 x 96 28, 27).  mlstm of up to 64 channels has
+// chunk_segments.h, which fills sooner, too (bf16 rows of 16 heads, 8 x 20 rows 19.8 -> 9.1, 1 x 40 21.9 -> 10.7; with a launch more, 14 x 18 25 -> 34, 16 x 40 19.9 -> 13.3).
 static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
   const long units = (long)n_seq * H * ((dv + 15) / 16);
   if (mode == LIGHT) {
@@ -1152,6 +1156,7 @@ static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
     if (units <= 768) return dk <= 64 ? 112 : 88;
     return dk <= 64 && (units <= 1280 || n_seq <= 16) ? 88 : 64;
   }
+  if (mode == MLSTM && dk <= 64) return n_seq > APART_FROM ? 24 : SHORT;
   if (mode != WKV || units <= 512) return 64;
   return dk > 64 ? 104 : units <= 3072 ? 136 : 224;
 }
@@ -1161,7 +1166,7 @@ static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
 // average and yet many rows are decode rows beside long portions.  Among many sequences both kernels are launched and each
 // sequence is taken by its own length; in between the launch of chunk_scan.hip would mostly be in vain.
 // gla and light have chunk_scan_decay.hip too, with little to fill: better than this file's kernel from some four rows a sequence on, or 128 rows
-// beside decode rows.
+// beside decode rows.  What of 1 and 2 goes to chunk_segments.h instead is dgi_chunk_segments_plan's to say.
 static int chunk_form(int mode, int dk, int dv, int G, int H, const void* q, int q_stride, const void* k, int k_stride, int in_f32, int n_seq,
                       int rows) {
   const long from = chunk_from(mode, dk, dv, H, n_seq);
@@ -1170,7 +1175,7 @@ static int chunk_form(int mode, int dk, int dv, int G, int H, const void* q, int
     if (from <= 64) portions |= rows - n_seq >= 256;
     else if (n_seq > APART_FROM) portions = 4l * rows > 3 * from * n_seq || (rows - n_seq >= 512 && rows <= 48l * n_seq);
   }
-  const bool ok = portions && dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32);
+  const bool ok = mode != GLA && portions && dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32);
   if ((mode == GLA || mode == LIGHT) && dk <= 256 && G == H) {
     if (ok) return 1;
     return rows > 4 * n_seq || rows - n_seq >= 128 ? 2 : 0;
@@ -1178,11 +1183,20 @@ static int chunk_form(int mode, int dk, int dv, int G, int H, const void* q, int
   return ok;
 }
 
+// The rows that portions of a step are cut into for chunk_segments.h, 0: they do not go there; *floats of workspace.
+extern "C" int dgi_linear_scan_segments(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
+                                        int in_f32, const float* aux1, int aux1_stride, long long* floats) {
+  *floats = 0;
+  if (n_seq == 0 || G != H || !chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows)) return 0;
+  if (!dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32) || (mode == GLA && (aux1_stride % 2 || ((uintptr_t)aux1 & 7)))) return 0;
+  return dgi_chunk_segments_plan(mode, dk, dv, H, n_seq, rows, in_f32, floats);
+}
+
 // whether the matrix memory of a step has several workgroups per head in one of its launches: its normaliser and maximum are staged
 extern "C" int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
-                                      int in_f32) {
+                                      int in_f32, int seg_rows) {
   const bool chunked = chunk_form(MLSTM, dk, dv, H, H, q, q_stride, k, k_stride, in_f32, n_seq, rows) != 0;
-  if (chunked && dv > 32) return 1;
+  if (chunked && (seg_rows ? dgi_chunk_segments_groups(MLSTM, dv) > 1 : dv > 32)) return 1;
   if (chunked && n_seq <= APART_FROM) return 0;
   const int R = scan_channels(dk, dv, H, n_seq, chunked ? n_seq : rows);
   int KS = 1;
@@ -1210,7 +1224,7 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
                                int aux2_stride, const float* par1, const float* par2, float* state, float* norm, float* mx,
                                const int* positions, const int* seq_row0, const int* seq_slots, int n_seq, int H, int G,
                                int dk, int dv, float cap, int rows, float* norm_new, float* mx_new, float* parts, int parts_chunks,
-                               hipStream_t st) {
+                               float* seg, int seg_rows, hipStream_t st) {
   if (n_seq == 0) return 0;
   if (mode < 0 || mode > 4 || H <= 0 || G <= 0 || H % G || dk <= 0 || dv <= 0) return -2;
   if (dk > 512) return -3;
@@ -1221,14 +1235,18 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   bool short_rows = rows <= 4 * n_seq;             // rows of the step: at most four per sequence on average
   const bool staged = mode == MLSTM && norm_new && mx_new;
   // Prompt portions: sixteen or 32 tokens at a time on the matrix cores (chunk_scan.hip, chunk_parts.hip, chunk_delta.hip).  Among many sequences there are decode
-  // rows and short portions beside the long ones: they stay with this kernel, in a launch of their own.
+  // rows and short portions beside the long ones: they stay with this kernel, in a launch of their own (gla and light beside chunk_segments.h's where
+  // that kernel's workgroups for all sequences are more than the chip has at once: its first chunk takes 7 us whatever a portion's rows.  16 heads of 64, 7 portions of 87
+  // rows in all and 12 decode rows 13.9 in two launches, 8.9 in one; 64 heads, 2 of 1539 and 15 decode rows 76 in one, 59 in two).
   const int form = chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows);
-  const int apart = n_seq > APART_FROM && (form == 1 || (form == 2 && rows <= 4 * n_seq))
-                        ? (mode == WKV && chunk_from(mode, dk, dv, H, n_seq) > 64 ? (int)chunk_from(mode, dk, dv, H, n_seq) : SHORT) : 0;
+  const bool beside = seg_rows && mode != MLSTM;
+  const bool two = n_seq > APART_FROM && (beside ? rows <= 160 * n_seq && n_seq * dgi_chunk_segments_share(mode, dk, dv, H) > 1.f
+                                                 : form == 1 || (form == 2 && rows <= 4 * n_seq));
+  const int apart = !two ? 0 : beside ? 4 : mode == WKV && chunk_from(mode, dk, dv, H, n_seq) > 64 ? (int)chunk_from(mode, dk, dv, H, n_seq) : SHORT;
   if (form) {
-    const int rc = form == 1 ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
+    const int rc = form == 1 || seg_rows ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
                                               aux2, aux2_stride, 0, par1, par2, nullptr, cap, state, norm, mx, norm_new, mx_new, positions,
-                                              seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, 0, nullptr, nullptr, parts, parts_chunks, st)
+                                              seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, seg_rows, seg, nullptr, parts, parts_chunks, rows, st)
                              : dgi_chunk_scan_decay(y, mode == LIGHT, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? par1 : aux1,
                                                    mode == LIGHT ? 0 : aux1_stride, state, positions, seq_row0, seq_slots, n_seq, H, dk, dv,
                                                    apart, st);

@@ -264,7 +264,7 @@ extern "C" int dgi_chunk_scan(float* y, int mode, const void* q, int q_stride, c
                               int aux_bf16, const float* par1, const float* par2, const float* par3, float cap, float* state,
                               float* norm, float* mx, float* norm_new, float* mx_new, const int* positions, const int* seq_row0,
                               const int* seq_slots, int n_seq, int H, int G, int dk, int dv, int skip_rows,
-                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, hipStream_t st);
+                              int segs, int seg_rows, float* ws, float* wsd, float* parts, int parts_chunks, int rows, hipStream_t st);
 
 extern "C" int dgi_chunk_scan_ok(int mode, int dk, const void* q, int q_stride, const void* k, int k_stride, int in_f32);
 bool dgi_chunk_parts_takes(int mode, int dk, int H, int G, int in_f32);
@@ -323,7 +323,7 @@ extern "C" int dgi_ssm_scan(float* y, const float* xbc, int xbc_stride, const vo
     most = apart_rows(n_seq, heads, dv, N, G);
     const int rc = dgi_chunk_scan(y, 5, B + (size_t)G * N, xbc_stride, B, xbc_stride, xbc, xbc_stride, 1, dt_raw, dt_stride, nullptr, 0,
                                   !dt_f32, a_log, dt_bias, d_skip, 0.f, state, nullptr, nullptr, nullptr, nullptr, positions, seq_row0,
-                                  seq_slots, n_seq, heads, G, N, dv, most, segs, seg_rows, ws, wsd, parts, parts_chunks, s);
+                                  seq_slots, n_seq, heads, G, N, dv, most, segs, seg_rows, ws, wsd, parts, parts_chunks, 0, s);
     if (rc || !most) return rc;
   }
   const int nq = (N + 63) / 64;
