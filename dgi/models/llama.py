@@ -725,7 +725,8 @@ class LlamaModel:
             if self._fold_ok(h):
                 return self._forward_layers_folded(h, meta, residual, trim_last)
             fq, fg = self._fused_decode(h, meta)
-            if fq or fg:
+            if (fq or fg) and (self.force_fused or not self._stream_ok(h)
+                             or not ops.stream_over_fused(T, self.layers[0].gate_up.shape[0] // 2, h.shape[1])):
                 h, residual = self._forward_layers_fused(h, meta, residual, fq, fg)
                 if trim_last is not None:     # same contract as the unfused path: only the logits rows
                     h, residual = h.index_select(0, trim_last), residual.index_select(0, trim_last)

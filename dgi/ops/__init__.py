@@ -663,7 +663,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
 # Where it pays (profiles/r2_decode8b_fused.md, hipGraph-timed, weights cold):
 # the qkv projection at M <= 8 (15 vs 18 us at M = 1 on 8B); gate_up on the persistent
 # one-ring workgroups (cfg 12-16: X staged once per CU, one weight stream per CU) at every
-# M <= 16 (55.5 vs 62.4 us unfused at M = 16, profiles/r3_decode/persistent_gemv.md).
+# M <= 16 (55.5 vs 62.4 us unfused at M = 16, profiles/r3_decode/persistent_gemv.md);
+# wide layers that may take the streaming products stay here up to 2 rows (stream_over_fused).
 # K <= 4096 (8B-class) like _use_skinny.
 # DGI_FUSED_DECODE=0 disables, =force uses it for every M <= 16 and K.
 FUSED_DECODE = os.environ.get("DGI_FUSED_DECODE", "1")
@@ -700,6 +701,15 @@ def fused_decode_ok(M: int, K: int, kind: str = "qkv") -> bool:
     if FUSED_DECODE == "force":
         return True
     return K <= 4096 and M <= min(SKINNY_MAX_M, FUSED_MAX_M.get(kind, 0))
+
+
+def stream_over_fused(M: int, I: int, K: int) -> bool:
+    """Whether layers of K wide rows and I wide feed-forwards are the faster on the streaming products than with the fused ones, where a step may take either: their
+    weights go straight to LDS in whole lines at any number of rows, the fused ones' rings slow down with it.  Four layers and the logits of a
+    decode step, us fused and streamed at 2, 3, 4, 8, 16 rows: 4096 x 14336 576 584, 590 587, 601 588, 633 594, 689 616; 4096 x 11008 with 32 kv
+    heads 656 573, 668 574, 684 573, 719 587, 781 638; 3072 x 8192 398 444, 408 450, 416 460, 444 470, 519 499 (12 rows 499 486); narrower ones have
+    too few units of 128 weight rows: 2048 x 8192 282 330, 291 335, 300 340, 325 348, 368 373."""
+    return FUSED_DECODE != "force" and (M > 2 if K >= 4096 else K >= 3072 and M > 8) and glu_streams(M, I, K)
 
 
 def fused_skinny_ref(y, x, res, res_out, gamma, eps, w, bias, pro, epi, positions=None, cos_sin=None,

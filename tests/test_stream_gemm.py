@@ -190,6 +190,17 @@ def test_layers_on_the_gpu(monkeypatch, T, prompts):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,K,stream", [(2, 4096, False), (3, 4096, True), (16, 4096, True), (8, 3072, False), (9, 3072, True), (16, 2048, False)])
+def test_few_rows(monkeypatch, T, K, stream):
+    """Rows and widths around the line between the fused layers and these."""
+    names, real = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (names.append(name), real(name, *a))[1])
+    plain, got = layers("cuda", T, [], monkeypatch, hidden_size=K, intermediate_size=5632, num_heads=16, num_kv_heads=4)
+    close(got, plain)
+    assert names.count("fused_skinny") and names.count("rope_cache_parts") == (2 if stream else 0)
+
+
+@pytest.mark.gpu
 def test_a_step_takes_them_and_replays(monkeypatch):
     """17 rows of a 2048-wide model: the layers run on the streaming products, eagerly and as a graph that is replayed between other work."""
     from dgi.engine import EngineConfig, LLMEngine
@@ -261,3 +272,6 @@ def test_sizes_that_stream():
     assert glu(14336, 4096) == glu(13824, 5120) == glu(8960, 1536) == [1, 32, 33, 64, 65, 96, 97, 128]
     assert glu(8192, 4096) == glu(28672, 8192) == glu(24576, 6144) == [1, 32, 33, 64]
     assert glu(4096, 2048) == [1, 32]
+    over = lambda I, K: [M for M in (1, 2, 3, 8, 9, 16) if ops.stream_over_fused(M, I, K)]  # noqa: E731
+    assert over(14336, 4096) == over(5632, 4096) == [3, 8, 9, 16] and over(8192, 3072) == [9, 16]
+    assert over(17408, 4096) == over(8192, 2048) == []
