@@ -17,7 +17,7 @@
 // 128-byte lines, straight to LDS.  Up to 64 places a tile: the workgroups share the weight rows out evenly and stream them with
 // the tile's rows of A kept in registers; where those do not fit (or K is no multiple of 64), a workgroup owns 64 weight rows
 // and both operands come through LDS stages.  Many rows: tiles of 128 places by 128 weight rows, K in steps of 64 through two
-// LDS stages (32x32x16 products).  Very many: 256 by 256, loaded to LDS directly and multiplied by two groups of waves in turn.
+// LDS stages (32x32x16 products), or 256 by 256, loaded to LDS directly and multiplied by two groups of waves in turn (launch_group says which).
 //
 // The tile a workgroup owns is found from seg alone, so the grid is sized for the worst split of the places over the
 // experts and a workgroup past the last tile leaves.  Weights are the A operand: a lane's result is four consecutive
@@ -602,25 +602,33 @@ __global__ __launch_bounds__(256, 2) void moe_group_tiles_kernel(GroupArgs g, in
 }
 
 // ---- very many rows per expert: up to 256 places x 256 weight rows (GLU: 128 outputs, gate and up), K in steps of 64
-// through two LDS stages of 64 KB, eight waves of 128 places x 64 weight rows.  The matrix cores bound it, so they have to
-// be fed: loads go to LDS directly, and the two waves of a SIMD run one section apart (one reads its operands and issues
+// through LDS, two stages of places and three of weights (all 160 KB), eight waves of 128 places x 64 weight rows.  The matrix cores
+// have to be fed: loads go to LDS directly, and the two waves of a SIMD run one section apart (one reads its operands and issues
 // loads while the other multiplies; every section ends at a barrier), so a SIMD's matrix core is never without work.
+// What bounds experts of one tile of places is reading their weights (without its products gate-up of 222 places each took 147 us
+// of 156, without the weights' loads 51): they are asked for one and a half steps ahead, half a step before, and marked as read once.
 //
-// An expert's n places are shared out evenly over ceil(n / 256) tiles, and a tile of r places multiplies
-// H = ceil(r / 64) blocks of 16 per wave and section, not 4: an expert of 520 places costs 3 x 3/4 tiles, not 3.
+// An expert's n places are shared out in blocks of 64 over ceil(n / 256) tiles, and a tile of H blocks multiplies
+// H blocks of 16 per wave and section, not 4: an expert of 520 places costs 3 x 3/4 tiles, not 3.
 // Tiles are counted expert by expert, an expert's places fastest, and every XCD takes a contiguous run: the 32 tiles it
 // works on at a time are a few tiles of places by about ten of weights of one or two experts, which meet in its L2
-// (places of all experts first: each tile would read weights of its own).
+// (places of all experts first: each tile would read weights of its own).  Tiles left after an XCD's whole rounds of 32 are cut along their
+// places where that gives its units more work: up to eight into four, up to sixteen into two (a tile takes about 0.32 + 0.17 H of a whole
+// one's time, so more than sixteen gain nothing).
 //
 // 16 experts, K 4096, ff 3584, 512 places each: gate-up 796 us -> 406 (1184 TF/s), down 407 -> 187 (1288); 1024 places
 // each 1342 and 1327 TF/s, 256 each 1028 (one tile of places: the weights come at 4.8 TB/s).  What is left is the last
-// round of tiles: 520 places each are 5.25 rounds of 256 workgroups and take 513 us.
+// round of tiles: 520 places each are 5.25 rounds of 256 workgroups and take 513 us.  The whole feed-forward of 16 experts with two stages of
+// weights, half a step ahead and nothing cut, and as it is: 2048 x 4096, 889 rows of top 4 320 us -> 279, 2000 490 -> 450; 2048 x 2048, top 2, 935 rows 147 ->
+// 123, 1641 160 -> 137; 4096 x 3584, top 2, 2200 rows 582 -> 555, 4096 752 -> 752.
 constexpr int WIDE = 256;
 constexpr int W_TILE = WIDE * 64 * 2;                  // one operand of one stage, bytes
-constexpr int W_STAGE = 2 * W_TILE;
+constexpr int W_AT = 2 * W_TILE;                       // the weights' stages behind the places'
+constexpr int MORE = 24;                               // workgroups of an XCD for tiles that are cut
 
 struct WideTile {
   int e, lo, hi, nt;                                   // expert, places [lo, hi), weight tile
+  bool once;                                           // no other tile has these weights
 };
 
 // Tile blockIdx.x of the places' tiles times `ntn` weight tiles; false past the last.  Uniform over the workgroup.
@@ -634,8 +642,18 @@ __device__ __forceinline__ bool find_wide(const int* __restrict__ seg, int E, in
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
   total *= ntn;
-  const int chunk = (total + 7) >> 3, at = blockIdx.x >> 3, id = (blockIdx.x & 7) * chunk + at;
-  if (at >= chunk || id >= total) return false;
+  const int chunk = (total + 7) >> 3, first_id = (blockIdx.x & 7) * chunk, mine = min(chunk, total - first_id);
+  if (mine <= 0) return false;
+  const int left = mine & 31, most = left > 16 ? 1 : left > 8 ? 2 : 4;      // at most MORE workgroups more
+  int at = blockIdx.x >> 3, parts = 1, part = 0;
+  if (at >= mine - left) {
+    const int k = at - (mine - left);
+    parts = most;
+    at = mine - left + k / most;
+    part = k % most;
+  }
+  if (at >= mine) return false;
+  const int id = first_id + at;
   int base = 0;
   for (int e0 = 0; e0 < E; e0 += 64) {
     const int ee = e0 + lane;
@@ -652,12 +670,19 @@ __device__ __forceinline__ bool find_wide(const int* __restrict__ seg, int E, in
       const int l = __ffsll(m) - 1;
       const int tiles = __shfl(n, l, 64), first = base + __shfl(inc, l, 64) - tiles;
       const int a = __shfl(s0, l, 64), b = __shfl(s1, l, 64);
-      const int per = (b - a + tiles - 1) / tiles, j = (id - first * ntn) % tiles;
+      const int blocks = (b - a + 63) >> 6, j = (id - first * ntn) % tiles;
+      int lo = j * blocks / tiles, hi = (j + 1) * blocks / tiles;
+      parts = min(parts, hi - lo);
+      if (part >= parts) return false;
+      t.once = tiles == 1 && parts == 1;
+      const int own = hi - lo;
+      hi = lo + (part + 1) * own / parts;
+      lo += part * own / parts;
       t.e = e0 + l;
       t.nt = (id - first * ntn) / tiles;
-      t.lo = a + j * per;
-      t.hi = min(b, a + (j + 1) * per);
-      return t.lo < t.hi;
+      t.lo = a + 64 * lo;
+      t.hi = min(b, a + 64 * hi);
+      return true;
     }
     base += __shfl(inc, 63, 64);
   }
@@ -676,46 +701,72 @@ __device__ __forceinline__ void st_pair(uint16_t* row, int n0, int N, int g, con
 // K a multiple of 128, N of 8, out at a 16-byte boundary; rows of A and the weights of an expert under 2 GiB each.
 template <bool GLU>
 __global__ __launch_bounds__(512) void moe_group_wide_kernel(GroupArgs g, int ntn) {
-  __shared__ __attribute__((aligned(16))) char lds[2 * W_STAGE];               // [stage][places | weights], rows of 128 bytes
+  __shared__ __attribute__((aligned(16))) char lds[5 * W_TILE];                // [stages][rows of 128 bytes]
   WideTile t;
   if (!find_wide(g.seg, g.E, ntn, t)) return;
   t.e = __builtin_amdgcn_readfirstlane(t.e);           // in scalar registers: bases and branches are
   t.nt = __builtin_amdgcn_readfirstlane(t.nt);
   t.lo = __builtin_amdgcn_readfirstlane(t.lo);
   t.hi = __builtin_amdgcn_readfirstlane(t.hi);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wm = w >> 2, wn = w & 3;
+  t.once = __builtin_amdgcn_readfirstlane(t.once);
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = w >> 2, wn = w & 3;
   const int H = (t.hi - t.lo + 63) >> 6;
   constexpr int NO = GLU ? 128 : 256;
   const int n0 = t.nt * NO;
   // Staging: slab i = 64 LDS rows.  Slabs 2 m, 2 m + 1 hold the first and second 16 H places of wave row m (rows past
   // 16 H repeat a place); slab i of the weights holds wave column i's rows (GLU: 32 gate rows, then the matching up rows).
   // Chunk c of LDS row r is chunk c ^ (r >> 1 & 7) of its 64 elements: reads of 16 rows spread over all banks.
-  const char* A = reinterpret_cast<const char*>(g.a);
-  const char* B = reinterpret_cast<const char*>(g.b + (size_t)t.e * (GLU ? 2 : 1) * g.N * g.K);
-  unsigned ao[4], bo[4];
-  {
-    const int q = tid >> 3, c = ((tid & 7) ^ ((tid >> 4) & 7)) * 16;
+  // Waves 0-3 load the weights, wave i slab i, eight rows a load; waves 4-7 the places, load j 16 rows of slab j / 2: loads land in
+  // order, so each waits for its own kind only.
+  const char* const src = wm ? reinterpret_cast<const char*>(g.a) : reinterpret_cast<const char*>(g.b + (size_t)t.e * (GLU ? 2 : 1) * g.N * g.K);
+  unsigned off[8];
+  if (wm) {
+    int row[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int place = min(t.lo + i * 16 * H + min(q, 16 * H - 1), t.hi - 1);
-      ao[i] = (unsigned)(g.order ? g.order[place] / g.top : place) * (unsigned)g.a_stride * 2u + c;
-      const int n = GLU ? n0 + 32 * i + (q & 31) : n0 + 64 * i + q;
-      bo[i] = (unsigned)(min(n, g.N - 1) + (GLU && q >= 32 ? g.N : 0)) * (unsigned)g.K * 2u + c;
+    for (int j = 0; j < 8; ++j) row[j] = min(t.lo + (j >> 1) * 16 * H + min(16 * wn + 8 * (j & 1) + (lane >> 3), 16 * H - 1), t.hi - 1);
+    if (g.order) {                                     // all asked for before the first is divided
+#pragma unroll
+      for (int j = 0; j < 8; ++j) row[j] = g.order[row[j]];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) row[j] = (int)((unsigned)row[j] / (unsigned)g.top);
     }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) off[j] = (unsigned)row[j] * (unsigned)g.a_stride * 2u;
+  } else {
+    auto row = [&](int q) { return (unsigned)(min(n0 + (GLU ? 32 * wn + (q & 31) : 64 * wn + q), g.N - 1) + (GLU && q >= 32 ? g.N : 0)) * (unsigned)g.K * 2u; };
+#pragma unroll
+    for (int j = 0; j < 8; ++j) off[j] = row(8 * j + (lane >> 3));
   }
-  char* const la = lds + w * 1024;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) off[j] += ((lane & 7) ^ ((4 * j + (lane >> 4)) & 7)) * 16;
+  char* const la = lds + wn * 2048;
+  char* const lb = lds + W_AT + wn * 8192;
   // the step's base stays in scalar registers, a lane keeps 32-bit offsets (64-bit addresses per lane spill)
-  auto at = [](const char* p, int kt) {
-    p += (size_t)kt * 128;
+  auto at = [&](int kt) {
+    const char* p = src + (size_t)kt * 128;
     asm volatile("" : "+s"(p));
     return p;
   };
-  auto ga = [&](int kt, int i, int st) { load_lds16(at(A, kt) + ao[i], la + st * W_STAGE + i * 8192); };
-  auto gb = [&](int kt, int i, int st) { load_lds16(at(B, kt) + bo[i], la + st * W_STAGE + W_TILE + i * 8192); };
+  auto ga = [&](int kt, int i, int st) {               // slab i of the places
+    const char* p = at(kt);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) load_lds16(p + off[2 * i + u], la + st * W_TILE + i * 8192 + u * 1024);
+  };
+  auto gb = [&](int kt, int st) {
+    const char* p = at(kt);
+    if (t.once) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) load_lds16_once(p + off[j], lb + st * W_TILE + j * 1024);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) load_lds16(p + off[j], lb + st * W_TILE + j * 1024);
+    }
+  };
+  const int steps = g.K >> 6;                          // even
 
   const int lr = lane & 15, lg = lane >> 4, key = (lane >> 1) & 7;
   const int p0 = (lg ^ key) * 16, p1 = ((4 + lg) ^ key) * 16;
-  const int abase = (wm * 128 + lr) * 128, bbase = W_TILE + (wn * 64 + lr) * 128;
+  const int abase = (wm * 128 + lr) * 128, bbase = W_AT + (wn * 64 + lr) * 128;
   f32x4 acc[2][4][4];                                  // [half][block of places][block of weights]
 #pragma unroll
   for (int h = 0; h < 2; ++h)
@@ -733,17 +784,18 @@ __global__ __launch_bounds__(512) void moe_group_wide_kernel(GroupArgs g, int nt
   };
   // the K loop with HB blocks of 16 places per half.  A step is two sections per wave:
   //
-  //   section  reads                        products             loads issued                 landed before its barrier
-  //   0        first half, weights          first x weights      weights, slab 2 of step + 1  slabs 1, 3 of this step
-  //   1        second half                  second x weights     slabs 3, 1 of + 1, 0 of + 2  all of + 1 but slabs 3, 1
+  //   section  reads                        products             loads issued: weights      places
+  //   0        first half, weights          first x weights      step + 2                   slabs 1, 3 of step + 1
+  //   1        second half                  second x weights                                slabs 0, 2 of step + 2
   //
-  // A slab is loaded again two sections or more after its last read, and a wave counts only its own loads: what it waits
-  // for is visible to the others behind the barrier.  MODE 1, 2: the last step but one, the last.
+  // Places have landed a step after they were asked for, weights, which come from further away, a step and a half.  A slab is loaded
+  // again two sections or more after its last read; what a wave waits for is visible to the others behind the barrier.
+  // MODE 1, 2: the last step but one, the last.
   auto run = [&](auto HB_) {
     constexpr int HB = decltype(HB_)::value;
     bf16x8 fa[HB][2], fb[4][2];
     auto rows = [&](int st, int h) {
-      const char* s = lds + st * W_STAGE + abase + h * 8192;
+      const char* s = lds + st * W_TILE + abase + h * 8192;
 #pragma unroll
       for (int i = 0; i < HB; ++i) {
         fa[i][0] = *reinterpret_cast<const bf16x8*>(s + i * 2048 + p0);
@@ -760,29 +812,39 @@ __global__ __launch_bounds__(512) void moe_group_wide_kernel(GroupArgs g, int nt
           for (int j = 0; j < 4; ++j) acc[h][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j][k], fa[i][k], acc[h][i][j], 0, 0, 0);
       __builtin_amdgcn_s_setprio(0);
     };
+    int wst = 0;                                       // the weights' stage of this step
     auto step = [&](int s, auto ST_, auto MODE_) {
       constexpr int ST = decltype(ST_)::value, MODE = decltype(MODE_)::value;
-      if constexpr (MODE < 2) {
-        gb(s + 1, 0, ST ^ 1); gb(s + 1, 1, ST ^ 1); gb(s + 1, 2, ST ^ 1); gb(s + 1, 3, ST ^ 1);
-        ga(s + 1, 2, ST ^ 1);
+      if (wm) {
+        if constexpr (MODE < 2) { ga(s + 1, 1, ST ^ 1); ga(s + 1, 3, ST ^ 1); }
+      } else {
+        if constexpr (MODE == 0) gb(s + 2, wst == 0 ? 2 : wst - 1);
       }
-      const char* bs = lds + ST * W_STAGE + bbase;
+      const char* bs = lds + wst * W_TILE + bbase;
+      wst = wst == 2 ? 0 : wst + 1;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         fb[j][0] = *reinterpret_cast<const bf16x8*>(bs + j * 2048 + p0);
         fb[j][1] = *reinterpret_cast<const bf16x8*>(bs + j * 2048 + p1);
       }
       rows(ST, 0);
-      if constexpr (MODE < 2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (wm) {                                        // slabs 1, 3 of this step
+        if constexpr (MODE < 2) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
       barrier();
       mma(0);
       barrier();
-      if constexpr (MODE < 2) { ga(s + 1, 3, ST ^ 1); ga(s + 1, 1, ST ^ 1); }
-      if constexpr (MODE == 0) ga(s + 2, 0, ST);
+      if (wm) {
+        if constexpr (MODE == 0) { ga(s + 2, 0, ST); ga(s + 2, 2, ST); }
+      }
       rows(ST, 1);
-      if constexpr (MODE == 0) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-      else if constexpr (MODE == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+      // the weights of the next step, slabs 0, 2 of its places
+      if constexpr (MODE == 0) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      else if constexpr (MODE == 1) {
+        if (wm) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      }
       barrier();
       mma(1);
       barrier();
@@ -790,12 +852,15 @@ __global__ __launch_bounds__(512) void moe_group_wide_kernel(GroupArgs g, int nt
     using Z = std::integral_constant<int, 0>;
     using O = std::integral_constant<int, 1>;
     using L = std::integral_constant<int, 2>;
-    ga(0, 0, 0); gb(0, 0, 0); gb(0, 1, 0); gb(0, 2, 0); gb(0, 3, 0); ga(0, 2, 0);
-    ga(0, 3, 0); ga(0, 1, 0); ga(1, 0, 1);
-    asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
+    if (wm) {
+      ga(0, 0, 0); ga(0, 2, 0); ga(0, 1, 0); ga(0, 3, 0); ga(1, 0, 1); ga(1, 2, 1);
+    } else {
+      gb(0, 0);
+      gb(1, 1);
+    }
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
     barrier();
     if (wm == 1) barrier();                            // waves 4-7 run one section behind
-    const int steps = g.K >> 6;                        // even
     int s = 0;
     for (; s + 4 <= steps; s += 2) {
       step(s, Z{}, Z{});
@@ -856,11 +921,17 @@ int launch_group(GroupArgs g, int places, int rows_per_tile, hipStream_t s) {
   // worst split of the places over the experts: every non-empty expert may end in a partial tile
   const int nonempty = g.E < places ? g.E : places;
   int bm = rows_per_tile;
-  if (bm == WIDE) {
-    // 32-bit byte offsets into A and into an expert's weights, whole steps of 128 of K, 16-byte stores
+  if (bm == 128 || bm == WIDE) {
+    // The wide tiles need 32-bit byte offsets into A and into an expert's weights, whole steps of 128 of K and 16-byte stores.  Where they can, they
+    // are faster than tiles of 128 (128, 256: 16 experts of 2048 x 2048 mean 62 144 us, 117; 2048 x 4096 mean 75 256, 209; 4096 x 3584 mean 50 333, 293; 8 of
+    // 4096 x 14336 mean 50 681, 614; 64 of 2048 x 1408 mean 61 292, 263; 128 of 2048 x 768 mean 81 393, 310; 16 of 1024 x 1024 mean 50 57, 52), but for small ones of
+    // few steps (32 of 1024 x 512 mean 38 50, 52, mean 75 52, 51).  Up to 52 places an expert, which seldom are more than 64, streamed weights are faster
+    // still (64, 256: 2048 x 2048 mean 50 101, 117, mean 62 141, 117; 2048 x 4096 mean 50 203, 213; 1024 x 2048 mean 50 44, 65; but 1024 x 1024 54, 52).
     const long long a_bytes = 2ll * g.a_stride * (g.order ? (places + g.top - 1) / g.top : places);
     const long long b_bytes = 2ll * g.N * g.K * (GLU ? 2 : 1);
     if (g.K % 128 || g.N % 8 || ((uintptr_t)g.out & 15) || a_bytes >= 1ll << 31 || b_bytes >= 1ll << 31) bm = 128;
+    else if (bm == 128 && places <= 52ll * g.E && (long long)g.N * g.K > 1 << 20 && streams(64, g.K)) bm = 64;
+    else if ((long long)g.N * g.K > 1 << 19 || places > 64ll * g.E) bm = WIDE;
   }
   g.mtiles = places / bm + nonempty;
   const int no = (bm >= 128 ? bm : 64) / (GLU ? 2 : 1);
@@ -869,7 +940,7 @@ int launch_group(GroupArgs g, int places, int rows_per_tile, hipStream_t s) {
   if (blocks > 0x3fffffff) return -4;
   const int padded = (int)((blocks + 7) / 8 * 8);
   if (bm == WIDE) {
-    moe_group_wide_kernel<GLU><<<padded, 512, 0, s>>>(g, ntn);
+    moe_group_wide_kernel<GLU><<<padded + 8 * MORE, 512, 0, s>>>(g, ntn);
   } else if (bm == 128) {
     moe_group_tiles_kernel<GLU><<<padded, 256, 0, s>>>(g, ntn);
   } else if (streams(bm, g.K)) {

@@ -58,3 +58,34 @@ def test_wide_tiles(monkeypatch, W, ff, act, weigh):
     bound = 2.0 ** -8 * (2 * mag + y.abs()) + 1e-5 * (1 + mag)
     worst = ((got.cpu().to(F64) - y).abs() / bound).max().item()
     assert worst <= 1.0, worst
+
+
+def run(counts, W, ff, tile, monkeypatch):
+    E = len(counts)
+    g = torch.Generator().manual_seed(9)
+    idx = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    idx = idx[torch.randperm(idx.numel(), generator=g)].reshape(-1, 1).to(torch.int32)
+    h = draw(idx.shape[0], W, seed=1)
+    gu, dn = draw(E, 2 * ff, W, seed=2, scale=W ** -0.5), draw(E, W, ff, seed=3, scale=ff ** -0.5)
+    w = torch.rand(idx.shape[0], 1, generator=g)
+    monkeypatch.setattr(moe, "group_tile", lambda *a: tile)
+    got = moe.moe_experts(h.cuda(), idx.cuda(), w.cuda(), gu.cuda(), dn.cuda())
+    y, mag = exact(h, idx, w, gu, dn, "silu", 0.8, "output")
+    bound = 2.0 ** -8 * (2 * mag + y.abs()) + 1e-5 * (1 + mag)      # as above
+    assert ((got.cpu().to(F64) - y).abs() / bound).max().item() <= 1.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,W", [([200], 2048), ([256], 16384), ([130, 60], 9216), ([256], 32768), ([65], 34816), ([250], 67584), ([600, 1], 2304),
+                                      ([1], 256)], ids=str)
+def test_tiles_that_are_cut(monkeypatch, counts, W):
+    """1, 8, 9, 16, 17 and 1 more than 32 tiles an XCD in the down product, several of them of one expert, fewer than there are XCDs."""
+    run(counts, W, 128, 256, monkeypatch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,W,ff", [([50, 40, 66, 3], 2048, 1024), ([60, 64, 30, 53], 2048, 1024), ([30, 80], 1024, 512), ([70, 80], 1024, 512), ([100, 28], 136, 1024)],
+                         ids=str)
+def test_middling_experts(monkeypatch, counts, W, ff):
+    """Tiles of 128 asked for: streamed ones of 64, wide ones or those, as means and widths say."""
+    run(counts, W, ff, 128, monkeypatch)
