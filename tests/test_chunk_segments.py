@@ -103,6 +103,7 @@ def test_non_finite_values_stay_behind(mode):
             assert not torch.isfinite(got[171, 3])
 
 
+@torch.inference_mode()      # as models run, and other tests capture
 def test_captured_segments_replay():
     """The states between segments in a graph's memory: every replay gives the eager result, with eager steps between them."""
     d = make("gla", [1500], 6, 64, 64, torch.bfloat16)
