@@ -194,13 +194,13 @@ def split_runs(rows: int, heads: int, max_keys: int) -> int:
     return int(max(1, min(16, SPLIT_WAVES // (rows * heads), max_keys // 128)))
 
 
-def tile_runs(rows: int, heads: int, max_keys: int) -> int:
+def tile_runs(rows: int, heads: int, max_keys: int, least: int = 128) -> int:
     """Runs of keys per row for the tile kernel (512 + 64 dims): its workgroups take a row, up to 32 heads and one run, one
-    to a compute unit (its four tiles of 32 keys are nearly all of the LDS), so as many as fill the 256 of them, every run at least 128 keys
-    long.  32 rows of 32 heads over 2000 keys: 8 runs 29 us and 8 to combine them."""
+    to a compute unit (its four tiles of 32 keys are nearly all of the LDS), so as many as fill the 256 of them, every run at least ``least``
+    keys long.  32 rows of 32 heads over 2000 keys: 8 runs 29 us and 8 to combine them."""
     if max_keys <= 0 or rows <= 0:
         return 1
-    return int(max(1, min(64, 256 // (rows * ((heads + 31) // 32)), max_keys // 128)))
+    return int(max(1, min(64, 256 // (rows * ((heads + 31) // 32)), max_keys // least)))
 
 
 def latent_attn_rows(q: torch.Tensor, q_lat: torch.Tensor, cache: torch.Tensor, block_tables: torch.Tensor,
@@ -258,12 +258,13 @@ def latent_decode_heads(q, uk, uv, cache, block_tables, positions, rot_dim: int,
     """Head outputs ``out`` [T, H * vdim] of decode rows on cached latents (``decode_heads_ok``): ``q`` [T, H * (dim + rot_dim)], the key
     and value up-projections ``uk`` [H, dim, 512] and ``uv`` [H, vdim, 512], the rest as ``latent_attn_rows`` and ``gate_heads``.  Three
     launches: queries folded, attention in runs of keys, and one that combines the runs, takes the sums to values and applies
-    the gate.  32 rows of 32 heads, 8 runs: 4.5 and 10.5 us around the attention's 29; the library's products, the combining pass
-    and the one that puts the heads side by side took 28."""
+    the gate.  32 rows of 32 heads, 8 runs: 4.5 and 8.3 us around the attention's 29; the library's products, the combining pass
+    and the one that puts the heads side by side took 28.  Runs of 64 keys pay here, as combining them is no pass of its own (a layer, runs of
+    128, 64 and 32 keys: 3 rows of 16 heads over 612 20.4, 18.0, 17.9 us; 29 over 136 23.4, 20.5, 21.2; 24 of 32 heads over 34 18.8, 19.0, 22.1)."""
     _native(q)
     T, (H, dim, kr) = q.shape[0], uk.shape
     q_lat, o_lat = (torch.empty(H, T, kr, dtype=q.dtype, device=q.device) for _ in range(2))
-    runs = tile_runs(T, H, min(max_keys, window) if window > 0 and max_keys > 0 else max_keys)
+    runs = tile_runs(T, H, min(max_keys, window) if window > 0 and max_keys > 0 else max_keys, 64)
     po = pm = None
     if runs > 1:
         po = torch.empty(runs * H * T * kr, dtype=torch.float32, device=q.device)

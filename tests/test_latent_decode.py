@@ -99,6 +99,13 @@ def test_decode_heads_many_runs(T, max_keys):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,vdim", [(1, 128), (2, 80), (3, 128), (5, 64), (6, 96), (11, 128)])
+def test_decode_heads_rows_that_share_threads(T, vdim):
+    """Values: one row, two and four at a time, whose threads share its runs, in fewer and more than a batch; a workgroup's value dims from 16 to all."""
+    compare(T, 20, 64, vdim, "element", keys=(128, 1 << 10, 1 << 12))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [5, 100])
 @pytest.mark.parametrize("window,dims,inter,gated", [(0, 64, True, None), (100, 64, False, "head"), (70, 32, True, "element"), (33, 0, True, None)])
 def test_layer_with_windows_and_rotation(T, window, dims, inter, gated):
