@@ -89,3 +89,23 @@ def test_tiles_that_are_cut(monkeypatch, counts, W):
 def test_middling_experts(monkeypatch, counts, W, ff):
     """Tiles of 128 asked for: streamed ones of 64, wide ones or those, as means and widths say."""
     run(counts, W, ff, 128, monkeypatch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,K", [(1, 16, 2, 4096), (17, 16, 16, 2048), (33, 9, 4, 6144), (5, 32, 3, 4160), (20, 64, 5, 2080), (2, 40, 2, 12288)])
+def test_router_widths(T, E, top, K):
+    """Routes of widths whose steps a wave takes eight, four or two at a time, some past the end: scores against 64 bits; rows of equal scores
+    take the lowest experts; a row that is not a number gets experts that there are, each once."""
+    from dgi.ops import moe
+    g = torch.Generator().manual_seed(K + T)
+    h = torch.randn(T + 2, K, generator=g).to(torch.bfloat16)
+    h[T], h[T + 1] = 0.0, float("nan")
+    router = (torch.randn(E, K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    idx, w = moe.moe_router(h.cuda(), router.float().cuda(), router.cuda(), top, False, 1.0)
+    idx, w = idx.cpu().long(), w.cpu()
+    score = torch.sigmoid(h.double() @ router.double().t())
+    best = torch.sort(score[:T], 1, descending=True).values[:, :top]
+    # fp32 sums of K products of about K ** -0.5 each: 1e-5 of a logit leaves room for every order
+    assert ((w[:T] - best).abs() < 1e-5).all() and ((score[:T].gather(1, idx[:T]) - best).abs() < 1e-5).all()
+    assert idx[T].tolist() == list(range(top)) and (w[T] == 0.5).all()
+    assert all(len(set(r)) == top and 0 <= min(r) and max(r) < E for r in idx.tolist())
