@@ -66,9 +66,6 @@ __device__ __forceinline__ void each(F f) {
 
 constexpr int KT = 64;  // keys per tile
 
-// 1 / scale from scale * log2(e)
-__device__ __forceinline__ float inv_scale_cap(float scale_log2) { return 1.4426950408889634f / scale_log2; }
-
 // NW waves x 32 query rows per workgroup (one K/V tile staging shared by all of them):
 // NW = 4 -> 128-row tiles, 2 workgroups per CU; NW = 8 -> 256-row tiles, 1 per CU
 // (same 2 waves per SIMD, half the K/V staging per query row).
@@ -104,12 +101,13 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   const int kvh = hx % nkv;
   const int head = kvh * (nh / nkv) + hx / nkv;
   // per-head score factor: folded into the scale; the softmax below takes maxima of raw scores, so a negative
-  // factor flips the raw scores' sign, and a factor of zero stays above it (masked keys are -inf)
+  // factor flips the raw scores' sign (the query's, and what is added to them), and a factor of zero stays above it (masked keys are -inf)
   bool flip = false;
   if (MASKED && head_scale) {
     scale_log2 *= head_scale[head];
     flip = scale_log2 < 0.f;
     scale_log2 = fmaxf(fabsf(scale_log2), 1e-30f);
+    if (flip) inv_scale = -inv_scale;
   }
   const int q0 = cu_seqlens_q[b];
   const int qlen = cu_seqlens_q[b + 1] - q0;
@@ -149,6 +147,10 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     // the next tile's loads issued a few instructions earlier: one full HBM round trip
     // per tile and no load/compute overlap at all.
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), expcnt / lgkmcnt untouched (gfx9 encoding)
+    if (MASKED && flip) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) qf[s] ^= 0x80008000u;
+    }
   }
 
   const int last_row = min(t0 + 32 * NW, qlen) - 1;
@@ -163,6 +165,9 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   const int kv_begin = MASKED ? (first_key(pos_base + t0) / KT) * KT : 0;
   const int my_first = first_key(my_pos);
 
+  // what the softmax multiplies the scores that it gets by
+  const float cap_log2 = MASKED && softcap > 0.f ? softcap * 1.4426950408889634f : 0.f;
+  const float soft_scale = MASKED && softcap > 0.f ? 2.f * cap_log2 : scale_log2;
   float m_run = -1e30f, l_run = 0.f;
   f32x16 o[ND];
 #pragma unroll
@@ -353,24 +358,15 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
           }
       }
     }
-    if (MASKED && flip) {
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sc[kb][r] = -sc[kb][r];
-    }
     if (MASKED && softcap > 0.f) {
-      // soft cap in natural score units, back to raw q.k units (the softmax below scales again):
-      // tanh(x) = 1 - 2 / (exp(2x) + 1) with the hardware exp2 / rcp
+      // soft cap of the scaled score: tanh(x) = 1 - 2 / (exp(2x) + 1) with the hardware exp2 / rcp.  What the softmax takes is -1 / (exp(2x) + 1) by
+      // twice the cap (soft_scale): the capped scores less the cap, which it does not see (that step with a cap 192 us, so 160; a polynomial for
+      // scores well below the cap took as long as exp and rcp: the multiplies and adds between them are what counts).
       const float to_arg = scale_log2 * 2.f / softcap;             // raw -> 2 x log2(e)
-      const float back = softcap * inv_scale_cap(scale_log2);
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float e = __builtin_amdgcn_exp2f(sc[kb][r] * to_arg);
-          sc[kb][r] = back * (1.f - 2.f * __builtin_amdgcn_rcpf(e + 1.f));
-        }
+        for (int r = 0; r < 16; ++r) sc[kb][r] = __builtin_amdgcn_rcpf(-1.f - __builtin_amdgcn_exp2f(sc[kb][r] * to_arg));
     }
     // ---- online softmax; lane owns query lr, keys kb0 + 32kb + (r&3) + 8(r>>2) + 4hh.
     // Interior tiles (every key visible to every row of this wave, no tree rows) skip the mask.
@@ -401,7 +397,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[kb][r]);
-    mx *= scale_log2;
+    mx *= soft_scale;
     // deferred max: rescale O / l only when the running max grows by > 2^8, so
     // most tiles skip the 64 O multiplies (P stays <= 256, safe in f32 / bf16) and the exchange with the half of the wave
     // that holds the query's other keys
@@ -420,7 +416,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     float ps[4];
     u32x4 pf;
     auto weight = [&](int kb, int r) __attribute__((always_inline)) {
-      sc[kb][r] = __builtin_amdgcn_exp2f(sc[kb][r] * scale_log2 - m_run);
+      sc[kb][r] = __builtin_amdgcn_exp2f(sc[kb][r] * soft_scale - m_run);
       ps[r & 3] = kb == 0 && r < 4 ? sc[kb][r] : ps[r & 3] + sc[kb][r];
     };
 #pragma unroll
@@ -448,10 +444,25 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
     step(kb0, ic<0>{});
     if (kb0 + KT < kv_end) step(kb0 + KT, ic<1>{});
   }
+  // The gates of a row's elements are all asked for at once; exp and quotient are the hardware's, as the weights' (64 heads of 128 dims, 7 prompts
+  // of 3637 rows in all behind 500 tokens each, blocks of 1024 163 us, so 140; without a gate 124).
+  const bool gated = MASKED && gate && !gate_heads;
+  uint2 gates[ND][4];
+  if (gated) {
+    const uint16_t* gp = gate + (size_t)(q0 + (row_valid ? my_row : 0)) * gate_stride + head * dv;
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const int dim = 32 * d + 8 * rr + 4 * hh;
+        gates[d][rr] = *reinterpret_cast<const uint2*>(gp + (PAD ? min(dim, dv - 4) : dim));
+      }
+  }
   l_run += __shfl_xor(l_run, 32, 64);
 
   if (!row_valid) return;
-  if (MASKED && sinks) l_run += __builtin_amdgcn_exp2f(sinks[head] * 1.4426950408889634f - m_run);   // sink: denominator only
+  // sink: denominator only (m_run lacks the cap)
+  if (MASKED && sinks) l_run += __builtin_amdgcn_exp2f(sinks[head] * 1.4426950408889634f - (m_run + cap_log2));
   float inv = l_run > 0.f ? 1.f / l_run : 0.f;
   if (MASKED && gate && gate_heads) inv *= 1.f / (1.f + expf(-bf16_to_f32(gate[(size_t)(q0 + my_row) * gate_stride + head])));
   uint16_t* op = out + (size_t)(q0 + my_row) * out_stride + head * dv;
@@ -462,12 +473,12 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
       const int dim = 32 * d + 8 * rr + 4 * hh;
       if (PAD && dim >= dv) continue;
       float ov[4] = {o[d][4 * rr] * inv, o[d][4 * rr + 1] * inv, o[d][4 * rr + 2] * inv, o[d][4 * rr + 3] * inv};
-      if (MASKED && gate && !gate_heads) {
-        const uint2 g = *reinterpret_cast<const uint2*>(gate + (size_t)(q0 + my_row) * gate_stride + head * dv + dim);
+      if (gated) {
+        const uint2 g = gates[d][rr];
         const float gf[4] = {__uint_as_float(g.x << 16), __uint_as_float(g.x & 0xffff0000u),
                              __uint_as_float(g.y << 16), __uint_as_float(g.y & 0xffff0000u)};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) ov[j] *= 1.f / (1.f + expf(-gf[j]));
+        for (int j = 0; j < 4; ++j) ov[j] *= __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(gf[j] * -1.4426950408889634f));
       }
       uint2 v;
       v.x = pack_bf16x2(ov[0], ov[1]);

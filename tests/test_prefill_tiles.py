@@ -139,3 +139,31 @@ def test_caches_off_sixteen_bytes(form):
         x.copy_(case[i])
         case[i] = x
     assert torch.equal(call(case), want)
+
+
+@pytest.mark.parametrize("D", [64, 80, 128])
+@pytest.mark.parametrize("cap,scale", [(0.0, 0.1), (0.5, 1.0), (30.0, 0.1), (1e4, 0.1)])
+def test_caps_factors_and_gates(D, cap, scale):
+    """Caps far below the scores, about them and far above, heads with factors below, at and above zero, sinks on both sides of the capped
+    scores, gates from shut to open; rows behind a prefix and a last tile that ends early."""
+    g = torch.Generator().manual_seed(D)
+    H, G, lens, pre, bs = 6, 2, [150, 37], 70, 16
+    cu, ctx = [0, 150, 187], [x + pre for x in lens]
+    width = -(-max(ctx) // bs)
+    table = (torch.randperm(2 * width, generator=g) + 1).view(2, width).int()
+    k, v = (torch.randn(2 * width + 1, G, bs, D, generator=g).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(187, H * D, generator=g).to(torch.bfloat16)
+    gate = (40.0 * torch.randn(187, H * D, generator=g)).to(torch.bfloat16)
+    sinks, factor = torch.linspace(-6, 9, H), torch.tensor([-1.5, -0.2, 0.0, 0.3, 1.0, 2.0])
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
+
+    def run(dev, dt):
+        to = lambda x: x.to(dev, dt)  # noqa: E731
+        return mix.paged_prefill_masked(to(q), to(k), to(v), table.to(dev), i32(cu).to(dev), i32(ctx).to(dev), H, G, scale, 100, to(gate),
+                                        softcap=cap, sinks=sinks.to(dev), head_scale=factor.to(dev)).float().cpu()
+
+    got, want = run("cuda", torch.bfloat16), run("cpu", torch.float32)
+    # each weight is rounded to bf16 once, as is the result; a cap adds the rounding of its quotient near 1/2, times twice the cap
+    open_ = torch.sigmoid(gate.float())
+    slack = open_ * v.float().abs().max() * (2.0 ** -8 + 2 * cap * 2.0 ** -23) + 2.0 ** -8 * want.abs() + 1e-6
+    assert torch.isfinite(got).all() and ((got - want).abs() <= slack).all(), ((got - want).abs() / slack).max()
