@@ -17,7 +17,9 @@ using namespace dgi;
 namespace {
 
 // A workgroup owns a head and 64 latent dims, wave w 16 of them; its slab of uk lies in LDS and is read transposed (the
-// product's A operand: latent dims by query dims).  DS = dim / 32 steps; rows sixteen at a time.
+// product's A operand: latent dims by query dims).  DS = dim / 32 steps; FOLD rows, sixteen at a time (128 rows of 16
+// heads one behind the other 5.7 us, so 4.5).
+constexpr int FOLD = 32;
 template <int DS>
 __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__ q_lat, const uint16_t* __restrict__ q, int q_stride,
                                                           const uint16_t* __restrict__ uk, int T, int qk, int kr) {
@@ -38,8 +40,9 @@ __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__
 #pragma unroll
     for (int s = 0; s < DS; ++s) b[s] = *reinterpret_cast<const u32x4*>(p + 32 * s);
   };
+  const int from = blockIdx.z * FOLD, to = min(T, from + FOLD);
   u32x4 b[DS];
-  load_q(0, b);
+  load_q(from, b);
 #pragma unroll
   for (int i = 0; i < DS; ++i) *reinterpret_cast<u32x4*>(slab + (threadIdx.x + 256 * i) * 8) = v[i];
   __syncthreads();
@@ -55,12 +58,12 @@ __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__
     a[s][2] = (uint32_t)(uint16_t)hi[0] | ((uint32_t)(uint16_t)hi[1] << 16);
     a[s][3] = (uint32_t)(uint16_t)hi[2] | ((uint32_t)(uint16_t)hi[3] << 16);
   }
-  for (int t0 = 0; t0 < T; t0 += 16) {
+  for (int t0 = from; t0 < to; t0 += 16) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < DS; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a[s]), as_bf16x8(b[s]), acc, 0, 0, 0);
-    if (t0 + 16 < T) load_q(t0 + 16, b);
-    if (t0 + lr < T)
+    if (t0 + 16 < to) load_q(t0 + 16, b);
+    if (t0 + lr < to)
       *reinterpret_cast<uint2*>(q_lat + ((size_t)head * T + t0 + lr) * kr + c0 + 16 * w + 4 * lg) =
           make_uint2(pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]));
   }
@@ -128,17 +131,25 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
     for (; r < rb; r += apart) {
       const float m = lane < runs ? e.x : -__builtin_inff();
       float M = fmaxf(m, -FLT_MAX);                        // finite also where no run has keys
+      // few runs: the lanes that have them; a loop of more turns costs what it saves
+      auto turns = [&](auto f) {
+        if (runs > 8) {
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+          for (int o = 1; o < 64; o <<= 1) f(o);
+        } else {
+          for (int o = 1; o < runs; o <<= 1) f(o);
+        }
+      };
+      turns([&](int o) { M = fmaxf(M, __shfl_xor(M, o, 64)); });
       const float f = expf(m - M);
       float L = lane < runs ? e.y * f : 0.f;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o, 64);
+      turns([&](int o) { L += __shfl_xor(L, o, 64); });
       float inv = L == 0.f ? 0.f : 1.f / L;
       if (sinks) {                                         // one more logit in the denominator, relative to the larger of the two
         const float sink = sinks[head], top = fmaxf(M, sink), g = expf(M - top);
         inv = g / (L * g + expf(sink - top));
       }
+      inv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv), 0));
       const bool more = r + apart < rb;
       if (more) e = load_ml(r + apart);
       float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -203,7 +214,8 @@ extern "C" int dgi_latent_fold(void* q_lat, const void* q, int q_stride, const v
   if (H <= 0 || dim % 32 || dim < 32 || dim > 128 || kr % 64 || qk % 8 || q_stride % 8 || (((uintptr_t)q | (uintptr_t)uk) & 15) ||
       ((uintptr_t)q_lat & 7))
     return -2;
-  const dim3 grid(H, kr / 64);
+  if ((T + FOLD - 1) / FOLD > 65535) return -4;
+  const dim3 grid(H, kr / 64, (T + FOLD - 1) / FOLD);
 #define DGI_LF(N_)                                                                                                             \
   latent_fold_kernel<N_><<<grid, 256, 0, s>>>((uint16_t*)q_lat, (const uint16_t*)q, q_stride, (const uint16_t*)uk, T, qk, kr)
   switch (dim / 32) {

@@ -260,11 +260,12 @@ def latent_decode_heads(q, uk, uv, cache, block_tables, positions, rot_dim: int,
     launches: queries folded, attention in runs of keys, and one that combines the runs, takes the sums to values and applies
     the gate.  32 rows of 32 heads, 8 runs: 4.5 and 8.3 us around the attention's 29; the library's products, the combining pass
     and the one that puts the heads side by side took 28.  Runs of 64 keys pay here, as combining them is no pass of its own (a layer, runs of
-    128, 64 and 32 keys: 3 rows of 16 heads over 612 20.4, 18.0, 17.9 us; 29 over 136 23.4, 20.5, 21.2; 24 of 32 heads over 34 18.8, 19.0, 22.1)."""
+    128, 64 and 32 keys: 3 rows of 16 heads over 612 20.4, 18.0, 17.9 us; 29 over 136 23.4, 20.5, 21.2), but not two runs instead of one (70 rows of 16 heads over 60, tables of 144: 24.2, in one run 20.9; 128 26.9, 22.1)."""
     _native(q)
     T, (H, dim, kr) = q.shape[0], uk.shape
     q_lat, o_lat = (torch.empty(H, T, kr, dtype=q.dtype, device=q.device) for _ in range(2))
-    runs = tile_runs(T, H, min(max_keys, window) if window > 0 and max_keys > 0 else max_keys, 64)
+    bound = min(max_keys, window) if window > 0 and max_keys > 0 else max_keys
+    runs = tile_runs(T, H, bound, 64) if bound >= 192 else 1
     po = pm = None
     if runs > 1:
         po = torch.empty(runs * H * T * kr, dtype=torch.float32, device=q.device)
