@@ -743,6 +743,69 @@ __global__ __launch_bounds__(128) void masked_attn_reduce_kernel(const float* __
   }
 }
 
+// The same for four runs and more.  It is a launch and a chain of latencies: lane z holds run z's factor, eight runs' sums are under way at a time, the first
+// eight while the factors are formed.  Four layers of one row of 16 heads of 128 dims, 8000 keys in 16 runs, 94 us with the one above, so 69; 6 runs 75, 68; 4 runs 135, 132;
+// but 3 runs 92.6, 92.2 and 2 59.4, 63.1.
+constexpr int MANY_RUNS = 4;
+template <typename T>
+__global__ __launch_bounds__(128) void masked_attn_reduce_many_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                                 int nsplit, int dv, const float* __restrict__ sinks,
+                                                                 const T* __restrict__ gate, int gate_stride, int gate_heads,
+                                                                 T* __restrict__ out, int out_stride) {
+  constexpr int BATCH = 8;
+  const int row = blockIdx.x, head = blockIdx.y, rows = gridDim.x, H = gridDim.y, lane = threadIdx.x & 63;
+  auto slot = [&](int z) { return ((size_t)min(z, nsplit - 1) * rows + row) * H + head; };
+  auto own = [&](int z0) {                             // maximum and sum of run z0 + lane
+    const float2 e = *reinterpret_cast<const float2*>(part_ml + 2 * slot(z0 + lane));
+    return z0 + lane < nsplit ? e : make_float2(-__builtin_inff(), 0.f);
+  };
+  float p[BATCH];
+  auto load = [&](int d, int z0) {
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) p[i] = part_o[slot(z0 + i) * dv + min(d, dv - 1)];
+  };
+  const float2 e0 = own(0);
+  load(threadIdx.x, 0);
+  float M = e0.x;                                      // run 0 is never empty
+  for (int z0 = 64; z0 < nsplit; z0 += 64) M = fmaxf(M, own(z0).x);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+  if (sinks) M = fmaxf(sinks[head], M);
+  auto factor = [&](const float2& e) { return expf(e.x - M); };      // no run: exp(-inf) = 0
+  float L = e0.y * factor(e0);
+  for (int z0 = 64; z0 < nsplit; z0 += 64) {
+    const float2 e = own(z0);
+    L += e.y * factor(e);
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) L += __shfl_xor(L, o, 64);
+  if (sinks) L += expf(sinks[head] - M);
+  const float inv = 1.f / L;
+  for (int d0 = 0; d0 < dv; d0 += 128) {
+    const int d = d0 + threadIdx.x;
+    if (d0 > 0) load(d, 0);
+    float O = 0.f, f = 0.f;
+    for (int z0 = 0; z0 < nsplit; z0 += BATCH) {
+      if ((z0 & 63) == 0) f = factor(z0 == 0 ? e0 : own(z0));
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i)
+        if (z0 + i < nsplit) O += p[i] * __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), (z0 + i) & 63));
+      if (z0 + BATCH < nsplit) load(d, z0 + BATCH);
+    }
+    if (d >= dv) continue;
+    float v = O * inv;
+    if (gate) v *= 1.f / (1.f + expf(-ldf<T>(gate + (size_t)row * gate_stride + (gate_heads ? (size_t)head : (size_t)head * dv + d))));
+    stf<T>(out + (size_t)row * out_stride + (size_t)head * dv + d, v);
+  }
+}
+
+template <typename T>
+void launch_reduce(const float* part_o, const float* part_ml, int rows, int H, int nsplit, int dv, const float* sinks, const void* gate, int gate_stride,
+                   int gate_heads, void* out, int out_stride, hipStream_t s) {
+  auto kernel = nsplit >= MANY_RUNS ? masked_attn_reduce_many_kernel<T> : masked_attn_reduce_kernel<T>;
+  kernel<<<dim3(rows, H), 128, 0, s>>>(part_o, part_ml, nsplit, dv, sinks, (const T*)gate, gate_stride, gate_heads, (T*)out, out_stride);
+}
+
 template <int R, int D>
 void launch_tiles_dims(const RowsArgs& a, int rows, int G, int nsplit, hipStream_t s) {
   // A workgroup per compute unit or fewer: eight waves each (30 rows of 2000 keys, 8 groups of 4 heads of 64 dims: 14.9 us, with four
@@ -772,8 +835,7 @@ void launch_tiles(RowsArgs a, int rows, int G, int nsplit, hipStream_t s) {
   else if (r <= 4) launch_tiles_heads<4>(a, rows, G, nsplit, s);
   else launch_tiles_heads<8>(a, rows, G, nsplit, s);
   if (nsplit > 1)
-    masked_attn_reduce_kernel<uint16_t><<<dim3(rows, a.H), 128, 0, s>>>(a.part_o, a.part_ml, nsplit, a.dv, a.sinks, a.gate, a.gate_stride,
-                                                                        a.gate_heads, a.out, a.out_stride);
+    launch_reduce<uint16_t>(a.part_o, a.part_ml, rows, a.H, nsplit, a.dv, a.sinks, a.gate, a.gate_stride, a.gate_heads, a.out, a.out_stride, s);
 }
 
 template <typename T, int R, int VP>
@@ -790,8 +852,7 @@ int launch_group(const void* q, int q_stride, const void* k_cache, const void* v
       positions, H, dk, dv, bs, scale, mask, (const T*)gate, gate_stride, (T*)out, out_stride, dist_bias, n_dist,
       softcap, sinks, head_scale, gate_heads, part_o, part_ml);
   if (nsplit > 1)
-    masked_attn_reduce_kernel<T><<<dim3(rows, H), 128, 0, s>>>(part_o, part_ml, nsplit, dv, sinks, (const T*)gate, gate_stride,
-                                                               gate_heads, (T*)out, out_stride);
+    launch_reduce<T>(part_o, part_ml, rows, H, nsplit, dv, sinks, gate, gate_stride, gate_heads, out, out_stride, s);
   return 0;
 }
 

@@ -106,3 +106,13 @@ def test_workgroups_around_the_lines_of_the_launch(rows):
     ctx = [1 + (53 * i) % 260 for i in range(rows)]
     q, kc, vc, table, pos, gate = case(ctx, 8, 2, 64, 64, 16, rows)
     check(q, kc, vc, table, pos, 8, 2, 0, gate)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("runs", [2, 8, 9, 31, 64, 65, 130])
+@pytest.mark.parametrize("H,G,dk,dv", [(4, 2, 64, 64), (4, 1, 128, 120), (2, 2, 96, 136)])
+def test_numbers_of_runs(H, G, dk, dv, runs):
+    """Runs around a batch of eight and a wave of 64, most of them without keys; values of one round of threads and of two."""
+    q, kc, vc, table, pos, gate = case([1, 70, 700, 2900], H, G, dk, dv, 16, runs)
+    check(q, kc, vc, table, pos, H, G, runs=runs)
+    check(q, kc, vc, table, pos, H, G, 0, gate, runs=runs, softcap=20.0, sinks=torch.linspace(-2.0, 3.0, H))
