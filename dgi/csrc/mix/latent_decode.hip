@@ -77,8 +77,8 @@ __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__
 // others of the row's runs, and those sums meet in LDS.  Lane z holds run z's factor, so that nobody waits for another wave's.  The rows then go
 // through LDS to the product, whose waves take sixteen value dims each over 512 / KP latent dims.  The weights, the gate and the first runs are
 // under way while the factors are formed.  Before, a wave had 64 latent dims of all value dims, lanes without a row of their own read another's again, and
-// few rows a workgroup meant all of uv for each: us then and now, rows x heads x runs: 32 x 32 x 8 10.7, 8.3; 3 x 16 x 6 8.6, 4.7; 8 x 16 x 32 10.7, 6.4;
-// 11 x 32 x 23 18.8, 9.1; 44 x 16 x 5 16.6, 7.0; without runs 24 x 32 10.4, 4.1; 2 x 32 5.6, 4.0.
+// few rows a workgroup meant all of uv for each: us then and now, rows x heads x runs: 32 x 32 x 8 10.7, 8.0; 3 x 16 x 6 8.6, 4.7; 8 x 16 x 32 10.7, 6.4;
+// 11 x 32 x 23 18.8, 9.3; 44 x 16 x 5 16.6, 7.1; without runs 24 x 32 10.4, 4.1; 2 x 32 5.6, 4.0.
 constexpr int KR = 512, RUNS = 64, BATCH = 8;
 
 template <int KP>

@@ -258,7 +258,7 @@ def latent_decode_heads(q, uk, uv, cache, block_tables, positions, rot_dim: int,
     """Head outputs ``out`` [T, H * vdim] of decode rows on cached latents (``decode_heads_ok``): ``q`` [T, H * (dim + rot_dim)], the key
     and value up-projections ``uk`` [H, dim, 512] and ``uv`` [H, vdim, 512], the rest as ``latent_attn_rows`` and ``gate_heads``.  Three
     launches: queries folded, attention in runs of keys, and one that combines the runs, takes the sums to values and applies
-    the gate.  32 rows of 32 heads, 8 runs: 4.5 and 8.3 us around the attention's 29; the library's products, the combining pass
+    the gate.  32 rows of 32 heads, 8 runs: 4.4 and 8.0 us around the attention's 29; the library's products, the combining pass
     and the one that puts the heads side by side took 28.  Runs of 64 keys pay here, as combining them is no pass of its own (a layer, runs of
     128, 64 and 32 keys: 3 rows of 16 heads over 612 20.4, 18.0, 17.9 us; 29 over 136 23.4, 20.5, 21.2), but not two runs instead of one (70 rows of 16 heads over 60, tables of 144: 24.2, in one run 20.9; 128 26.9, 22.1)."""
     _native(q)
