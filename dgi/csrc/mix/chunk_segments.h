@@ -147,14 +147,14 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, NB, ONLY>::WAVES), (Lay<MOD
   constexpr int DP = L::DP, NT = L::NT, PQ = L::PQ, PU = L::PU, GC = L::GC;
   extern __shared__ __attribute__((aligned(16))) char sm[];
   Segment at;
-  const int index = blockIdx.y;
   if (!a.ws) {                                                 // all portions whole
-    at = {index, 0, 1, 0};
-    at.each = a.seq_row0[index + 1] - a.seq_row0[index];
+    at = {(int)blockIdx.y, 0, 1, 0, 0};
+    at.each = a.seq_row0[at.seq + 1] - a.seq_row0[at.seq];
     if (at.each <= a.skip_rows) return;
-  } else if (!find_segment(a.seq_row0, a.n_seq, a.skip_rows, a.seg_rows, a.share, C, index, at)) {
+  } else if (!find_segment(a.seq_row0, a.n_seq, a.skip_rows, a.seg_rows, a.share, C, blockIdx.y, reinterpret_cast<int*>(sm), at)) {
     return;
   }
+  const int index = at.place;
   const int seq = at.seq, seg = at.seg, segs = at.segs;
   if (ONLY && seg + 1 == segs) return;
   const int H = a.H, dk = a.dk, dv = a.dv;

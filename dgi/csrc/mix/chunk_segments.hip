@@ -18,6 +18,9 @@ static long state_floats(int mode, int dk, int dv) {
 }
 static long decay_floats(int mode, int dk) { return mode == GLA ? dk : 4; }
 
+// places in the workspace of all cut portions (segments_of): at most 1.2 times what the chip has at once, so 20 MB in all
+static long long places(long rows, long each) { return 6ll * rows / (5 * each); }
+
 // workgroups of a portion over those the chip has at once: a compute unit has two of eight waves, one of more
 float dgi_chunk_segments_share(int mode, int dk, int dv, int H) {
   return (float)H * dgi_chunk_segments_groups(mode, dv) / (dk <= 64 && dv <= 64 && mode != MLSTM ? 512.f : 256.f);
@@ -55,22 +58,20 @@ int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows
   if (!here) return 0;
   // segments that fill the chip once
   const float share = dgi_chunk_segments_share(mode, dk, dv, H);
-  const long each = (std::max({96l, (long)(rows * share), (rows + 15l) / 16}) + C - 1) / C * C;
-  const long most = rows / each + n_seq;
-  const long long f = (long long)most * H * (state_floats(mode, dk, dv) + decay_floats(mode, dk));
-  if (over < (!many ? 1 : n_seq > 16 ? 768 : 1000) || whole(over + 1, rows, share, each) || most > 65535 || f > 1ll << 27) return 1 << 29;
-  *floats = f;
+  const long each = (std::max({96l, (long)(rows * share), std::min(128l, rows / 16l)}) + C - 1) / C * C;
+  if (over < (!many ? 1 : n_seq > 16 ? 768 : 1000) || whole(over + 1, rows, share, each) || !places(rows, each)) return 1 << 29;
+  *floats = places(rows, each) * H * (state_floats(mode, dk, dv) + decay_floats(mode, dk));
   return (int)each;
 }
 
 // a.seg_rows and ws as the plan says
 int dgi_chunk_segments(ChunkArgs a, int mode, int in_f32, int rows, float* ws, hipStream_t st) {
   const int groups = dgi_chunk_segments_groups(mode, a.dv);
-  const long most = ws ? rows / a.seg_rows + a.n_seq : a.n_seq;
+  const long most = ws ? rows / a.seg_rows + std::min(a.n_seq, rows / (a.skip_rows + 1)) : a.n_seq;
   a.blocks = groups * wide(mode, a.dv) + (mode == MLSTM ? 1 : 0);
   a.share = dgi_chunk_segments_share(mode, a.dk, a.dv, a.H);
   a.wsd = ws;
-  a.ws = ws ? ws + most * a.H * decay_floats(mode, a.dk) : nullptr;
+  a.ws = ws ? ws + places(rows, a.seg_rows) * a.H * decay_floats(mode, a.dk) : nullptr;
   if (most > 65535 || (long)a.H * groups > 0x3fffffff) return -3;
   const dim3 grid(a.H * groups, (unsigned)most);
   for (int only = ws ? 1 : 0; only >= 0; --only) {

@@ -13,6 +13,7 @@ F64 = torch.float64
 pytestmark = pytest.mark.gpu
 EDGES = [63, 64, 65, 33, 31, 0, 1, 97, 300]
 MIXED = [1] * 40 + [700] + [2] * 30 + [150, 17]
+MANY = [1] * 500 + [700] + [2] * 30 + [1900, 17] + [1] * 600 + [300, 40, 0]      # more sequences than a workgroup has threads
 
 
 def make(mode, lens, H, D, V, dtype, strong=False):
@@ -69,7 +70,7 @@ def oracle(d):
 @pytest.mark.parametrize("lens,H,D,V,dtype", [
     (EDGES, 32, 64, 64, torch.bfloat16), (EDGES, 32, 48, 40, torch.float32), (EDGES, 16, 100, 128, torch.bfloat16), (EDGES, 16, 128, 72, torch.float32),
     ([1500], 6, 64, 64, torch.bfloat16), ([850, 1900], 3, 64, 100, torch.float32), ([1300, 40], 5, 128, 128, torch.bfloat16), ([1700], 4, 128, 48, torch.float32),
-    (MIXED, 8, 64, 64, torch.bfloat16), (MIXED, 4, 64, 128, torch.float32)], ids=lambda x: "x".join(map(str, x))[:12] if isinstance(x, list) else str(x))
+    (MIXED, 8, 64, 64, torch.bfloat16), (MIXED, 4, 64, 128, torch.float32), (MANY, 4, 48, 64, torch.bfloat16)], ids=lambda x: "x".join(map(str, x))[:12] if isinstance(x, list) else str(x))
 def test_portions(mode, lens, H, D, V, dtype):
     d = make(mode, lens, H, D, V, dtype)
     got, want = call(d), oracle(d)
