@@ -4,6 +4,7 @@
 #include "segments.h"
 
 constexpr int GLA = 3;
+constexpr int APART_FROM = 8;        // as linear_scan.hip's
 int dgi_segments_mlstm(const ChunkArgs& a, int in_f32, bool only, dim3 grid, hipStream_t st);
 int dgi_segments_light(const ChunkArgs& a, int in_f32, bool only, dim3 grid, hipStream_t st);
 int dgi_segments_gla(const ChunkArgs& a, int in_f32, bool only, dim3 grid, hipStream_t st);
@@ -26,40 +27,56 @@ float dgi_chunk_segments_share(int mode, int dk, int dv, int H) {
   return (float)H * dgi_chunk_segments_groups(mode, dv) / (dk <= 64 && dv <= 64 && mode != MLSTM ? 512.f : 256.f);
 }
 
-// How a step of `rows` rows in n_seq portions goes: 0 not here but by the kernels of few tokens or of a pipeline for 16 or 32 columns (chunk_scan_decay.hip,
-// chunk_parts.hip), else about how many rows a segment has; *floats of workspace (0: all portions whole).
+// How a step of `rows` rows in n_seq portions goes: 0 not here but by the kernels of few tokens or of a pipeline for 16 or 32 columns
+// (chunk_scan_decay.hip, chunk_parts.hip, mlstm's token loop), else about how many rows a segment has; *floats of workspace (0: all portions whole).
 //
 // A workgroup here takes all columns of a head, so it repeats nothing, but goes 2.0 us a chunk of 32 tokens (mlstm 2.4) and 7 us before the first; the others
-// repeat what columns share, but have it sooner.  So
-// - many portions and heads go here (us there, here; 64 channels; heads, portions x rows: gla 64, 3 x 40 13.1, 10.9; 64, 16 x 70 83, 33; 64, 8 x 250 117, 39; 16, 16 x 20 12.3,
-//   9.0, but 16, 8 x 20 7.6, 8.4; light 64, 3 x 70 17.4, 12.8; 64, 8 x 250 68, 40; but 16, 8 x 120 14.4, 16.8; mlstm fp32 64, 3 x 300 54, 39; 128 channels: gla 64, 8 x 70 130, 53;
-//   16, 8 x 40 26, 20; light 64, 3 x 100 46, 30), but not few sequences of up to sixteen rows, which the others take in one launch (gla 16, 10 x 10 9.2, 12.6);
-// - long portions of few heads go here in segments (gla 16, 1 x 2000 123, 31; 32, 2 x 500 41, 28; 64, 1 x 400 30, 24; light 16, 1 x 2000 96, 27; 64, 2 x 2048 125, 109; 128
-//   channels 32, 2 x 750 78, 70; mlstm 32, 1 x 661 39, 25; 16, 1 x 2000 89, 33; but gla 16, 1 x 250 19, 21; light 16, 3 x 300 22, 22; 64, 2 x 549 39, 42; mlstm 16, 3 x 300 26, 26);
-// - mlstm's nine waves fill a compute unit, so a chip nearly full of long portions is the pipeline's (32, 5 x 600 55, 60; bf16 64, 5 x 613 83, 98; fp32 64, 8 x 250 100,
-//   77), and so are long portions beside decode rows (64, 8 of 3173 rows and 59 147, 195); more than 64 channels would spill.  Its token loop takes 0.5 us a token, so short
-//   portions come here (64, 3 x 40 35, 12; 16, 8 x 20 20, 9; fp32 16, 8 x 40 14.6, 16.6; 64, 3 x 100 25, 16; 32, 4 x 117 19.9, 21.6).
-// Where only the step's rows are known, 2.5 times a portion's least length may as well be one portion beside decode rows (64 channels of 64 or more workgroups: 4 times;
-// light 32, 4 x 779 54, 58).  The launch of the states, in vain if the portions turn out to be alike, costs 2 to 3 us: many portions have to leave room for a long one,
-// more than sixteen (decode rows, mostly) for a shorter one.
+// repeat what columns share, but have it sooner.  Only the step's rows and portions are known, not who has the rows: the workgroups decide by the lengths how portions
+// are cut, but a line here is where one long portion beside decode rows gains several times what portions that are alike lose ("but").
+// us there, here; 64 channels and bf16 rows unless said; heads, portions x rows:
+// - many portions and heads: gla 64, 3 x 40 13, 11; 64, 16 x 70 83, 33; 64, 8 x 250 117, 39; 16, 16 x 20 12.3, 9.0, but 16, 8 x 20 7.6, 8.4; light 64, 8 x 250 68, 40; 128
+//   channels: gla 64, 8 x 70 130, 53; 16, 8 x 40 26, 20; light 64, 3 x 100 46, 30; not few sequences of up to sixteen rows (gla 16, 10 x 10 9.2, 12.6);
+// - long portions of few heads, in segments: gla 16, 1 x 2000 123, 31; 32, 2 x 500 41, 28; light 16, 1 x 2000 96, 27; 64, 2 x 2048 125, 109; but gla 64, 1 x 300 23.2, 25.3; 128
+//   channels, 300 rows 33, 42, so 400 there;
+// - rows enough for one portion to be long: gla 16, 1 of 1521 among 5 95, 26; light 16, 1 of 1473 among 11 82, 47; but gla 16, 4 x 190 17, 23; fp32 4, 4 x 228 of 128
+//   channels 28, 60, so from 1000 rows there; light 16, 8 x 500 38, 42;
+// - mlstm's nine waves fill a compute unit, and its pipeline is the closer one: a nearly full chip of bf16 rows stays there (32, 5 x 600 55, 60; 64, 5 x 613 83, 98), as do long
+//   portions beside decode rows of many heads (64, 8 of 3173 rows and 59 147, 195); more than 64 channels would spill.  Its token loop takes 0.5 us a token, so short portions come here
+//   (64, 3 x 40 35, 12; 16, 8 x 20 20, 9), among nine sequences and more it has two launches to lose (16, 16 x 62 20, 14; fp32 64, 12 x 75 71, 56); full chips: 64, 3 x 100 25, 17; 32, 8 x 83
+//   23, 15; fp32 64, 3 x 300 55, 40; 8 x 500 155, 118; long portions: 32, 1 x 661 39, 25; 16, 1 x 2000 89, 33; 32, 1 of 2000 among 17 111, 69; but 32, 3 x 459 35, 46.
+// The launch of the states, in vain if no portion turns out to be worth cutting, costs 3 to 6 us; a long portion left whole 2 us for 32 rows of it, 4 of 128 channels.  Many portions
+// and heads: it is launched where one may have more than 400 to 1000 rows (64 heads, 3 x 300 29, in vain 36; 1 of 765 among 7 51, 35).
 int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows, int in_f32, long long* floats) {
   *floats = 0;
   if ((mode != MLSTM && mode != LIGHT && mode != GLA) || dk > (mode == MLSTM ? 64 : 128) || n_seq > 32767) return 0;
-  const long units = (long)n_seq * H * dgi_chunk_segments_groups(mode, dv), mean = rows / n_seq, over = rows - n_seq;
-  const long least = mode == GLA ? 280 : units > 64 ? 800 : dk <= 64 ? 400 : 600;      // rows of a portion from which segments gain
-  bool many = units >= (mode != MLSTM && dk > 64 ? 128 : 160);
-  if (mode == GLA && units >= 128 && mean >= 48) many = true;
-  if (mode != MLSTM && mean < 16 && n_seq <= 16) many = false;      // one launch takes them all
-  bool here = many || mean >= least || over >= (units > 64 && mode != GLA ? 4 : 2.5) * least;
+  const int groups = dgi_chunk_segments_groups(mode, dv);
+  const long units = (long)n_seq * H * groups, mean = rows / n_seq, over = rows - n_seq;
+  const float share = dgi_chunk_segments_share(mode, dk, dv, H), fill = rows * share;
+  bool many, here;
   if (mode == MLSTM) {
-    if (mean < 64) here = mean >= (n_seq > 8 ? 24 : 16) && over < (units >= 160 ? 640 : 256);
-    else here = (here && !(units >= 100 && (in_f32 ? units < 512 && mean >= 240 : mean >= 160 || n_seq > 16))) || (units >= 64 && mean < 80 && !in_f32);
+    const bool f = in_f32;
+    if (mean < 64 && over < (units >= 160 ? 640 : 256)) {      // the token loop's
+      many = here = mean >= (n_seq > 2 * APART_FROM ? 24 : 16);
+    } else if (n_seq > 2 * APART_FROM) {
+      many = false;
+      here = over >= (f ? 1000 : 1600) && H * groups <= (f && n_seq <= 32 ? 64 : 32) && n_seq <= 100 && fill < (f ? 700.f : 500.f);
+    } else if (n_seq > APART_FROM) {
+      many = here = mean >= 16 && (f || fill < 400.f);
+    } else {
+      many = f && mean >= 100 ? units >= 192 : units >= 96 && mean < 160;
+      here = many || (units <= 100 && mean >= 400) || (units <= 64 && over >= 1000);
+    }
+  } else {
+    const bool gla = mode == GLA, wide = dk > 64;
+    const long least = gla ? (wide ? 400 : 280) : units > 64 ? 800 : wide ? 600 : 400;
+    many = (units >= (wide ? 128 : 160) || (gla && units >= 128 && mean >= 48)) && (mean >= 16 || n_seq > 2 * APART_FROM);
+    here = many || mean >= least || over >= (gla ? (wide ? 1000 : 700) : units > 64 ? 4 * least : 5 * least / 2);
   }
   if (!here) return 0;
-  // segments that fill the chip once
-  const float share = dgi_chunk_segments_share(mode, dk, dv, H);
-  const long each = (std::max({96l, (long)(rows * share), std::min(128l, rows / 16l)}) + C - 1) / C * C;
-  if (over < (!many ? 1 : n_seq > 16 ? 768 : 1000) || whole(over + 1, rows, share, each) || !places(rows, each)) return 1 << 29;
+  // segments that fill the chip once; of 128 rows at least where sixteen of them are no more than a portion
+  const long each = (std::max({96l, (long)fill, std::min(128l, rows / 16l)}) + C - 1) / C * C;
+  const long keep = !many ? 1 : n_seq > 64 ? std::max(400l, (long)(80 * share * std::min(n_seq, rows / 17))) : n_seq > 2 * APART_FROM ? 768 : n_seq > APART_FROM ? 1000 : mode == MLSTM ? 600 : dk > 64 ? 700 : 1000;
+  if (over < keep || whole(over + 1, rows, share, each) || !places(rows, each)) return 1 << 29;
   *floats = places(rows, each) * H * (state_floats(mode, dk, dv) + decay_floats(mode, dk));
   return (int)each;
 }

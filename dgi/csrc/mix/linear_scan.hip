@@ -1147,8 +1147,7 @@ constexpr int APART_FROM = 8;        // sequences of a step above which those ar
 // 13; 400 rows 31, 25; 512 units, 100 rows 16, 12; 1024 units, 64 rows 20, 17; 2048 units, 64 rows 36, 35; 128-wide heads: 128 units, 100 rows 15, 15;
 // 1024 units, 64 rows 30, 25; 4096 units, 64 rows 108, 91).
 // Among more than APART_FROM sequences it has a launch more to lose (64-wide heads: 9 x 80 rows, 16 heads 17, 20; 12 x 112 22, 24; 12 x 128 24, 24; 9 x 80, 32
-// heads 24, 28; 9 x 96 28, 28; 24 x 65, 32 heads 52, 49; 128-wide: 9 x 80, 8 heads 24, 27; 9 x 96 28, 27).  mlstm of up to 64 channels has
-// chunk_segments.h, which fills sooner, too (bf16 rows of 16 heads, 8 x 20 rows 19.8 -> 9.1, 1 x 40 21.9 -> 10.7; with a launch more, 14 x 18 25 -> 34, 16 x 40 19.9 -> 13.3).
+// heads 24, 28; 9 x 96 28, 28; 24 x 65, 32 heads 52, 49; 128-wide: 9 x 80, 8 heads 24, 27; 9 x 96 28, 27).
 static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
   const long units = (long)n_seq * H * ((dv + 15) / 16);
   if (mode == LIGHT) {
@@ -1156,7 +1155,6 @@ static long chunk_from(int mode, int dk, int dv, int H, int n_seq) {
     if (units <= 768) return dk <= 64 ? 112 : 88;
     return dk <= 64 && (units <= 1280 || n_seq <= 16) ? 88 : 64;
   }
-  if (mode == MLSTM && dk <= 64) return n_seq > APART_FROM ? 24 : SHORT;
   if (mode != WKV || units <= 512) return 64;
   return dk > 64 ? 104 : units <= 3072 ? 136 : 224;
 }
@@ -1187,7 +1185,7 @@ static int chunk_form(int mode, int dk, int dv, int G, int H, const void* q, int
 extern "C" int dgi_linear_scan_segments(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
                                         int in_f32, const float* aux1, int aux1_stride, long long* floats) {
   *floats = 0;
-  if (n_seq == 0 || G != H || !chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows)) return 0;
+  if (n_seq == 0 || G != H || (mode != MLSTM && !chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows))) return 0;
   if (!dgi_chunk_scan_ok(mode, dk, q, q_stride, k, k_stride, in_f32) || (mode == GLA && (aux1_stride % 2 || ((uintptr_t)aux1 & 7)))) return 0;
   return dgi_chunk_segments_plan(mode, dk, dv, H, n_seq, rows, in_f32, floats);
 }
@@ -1195,9 +1193,9 @@ extern "C" int dgi_linear_scan_segments(int mode, int dk, int dv, int H, int G, 
 // whether the matrix memory of a step has several workgroups per head in one of its launches: its normaliser and maximum are staged
 extern "C" int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
                                       int in_f32, int seg_rows) {
-  const bool chunked = chunk_form(MLSTM, dk, dv, H, H, q, q_stride, k, k_stride, in_f32, n_seq, rows) != 0;
+  const bool chunked = seg_rows || chunk_form(MLSTM, dk, dv, H, H, q, q_stride, k, k_stride, in_f32, n_seq, rows) != 0;
   if (chunked && (seg_rows ? dgi_chunk_segments_groups(MLSTM, dv) > 1 : dv > 32)) return 1;
-  if (chunked && n_seq <= APART_FROM) return 0;
+  if (chunked && n_seq <= (seg_rows ? 2 : 1) * APART_FROM) return 0;
   const int R = scan_channels(dk, dv, H, n_seq, chunked ? n_seq : rows);
   int KS = 1;
   while (KS * R < dk) KS <<= 1;
@@ -1235,16 +1233,15 @@ extern "C" int dgi_linear_scan(float* y, int mode, const void* q, int q_stride, 
   bool short_rows = rows <= 4 * n_seq;             // rows of the step: at most four per sequence on average
   const bool staged = mode == MLSTM && norm_new && mx_new;
   // Prompt portions: sixteen or 32 tokens at a time on the matrix cores (chunk_scan.hip, chunk_parts.hip, chunk_delta.hip).  Among many sequences there are decode
-  // rows and short portions beside the long ones: they stay with this kernel, in a launch of their own (gla and light beside chunk_segments.h's where
-  // that kernel's workgroups for all sequences are more than the chip has at once: its first chunk takes 7 us whatever a portion's rows.  16 heads of 64, 7 portions of 87
-  // rows in all and 12 decode rows 13.9 in two launches, 8.9 in one; 64 heads, 2 of 1539 and 15 decode rows 76 in one, 59 in two).
-  const int form = chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows);
-  const bool beside = seg_rows && mode != MLSTM;
-  const bool two = n_seq > APART_FROM && (beside ? rows <= 160 * n_seq && n_seq * dgi_chunk_segments_share(mode, dk, dv, H) > 1.f
-                                                 : form == 1 || (form == 2 && rows <= 4 * n_seq));
-  const int apart = !two ? 0 : beside ? 4 : mode == WKV && chunk_from(mode, dk, dv, H, n_seq) > 64 ? (int)chunk_from(mode, dk, dv, H, n_seq) : SHORT;
+  // rows and short portions beside the long ones: they stay with this kernel, in a launch of their own.  chunk_segments.h's workgroups for all sequences
+  // are waited for only once they are more than the chip has at once (16 heads of 64, 7 portions of 87 rows in all and 12 decode rows 13.9 us in two launches, 8.9 in one; 64 heads,
+  // 2 of 1539 and 15 decode rows 76 in one, 59 in two); up to sixteen sequences are one launch (16 heads, 12 x 58 rows 12.4 in two, 10.2 in one).
+  const int form = seg_rows ? 1 : chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows);
+  const bool two = seg_rows ? n_seq > 2 * APART_FROM && rows <= 160 * n_seq && (mode == MLSTM || n_seq * dgi_chunk_segments_share(mode, dk, dv, H) > 1.f)
+                            : n_seq > APART_FROM && (form == 1 || (form == 2 && rows <= 4 * n_seq));
+  const int apart = !two ? 0 : mode == WKV && chunk_from(mode, dk, dv, H, n_seq) > 64 ? (int)chunk_from(mode, dk, dv, H, n_seq) : SHORT;
   if (form) {
-    const int rc = form == 1 || seg_rows ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
+    const int rc = form == 1 ? dgi_chunk_scan(y, mode, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? nullptr : aux1, aux1_stride,
                                               aux2, aux2_stride, 0, par1, par2, nullptr, cap, state, norm, mx, norm_new, mx_new, positions,
                                               seq_row0, seq_slots, n_seq, H, G, dk, dv, apart, 1, seg_rows, seg, nullptr, parts, parts_chunks, rows, st)
                              : dgi_chunk_scan_decay(y, mode == LIGHT, q, q_stride, k, k_stride, v, v_stride, in_f32, mode == LIGHT ? par1 : aux1,
