@@ -42,10 +42,12 @@ float dgi_chunk_segments_share(int mode, int dk, int dv, int H) {
 //   channels 28, 60, so from 1000 rows there; light 16, 8 x 500 38, 42;
 // - mlstm's nine waves fill a compute unit, and its pipeline is the closer one: a nearly full chip of bf16 rows stays there (32, 5 x 600 55, 60; 64, 5 x 613 83, 98), as do long
 //   portions beside decode rows of many heads (64, 8 of 3173 rows and 59 147, 195); more than 64 channels would spill.  Its token loop takes 0.5 us a token, so short portions come here
-//   (64, 3 x 40 35, 12; 16, 8 x 20 20, 9), among nine sequences and more it has two launches to lose (16, 16 x 62 20, 14; fp32 64, 12 x 75 71, 56); full chips: 64, 3 x 100 25, 17; 32, 8 x 83
-//   23, 15; fp32 64, 3 x 300 55, 40; 8 x 500 155, 118; long portions: 32, 1 x 661 39, 25; 16, 1 x 2000 89, 33; 32, 1 of 2000 among 17 111, 69; but 32, 3 x 459 35, 46.
+//   (64, 3 x 40 35, 12; 16, 8 x 20 20, 9), among nine sequences and more it has two launches to lose (16, 16 x 62 23, 15; fp32 64, 12 x 75 79, 45); full chips: 64, 3 x 100 25, 17; 32, 8 x 83
+//   23, 15; fp32 64, 3 x 300 55, 45; 8 x 500 153, 128; long portions: 32, 1 x 661 39, 25; 16, 1 x 2000 89, 33; 32, 1 of 2000 among 17 107, 64; but 32, 3 x 459 35, 46.
 // The launch of the states, in vain if no portion turns out to be worth cutting, costs 3 to 6 us; a long portion left whole 2 us for 32 rows of it, 4 of 128 channels.  Many portions
-// and heads: it is launched where one may have more than 400 to 1000 rows (64 heads, 3 x 300 29, in vain 36; 1 of 765 among 7 51, 35).
+// and heads: it is launched where one may have more than 400 to 1000 rows (64 heads, 3 x 300 29, in vain 36; 32, 1 of 765 among 7 52, 28), and, among more than 64 sequences, than
+// the workgroups of those that turn out to be short cost: 2 us for as many as the chip has at once, in both launches (64 heads of 128 channels, 3747 rows of 203 sequences 772, cut 996; of
+// 64, 4000 rows and 500 decode rows 635, 525; 2 of 2000 and 1000 744, 790).
 int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows, int in_f32, long long* floats) {
   *floats = 0;
   if ((mode != MLSTM && mode != LIGHT && mode != GLA) || dk > (mode == MLSTM ? 64 : 128) || n_seq > 32767) return 0;
