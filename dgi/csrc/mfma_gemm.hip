@@ -1305,23 +1305,35 @@ Shares shares(int total, int P, int skmode) {
 
 // Row tiles of 16 per wave group (IT, tiles of 32 IT rows) of M rows: the fewest rows of padding are not the least time, since a round of the chip
 // takes (5.4 + IT) / 13.4 of one of 256 rows (its weights come through at 3 TB/s whatever the rows: 57344 x 8192, 896 tiles in 3.5 rounds, 677 us of
-// 256 rows, 614 of 224, 571 of 192, 524 of 160), lower tiles are more of them, and pieces along K take some 25 us to add up (28672 x 4096, 900 rows: 448 tiles of
-// 256 180 us, 560 of 192, the last 48 in pieces, 199).  So the least of rounds times that, 256 rows unless others gain 2 %.  us of 256 rows and of the rule's: 57344 x 8192, 319 rows 362, 321 (160), 435 375, 347 (224), 576 528, 473 (192), 802 670, 617 (224), 512 372 (224: 494); 8192 x 28672
-// in pieces, 319 196, 172; 435 200, 191; 659 312, 293; 8192 x 8192, 319 79, 65; 435 86, 77; 10240 x 8192, 435 92, 88.
+// 256 rows, 614 of 224, 571 of 192, 524 of 160), lower tiles are more of them, and pieces along K wait for each other and are added up: three and a half of K's steps of 64 for each piece
+// of a tile, 9 for a slab of 256 rows from every unit.  So the least of that, 256 rows unless others gain 2 %, or 5 % where other elements or other lengths would be summed in
+// pieces: then the results' last bits are not those of 256 rows.
+//
+// Measured at 1 to 2560 rows of 22 sizes of 2048 x 4096 and more (in us of 256 rows and of the rule's): 57344 x 8192, 319 rows 362, 321 (160), 435 375, 347 (224), 576 528, 473 (192), 802
+// 670, 617 (224), 512 349 (224: 490), 2400 1620 (224: 1663); 8192 x 28672 in pieces, 319 196, 172; 435 200, 191; 659 312, 293; 1792 575, 559 (224); 8192 x 8192, 319 79, 65; 435 86, 77; 1200 154, 148 (224);
+// 12288 x 4096, 512 64 (160: 74, one round without pieces); 28672 x 4096, 256 82 (160: 87); 6144 x 4096, 1200 67 (160: 72); 4096 x 4096, 1200 70, 56 (160); 256 48, 42; one row 0.75 to 0.98 of 256.
+// In all 7 % less than 256 rows, half a per cent from the best height each; slower than 256 rows by more than 3 %: 53248 x 16384, 129 391, 404; 22016 x 4096, 640 119, 125; 37888 x 3584, 129 79, 84.
+double tiles_time(const Shares& sh, int it, int K) {
+  const double k = K / kBK, row = 5.4 + it;
+  double t = (sh.full + (sh.rem && !sh.hybrid ? 1 : 0)) * k * row;
+  if (sh.hybrid) t += k / sh.splits * row + 15. * (3 * sh.splits + sh.rem * sh.splits / 32. * it / 8);
+  return t;
+}
 int row_tiles(int M, int tiles_n, int K, int P, int skmode) {
+  const Shares all = shares((M + kBM - 1) / kBM * tiles_n, P, skmode);
   int best = 8;
-  double least = 0.;
-  for (int it = 8; it >= 5; --it) {
+  double least = tiles_time(all, 8, K);
+  for (int it = 7; it >= 5; --it) {
     const Shares sh = shares((M + 32 * it - 1) / (32 * it) * tiles_n, P, skmode);
-    const double rounds = sh.full + (sh.hybrid ? 1. / sh.splits + 20. * kBK / K : sh.rem ? 1. : 0.), cost = rounds * (5.4 + it) * (it == 8 ? 0.98 : 1.);
-    if (it == 8 || cost < least) {
+    const bool same = all.hybrid ? sh.hybrid && all.full + sh.full == 0 && all.splits == sh.splits : !sh.hybrid;
+    const double t = tiles_time(sh, it, K) / (same ? 0.98 : 0.95);
+    if (t < least) {
       best = it;
-      least = cost;
+      least = t;
     }
   }
   return best;
 }
-
 template <int EPI>
 void launch_pp(const void* x, int ldx, const void* w, void* y, int ldy, int M, int I, int K, int tiles_n,
                int skmode, int prio, hipStream_t s, const NormArgs& na = NormArgs{}, const SkWorkspace& own = SkWorkspace{}) {
@@ -1390,6 +1402,16 @@ void launch(const void* x, int ldx, const void* w, void* y, int ldy, int M, int 
 }
 
 }  // namespace
+
+// what the rule says for a launch of P units (tests)
+extern "C" int dgi_mfma_row_tiles(int M, int tiles_n, int K, int P, int skmode, int* full, int* rem, int* splits) {
+  const int it = row_tiles(M, tiles_n, K, P, skmode);
+  const Shares sh = shares((M + 32 * it - 1) / (32 * it) * tiles_n, P, skmode);
+  *full = sh.full;
+  *rem = sh.rem;
+  *splits = sh.hybrid ? sh.splits : 1;
+  return 32 * it;
+}
 
 // epi & 1: 0 = Y[M, N] = X W^T with N = rows of W; 1 = Y[M, I] = SwiGLU with W = [gate; up] (2I rows).
 // epi >> 4: K-loop schedule (0 = compiler order, 1 = interleaved, 2 = 4-slot ring of 32-deep sub-steps,

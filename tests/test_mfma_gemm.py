@@ -110,7 +110,8 @@ def test_mfma_gemm_splitk_matches_fp32_and_is_deterministic(M, N, K, epi, stream
     remainder tile reduced by the last arriving block through fp32 slabs; uneven
     piece lengths at K = 512; N = 19200 at M = 2048: a split piece, then two whole
     tiles whose second loads under the first's epilogue; N = 57344 at M = 512 / 200 and
-    N = 48896 at M = 1000: a last wave more than half full, no split): matches the fp32
+    N = 48896 at M = 1000: a last wave more than half full, no split).  So with four phases; with two, some have
+    lower tiles and other pieces (test_mfma_gemm_lower_tiles_in_pieces has those of every height).  Matches the fp32
     reference, and repeated launches agree bit for bit (slabs are summed in piece order
     whichever piece arrives last)."""
     ops.load_native(required=True)
@@ -312,3 +313,71 @@ def test_mfma_gemm_tiles_of_fewer_rows(M, kind):
         assert (two[0].float() - ref).abs().max().item() <= 2e-2 * ref.abs().max().item() + 1e-3
     for a, b in zip(two, four):
         assert torch.equal(a, b)
+
+
+def row_tiles(M, tiles_n, K, units=256, skmode=1):
+    """(rows of a tile, whole tiles a unit, tiles left, their pieces) that two-phase launches take."""
+    import ctypes
+
+    import dgi.build
+    lib = ctypes.CDLL(dgi.build.build())
+    out = [ctypes.c_int() for _ in range(3)]
+    return (lib.dgi_mfma_row_tiles(M, tiles_n, K, units, skmode, *map(ctypes.byref, out)),) + tuple(v.value for v in out)
+
+
+@pytest.mark.parametrize("M,N,K,rows", [
+    (319, 57344, 8192, 160), (435, 57344, 8192, 224), (576, 57344, 8192, 192), (802, 57344, 8192, 224), (512, 57344, 8192, 256), (2400, 57344, 8192, 256),
+    (319, 8192, 28672, 160), (435, 8192, 28672, 224), (1792, 8192, 28672, 224), (319, 8192, 8192, 160), (435, 8192, 8192, 224), (256, 4096, 4096, 160),
+    (1200, 4096, 4096, 160), (1, 4096, 4096, 160), (512, 12288, 4096, 256), (256, 28672, 4096, 256), (256, 22016, 4096, 256), (1200, 6144, 4096, 256),
+    (1024, 8192, 3584, 256), (1792, 10240, 8192, 256), (1792, 57344, 8192, 256)])
+def test_row_tiles_are_the_faster_ones_cpu(M, N, K, rows):
+    """The heights measured as the faster, among them products that the first rule sent to lower tiles that took 5 to 16 % longer."""
+    assert row_tiles(M, N // 256, K)[0] == rows
+
+
+def _two_phase_matches(M, tiles_n, K, kind, exact):
+    """``kind`` 0 / 1 plain and SwiGLU, 2 .. 5 the norm epilogues, two phases a K tile: against the reference, and bit for bit against 256 rows."""
+    ops.load_native(required=True)
+    N = tiles_n * 256
+    if kind == 5:
+        got, want = _rope_case(M, tiles_n * 2 - 4, 2, K, "cuda", 2)
+        four = _rope_case(M, tiles_n * 2 - 4, 2, K, "cuda", 4)[0] if exact else None
+    elif kind >= 2:
+        got, want = _norm_case(M, N, K, kind, "cuda", 2)
+        four = _norm_case(M, N, K, kind, "cuda", 4)[0] if exact else None
+    else:
+        x, w = _rand(M, K, device="cuda", seed=M), _rand(N, K, device="cuda", scale=0.05, seed=1)
+        got, want = (ops.mfma_gemm(x, w, kind, sched=3, phases=2),), (ops.mfma_gemm_ref(x, w, kind),)
+        four = (ops.mfma_gemm(x, w, kind, sched=1),) if exact else None
+        for _ in range(4):
+            assert torch.equal(ops.mfma_gemm(x, w, kind, sched=3, phases=2), got[0])
+        if exact:
+            assert torch.equal(ops.mfma_gemm(x, w, kind, sched=3, phases=2, overlap=False), got[0])
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert (g.float() - w.float()).abs().max().item() <= 2e-2 * w.float().abs().max().item() + 1e-3
+    for g, f in zip(got, four or ()):
+        assert torch.equal(g, f)
+    assert ops.gemm_split_timeouts(reset=True) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,rows", [(260, 160), (320, 160), (330, 192), (384, 192), (390, 224), (448, 224)])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3, 4, 5])
+def test_mfma_gemm_lower_tiles_in_whole_rounds(M, rows, kind):
+    """Two whole lower tiles a unit, the second's loads under the first's epilogue where that stores every row: the bits of 256 rows and of no overlap."""
+    assert row_tiles(M, 256, 512) == (rows, 2, 0, 1)
+    _two_phase_matches(M, 256, 512, kind, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,tiles_n,rows,full,pieces", [
+    (170, 43, 160, 0, 2), (170, 33, 160, 0, 3), (140, 8, 160, 0, 4), (260, 264, 160, 2, 4), (260, 296, 160, 2, 3), (170, 304, 160, 2, 2),
+    (490, 29, 192, 0, 2), (650, 17, 192, 0, 3), (180, 8, 192, 0, 4), (330, 264, 192, 2, 4), (330, 296, 192, 2, 3), (520, 200, 192, 2, 2),
+    (200, 16, 224, 0, 4), (390, 176, 224, 1, 2), (390, 272, 224, 2, 4), (580, 200, 224, 2, 2), (580, 195, 224, 2, 3)])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3, 4, 5])
+def test_mfma_gemm_lower_tiles_in_pieces(M, tiles_n, rows, full, pieces, kind):
+    """Lower tiles of which some are cut along K, uneven at three pieces of 8 K tiles, alone and before whole tiles."""
+    got = row_tiles(M, tiles_n, 512)
+    assert (got[0], got[1], got[3]) == (rows, full, pieces)
+    _two_phase_matches(M, tiles_n, 512, kind, False)
