@@ -17,12 +17,11 @@ using namespace dgi;
 namespace {
 
 // A workgroup owns a head and 64 latent dims, wave w 16 of them; its slab of uk lies in LDS and is read transposed (the
-// product's A operand: latent dims by query dims).  DS = dim / 32 steps; FOLD rows, sixteen at a time (128 rows of 16
-// heads one behind the other 5.7 us, so 4.5).
-constexpr int FOLD = 32;
+// product's A operand: latent dims by query dims).  DS = dim / 32 steps; `fold` rows, sixteen at a time: 32 (128 rows of
+// 16 heads one behind the other 5.7 us, so 4.5), 64 where heads alone fill the chip (256 rows of 32 heads: all 7.7, by 64 8.0, by 32 8.2).
 template <int DS>
 __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__ q_lat, const uint16_t* __restrict__ q, int q_stride,
-                                                          const uint16_t* __restrict__ uk, int T, int qk, int kr) {
+                                                          const uint16_t* __restrict__ uk, int T, int qk, int kr, int fold) {
   constexpr int DIM = 32 * DS;
   __shared__ __attribute__((aligned(16))) uint16_t slab[DIM * 64];
   const int head = blockIdx.x, c0 = blockIdx.y * 64;
@@ -40,7 +39,7 @@ __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__
 #pragma unroll
     for (int s = 0; s < DS; ++s) b[s] = *reinterpret_cast<const u32x4*>(p + 32 * s);
   };
-  const int from = blockIdx.z * FOLD, to = min(T, from + FOLD);
+  const int from = blockIdx.z * fold, to = min(T, from + fold);
   u32x4 b[DS];
   load_q(from, b);
 #pragma unroll
@@ -75,13 +74,16 @@ __global__ __launch_bounds__(256) void latent_fold_kernel(uint16_t* __restrict__
 // What bounds it is its bytes through the caches (32 rows of 32 heads, 8 runs: 17 MB of partial sums and 128 KB of uv a workgroup) and a chain of
 // latencies.  The partial sums are read as they lie, four dims a thread, 128 threads a row; rows fewer than four leave their threads to
 // others of the row's runs, and those sums meet in LDS.  Lane z holds run z's factor, so that nobody waits for another wave's.  The rows then go
-// through LDS to the product, whose waves take sixteen value dims each over 512 / KP latent dims.  The weights, the gate and the first runs are
+// through LDS to the product, whose waves take sixteen value dims each over 512 / KP latent dims (so do rows without runs where most waves read the same dims).
+// Two to four runs: a group asks for four or two rows at once, so that eight loads are under way.  The weights, the gate and the first runs are
 // under way while the factors are formed.  Before, a wave had 64 latent dims of all value dims, lanes without a row of their own read another's again, and
-// few rows a workgroup meant all of uv for each: us then and now, rows x heads x runs: 32 x 32 x 8 10.7, 8.0; 3 x 16 x 6 8.6, 4.7; 8 x 16 x 32 10.7, 6.4;
-// 11 x 32 x 23 18.8, 9.3; 44 x 16 x 5 16.6, 7.1; without runs 24 x 32 10.4, 4.1; 2 x 32 5.6, 4.0.
+// few rows a workgroup meant all of uv for each: us then and now, rows x heads x runs: 32 x 32 x 8 11.3, 8.5; 3 x 16 x 6 8.6, 4.7; 8 x 16 x 16 10.3, 5.9;
+// 24 x 32 x 16 20.3, 9.5; 48 x 16 x 4 14.1, 7.0; 64 x 32 x 2 9.2, 7.0; 4 9.7, 9.4; 128 x 32 x 2 10.7, 8.7; without runs 24 x 32 10.9, 4.8; 2 x 32 5.6, 3.7; 128 x 32 7.1, 6.6 (each wave reading all rows
+// from memory 9.8); 256 x 32 12.0, 10.5.
 constexpr int KR = 512, RUNS = 64, BATCH = 8;
 
-template <int KP>
+// RP: rows of a group of threads at once, where a row's runs are BATCH / RP at most
+template <int KP, int RP>
 __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict__ out, const uint16_t* __restrict__ o_lat,
                                                             const float* __restrict__ part, const float* __restrict__ ml, int runs,
                                                             const float* __restrict__ sinks, const uint16_t* __restrict__ uv,
@@ -111,74 +113,104 @@ __global__ __launch_bounds__(512) void latent_values_kernel(uint16_t* __restrict
   };
   u32x4 b[NS];
   if (runs > 1) {
-    const int apart = min(rb, 4), sharers = 4 / apart;     // rows at a time, groups of threads of a row
+    const int apart = RP > 1 ? 4 : min(rb, 4), sharers = 4 / apart;        // rows at a time, groups of threads of a row
     const int group = w >> 1, sub = group / apart, col = threadIdx.x & 127;
     const size_t next = (size_t)H * T;
-    float4 p[BATCH];
-    auto load_runs = [&](int r, int i0) {                  // the batch of this group's runs, sub + sharers i
-      const float* src = part + ((size_t)head * T + t0 + min(r, nr - 1)) * KR + 4 * col;
+    constexpr int S = BATCH / RP;
+    float4 p[RP][S];
+    float2 e[RP];
+    auto load_runs = [&](int r, int i0) {                // the batch of this group's runs, sub + sharers i
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) p[i] = *reinterpret_cast<const float4*>(src + (size_t)min(sub + (i0 + i) * sharers, runs - 1) * next * KR);
+      for (int u = 0; u < RP; ++u) {
+        const float* src = part + ((size_t)head * T + t0 + min(r + u * apart, nr - 1)) * KR + 4 * col;
+#pragma unroll
+        for (int i = 0; i < S; ++i) p[u][i] = *reinterpret_cast<const float4*>(src + (size_t)min(sub + (i0 + i) * sharers, runs - 1) * next * KR);
+      }
+    };
+    auto load_ml = [&](int r) {
+#pragma unroll
+      for (int u = 0; u < RP; ++u)
+        e[u] = *reinterpret_cast<const float2*>(ml + 2 * ((size_t)min(lane, runs - 1) * next + (size_t)head * T + t0 + min(r + u * apart, nr - 1)));
     };
     int r = group % apart;
-    auto load_ml = [&](int r) {
-      return *reinterpret_cast<const float2*>(ml + 2 * ((size_t)min(lane, runs - 1) * next + (size_t)head * T + t0 + min(r, nr - 1)));
-    };
-    float2 e = load_ml(r);
+    load_ml(r);
     load_runs(r, 0);
     load_uv();
     load_gate();
-    for (; r < rb; r += apart) {
-      const float m = lane < runs ? e.x : -__builtin_inff();
-      float M = fmaxf(m, -FLT_MAX);                        // finite also where no run has keys
+    for (; RP == 4 || r < rb; r += RP * apart) {           // RP 4: rb is 16
+      float f[RP], inv[RP];
       // few runs: the lanes that have them; a loop of more turns costs what it saves
-      auto turns = [&](auto f) {
+      auto turns = [&](auto g) {
         if (runs > 8) {
 #pragma unroll
-          for (int o = 1; o < 64; o <<= 1) f(o);
+          for (int o = 1; o < 64; o <<= 1) g(o);
         } else {
-          for (int o = 1; o < runs; o <<= 1) f(o);
+          for (int o = 1; o < runs; o <<= 1) g(o);
         }
       };
-      turns([&](int o) { M = fmaxf(M, __shfl_xor(M, o, 64)); });
-      const float f = expf(m - M);
-      float L = lane < runs ? e.y * f : 0.f;
-      turns([&](int o) { L += __shfl_xor(L, o, 64); });
-      float inv = L == 0.f ? 0.f : 1.f / L;
-      if (sinks) {                                         // one more logit in the denominator, relative to the larger of the two
-        const float sink = sinks[head], top = fmaxf(M, sink), g = expf(M - top);
-        inv = g / (L * g + expf(sink - top));
-      }
-      inv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(inv), 0));
-      const bool more = r + apart < rb;
-      if (more) e = load_ml(r + apart);
-      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int i0 = 0; sub + i0 * sharers < runs; i0 += BATCH) {
 #pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-          const int z = sub + (i0 + i) * sharers;
-          if (z < runs) {
-            const float fz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f), z));
-            x.x += p[i].x * fz; x.y += p[i].y * fz; x.z += p[i].z * fz; x.w += p[i].w * fz;
-          }
+      for (int u = 0; u < RP; ++u) {
+        const float m = lane < runs ? e[u].x : -__builtin_inff();
+        float M = fmaxf(m, -FLT_MAX);                    // finite also where no run has keys
+        turns([&](int o) { M = fmaxf(M, __shfl_xor(M, o, 64)); });
+        f[u] = expf(m - M);
+        float L = lane < runs ? e[u].y * f[u] : 0.f;
+        turns([&](int o) { L += __shfl_xor(L, o, 64); });
+        float v = L == 0.f ? 0.f : 1.f / L;
+        if (sinks) {                                     // one more logit in the denominator, relative to the larger of the two
+          const float sink = sinks[head], top = fmaxf(M, sink), g = expf(M - top);
+          v = g / (L * g + expf(sink - top));
         }
-        if (sub + (i0 + BATCH) * sharers < runs) load_runs(r, i0 + BATCH);
-        else if (more) load_runs(r + apart, 0);
+        inv[u] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), 0));
       }
-      if (sharers > 1) {                                   // one row a group: all pass these once
-        if (sub > 0) others[(sub - 1) * apart + r][col] = x;
+      const bool more = RP < 4 && r + RP * apart < rb;
+      if (more) load_ml(r + RP * apart);
+      float4 x[RP];
+#pragma unroll
+      for (int u = 0; u < RP; ++u) x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int i0 = 0; sub + i0 * sharers < runs; i0 += S) {
+#pragma unroll
+        for (int u = 0; u < RP; ++u)
+#pragma unroll
+          for (int i = 0; i < S; ++i) {
+            const int z = sub + (i0 + i) * sharers;
+            if (z < runs) {
+              const float fz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f[u]), z));
+              x[u].x += p[u][i].x * fz; x[u].y += p[u][i].y * fz; x[u].z += p[u][i].z * fz; x[u].w += p[u][i].w * fz;
+            }
+          }
+        if (sub + (i0 + S) * sharers < runs) load_runs(r, i0 + S);
+        else if (more) load_runs(r + RP * apart, 0);
+      }
+      if (RP == 1 && sharers > 1) {                      // one row a group: all pass these once
+        if (sub > 0) others[(sub - 1) * apart + r][col] = x[0];
         __syncthreads();
         if (sub > 0) break;
         for (int q = 1; q < sharers; ++q) {
           const float4 y = others[(q - 1) * apart + r][col];
-          x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w;
+          x[0].x += y.x; x[0].y += y.y; x[0].z += y.z; x[0].w += y.w;
         }
       }
-      *reinterpret_cast<uint2*>(&rows[r][4 * col]) = make_uint2(pack_bf16x2(x.x * inv, x.y * inv), pack_bf16x2(x.z * inv, x.w * inv));
+#pragma unroll
+      for (int u = 0; u < RP; ++u)
+        *reinterpret_cast<uint2*>(&rows[r + u * apart][4 * col]) =
+            make_uint2(pack_bf16x2(x[u].x * inv[u], x[u].y * inv[u]), pack_bf16x2(x[u].z * inv[u], x[u].w * inv[u]));
+      if (RP == 4) break;
     }
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < NS; ++s) b[s] = *reinterpret_cast<const u32x4*>(&rows[min(lr, rb - 1)][k + 32 * s]);
+  } else if constexpr (KP <= 2) {                            // most waves read the same dims: through LDS, a row a wave
+    u32x4 v[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) v[i] = *reinterpret_cast<const u32x4*>(o_lat + ((size_t)head * T + t0 + min(w + 8 * i, nr - 1)) * KR + 8 * lane);
+    load_uv();
+    load_gate();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(&rows[w + 8 * i][8 * lane]) = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) b[s] = *reinterpret_cast<const u32x4*>(&rows[lr][k + 32 * s]);
   } else {
 #pragma unroll
     for (int s = 0; s < NS; ++s) b[s] = *reinterpret_cast<const u32x4*>(o_lat + ((size_t)head * T + t0 + min(lr, nr - 1)) * KR + k + 32 * s);
@@ -214,10 +246,11 @@ extern "C" int dgi_latent_fold(void* q_lat, const void* q, int q_stride, const v
   if (H <= 0 || dim % 32 || dim < 32 || dim > 128 || kr % 64 || qk % 8 || q_stride % 8 || (((uintptr_t)q | (uintptr_t)uk) & 15) ||
       ((uintptr_t)q_lat & 7))
     return -2;
-  if ((T + FOLD - 1) / FOLD > 65535) return -4;
-  const dim3 grid(H, kr / 64, (T + FOLD - 1) / FOLD);
+  const int fold = H * (kr / 64) >= 256 ? 64 : 32;
+  if ((T + fold - 1) / fold > 65535) return -4;
+  const dim3 grid(H, kr / 64, (T + fold - 1) / fold);
 #define DGI_LF(N_)                                                                                                             \
-  latent_fold_kernel<N_><<<grid, 256, 0, s>>>((uint16_t*)q_lat, (const uint16_t*)q, q_stride, (const uint16_t*)uk, T, qk, kr)
+  latent_fold_kernel<N_><<<grid, 256, 0, s>>>((uint16_t*)q_lat, (const uint16_t*)q, q_stride, (const uint16_t*)uk, T, qk, kr, fold)
   switch (dim / 32) {
     case 1: DGI_LF(1); break;
     case 2: DGI_LF(2); break;
@@ -253,13 +286,18 @@ extern "C" int dgi_latent_values(void* out, const void* o_lat, const float* part
   }
   if ((T + rb - 1) / rb > 65535) return -4;
   const dim3 grid(H, (T + rb - 1) / rb, nv / np);
-#define DGI_LV(N_)                                                                                                                      \
-  latent_values_kernel<N_><<<grid, 512, 0, s>>>((uint16_t*)out, (const uint16_t*)o_lat, part, ml, runs, sinks, (const uint16_t*)uv,     \
-                                                (const uint16_t*)gate, gate_stride, per_head, T, H, vdim, rb, np)
-  if (np == 1) DGI_LV(8);
-  else if (np == 2) DGI_LV(4);
-  else if (np <= 4) DGI_LV(2);
-  else DGI_LV(1);
+#define DGI_LV(N_, R_)                                                                                                                  \
+  latent_values_kernel<N_, R_><<<grid, 512, 0, s>>>((uint16_t*)out, (const uint16_t*)o_lat, part, ml, runs, sinks, (const uint16_t*)uv, \
+                                                    (const uint16_t*)gate, gate_stride, per_head, T, H, vdim, rb, np)
+#define DGI_LV_ROWS(N_)                                                              \
+  if (runs == 2 && rb == 16) DGI_LV(N_, 4);                                          \
+  else if (runs > 1 && runs <= 4 && rb >= 8) DGI_LV(N_, 2);                          \
+  else DGI_LV(N_, 1)
+  if (np == 1) { DGI_LV_ROWS(8); }
+  else if (np == 2) { DGI_LV_ROWS(4); }
+  else if (np <= 4) { DGI_LV_ROWS(2); }
+  else { DGI_LV_ROWS(1); }
+#undef DGI_LV_ROWS
 #undef DGI_LV
   DGI_CHECK_LAUNCH();
   return 0;

@@ -253,19 +253,29 @@ def decode_heads_ok(q: torch.Tensor, rows: int, dim: int, rot_dim: int, kv_rank:
             and q.data_ptr() % 16 == 0 and (gate is None or gate.dtype == torch.bfloat16))
 
 
+def decode_runs(rows: int, heads: int, bound: int) -> int:
+    """Runs of keys per row of ``latent_decode_heads`` where no row has more than ``bound``: of 64 keys at least, as many as fill the chip, and no more than
+    pay: a layer takes about 0.05 us a key of ``bound`` over the runs, and for every run (its sums are written and read again) 0.045 us a row of 32 heads, two thirds of that of 16.
+    Us a layer in 1, 2, 3, 4, 8 runs, rows x heads, keys of about 0.75 ``bound``: 8 x 32, 200 28.1, 22.3, 20.7, 19.7, 19.7; 32 x 32, 160 28.1, 24.7, 24.4, 25.2, 27.3; 400 44.4, 32.2,
+    29.7, 27.4, 29.0; 64 x 32, 100 24.3, 25.8, 28.2, 29.8; 200 31.7, 27.9, 28.9, 31.0; 128 x 32, 250 38.9, 39.1; 128 x 16, 130 26.2, 28.1."""
+    if bound < 192:
+        return 1
+    best = (80 * bound / (max(rows, 1) * (heads + 32))) ** 0.5
+    return max(1, min(tile_runs(rows, heads, bound, 64), int(best + (0.7 if best > 3.5 else 0))))      # of many a few more fill the chip
+
+
 def latent_decode_heads(q, uk, uv, cache, block_tables, positions, rot_dim: int, scale: float, window: int, cos_sin, interleaved: bool,
                         out, max_keys: int = 0, sinks=None, gate=None, per_head: bool = False) -> torch.Tensor:
     """Head outputs ``out`` [T, H * vdim] of decode rows on cached latents (``decode_heads_ok``): ``q`` [T, H * (dim + rot_dim)], the key
     and value up-projections ``uk`` [H, dim, 512] and ``uv`` [H, vdim, 512], the rest as ``latent_attn_rows`` and ``gate_heads``.  Three
-    launches: queries folded, attention in runs of keys, and one that combines the runs, takes the sums to values and applies
+    launches: queries folded, attention in runs of keys (``decode_runs``), and one that combines the runs, takes the sums to values and applies
     the gate.  32 rows of 32 heads, 8 runs: 4.4 and 8.0 us around the attention's 29; the library's products, the combining pass
-    and the one that puts the heads side by side took 28.  Runs of 64 keys pay here, as combining them is no pass of its own (a layer, runs of
-    128, 64 and 32 keys: 3 rows of 16 heads over 612 20.4, 18.0, 17.9 us; 29 over 136 23.4, 20.5, 21.2), but not two runs instead of one (70 rows of 16 heads over 60, tables of 144: 24.2, in one run 20.9; 128 26.9, 22.1)."""
+    and the one that puts the heads side by side took 28."""
     _native(q)
     T, (H, dim, kr) = q.shape[0], uk.shape
     q_lat, o_lat = (torch.empty(H, T, kr, dtype=q.dtype, device=q.device) for _ in range(2))
     bound = min(max_keys, window) if window > 0 and max_keys > 0 else max_keys
-    runs = tile_runs(T, H, bound, 64) if bound >= 192 else 1
+    runs = decode_runs(T, H, bound)
     po = pm = None
     if runs > 1:
         po = torch.empty(runs * H * T * kr, dtype=torch.float32, device=q.device)

@@ -170,3 +170,24 @@ def test_contexts_around_the_tiles(H):
         # both roundings that move a score (the folded query, a rotated value between two bf16 numbers) are the reference's up to their ties; the
         # values and the result are rounded once each
         assert ((one.cpu().to(F64) - want).norm() / want.norm()) <= 2.0 ** -6, p
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,pos", [(64, 32, None), (70, 16, None), (129, 16, None), (17, 32, None), (256, 32, 100)])
+def test_many_rows(T, H, pos):
+    """Rows of several workgroups each way: no runs, two (four rows of a group at once), three and four (two at once), and folds of 32 and 64 rows."""
+    for keys in (1 << 7, 250, 400, 600):
+        compare(T, H, 64, 128, None if keys == 250 else "element", keys=(keys,), pos=None if pos is None else [t % pos for t in range(T)])
+
+
+def test_runs_of_keys_cpu():
+    """At most what fills the chip, at least 64 keys each; fewer for many rows, where writing a run's sums costs more than it saves."""
+    for rows in (0, 1, 7, 32, 64, 100, 128, 300):
+        for heads in (1, 16, 32, 64):
+            last = 1
+            for bound in (0, 100, 191, 192, 300, 700, 3000, 30000, 1 << 20):
+                n = latent.decode_runs(rows, heads, bound)
+                assert 1 <= n <= max(1, min(64, bound // 64)) and n * max(rows, 1) <= max(256, rows) and n >= last
+                last = n
+    assert [latent.decode_runs(64, 32, b) for b in (192, 240, 320, 576, 1312)] == [1, 2, 2, 3, 4]
+    assert [latent.decode_runs(128, h, 384) for h in (16, 32)] == [2, 1] and latent.decode_runs(32, 32, 2564) == 8
