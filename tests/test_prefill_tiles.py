@@ -167,3 +167,22 @@ def test_caps_factors_and_gates(D, cap, scale):
     open_ = torch.sigmoid(gate.float())
     slack = open_ * v.float().abs().max() * (2.0 ** -8 + 2 * cap * 2.0 ** -23) + 2.0 ** -8 * want.abs() + 1e-6
     assert torch.isfinite(got).all() and ((got - want).abs() <= slack).all(), ((got - want).abs() / slack).max()
+
+
+def test_element_gates_to_the_last_bits():
+    """A row that sees its own key alone is its value times the gate's sigmoid: exp, sum, quotient and product are off by 4 x 2^-24 at most (two and a half measured for
+    the sigmoid over all gates, half a unit of the product's), so a result is not the nearest bf16 number only where two are as near as that."""
+    n, nh, hd = 512, 16, 128
+    g = torch.Generator(device="cuda").manual_seed(9)
+    kc = torch.zeros(n, nh, 16, hd, device="cuda", dtype=torch.bfloat16)
+    vc = torch.randn(n, nh, 16, hd, device="cuda", generator=g).bfloat16()
+    gate = ((torch.rand(n, nh * hd, device="cuda", generator=g) * 2 - 1) * 30).bfloat16()
+    i32 = dict(device="cuda", dtype=torch.int32)
+    out = mix.paged_prefill_masked(torch.zeros(n, nh * hd, device="cuda", dtype=torch.bfloat16), kc, vc, torch.arange(n, **i32)[:, None].contiguous(),
+                                   torch.arange(n + 1, **i32), torch.ones(n, **i32), nh, nh, 1.0, 1024, gate)
+    want = vc[:, :, 0].reshape(n, -1).double() * torch.sigmoid(gate.double())
+    near = want.float().bfloat16()
+    wrong = out != near
+    middle = (out.double() + near.double()) / 2
+    assert bool(((want - middle).abs() <= 4 * 2.0 ** -24 * want.abs())[wrong].all())
+    assert wrong.float().mean() <= 4 * 2 * 2.0 ** -24 * 2 ** 8      # that near lie at most so many
