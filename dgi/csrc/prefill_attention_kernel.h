@@ -112,13 +112,12 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void prefill_attn_kernel(
   const int kvh = hx % nkv;
   const int head = kvh * (nh / nkv) + hx / nkv;
   // per-head score factor: folded into the scale; the softmax below takes maxima of raw scores, so a negative
-  // factor flips the raw scores' sign (the query's, and what is added to them), and a factor of zero stays above it (masked keys are -inf)
+  // factor flips the raw scores' sign (the query's; a distance bias never comes with factors), and a factor of zero stays above it (masked keys are -inf)
   bool flip = false;
   if (MASKED && head_scale) {
     scale_log2 *= head_scale[head];
     flip = scale_log2 < 0.f;
     scale_log2 = fmaxf(fabsf(scale_log2), 1e-30f);
-    if (flip) inv_scale = -inv_scale;
   }
   const int q0 = cu_seqlens_q[b];
   const int qlen = cu_seqlens_q[b + 1] - q0;
