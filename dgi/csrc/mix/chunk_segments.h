@@ -82,7 +82,7 @@ __device__ __forceinline__ uint32_t take_part(float& x0, float& x1) {
   return p;
 }
 template <int PARTS>
-__device__ __forceinline__ float take_parts8(const float* x, u32x4* p) {      // not 0: one was not a finite number, or too large for three parts
+__device__ __forceinline__ float take_parts8(const float* x, u32x4* p) {      // not 0: one of three parts' was not a finite number
   float none = 0.f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -349,11 +349,9 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, NB, ONLY>::WAVES), (Lay<MOD
             for (int i = 0; i < 8; ++i) x[i] = row < left && 8 * piece + i < dk ? x[i] : 0.f;
           }
           u32x4 p[3];
-          if constexpr (PQ == 1) {                             // what is not a number stays in its channel
 #pragma unroll
-            for (int i = 0; i < 8; i += 2) most = larger3(most, x[i], x[i + 1]);
-          }
-          none += take_parts8<PQ>(x, p);
+          for (int i = 0; i < 8; i += 2) most = larger3(most, x[i], x[i + 1]);
+          none += take_parts8<PQ>(x, p);                       // one part: what is not a number stays in its channel
           char* to = sm + (u < HALF ? L::K : L::Q) + buf * L::ARRB + place(row, piece);
 #pragma unroll
           for (int i = 0; i < PQ; ++i) *reinterpret_cast<u32x4*>(to + i * L::PARTB) = p[i];
@@ -853,7 +851,11 @@ __global__ __launch_bounds__((64 * Lay<MODE, TI, NK, NB, ONLY>::WAVES), (Lay<MOD
     }
     take_products<GRID>(u, f, l, grid, xp);
     if constexpr (!ONLY && PU == 3) {
-      odd |= take_parts8<PU>(u, up) != 0.f;
+      float largest = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) largest = larger3(largest, u[i], u[i + 1]);
+      const float none = take_parts8<PU>(u, up);
+      odd |= !(largest < MOST) || none != 0.f;
     } else {
       float none = 0.f;
 #pragma unroll

@@ -1190,6 +1190,14 @@ extern "C" int dgi_linear_scan_segments(int mode, int dk, int dv, int H, int G, 
   return dgi_chunk_segments_plan(mode, dk, dv, H, n_seq, rows, in_f32, floats);
 }
 
+// The kernel of a step's portions, arguments as above: 0 this file's, 1 chunk_scan.hip or one of those it passes steps on to, 2 chunk_scan_decay.hip, 3 chunk_segments.h.
+extern "C" int dgi_linear_scan_form(int mode, int dk, int dv, int H, int G, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
+                                    int in_f32, const float* aux1, int aux1_stride) {
+  long long floats;
+  if (dgi_linear_scan_segments(mode, dk, dv, H, G, n_seq, rows, q, q_stride, k, k_stride, in_f32, aux1, aux1_stride, &floats)) return 3;
+  return n_seq ? chunk_form(mode, dk, dv, G, H, q, q_stride, k, k_stride, in_f32, n_seq, rows) : 0;
+}
+
 // whether the matrix memory of a step has several workgroups per head in one of its launches: its normaliser and maximum are staged
 extern "C" int dgi_linear_scan_staged(int dk, int dv, int H, int n_seq, int rows, const void* q, int q_stride, const void* k, int k_stride,
                                       int in_f32, int seg_rows) {

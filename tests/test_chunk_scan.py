@@ -5,9 +5,12 @@ sequences with and without a state, decode rows beside portions, segments, extre
 Tolerance: every output is a sum of at most a few hundred products whose factors carry relative errors of some 16 roundings (the
 products of decays inside a chunk) of 6e-8, about 1e-6 of the sum of magnitudes; 3e-5 of the largest output, as the other tests of
 these recurrences allow."""
+import ctypes
+
 import pytest
 import torch
 
+import dgi.build
 from dgi.ops import linrec, recur
 
 F64 = torch.float64
@@ -41,6 +44,19 @@ def make(mode, lens, H, D, V, dtype, past, seed=0, pad=0):
     else:
         d["par"] = (torch.rand(H, generator=g) ** 0.1,)
     return d
+
+
+def route(d):
+    """The kernel that takes the step's portions: 0 the token loop, 1 chunk_scan.hip or those it passes steps on to (all of light: chunk_parts.hip),
+    2 chunk_scan_decay.hip, 3 chunk_segments.h; with the last one, whether long portions are cut."""
+    lib, floats, at = ctypes.CDLL(dgi.build.build(group="mix")), ctypes.c_longlong(), ctypes.c_void_p(4096)
+    H, G, D, V, fp32 = d["H"], d.get("G", d["H"]), d["D"], d["V"], d["q"].dtype == torch.float32
+    row = 2 * G * D + H * V + d["pad"]
+    args = (["wkv", "delta", "mlstm", "gla", "light"].index(d["mode"]), D, V, H, G, len(d["lens"]), sum(d["lens"]), at, row,
+            ctypes.c_void_p(4096 + G * D * (4 if fp32 else 2)), row, int(fp32), at, H * D)
+    form = lib.dgi_linear_scan_form(*args)
+    lib.dgi_linear_scan_segments(*args, ctypes.byref(floats))
+    return (form, floats.value > 0) if form == 3 else form
 
 
 def call(d, **kw):

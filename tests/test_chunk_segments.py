@@ -8,6 +8,8 @@ import torch
 
 import test_chunk_scan as base
 from dgi.ops import linrec
+from test_chunk_parts import where_finite
+from test_scan_precision import compare, in_short_portions, of_kind
 
 F64 = torch.float64
 pytestmark = pytest.mark.gpu
@@ -102,6 +104,47 @@ def test_non_finite_values_stay_behind(mode):
             assert (a - b).abs().max() <= 1e-5 * want.abs().max()
         if bad != 3e38:
             assert not torch.isfinite(got[171, 3])
+
+
+# more than sixteen chunks of one portion in segments; whole portions of many heads
+STEPS = pytest.mark.parametrize("lens,H,cut", [([450], 6, True), ([130, 40, 170], 66, False)], ids=["segments", "whole"])
+
+
+def loop(d):
+    """The same tokens one by one: the matrix memory's loop takes rows off a four-element boundary, the others' steps of up to four rows."""
+    return base.call(dict(d, pad=1)) if d["mode"] == "mlstm" else in_short_portions(d, 4, call)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("mode", ["gla", "light", "mlstm"])
+@pytest.mark.parametrize("what", ["q", "k", "v", "gate", "state", "large"])
+@STEPS
+def test_not_finite(lens, H, cut, what, mode, dtype):
+    """Infinities and NaN in what a token brings, or in the state: the same results are finite as token by token.  Values too large for three parts."""
+    if mode == "light" and what == "gate":
+        pytest.skip("light layers have one decay a head")
+    for bad in (float("inf"), float("nan")) if what != "large" else (3.39e38,):
+        d = make(mode, lens, H, 64, 64, dtype)
+        d["past"] = [3] * len(lens)
+        if what == "state":
+            d["S"][len(lens), 2, 3, 4] = bad
+        elif what == "gate":
+            d["decay" if mode == "gla" else "a"][71, 2] = bad
+        else:
+            d["k" if what == "large" else what][71, 5] = bad
+        assert base.route(d) == (3, cut)
+        where_finite(call(d)[:2], loop(d)[:2])
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (64, torch.float32), (128, torch.bfloat16), (128, torch.float32)])
+@pytest.mark.parametrize("mode,kind", [("gla", "plain"), ("gla", "share"), ("light", "plain"), ("light", "slow")])
+@pytest.mark.parametrize("lens,H,cut", [([800], 6, True), ([130, 40, 170], 66, False)], ids=["segments", "whole"])
+def test_no_further_off_than_the_loop(lens, H, cut, mode, kind, D, dtype):
+    """As test_scan_precision.py's."""
+    d = of_kind(make(mode, lens, H, D, 64, dtype), kind, 3)
+    d["past"] = [7] * len(lens)
+    assert base.route(d) == (3, cut)
+    compare(mode, call(d)[:2], loop(d)[:2], oracle(d)[:2])
 
 
 @torch.inference_mode()      # as models run, and other tests capture

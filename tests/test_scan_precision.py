@@ -28,7 +28,7 @@ def compare(mode, fast, loop, want, limit=1.05):
         assert x <= limit * y, (n, x, y)
 
 
-def in_short_portions(d, rows):
+def in_short_portions(d, rows, call=call):
     """The same tokens, at most ``rows`` of a sequence per call."""
     at, done, outs = [0] * len(d["lens"]), [], [[] for _ in d["lens"]]
     cur = dict(d)
@@ -39,7 +39,7 @@ def in_short_portions(d, rows):
             return (torch.cat([torch.cat(o) for o in outs]),) + tuple(done)
         idx = torch.cat([torch.arange(f + a, f + a + t) for f, a, t in zip(first, at, take)])
         cur.update(lens=take, past=[p + a for p, a in zip(d["past"], at)])
-        for k in ("q", "k", "v", "a", "b", "xbc", "dt"):
+        for k in ("q", "k", "v", "a", "b", "xbc", "dt", "decay"):
             if k in d:
                 cur[k] = d[k][idx]
         done = call(cur)
