@@ -6,7 +6,7 @@ Tolerance: as test_chunk_scan's, 3e-5 of the largest output."""
 import pytest
 import torch
 
-from test_chunk_scan import F64, call, check, make, oracle
+from test_chunk_scan import F64, call, check, make, oracle, route
 from test_scan_precision import in_short_portions
 
 pytestmark = pytest.mark.gpu
@@ -17,7 +17,7 @@ def run(d):
 
 
 def heads(mode, V):
-    return 8 if mode == "ssm" else 400 // -(-V // 16) + 1 if mode == "light" else 4      # light: enough workgroups for this kernel
+    return 8 if mode == "ssm" else 400 // -(-V // 16) + 1 if mode == "light" else 4      # light: so many that most steps are chunk_segments.h's
 
 
 @pytest.mark.parametrize("mode", ["mlstm", "light", "ssm"])
@@ -29,6 +29,27 @@ def test_sizes(mode, dtype, D, V, lens):
         lens = [n + 96 if n > 90 else n for n in lens]
     d = make(mode, lens, heads(mode, V), D, V, dtype, [3 * (i % 2) for i in range(len(lens))], seed=D + V)
     check(run(d), oracle(d))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,V", [(64, 64), (4, 16), (20, 8), (36, 17), (64, 33), (68, 48), (100, 48), (128, 33), (128, 100)])
+@pytest.mark.parametrize("lens", [[257], [288, 225, 320, 31, 32, 33, 1], [255, 289], [170, 166]], ids=lambda x: "-".join(map(str, x)))
+def test_sizes_of_light(dtype, D, V, lens):
+    """Few heads, so that these portions are this kernel's: the lengths of the other layers with five chunks more."""
+    d = make("light", lens, 4, D, V, dtype, [3 * (i % 2) for i in range(len(lens))], seed=D + V)
+    assert route(d) == 1
+    check(call(d), oracle(d))
+
+
+@pytest.mark.parametrize("lens,H,D,V", [([65], 70, 64, 64), ([257], 70, 64, 64), ([272, 273], 70, 64, 64), ([15, 400, 1], 50, 64, 64), ([1] * 9 + [17, 520, 300], 10, 128, 128),
+                                        ([280, 284, 384, 260, 320, 256, 324, 264, 316], 17, 64, 64), ([280, 284, 384, 260, 320, 256, 324, 264, 316], 16, 48, 33),
+                                        ([2000] + [68, 80, 72, 132, 76, 68, 84, 72], 17, 64, 64), ([280, 284, 384, 260, 320, 256, 324, 264, 316], 8, 60, 130)],
+                         ids=lambda x: "-".join(map(str, x))[:16] if isinstance(x, list) else str(x))
+def test_lengths_of_light(lens, H, D, V):
+    """One block of value columns a workgroup and, of more than 256 workgroups, two; up to eight sequences in one launch, more in two."""
+    d = make("light", lens, H, D, V, torch.bfloat16 if H in (16, 17) else torch.float32, [3 * (i % 2) for i in range(len(lens))], seed=len(lens) + V)
+    assert route(d) == 1
+    check(call(d), oracle(d))
 
 
 @pytest.mark.parametrize("H,D,lens", [(8, 128, [1500, 40]), (8, 60, [700]), (12, 64, [600, 0, 70])])
@@ -115,6 +136,7 @@ def test_not_finite_bf16(what, mode, D):
                 d["S"][1, 2, 3, 4] = bad
             else:
                 d["k" if what == "large" else what][71, 5] = bad
+            assert route(d) == 1
             slow = call(dict(d, pad=1)) if mode == "mlstm" else in_short_portions(d, 4)
             where_finite(call(d)[:2], slow[:2])
 
@@ -123,6 +145,7 @@ def test_light_decays_that_are_none():
     """Decays of 0, below 0 and above 1 (whose powers may leave the fp32 range)."""
     d = make("light", [200], 104, 64, 32, torch.float32, [3])
     d["par"][0][:6] = torch.tensor([0.0, -0.5, 1.0, 1.01, 1e-30, 100.0])
+    assert route(d) == 1
     got, want = run(d), oracle(d)
     for h in range(104):
         g, w = got[0].view(200, 104, 32)[:, h].to(F64), want[0].view(200, 104, 32)[:, h]
