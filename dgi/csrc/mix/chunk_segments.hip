@@ -9,7 +9,8 @@ int dgi_segments_mlstm(const ChunkArgs& a, int in_f32, bool only, dim3 grid, hip
 int dgi_segments_light(const ChunkArgs& a, int in_f32, bool only, dim3 grid, hipStream_t st);
 int dgi_segments_gla(const ChunkArgs& a, int in_f32, bool only, dim3 grid, hipStream_t st);
 
-// blocks of 16 columns of a workgroup (the matrix memory's thirteen waves would have 128 registers each, and spill)
+// blocks of 16 columns of a workgroup.  The matrix memory's thirteen waves would have 128 registers each, and spill.  gla's twelve, of more than 64 key channels, have 168
+// and spill as well: the outputs' launch 78 registers of fp32 rows (52 bytes a lane), 10 of bf16 ones.
 static int wide(int mode, int dv) { return dv <= 64 || mode == MLSTM ? 4 : 8; }
 // workgroups of a head: the matrix memory's normaliser is staged if there are several
 int dgi_chunk_segments_groups(int mode, int dv) { return (dv + 16 * wide(mode, dv) - 1) / (16 * wide(mode, dv)); }
