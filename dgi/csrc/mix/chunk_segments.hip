@@ -40,13 +40,17 @@ float dgi_chunk_segments_share(int mode, int dk, int dv, int H) {
 // - long portions of few heads, in segments: gla 16, 1 x 2000 123, 31; 32, 2 x 500 41, 28; light 16, 1 x 2000 96, 27; 64, 2 x 2048 125, 109; but gla 64, 1 x 300 23.2, 25.3; 128
 //   channels, 300 rows 33, 42, so 400 there;
 // - rows enough for one portion to be long: gla 16, 1 of 1521 among 5 95, 26; light 16, 1 of 1473 among 11 82, 47; but gla 16, 4 x 190 17, 23; fp32 4, 4 x 228 of 128
-//   channels 28, 60, so from 1000 rows there; light 16, 8 x 500 38, 42;
+//   channels 28, 60, so from 1000 rows there; light 16, 8 x 500 38, 42;  of four and eight heads alike portions lose most, and long ones gain most: gla 8, 8 x 108 12, 20, but 1 of 850
+//   among 10 55, 22; light of 128 channels 4, 10 x 270 34, 60, but 1 of 1554 among 30 164, 52;
 // - mlstm's nine waves fill a compute unit, and its pipeline is the closer one: a nearly full chip of bf16 rows stays there (32, 5 x 600 55, 60; 64, 5 x 613 83, 98), as do long
 //   portions beside decode rows of many heads (64, 8 of 3173 rows and 59 147, 195); more than 64 channels would spill.  Its token loop takes 0.5 us a token, so short portions come here
 //   (64, 3 x 40 35, 12; 16, 8 x 20 20, 9), among nine sequences and more it has two launches to lose (16, 16 x 62 23, 15; fp32 64, 12 x 75 79, 45); full chips: 64, 3 x 100 25, 17; 32, 8 x 83
-//   23, 15; fp32 64, 3 x 300 55, 45; 8 x 500 153, 128; long portions: 32, 1 x 661 39, 25; 16, 1 x 2000 89, 33; 32, 1 of 2000 among 17 107, 64; but 32, 3 x 459 35, 46.
+//   23, 15; fp32 64, 3 x 300 55, 45; 8 x 500 153, 128; long portions: 32, 1 x 661 39, 25; 16, 1 x 2000 89, 33; 32, 1 of 2000 among 17 107, 64; but 32, 3 x 459 35, 46;
+//   fp32 rows of a third of the chip and more stay there (32, 3 x 535 48, 67), as do those beside more decode rows (32, 2 of 1547 and 92 114, 139).
 // The launch of the states, in vain if no portion turns out to be worth cutting, costs 3 to 6 us; a long portion left whole 2 us for 32 rows of it, 4 of 128 channels.  Many portions
-// and heads: it is launched where one may have more than 400 to 1000 rows (64 heads, 3 x 300 29, in vain 36; 32, 1 of 765 among 7 52, 28), and, among more than 64 sequences, than
+// and heads: it is launched where one may have more than 350 to 550 rows, which is where alike ones in vain are no slower than there (there, whole, cut: light 32 heads of 128 channels, 1 of 665
+// rows and 9 74, 110, 61; 32, 1 of 801 and 5 43, 55, 29; mlstm 16, 1 of 597 and 6 37, 46, 28; alike: light 64, 3 of 602 rows in all 30, 24, 29; 5 of 1043 47, 33, 39; but mlstm 32, 3 of 626 25, 24,
+// 30), and, among more than 64 sequences, than
 // the workgroups of those that turn out to be short cost: 2 us for as many as the chip has at once, in both launches (64 heads of 128 channels, 3747 rows of 203 sequences 772, cut 996; of
 // 64, 4000 rows and 500 decode rows 635, 525; 2 of 2000 and 1000 744, 790).
 int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows, int in_f32, long long* floats) {
@@ -62,12 +66,12 @@ int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows
       many = here = mean >= (n_seq > 2 * APART_FROM ? 24 : 16);
     } else if (n_seq > 2 * APART_FROM) {
       many = false;
-      here = over >= (f ? 1000 : 1600) && H * groups <= (f && n_seq <= 32 ? 64 : 32) && n_seq <= 100 && fill < (f ? 700.f : 500.f);
+      here = over >= (f ? 1000 : 1600) && H * groups <= (f && n_seq <= 32 ? 64 : 32) && n_seq <= 80 && fill < (f ? 700.f : 500.f);
     } else if (n_seq > APART_FROM) {
       many = here = mean >= 16 && (f || fill < 400.f);
     } else {
       many = f && mean >= 100 ? units >= 192 : units >= 96 && mean < 160;
-      here = many || (units <= 100 && mean >= 400) || (units <= 64 && over >= 1000);
+      here = many || (units <= (f ? 64 : 100) && mean >= 400) || (units <= 64 && over >= 1000);
     }
   } else {
     const bool gla = mode == GLA, wide = dk > 64;
@@ -78,7 +82,7 @@ int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows
   if (!here) return 0;
   // segments that fill the chip once; of 128 rows at least where sixteen of them are no more than a portion
   const long each = (std::max({96l, (long)fill, std::min(128l, rows / 16l)}) + C - 1) / C * C;
-  const long keep = !many ? 1 : n_seq > 64 ? std::max(400l, (long)(80 * share * std::min(n_seq, rows / 17))) : n_seq > 2 * APART_FROM ? 768 : n_seq > APART_FROM ? 1000 : mode == MLSTM ? 600 : dk > 64 ? 700 : 1000;
+  const long keep = !many ? 1 : n_seq > 64 ? std::max(400l, (long)(80 * share * std::min(n_seq, rows / 17))) : mode == MLSTM ? 550 : dk > 64 ? 350 : 500;
   if (over < keep || whole(over + 1, rows, share, each) || !places(rows, each)) return 1 << 29;
   *floats = places(rows, each) * H * (state_floats(mode, dk, dv) + decay_floats(mode, dk));
   return (int)each;

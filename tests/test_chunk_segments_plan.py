@@ -67,7 +67,8 @@ HERE = [("gla", 64, 3, 120, 64, 0), ("gla", 64, 16, 1120, 64, 0), ("gla", 64, 8,
         ("mlstm", 64, 12, 900, 64, 1), ("mlstm", 64, 3, 300, 64, 0), ("mlstm", 32, 8, 664, 64, 0), ("mlstm", 64, 3, 900, 64, 1), ("mlstm", 64, 8, 4000, 64, 1),
         ("mlstm", 32, 1, 661, 64, 0), ("mlstm", 16, 1, 2000, 64, 0), ("mlstm", 32, 17, 2016, 64, 0), ("mlstm", 32, 3, 1377, 64, 0)]
 THERE = [("gla", 16, 8, 160, 64, 0), ("gla", 4, 4, 912, 128, 1), ("gla", 16, 10, 100, 64, 0), ("gla", 16, 1, 300, 128, 0), ("gla", 16, 1, 250, 64, 0), ("light", 16, 3, 300, 64, 0),
-         ("mlstm", 32, 5, 3000, 64, 0), ("mlstm", 64, 5, 3065, 64, 0), ("mlstm", 64, 67, 3232, 64, 0), ("mlstm", 16, 1, 2000, 128, 0), ("mlstm", 64, 2, 5438, 64, 1)]
+         ("mlstm", 32, 5, 3000, 64, 0), ("mlstm", 64, 5, 3065, 64, 0), ("mlstm", 64, 67, 3232, 64, 0), ("mlstm", 16, 1, 2000, 128, 0), ("mlstm", 64, 2, 5438, 64, 1),
+         ("mlstm", 32, 3, 1605, 64, 1), ("mlstm", 32, 94, 1639, 64, 1)]
 
 
 @pytest.mark.parametrize("mode,H,n,rows,D,fp32", HERE + THERE)
@@ -78,8 +79,9 @@ def test_rule(lib, mode, H, n, rows, D, fp32):
 def test_long_portions_are_cut(lib):
     """One portion that may have most of the rows gets a launch of its states; alike ones among few heads are cut fine enough to fill the chip."""
     for mode, H, n, rows, D in (("gla", 16, 1, 2000, 64), ("light", 16, 8, 4000, 64), ("light", 64, 8, 2000, 64), ("light", 32, 4, 758, 128), ("gla", 16, 500, 2754, 64),
-                                ("mlstm", 32, 17, 2016, 64), ("gla", 64, 501, 4500, 64)):
+                                ("mlstm", 32, 17, 2016, 64), ("gla", 64, 501, 4500, 64), ("light", 32, 4, 698, 128), ("light", 32, 10, 674, 128), ("light", 32, 6, 806, 64),
+                                ("light", 64, 3, 900, 64), ("mlstm", 16, 7, 603, 64), ("mlstm", 32, 14, 750, 64)):
         each, floats = plan(lib, mode, H, n, rows, D)
         assert 0 < each <= max(128, rows * H // 256 + 31) and floats > 0
-    for mode, H, n, rows, D in (("gla", 64, 3, 300, 64), ("light", 64, 3, 900, 64), ("gla", 64, 203, 3747, 128)):
+    for mode, H, n, rows, D in (("gla", 64, 3, 300, 64), ("light", 64, 3, 480, 64), ("mlstm", 64, 3, 300, 64), ("gla", 64, 203, 3747, 128)):
         assert plan(lib, mode, H, n, rows, D) == (1 << 29, 0)
