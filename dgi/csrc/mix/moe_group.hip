@@ -928,14 +928,16 @@ int launch_group(GroupArgs g, int places, int rows_per_tile, hipStream_t s) {
     // are faster than tiles of 128 (128, 256: 16 experts of 2048 x 2048 mean 62 144 us, 117; 2048 x 4096 mean 75 256, 209; 4096 x 3584 mean 50 333, 293; 8 of
     // 4096 x 14336 mean 50 681, 614; 64 of 2048 x 1408 mean 61 292, 263; 128 of 2048 x 768 mean 81 393, 310; 16 of 1024 x 1024 mean 50 57, 52), but for small ones of
     // few steps (32 of 1024 x 512 mean 38 50, 52, mean 75 52, 51).  Up to 52 places an expert, which seldom are more than 64, streamed weights are faster
-    // still (64, 256: 2048 x 2048 mean 50 101, 117, mean 62 141, 117; 2048 x 4096 mean 50 203, 213; 1024 x 2048 mean 50 44, 65; but 1024 x 1024 54, 52).
+    // still (64, 256: 2048 x 2048 mean 50 101, 117, mean 62 141, 117; 2048 x 4096 mean 50 203, 213; 1024 x 2048 mean 50 44, 65; but 1024 x 1024 54, 52); of more than
+    // sixteen experts one of them has more than 64 sooner, which costs those least whose weights are most of the work (mean 46, 51, 128 there, 64, 256: 32 of 1536 x 1024 92, 92, 78, 93, 97, 80; 32 of 1024 x 2048 119, 100, 106, 121, 120, 106; 32 of
+    // 1536 x 1536 136, 117, 115, 137, 126, 118; 64 of 2048 x 1408 286, 233, 248, 289, 257, 253; but 32 of 2048 x 2048 226, 177, 210, 227, 182, 211).
     // The line is that of routes that are alike.  Where experts get very different numbers (the router's logits biased by normal values of spread 0.8) and the step
     // is one round of tiles of 128, small experts lose what alike ones gain (128, 256: 32 of 1024 x 512 mean 112 alike 56, 49, biased 55, 61; 16 of 1024 x 1024 mean 137
     // 57, 52, 57, 61; 8 of 1024 x 2048 mean 187 67, 61, 66, 73); from two rounds on both gain (16 of 1024 x 1024 mean 250 85, 65; 32 of 1536 x 1024 mean 112 135, 110).
     const long long a_bytes = 2ll * g.a_stride * (g.order ? (places + g.top - 1) / g.top : places);
     const long long b_bytes = 2ll * g.N * g.K * (GLU ? 2 : 1);
     if (g.K % 128 || g.N % 8 || ((uintptr_t)g.out & 15) || a_bytes >= 1ll << 31 || b_bytes >= 1ll << 31) bm = 128;
-    else if (bm == 128 && places <= 52ll * g.E && (long long)g.N * g.K > 1 << 20 && streams(64, g.K)) bm = 64;
+    else if (bm == 128 && places <= (g.E > 16 && (long long)g.N * g.K < 3 << 20 ? 48ll : 52ll) * g.E && (long long)g.N * g.K > 1 << 20 && streams(64, g.K)) bm = 64;
     else if ((long long)g.N * g.K > 1 << 19 || places > 64ll * g.E) bm = WIDE;
   }
   g.mtiles = places / bm + nonempty;
