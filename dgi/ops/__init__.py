@@ -607,24 +607,27 @@ def _linear_stream(x, w, bias, out) -> Optional[torch.Tensor]:
 
 def tile_gemm(M: int, N: int) -> bool:
     """Rows and outputs whose tiles nearly fill whole rounds of the chip on the ping-pong kernel (``mfma_gemm``, whole tiles: its split-K
-    workspace belongs to one stream at a time): large vocabularies and 129 to 1024 rows.  ``linear`` takes it where ``tile_pays`` too."""
+    workspace belongs to one stream at a time): large vocabularies and 129 to 1024 rows.  ``linear`` takes it where ``tile_pays`` too.  Tiles are
+    counted at 256 rows here; the launch takes lower ones where that is less time (``row_tiles`` in mfma_gemm.hip)."""
     tiles = -(-M // 256) * (N // 256)
     return 128 < M <= 1024 and N >= 384 * 256 and 8 * tiles >= 7 * -(-tiles // 256) * 256
 
 
 def tile_pays(M: int, N: int) -> bool:
-    """Where the vendor's product is the slower of the two: outputs that are no multiple of 512, the last rows more than a third of a tile.  Its
-    time over this one's at 129, 256, 300, 353, 400, 512, 1024 rows: 128256 x 4096 1.32, 1.15, 0.92, 1.04, 1.18, 1.16, 1.07, 115968 x 3584 1.32, 1.25,
-    0.97, 1.06, 1.20, 1.23, 0.95, 256256 x 2048 1.26, 1.16, 0.84, 0.94, 1.11, 1.12, 1.02; but 128512 x 3584 0.90, 0.93, 0.78, 0.87, 0.98, 0.96, 0.91,
-    131072 x 2304 0.95, 0.90, 0.85, 0.89, -, 0.93, 0.94."""
+    """Where the vendor's product is the slower of the two: outputs that are no multiple of 512, the last rows more than a third of a tile of 256.  Its
+    time over this one's at 129, 256, 353, 400, 512, 640, 900, 1024 rows: 128256 x 4096 1.36, 1.25, 1.20, 1.33, 1.25, 1.15, 1.09, 1.13, 115968 x 3584 1.33,
+    1.28, 1.12, 1.25, 1.23, 1.07, 0.93, 1.00, 256256 x 2048 1.22, 1.15, 0.98, 1.12, 1.11, 1.13, 1.06, 1.07; but 128512 x 3584 0.87, 0.92, 0.87, 0.94, 0.92, 1.01,
+    0.98, 1.00, 131072 x 2304 0.91, 0.85, 0.89, 0.99, 0.96, 0.98, 0.98, 0.95.  The line was drawn with tiles of 256 rows (300 rows of the first three 0.92,
+    0.97, 0.84); with lower ones it leaves something there (1.15, 1.07, 0.97) and at 151552 x 4096 (1.03, 1.07, 1.13, 1.19, 1.13, 1.15, 1.02, 1.04)."""
     return N % 512 == 256 and (M - 1) % 256 >= 96
 
 
 def split_gemm(M: int, N: int, K: int) -> bool:
     """Whether a product of long rows, 129 to 512 of them, is better split along K by ``mfma_gemm``: where its tiles of 256 x 256 give 96 to 256
-    blocks in four pieces.  Vendor's product and this one, us, at 129 / 256 / 353 / 512 rows: 8192 x 28672 299, 197 / 312, 195 / 199, 196 / 315, 201; 6144 x
-    24576 184, 166 / 279, 172 / 215, 170 / 285, 175; 8192 x 16384 94, 130 / 157, 139 / 129, 126 / 160, 128.  Not 4096 x 32768 up to 256 rows (64 blocks:
-    160, 187 / 191, 194), 16384 x 53248 from 257 on (two pieces: 257 rows 508, 635), 640 rows of 8192 x 28672 (264, 310)."""
+    blocks in four pieces (counted so; the launch may take lower tiles, ``row_tiles`` in mfma_gemm.hip).  Vendor's product and this one, us, at 129 / 256 / 353
+    / 512 rows: 8192 x 28672 300, 174 / 312, 170 / 185, 177 / 309, 190; 6144 x 24576 178, 149 / 291, 143 / 212, 150 / 281, 163; 8192 x 16384 91, 115 / 144, 109 /
+    120, 116 / 147, 125.  Not 16384 x 53248 from 257 rows on (two pieces: 467, 558), 640 rows of 8192 x 28672 (252, 283), 129 to 192 of 4096 x 32768 (64 blocks: 156,
+    171 / 161, 172 / 168, 160), though 256 of them would gain (187, 164) as would 256 of 5120 x 27648 (264, 151)."""
     tiles = -(-M // 256) * (N // 256)
     return 128 < M <= 512 and K >= 16384 and N * K >= 1 << 27 and 24 <= tiles <= 64 and (M > 160 or K >= 24576)
 
