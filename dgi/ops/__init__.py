@@ -626,8 +626,8 @@ def split_gemm(M: int, N: int, K: int) -> bool:
     """Whether a product of long rows, 129 to 512 of them, is better split along K by ``mfma_gemm``: where its tiles of 256 x 256 give 96 to 256
     blocks in four pieces (counted so; the launch may take lower tiles, ``row_tiles`` in mfma_gemm.hip).  Vendor's product and this one, us, at 129 / 256 / 353
     / 512 rows: 8192 x 28672 300, 174 / 312, 170 / 185, 177 / 309, 190; 6144 x 24576 178, 149 / 291, 143 / 212, 150 / 281, 163; 8192 x 16384 91, 115 / 144, 109 /
-    120, 116 / 147, 125.  Not 16384 x 53248 from 257 rows on (two pieces: 467, 558), 640 rows of 8192 x 28672 (252, 283), 129 to 192 of 4096 x 32768 (64 blocks: 156,
-    171 / 161, 172 / 168, 160), though 256 of them would gain (187, 164) as would 256 of 5120 x 27648 (264, 151)."""
+    120, 116 / 147, 125.  Not 16384 x 53248 from 257 rows on (two pieces: 467, 558), 640 rows of 8192 x 28672 (252, 283), 129 and 160 of 4096 x 32768 (64 blocks: 156,
+    171 / 161, 172), though 256 of them would gain (187, 164) as would 256 of 5120 x 27648 (264, 151)."""
     tiles = -(-M // 256) * (N // 256)
     return 128 < M <= 512 and K >= 16384 and N * K >= 1 << 27 and 24 <= tiles <= 64 and (M > 160 or K >= 24576)
 
