@@ -48,9 +48,10 @@ float dgi_chunk_segments_share(int mode, int dk, int dv, int H) {
 //   23, 15; fp32 64, 3 x 300 55, 45; 8 x 500 153, 128; long portions: 32, 1 x 661 39, 25; 16, 1 x 2000 89, 33; 32, 1 of 2000 among 17 107, 64; but 32, 3 x 459 35, 46;
 //   fp32 rows of a third of the chip and more stay there (32, 3 x 535 48, 67), as do those beside more decode rows (32, 2 of 1547 and 92 114, 139).
 // The launch of the states, in vain if no portion turns out to be worth cutting, costs 3 to 6 us; a long portion left whole 2 us for 32 rows of it, 4 of 128 channels.  Many portions
-// and heads: it is launched where one may have more than 350 to 550 rows, which is where alike ones in vain are no slower than there (there, whole, cut: light 32 heads of 128 channels, 1 of 665
-// rows and 9 74, 110, 61; 32, 1 of 801 and 5 43, 55, 29; mlstm 16, 1 of 597 and 6 37, 46, 28; alike: light 64, 3 of 602 rows in all 30, 24, 29; 5 of 1043 47, 33, 39; but mlstm 32, 3 of 626 25, 24,
-// 30), and, among more than 64 sequences, than
+// and heads: it is launched where one may have more than 600 to 1000 rows, or, but for gla, whose kernel there is slower than whole portions here, more than it takes cut by 150 to 250 and by 10 a
+// sequence: those lose most whole (there, whole, cut: light 32 heads of 128 channels, 1 of 665 rows and 9 74, 110, 61; 32, 1 of 801 and 5 43, 55, 29; mlstm 16, 1 of 597 and 6 37, 46, 28; 32, 1 of 900
+// and 10 73, 91, 48), and where they are alike it is in vain, but no slower than there (light 64, 3 of 602 rows in all 30, 23, 29; 5 of 1043 47, 33, 39; gla 64 of 128 channels, 8 of 560 119, 44, 54, so
+// whole).  Among more than 64 sequences it is launched where one may have more than 400 and more than
 // the workgroups of those that turn out to be short cost: 2 us for as many as the chip has at once, in both launches (64 heads of 128 channels, 3747 rows of 203 sequences 772, cut 996; of
 // 64, 4000 rows and 500 decode rows 635, 525; 2 of 2000 and 1000 744, 790).
 int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows, int in_f32, long long* floats) {
@@ -82,8 +83,11 @@ int dgi_chunk_segments_plan(int mode, int dk, int dv, int H, int n_seq, int rows
   if (!here) return 0;
   // segments that fill the chip once; of 128 rows at least where sixteen of them are no more than a portion
   const long each = (std::max({96l, (long)fill, std::min(128l, rows / 16l)}) + C - 1) / C * C;
-  const long keep = !many ? 1 : n_seq > 64 ? std::max(400l, (long)(80 * share * std::min(n_seq, rows / 17))) : mode == MLSTM ? 550 : dk > 64 ? 350 : 500;
-  if (over < keep || whole(over + 1, rows, share, each) || !places(rows, each)) return 1 << 29;
+  const float cut = 1.3f * (fill + each) + 96;         // as whole's
+  const long least_cut = n_seq > 64 ? std::max(400l, (long)(80 * share * std::min(n_seq, rows / 17)))
+                         : n_seq > 2 * APART_FROM ? 768 : n_seq > APART_FROM ? 1000 : mode == MLSTM ? 600 : dk > 64 ? 700 : 1000;
+  const long gains = mode == GLA || n_seq > 64 ? least_cut : (long)cut + (mode == MLSTM ? 250 : dk > 64 ? 150 : 200) + 10 * n_seq;
+  if ((many && over < std::min(least_cut, gains)) || whole(over + 1, rows, share, each) || !places(rows, each)) return 1 << 29;
   *floats = places(rows, each) * H * (state_floats(mode, dk, dv) + decay_floats(mode, dk));
   return (int)each;
 }

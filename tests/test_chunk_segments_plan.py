@@ -83,5 +83,5 @@ def test_long_portions_are_cut(lib):
                                 ("light", 64, 3, 900, 64), ("mlstm", 16, 7, 603, 64), ("mlstm", 32, 14, 750, 64)):
         each, floats = plan(lib, mode, H, n, rows, D)
         assert 0 < each <= max(128, rows * H // 256 + 31) and floats > 0
-    for mode, H, n, rows, D in (("gla", 64, 3, 300, 64), ("light", 64, 3, 480, 64), ("mlstm", 64, 3, 300, 64), ("gla", 64, 203, 3747, 128)):
+    for mode, H, n, rows, D in (("gla", 64, 3, 300, 64), ("gla", 64, 8, 560, 128), ("light", 64, 3, 480, 64), ("mlstm", 64, 3, 300, 64), ("gla", 64, 203, 3747, 128)):
         assert plan(lib, mode, H, n, rows, D) == (1 << 29, 0)
