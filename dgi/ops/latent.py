@@ -257,11 +257,11 @@ def decode_runs(rows: int, heads: int, bound: int) -> int:
     """Runs of keys per row of ``latent_decode_heads`` where no row has more than ``bound``: of 64 keys at least, as many as fill the chip, and no more than
     pay: a layer takes about 0.05 us a key of ``bound`` over the runs, and for every run (its sums are written and read again) 0.045 us a row of 32 heads, two thirds of that of 16.
     Us a layer in 1, 2, 3, 4, 8 runs, rows x heads, keys of about 0.75 ``bound``: 8 x 32, 200 28.1, 22.3, 20.7, 19.7, 19.7; 32 x 32, 160 28.1, 24.7, 24.4, 25.2, 27.3; 400 44.4, 32.2,
-    29.7, 27.4, 29.0; 64 x 32, 100 24.3, 25.8, 28.2, 29.8; 200 31.7, 27.9, 28.9, 31.0; 128 x 32, 250 38.9, 39.1; 128 x 16, 130 26.2, 28.1."""
+    29.7, 27.4, 29.0; 60 x 32, 410 46.5, 34.7, 33.9, 31.7, 41.3; 52 x 32, 330 40.6, 32.4, 32.0, 30.7, 39.1; 64 x 32, 100 24.3, 25.8, 28.2, 29.8; 200 31.7, 27.9, 28.9, 31.0; 128 x 32, 250 38.9, 39.1; 128 x 16, 130 26.2, 28.1."""
     if bound < 192:
         return 1
     best = (80 * bound / (max(rows, 1) * (heads + 32))) ** 0.5
-    return max(1, min(tile_runs(rows, heads, bound, 64), int(best + (0.7 if best > 3.5 else 0))))      # of many a few more fill the chip
+    return max(1, min(tile_runs(rows, heads, bound, 64), max(4, int(best + 0.7)) if best > 3.2 else int(best)))      # of many a few more fill the chip
 
 
 def latent_decode_heads(q, uk, uv, cache, block_tables, positions, rot_dim: int, scale: float, window: int, cos_sin, interleaved: bool,

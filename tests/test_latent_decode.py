@@ -189,5 +189,6 @@ def test_runs_of_keys_cpu():
                 n = latent.decode_runs(rows, heads, bound)
                 assert 1 <= n <= max(1, min(64, bound // 64)) and n * max(rows, 1) <= max(256, rows) and n >= last
                 last = n
-    assert [latent.decode_runs(64, 32, b) for b in (192, 240, 320, 576, 1312)] == [1, 2, 2, 3, 4]
+    assert [latent.decode_runs(64, 32, b) for b in (192, 240, 320, 480, 576, 1312)] == [1, 2, 2, 3, 4, 4]
+    assert latent.decode_runs(60, 32, 512) == 4 and latent.decode_runs(32, 32, 240) == 3      # four take less than three from about 450 keys on
     assert [latent.decode_runs(128, h, 384) for h in (16, 32)] == [2, 1] and latent.decode_runs(32, 32, 2564) == 8
